@@ -152,11 +152,8 @@ int32_t forge_hip_quantize_act(const float* x_dev, uint32_t M, uint32_t K, int8_
 int32_t forge_hip_gemv_q(const forge_hip_qweight* w, const float* x_dev, float* y_dev, void* stream) {
     FH_CHECK(w && x_dev && y_dev, "gemv_q: null pointer");
     FH_CHECK(gemv_k_supported(w->w.K), "gemv_q: K must be a multiple of 32, at most 16384");
-    int8_t* q; uint16_t* sc;
-    int32_t rc = quantise_into_scratch(x_dev, 1, w->w.K, &q, &sc, (hipStream_t)stream);
-    if (rc) return rc;
-    if (w->w.kquant()) launch_gemv_kquant(w->w, q, sc, y_dev, false, (hipStream_t)stream);
-    else launch_gemv(w->w, q, sc, y_dev, false, GemvOrder::MatmulVec, (hipStream_t)stream);
+    if (w->w.kquant()) launch_gemv_kquant_act(w->w, x_dev, y_dev, (hipStream_t)stream);
+    else launch_gemv_act(w->w, x_dev, y_dev, (hipStream_t)stream);
     FH_HIP(hipGetLastError());
     return FORGE_HIP_OK;
 }

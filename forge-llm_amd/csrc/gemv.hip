@@ -21,7 +21,10 @@
 //
 // A kernel boundary costs several microseconds on this GPU, more than streaming a small
 // matrix, so the decode step's neighbours are fused in:
-//   prologue  RmsNorm: rms_norm (emit.rs:327-334, the 16-lane FMA order of emit.rs:272-295) and the
+//   prologue  Act: the activation quantiser alone (the op-level product: one launch instead of two, 2048 -> 2048 Q8_0
+//             5.4 -> 4.0 us, 8192 -> 2048 7.9 -> 7.3, 2048 -> 128256 45.7 -> 43.7 as nodes of a graph; quantising in the
+//             registers of every wave instead took 4.4, 9.3 and 44.5)
+//             RmsNorm: rms_norm (emit.rs:327-334, the 16-lane FMA order of emit.rs:272-295) and the
 //             activation quantiser (emit.rs:1410-1440), recomputed by every workgroup from x, once per
 //             workgroup: codes and scales go to LDS, every wave reads its fragment from there
 //   epilogue  Add: residual_add (emit.rs:455-459);  RopeKv: rope (emit.rs:508-528) on the q and k
@@ -42,7 +45,7 @@ __device__ __forceinline__ int dot16(int4 w, int4 a, int acc) {
     return acc;
 }
 
-enum class Pro { Quant, RmsNorm };
+enum class Pro { Quant, RmsNorm, Act };
 enum class Epi { Store, Add, RopeKv, SiluQuant, Isums };
 
 
@@ -56,7 +59,7 @@ struct GemvArgs {
     // Pro::Quant
     const int8_t* aq;
     const uint16_t* as;
-    // Pro::RmsNorm
+    // Pro::RmsNorm, Pro::Act
     const float* x;
     const float* norm_w;
     float eps;
@@ -157,13 +160,22 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_kernel(GemvArgs a) {
     // fetched later, behind the weights): loads return in issue order, so behind the weights they would arrive only after them, and the
     // norm would wait for the weights instead of running while they travel.
     constexpr int XE = THREADS >= 1024 ? 1 : THREADS >= 512 ? 2 : 4;   // 4096 elements, at 16 waves within their 128 registers
-    float4 xe[PRO == Pro::RmsNorm ? XE : 1], we[PRO == Pro::RmsNorm ? XE : 1];
+    float4 xe[PRO != Pro::Quant ? XE : 1], we[PRO == Pro::RmsNorm ? XE : 1];
     if (PRO == Pro::RmsNorm) {
 #pragma unroll
         for (int i = 0; i < XE; i++) {
             const uint32_t e4 = i * THREADS + tid;
             xe[i] = we[i] = make_float4(0.f, 0.f, 0.f, 0.f);
             if (e4 < K / 4) { xe[i] = reinterpret_cast<const float4*>(a.x)[e4]; we[i] = reinterpret_cast<const float4*>(a.norm_w)[e4]; }
+        }
+    }
+
+    // (Pro::Act likewise)
+    if (PRO == Pro::Act) {
+#pragma unroll
+        for (int i = 0; i < XE; i++) {
+            const uint32_t e4 = i * THREADS + tid;
+            xe[i] = e4 < K / 4 ? reinterpret_cast<const float4*>(a.x)[e4] : make_float4(0.f, 0.f, 0.f, 0.f);
         }
     }
 
@@ -189,13 +201,20 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_kernel(GemvArgs a) {
     int4 av[NL], av2[Q4 ? NL : 1];
     int asum8[Q4 ? NL : 1];
     float asf[NL];
-    if (PRO == Pro::RmsNorm) {
-        // rms_norm of x[K] in the reference's summation order, then block quantisation, once per workgroup: 8 lanes
+    if (PRO != Pro::Quant) {
+        // rms_norm of x[K] in the reference's summation order (Act: x as it is), then block quantisation, once per workgroup: 8 lanes
         // share a block of 32, codes and scales go to LDS and every wave picks its fragment up from there
-        float* xs = shared_tail;                              // K floats
-        float* part = xs + K;                                 // 17 (32 reserved)
-        float* qsc = part + 32;                               // K/32 scales, as the f32 value of their fp16 rounding
+        float* xs = shared_tail;                              // K floats (RmsNorm only)
+        float* part = xs + K;                                 // 17 (32 reserved; RmsNorm only)
+        float* qsc = PRO == Pro::RmsNorm ? part + 32 : shared_tail;      // K/32 scales, as the f32 value of their fp16 rounding
         uint32_t* qcd = reinterpret_cast<uint32_t*>(qsc + ((nblk + 3u) & ~3u));   // K codes, 16-byte aligned
+        // (K / 4 is a multiple of 8 and so is THREADS: the 8 lanes of a block are in or out together)
+        auto quantise4 = [&](uint32_t e4, float4 v) {
+            uint16_t sb;
+            qcd[e4] = quantize_block_part(v, sb);
+            if ((e4 & 7u) == 0) qsc[e4 >> 3] = f16_bits_to_f32(sb);
+        };
+      if (PRO == Pro::RmsNorm) {
 #pragma unroll
         for (int i = 0; i < XE; i++) { const uint32_t e4 = i * THREADS + tid; if (e4 < K / 4) reinterpret_cast<float4*>(xs)[e4] = xe[i]; }
         for (uint32_t e4 = XE * THREADS + tid; e4 < K / 4; e4 += THREADS) reinterpret_cast<float4*>(xs)[e4] = reinterpret_cast<const float4*>(a.x)[e4];
@@ -224,16 +243,17 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_kernel(GemvArgs a) {
         }
         __syncthreads();
         const float inv_rms = 1.0f / sqrtf(part[16] / (float)K + a.eps);
-        auto quantise4 = [&](uint32_t e4, float4 xv, float4 w4) {
-            const float4 v = make_float4(xv.x * inv_rms * w4.x, xv.y * inv_rms * w4.y, xv.z * inv_rms * w4.z, xv.w * inv_rms * w4.w);
-            uint16_t sb;
-            qcd[e4] = quantize_block_part(v, sb);
-            if ((e4 & 7u) == 0) qsc[e4 >> 3] = f16_bits_to_f32(sb);
+        auto normed4 = [&](uint32_t e4, float4 xv, float4 w4) {
+            quantise4(e4, make_float4(xv.x * inv_rms * w4.x, xv.y * inv_rms * w4.y, xv.z * inv_rms * w4.z, xv.w * inv_rms * w4.w));
         };
-        // (K / 4 is a multiple of 8 and so is THREADS: the 8 lanes of a block are in or out together)
 #pragma unroll
-        for (int i = 0; i < XE; i++) { const uint32_t e4 = i * THREADS + tid; if (e4 < K / 4) quantise4(e4, reinterpret_cast<const float4*>(xs)[e4], we[i]); }
-        for (uint32_t e4 = XE * THREADS + tid; e4 < K / 4; e4 += THREADS) quantise4(e4, reinterpret_cast<const float4*>(xs)[e4], reinterpret_cast<const float4*>(a.norm_w)[e4]);
+        for (int i = 0; i < XE; i++) { const uint32_t e4 = i * THREADS + tid; if (e4 < K / 4) normed4(e4, reinterpret_cast<const float4*>(xs)[e4], we[i]); }
+        for (uint32_t e4 = XE * THREADS + tid; e4 < K / 4; e4 += THREADS) normed4(e4, reinterpret_cast<const float4*>(xs)[e4], reinterpret_cast<const float4*>(a.norm_w)[e4]);
+      } else {
+#pragma unroll
+        for (int i = 0; i < XE; i++) { const uint32_t e4 = i * THREADS + tid; if (e4 < K / 4) quantise4(e4, xe[i]); }
+        for (uint32_t e4 = XE * THREADS + tid; e4 < K / 4; e4 += THREADS) quantise4(e4, reinterpret_cast<const float4*>(a.x)[e4]);
+      }
         __syncthreads();
 #pragma unroll
         for (int j = 0; j < NL; j++) {
@@ -380,9 +400,10 @@ uint32_t rows_per_group(uint32_t nblk, uint32_t N, uint32_t rw) {
 }
 
 constexpr size_t LDS_LIMIT = 64 * 1024;
-size_t lds_tail_bytes(bool norm, bool silu, uint32_t K) {
-    // the norm prologue: x [K] f32, 32 words of partial sums, the scales [K/32] f32 (padded to 16 bytes), the codes [K]
-    size_t tail = norm ? (size_t)(K + 32 + ((K / 32 + 3) & ~3u)) * sizeof(float) + K : 0;
+size_t lds_tail_bytes(bool norm, bool silu, uint32_t K, bool act = false) {
+    // the norm prologue: x [K] f32, 32 words of partial sums, the scales [K/32] f32 (padded to 16 bytes), the codes [K];
+    // the quantising prologue: scales and codes
+    size_t tail = norm ? (size_t)(K + 32 + ((K / 32 + 3) & ~3u)) * sizeof(float) + K : act ? (size_t)((K / 32 + 3) & ~3u) * sizeof(float) + K : 0;
     if (silu && tail < 64 * sizeof(float)) tail = 64 * sizeof(float);
     return tail;
 }
@@ -391,7 +412,7 @@ template <bool Q4, int NCH, int RW, Pro PRO, Epi EPI, int KS = 1>
 void launch_one(GemvArgs a, hipStream_t s) {
     constexpr int WAVES = EPI == Epi::SiluQuant ? 16 : 4;      // waves that own row groups; the kernel runs WAVES * KS
     const uint32_t nblk = a.K / 32;
-    const size_t tail = lds_tail_bytes(PRO == Pro::RmsNorm, EPI == Epi::SiluQuant, a.K);
+    const size_t tail = lds_tail_bytes(PRO == Pro::RmsNorm, EPI == Epi::SiluQuant, a.K, PRO == Pro::Act);
     a.rc = EPI == Epi::SiluQuant ? 4 : rows_per_group(nblk, a.N, RW);
     // shrink the group if the products and the prologue's copy of x do not fit LDS together
     constexpr uint32_t step = RW < 2 ? 2 : RW;
@@ -474,6 +495,12 @@ void launch_gemv(const QWeight& w, const int8_t* aq, const uint16_t* as, float* 
     a.aq = aq; a.as = as; a.y = y;
     if (accumulate) dispatch<Pro::Quant, Epi::Add>(w.wdtype, a, s);
     else dispatch<Pro::Quant, Epi::Store>(w.wdtype, a, s);
+}
+
+void launch_gemv_act(const QWeight& w, const float* x, float* y, hipStream_t s) {
+    GemvArgs a = base_args(w, GemvOrder::MatmulVec);
+    a.x = x; a.y = y;
+    dispatch<Pro::Act, Epi::Store>(w.wdtype, a, s);
 }
 
 void launch_gemv_isums(const QWeight& w, const int8_t* aq, int32_t* out, hipStream_t s) {

@@ -35,7 +35,7 @@ __device__ __forceinline__ float pair_swap(float v) { return __builtin_amdgcn_up
 // (x - 32) for each of four 6-bit values held one per byte
 __device__ __forceinline__ int sub32x4(uint32_t x) { return (int)(((x | 0x80808080u) - 0x20202020u) ^ 0x80808080u); }
 
-constexpr int KQ_WAVES = 4;
+constexpr int KQ_WAVES = 4;                      // waves of a workgroup (the quantising form has eight for deep matrices)
 
 // What a lane holds of RW rows for one pass of 64 pieces: its 16 bytes of quants and the super-block's scales.
 template <bool Q6, int RW>
@@ -152,13 +152,13 @@ __device__ __forceinline__ void kq_products(const KqFrag<Q6, RW>& f, uint32_t ns
 // pass is requested before this one is multiplied).  The weights do not depend on the activations: the first pass is on its
 // way while `activations()` brings the codes, scales and (Q4_K) block sums into LDS.  Lane r adds row r's products in block
 // order.
-template <bool Q6, int RW, typename Activations>
+template <bool Q6, int RW, int W, typename Activations>
 __device__ __forceinline__ void kq_matrix(const uint8_t* __restrict__ qs, const uint8_t* __restrict__ meta, float* __restrict__ y, uint32_t K,
                                           uint32_t N, int accumulate, uint32_t blk, uint32_t nblks, const int8_t* xa, const float* xs,
                                           const float* xsum, float* prod, uint32_t lane, uint32_t wave, Activations&& activations) {
     const uint32_t nblk = K / 32, nsb = K / 256, pstride = prod_stride(nblk);
     const uint32_t pieces = nsb * 8;
-    const uint32_t first = (blk * KQ_WAVES + wave) * RW, step = nblks * KQ_WAVES * RW;
+    const uint32_t first = (blk * W + wave) * RW, step = nblks * W * RW;
     const uint32_t groups = first < N ? (N - first + step - 1) / step : 0u;
     const uint32_t total = groups * ((pieces + 63) / 64);
     KqFrag<Q6, RW> cur;
@@ -197,35 +197,67 @@ __device__ __forceinline__ void kq_load_activations(const int8_t* __restrict__ a
     __syncthreads();
 }
 
-// Where the quantised vector comes from.  Quantised: from memory.  RmsNorm: rms_norm(x) * norm_w, quantised by the workgroup
+// Where the quantised vector comes from.  Quantised: from memory.  Act: every workgroup quantises x for itself.  RmsNorm: rms_norm(x) * norm_w, quantised by the workgroup
 // itself (the arithmetic and the summation order of the stand-alone norm kernel: 16 strided partial sums, a fixed tree, then
 // one block of 32 per 8 lanes).
-enum class KqPro { Quantised, RmsNorm };
+enum class KqPro { Quantised, Act, RmsNorm };
 struct KqIn {
     const int8_t* aq;
     const uint16_t* as;
-    const float* x;          // RmsNorm: the residual row
+    const float* x;          // Act: the vector; RmsNorm: the residual row
     const float* w;          // RmsNorm: the norm weights
     float eps;
 };
 
+template <int W>
 __device__ __forceinline__ void kq_block_sums(uint32_t K, const int8_t* xa, float* xsum, uint32_t tid) {
-    for (uint32_t b = tid; b < K / 32; b += KQ_WAVES * 64) {
+    for (uint32_t b = tid; b < K / 32; b += W * 64) {
         const int4 ones = make_int4(0x01010101, 0x01010101, 0x01010101, 0x01010101);
         const int4 a0 = reinterpret_cast<const int4*>(xa + (size_t)b * 32)[0], a1 = reinterpret_cast<const int4*>(xa + (size_t)b * 32)[1];
         xsum[b] = (float)kq_dot16(ones, a1, kq_dot16(ones, a0, 0));
     }
 }
 
+// Act: the first KQ_XE float4 of a thread's share of x are requested ahead of the weights (loads return in issue order).
+constexpr int KQ_XE = 2;                        // K = 2048 at 256 threads
+struct KqAhead { float4 v[KQ_XE]; };
+template <KqPro PRO, int W>
+__device__ __forceinline__ KqAhead kq_request_x(const KqIn& in, uint32_t K, uint32_t tid) {
+    KqAhead p;
+#pragma unroll
+    for (int i = 0; i < KQ_XE; i++) {
+        const uint32_t e4 = i * W * 64 + tid;
+        p.v[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (PRO == KqPro::Act && e4 < K / 4) p.v[i] = reinterpret_cast<const float4*>(in.x)[e4];
+    }
+    return p;
+}
+
 // `tail`: K + 32 floats of LDS behind the products (RmsNorm only).
-template <KqPro PRO>
-__device__ __forceinline__ void kq_activations(const KqIn& in, uint32_t K, int8_t* xa, float* xs, float* xsum, float* tail, uint32_t tid) {
-    constexpr uint32_t THREADS = KQ_WAVES * 64;
+template <KqPro PRO, int W>
+__device__ __forceinline__ void kq_activations(const KqIn& in, uint32_t K, int8_t* xa, float* xs, float* xsum, float* tail, uint32_t tid, const KqAhead& ahead) {
+    constexpr uint32_t THREADS = W * 64;
     if (PRO == KqPro::Quantised) {
+        static_assert(PRO != KqPro::Quantised || W == KQ_WAVES, "kq_load_activations strides by KQ_WAVES");
         kq_load_activations(in.aq, in.as, K, xa, xs, xsum, tid);
         return;
     }
     uint32_t* codes = reinterpret_cast<uint32_t*>(xa);
+    // (K / 4 is a multiple of 8 and so is THREADS: the 8 lanes of a block are in or out together)
+    auto quantise4 = [&](uint32_t e4, float4 v) {
+        uint16_t sb;
+        codes[e4] = quantize_block_part(v, sb);
+        if ((e4 & 7u) == 0) xs[e4 >> 3] = f16_bits_to_f32(sb);
+    };
+    if (PRO == KqPro::Act) {
+#pragma unroll
+        for (int i = 0; i < KQ_XE; i++) { const uint32_t e4 = i * THREADS + tid; if (e4 < K / 4) quantise4(e4, ahead.v[i]); }
+        for (uint32_t e4 = KQ_XE * THREADS + tid; e4 < K / 4; e4 += THREADS) quantise4(e4, reinterpret_cast<const float4*>(in.x)[e4]);
+        __syncthreads();
+        kq_block_sums<W>(K, xa, xsum, tid);
+        __syncthreads();
+        return;
+    }
     float* xf = tail;
     float* part = tail + K;
     for (uint32_t e4 = tid; e4 < K / 4; e4 += THREADS) reinterpret_cast<float4*>(xf)[e4] = reinterpret_cast<const float4*>(in.x)[e4];
@@ -250,16 +282,12 @@ __device__ __forceinline__ void kq_activations(const KqIn& in, uint32_t K, int8_
     }
     __syncthreads();
     const float inv_rms = 1.0f / sqrtf(part[16] / (float)K + in.eps);
-    // (K / 4 is a multiple of 8 and so is THREADS: the 8 lanes of a block are in or out together)
     for (uint32_t e4 = tid; e4 < K / 4; e4 += THREADS) {
         const float4 xv = reinterpret_cast<const float4*>(xf)[e4], w4 = reinterpret_cast<const float4*>(in.w)[e4];
-        const float4 v = make_float4(xv.x * inv_rms * w4.x, xv.y * inv_rms * w4.y, xv.z * inv_rms * w4.z, xv.w * inv_rms * w4.w);
-        uint16_t sb;
-        codes[e4] = quantize_block_part(v, sb);
-        if ((e4 & 7u) == 0) xs[e4 >> 3] = f16_bits_to_f32(sb);
+        quantise4(e4, make_float4(xv.x * inv_rms * w4.x, xv.y * inv_rms * w4.y, xv.z * inv_rms * w4.z, xv.w * inv_rms * w4.w));
     }
     __syncthreads();
-    kq_block_sums(K, xa, xsum, tid);
+    kq_block_sums<W>(K, xa, xsum, tid);
     __syncthreads();
 }
 
@@ -267,8 +295,8 @@ __device__ __forceinline__ void kq_activations(const KqIn& in, uint32_t K, int8_
 // [RW][prod_stride(K/32)] (and the norm prologue's K + 32 floats).  A wave works RW rows at a time: all their loads are issued
 // before the first is used (one row of K = 2048 is a single kilobyte, far too little in flight for HBM), and lane r adds row
 // r's products in block order.
-template <bool Q6, int RW, KqPro PRO>
-__global__ __launch_bounds__(KQ_WAVES * 64) void gemv_kquant_kernel(const uint8_t* __restrict__ qs, const uint8_t* __restrict__ meta, KqIn in,
+template <bool Q6, int RW, KqPro PRO, int W = KQ_WAVES>
+__global__ __launch_bounds__(W * 64) void gemv_kquant_kernel(const uint8_t* __restrict__ qs, const uint8_t* __restrict__ meta, KqIn in,
                                                                   float* __restrict__ y, uint32_t K, uint32_t N, int accumulate) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -277,8 +305,9 @@ __global__ __launch_bounds__(KQ_WAVES * 64) void gemv_kquant_kernel(const uint8_
     float* xs = reinterpret_cast<float*>(lds + K);
     float* xsum = xs + nblk;
     float* prod = xsum + nblk + (size_t)wave * RW * pstride;
-    auto act = [&]() { kq_activations<PRO>(in, K, xa, xs, xsum, xsum + nblk + (size_t)KQ_WAVES * RW * pstride, tid); };
-    kq_matrix<Q6, RW>(qs, meta, y, K, N, accumulate, blockIdx.x, gridDim.x, xa, xs, xsum, prod, lane, wave, act);
+    const KqAhead ahead = kq_request_x<PRO, W>(in, K, tid);
+    auto act = [&]() { kq_activations<PRO, W>(in, K, xa, xs, xsum, xsum + nblk + (size_t)W * RW * pstride, tid, ahead); };
+    kq_matrix<Q6, RW, W>(qs, meta, y, K, N, accumulate, blockIdx.x, gridDim.x, xa, xs, xsum, prod, lane, wave, act);
 }
 
 // Up to three matrices that multiply the SAME vector (q, k, v; gate, up) in one launch: a workgroup belongs to one of them.
@@ -301,12 +330,13 @@ __global__ __launch_bounds__(KQ_WAVES * 64) void gemv_kquant_multi_kernel(KqMult
     float* xs = reinterpret_cast<float*>(lds + K);
     float* xsum = xs + nblk;
     float* prod = xsum + nblk + (size_t)wave * RW * pstride;
-    auto act = [&]() { kq_activations<PRO>(in, K, xa, xs, xsum, xsum + nblk + (size_t)KQ_WAVES * RW * pstride, tid); };
+    const KqAhead ahead = kq_request_x<PRO, KQ_WAVES>(in, K, tid);
+    auto act = [&]() { kq_activations<PRO, KQ_WAVES>(in, K, xa, xs, xsum, xsum + nblk + (size_t)KQ_WAVES * RW * pstride, tid, ahead); };
     uint32_t i = 0;
     while (i + 1 < a.n && blockIdx.x >= a.m[i + 1].blk0) i++;
     const KqMat mt = a.m[i];
-    if (mt.q6) kq_matrix<true, RW>(mt.qs, mt.meta, mt.y, K, mt.N, accumulate, blockIdx.x - mt.blk0, mt.nblks, xa, xs, xsum, prod, lane, wave, act);
-    else kq_matrix<false, RW>(mt.qs, mt.meta, mt.y, K, mt.N, accumulate, blockIdx.x - mt.blk0, mt.nblks, xa, xs, xsum, prod, lane, wave, act);
+    if (mt.q6) kq_matrix<true, RW, KQ_WAVES>(mt.qs, mt.meta, mt.y, K, mt.N, accumulate, blockIdx.x - mt.blk0, mt.nblks, xa, xs, xsum, prod, lane, wave, act);
+    else kq_matrix<false, RW, KQ_WAVES>(mt.qs, mt.meta, mt.y, K, mt.N, accumulate, blockIdx.x - mt.blk0, mt.nblks, xa, xs, xsum, prod, lane, wave, act);
 }
 
 // The same matmul for MB rows of activations at once (a prompt through a model with K-quant projections): a workgroup holds
@@ -504,18 +534,18 @@ void repack_kquant_host(uint32_t wdtype, const uint8_t* raw, uint32_t K, uint64_
 bool kquant_k_supported(uint32_t K) { return K >= 256 && K % 256 == 0 && K <= 16384; }
 
 namespace {
-template <KqPro PRO>
+template <KqPro PRO, int W = KQ_WAVES>
 void launch_kq_one(const QWeight& w, const KqIn& in, float* y, bool accumulate, hipStream_t s) {
     if (w.N == 0) return;
     const uint32_t nblk = w.K / 32;
     // rows a wave keeps in flight: four when that still leaves every CU several workgroups
     const int rw = w.N >= 16384 ? 4 : w.N >= 4096 ? 2 : 1;
-    const size_t lds = (size_t)w.K + (size_t)nblk * 8 + (size_t)KQ_WAVES * rw * prod_stride(nblk) * 4;
-    uint32_t grid = (w.N + KQ_WAVES * rw - 1) / (KQ_WAVES * rw);
+    const size_t lds = (size_t)w.K + (size_t)nblk * 8 + (size_t)W * rw * prod_stride(nblk) * 4;
+    uint32_t grid = (w.N + W * rw - 1) / (W * rw);
     if (grid > 256 * 8) grid = 256 * 8;
     const uint8_t* meta = reinterpret_cast<const uint8_t*>(w.scales);
     const int acc = accumulate ? 1 : 0;
-#define FH_KQ(Q6_, RW_) fh::launch(gemv_kquant_kernel<Q6_, RW_, PRO>, grid, KQ_WAVES * 64, lds, s, w.qs, meta, in, y, w.K, w.N, acc)
+#define FH_KQ(Q6_, RW_) fh::launch(gemv_kquant_kernel<Q6_, RW_, PRO, W>, grid, W * 64, lds, s, w.qs, meta, in, y, w.K, w.N, acc)
     if (w.wdtype == FORGE_HIP_Q6_K) { if (rw == 4) FH_KQ(true, 4); else if (rw == 2) FH_KQ(true, 2); else FH_KQ(true, 1); }
     else { if (rw == 4) FH_KQ(false, 4); else if (rw == 2) FH_KQ(false, 2); else FH_KQ(false, 1); }
 #undef FH_KQ
@@ -548,6 +578,14 @@ void launch_kq_multi(const QWeight* const* w, float* const* y, uint32_t n, const
 
 void launch_gemv_kquant(const QWeight& w, const int8_t* aq, const uint16_t* as, float* y, bool accumulate, hipStream_t s) {
     launch_kq_one<KqPro::Quantised>(w, KqIn{aq, as, nullptr, nullptr, 0.f}, y, accumulate, s);
+}
+
+// The product with quantise(x), quantised by every workgroup for itself: no launch in front, the same bits.
+void launch_gemv_kquant_act(const QWeight& w, const float* x, float* y, hipStream_t s) {
+    const KqIn in{nullptr, nullptr, x, nullptr, 0.f};
+    // a deep vector is quantised by eight waves in half as many workgroups (8192 -> 2048, Q4_K: 8.7 against 7.4 us with four)
+    if (w.K > 2048) launch_kq_one<KqPro::Act, 8>(w, in, y, false, s);
+    else launch_kq_one<KqPro::Act>(w, in, y, false, s);
 }
 
 // Up to three K-quant matrices over the same quantised vector in ONE launch (same K; each y[i] has N_i floats).  Every row has

@@ -238,6 +238,29 @@ def test_matmul_mat_parity(fh, oracle, torch_gpu, wd, M, K, N):
     close(fh.ops.matmul_mat_q(w, xd, 0).cpu().numpy(), want)
 
 
+@pytest.mark.parametrize("ty", [Q8, Q4, 12, 14])
+@pytest.mark.parametrize("K,N", [(256, 7), (2048, 33), (2304, 64), (8192, 130), (16384, 5)])
+def test_matmul_vec_quantises_like_the_quantiser(fh, torch_gpu, ty, K, N):
+    """The vector product quantises its vector itself: block by block the codes and scales of the stand-alone quantiser, for zero
+    blocks, tiny and huge blocks and NaN too (the rows product takes the quantiser's own codes)."""
+    torch = torch_gpu
+    raw = make_weight(fh, ty, N, K, K + N) if ty in (Q8, Q4) else random_superblocks(ty, N * (K // 256), K + N)
+    w = fh.ops.QWeight(ty, raw, K, N)
+    x = fh.synth.normal(K, K, 1.0)
+    x[:32] = 0.0
+    x[32:64] *= np.float32(1e-30)
+    x[64:96] *= np.float32(1e6)
+    for last in (x[-1], np.float32("nan")):
+        x[-1] = last
+        xd = torch.from_numpy(x).cuda()
+        one, rows = fh.ops.matmul_vec_q(w, xd).cpu().numpy(), fh.ops.matmul_mat_q(w, xd[None], EXACT).cpu().numpy()[0]
+        assert np.array_equal(np.isnan(one), np.isnan(rows))
+        if ty in (12, 14):                                    # (Q8_0 / Q4_0 tail rows: the two have orders of their own)
+            same_bits(one[~np.isnan(one)], rows[~np.isnan(rows)])
+        else:
+            close(one, rows, 1e-4, 1e-4 * float(np.abs(x[64:96]).max()))
+
+
 @pytest.mark.parametrize("wd", [Q8, Q4])
 @pytest.mark.parametrize("M,K,N", [(2502, 2048, 2048), (2502, 8192, 2048), (2100, 1152, 3072), (2502, 576, 2176)])
 def test_matmul_mat_k_ranges_of_leftover_tiles(fh, torch_gpu, wd, M, K, N):
