@@ -201,6 +201,11 @@ bool gemm_silu_supported(const QWeight& w, uint32_t inter, uint32_t M);
 void launch_gemm(const QWeight& w, const int8_t* aq, const uint16_t* as, uint32_t M, float* y, uint32_t ldy,
                  bool accumulate, bool exact, int32_t* isums, hipStream_t s, void* split_ws = nullptr, int8_t* silu_q = nullptr,
                  uint16_t* silu_sc = nullptr, const float* mt_a = nullptr, const float* mt_w = nullptr);
+// gemm_rows.hip -- the fast mode's product for few rows (the arguments of launch_gemm): launch_gemm goes there itself
+bool gemm_rows_supported(const QWeight& w, uint32_t M, bool silu);
+double gemm_rows_cost(const QWeight& w, uint32_t M);
+void launch_gemm_rows(const QWeight& w, const int8_t* aq, const uint16_t* as, uint32_t M, float* y, uint32_t ldy, bool accumulate, hipStream_t s,
+                      int8_t* silu_q, uint16_t* silu_sc);
 
 // llama.hip — the part of forge_hip_model_create's checks that sizes depend on (formats, dimensions the kernels cover);
 // sets the error message.

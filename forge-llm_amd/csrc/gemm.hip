@@ -672,7 +672,7 @@ void launch_gemm(const QWeight& w, const int8_t* aq, const uint16_t* as, uint32_
             // stage of a workgroup that has a CU to itself, measured: 1.3 for a 128-row tile, 1.1 for a 64-row one).
             GemmSplit fsp{};
             uint32_t items = 0;
-            if (split_ws && !exact && !isums && mc == M && nc == w.N) {
+            if (!exact && !isums && mc == M && nc == w.N) {
                 struct Plan { int tm; GemmSplit sp; uint32_t items; double cost; };
                 const uint32_t stages = (w.K + BK - 1) / BK;
                 auto plan = [&](int tm_) {
@@ -680,7 +680,7 @@ void launch_gemm(const QWeight& w, const int8_t* aq, const uint16_t* as, uint32_
                     const double t_stage = tm_ == 1 ? 1.1 : 1.3;
                     Plan p{tm_, GemmSplit{}, 0, (double)((tiles + cus - 1) / cus) * stages * t_stage};   // items 0: not cut
                     const uint32_t rem = tiles % (uint32_t)cus;
-                    const uint32_t split = rem ? std::min<uint32_t>({(uint32_t)cus / rem, 8u, stages / 2, GEMM_SPLIT_MAX_ITEMS / rem}) : 0;
+                    const uint32_t split = rem && split_ws ? std::min<uint32_t>({(uint32_t)cus / rem, 8u, stages / 2, GEMM_SPLIT_MAX_ITEMS / rem}) : 0;
                     if (tiles / (uint32_t)cus < 4 && split >= 2) {
                         GemmSplit sp{};
                         sp.stages_per_part = ((stages + split - 1) / split + 1) & ~1u;
@@ -698,6 +698,13 @@ void launch_gemm(const QWeight& w, const int8_t* aq, const uint16_t* as, uint32_
                 };
                 Plan best = plan(tm);
                 if (tm == 1) { const Plan other = plan(2); if (other.cost < best.cost) best = other; }
+                // Few rows: the kernel without stages (gemm_rows.hip) where its own estimate is lower.  The SiLU epilogue costs a tile
+                // here about 7 us more than the plan counts (64 rows of 2048 -> 16384: 29.5 us, 20.8 planned); the other kernel has the
+                // extra f32 term (MINT) not at all.
+                if (!mt_a && gemm_rows_supported(w, M, silu) && gemm_rows_cost(w, M) < best.cost + (silu ? 7.0 : 0.0)) {
+                    launch_gemm_rows(w, aq, as, M, y, ldy, accumulate, s, silu_q, silu_sc);
+                    return;
+                }
                 tm = best.tm;
                 if (best.items) { fsp = best.sp; items = best.items; }
             }

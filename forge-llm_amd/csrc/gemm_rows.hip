@@ -1,0 +1,262 @@
+// Quantised matmul for a few rows of activations (matmul_mat_q8_0_KxN / matmul_mat_q4_0_KxN, emit.rs:2108-2302, 3667-3817), fast
+// mode: what a short prompt, or a handful of sequences side by side, multiplies.
+//
+// What bounds it: the weights' way from memory (each byte is used for a few rows only) and latency.  The tile kernel (gemm.hip) walks
+// the whole of K in one workgroup of 128 columns, about 1.1 us per 128-deep stage however few rows there are, on N / 128 workgroups.
+// Here a workgroup takes a 32 x 32 tile (two with the SiLU epilogue) and its waves share out K, each through a strip of LDS of its own:
+// no barrier until the waves' partial tiles meet at the end, where they are added in the order of K.
+// Block sums are exact (v_mfma_i32_32x32x32_i8, one quant block per instruction); the scales' products come from a rank-1
+// v_mfma_f32_32x32x8_f16, exact in f32.  Up to a depth of 4096 a block's sum is converted and added with one FMA: an error of 2e-7 of the
+// typical output, and with so few rows no slower than the tile kernel's biased sums (2e-5).  Deeper sums are biased (BIASED): there
+// that kernel's own rounding reaches 1e-4 of a result, and a row would differ by all of it between a small and a large batch.
+// 32 rows of 2048 -> 8192: 6.2 us (2.7 TB/s of weights) against the tile kernel's 22; 8192 -> 2048: 12.5 against 76 (22 with K ranges);
+// [gate; up] with its epilogue, 2048 -> 16384: 10.5 against 29.5.  Operands fetched straight into registers took 10 and 31 us.
+#include <algorithm>
+
+#include "common.h"
+#include "device_utils.h"
+
+namespace fh {
+
+namespace {
+
+typedef int v4i __attribute__((ext_vector_type(4)));
+typedef int v16i __attribute__((ext_vector_type(16)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef _Float16 v4h __attribute__((ext_vector_type(4)));
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+
+constexpr int FR_U = 4;                      // blocks of a step: 128 bytes of a Q8_0 or activation row, 64 of a Q4_0 row
+constexpr uint32_t FR_RSRC = 0x00020000;     // raw buffer, 32-bit data format
+constexpr uint32_t FR_MAGIC = 0x4B400000u;   // 12582912.0f: the bias that makes a block sum a float (gemm.hip)
+constexpr int FR_A_LOG2 = 8;                 // its removal: activation scales times 2^8, weight scales times 2^15 and 2^14
+
+struct FewArgs {
+    const uint8_t* wq;
+    const uint16_t* wsc;
+    const int8_t* aq;            // odd blocks negated, as for the tile kernel
+    const uint16_t* asc;
+    float* y;
+    uint32_t M, N, K, ldy, accumulate;
+    int8_t* silu_q;              // SILU: [M][inter] codes (odd blocks negated), [M][inter / 32] scales
+    uint16_t* silu_sc;
+    uint32_t inter;
+};
+
+// One workgroup: 32 rows of activations x 32 columns.  SILU: the matrix is [gate; up], a workgroup takes 32 gate columns and the up
+// columns of the same indices and writes quantize(silu(gate) * up) as gemm.hip's epilogue does.
+template <bool Q4, int WAVES, bool SILU, bool BIASED>
+__global__ __launch_bounds__(WAVES * 64) void gemm_rows_kernel(FewArgs a) {
+    constexpr int NT = SILU ? 2 : 1, KW = WAVES / NT;         // column tiles; waves that share K of one
+    constexpr int THREADS = WAVES * 64, TILE = 1024;
+    constexpr int WB = Q4 ? 64 : 128;                         // bytes of a weight row in a step
+    constexpr int LA = 32 * 128, LB = 32 * WB;                // LDS bytes of a step's activation tile / weight tile
+    constexpr int WAVE_LDS = LA + LB;
+    static_assert(WAVE_LDS >= TILE * 4, "a wave's strip holds its partial tile");
+    __shared__ __attribute__((aligned(16))) uint8_t lds[WAVES * WAVE_LDS];
+    const uint32_t tid = threadIdx.x, lane = tid & 63;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+    const uint32_t c = lane & 31, h = lane >> 5;
+    const uint32_t nblk = a.K / 32, n0 = blockIdx.x * 32, m0 = blockIdx.y * 32;
+    const uint32_t steps = (nblk + FR_U - 1) / FR_U, each = (steps + KW - 1) / KW, per = BIASED ? (each + 1) & ~1u : each;
+    const uint32_t s0 = min(steps, wave % KW * per), s1 = min(steps, s0 + per);
+    const uint32_t col0 = n0 + (SILU ? wave / KW * a.inter : 0u);        // this wave's columns: rows col0 .. + 32 of the matrix
+    uint8_t* la = lds + wave * WAVE_LDS;                      // this wave's own: no barrier until the partial tiles meet
+    uint8_t* lb = la + LA;
+
+    // A wave fetches whole 128-byte (Q4_0: 64-byte) pieces of its rows, eight (four) lanes to a row, and leaves them in its strip of
+    // LDS, 16-byte pieces XOR-swizzled by the row; the MFMA operands (one 16-byte piece per lane: row c, half h of a block) come from
+    // there.  Fetching the operands directly touches 32 cache lines per instruction, for the scales as well: the vector memory pipe
+    // then took longer than the weights' way from memory.  Rows past the end and bytes past the last row read as zero.
+    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void*)a.wq, 0, a.N * nblk * (Q4 ? 16 : 32), FR_RSRC);
+    const __amdgpu_buffer_rsrc_t rws = __builtin_amdgcn_make_buffer_rsrc((void*)a.wsc, 0, a.N * nblk * 2, FR_RSRC);
+    const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)a.aq, 0, a.M * a.K, FR_RSRC);
+    const __amdgpu_buffer_rsrc_t ras = __builtin_amdgcn_make_buffer_rsrc((void*)a.asc, 0, a.M * nblk * 2, FR_RSRC);
+    constexpr int NLA = 4, NLB = Q4 ? 2 : 4;                  // loads of a step per tile: 8 rows (Q4_0 weights: 16) each
+    const uint32_t ar = lane >> 3, ap = lane & 7;
+    const uint32_t br = Q4 ? lane >> 2 : lane >> 3, bp = Q4 ? lane & 3 : lane & 7;
+    struct Step { v4i A[NLA], B[NLB]; uint2 sa, sb; };
+    // A row's four scales.  An even number of blocks to a row keeps them on 4-byte boundaries and the matrix's end on one; otherwise they
+    // are fetched one by one (a word that reaches past the end reads as zero altogether).
+    const bool odd_row = (nblk & 1u) != 0;
+    auto load_scales = [&](const __amdgpu_buffer_rsrc_t& rsrc, uint32_t at) {
+        if (!odd_row) return __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(rsrc, at, 0, 0));
+        uint32_t v[FR_U];
+#pragma unroll
+        for (int u = 0; u < FR_U; u++) v[u] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(rsrc, at + 2 * u, 0, 0) & 0xFFFFu;
+        return make_uint2(v[0] | (v[1] << 16), v[2] | (v[3] << 16));
+    };
+    auto load = [&](Step& g, uint32_t st) {
+#pragma unroll
+        for (int i = 0; i < NLB; i++)
+            g.B[i] = __builtin_amdgcn_raw_buffer_load_b128(rw, (col0 + i * (Q4 ? 16 : 8) + br) * nblk * (Q4 ? 16 : 32) + st * WB + bp * 16, 0, 0);
+        g.sb = load_scales(rws, (col0 + c) * nblk * 2 + st * 8);
+#pragma unroll
+        for (int i = 0; i < NLA; i++) g.A[i] = __builtin_amdgcn_raw_buffer_load_b128(ra, (m0 + i * 8 + ar) * a.K + st * 128 + ap * 16, 0, 0);
+        g.sa = load_scales(ras, (m0 + c) * nblk * 2 + st * 8);
+    };
+
+    float acc[16];
+#pragma unroll
+    for (int r = 0; r < 16; r++) acc[r] = 0.f;
+    v16i c_in;
+#pragma unroll
+    for (int r = 0; r < 16; r++) c_in[r] = BIASED ? (int)FR_MAGIC : 0;
+    const v16f zero_f = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    // operand of the rank-1 product: the scale in k = 0 (the lower half-wave's first element), zeros elsewhere
+    auto scale_operand = [&](uint32_t bits) {
+        const _Float16 z = (_Float16)0.0f;
+        return (v4h){__builtin_bit_cast(_Float16, (uint16_t)(h ? 0u : bits)), z, z, z};
+    };
+    auto scale_of = [](const uint2& v, int u) { return (u < 2 ? v.x : v.y) >> (16 * (u & 1)); };
+    // the scales of a step as they count: 0 past the end of K (those are the next row's), a minus sign on the weights' odd blocks
+    auto valid_scales = [&](uint2 v, uint32_t st, bool weights) {
+        const uint32_t left = st * FR_U < nblk ? nblk - st * FR_U : 0u;
+        v.x = left > 1 ? v.x : left ? v.x & 0xFFFFu : 0u;
+        v.y = left > 3 ? v.y : left > 2 ? v.y & 0xFFFFu : 0u;
+        if (weights) { v.x ^= 0x80000000u; v.y ^= 0x80000000u; }
+        return v;
+    };
+
+    auto compute = [&](Step& g, uint32_t st) {
+        g.sa = valid_scales(g.sa, st, false);
+        g.sb = valid_scales(g.sb, st, true);
+#pragma unroll
+        for (int i = 0; i < NLA; i++) {
+            const uint32_t row = i * 8 + ar;
+            *reinterpret_cast<v4i*>(la + row * 128 + ((ap ^ ((row >> 1) & 7)) * 16)) = g.A[i];
+        }
+#pragma unroll
+        for (int i = 0; i < NLB; i++) {
+            const uint32_t row = i * (Q4 ? 16 : 8) + br;
+            *reinterpret_cast<v4i*>(lb + row * WB + ((bp ^ (Q4 ? (row >> 2) & 3 : (row >> 1) & 7)) * 16)) = g.B[i];
+        }
+#pragma unroll
+        for (int u = 0; u < FR_U; u++) {
+            const v4i A = *reinterpret_cast<const v4i*>(la + c * 128 + (((2 * u + h) ^ ((c >> 1) & 7)) * 16));
+            const v4h fa = scale_operand(scale_of(g.sa, u));
+            v4i B;
+            if (Q4) {
+                const v4i p = *reinterpret_cast<const v4i*>(lb + c * WB + ((u ^ ((c >> 2) & 3)) * 16));
+                // elements 0..15 in the low nibbles, 16..31 in the high ones, as 16 (code - 8): the sum is divided by 16 at the end
+                const uint32_t sh = h ? 0u : 4u;
+#pragma unroll
+                for (int i = 0; i < 4; i++) B[i] = (int)((((uint32_t)p[i] << sh) & 0xF0F0F0F0u) ^ 0x80808080u);
+            } else {
+                B = *reinterpret_cast<const v4i*>(lb + c * WB + (((2 * u + h) ^ ((c >> 1) & 7)) * 16));
+            }
+            const v4h fb = scale_operand(scale_of(g.sb, u));
+            const v16i isum = __builtin_amdgcn_mfma_i32_32x32x32_i8(A, B, c_in, 0, 0, 0);
+            const v16f S = __builtin_amdgcn_mfma_f32_32x32x8f16(fa, fb, zero_f, 0, 0, 0);
+            const v16f biased = __builtin_bit_cast(v16f, isum);          // 12582912 +- block sum
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[r] = fmaf(S[r], BIASED ? biased[r] : (float)isum[r], acc[r]);
+        }
+        // the sums are final here: left alone, the compiler works on two steps' products at once and has no registers for them
+#pragma unroll
+        for (int r = 0; r < 16; r++) asm volatile("" : "+v"(acc[r]));
+    };
+    // What eight blocks left of the bias, 1.5 * 2^23 * sum_b a_s[b] * (+-w_s[b]), off the sums: gemm.hip's f16 MFMA over the same eight
+    // blocks (most of the biased sums' rounding is made here, and the same eight blocks make the same).
+    auto unbias = [&](uint2 a0, uint2 a1, uint2 w0, uint2 w1) {
+        const _Float16 af = (_Float16)(float)(1 << FR_A_LOG2);
+        const _Float16 bf = h ? (_Float16)(-(float)(1 << (22 - FR_A_LOG2))) : (_Float16)(-(float)(1 << (23 - FR_A_LOG2)));
+        const v8h ta = __builtin_bit_cast(v8h, make_uint4(a0.x, a0.y, a1.x, a1.y)) * (v8h){af, af, af, af, af, af, af, af};
+        const v8h tb = __builtin_bit_cast(v8h, make_uint4(w0.x, w0.y, w1.x, w1.y)) * (v8h){bf, bf, bf, bf, bf, bf, bf, bf};
+        v16f d;
+#pragma unroll
+        for (int r = 0; r < 16; r++) d[r] = acc[r];
+        d = __builtin_amdgcn_mfma_f32_32x32x16_f16(ta, tb, d, 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[r] = d[r];
+    };
+    // two steps in flight
+    Step x0, x1;
+    if (s0 < s1) load(x0, s0);
+    if (s0 + 1 < s1) load(x1, s0 + 1);
+    for (uint32_t st = s0; st < s1; st += 2) {
+        compute(x0, st);
+        const uint2 a0 = x0.sa, w0 = x0.sb;
+        uint2 a1 = make_uint2(0u, 0u), w1 = a1;
+        if (st + 2 < s1) load(x0, st + 2);
+        if (st + 1 < s1) {
+            compute(x1, st + 1);
+            a1 = x1.sa; w1 = x1.sb;
+        }
+        if (st + 3 < s1) load(x1, st + 3);
+        if (BIASED) unbias(a0, a1, w0, w1);
+    }
+
+    // lane: column c, rows 8 (r / 4) + 4 h + r % 4 of the tile.  Element e = r * 64 + lane of a partial tile; the waves' partial tiles are
+    // added in the order of K.
+    float* red = reinterpret_cast<float*>(la);
+#pragma unroll
+    for (int r = 0; r < 16; r++) red[r * 64 + lane] = acc[r];
+    __syncthreads();
+    for (uint32_t e = tid; e < TILE; e += THREADS) {
+        float v[NT];
+#pragma unroll
+        for (int j = 0; j < NT; j++) {
+            float p[KW];
+#pragma unroll
+            for (int w = 0; w < KW; w++) p[w] = reinterpret_cast<const float*>(lds + (j * KW + w) * WAVE_LDS)[e];
+            v[j] = p[0];
+#pragma unroll
+            for (int w = 1; w < KW; w++) v[j] = v[j] + p[w];
+            if (Q4) v[j] *= 0.0625f;
+        }
+        const uint32_t r = e >> 6, el = e & 63, col = el & 31;
+        const uint32_t m = m0 + 8 * (r >> 2) + 4 * (el >> 5) + (r & 3);
+        if (SILU) {
+            // gemm.hip's epilogue: the 32 lanes of a half-wave are one block of one row
+            const float o = v[0] * __builtin_amdgcn_rcpf(1.0f + __expf(-v[0])) * v[NT - 1];
+            const float amax = half_wave_max(fabsf(o));
+            const float scl = amax * (1.0f / 127.0f);
+            float inv = amax > 0.f ? 127.0f * __builtin_amdgcn_rcpf(amax) : 0.f;
+            if (blockIdx.x & 1u) inv = -inv;
+            const uint32_t code = (uint32_t)(int)__builtin_rintf(o * inv) & 0xFFu;
+            const uint32_t pk = quad_broadcast<0>(code) | (quad_broadcast<1>(code) << 8) | (quad_broadcast<2>(code) << 16) | (quad_broadcast<3>(code) << 24);
+            if (m < a.M) {
+                if ((col & 3u) == 0) *reinterpret_cast<uint32_t*>(a.silu_q + (size_t)m * a.inter + n0 + col) = pk;
+                if (col == 0) a.silu_sc[(size_t)m * (a.inter / 32) + blockIdx.x] = f32_to_f16_bits(scl);
+            }
+        } else if (m < a.M && n0 + col < a.N) {
+            float* dst = a.y + (size_t)m * a.ldy + n0 + col;
+            *dst = a.accumulate ? *dst + v[0] : v[0];
+        }
+    }
+}
+
+template <bool Q4, bool SILU>
+void launch_rows(const FewArgs& a, hipStream_t s) {
+    constexpr int WAVES = 8;       // sixteen leave a wave 128 registers, and two steps in flight do not fit them
+    const dim3 grid(((SILU ? a.inter : a.N) + 31) / 32, (a.M + 31) / 32);
+    if (a.K > 4096) fh::launch(gemm_rows_kernel<Q4, WAVES, SILU, true>, grid, WAVES * 64, 0, s, a);
+    else fh::launch(gemm_rows_kernel<Q4, WAVES, SILU, false>, grid, WAVES * 64, 0, s, a);
+}
+
+}  // namespace
+
+bool gemm_rows_supported(const QWeight& w, uint32_t M, bool silu) {
+    return (!silu || w.N % 64 == 0) && (uint64_t)M * w.K <= 0x7FFFFFFFull && (uint64_t)w.N * std::max<uint64_t>(w.qs_row_bytes(), w.K / 16) <= 0x7FFFFFFFull;
+}
+
+// Microseconds of a launch, for the choice between the kernels: 2.9 plus 2.9 per 2048 of depth while the tiles find a CU each (5.6 us
+// measured for 32 rows of 2048 -> 2048, 12.5 for 8192 -> 2048), then 0.0148 per tile and 2048 of depth (2048 -> 8192: 10.3 us for 64
+// rows, 18.9 for 128, 31 for 200).  A SiLU workgroup works two tiles.
+double gemm_rows_cost(const QWeight& w, uint32_t M) {
+    const double depth = w.K / 2048.0, tiles = (double)((w.N + 31) / 32) * ((M + 31) / 32);
+    return 2.9 + depth * (2.9 + 0.0148 * std::max(0.0, tiles - 256.0));
+}
+
+void launch_gemm_rows(const QWeight& w, const int8_t* aq, const uint16_t* as, uint32_t M, float* y, uint32_t ldy, bool accumulate, hipStream_t s,
+                      int8_t* silu_q, uint16_t* silu_sc) {
+    const FewArgs a{w.qs, w.scales, aq, as, y, M, w.N, w.K, ldy, accumulate ? 1u : 0u, silu_q, silu_sc, w.N / 2};
+    const bool q4 = w.wdtype == FORGE_HIP_Q4_0, silu = silu_q != nullptr;
+    if (q4 && silu) launch_rows<true, true>(a, s);
+    else if (q4) launch_rows<true, false>(a, s);
+    else if (silu) launch_rows<false, true>(a, s);
+    else launch_rows<false, false>(a, s);
+}
+
+}  // namespace fh

@@ -238,6 +238,29 @@ def test_matmul_mat_parity(fh, oracle, torch_gpu, wd, M, K, N):
     close(fh.ops.matmul_mat_q(w, xd, 0).cpu().numpy(), want)
 
 
+@pytest.mark.parametrize("wd", [Q8, Q4])
+@pytest.mark.parametrize("M,K,N", [(1, 288, 5), (2, 416, 32), (31, 544, 33), (32, 576, 64), (33, 2048, 100), (64, 1120, 31), (70, 4096, 512), (33, 4128, 40), (5, 8192, 96)])
+def test_matmul_mat_few_rows(fh, torch_gpu, wd, M, K, N):
+    """Few rows (32 x 32 tiles, K shared out to the waves): edges of the tiles, depths that are no multiple of a step or of the
+    waves, against the order-faithful product.  Both add the same exact block terms t_b; sums of n terms differ by at most
+    2 n 2^-24 sum |t_b| (one rounding per multiply and add).  Beyond a depth of 4096 a term is added as S (12582912 +- isum) and
+    the bias taken off again: three roundings per block of at most 2^-24 S 13.1e6."""
+    torch = torch_gpu
+    raw = make_weight(fh, wd, N, K, 11 * K + N)
+    w = fh.ops.QWeight(wd, raw, K, N)
+    x = torch.from_numpy(fh.synth.normal(M + K, M * K, 1.0).reshape(M, K)).cuda()
+    fast, exact = fh.ops.matmul_mat_q(w, x), fh.ops.matmul_mat_q(w, x, EXACT)
+    nblk = K // 32
+    a_s = fh.ops.quantize_act(x)[1].cpu().numpy().view(np.float16).astype(np.float64)
+    w_s = raw.reshape(N, nblk, -1)[:, :, :2].copy().view(np.float16)[:, :, 0].astype(np.float64)
+    terms = np.abs(a_s[:, None] * w_s[None] * fh.ops.block_isums(w, x, 0).cpu().numpy()).sum(-1)
+    bound = 2.0 * (nblk + 2) * 2.0 ** -24 * terms
+    if K > 4096:
+        bound += 3.0 * 2.0 ** -24 * 13.1e6 * (a_s @ w_s.T)
+    assert (np.abs(fast.cpu().numpy().astype(np.float64) - exact.cpu().numpy()) <= bound).all()
+    same_bits(fh.ops.matmul_mat_q(w, x).cpu().numpy(), fast.cpu().numpy())
+
+
 @pytest.mark.parametrize("ty", [Q8, Q4, 12, 14])
 @pytest.mark.parametrize("K,N", [(256, 7), (2048, 33), (2304, 64), (8192, 130), (16384, 5)])
 def test_matmul_vec_quantises_like_the_quantiser(fh, torch_gpu, ty, K, N):
