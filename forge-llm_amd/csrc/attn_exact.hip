@@ -501,6 +501,135 @@ __global__ __launch_bounds__(HD <= 64 ? 64 : 128) void attn_exact_decode_chain_k
     }
 }
 
+// The same steps for a short context in ONE launch: a workgroup per head, each of its waves one 64-key block (lane = key for the scores,
+// lane = head dim for sum[d]); maxima, weights and block records meet in LDS.  What bounds a short context is the launches: the three
+// take 8.2 us over 33 rows (9 heads of 64), this one 5.4.  What bounds this one is the compute unit that fetches a head's rows alone, so
+// it loses beyond about 800 rows of 64 (512: 7.7 against 9.5 us, 1000: 11.7 against 10.2), and 300 of 96 or 128 (256: 9.0 against
+// 9.8, 512: 11.3 against 10.2).
+constexpr uint32_t XO_WAVES = 16;            // = the most blocks
+struct XoTab {
+    const uint64_t* p;
+    __device__ __forceinline__ uint64_t operator()(int i) const { return p[i]; }
+};
+
+template <int HD>
+__global__ __launch_bounds__(XO_WAVES * 64) void attn_exact_decode_one_kernel(const float* __restrict__ q, const uint16_t* __restrict__ kc,
+                                                                             const uint16_t* __restrict__ vc, float* __restrict__ out,
+                                                                             int8_t* __restrict__ oq, uint16_t* __restrict__ osc,
+                                                                             uint32_t base_pos, const uint32_t* __restrict__ pos_dev,
+                                                                             uint32_t heads, uint32_t kv_heads) {
+    constexpr int DPL = (HD + 63) / 64;                       // head dims per lane: lane, lane + 64
+    constexpr int KC = 32 / DPL;                              // keys whose V elements a lane holds at a time
+    __shared__ __attribute__((aligned(16))) float qs[HD];
+    __shared__ __attribute__((aligned(16))) float e[XO_WAVES][XB];
+    __shared__ float sums[XO_WAVES][HD];
+    __shared__ float bmax[XO_WAVES], mi[XO_WAVES], lblk[XO_WAVES], es[XO_WAVES];
+    __shared__ uint64_t tab_s[32];
+    const uint32_t tid = threadIdx.x, lane = tid & 63, h = blockIdx.x;
+    const uint32_t b = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));        // this wave's block
+    const uint32_t seq = (pos_dev ? *pos_dev : base_pos) + 1, nb = (seq + XB - 1) / XB;
+    if (nb > XO_WAVES) return;                                // the caller's promise did not hold: nothing is read or written
+    const uint32_t kvh = h / (heads / kv_heads), kv_stride = kv_heads * HD;
+    const uint32_t bs = b * XB, bl = bs < seq ? min((uint32_t)XB, seq - bs) : 0u;        // 0: no block for this wave
+    const float scale = 1.0f / sqrtf((float)HD);
+    const XoTab tab{tab_s};
+    // keys and the first values do not wait for q (rows past the last key re-read it)
+    uint4 kr[HD / 8];
+    uint16_t v[KC][DPL];
+    const uint16_t* vcol = vc + (size_t)bs * kv_stride + kvh * HD;
+    auto load_values = [&](uint32_t k0) {
+#pragma unroll
+        for (int i = 0; i < KC; i++)
+#pragma unroll
+            for (int t = 0; t < DPL; t++) {
+                const uint32_t d = lane + 64 * t;
+                v[i][t] = d < HD ? vcol[(size_t)min(k0 + i, bl - 1) * kv_stride + d] : (uint16_t)0;
+            }
+    };
+    if (bl) {
+        const uint16_t* krow = kc + (size_t)(bs + min(lane, bl - 1)) * kv_stride + kvh * HD;
+#pragma unroll
+        for (int c = 0; c < HD / 8; c++) kr[c] = *reinterpret_cast<const uint4*>(krow + c * 8);
+    }
+    if (tid < HD) qs[tid] = q[h * HD + tid];
+    if (tid >= 128 && tid < 160) tab_s[tid - 128] = expf_detail::tab((int)tid - 128);
+    if (bl) load_values(0);
+    __syncthreads();
+    float sc = -INFINITY;
+    if (bl) {
+        float sum = 0.f;
+#pragma unroll
+        for (int c = 0; c < HD / 8; c++) {
+            const uint32_t ww[4] = {kr[c].x, kr[c].y, kr[c].z, kr[c].w};
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                sum = sum + qs[c * 8 + 2 * j] * f16_bits_to_f32((uint16_t)(ww[j] & 0xFFFFu));
+                sum = sum + qs[c * 8 + 2 * j + 1] * f16_bits_to_f32((uint16_t)(ww[j] >> 16));
+            }
+        }
+        if (lane < bl) sc = sum * scale;
+        const float mb = wave_max(sc);
+        if (lane == 0) bmax[b] = mb;
+    }
+    __syncthreads();
+    if (bl) {
+        // m_i after this block: the largest block maximum so far
+        const float m = wave_max(lane <= b ? bmax[lane] : -INFINITY);
+        e[b][lane] = lane < bl ? expf_ref_with<true>(sc - m, tab) : 0.f;       // LDS operations of one wave execute in order
+        float l_block = 0.f, sum[DPL];
+#pragma unroll
+        for (int t = 0; t < DPL; t++) sum[t] = 0.f;
+#pragma nounroll
+        for (int k0 = 0; k0 < XB; k0 += KC) {
+            if (k0) load_values(k0);
+#pragma unroll
+            for (int i4 = 0; i4 < KC; i4 += 4) {
+                const float4 w4 = *reinterpret_cast<const float4*>(&e[b][k0 + i4]);
+                const float ww[4] = {w4.x, w4.y, w4.z, w4.w};
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    // keys past the last one: a selection, not a weight of 0 (0 * v is not 0 for an infinite v)
+                    const bool in = (uint32_t)(k0 + i4 + i) < bl;
+                    l_block = in ? l_block + ww[i] : l_block;
+#pragma unroll
+                    for (int t = 0; t < DPL; t++) sum[t] = in ? sum[t] + ww[i] * f16_bits_to_f32(v[i4 + i][t]) : sum[t];
+                }
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < DPL; t++)
+            if (lane + 64 * t < HD) sums[b][lane + 64 * t] = sum[t];
+        if (lane == 0) { mi[b] = m; lblk[b] = l_block; }
+    }
+    __syncthreads();
+    if (tid < nb) es[tid] = expf_ref_with<true>((tid ? mi[tid - 1] : -INFINITY) - mi[tid], tab);
+    __syncthreads();
+    if (tid >= (HD <= 64 ? 64 : 128)) return;
+    float l_i = 0.f, acc = 0.f;
+    const uint32_t d = tid < HD ? tid : 0;
+#pragma unroll 4
+    for (uint32_t i = 0; i < nb; i++) {
+        const float exp_scale = es[i];
+        l_i = l_i * exp_scale;
+        acc = acc * exp_scale;
+        l_i = l_i + lblk[i];
+        acc = acc + sums[i][d];
+    }
+    const float inv_l = 1.0f / l_i;
+    const float o = acc * inv_l;
+    if (tid < HD && out) out[h * HD + tid] = o;
+    if (oq) {
+        const float amax = half_wave_max(tid < HD ? fabsf(o) : 0.f);
+        float inv;
+        const float sq = act_scale(amax, inv);
+        if (tid < HD) {
+            const size_t idx = (size_t)h * HD + tid;
+            oq[idx] = (int8_t)quant_code(o * inv);
+            if ((tid & 31) == 0) osc[idx / 32] = f32_to_f16_bits(sq);
+        }
+    }
+}
+
 // Workspace of the spread-out decode attention for a cache of up to max_rows rows; 0 if it does not apply (then the
 // one-workgroup kernel runs).
 size_t attn_exact_decode_workspace_bytes(uint32_t heads, uint32_t hd, uint32_t max_rows) {
@@ -509,14 +638,23 @@ size_t attn_exact_decode_workspace_bytes(uint32_t heads, uint32_t hd, uint32_t m
     return (size_t)heads * xd_head_floats(nb_cap, hd) * sizeof(float);
 }
 
+// Rows up to which the decode attention is one launch (measured at attn_exact_decode_one_kernel).
+uint32_t attn_exact_one_launch_rows(uint32_t hd) { return hd <= 64 ? 768u : 256u; }
+
 // Longest window (rows whose scores one workgroup keeps in LDS) the order-faithful decode attention takes.
 uint32_t attn_exact_max_window() { return 12288; }
 
 void launch_attn_exact(bool batch_order, const float* q, uint32_t q_stride, const uint16_t* kc, const uint16_t* vc,
                        float* out, uint32_t out_stride, int8_t* oq, uint16_t* osc, uint32_t M, uint32_t base_pos,
                        const uint32_t* pos_dev, uint32_t heads, uint32_t kv_heads, uint32_t hd, uint32_t window, uint32_t max_rows,
-                       void* ws, hipStream_t s) {
+                       void* ws, hipStream_t s, uint32_t rows_at_most) {
     if (M == 0) return;
+    if (!batch_order && window == 0 && M == 1 && (pos_dev ? rows_at_most : base_pos + 1) <= attn_exact_one_launch_rows(hd)) {
+#define FH_XO(HD_) fh::launch(attn_exact_decode_one_kernel<HD_>, dim3(heads), XO_WAVES * 64, 0, s, q, kc, vc, out, oq, osc, base_pos, pos_dev, heads, kv_heads)
+        if (hd == 64) FH_XO(64); else if (hd == 96) FH_XO(96); else FH_XO(128);
+#undef FH_XO
+        return;
+    }
     if (ws && !batch_order && window == 0 && M == 1 && attn_exact_decode_workspace_bytes(heads, hd, max_rows) != 0) {
         const uint32_t nb_cap = (max_rows + XB - 1) / XB;
         // blocks past the position (known to the device only when pos_dev is set) return at once

@@ -79,6 +79,8 @@ struct LlamaModel : forge_hip_model {
     }
 
     void enqueue_decode_step() override;
+    uint32_t decode_form() const override;
+    uint32_t decode_rows_at_most() const { return decode_form() == 0 ? attn_exact_one_launch_rows(cfg.head_dim) : cfg.max_seq; }
     int32_t enqueue_prompt_rows(uint32_t rows, uint32_t base_pos) override;
     void enqueue_row_logits(uint32_t row) override;
     bool keeps_rows() const override { return !mixed || mixed_batched; }
@@ -142,7 +144,7 @@ void enqueue_decode_attention(LlamaModel* m, uint32_t l, const float* q, uint32_
         StageMark t(m, ST_ATTN);
         if (exact)
             launch_attn_exact(false, q, q_stride, m->kc(l), m->vc(l), nullptr, m->QKS, aq, asc, 1, 0, m->d_pos(), c.heads,
-                              c.kv_heads, c.head_dim, c.sliding_window, c.max_seq, m->attn_ws.p, s);
+                              c.kv_heads, c.head_dim, c.sliding_window, c.max_seq, m->attn_ws.p, s, m->decode_rows_at_most());
         else
             launch_attn_decode(q, m->kc(l), m->vc(l), nullptr, aq, asc, 0, m->d_pos(), c.heads, c.kv_heads, c.head_dim,
                                c.sliding_window, m->attn_ws.p, s, m->pt);
@@ -213,7 +215,7 @@ void enqueue_mixed_layer(LlamaModel* m, uint32_t l, uint32_t pos, const uint32_t
         const uint32_t win = c.sliding_window == 0 ? 0u : pos_dev ? c.sliding_window : c.max_seq;
         if (exact)
             launch_attn_exact(false, qkv, QKS, m->kc(l), m->vc(l), nullptr, QKS, aq, asc, 1, pos, pos_dev, c.heads, c.kv_heads,
-                              c.head_dim, win, c.max_seq, m->attn_ws.p, s);
+                              c.head_dim, win, c.max_seq, m->attn_ws.p, s, m->decode_rows_at_most());
         else
             launch_attn_decode(qkv, m->kc(l), m->vc(l), nullptr, aq, asc, pos + 1, pos_dev, c.heads, c.kv_heads, c.head_dim,
                                pos_dev ? c.sliding_window : 0u, m->attn_ws.p, s, m->pt);
@@ -474,6 +476,11 @@ void enqueue_head(LlamaModel* m, const float* xrow, bool after_prefill, bool adv
     }
     // the token sampled right after a prefill is not penalised (project.rs:719-720), those inside the loop are (:742-744)
     m->enqueue_argmax(!after_prefill, advance);
+}
+
+// Order-faithful attention: one launch over a short context, three spread over the chip beyond it.
+uint32_t LlamaModel::decode_form() const {
+    return (cfg.flags & FORGE_HIP_FLAG_EXACT) && cfg.sliding_window == 0 && pos + 1 > (int64_t)attn_exact_one_launch_rows(cfg.head_dim) ? 1u : 0u;
 }
 
 void LlamaModel::enqueue_decode_step() {

@@ -45,7 +45,7 @@ struct forge_hip_model {
     float* h_logits = nullptr;           // pinned: logits come home at PCIe speed and are copied to the caller's (pageable) buffer from here
     int64_t pos = 0;
     bool use_graph = true;
-    hipGraphExec_t decode_graph = nullptr;
+    hipGraphExec_t decode_graph[2] = {nullptr, nullptr};      // by decode_form()
     // forward_profile / prefill_profile: one event pair per kernel launch, tagged with the stage of the
     // enclosing StageMark (ST_COUNT = outside any stage, not measured)
     int prof_cur = 0;
@@ -60,12 +60,15 @@ struct forge_hip_model {
     virtual ~forge_hip_model();
     // Stream, pinned staging, decode state and sampling state for cfg (set before the call).
     int32_t init_shared();
+    void drop_decode_graphs();           // what the captured launches carry has changed: capture again at the next step
     // Last maximum of `logits` -> d_next() (+ position and token advance when `advance`).
     void enqueue_argmax(bool penalise, bool advance);
 
     // ---- the network -----------------------------------------------------------------------------
     // One decode step: the token *d_token() at position *d_pos(), logits, argmax, advance.  Captured into a graph.
     virtual void enqueue_decode_step() = 0;
+    // Which of (at most) two forms enqueue_decode_step gives the step at the host's position `pos`: each is captured into a graph of its own.
+    virtual uint32_t decode_form() const { return 0; }
     // `rows` tokens of a prompt (ptok) at positions base_pos..; fills the cache and leaves the rows' residual stream.
     virtual int32_t enqueue_prompt_rows(uint32_t rows, uint32_t base_pos) = 0;
     // Logits of row `row` of the last chunk (and their argmax) as they follow a prompt.

@@ -10,8 +10,15 @@
 
 using namespace fh;
 
+void forge_hip_model::drop_decode_graphs() {
+    for (hipGraphExec_t& g : decode_graph) {
+        if (g) (void)hipGraphExecDestroy(g);
+        g = nullptr;
+    }
+}
+
 forge_hip_model::~forge_hip_model() {
-    if (decode_graph) (void)hipGraphExecDestroy(decode_graph);
+    drop_decode_graphs();
     for (hipEvent_t e : prof_ev) (void)hipEventDestroy(e);
     if (h_stage) (void)hipHostFree(h_stage);
     if (h_logits) (void)hipHostFree(h_logits);
@@ -98,17 +105,18 @@ int32_t run_decode_step(forge_hip_model* m, uint32_t token) {
     if (m->resident()) return m->resident_enqueue(false, token);   // the token rides with the launch
     m->h_stage[0] = token;
     FH_HIP(hipMemcpyAsync(m->d_token(), &m->h_stage[0], 4, hipMemcpyHostToDevice, m->stream));
-    if (m->use_graph && !m->decode_graph) {
+    hipGraphExec_t& graph = m->decode_graph[m->decode_form()];
+    if (m->use_graph && !graph) {
         hipGraph_t g = nullptr;
         FH_HIP(hipStreamBeginCapture(m->stream, hipStreamCaptureModeThreadLocal));
         m->enqueue_decode_step();
         hipError_t e = hipStreamEndCapture(m->stream, &g);
         if (e != hipSuccess || !g) return fail(FORGE_HIP_ERR_HIP, std::string("graph capture failed: ") + hipGetErrorString(e));
-        e = hipGraphInstantiate(&m->decode_graph, g, nullptr, nullptr, 0);
+        e = hipGraphInstantiate(&graph, g, nullptr, nullptr, 0);
         (void)hipGraphDestroy(g);
-        if (e != hipSuccess) { m->decode_graph = nullptr; return fail(FORGE_HIP_ERR_HIP, std::string("graph instantiate failed: ") + hipGetErrorString(e)); }
+        if (e != hipSuccess) { graph = nullptr; return fail(FORGE_HIP_ERR_HIP, std::string("graph instantiate failed: ") + hipGetErrorString(e)); }
     }
-    if (m->decode_graph) FH_HIP(hipGraphLaunch(m->decode_graph, m->stream));
+    if (graph) FH_HIP(hipGraphLaunch(graph, m->stream));
     else { m->enqueue_decode_step(); FH_HIP(hipGetLastError()); }
     return FORGE_HIP_OK;
 }
@@ -316,8 +324,7 @@ int32_t forge_hip_model_set_repeat_penalty(forge_hip_model* m, float penalty) {
     const int32_t rc = m->repeat_penalty_changed(penalty);
     if (rc) return rc;
     m->repeat_penalty = penalty;
-    // the captured kernel sequence carries the old value in its launch arguments: capture again at the next step
-    if (m->decode_graph) { (void)hipGraphExecDestroy(m->decode_graph); m->decode_graph = nullptr; }
+    m->drop_decode_graphs();             // the captured kernel sequence carries the old value in its launch arguments
     return FORGE_HIP_OK;
 }
 
@@ -336,8 +343,7 @@ int32_t forge_hip_model_set_kv_pages(forge_hip_model* m, uint32_t page_rows, con
     FH_HIP(hipStreamSynchronize(m->stream));
     const int32_t rc = m->set_kv_pages(page_rows, page_table_host, n_pages);
     if (rc) return rc;
-    // the captured kernel sequence carries the old layout in its launch arguments: capture again at the next step
-    if (m->decode_graph) { (void)hipGraphExecDestroy(m->decode_graph); m->decode_graph = nullptr; }
+    m->drop_decode_graphs();             // the captured kernel sequence carries the old layout in its launch arguments
     return FORGE_HIP_OK;
 }
 

@@ -42,6 +42,26 @@ def tiny_cfg(fh, wd, flags):
     return cfg
 
 
+def test_exact_mode_across_the_line_between_the_attention_forms(fh, oracle, torch_gpu):
+    """The decode step's attention is one launch while the context has at most 768 rows and three beyond: steps on both sides of
+    the line (each form is a graph of its own), back below it after a reset, and once more across: the oracle's bits."""
+    cfg = dict(tiny_cfg(fh, Q8, EXACT), max_seq=1024)
+    blob = fh.synth.make_weights_blob(cfg, seed=13)
+    toks = fh.synth.uniform_ids(14, 766, cfg["vocab"])
+    gm, om = fh.HipModel(cfg, blob), oracle.Model(cfg, blob, A, KV_F16)
+    same_bits(gm.forward_prefill(toks), om.prefill_batched(toks))
+    want = [om.forward(t) for t in (5, 6, 7, 8)]
+    for turn in range(2):
+        for t, w in zip((5, 6, 7, 8), want):
+            same_bits(gm.forward(t), w)
+        gm.reset()
+        gm.forward_prefill(toks[:20])
+        gm.forward(9)
+        gm.reset()
+        gm.forward_prefill_batch(toks)
+    gm.close()
+
+
 @pytest.mark.parametrize("wd", [Q8, Q4])
 def test_tiny_model_exact_mode_is_bit_identical(fh, oracle, torch_gpu, wd):
     cfg = tiny_cfg(fh, wd, EXACT)

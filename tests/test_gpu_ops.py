@@ -413,6 +413,18 @@ def test_attention_decode_parity(fh, oracle, torch_gpu, heads, kv_heads, hd, seq
     close(fh.ops.attention_flash(qd, kd, vd, seq, heads, kv_heads, hd, 0).cpu().numpy(), want)
 
 
+@pytest.mark.parametrize("heads,kv_heads,hd", [(9, 3, 64), (8, 8, 96), (6, 2, 128)])
+@pytest.mark.parametrize("seq", [63, 65, 128, 256, 257, 300, 767, 768, 769])
+def test_attention_decode_order_faithful_at_the_launch_forms_edges(fh, oracle, torch_gpu, heads, kv_heads, hd, seq):
+    """One launch up to 768 (heads of 64) or 256 rows, three beyond: the oracle's bits on both sides of the line and of a block."""
+    torch = torch_gpu
+    k, v = _kv_cache(fh, oracle, seq, kv_heads, hd, seq + hd)
+    q = fh.synth.normal(7 + seq, heads * hd, 1.0)
+    want = oracle.attention("flash", q, k, v, seq, heads, kv_heads, hd)
+    got = fh.ops.attention_flash(torch.from_numpy(q).cuda(), _dev16(torch, k), _dev16(torch, v), seq, heads, kv_heads, hd, EXACT)
+    same_bits(got.cpu().numpy(), want)
+
+
 @pytest.mark.parametrize("heads,kv_heads,hd", [(32, 8, 64), (9, 3, 64), (32, 32, 96), (24, 8, 128)])
 @pytest.mark.parametrize("seq,page_rows", [(1, 16), (70, 16), (900, 64), (2250, 16), (2250, 256), (8192, 128), (777, 1)])
 def test_attention_decode_paged_cache(fh, oracle, torch_gpu, heads, kv_heads, hd, seq, page_rows):
