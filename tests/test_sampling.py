@@ -126,6 +126,21 @@ def test_sample_equals_oracle_and_brackets_r(fh, oracle, so, temp, top_k, top_p)
             assert tok_l == n - 1
 
 
+@pytest.mark.parametrize("n,top_k,top_p", [(4097, 4095, 1.0), (4097, 4096, 1.0), (9001, 4096, 0.999), (9002, 5120, 0.9), (9003, 9002, 1.0), (30001, 0, 0.5),
+                                           (30002, 0, 0.99), (30003, 1, 0.99), (3, 2, 0.7), (1, 0, 0.5)])
+@pytest.mark.parametrize("spread", [0.0, 0.3, 3.0, 40.0])
+def test_cuts_at_the_edges_of_the_partial_order(fh, oracle, so, n, top_k, top_p, spread):
+    """The descending order is worked out batch by batch (1024 or top_k entries, then four times as many; sorted by bits from 4096 up) and
+    exp runs in fours: sizes on both sides of those lines, from all entries equal (0.0) over many ties (logits in steps of a half) to
+    probabilities that underflow (40.0).  Every result equals the oracle's full stable sort bit for bit."""
+    base = logits_of(fh, n + top_k, n, spread)
+    for l in (base, np.round(base * 2) / 2):
+        l = np.ascontiguousarray(l, np.float32)
+        a, b = l.copy(), l.copy()
+        assert fh.ops.sample(a, 0.9, top_k, top_p, 991) == so.sample(oracle, b, 0.9, top_k, top_p, 991)
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
 def test_top_p_drops_the_entry_that_crosses_the_threshold(fh, oracle, so):
     """project.rs:535-540 zeroes every entry from the first whose running sum exceeds top_p, that entry included."""
     l = np.log(np.array([0.5, 0.3, 0.15, 0.05], np.float32))
