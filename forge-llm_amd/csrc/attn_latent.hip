@@ -61,7 +61,7 @@ __global__ __launch_bounds__(256) void latent_norm_store_kernel(LatentShape sh, 
 
 // ---- decode ----------------------------------------------------------------------------------------------------------------
 // [RMS norm of the query latent | W_uq | rotation]; the last workgroup writes the position's cache row instead.
-template <typename T, int KS>
+template <typename T, int KS, int STEPS>
 __global__ __launch_bounds__(GEMV_THREADS) void latent_query_kernel(LatentShape sh, const float* __restrict__ raw, const float* __restrict__ q_norm,
                                                                     const float* __restrict__ kv_norm, const T* __restrict__ uq, DenseEpiArgs e,
                                                                     T* __restrict__ cache) {
@@ -73,7 +73,7 @@ __global__ __launch_bounds__(GEMV_THREADS) void latent_query_kernel(LatentShape 
         store_cache_row<T>(sh, raw, kv_norm, e.cos_t, e.sin_t, e.pos_dev ? *e.pos_dev : e.base_pos, cache, red, tid, GEMV_THREADS);
         return;
     }
-    gemv_body<T, KS, DenseEpi::Rope>(uq, sh.q_row(), K, blockIdx.x * gemv_rows<KS>(), xs, red, e, [&]() {
+    gemv_body<T, KS, DenseEpi::Rope, STEPS>(uq, sh.q_row(), K, blockIdx.x * gemv_rows<KS>(), xs, red, e, [&]() {
         float ss = 0.f;
         for (uint32_t i = tid; i < K; i += GEMV_THREADS) ss = fmaf(raw[i], raw[i], ss);
         const float inv = 1.0f / sqrtf(block_sum(ss, red, tid, GEMV_THREADS) / (float)sh.q_rank_n + sh.eps);
@@ -224,7 +224,7 @@ __global__ __launch_bounds__(NW * 64) void latent_attn_decode_kernel(LatentShape
 }
 
 // [merge of the parts | W_uv | gate]: a workgroup's rows belong to one head.
-template <typename T>
+template <typename T, int STEPS>
 __global__ __launch_bounds__(GEMV_THREADS) void latent_value_kernel(LatentShape sh, const float* __restrict__ parts, uint32_t nparts, const T* __restrict__ uv, DenseEpiArgs e) {
     extern __shared__ __attribute__((aligned(16))) float lv_lds[];
     // the workgroups of a head are `heads` apart: with a multiple of 8 heads they sit on one XCD and share the parts in its L2
@@ -233,7 +233,7 @@ __global__ __launch_bounds__(GEMV_THREADS) void latent_value_kernel(LatentShape 
     float* xs = lv_lds;
     float* red = lv_lds + K;
     float* wt = red + 16;           // [SPLITS_MAX]
-    gemv_body<T, 1, DenseEpi::GateMul>(uv, sh.heads * sh.vdim, K, row0, xs, red, e, [&]() {
+    gemv_body<T, 1, DenseEpi::GateMul, STEPS>(uv, sh.heads * sh.vdim, K, row0, xs, red, e, [&]() {
         const size_t step = (size_t)sh.heads * (sh.rank + 4);
         const float* rec = parts + (size_t)head * (sh.rank + 4);
         // the first sums are requested ahead of the statistics they are weighted with
@@ -281,12 +281,18 @@ void go_decode(const LatentShape& sh, const LatentDecodeIo& io, hipStream_t s) {
                (const T*)io.ql, (const T*)io.cache, io.parts, io.base_pos, io.pos_dev);
 }
 
+template <typename T, int KS, int STEPS>
+void query_steps(const LatentShape& sh, const LatentDecodeIo& io, const DenseEpiArgs& e, hipStream_t s) {
+    static const hipError_t ok = hipFuncSetAttribute((const void*)latent_query_kernel<T, KS, STEPS>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    (void)ok;
+    fh::launch(latent_query_kernel<T, KS, STEPS>, dim3((sh.q_row() + gemv_rows<KS>() - 1) / gemv_rows<KS>() + 1), GEMV_THREADS, (sh.q_rank + 16) * 4, s, sh, io.raw,
+               io.q_norm, io.kv_norm, (const T*)io.uq.p, e, (T*)io.cache);
+}
+
 template <typename T, int KS>
 void go_query(const LatentShape& sh, const LatentDecodeIo& io, const DenseEpiArgs& e, hipStream_t s) {
-    static const hipError_t ok = hipFuncSetAttribute((const void*)latent_query_kernel<T, KS>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    (void)ok;
-    fh::launch(latent_query_kernel<T, KS>, dim3((sh.q_row() + gemv_rows<KS>() - 1) / gemv_rows<KS>() + 1), GEMV_THREADS, (sh.q_rank + 16) * 4, s, sh, io.raw,
-               io.q_norm, io.kv_norm, (const T*)io.uq.p, e, (T*)io.cache);
+    if (sh.q_rank <= gemv_step<T, KS>()) query_steps<T, KS, 1>(sh, io, e, s);
+    else query_steps<T, KS, 2>(sh, io, e, s);
 }
 
 template <typename T>
@@ -326,7 +332,9 @@ void decode(const LatentShape& sh, const LatentDecodeIo& io, hipStream_t s) {
     // the 16 rows of a workgroup lie in one head (vdim is a multiple of 32); every workgroup merges its head's parts, so few of them
     const T* uv = (const T*)io.ukv.p + (size_t)sh.heads * sh.dim * sh.rank;
     const uint32_t N = sh.heads * sh.vdim, lds = (sh.rank + 16 + SPLITS_MAX) * 4, np = latent_splits(sh, io.max_seq);
-    fh::launch(latent_value_kernel<T>, dim3(N / gemv_rows<1>()), GEMV_THREADS, lds, s, sh, io.parts, np, uv, e);
+    auto value = [&](auto kernel) { fh::launch(kernel, dim3(N / gemv_rows<1>()), GEMV_THREADS, lds, s, sh, io.parts, np, uv, e); };
+    if (sh.rank <= gemv_step<T, 1>()) value(latent_value_kernel<T, 1>);
+    else value(latent_value_kernel<T, 2>);
 }
 
 }  // namespace

@@ -117,65 +117,134 @@ void dense_gemm_kernel(const T* __restrict__ w, const T* __restrict__ a, uint32_
 }
 
 // The vector of a one-row product goes into LDS as floats, made from what DenseIn names.
-template <typename T, int KS, DenseEpi MODE, DenseIn::Kind IN>
+template <typename T, int KS, DenseEpi MODE, DenseIn::Kind IN, int STEPS>
 __global__ __launch_bounds__(GEMV_THREADS) void dense_gemv_kernel(const T* __restrict__ w, DenseIn in, uint32_t N, uint32_t K, DenseEpiArgs e) {
     extern __shared__ __attribute__((aligned(16))) float gemv_lds[];
     const uint32_t tid = threadIdx.x;
     float* xs = gemv_lds;
     float* red = gemv_lds + K;
-    gemv_body<T, KS, MODE>(w, N, K, blockIdx.x * gemv_rows<KS>(), xs, red, e, [&]() {
-        if constexpr (IN == DenseIn::Rows) {
-            const T* a = (const T*)in.rows;
-            for (uint32_t k = tid * 8; k < K; k += GEMV_THREADS * 8) {
-                const typename Vec<T>::x8 v = load8(a + k);
+    typedef typename Vec<T>::x4 x4;
+    typedef typename Vec<T>::x8 x8;
+    // What the prologue reads first is requested ahead of the matrix, into registers: NV pieces per thread of 4 columns (Rows: 8).
+    constexpr uint32_t NV = STEPS == 1 ? 1 : 3;
+    if constexpr (IN == DenseIn::Rows) {
+        const T* a = (const T*)in.rows;
+        x8 v[NV];
 #pragma unroll
-                for (int j = 0; j < 8; j++) xs[k + j] = (float)v[j];
+        for (uint32_t i = 0; i < NV; i++) {
+            const uint32_t k = (tid + i * GEMV_THREADS) * 8;
+            if (k < K) v[i] = load8(a + k);
+        }
+        gemv_body<T, KS, MODE, STEPS>(w, N, K, blockIdx.x * gemv_rows<KS>(), xs, red, e, [&]() {
+            auto put = [&](uint32_t k, const x8& x) {
+#pragma unroll
+                for (int j = 0; j < 8; j++) xs[k + j] = (float)x[j];
+            };
+#pragma unroll
+            for (uint32_t i = 0; i < NV; i++) {
+                const uint32_t k = (tid + i * GEMV_THREADS) * 8;
+                if (k < K) put(k, v[i]);
             }
-        } else if constexpr (IN == DenseIn::Normed) {
-            // a thread keeps to its own elements until the product's barrier
+            for (uint32_t k = (tid + NV * GEMV_THREADS) * 8; k < K; k += GEMV_THREADS * 8) put(k, load8(a + k));
+        });
+    } else if constexpr (IN == DenseIn::Normed) {
+        v4f v[NV], lw[NV], lb[NV];
+#pragma unroll
+        for (uint32_t i = 0; i < NV; i++) {
+            const uint32_t k = (tid + i * GEMV_THREADS) * 4;
+            v[i] = (v4f){0.f, 0.f, 0.f, 0.f};
+            if (k < K) {
+                v[i] = *reinterpret_cast<const v4f*>(in.f32 + k);
+                lw[i] = *reinterpret_cast<const v4f*>(in.ln.w + k);
+                lb[i] = *reinterpret_cast<const v4f*>(in.ln.b + k);
+            }
+        }
+        gemv_body<T, KS, MODE, STEPS>(w, N, K, blockIdx.x * gemv_rows<KS>(), xs, red, e, [&]() {
+            // a thread keeps to its own elements until the product's barrier; those past the registers wait in LDS
+            constexpr uint32_t REST = NV * GEMV_THREADS * 4;
             float s = 0.f;
-            for (uint32_t k = tid * 4; k < K; k += GEMV_THREADS * 4) {
-                const v4f v = *reinterpret_cast<const v4f*>(in.f32 + k);
-                *reinterpret_cast<v4f*>(xs + k) = v;
-                s += (v[0] + v[1]) + (v[2] + v[3]);                       // zero past ln.n
+#pragma unroll
+            for (uint32_t i = 0; i < NV; i++) s += (v[i][0] + v[i][1]) + (v[i][2] + v[i][3]);      // zero past ln.n
+            for (uint32_t k = REST + tid * 4; k < K; k += GEMV_THREADS * 4) {
+                const v4f x = *reinterpret_cast<const v4f*>(in.f32 + k);
+                *reinterpret_cast<v4f*>(xs + k) = x;
+                s += (x[0] + x[1]) + (x[2] + x[3]);
             }
             const float mean = block_sum(s, red, tid, GEMV_THREADS) / (float)in.ln.n;
             float ss = 0.f;
-            for (uint32_t k = tid * 4; k < K; k += GEMV_THREADS * 4)
+            auto square = [&](uint32_t k, const v4f& x) {
 #pragma unroll
                 for (int j = 0; j < 4; j++) {
-                    const float d = xs[k + j] - mean;
+                    const float d = x[j] - mean;
                     if (k + j < in.ln.n) ss = fmaf(d, d, ss);
                 }
+            };
+#pragma unroll
+            for (uint32_t i = 0; i < NV; i++) square((tid + i * GEMV_THREADS) * 4, v[i]);
+            for (uint32_t k = REST + tid * 4; k < K; k += GEMV_THREADS * 4) square(k, *reinterpret_cast<const v4f*>(xs + k));
             const float inv = 1.0f / sqrtf(block_sum(ss, red, tid, GEMV_THREADS) / (float)in.ln.n + in.ln.eps);
-            for (uint32_t k = tid * 4; k < K; k += GEMV_THREADS * 4) {
-                const v4f lw = *reinterpret_cast<const v4f*>(in.ln.w + k), lb = *reinterpret_cast<const v4f*>(in.ln.b + k);
+            auto put = [&](uint32_t k, const v4f& x, const v4f& nw, const v4f& nb) {
+                v4f y;
 #pragma unroll
-                for (int j = 0; j < 4; j++) xs[k + j] = (xs[k + j] - mean) * inv * lw[j] + lb[j];
+                for (int j = 0; j < 4; j++) y[j] = (x[j] - mean) * inv * nw[j] + nb[j];
+                *reinterpret_cast<v4f*>(xs + k) = y;
+            };
+#pragma unroll
+            for (uint32_t i = 0; i < NV; i++) {
+                const uint32_t k = (tid + i * GEMV_THREADS) * 4;
+                if (k < K) put(k, v[i], lw[i], lb[i]);
             }
-        } else {
-            // head = a multiple of 32 columns: lane group of 16, 4 columns per lane and step
-            const uint32_t n = in.heads * in.head;
-            for (uint32_t k = n + tid; k < K; k += GEMV_THREADS) xs[k] = 0.f;
-            for (uint32_t h = tid / 16; h < in.heads; h += GEMV_THREADS / 16) {
-                const float* o = in.f32 + h * in.head;
-                float ss = 0.f;
-                for (uint32_t c = tid % 16 * 4; c < in.head; c += 64) {
-                    const v4f v = *reinterpret_cast<const v4f*>(o + c);
+            for (uint32_t k = REST + tid * 4; k < K; k += GEMV_THREADS * 4)
+                put(k, *reinterpret_cast<const v4f*>(xs + k), *reinterpret_cast<const v4f*>(in.ln.w + k), *reinterpret_cast<const v4f*>(in.ln.b + k));
+        });
+    } else {
+        // head = a multiple of 32 columns: lane group of 16, 4 columns per lane and step; the first head's first 128 columns in registers
+        constexpr uint32_t NH = 2;
+        const uint32_t h0 = tid / 16, c0 = tid % 16 * 4;
+        v4f v0[NH], hw0[NH];
+        x4 g0[NH];
 #pragma unroll
-                    for (int j = 0; j < 4; j++) ss = fmaf(v[j], v[j], ss);      // zero past head_n
-                }
-                ss = lane_xor_add<8>(ss); ss = lane_xor_add<4>(ss); ss = lane_xor_add<2>(ss); ss = lane_xor_add<1>(ss);
-                const float inv = 1.0f / sqrtf(ss / (float)in.head_n + in.eps);
-                for (uint32_t c = tid % 16 * 4; c < in.head; c += 64) {
-                    const v4f v = *reinterpret_cast<const v4f*>(o + c), hw = *reinterpret_cast<const v4f*>(in.w + c);
-                    const typename Vec<T>::x4 g = *reinterpret_cast<const typename Vec<T>::x4*>((const T*)in.gate + h * in.head + c);
-#pragma unroll
-                    for (int j = 0; j < 4; j++) xs[h * in.head + c + j] = v[j] * inv * hw[j] * (float)g[j];
-                }
+        for (uint32_t i = 0; i < NH; i++) {
+            const uint32_t c = c0 + 64 * i;
+            v0[i] = (v4f){0.f, 0.f, 0.f, 0.f};
+            if (h0 < in.heads && c < in.head) {
+                v0[i] = *reinterpret_cast<const v4f*>(in.f32 + h0 * in.head + c);
+                hw0[i] = *reinterpret_cast<const v4f*>(in.w + c);
+                g0[i] = *reinterpret_cast<const x4*>((const T*)in.gate + h0 * in.head + c);
             }
         }
-    });
+        gemv_body<T, KS, MODE, STEPS>(w, N, K, blockIdx.x * gemv_rows<KS>(), xs, red, e, [&]() {
+            const uint32_t n = in.heads * in.head;
+            for (uint32_t k = n + tid; k < K; k += GEMV_THREADS) xs[k] = 0.f;
+            for (uint32_t h = h0; h < in.heads; h += GEMV_THREADS / 16) {
+                const float* o = in.f32 + h * in.head;
+                float ss = 0.f;
+                auto square = [&](const v4f& v) {
+#pragma unroll
+                    for (int j = 0; j < 4; j++) ss = fmaf(v[j], v[j], ss);      // zero past head_n
+                };
+                const bool first = h == h0;
+                if (first) {
+#pragma unroll
+                    for (uint32_t i = 0; i < NH; i++) square(v0[i]);
+                }
+                for (uint32_t c = c0 + (first ? 64 * NH : 0); c < in.head; c += 64) square(*reinterpret_cast<const v4f*>(o + c));
+                ss = lane_xor_add<8>(ss); ss = lane_xor_add<4>(ss); ss = lane_xor_add<2>(ss); ss = lane_xor_add<1>(ss);
+                const float inv = 1.0f / sqrtf(ss / (float)in.head_n + in.eps);
+                auto put = [&](uint32_t c, const v4f& v, const v4f& hw, const x4& g) {
+#pragma unroll
+                    for (int j = 0; j < 4; j++) xs[h * in.head + c + j] = v[j] * inv * hw[j] * (float)g[j];
+                };
+                if (first) {
+#pragma unroll
+                    for (uint32_t i = 0; i < NH; i++)
+                        if (c0 + 64 * i < in.head) put(c0 + 64 * i, v0[i], hw0[i], g0[i]);
+                }
+                for (uint32_t c = c0 + (first ? 64 * NH : 0); c < in.head; c += 64)
+                    put(c, *reinterpret_cast<const v4f*>(o + c), *reinterpret_cast<const v4f*>(in.w + c), *reinterpret_cast<const x4*>((const T*)in.gate + h * in.head + c));
+            }
+        });
+    }
 }
 
 // One workgroup per row; a thread holds NV groups of four elements.
@@ -245,12 +314,18 @@ void go_gemm(const DenseWeight& w, const void* a, uint32_t lda, uint32_t M, cons
     fh::launch(dense_gemm_kernel<T, TN, TM, MODE>, dim3(tn * tm), 256, lds, s, (const T*)w.p, (const T*)a, lda, M, w.N, w.K, tn, e);
 }
 
+template <typename T, int KS, DenseEpi MODE, DenseIn::Kind IN, int STEPS>
+void gemv_steps(const DenseWeight& w, const DenseIn& in, const DenseEpiArgs& e, hipStream_t s) {
+    static const hipError_t lds_ok = hipFuncSetAttribute((const void*)dense_gemv_kernel<T, KS, MODE, IN, STEPS>, hipFuncAttributeMaxDynamicSharedMemorySize, (DENSE_K_MAX + 16) * 4);
+    (void)lds_ok;
+    fh::launch(dense_gemv_kernel<T, KS, MODE, IN, STEPS>, dim3((w.N + gemv_rows<KS>() - 1) / gemv_rows<KS>()), GEMV_THREADS, (w.K + 16) * 4, s, (const T*)w.p,
+               in, w.N, w.K, e);
+}
+
 template <typename T, int KS, DenseEpi MODE, DenseIn::Kind IN>
 void go_gemv(const DenseWeight& w, const DenseIn& in, const DenseEpiArgs& e, hipStream_t s) {
-    static const hipError_t lds_ok = hipFuncSetAttribute((const void*)dense_gemv_kernel<T, KS, MODE, IN>, hipFuncAttributeMaxDynamicSharedMemorySize, (DENSE_K_MAX + 16) * 4);
-    (void)lds_ok;
-    fh::launch(dense_gemv_kernel<T, KS, MODE, IN>, dim3((w.N + gemv_rows<KS>() - 1) / gemv_rows<KS>()), GEMV_THREADS, (w.K + 16) * 4, s, (const T*)w.p,
-               in, w.N, w.K, e);
+    if (w.K <= gemv_step<T, KS>()) gemv_steps<T, KS, MODE, IN, 1>(w, in, e, s);
+    else gemv_steps<T, KS, MODE, IN, 2>(w, in, e, s);
 }
 
 template <typename T, DenseEpi MODE, DenseIn::Kind IN>

@@ -377,6 +377,18 @@ def test_the_cap_bends_large_logits_only(fh, ko, torch_gpu, tmp_path):
         m.close()
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("width,heads,value", [(1024, 16, 128), (1030, 17, 130), (3072, 3, 96), (3080, 33, 40)])
+def test_decode_prologues_past_their_registers(fh, ko, torch_gpu, tmp_path, width, heads, value, dtype):
+    """A matrix-vector product's prologue holds the first columns (1024 or 3072 of a norm; 16 heads, 128 values of each, of a gate) in
+    registers and reads the rest when it comes to it: sizes on both sides of these lines, step by step."""
+    cfg = fh.synth.kakirax_config(width, 61, [fh.synth.kakirax_gla(heads, 8, value, 70, tau=5.0)], embedding_scale=3.0)
+    c = Case(fh, ko, tmp_path, cfg)
+    m = c.model(dtype=dtype, max_seq=8)
+    check(decode_all(m, c.ids(5)), c.oracle.forward(c.ids(5))[0], dtype)
+    m.close()
+
+
 # ---- generation, loading, replay --------------------------------------------------------------------------------------------------
 
 def test_greedy_generation(get):

@@ -311,6 +311,14 @@ def test_dense_products(fh, torch_gpu, M, N, K):
             fh.check(fh.lib().forge_hip_dense_matmul(fh.F32, wd.data_ptr(), ad.data_ptr(), *bad, y.data_ptr(), None))
 
 
+@pytest.mark.parametrize("N,K", [(5, 512), (5, 576), (7, 1024), (7, 1088), (5, 2048), (5, 2112), (3, 4096), (3, 4160), (5, 8256), (12289, 512), (12289, 576),
+                                 (12290, 1024), (12290, 1088), (12291, 2048), (12292, 2112), (12301, 3136)])
+def test_dense_products_of_one_row_at_the_edges_of_a_step(fh, torch_gpu, N, K):
+    """A wave requests two steps of weights ahead, or the only one: depths that fill a step of 512 or 1024 columns per wave (1, 2 or 4 waves
+    to a row), that begin the next one, and that begin the third (the first to be requested in the loop)."""
+    test_dense_products(fh, torch_gpu, 1, N, K)
+
+
 # ---- generation, loading, replay --------------------------------------------------------------------------------------------------
 
 def test_greedy_generation(get):
