@@ -86,14 +86,42 @@ __device__ __forceinline__ float block_sum(float v, float* red, uint32_t tid, ui
     return s;
 }
 
+// What an epilogue reads from memory: what belongs to the columns n .. n + 3, and what belongs to one row of them.
+template <DenseEpi MODE> struct EpiCols {};
+template <> struct EpiCols<DenseEpi::Residual> { float4 pw, pb, nw, nb; };
+template <typename T, DenseEpi MODE> struct EpiRow {};
+template <typename T> struct EpiRow<T, DenseEpi::Residual> { float4 x; };
+template <typename T> struct EpiRow<T, DenseEpi::GateMul> { typename Vec<T>::x4 gate; };
+
+template <DenseEpi MODE> __device__ __forceinline__ EpiCols<MODE> epilogue_cols(const DenseEpiArgs& e, uint32_t n) {
+    EpiCols<MODE> c;
+    if constexpr (MODE == DenseEpi::Residual) {
+        const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+        c.pw = e.post.w ? *reinterpret_cast<const float4*>(e.post.w + n) : zero; c.pb = e.post.w ? *reinterpret_cast<const float4*>(e.post.b + n) : zero;
+        c.nw = e.next.w ? *reinterpret_cast<const float4*>(e.next.w + n) : zero; c.nb = e.next.w ? *reinterpret_cast<const float4*>(e.next.b + n) : zero;
+    }
+    return c;
+}
+template <typename T, DenseEpi MODE> __device__ __forceinline__ EpiRow<T, MODE> epilogue_row(const DenseEpiArgs& e, uint32_t m, uint32_t n) {
+    EpiRow<T, MODE> r;
+    if constexpr (MODE == DenseEpi::Residual) r.x = e.add ? *reinterpret_cast<const float4*>(e.f32 + (size_t)m * e.ld_f32 + n) : make_float4(0.f, 0.f, 0.f, 0.f);
+    if constexpr (MODE == DenseEpi::GateMul) r.gate = *reinterpret_cast<const typename Vec<T>::x4*>((const T*)e.gate + (size_t)m * e.ld_out + n);
+    return r;
+}
+
 // What happens to the results (m, n .. n + 3) of a product; n is a multiple of 4.
 template <typename T, DenseEpi MODE>
-__device__ __forceinline__ void dense_epilogue(const DenseEpiArgs& e, uint32_t m, uint32_t n, uint32_t N, const float* v) {
+__device__ __forceinline__ void dense_epilogue(const DenseEpiArgs& e, uint32_t m, uint32_t n, uint32_t N, const float* v, const EpiCols<MODE>& cols,
+                                               const EpiRow<T, MODE>& row) {
     if constexpr (MODE == DenseEpi::F32) {
         float* y = e.f32 + (size_t)m * e.ld_f32 + n;
+        float a[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) a[i] = e.cap > 0.f ? e.cap * tanhf(v[i] / e.cap) : v[i];
+        if (n + 3 < N && (reinterpret_cast<uintptr_t>(y) & 15) == 0) { *reinterpret_cast<float4*>(y) = make_float4(a[0], a[1], a[2], a[3]); return; }
 #pragma unroll
         for (int i = 0; i < 4; i++)
-            if (n + i < N) y[i] = e.cap > 0.f ? e.cap * tanhf(v[i] / e.cap) : v[i];
+            if (n + i < N) y[i] = a[i];
     } else if constexpr (MODE == DenseEpi::RawGate) {
         if (n < e.split) *reinterpret_cast<float4*>(e.f32 + (size_t)m * e.ld_f32 + n) = make_float4(v[0], v[1], v[2], v[3]);
         else store4<T>((T*)e.out + (size_t)m * e.ld_out + (n - e.split), act_f(e.act, v[0]), act_f(e.act, v[1]), act_f(e.act, v[2]), act_f(e.act, v[3]));
@@ -118,19 +146,18 @@ __device__ __forceinline__ void dense_epilogue(const DenseEpiArgs& e, uint32_t m
         T* y = n < e.split ? (T*)e.out + (size_t)m * e.ld_out + n : (T*)e.out2 + (size_t)m * e.ld_out2 + (n - e.split);
         store4<T>(y, v[0], v[1], v[2], v[3]);
     } else if constexpr (MODE == DenseEpi::GateMul) {
-        const T* g = (const T*)e.gate + (size_t)m * e.ld_out + n;
+        const typename Vec<T>::x4 g = row.gate;
         store4<T>((T*)e.out + (size_t)m * e.ld_out + n, v[0] * (float)g[0], v[1] * (float)g[1], v[2] * (float)g[2], v[3] * (float)g[3]);
     } else if constexpr (MODE == DenseEpi::ActPair) {
         T* y = (T*)e.out + (size_t)m * e.ld_out + n / 2;
-        y[0] = (T)(act_f(e.act, v[0]) * v[1]);
-        y[1] = (T)(act_f(e.act, v[2]) * v[3]);
+        typedef T T2 __attribute__((ext_vector_type(2)));
+        T2 p;
+        p[0] = (T)(act_f(e.act, v[0]) * v[1]);
+        p[1] = (T)(act_f(e.act, v[2]) * v[3]);
+        *reinterpret_cast<T2*>(y) = p;
     } else if constexpr (MODE == DenseEpi::Residual) {
-        // everything the four results need is requested at once
         float4* xp = reinterpret_cast<float4*>(e.f32 + (size_t)m * e.ld_f32 + n);
-        const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
-        const float4 x = e.add ? *xp : zero;
-        const float4 pw = e.post.w ? *reinterpret_cast<const float4*>(e.post.w + n) : zero, pb = e.post.w ? *reinterpret_cast<const float4*>(e.post.b + n) : zero;
-        const float4 nw = e.next.w ? *reinterpret_cast<const float4*>(e.next.w + n) : zero, nb = e.next.w ? *reinterpret_cast<const float4*>(e.next.b + n) : zero;
+        const float4 x = row.x;
         float a[4] = {v[0], v[1], v[2], v[3]};
         auto norm4 = [&](const DynTanh& t, const float4& w, const float4& b) {
             if (!t.w) return;
@@ -139,11 +166,11 @@ __device__ __forceinline__ void dense_epilogue(const DenseEpiArgs& e, uint32_t m
             a[2] = tanhf(t.alpha * a[2]) * w.z + b.z;
             a[3] = tanhf(t.alpha * a[3]) * w.w + b.w;
         };
-        norm4(e.post, pw, pb);
+        norm4(e.post, cols.pw, cols.pb);
         a[0] += x.x; a[1] += x.y; a[2] += x.z; a[3] += x.w;
         *xp = make_float4(a[0], a[1], a[2], a[3]);
         if (!e.out) return;
-        norm4(e.next, nw, nb);
+        norm4(e.next, cols.nw, cols.nb);
         store4<T>((T*)e.out + (size_t)m * e.ld_out + n, a[0], a[1], a[2], a[3]);
     }
 }

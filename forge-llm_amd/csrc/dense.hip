@@ -1,11 +1,20 @@
 // Products with dense matrices (bfloat16 or 32-bit), y = a W^T, and the small kernels around them.
 //
-// M > 1: tiles on the matrix unit.  Workgroup = 4 waves (2 x 2), each TN x TM tiles of 32 x 32; the weights are the MFMA A operand,
-// so a lane ends up with four consecutive columns n of one row m and the epilogue writes them at once (and has pairs of columns,
-// rotary pairs and gate / up, in one lane).  A stage of 128 bytes of depth (64 bfloat16, 32 floats) goes from global memory
-// straight into one of two LDS buffers while the other one is worked; LDS rows are 128 bytes, the 16-byte piece c of row r at
-// position c ^ ((r >> 1) & 7), which keeps the fragment reads free of bank conflicts.  Rows past the end of a matrix read as
-// zero through the buffer descriptors' range check.
+// M > 1: tiles on the matrix unit.  Workgroup = WN x WM x KG waves, each TN x TM tiles of 32 x 32 over a KG-th of every stage's depth;
+// the weights are the MFMA A operand, so a lane ends up with four consecutive columns n of one row m (pairs of columns, rotary pairs
+// and gate / up in one lane).  A stage of 128 bytes of depth (64 bfloat16, 32 floats) goes from global memory straight into one of NBUF
+// LDS buffers while another one is worked; LDS rows are 128 bytes, the 16-byte piece c of row r at position c ^ ((r >> 1) & 7), which
+// keeps the fragment reads free of bank conflicts.  Rows past the end of a matrix read as zero through the buffer descriptors' range
+// check.
+//
+// What bounds it (bfloat16; matrix unit busy 38 % of 16384 x 2048 by 902 rows before, LDS 16 %, no bank conflicts):
+// - The results.  A lane holds 16 bytes of a row and its neighbours other rows, so stores straight from the registers touched a cache
+//   line per lane: 6 us for a tile of 128 x 128, 24 us for 256 x 256.  They go through LDS and out by whole rows.
+// - Operands that several XCDs fetch.  Tiles are dealt out in groups of 8 rows of tiles, column by column, and an XCD works a run of
+//   them: at 902 rows each XCD reads an eighth of the weights where it used to read all of them.
+// - The latency of a stage's loads where a compute unit has one workgroup: 3 or 4 buffers, and the depth shared out to the waves.
+// Times in us, 32-bit results, before / now: 16384 x 2048 by 902 rows 109 / 64.5 (940 TFLOP/s), 2048 x 8192 by 902 73.6 / 48.0,
+// 2048 x 2048 by 902 24.2 / 15.7, 6144 x 2048 by 902 49.3 / 33.7, 3072 x 576 by 2502 30.6 / 18.2, 576 x 576 by 2502 10.1 / 6.5.
 // M = 1: dense_gemv.h.
 #include <hip/hip_runtime.h>
 
@@ -24,41 +33,49 @@ constexpr uint32_t DENSE_K_MAX = 32768;             // a GEMV keeps its vector a
 
 #define FH_LDS3(p) ((__attribute__((address_space(3))) void*)(p))
 
-template <typename T, int TN, int TM, DenseEpi MODE>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+// LDS of a tile that goes out JP tiles of 32 rows per wave at a time: all of them if they fit in 128 KB.
+constexpr uint32_t dense_box(int WN, int WM, int KG, int TN, int JP) { return KG * (32 * TN * WN) * (32 * JP * WM) * 4; }
+constexpr int dense_pass(int WN, int WM, int KG, int TN, int TM) { return dense_box(WN, WM, KG, TN, TM) <= 128 * 1024 ? TM : TM / 2; }
+
+template <typename T, int WN, int WM, int KG, int TN, int TM, int NBUF, DenseEpi MODE>
+__global__ __launch_bounds__(64 * WN * WM * KG) __attribute__((amdgpu_waves_per_eu(2)))
 void dense_gemm_kernel(const T* __restrict__ w, const T* __restrict__ a, uint32_t lda, uint32_t M, uint32_t N, uint32_t K, uint32_t tiles_n,
                        DenseEpiArgs e) {
     extern __shared__ __attribute__((aligned(16))) uint8_t dense_lds[];
-    constexpr uint32_t BN = 64 * TN, BM = 64 * TM, BK = ROW_BYTES / sizeof(T), ES = sizeof(T);
+    constexpr uint32_t WAVES = WN * WM * KG, BN = 32 * TN * WN, BM = 32 * TM * WM, BK = ROW_BYTES / sizeof(T), ES = sizeof(T), LR = 8 * WAVES;
     constexpr uint32_t BUF = (BN + BM) * ROW_BYTES;
     const uint32_t tid = threadIdx.x, lane = tid & 63;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
-    const uint32_t wn = wave & 1, wm = wave >> 1, lrow = lane & 31, lh = lane >> 5;
+    const uint32_t wn = wave % WN, wm = wave / WN % WM, kg = wave / (WN * WM), lrow = lane & 31, lh = lane >> 5;
     // Workgroups go round robin over the 8 XCDs: give each XCD a run of neighbouring tiles (they share operand rows in its L2).
     uint32_t tile = blockIdx.x;
     {
         const uint32_t total = gridDim.x, per = total / 8, x = tile % 8, i = tile / 8;
         if (i < per) tile = x * per + i;          // the last total % 8 tiles stay where they are
     }
-    const uint32_t n0 = (tile % tiles_n) * BN, m0 = (tile / tiles_n) * BM;
+    // Tiles are counted in groups of GROUP rows of tiles, down the column first: the tiles that run at a time share both operands.
+    constexpr uint32_t GROUP = 8;
+    const uint32_t tiles_m = (M + BM - 1) / BM, first = tile / (GROUP * tiles_n) * GROUP, rows = min(GROUP, tiles_m - first), in = tile - first * tiles_n;
+    const uint32_t n0 = in / rows * BN, m0 = (first + in % rows) * BM;
     const uint32_t stages = K / BK;
 
     const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void*)(w + (size_t)n0 * K), 0, min(N - n0, BN) * K * ES, DENSE_RSRC_FLAGS);
     const __amdgpu_buffer_rsrc_t ra =
         __builtin_amdgcn_make_buffer_rsrc((void*)(a + (size_t)m0 * lda), 0, ((min(M - m0, BM) - 1) * lda + K) * ES, DENSE_RSRC_FLAGS);
-    // load i of wave v fills LDS rows (4 i + v) * 8 .. + 8, lane -> (row, position)
+    // load i of wave v fills LDS rows LR i + 8 v .. + 8, lane -> (row, position)
     const uint32_t ld_row = wave * 8 + (lane >> 3);
-    const uint32_t ld_piece = (lane & 7) ^ ((ld_row >> 1) & 7);       // rows 32 i further on have the same swizzle
+    const uint32_t ld_piece = (lane & 7) ^ ((ld_row >> 1) & 7);       // rows LR i further on have the same swizzle
     const uint32_t w_off = ld_row * K * ES + ld_piece * 16, a_off = ld_row * lda * ES + ld_piece * 16;
+    constexpr uint32_t LOADS = (BN + BM) / LR;
     auto issue = [&](uint32_t stage, uint32_t buf) {
         uint8_t* base = dense_lds + buf * BUF + wave * 1024;
         const uint32_t k = stage * ROW_BYTES;
 #pragma unroll
-        for (uint32_t i = 0; i < BN / 32; i++)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, FH_LDS3(base + i * 4096), 16, w_off + i * 32 * K * ES, k, 0, 0);
+        for (uint32_t i = 0; i < BN / LR; i++)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, FH_LDS3(base + i * LR * ROW_BYTES), 16, w_off + i * LR * K * ES, k, 0, 0);
 #pragma unroll
-        for (uint32_t i = 0; i < BM / 32; i++)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, FH_LDS3(base + BN * ROW_BYTES + i * 4096), 16, a_off + i * 32 * lda * ES, k, 0, 0);
+        for (uint32_t i = 0; i < BM / LR; i++)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, FH_LDS3(base + (BN + i * LR) * ROW_BYTES), 16, a_off + i * LR * lda * ES, k, 0, 0);
     };
     v16f acc[TN][TM];
 #pragma unroll
@@ -77,16 +94,26 @@ void dense_gemm_kernel(const T* __restrict__ w, const T* __restrict__ a, uint32_
             return (v8f){lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
         }
     };
-    issue(0, 0);
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
+    // The next stage's tiles are in LDS (those of the stages after it may still be on their way), and every wave is done with this one's.
+    auto arrive = [&](bool last) {
+        if (NBUF > 2 && !last) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"((NBUF - 2) * LOADS) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+#pragma unroll
+    for (uint32_t st = 0; st < NBUF - 1; st++)
+        if (st < stages) issue(st, st);
+    arrive(stages < NBUF - 1);
+    uint32_t buf = 0;
     for (uint32_t st = 0; st < stages; st++) {
-        const uint32_t buf = st & 1;
-        if (st + 1 < stages) issue(st + 1, buf ^ 1);
+        const uint32_t ahead = st + NBUF - 1;
+        if (ahead < stages) issue(ahead, buf == 0 ? NBUF - 1 : buf - 1);
         const uint8_t* wb = dense_lds + buf * BUF + (wn * 32 * TN + lrow) * ROW_BYTES;
         const uint8_t* ab = dense_lds + buf * BUF + (BN + wm * 32 * TM + lrow) * ROW_BYTES;
 #pragma unroll
-        for (uint32_t kk = 0; kk < BK / 16; kk++) {
+        for (uint32_t k = 0; k < BK / 16 / KG; k++) {
+            const uint32_t kk = kg * (BK / 16 / KG) + k;
             typename Vec<T>::x8 fw[TN], fa[TM];
 #pragma unroll
             for (int i = 0; i < TN; i++) fw[i] = frag(wb + i * 32 * ROW_BYTES, kk);
@@ -97,22 +124,53 @@ void dense_gemm_kernel(const T* __restrict__ w, const T* __restrict__ a, uint32_
 #pragma unroll
                 for (int j = 0; j < TM; j++) acc[i][j] = mma32(fw[i], fa[j], acc[i][j]);
         }
-        __builtin_amdgcn_s_waitcnt(0);          // the next stage's tiles are in LDS
-        __syncthreads();
+        arrive(ahead >= stages);
+        buf = buf == NBUF - 1 ? 0 : buf + 1;
     }
+    // The tile goes through LDS, so that a row's neighbouring columns are written (and read) by neighbouring lanes; the waves that shared
+    // out the depth of a tile meet there.  The 16-byte piece c of row r sits at c ^ (r & 7): no bank conflicts either way.
+    constexpr int JP = dense_pass(WN, WM, KG, TN, TM);
+    constexpr uint32_t THREADS = 64 * WAVES, ROWS = 32 * JP * WM, PIECES = BN / 4, STEP = THREADS / PIECES, STEPS = ROWS / STEP, G = STEPS < 4 ? STEPS : 4;
+    static_assert(THREADS % PIECES == 0 && ROWS % STEP == 0 && STEPS % G == 0, "whole steps");
+    v4f* box = reinterpret_cast<v4f*>(dense_lds);
+    const uint32_t piece = tid % PIECES, n = n0 + 4 * piece;
+    const EpiCols<MODE> cols = n < N ? epilogue_cols<MODE>(e, n) : EpiCols<MODE>{};
 #pragma unroll
-    for (int j = 0; j < TM; j++) {
-        const uint32_t m = m0 + (wm * TM + j) * 32 + lrow;
-        if (m >= M) continue;
+    for (uint32_t p = 0; p < TM / JP; p++) {
+        if (p > 0) __syncthreads();
 #pragma unroll
         for (int i = 0; i < TN; i++)
 #pragma unroll
-            for (int g = 0; g < 4; g++) {
-                const uint32_t n = n0 + (wn * TN + i) * 32 + 8 * g + 4 * lh;
-                if (n >= N) continue;
-                const float v[4] = {acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
-                dense_epilogue<T, MODE>(e, m, n, N, v);
+            for (int j = 0; j < JP; j++)
+#pragma unroll
+                for (int g = 0; g < 4; g++) {
+                    const v16f& c = acc[i][p * JP + j];
+                    const uint32_t r = (wm * JP + j) * 32 + lrow, at = (wn * TN + i) * 8 + 2 * g + lh;
+                    box[(kg * ROWS + r) * PIECES + (at ^ (r & 7))] = (v4f){c[4 * g], c[4 * g + 1], c[4 * g + 2], c[4 * g + 3]};
+                }
+        __syncthreads();
+        if (n >= N) continue;
+#pragma unroll
+        for (uint32_t s0 = 0; s0 < STEPS; s0 += G) {
+            EpiRow<T, MODE> row[G];
+            uint32_t m[G];
+            v4f v[G];
+#pragma unroll
+            for (uint32_t s = 0; s < G; s++) {
+                const uint32_t r = (s0 + s) * STEP + tid / PIECES;
+                m[s] = m0 + ((r / (32 * JP)) * TM + p * JP) * 32 + r % (32 * JP);
+                if (m[s] < M) row[s] = epilogue_row<T, MODE>(e, m[s], n);
+                v[s] = box[r * PIECES + (piece ^ (r & 7))];
+#pragma unroll
+                for (int k = 1; k < KG; k++) v[s] += box[(k * ROWS + r) * PIECES + (piece ^ (r & 7))];
             }
+#pragma unroll
+            for (uint32_t s = 0; s < G; s++)
+                if (m[s] < M) {
+                    const float f[4] = {v[s][0], v[s][1], v[s][2], v[s][3]};
+                    dense_epilogue<T, MODE>(e, m[s], n, N, f, cols, row[s]);
+                }
+        }
     }
 }
 
@@ -305,13 +363,15 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(const T* __restrict__ 
 
 namespace {
 
-template <typename T, int TN, int TM, DenseEpi MODE>
+template <typename T, int WN, int WM, int KG, int TN, int TM, int NBUF, DenseEpi MODE>
 void go_gemm(const DenseWeight& w, const void* a, uint32_t lda, uint32_t M, const DenseEpiArgs& e, hipStream_t s) {
-    constexpr uint32_t lds = (64 * TN + 64 * TM) * ROW_BYTES * 2;
-    static const hipError_t lds_ok = hipFuncSetAttribute((const void*)dense_gemm_kernel<T, TN, TM, MODE>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    constexpr uint32_t BN = 32 * TN * WN, BM = 32 * TM * WM, stage = (BN + BM) * ROW_BYTES * NBUF, box = dense_box(WN, WM, KG, TN, dense_pass(WN, WM, KG, TN, TM)),
+                       lds = stage > box ? stage : box;
+    const auto kernel = dense_gemm_kernel<T, WN, WM, KG, TN, TM, NBUF, MODE>;
+    static const hipError_t lds_ok = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     (void)lds_ok;
-    const uint32_t tn = (w.N + 64 * TN - 1) / (64 * TN), tm = (M + 64 * TM - 1) / (64 * TM);
-    fh::launch(dense_gemm_kernel<T, TN, TM, MODE>, dim3(tn * tm), 256, lds, s, (const T*)w.p, (const T*)a, lda, M, w.N, w.K, tn, e);
+    const uint32_t tn = (w.N + BN - 1) / BN, tm = (M + BM - 1) / BM;
+    fh::launch(kernel, dim3(tn * tm), 64 * WN * WM * KG, lds, s, (const T*)w.p, (const T*)a, lda, M, w.N, w.K, tn, e);
 }
 
 template <typename T, int KS, DenseEpi MODE, DenseIn::Kind IN, int STEPS>
@@ -348,10 +408,28 @@ void go(const DenseWeight& w, const DenseIn& in, uint32_t M, const DenseEpiArgs&
     }
     const void* a = in.rows;
     const uint32_t lda = in.lda;
-    // the large tile when its tiles give most compute units work, else the small one
-    const uint64_t big = (uint64_t)((w.N + 127) / 128) * ((M + 127) / 128);
-    if (big >= 192) go_gemm<T, 2, 2, MODE>(w, a, lda, M, e, s);
-    else go_gemm<T, 1, 1, MODE>(w, a, lda, M, e, s);
+    auto tiles = [&](uint32_t bn, uint32_t bm) { return (uint64_t)((w.N + bn - 1) / bn) * ((M + bm - 1) / bm); };
+    constexpr uint64_t CUS = 256;
+    if constexpr (sizeof(T) == 2) {
+        // The largest tile that keeps the chip busy (us, 256 x 256 / 128 x 128 / 128 x 64 / 64 x 64):
+        // - 256 x 256, one workgroup a compute unit, if its last round is at least 0.8 full on average: 16384 x 2048 by 902 rows (256 tiles)
+        //   64.5 / 73.5 / 88 / 98, 6144 x 2048 by 2502 (240) 63.7 / 72 / 88 / 98, by 902 (96) 49 / 33.7 / 36.5 / 41.
+        // - 128 x 128, two workgroups a compute unit, from more than one on: 2048 x 2048 by 2502 (320) 50 / 32.8 / 36 / 39,
+        //   3072 x 576 by 2502 (480) 24 / 18.2 / 22 / 21; one on each, 16384 x 2048 by 200 (256): 48 / 31 / 25 / 28.
+        // - 64 x 64 where two a compute unit hold all of them: 2048 x 8192 by 902 (480) 157 / 83 / 49.7 / 48.0, 6144 x 2048 by 200 (384)
+        //   46 / 23.3 / 15.6 / 13.4.  Deep ones are a chain of stages: four buffers and a quarter of the depth for each wave against two buffers
+        //   and a quarter of the tile: 2048 x 8192 by 200 rows 34 / 61, 576 x 1536 by 200 9.1 / 9.7, but 576 x 576 by 2502 7.4 / 6.5.
+        const uint64_t t256 = tiles(256, 256), rounds = (t256 + CUS - 1) / CUS;
+        if (5 * t256 >= 4 * CUS * rounds) go_gemm<T, 4, 2, 1, 2, 4, 2, MODE>(w, a, lda, M, e, s);
+        else if (tiles(128, 128) > CUS) go_gemm<T, 2, 2, 1, 2, 2, 2, MODE>(w, a, lda, M, e, s);
+        else if (tiles(64, 64) > 2 * CUS) go_gemm<T, 2, 2, 2, 2, 1, 3, MODE>(w, a, lda, M, e, s);
+        else if (w.K >= 1024) go_gemm<T, 1, 1, 4, 2, 2, 4, MODE>(w, a, lda, M, e, s);
+        else go_gemm<T, 2, 2, 1, 1, 1, 2, MODE>(w, a, lda, M, e, s);
+    } else {
+        // 32-bit: bound by the matrix unit's rate; the large tile when its tiles give most compute units work
+        if (tiles(128, 128) >= 192) go_gemm<T, 2, 2, 1, 2, 2, 2, MODE>(w, a, lda, M, e, s);
+        else go_gemm<T, 2, 2, 1, 1, 1, 2, MODE>(w, a, lda, M, e, s);
+    }
 }
 
 template <typename T>

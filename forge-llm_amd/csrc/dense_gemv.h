@@ -87,7 +87,7 @@ __device__ __forceinline__ void gemv_body(const T* __restrict__ w, uint32_t N, u
             for (int i = 0; i < 4; i++)
                 if (part == 0) acc[i] += red[(wave + p) * 4 + i];
     }
-    if (part == 0 && lane == 0 && n0 < N) dense_epilogue<T, MODE>(e, 0, n0, N, acc);
+    if (part == 0 && lane == 0 && n0 < N) dense_epilogue<T, MODE>(e, 0, n0, N, acc, epilogue_cols<MODE>(e, n0), epilogue_row<T, MODE>(e, 0, n0));
 }
 
 // Depth split of an N-row matrix: as many waves per row group as it takes to have a few workgroups on every compute unit.

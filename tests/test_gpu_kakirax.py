@@ -389,6 +389,20 @@ def test_decode_prologues_past_their_registers(fh, ko, torch_gpu, tmp_path, widt
     m.close()
 
 
+@pytest.mark.parametrize("n,width,ff", [(1300, 320, 5000), (700, 1100, 1100)])
+def test_prompts_through_the_larger_tiles(fh, ko, torch_gpu, tmp_path, n, width, ff):
+    """Prompts whose products fill tiles of 256 x 256 (gate and up of 5000 by 1300 rows) and 64 x 64 with the depth shared out, with the
+    epilogues of a layer behind them."""
+    layers = [fh.synth.kakirax_gla(3, 24, 40, ff, tau=5.0), fh.synth.kakirax_attention(4, 2, 24, 16, ff)]
+    c = Case(fh, ko, tmp_path, fh.synth.kakirax_config(width, 61, layers, embedding_scale=3.0))
+    ids = c.ids(n)
+    want = c.oracle.forward(ids)[0]
+    for dtype in DTYPES:
+        m = c.model(dtype=dtype, max_seq=n)
+        check(m.prefill_logits(ids, np.arange(n)), want, dtype)
+        m.close()
+
+
 # ---- generation, loading, replay --------------------------------------------------------------------------------------------------
 
 def test_greedy_generation(get):

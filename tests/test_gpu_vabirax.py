@@ -319,6 +319,14 @@ def test_dense_products_of_one_row_at_the_edges_of_a_step(fh, torch_gpu, N, K):
     test_dense_products(fh, torch_gpu, 1, N, K)
 
 
+@pytest.mark.parametrize("M,N,K", [(1100, 12290, 64), (1020, 16128, 192), (2500, 2050, 64), (2497, 2052, 192), (130, 16300, 64), (65, 20000, 128), (150, 11905, 192),
+                                   (130, 16300, 256), (70, 131, 1024), (1000, 1100, 1088), (2, 260, 1152), (513, 1023, 1216), (600, 2047, 960)])
+def test_dense_products_of_every_tile(fh, torch_gpu, M, N, K):
+    """Tiles of 256 x 256, 128 x 128, 128 x 64 (three buffers) and 64 x 64 (two, or four with the depth shared out), with ragged last rows and
+    columns, columns that are and are not a multiple of 4, and fewer stages than buffers, as many, and more."""
+    test_dense_products(fh, torch_gpu, M, N, K)
+
+
 # ---- generation, loading, replay --------------------------------------------------------------------------------------------------
 
 def test_greedy_generation(get):
