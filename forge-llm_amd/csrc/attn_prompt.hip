@@ -10,26 +10,26 @@ namespace fh {
 
 constexpr float LOG2E = 1.4426950408889634f;
 
-// Workgroup = 8 waves = 128 consecutive queries of one head: four groups of 32, each shared by two waves that take one half
-// (32 keys) of every key tile and merge their (maximum, sum, output) at the end, which halves the longest chain of dependent
-// tile steps.  Keys and values stream through LDS in tiles of 64 (K row-major: the head's own part, the shared part; V transposed), the
+// Workgroup = 8 waves: 8 / KG groups of 32 consecutive queries of one head, each shared by KG waves that take 32 keys each of every tile
+// of 32 KG and merge their (maximum, sum, output) at the end, which cuts the longest chain of dependent tile steps to a KG-th.  Keys
+// and values stream through LDS (K row-major: the head's own part, the shared part; V transposed), the
 // next tile's loads in registers while this one is worked.  Both products are computed transposed (S^T = K Q^T, O^T = V^T P^T):
 // a lane owns one query, so the softmax statistics are per-lane scalars, and the exponentiated scores are already the second
 // product's operand.  Scores stay in the base-2 domain.
 // DQ >= dim + rot and DV >= vdim: the register tiles' sizes; columns past the real ones are zero.
-constexpr uint32_t LP_KT = 64, LP_QB = 128, LP_THREADS = 512;
-template <typename T, int DQ, int DV> constexpr uint32_t prompt_lds() {
-    const uint32_t tiles = (LP_KT * (DQ + 16 / sizeof(T)) + DV * (LP_KT + 8 / sizeof(T))) * sizeof(T), merge = 4 * 64 * 18 * 4;
+constexpr uint32_t LP_THREADS = 512;
+template <typename T, int DQ, int DV, int KG> constexpr uint32_t prompt_lds() {
+    const uint32_t tiles = (32 * KG * (DQ + 16 / sizeof(T)) + DV * (32 * KG + 8 / sizeof(T))) * sizeof(T), merge = 8 / KG * (KG - 1) * 64 * 18 * 4;
     return tiles > merge ? tiles : merge;
 }
 
-template <typename T, int DQ, int DV>
+template <typename T, int DQ, int DV, int KG>
 __global__ __launch_bounds__(LP_THREADS) __attribute__((amdgpu_waves_per_eu(2)))
 void attn_prompt_kernel(PromptAttn sh, const T* __restrict__ q, const T* __restrict__ kbuf, const T* __restrict__ vbuf, const T* __restrict__ shared,
                         const T* __restrict__ gate, T* __restrict__ out, uint32_t M, uint32_t base_pos) {
     typedef typename Vec<T>::x4 x4;
     typedef typename Vec<T>::x8 x8;
-    constexpr uint32_t KT = LP_KT, QB = LP_QB, NT = LP_THREADS, PAD = 16 / sizeof(T);
+    constexpr uint32_t KT = 32 * KG, QB = 32 * (8 / KG), NT = LP_THREADS, PAD = 16 / sizeof(T);
     constexpr uint32_t KS = DQ + PAD, VS = KT + 8 / sizeof(T);         // LDS row strides
     constexpr uint32_t NS = DQ / 16, ND = DV / 32;
     constexpr uint32_t KTOTAL = KT * DQ / 8, VTOTAL = (KT / 2) * (DV / 4);       // pieces of a tile
@@ -39,7 +39,7 @@ void attn_prompt_kernel(PromptAttn sh, const T* __restrict__ q, const T* __restr
     T* Vt = Ks + KT * KS;
 
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, lq = lane & 31, lh = lane >> 5;
-    const uint32_t qg = wave >> 1, kh = wave & 1;        // query group, half of every key tile
+    const uint32_t qg = wave / KG, kh = wave % KG;       // query group, 32 keys of every key tile
     // latest (longest) query tiles first
     const uint32_t head = blockIdx.x % sh.heads, ntq = gridDim.x / sh.heads;
     const uint32_t q0 = (ntq - 1 - blockIdx.x / sh.heads) * QB;
@@ -67,7 +67,8 @@ void attn_prompt_kernel(PromptAttn sh, const T* __restrict__ q, const T* __restr
     const uint32_t wave_min = wg_min + qg * 32, wave_max = base_pos + min(q0 + qg * 32 + 32, M) - 1;
     auto first_visible = [&](uint32_t p) { return p >= window ? p - window + 1 : 0u; };
     const uint32_t wave_lo = first_visible(wave_min), last_lo = first_visible(wave_max);
-    const uint32_t tile0 = first_visible(wg_min) / KT, ntiles = wg_max / KT + 1;
+    // tiles are counted from kv_lo, the first row that is there
+    const uint32_t tile0 = (first_visible(wg_min) - kv_lo) / KT, ntiles = (wg_max - kv_lo) / KT + 1;
 
     const uint32_t kst = sh.k_row, vst = sh.v_row, cst = sh.shared_row;
     x8 kreg[KP];
@@ -75,14 +76,14 @@ void attn_prompt_kernel(PromptAttn sh, const T* __restrict__ q, const T* __restr
     auto load_tile = [&](uint32_t kt) {
 #pragma unroll
         for (uint32_t i = 0; i < KP; i++) {
-            const uint32_t idx = tid + NT * i, key = idx / (DQ / 8), d = idx % (DQ / 8) * 8, t = kt * KT + key;
+            const uint32_t idx = tid + NT * i, key = idx / (DQ / 8), d = idx % (DQ / 8) * 8, t = kv_lo + kt * KT + key;
             if (idx >= KTOTAL || t >= total || d >= dq) kreg[i] = zero8<T>();
             else kreg[i] = d < sh.dim ? load8(kbuf + (size_t)(t - kv_lo) * kst + kvh * sh.dim + d)
                                       : load8(shared + (size_t)t * cst + (d - sh.dim));
         }
 #pragma unroll
         for (uint32_t i = 0; i < VP; i++) {
-            const uint32_t idx = tid + NT * i, kp = idx / (DV / 4), d = idx % (DV / 4) * 4, t = kt * KT + 2 * kp;
+            const uint32_t idx = tid + NT * i, kp = idx / (DV / 4), d = idx % (DV / 4) * 4, t = kv_lo + kt * KT + 2 * kp;
             const T* src = vbuf + (size_t)(t - kv_lo) * vst + kvh * sh.vdim + d;
             const bool in = idx < VTOTAL && d < sh.vdim;
             x4 z;
@@ -117,7 +118,7 @@ void attn_prompt_kernel(PromptAttn sh, const T* __restrict__ q, const T* __restr
         store_tile();
         __syncthreads();
         if (kt + 1 < ntiles) load_tile(kt + 1);
-        const uint32_t k0 = kt * KT + kh * 32;                                     // the wave's 32 keys
+        const uint32_t k0 = kv_lo + kt * KT + kh * 32;                                     // the wave's 32 keys
         if (!(wave_active && k0 <= wave_max && k0 + 32 > wave_lo)) continue;       // all in the wave's future, or before its windows
         // two accumulators: a product waits for the one before the last
         v16f sacc, sodd;
@@ -172,20 +173,29 @@ void attn_prompt_kernel(PromptAttn sh, const T* __restrict__ q, const T* __restr
             }
     }
 
-    // ---- merge: the odd wave of a group hands its state over through LDS, 32 output columns at a time
-    float* mg = reinterpret_cast<float*>(ap_lds) + (qg * 64 + lane) * 18;
+    // ---- merge: the first wave of a group takes the states of the others through LDS, 32 output columns at a time
+    float* mg = reinterpret_cast<float*>(ap_lds) + (qg * (KG - 1) * 64 + lane) * 18;      // wave k of the group: + (k - 1) 64 18
+    float* mine = mg + (kh - 1) * (64 * 18);
     __syncthreads();
-    if (kh) { mg[16] = m_run; mg[17] = l_run; }
+    if (kh) { mine[16] = m_run; mine[17] = l_run; }
     __syncthreads();
-    const float m1 = mg[16], l1 = mg[17], m_all = fmaxf(m_run, m1);       // finite for rows < M: a query sees itself
+    float m_all = m_run;                                                   // finite for rows < M: a query sees itself
+#pragma unroll
+    for (int k = 0; k < KG - 1; k++) m_all = fmaxf(m_all, mg[k * (64 * 18) + 16]);
     const float m_ref = m_all == -INFINITY ? 0.f : m_all;
-    const float a0 = __builtin_amdgcn_exp2f(m_run - m_ref), a1 = __builtin_amdgcn_exp2f(m1 - m_ref);
-    const float inv = 1.0f / lane_xor_add<32>(l_run * a0 + l1 * a1);
+    const float a0 = __builtin_amdgcn_exp2f(m_run - m_ref);
+    float a1[KG - 1], l_all = l_run * a0;
+#pragma unroll
+    for (int k = 0; k < KG - 1; k++) {
+        a1[k] = __builtin_amdgcn_exp2f(mg[k * (64 * 18) + 16] - m_ref);
+        l_all += mg[k * (64 * 18) + 17] * a1[k];
+    }
+    const float inv = 1.0f / lane_xor_add<32>(l_all);
 #pragma unroll
     for (uint32_t d = 0; d < ND; d++) {
         if (kh) {
 #pragma unroll
-            for (int r = 0; r < 16; r++) mg[r] = oacc[d][r];
+            for (int r = 0; r < 16; r++) mine[r] = oacc[d][r];
         }
         __syncthreads();
         if (!kh && qrow < M) {
@@ -197,7 +207,12 @@ void attn_prompt_kernel(PromptAttn sh, const T* __restrict__ q, const T* __restr
                 const x4 gt = *reinterpret_cast<const x4*>(gate + at);
                 float o[4];
 #pragma unroll
-                for (int i = 0; i < 4; i++) o[i] = (oacc[d][4 * g + i] * a0 + mg[4 * g + i] * a1) * inv * (float)gt[i];
+                for (int i = 0; i < 4; i++) {
+                    float v = oacc[d][4 * g + i] * a0;
+#pragma unroll
+                    for (int k = 0; k < KG - 1; k++) v = v + mg[k * (64 * 18) + 4 * g + i] * a1[k];
+                    o[i] = v * inv * (float)gt[i];
+                }
                 store4<T>(out + at, o[0], o[1], o[2], o[3]);
             }
         }
@@ -207,14 +222,28 @@ void attn_prompt_kernel(PromptAttn sh, const T* __restrict__ q, const T* __restr
 
 namespace {
 
+template <typename T, int DQ, int DV, int KG>
+void go_keys(const PromptAttn& a, uint32_t M, uint32_t base_pos, hipStream_t s) {
+    constexpr uint32_t lds = prompt_lds<T, DQ, DV, KG>(), QB = 32 * (8 / KG);
+    static_assert(lds <= 160 * 1024, "LDS of a compute unit");
+    static const hipError_t ok = hipFuncSetAttribute((const void*)attn_prompt_kernel<T, DQ, DV, KG>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    (void)ok;
+    fh::launch(attn_prompt_kernel<T, DQ, DV, KG>, dim3((M + QB - 1) / QB * a.heads), LP_THREADS, lds, s, a, (const T*)a.q, (const T*)a.k, (const T*)a.v,
+               (const T*)a.shared, (const T*)a.gate, (T*)a.out, M, base_pos);
+}
+
 template <typename T, int DQ, int DV>
 void go(const PromptAttn& a, uint32_t M, uint32_t base_pos, hipStream_t s) {
-    constexpr uint32_t lds = prompt_lds<T, DQ, DV>();
-    static_assert(lds <= 160 * 1024, "LDS of a compute unit");
-    static const hipError_t ok = hipFuncSetAttribute((const void*)attn_prompt_kernel<T, DQ, DV>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    (void)ok;
-    fh::launch(attn_prompt_kernel<T, DQ, DV>, dim3((M + LP_QB - 1) / LP_QB * a.heads), LP_THREADS, lds, s, a, (const T*)a.q, (const T*)a.k, (const T*)a.v,
-               (const T*)a.shared, (const T*)a.gate, (T*)a.out, M, base_pos);
+    // Bound by the chain of tile steps (about 1.8 us each), not by work, as long as the workgroups are few: four waves to a query group while
+    // the workgroups of 64 queries are at most one a compute unit (that is how many run at a time) under a window, which makes them all equally
+    // long, and at most two without, where the short ones fill the gaps.  Whole prompts in ms, two / four: 9 heads with a window
+    // of 1024, 902 tokens (135 workgroups) 2.77 / 2.48, 1500 (216) 3.24 / 2.87, 2502 (360) 3.60 / 3.58; 9 heads without, 2502 3.69 / 3.51; 32
+    // heads without, 902 (480) 4.06 / 4.03, 2502 (1280) 8.79 / 8.82.  Shapes whose tiles of 128 keys fill LDS stay with two.
+    constexpr uint32_t CUS = 256;
+    const uint32_t at_most = a.window && a.window < base_pos + M ? CUS : 2 * CUS;
+    if constexpr (prompt_lds<T, DQ, DV, 4>() <= 80 * 1024)
+        if ((uint64_t)((M + 63) / 64) * a.heads <= at_most) { go_keys<T, DQ, DV, 4>(a, M, base_pos, s); return; }
+    go_keys<T, DQ, DV, 2>(a, M, base_pos, s);
 }
 
 template <typename T>

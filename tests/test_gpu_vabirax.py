@@ -327,6 +327,23 @@ def test_dense_products_of_every_tile(fh, torch_gpu, M, N, K):
     test_dense_products(fh, torch_gpu, M, N, K)
 
 
+@pytest.mark.parametrize("heads,window", [(60, 100), (60, None), (3, 100), (3, 257)])
+def test_prompt_attention_forms(fh, vo, torch_gpu, tmp_path, heads, window):
+    """Two waves to a query group from 513 workgroups of 64 queries on (60 heads, 530 rows; 257 under a window), four below: portions that begin anywhere in a tile,
+    with keys kept from a multiple of 64 on that is none of a four-wave tile's 128 (row 448 for a portion from 600 on under a window of 100)."""
+    c = Case(fh, vo, tmp_path, fh.synth.vabirax_config(48, 61, [fh.synth.vabirax_layer(heads, 40, 8, 24, 32, 32, None, window)], embedding_scale=3.0))
+    ids = c.ids(765)
+    want = c.oracle.forward(ids)[0]
+    scale = np.sqrt((want ** 2).mean())
+    for dtype in DTYPES:
+        m = c.model(max_seq=765, dtype=dtype)
+        at = 0
+        for n in (70, 530, 65, 100):
+            check(m.prefill_logits(ids[at:at + n], np.arange(n)), want[at:at + n], dtype, scale)
+            at += n
+        m.close()
+
+
 # ---- generation, loading, replay --------------------------------------------------------------------------------------------------
 
 def test_greedy_generation(get):
