@@ -7,7 +7,7 @@
 // keeps the fragment reads free of bank conflicts.  Rows past the end of a matrix read as zero through the buffer descriptors' range
 // check.
 //
-// What bounds it (bfloat16; matrix unit busy 38 % of 16384 x 2048 by 902 rows before, LDS 16 %, no bank conflicts):
+// What bounds it (bfloat16; matrix unit busy 31 % of 16384 x 2048 by 902 rows before, LDS 16 %, no bank conflicts):
 // - The results.  A lane holds 16 bytes of a row and its neighbours other rows, so stores straight from the registers touched a cache
 //   line per lane: 6 us for a tile of 128 x 128, 24 us for 256 x 256.  They go through LDS and out by whole rows.
 // - Operands that several XCDs fetch.  Tiles are dealt out in groups of 8 rows of tiles, column by column, and an XCD works a run of
