@@ -70,6 +70,12 @@ Scratch g_twin;   // K-quant twins: block sums of the activations, or the activa
 
 inline size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 
+// Whether the byte ranges [a, a + na) and [b, b + nb) have a byte in common.
+bool overlap(const void* a, size_t na, const void* b, size_t nb) {
+    const uintptr_t pa = reinterpret_cast<uintptr_t>(a), pb = reinterpret_cast<uintptr_t>(b);
+    return pa < pb + nb && pb < pa + na;
+}
+
 bool valid_wdtype(uint32_t t) { return t == FORGE_HIP_Q8_0 || t == FORGE_HIP_Q4_0; }
 
 // Quantise x[M][K] into the shared scratch; returns pointers.
@@ -152,7 +158,14 @@ int32_t forge_hip_quantize_act(const float* x_dev, uint32_t M, uint32_t K, int8_
 int32_t forge_hip_gemv_q(const forge_hip_qweight* w, const float* x_dev, float* y_dev, void* stream) {
     FH_CHECK(w && x_dev && y_dev, "gemv_q: null pointer");
     FH_CHECK(gemv_k_supported(w->w.K), "gemv_q: K must be a multiple of 32, at most 16384");
-    if (w->w.kquant()) launch_gemv_kquant_act(w->w, x_dev, y_dev, (hipStream_t)stream);
+    if (overlap(x_dev, (size_t)w->w.K * 4, y_dev, (size_t)w->w.N * 4)) {
+        // workgroups that are done store y while others have yet to read x: all of x is quantised before the product starts
+        int8_t* q; uint16_t* sc;
+        int32_t rc = quantise_into_scratch(x_dev, 1, w->w.K, &q, &sc, (hipStream_t)stream);
+        if (rc) return rc;
+        if (w->w.kquant()) launch_gemv_kquant(w->w, q, sc, y_dev, false, (hipStream_t)stream);
+        else launch_gemv(w->w, q, sc, y_dev, false, GemvOrder::MatmulVec, (hipStream_t)stream);
+    } else if (w->w.kquant()) launch_gemv_kquant_act(w->w, x_dev, y_dev, (hipStream_t)stream);
     else launch_gemv_act(w->w, x_dev, y_dev, (hipStream_t)stream);
     FH_HIP(hipGetLastError());
     return FORGE_HIP_OK;

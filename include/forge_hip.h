@@ -248,7 +248,7 @@ int32_t forge_hip_quantize_act(const float* x_dev, uint32_t M, uint32_t K, int8_
                                void* stream);
 
 /* matmul_vec_q8_0_KxN / matmul_vec_q4_0_KxN (emit.rs:1926-2092, 2797-2958): y[N] = W x.
- * x_dev f32 [K], y_dev f32 [N].  For a Q4_K / Q6_K handle: matmul_vec_q4_k_KxN / matmul_vec_q6_k_KxN (emit.rs:3388-3490,
+ * x_dev f32 [K], y_dev f32 [N], which may overlap.  For a Q4_K / Q6_K handle: matmul_vec_q4_k_KxN / matmul_vec_q6_k_KxN (emit.rs:3388-3490,
  * 3622-3655; dots emit.rs:3035-3306, 3553-3612), bit-identical f32. */
 int32_t forge_hip_gemv_q(const forge_hip_qweight* w, const float* x_dev, float* y_dev, void* stream);
 

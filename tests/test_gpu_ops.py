@@ -284,6 +284,26 @@ def test_matmul_vec_quantises_like_the_quantiser(fh, torch_gpu, ty, K, N):
             close(one, rows, 1e-4, 1e-4 * float(np.abs(x[64:96]).max()))
 
 
+@pytest.mark.parametrize("ty", [Q8, Q4, 12, 14])
+@pytest.mark.parametrize("K,N", [(2048, 2048), (8192, 8192), (2048, 40000)])
+def test_matmul_vec_in_place(fh, torch_gpu, ty, K, N):
+    """A result that overlaps its vector (in place, begins inside it, ends inside it) has the bits of one that does not, also where
+    the matrix is several rounds of workgroups and the late ones would find results in the vector's place."""
+    import ctypes as C
+    torch = torch_gpu
+    raw = make_weight(fh, ty, N, K, K + N) if ty in (Q8, Q4) else random_superblocks(ty, N * (K // 256), K + N)
+    w = fh.ops.QWeight(ty, raw, K, N)
+    x = torch.from_numpy(fh.synth.normal(K, K, 1.0)).cuda()
+    want = fh.ops.matmul_vec_q(w, x).cpu().numpy()
+    for x_at, y_at in ((0, 0), (0, K - 1), (0, 5), (N - 4, 0), (N // 8 * 4, 1)):
+        buf = torch.zeros(K + N + 8, device="cuda")
+        buf[x_at:x_at + K] = x
+        fh.check(fh.lib().forge_hip_gemv_q(w._h, C.c_void_p(buf.data_ptr() + 4 * x_at), C.c_void_p(buf.data_ptr() + 4 * y_at), None))
+        torch.cuda.synchronize()
+        same_bits(buf[y_at:y_at + N].cpu().numpy(), want)
+    w.close()
+
+
 @pytest.mark.parametrize("wd", [Q8, Q4])
 @pytest.mark.parametrize("M,K,N", [(2502, 2048, 2048), (2502, 8192, 2048), (2100, 1152, 3072), (2502, 576, 2176)])
 def test_matmul_mat_k_ranges_of_leftover_tiles(fh, torch_gpu, wd, M, K, N):
