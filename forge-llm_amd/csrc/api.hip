@@ -70,12 +70,6 @@ Scratch g_twin;   // K-quant twins: block sums of the activations, or the activa
 
 inline size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 
-// Whether the byte ranges [a, a + na) and [b, b + nb) have a byte in common.
-bool overlap(const void* a, size_t na, const void* b, size_t nb) {
-    const uintptr_t pa = reinterpret_cast<uintptr_t>(a), pb = reinterpret_cast<uintptr_t>(b);
-    return pa < pb + nb && pb < pa + na;
-}
-
 bool valid_wdtype(uint32_t t) { return t == FORGE_HIP_Q8_0 || t == FORGE_HIP_Q4_0; }
 
 // Quantise x[M][K] into the shared scratch; returns pointers.

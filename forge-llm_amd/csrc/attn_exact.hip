@@ -649,7 +649,11 @@ void launch_attn_exact(bool batch_order, const float* q, uint32_t q_stride, cons
                        const uint32_t* pos_dev, uint32_t heads, uint32_t kv_heads, uint32_t hd, uint32_t window, uint32_t max_rows,
                        void* ws, hipStream_t s, uint32_t rows_at_most) {
     if (M == 0) return;
-    if (!batch_order && window == 0 && M == 1 && (pos_dev ? rows_at_most : base_pos + 1) <= attn_exact_one_launch_rows(hd)) {
+    // In one launch a head's result is stored while others still read: not over the cache, nor over the query unless it is in place (where
+    // it was, only its own head read).
+    const size_t result = out ? (size_t)heads * hd * 4 : 0, cache = (size_t)(base_pos + 1) * kv_heads * hd * 2;
+    const bool apart = (out == q || !overlap(out, result, q, (size_t)heads * hd * 4)) && !overlap(out, result, kc, cache) && !overlap(out, result, vc, cache);
+    if (!batch_order && window == 0 && M == 1 && apart && (pos_dev ? rows_at_most : base_pos + 1) <= attn_exact_one_launch_rows(hd)) {
 #define FH_XO(HD_) fh::launch(attn_exact_decode_one_kernel<HD_>, dim3(heads), XO_WAVES * 64, 0, s, q, kc, vc, out, oq, osc, base_pos, pos_dev, heads, kv_heads)
         if (hd == 64) FH_XO(64); else if (hd == 96) FH_XO(96); else FH_XO(128);
 #undef FH_XO

@@ -51,6 +51,12 @@ inline void launch(void (*kernel)(KArgs...), dim3 grid, dim3 block, size_t lds_b
         hipLaunchKernelGGL(kernel, grid, block, (uint32_t)lds_bytes, s, static_cast<KArgs>(args)...);
 }
 
+// Whether the byte ranges [a, a + na) and [b, b + nb) have a byte in common.
+inline bool overlap(const void* a, size_t na, const void* b, size_t nb) {
+    const uintptr_t pa = reinterpret_cast<uintptr_t>(a), pb = reinterpret_cast<uintptr_t>(b);
+    return pa < pb + nb && pb < pa + na;
+}
+
 // ---- device weight layout ----------------------------------------------------------------
 // GGUF interleaves a 2-byte scale with every 32 quants (34- or 18-byte blocks, 2-byte
 // aligned).  On upload each matrix is split into two planes so that every lane can issue

@@ -445,6 +445,29 @@ def test_attention_decode_order_faithful_at_the_launch_forms_edges(fh, oracle, t
     same_bits(got.cpu().numpy(), want)
 
 
+@pytest.mark.parametrize("heads,kv_heads,hd", [(300, 100, 64), (300, 3, 96), (300, 300, 128)])
+def test_attention_decode_order_faithful_over_its_inputs(fh, torch_gpu, heads, kv_heads, hd):
+    """A short context is one launch, in which heads that are done store their result while others still read: a result in place of the
+    query, over a part of it, or over a part of the cache has the bits of one with a buffer of its own."""
+    import ctypes as C
+    torch = torch_gpu
+    seq, n = 200, heads * hd
+    gen = torch.Generator().manual_seed(hd)
+    q = torch.randn(n, generator=gen).cuda()
+    k, v = ((torch.randn(seq, kv_heads * hd, generator=gen).half().view(torch.int16)).cuda() for _ in range(2))
+    want = fh.ops.attention_flash(q, k, v, seq, heads, kv_heads, hd, EXACT).cpu().numpy()
+    cache = seq * kv_heads * hd // 2                         # in floats
+    sizes = {"q": n, "k": cache, "v": cache}
+    for name, at in (("q", 0), ("q", hd), ("q", n - 1), ("k", 0), ("v", cache - hd), ("v", 0)):
+        buf = {key: torch.zeros(sizes[key] + n, device="cuda") for key in sizes}
+        for key, src in (("q", q), ("k", k), ("v", v)):
+            buf[key][:sizes[key]] = src.view(-1).view(torch.float32)
+        p = {key: C.c_void_p(buf[key].data_ptr()) for key in buf}
+        fh.check(fh.lib().forge_hip_attn_decode_f16kv(p["q"], p["k"], p["v"], C.c_void_p(buf[name].data_ptr() + 4 * at), seq, heads, kv_heads, hd, EXACT, None))
+        torch.cuda.synchronize()
+        same_bits(buf[name][at:at + n].cpu().numpy(), want)
+
+
 @pytest.mark.parametrize("heads,kv_heads,hd", [(32, 8, 64), (9, 3, 64), (32, 32, 96), (24, 8, 128)])
 @pytest.mark.parametrize("seq,page_rows", [(1, 16), (70, 16), (900, 64), (2250, 16), (2250, 256), (8192, 128), (777, 1)])
 def test_attention_decode_paged_cache(fh, oracle, torch_gpu, heads, kv_heads, hd, seq, page_rows):
