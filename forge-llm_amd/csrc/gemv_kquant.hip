@@ -539,8 +539,11 @@ void launch_kq_one(const QWeight& w, const KqIn& in, float* y, bool accumulate, 
     if (w.N == 0) return;
     const uint32_t nblk = w.K / 32;
     // rows a wave keeps in flight: four when that still leaves every CU several workgroups
-    const int rw = w.N >= 16384 ? 4 : w.N >= 4096 ? 2 : 1;
-    const size_t lds = (size_t)w.K + (size_t)nblk * 8 + (size_t)W * rw * prod_stride(nblk) * 4;
+    int rw = w.N >= 16384 ? 4 : w.N >= 4096 ? 2 : 1;
+    auto lds_bytes = [&] { return (size_t)w.K + (size_t)nblk * 8 + (size_t)W * rw * prod_stride(nblk) * 4; };
+    // and while codes, scales and products fit the LDS that a launch may ask for (eight waves: fewer rows from K = 12544 on)
+    while (rw > 1 && lds_bytes() > 64 * 1024) rw /= 2;
+    const size_t lds = lds_bytes();
     uint32_t grid = (w.N + W * rw - 1) / (W * rw);
     if (grid > 256 * 8) grid = 256 * 8;
     const uint8_t* meta = reinterpret_cast<const uint8_t*>(w.scales);

@@ -284,6 +284,18 @@ def test_matmul_vec_quantises_like_the_quantiser(fh, torch_gpu, ty, K, N):
             close(one, rows, 1e-4, 1e-4 * float(np.abs(x[64:96]).max()))
 
 
+@pytest.mark.parametrize("ty", [12, 14])
+@pytest.mark.parametrize("K,N", [(12288, 16384), (12544, 16384), (12544, 16400), (16384, 16387)])
+def test_matmul_vec_kquant_deep_and_wide(fh, torch_gpu, ty, K, N):
+    """Depths whose codes, scales and products of four rows a wave would take more than 64 KB of LDS, and the last that do not: the bits
+    of the rows product."""
+    torch = torch_gpu
+    w = fh.ops.QWeight(ty, np.tile(random_superblocks(ty, 1024 * (K // 256), K + N), N // 1024 + 1)[:N * (K // 256) * {12: 144, 14: 210}[ty]], K, N)
+    x = torch.from_numpy(fh.synth.normal(K, K, 1.0)).cuda()
+    same_bits(fh.ops.matmul_vec_q(w, x).cpu().numpy(), fh.ops.matmul_mat_q(w, x[None], EXACT).cpu().numpy()[0])
+    w.close()
+
+
 @pytest.mark.parametrize("ty", [Q8, Q4, 12, 14])
 @pytest.mark.parametrize("K,N", [(2048, 2048), (8192, 8192), (2048, 40000)])
 def test_matmul_vec_in_place(fh, torch_gpu, ty, K, N):
