@@ -72,11 +72,20 @@ inline size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 
 bool valid_wdtype(uint32_t t) { return t == FORGE_HIP_Q8_0 || t == FORGE_HIP_Q4_0; }
 
+size_t act_bytes(uint32_t M, uint32_t K) { return align256((size_t)M * K) + (size_t)M * (K / 32) * 2; }
+
+// Whether one quantised row of K can be put into the shared scratch now: the area is large enough, or the stream is not being captured (which
+// forbids the allocation).
+bool scratch_at_hand(uint32_t K, hipStream_t s) {
+    if (act_bytes(1, K) <= g_act.capacity()) return true;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(s, &st) == hipSuccess && st == hipStreamCaptureStatusNone;
+}
+
 // Quantise x[M][K] into the shared scratch; returns pointers.
 int32_t quantise_into_scratch(const float* x, uint32_t M, uint32_t K, int8_t** q, uint16_t** sc, hipStream_t s, bool neg_odd = false) {
     const size_t qbytes = align256((size_t)M * K);
-    const size_t sbytes = (size_t)M * (K / 32) * 2;
-    int32_t rc = g_act.reserve(qbytes + sbytes);
+    int32_t rc = g_act.reserve(act_bytes(M, K));
     if (rc) return rc;
     *q = reinterpret_cast<int8_t*>(g_act.ptr());
     *sc = reinterpret_cast<uint16_t*>(reinterpret_cast<uint8_t*>(g_act.ptr()) + qbytes);
@@ -152,15 +161,20 @@ int32_t forge_hip_quantize_act(const float* x_dev, uint32_t M, uint32_t K, int8_
 int32_t forge_hip_gemv_q(const forge_hip_qweight* w, const float* x_dev, float* y_dev, void* stream) {
     FH_CHECK(w && x_dev && y_dev, "gemv_q: null pointer");
     FH_CHECK(gemv_k_supported(w->w.K), "gemv_q: K must be a multiple of 32, at most 16384");
-    if (overlap(x_dev, (size_t)w->w.K * 4, y_dev, (size_t)w->w.N * 4)) {
-        // workgroups that are done store y while others have yet to read x: all of x is quantised before the product starts
+    hipStream_t s = (hipStream_t)stream;
+    const bool kq = w->w.kquant();
+    // in one launch, workgroups that are done store y while others have yet to read x
+    const bool apart = !overlap(x_dev, (size_t)w->w.K * 4, y_dev, (size_t)w->w.N * 4);
+    if (apart && ((kq ? gemv_kquant_act_pays(w->w) : gemv_act_pays(w->w)) || !scratch_at_hand(w->w.K, s))) {
+        if (kq) launch_gemv_kquant_act(w->w, x_dev, y_dev, s);
+        else launch_gemv_act(w->w, x_dev, y_dev, s);
+    } else {
         int8_t* q; uint16_t* sc;
-        int32_t rc = quantise_into_scratch(x_dev, 1, w->w.K, &q, &sc, (hipStream_t)stream);
+        int32_t rc = quantise_into_scratch(x_dev, 1, w->w.K, &q, &sc, s);
         if (rc) return rc;
-        if (w->w.kquant()) launch_gemv_kquant(w->w, q, sc, y_dev, false, (hipStream_t)stream);
-        else launch_gemv(w->w, q, sc, y_dev, false, GemvOrder::MatmulVec, (hipStream_t)stream);
-    } else if (w->w.kquant()) launch_gemv_kquant_act(w->w, x_dev, y_dev, (hipStream_t)stream);
-    else launch_gemv_act(w->w, x_dev, y_dev, (hipStream_t)stream);
+        if (kq) launch_gemv_kquant(w->w, q, sc, y_dev, false, s);
+        else launch_gemv(w->w, q, sc, y_dev, false, GemvOrder::MatmulVec, s);
+    }
     FH_HIP(hipGetLastError());
     return FORGE_HIP_OK;
 }

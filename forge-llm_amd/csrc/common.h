@@ -139,6 +139,7 @@ void launch_gemv(const QWeight& w, const int8_t* aq, const uint16_t* as, float* 
                  hipStream_t s);
 // y = W * quant(x): the activation quantiser in the prologue
 void launch_gemv_act(const QWeight& w, const float* x, float* y, hipStream_t s);
+bool gemv_act_pays(const QWeight& w);
 void launch_gemv_isums(const QWeight& w, const int8_t* aq, int32_t* out, hipStream_t s);
 bool gemv_k_supported(uint32_t K);
 // Fused decode variants (one launch instead of three): rms_norm + activation quantiser in the prologue.
@@ -165,6 +166,7 @@ void repack_kquant_host(uint32_t wdtype, const uint8_t* raw, uint32_t K, uint64_
 bool kquant_k_supported(uint32_t K);
 void launch_gemv_kquant(const QWeight& w, const int8_t* aq, const uint16_t* as, float* y, bool accumulate, hipStream_t s);
 void launch_gemv_kquant_act(const QWeight& w, const float* x, float* y, hipStream_t s);
+bool gemv_kquant_act_pays(const QWeight& w);
 // Up to three Q4_K / Q6_K matrices of the same K over one quantised vector in a single launch (q, k, v; gate, up).
 void launch_gemv_kquant_multi(const QWeight* const* w, float* const* y, uint32_t n, const int8_t* aq, const uint16_t* as, bool accumulate,
                               hipStream_t s);

@@ -30,6 +30,8 @@
 //   epilogue  Add: residual_add (emit.rs:455-459);  RopeKv: rope (emit.rs:508-528) on the q and k
 //             rows and the fp16 KV-cache write;  SiluQuant: silu_mul (emit.rs:380-386) of the gate
 //             and up rows of a fused [gate;up] matrix and the quantisation of the result.
+#include <algorithm>
+
 #include "common.h"
 #include "device_utils.h"
 #include "expf_ref.h"
@@ -420,8 +422,20 @@ void launch_one(GemvArgs a, hipStream_t s) {
     const uint32_t ngroups = EPI == Epi::SiluQuant ? (a.inter + 31) / 32 : ((a.N + a.rc - 1) / a.rc + WAVES - 1) / WAVES;
     uint32_t grid = ngroups;
     if (grid > 256 * 8) grid = 256 * 8;
+    constexpr auto kernel = gemv_kernel<Q4, NCH, (EPI == Epi::SiluQuant ? (RW > 4 ? 4 : RW) : RW), WAVES * KS, KS, PRO, EPI>;
     const size_t lds = EPI == Epi::Isums ? 0 : (size_t)WAVES * a.rc * prod_stride(nblk) * sizeof(float);
-    fh::launch(gemv_kernel<Q4, NCH, (EPI == Epi::SiluQuant ? (RW > 4 ? 4 : RW) : RW), WAVES * KS, KS, PRO, EPI>, grid, WAVES * KS * 64, lds + tail, s, a);
+    if (PRO == Pro::Act) {
+        // Every workgroup quantises the vector: no more of them than the chip holds at a time, each goes on to further groups of rows
+        // (us, as many as there are groups / this: 16384 -> 12288 Q8_0 97.7 / 56.0, 8192 -> 8192 Q4_0 17.9 / 14.5).
+        static const int by_registers = [] {
+            int n = 0;
+            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, (const void*)kernel, WAVES * KS * 64, 0) != hipSuccess) n = 0;
+            return n > 0 ? n : 8;
+        }();
+        const uint32_t per_cu = std::min<uint32_t>(by_registers, std::max<uint32_t>(1, (uint32_t)(160 * 1024 / (lds + tail))));
+        grid = std::min(grid, per_cu * 256);
+    }
+    fh::launch(kernel, grid, WAVES * KS * 64, lds + tail, s, a);
 }
 
 template <Pro PRO, Epi EPI>
@@ -495,6 +509,14 @@ void launch_gemv(const QWeight& w, const int8_t* aq, const uint16_t* as, float* 
     a.aq = aq; a.as = as; a.y = y;
     if (accumulate) dispatch<Pro::Quant, Epi::Add>(w.wdtype, a, s);
     else dispatch<Pro::Quant, Epi::Store>(w.wdtype, a, s);
+}
+
+// Where that is as fast as the quantiser's own launch and the product (us as graph nodes, two launches / one; a caller's loop gains 2 more):
+// 2048 -> 2048 Q8_0 5.6 / 4.2, 8192 -> 32000 52.6 / 49.4, 16384 -> 8192 60.1 / 42.9; Q4_0 8192 -> 2048 7.4 / 6.8, 8192 -> 8192 16.2 / 14.5.
+// Q4_0 has half the bytes per column to hide the quantising behind: not at the greatest depth (16384 -> 8192 26.1 / 27.3), nor where the
+// workgroups are one round of four waves (from 4096 rows on they do not share out the depth, up to 6144 the chip holds all: 8192 -> 6144 11.0 / 11.8).
+bool gemv_act_pays(const QWeight& w) {
+    return w.wdtype == FORGE_HIP_Q8_0 || w.K < 8192 || (w.K <= 12544 && !(w.N > 4096 && w.N <= 6144));
 }
 
 void launch_gemv_act(const QWeight& w, const float* x, float* y, hipStream_t s) {

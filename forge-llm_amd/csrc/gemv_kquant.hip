@@ -540,12 +540,23 @@ void launch_kq_one(const QWeight& w, const KqIn& in, float* y, bool accumulate, 
     const uint32_t nblk = w.K / 32;
     // rows a wave keeps in flight: four when that still leaves every CU several workgroups
     int rw = w.N >= 16384 ? 4 : w.N >= 4096 ? 2 : 1;
+    constexpr uint32_t CUS = 256;
+    if (W == 8) {
+        // Q6_K's wider pieces leave no registers for four; fewer rows also where the busiest CU then has at least a tenth less to do
+        // (N = 6144: 32 rows in steps of 16, 24 in steps of 8; 8192 -> 6144 Q4_K 12.8 against 10.7 us)
+        if (w.wdtype == FORGE_HIP_Q6_K && rw == 4) rw = 2;
+        auto most = [&](uint32_t r) { const uint32_t step = CUS * W * r; return (uint64_t)((w.N + step - 1) / step) * r; };
+        while (rw > 1 && 10 * most(rw / 2) <= 9 * most(rw)) rw /= 2;
+    }
     auto lds_bytes = [&] { return (size_t)w.K + (size_t)nblk * 8 + (size_t)W * rw * prod_stride(nblk) * 4; };
     // and while codes, scales and products fit the LDS that a launch may ask for (eight waves: fewer rows from K = 12544 on)
     while (rw > 1 && lds_bytes() > 64 * 1024) rw /= 2;
     const size_t lds = lds_bytes();
     uint32_t grid = (w.N + W * rw - 1) / (W * rw);
-    if (grid > 256 * 8) grid = 256 * 8;
+    if (grid > CUS * 8) grid = CUS * 8;
+    // Eight waves quantise their vector themselves: every workgroup past the two that a CU holds at a time would do it once more before its
+    // rows.  Two go on to further rows instead (3072 -> 65536 Q6_K 50.9 against 39.3 us, 8192 -> 32000 47.9 against 41.8).
+    if (W == 8 && grid > CUS * 2) grid = CUS * 2;
     const uint8_t* meta = reinterpret_cast<const uint8_t*>(w.scales);
     const int acc = accumulate ? 1 : 0;
 #define FH_KQ(Q6_, RW_) fh::launch(gemv_kquant_kernel<Q6_, RW_, PRO, W>, grid, W * 64, lds, s, w.qs, meta, in, y, w.K, w.N, acc)
@@ -583,10 +594,16 @@ void launch_gemv_kquant(const QWeight& w, const int8_t* aq, const uint16_t* as, 
     launch_kq_one<KqPro::Quantised>(w, KqIn{aq, as, nullptr, nullptr, 0.f}, y, accumulate, s);
 }
 
+// Where that is as fast as the quantiser's own launch and the product (us as graph nodes, two launches / one; a caller's loop gains 2 more):
+// 2048 -> 2048 Q4_K 5.0 / 3.9, 8192 -> 2048 7.8 / 6.8, 4096 -> 32000 18.3 / 16.2, 8192 -> 32000 Q6_K 42.2 / 41.8.  Not where a deep vector
+// meets more rows than one a wave but too few for each workgroup to go on to others (8192 -> 3072 Q6_K 10.0 / 10.8, 12544 -> 3072 Q4_K
+// 11.7 / 13.6), and not for the deepest (16384 -> 512 Q6_K 12.8 / 14.7, 16384 -> 8192 27.4 / 28.5).
+bool gemv_kquant_act_pays(const QWeight& w) { return w.K < 8192 || (w.K <= 12544 && !(w.N > 2048 && w.N < 4096)); }
+
 // The product with quantise(x), quantised by every workgroup for itself: no launch in front, the same bits.
 void launch_gemv_kquant_act(const QWeight& w, const float* x, float* y, hipStream_t s) {
     const KqIn in{nullptr, nullptr, x, nullptr, 0.f};
-    // a deep vector is quantised by eight waves in half as many workgroups (8192 -> 2048, Q4_K: 8.7 against 7.4 us with four)
+    // a deep vector is quantised by eight waves in half as many workgroups (8192 -> 2048 Q4_K: 8.4 us with four, 6.7 with eight)
     if (w.K > 2048) launch_kq_one<KqPro::Act, 8>(w, in, y, false, s);
     else launch_kq_one<KqPro::Act>(w, in, y, false, s);
 }

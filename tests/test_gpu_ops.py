@@ -297,6 +297,26 @@ def test_matmul_vec_kquant_deep_and_wide(fh, torch_gpu, ty, K, N):
 
 
 @pytest.mark.parametrize("ty", [Q8, Q4, 12, 14])
+@pytest.mark.parametrize("K,N", [(2304, 33001), (3072, 12290), (4096, 6143), (8192, 2049), (8192, 4095), (8192, 4097), (8192, 6145), (8192, 14001), (12800, 70), (12800, 9000)])
+def test_matmul_vec_routes_agree(fh, torch_gpu, ty, K, N):
+    """A vector is quantised by the product's workgroups (no more of them than the chip holds, so each goes on to further rows) or, past
+    the lines in depth and rows where that costs more, by a launch of its own.  A result that overlaps its vector always takes the second
+    way: both sides of each line have its bits."""
+    import ctypes as C
+    torch = torch_gpu
+    size = K // 32 * {Q8: 34, Q4: 18}[ty] if ty in (Q8, Q4) else K // 256 * {12: 144, 14: 210}[ty]
+    some = make_weight(fh, ty, 512, K, K + N).reshape(-1) if ty in (Q8, Q4) else random_superblocks(ty, 512 * (K // 256), K + N)
+    w = fh.ops.QWeight(ty, np.tile(some, N // 512 + 1)[:N * size], K, N)
+    buf = torch.zeros(K + N, device="cuda")
+    buf[:K] = torch.from_numpy(fh.synth.normal(K, K, 1.0)).cuda()
+    got = fh.ops.matmul_vec_q(w, buf[:K].clone()).cpu().numpy()
+    fh.check(fh.lib().forge_hip_gemv_q(w._h, C.c_void_p(buf.data_ptr()), C.c_void_p(buf.data_ptr()), None))
+    torch.cuda.synchronize()
+    same_bits(got, buf[:N].cpu().numpy())
+    w.close()
+
+
+@pytest.mark.parametrize("ty", [Q8, Q4, 12, 14])
 @pytest.mark.parametrize("K,N", [(2048, 2048), (8192, 8192), (2048, 40000)])
 def test_matmul_vec_in_place(fh, torch_gpu, ty, K, N):
     """A result that overlaps its vector (in place, begins inside it, ends inside it) has the bits of one that does not, also where
