@@ -237,8 +237,9 @@ void launch_rows(const FewArgs& a, hipStream_t s) {
 
 }  // namespace
 
+// 32-bit byte offsets, and a grid's second dimension ends at 65535 (2.1 million rows, which its estimate would take for narrow, shallow matrices).
 bool gemm_rows_supported(const QWeight& w, uint32_t M, bool silu) {
-    return (!silu || w.N % 64 == 0) && (uint64_t)M * w.K <= 0x7FFFFFFFull && (uint64_t)w.N * std::max<uint64_t>(w.qs_row_bytes(), w.K / 16) <= 0x7FFFFFFFull;
+    return (!silu || w.N % 64 == 0) && M <= 65535u * 32u && (uint64_t)M * w.K <= 0x7FFFFFFFull && (uint64_t)w.N * std::max<uint64_t>(w.qs_row_bytes(), w.K / 16) <= 0x7FFFFFFFull;
 }
 
 // Microseconds of a launch, for the choice between the kernels: 2.9 plus 2.9 per 2048 of depth while the tiles find a CU each (5.6 us

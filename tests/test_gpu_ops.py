@@ -284,6 +284,21 @@ def test_matmul_vec_quantises_like_the_quantiser(fh, torch_gpu, ty, K, N):
             close(one, rows, 1e-4, 1e-4 * float(np.abs(x[64:96]).max()))
 
 
+def test_matmul_mat_millions_of_rows(fh, torch_gpu):
+    """Rows on both sides of what a grid of 32-row tiles can count (65 535 tiles), in the narrow, shallow shape that such tiles suit best.  One block
+    of 32: where the sum S isum is made as S (12582912 +- isum), three roundings of at most 2^-24 S 13.1e6."""
+    torch = torch_gpu
+    K, N, line = 32, 5, 65535 * 32
+    raw = make_weight(fh, Q8, N, K, 3)
+    w = fh.ops.QWeight(Q8, raw, K, N)
+    w_s = torch.from_numpy(raw.reshape(N, 34)[:, :2].copy().view(np.float16)[:, 0].astype(np.float32)).cuda()
+    x = torch.randn(line + 33, K, generator=torch.Generator(device="cuda").manual_seed(1), device="cuda")
+    bound = 1.01 * 3.0 * 2.0 ** -24 * 13.1e6 * (x.abs().amax(1) / 127.0)[:, None] * w_s[None]
+    for M in (line, line + 1, line + 33):
+        assert bool(((fh.ops.matmul_mat_q(w, x[:M]) - fh.ops.matmul_mat_q(w, x[:M], EXACT)).abs() <= bound[:M]).all())
+    w.close()
+
+
 @pytest.mark.parametrize("ty", [12, 14])
 @pytest.mark.parametrize("K,N", [(12288, 16384), (12544, 16384), (12544, 16400), (16384, 16387)])
 def test_matmul_vec_kquant_deep_and_wide(fh, torch_gpu, ty, K, N):
