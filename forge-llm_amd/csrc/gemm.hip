@@ -698,10 +698,11 @@ void launch_gemm(const QWeight& w, const int8_t* aq, const uint16_t* as, uint32_
                 };
                 Plan best = plan(tm);
                 if (tm == 1) { const Plan other = plan(2); if (other.cost < best.cost) best = other; }
-                // Few rows: the kernel without stages (gemm_rows.hip) where its own estimate is lower.  The SiLU epilogue costs a tile
-                // here about 7 us more than the plan counts (64 rows of 2048 -> 16384: 29.5 us, 20.8 planned); the other kernel has the
-                // extra f32 term (MINT) not at all.
-                if (!mt_a && gemm_rows_supported(w, M, silu) && gemm_rows_cost(w, M) < best.cost + (silu ? 7.0 : 0.0)) {
+                // Few rows: the kernel without stages (gemm_rows.hip) where its own estimate is lower.  The plan counts neither what a tile
+                // takes before and after its stages, about 5 us (that of a cut tile is in the cost of meeting), nor the SiLU epilogue, about
+                // 4 us (1024 -> 8192 by 200 rows: 8.8 planned, 15.5 without and 19.0 with it).  The other kernel has no extra f32 term (MINT).
+                const double tiles_cost = best.cost + (best.items ? 0.0 : 5.0) + (silu ? 4.0 : 0.0);
+                if (!mt_a && gemm_rows_supported(w, M, silu) && gemm_rows_cost(w, M) < tiles_cost) {
                     launch_gemm_rows(w, aq, as, M, y, ldy, accumulate, s, silu_q, silu_sc);
                     return;
                 }

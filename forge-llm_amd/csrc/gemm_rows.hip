@@ -242,12 +242,14 @@ bool gemm_rows_supported(const QWeight& w, uint32_t M, bool silu) {
     return (!silu || w.N % 64 == 0) && M <= 65535u * 32u && (uint64_t)M * w.K <= 0x7FFFFFFFull && (uint64_t)w.N * std::max<uint64_t>(w.qs_row_bytes(), w.K / 16) <= 0x7FFFFFFFull;
 }
 
-// Microseconds of a launch, for the choice between the kernels: 2.9 plus 2.9 per 2048 of depth while the tiles find a CU each (5.6 us
-// measured for 32 rows of 2048 -> 2048, 12.5 for 8192 -> 2048), then 0.0148 per tile and 2048 of depth (2048 -> 8192: 10.3 us for 64
-// rows, 18.9 for 128, 31 for 200).  A SiLU workgroup works two tiles.
+// Microseconds of a launch, for the choice between the kernels.  Tiles come in rounds of one to a compute unit; a round takes 1.8 plus 2.7 per
+// 2048 of depth, or what its columns take from memory at 4.8 TB/s (with the quantiser, 1 / 2 / 3 / 4 rounds: K = 2048 9.9 / 14.2 / 18.8 / 23.5,
+// K = 4096 13 / 20 / 27 / 34, K = 8192 17.5 / 29 / 40 / 52).  1422 products of 2 to 1300 rows were timed both ways: the kernel that the estimates
+// prefer is within 3 % of the faster one in all but 9, within 8 % in all.  A SiLU workgroup works two tiles.
 double gemm_rows_cost(const QWeight& w, uint32_t M) {
-    const double depth = w.K / 2048.0, tiles = (double)((w.N + 31) / 32) * ((M + 31) / 32);
-    return 2.9 + depth * (2.9 + 0.0148 * std::max(0.0, tiles - 256.0));
+    const uint64_t tiles = (uint64_t)((w.N + 31) / 32) * ((M + 31) / 32);
+    const double columns = std::min<uint32_t>(w.N, 256 * 32), row_bytes = (double)w.qs_row_bytes() + w.K / 16;
+    return 2.0 + (double)((tiles + 255) / 256) * std::max(1.8 + 2.7 * w.K / 2048.0, columns * row_bytes / 4.8e6);
 }
 
 void launch_gemm_rows(const QWeight& w, const int8_t* aq, const uint16_t* as, uint32_t M, float* y, uint32_t ldy, bool accumulate, hipStream_t s,
