@@ -95,11 +95,18 @@ void dense_gemm_kernel(const T* __restrict__ w, const T* __restrict__ a, uint32_
         }
     };
     // The next stage's tiles are in LDS (those of the stages after it may still be on their way), and every wave is done with this one's.
+    // Two buffers: the compiler's own wait, around which it moves the next fragments' reads (32-bit 2048 x 8192 by 130 rows 161.8 us behind a wait
+    // in assembly, 159.0 this way; 576 x 576 by 64 with two norms 18.2 / 17.4).
     auto arrive = [&](bool last) {
-        if (NBUF > 2 && !last) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"((NBUF - 2) * LOADS) : "memory");
-        else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
+        if constexpr (NBUF == 2) {
+            __builtin_amdgcn_s_waitcnt(0);
+            __syncthreads();
+        } else {
+            if (!last) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"((NBUF - 2) * LOADS) : "memory");
+            else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+        }
     };
 #pragma unroll
     for (uint32_t st = 0; st < NBUF - 1; st++)
