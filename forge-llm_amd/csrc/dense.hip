@@ -10,8 +10,8 @@
 // What bounds it (bfloat16; matrix unit busy 31 % of 16384 x 2048 by 902 rows before, LDS 16 %, no bank conflicts):
 // - The results.  A lane holds 16 bytes of a row and its neighbours other rows, so stores straight from the registers touched a cache
 //   line per lane: 6 us for a tile of 128 x 128, 24 us for 256 x 256.  They go through LDS and out by whole rows.
-// - Operands that several XCDs fetch.  Tiles are dealt out in groups of 8 rows of tiles, column by column, and an XCD works a run of
-//   them: at 902 rows each XCD reads an eighth of the weights where it used to read all of them.
+// - Operands that several XCDs fetch.  Tiles are dealt out in groups of a few rows of tiles, column by column, and an XCD works a run of
+//   them: at 902 rows each XCD reads a part of the weights where it used to read all of them.
 // - The latency of a stage's loads where a compute unit has one workgroup: 3 or 4 buffers, and the depth shared out to the waves.
 // Times in us, 32-bit results, before / now: 16384 x 2048 by 902 rows 109 / 64.5 (940 TFLOP/s), 2048 x 8192 by 902 73.6 / 48.0,
 // 2048 x 2048 by 902 24.2 / 15.7, 6144 x 2048 by 902 49.3 / 33.7, 3072 x 576 by 2502 30.6 / 18.2, 576 x 576 by 2502 10.1 / 6.5.
@@ -53,8 +53,11 @@ void dense_gemm_kernel(const T* __restrict__ w, const T* __restrict__ a, uint32_
         const uint32_t total = gridDim.x, per = total / 8, x = tile % 8, i = tile / 8;
         if (i < per) tile = x * per + i;          // the last total % 8 tiles stay where they are
     }
-    // Tiles are counted in groups of GROUP rows of tiles, down the column first: the tiles that run at a time share both operands.
-    constexpr uint32_t GROUP = 8;
+    // Tiles are counted in groups of GROUP rows of tiles, down the column first: the tiles that run at a time share both operands.  512 rows
+    // of activations to a group, which an XCD's L2 holds beside the weights (products with a gate, bfloat16, us by 1 / 2 / 4 / 8 rows of tiles:
+    // 128 x 128 tiles 3392 x 2048 by 2502 rows 69.0 / 71.8 / 68.0 / 73.9, 6144 x 2048 by 1500 69.7 / 63.5 / 62.7 / 68.2; 128 x 64 tiles
+    // 6144 x 2048 by 902 55.8 / 42.3 / 40.9 / 40.9; 256 x 256 tiles 9216 x 3072 by 2502 187.9 / 183.5 / 184.3 / 195.1).
+    constexpr uint32_t GROUP = 512 / BM;
     const uint32_t tiles_m = (M + BM - 1) / BM, first = tile / (GROUP * tiles_n) * GROUP, rows = min(GROUP, tiles_m - first), in = tile - first * tiles_n;
     const uint32_t n0 = in / rows * BN, m0 = (first + in % rows) * BM;
     const uint32_t stages = K / BK;
