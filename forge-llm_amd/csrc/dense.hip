@@ -421,20 +421,25 @@ void go(const DenseWeight& w, const DenseIn& in, uint32_t M, const DenseEpiArgs&
     auto tiles = [&](uint32_t bn, uint32_t bm) { return (uint64_t)((w.N + bn - 1) / bn) * ((M + bm - 1) / bm); };
     constexpr uint64_t CUS = 256;
     if constexpr (sizeof(T) == 2) {
-        // The largest tile that keeps the chip busy (us, 256 x 256 / 128 x 128 / 128 x 64 / 64 x 64):
-        // - 256 x 256, one workgroup a compute unit, if its last round is at least 0.8 full on average: 16384 x 2048 by 902 rows (256 tiles)
-        //   64.5 / 73.5 / 88 / 98, 6144 x 2048 by 2502 (240) 63.7 / 72 / 88 / 98, by 902 (96) 49 / 33.7 / 36.5 / 41.
-        // - 128 x 128, two workgroups a compute unit, from more than one on: 2048 x 2048 by 2502 (320) 50 / 32.8 / 36 / 39,
-        //   3072 x 576 by 2502 (480) 24 / 18.2 / 22 / 21; one on each, 16384 x 2048 by 200 (256): 48 / 31 / 25 / 28.
-        // - 64 x 64 where two a compute unit hold all of them: 2048 x 8192 by 902 (480) 157 / 83 / 49.7 / 48.0, 6144 x 2048 by 200 (384)
-        //   46 / 23.3 / 15.6 / 13.4.  Deep ones are a chain of stages: four buffers and a quarter of the depth for each wave against two buffers
-        //   and a quarter of the tile: 2048 x 8192 by 200 rows 34 / 61, 576 x 1536 by 200 9.1 / 9.7, but 576 x 576 by 2502 7.4 / 6.5.
-        const uint64_t t256 = tiles(256, 256), rounds = (t256 + CUS - 1) / CUS;
-        if (5 * t256 >= 4 * CUS * rounds) go_gemm<T, 4, 2, 1, 2, 4, 2, MODE>(w, a, lda, M, e, s);
+        // The largest tile that keeps the chip busy (us, 256 x 256 / 128 x 128 / 128 x 64 / 64 x 64; gate: input products, up: gate and up,
+        // res: residual products of a prompt):
+        // - 256 x 256, one workgroup a compute unit, if its last round is at least 0.8 full on average: up 16384 x 2048 by 902 rows (256 tiles)
+        //   65.4 / 74.7 / 85 / 92, gate 6144 x 2048 by 2502 (240) 71.1 / 73.7 / 87 / 94, by 902 (96) 59.5 / 38.3 / 37.5 / 42.9.  Not for up to 128
+        //   rows, of which it would compute 256: 128256 x 2048 by 128 165 / 156 / 153 / 169, by 200 175 / 195 / 217 / 253.
+        // - 128 x 128, two workgroups a compute unit, from more than one on: res 2048 x 2048 by 2502 (320) 54 / 35.0 / 37.4 / 39.9, up
+        //   3072 x 576 by 2502 (480) 26.7 / 17.6 / 18.7 / 19.0; one on each, 16384 x 2048 by 130 (256): 46 / 29 / 21.7 / 20.9.
+        // - 64 x 64 where two a compute unit hold all of them: res 2048 x 8192 by 902 (480) 160 / 80 / 50.4 / 46.0, gate 6144 x 2048 by 300 (480)
+        //   57 / 31 / 17.4 / 16.5; and for up to 64 rows, of which the others would compute 128: 128256 x 2048 by 2 144 / 126 / 109 / 97, by 64
+        //   154 / 140 / 126 / 122, 49152 x 576 by 2 18.7 / 13.1 / 12.1 / 11.2.
+        //   Deep ones are a chain of stages: four buffers and a quarter of the depth for each wave against two buffers and a quarter of the tile:
+        //   res 2048 x 8192 by 130 rows 35.5 / 59.5, 2048 x 2048 by 520 14.5 / 18.4, but gate 1152 x 576 by 902 8.4 / 7.7.
+        const uint64_t t64 = tiles(64, 64), t256 = tiles(256, 256), rounds = (t256 + CUS - 1) / CUS;
+        const bool deep = w.K >= 1024, small = M <= 64 || t64 <= 2 * CUS;
+        if (small && deep) go_gemm<T, 1, 1, 4, 2, 2, 4, MODE>(w, a, lda, M, e, s);
+        else if (small) go_gemm<T, 2, 2, 1, 1, 1, 2, MODE>(w, a, lda, M, e, s);
+        else if (M > 128 && 5 * t256 >= 4 * CUS * rounds) go_gemm<T, 4, 2, 1, 2, 4, 2, MODE>(w, a, lda, M, e, s);
         else if (tiles(128, 128) > CUS) go_gemm<T, 2, 2, 1, 2, 2, 2, MODE>(w, a, lda, M, e, s);
-        else if (tiles(64, 64) > 2 * CUS) go_gemm<T, 2, 2, 2, 2, 1, 3, MODE>(w, a, lda, M, e, s);
-        else if (w.K >= 1024) go_gemm<T, 1, 1, 4, 2, 2, 4, MODE>(w, a, lda, M, e, s);
-        else go_gemm<T, 2, 2, 1, 1, 1, 2, MODE>(w, a, lda, M, e, s);
+        else go_gemm<T, 2, 2, 2, 2, 1, 3, MODE>(w, a, lda, M, e, s);
     } else {
         // 32-bit: bound by the matrix unit's rate; the large tile when its tiles give most compute units work
         if (tiles(128, 128) >= 192) go_gemm<T, 2, 2, 1, 2, 2, 2, MODE>(w, a, lda, M, e, s);

@@ -327,6 +327,21 @@ def test_dense_products_of_every_tile(fh, torch_gpu, M, N, K):
     test_dense_products(fh, torch_gpu, M, N, K)
 
 
+@pytest.mark.parametrize("M,N,K", [(130, 16300, 1024), (150, 11905, 1088), (64, 40001, 192), (65, 40001, 64), (2, 33000, 1024), (64, 33003, 1088), (128, 33002, 128),
+                                   (129, 33002, 64)])
+def test_dense_products_at_the_lines_between_tiles(fh, torch_gpu, M, N, K):
+    """Wide matrices by up to 64, up to 128 and more rows, and 128 x 64 tiles of deep ones.
+    A 32-bit sum of K products in any order is off by at most K 2^-24 times the sum of their magnitudes (one rounding an addition, one a product)."""
+    torch = torch_gpu
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    a, w = (torch.randn(r, K, generator=g, device="cuda").bfloat16() for r in (M, N))
+    y = torch.full((M, N), float("nan"), device="cuda")
+    fh.check(fh.lib().forge_hip_dense_matmul(fh.BF16, w.data_ptr(), a.data_ptr(), M, N, K, y.data_ptr(), None))
+    a, w = a.double(), w.double()
+    err, bound = (y.double() - a @ w.T).abs(), (K + 1) * 2.0 ** -24 * (a.abs() @ w.abs().T)
+    assert bool((err <= bound).all())
+
+
 @pytest.mark.parametrize("heads,window", [(60, 100), (60, None), (3, 100), (3, 257)])
 def test_prompt_attention_forms(fh, vo, torch_gpu, tmp_path, heads, window):
     """Two waves to a query group from 513 workgroups of 64 queries on (60 heads, 530 rows; 257 under a window), four below: portions that begin anywhere in a tile,
