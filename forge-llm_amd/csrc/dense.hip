@@ -432,9 +432,11 @@ void go(const DenseWeight& w, const DenseIn& in, uint32_t M, const DenseEpiArgs&
         //   57 / 31 / 17.4 / 16.5; and for up to 64 rows, of which the others would compute 128: 128256 x 2048 by 2 144 / 126 / 109 / 97, by 64
         //   154 / 140 / 126 / 122, 49152 x 576 by 2 18.7 / 13.1 / 12.1 / 11.2.
         //   Deep ones are a chain of stages: four buffers and a quarter of the depth for each wave against two buffers and a quarter of the tile:
-        //   res 2048 x 8192 by 130 rows 35.5 / 59.5, 2048 x 2048 by 520 14.5 / 18.4, but gate 1152 x 576 by 902 8.4 / 7.7.
+        //   res 2048 x 8192 by 130 rows 35.5 / 59.5, 2048 x 2048 by 520 14.5 / 18.4, but gate 1152 x 576 by 902 8.4 / 7.7.  The shallow form
+        //   has four and more to a compute unit: gate 928 x 576 by 2502 rows (600) 32 / 17 / 11.4 / 9.9, up 3072 x 576 by 1500 (1152)
+        //   24.6 / 15.7 / 14.9 / 13.8, but 2048 x 512 by 2502 (1280) 21 / 15.0 / 16.1 / 15.6.
         const uint64_t t64 = tiles(64, 64), t256 = tiles(256, 256), rounds = (t256 + CUS - 1) / CUS;
-        const bool deep = w.K >= 1024, small = M <= 64 || t64 <= 2 * CUS;
+        const bool deep = w.K >= 1024, small = M <= 64 || t64 <= 2 * CUS || (!deep && 2 * t64 <= 9 * CUS);
         if (small && deep) go_gemm<T, 1, 1, 4, 2, 2, 4, MODE>(w, a, lda, M, e, s);
         else if (small) go_gemm<T, 2, 2, 1, 1, 1, 2, MODE>(w, a, lda, M, e, s);
         else if (M > 128 && 5 * t256 >= 4 * CUS * rounds) go_gemm<T, 4, 2, 1, 2, 4, 2, MODE>(w, a, lda, M, e, s);
