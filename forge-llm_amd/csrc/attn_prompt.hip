@@ -238,11 +238,12 @@ void go(const PromptAttn& a, uint32_t M, uint32_t base_pos, hipStream_t s) {
     // the workgroups of 64 queries are at most one a compute unit (that is how many run at a time) under a window, which makes them all equally
     // long, and at most two without, where the short ones fill the gaps.  Whole prompts in ms, two / four: 9 heads with a window
     // of 1024, 902 tokens (135 workgroups) 2.77 / 2.48, 1500 (216) 3.24 / 2.87, 2502 (360) 3.60 / 3.58; 9 heads without, 2502 3.69 / 3.51; 32
-    // heads without, 902 (480) 4.06 / 4.03, 2502 (1280) 8.79 / 8.82.  Shapes whose tiles of 128 keys fill LDS stay with two.
+    // heads without, 902 (480) 4.06 / 4.03, 2502 (1280) 8.79 / 8.82.  Shapes whose tiles of 128 keys fill LDS stay with two, and so do up to 64 keys,
+    // one tile for two waves: four would only load and merge more (30 layers of 9 heads, 2 tokens 0.16 / 0.19 ms, 64 tokens 0.19 / 0.22).
     constexpr uint32_t CUS = 256;
     const uint32_t at_most = a.window && a.window < base_pos + M ? CUS : 2 * CUS;
     if constexpr (prompt_lds<T, DQ, DV, 4>() <= 80 * 1024)
-        if ((uint64_t)((M + 63) / 64) * a.heads <= at_most) { go_keys<T, DQ, DV, 4>(a, M, base_pos, s); return; }
+        if (base_pos + M > 64 && (uint64_t)((M + 63) / 64) * a.heads <= at_most) { go_keys<T, DQ, DV, 4>(a, M, base_pos, s); return; }
     go_keys<T, DQ, DV, 2>(a, M, base_pos, s);
 }
 
