@@ -62,6 +62,42 @@ def test_exact_mode_across_the_line_between_the_attention_forms(fh, oracle, torc
     gm.close()
 
 
+@pytest.mark.parametrize("heads,kv_heads,head_dim,line", [(4, 2, 64, 768), (4, 4, 96, 256), (4, 2, 128, 256)])
+def test_exact_mode_across_the_line_with_a_changing_penalty(fh, oracle, torch_gpu, heads, kv_heads, head_dim, line):
+    """Greedy steps across the line between the attention's forms with a repeat penalty: the graph of the form past the line is there before the
+    step that takes it, carries the penalty that holds then, and both are made again when the penalty (or the cache's layout) is set.  Tokens
+    and logits are the oracle's, whose logits the penalty is applied to on the host."""
+    cfg = fh.synth.tiny(wdtype=Q8, max_seq=1024, hidden=256, inter=512, layers=2, heads=heads, kv_heads=kv_heads, head_dim=head_dim, vocab=1000)
+    cfg["flags"] = EXACT
+    blob = fh.synth.make_weights_blob(cfg, seed=head_dim)
+    prompt = fh.synth.uniform_ids(15, line - 6, cfg["vocab"])
+    gm, om = fh.HipModel(cfg, blob), oracle.Model(cfg, blob, A, KV_F16)
+    for turn in range(2):
+        gm.reset()
+        gm.set_kv_pages(0)
+        om.reset()
+        tok, seen = oracle.argmax(om.prefill_batched(prompt)), list(prompt)
+        gm.forward_prefill_batch(prompt)
+        gm.set_repeat_penalty(1.0)
+        changes = {1: 1.3, 7: 1.7, 9: 1.0}
+        penalty = 1.0
+        for step in range(11):                                # the line lies between steps 5 and 6
+            if step in changes:
+                penalty = changes[step]
+                gm.set_repeat_penalty(penalty)
+            seen.append(tok)
+            want = om.forward(tok)
+            if step % 3 == 2:
+                same_bits(gm.forward(tok), want)
+                tok = oracle.argmax(want)
+            else:
+                fh.ops.apply_repeat_penalty(want, np.array(seen, np.uint32), penalty)
+                got = gm.forward_greedy(tok)
+                tok = oracle.argmax(want)
+                assert got == tok, (turn, step)
+    gm.close()
+
+
 @pytest.mark.parametrize("wd", [Q8, Q4])
 def test_tiny_model_exact_mode_is_bit_identical(fh, oracle, torch_gpu, wd):
     cfg = tiny_cfg(fh, wd, EXACT)
