@@ -82,8 +82,21 @@ struct Descending {
     std::vector<uint32_t> count;
     std::vector<Entry> order, spare;      // the sorted prefix, and room to sort in
     uint32_t floor = BUCKETS;             // buckets from here up are in `order`
-    Descending(const float* l_, uint64_t n_) : l(l_), n(n_), count(BUCKETS, 0u) {
+    // Few entries, of which a first batch of `want` would take most, are sorted at once: the histogram alone takes 15 to 25 us (50 entries with
+    // top_p 3.5 us against 29, 1000 with top_p 45 against 69, 300 with top_k 40 11 against 21; but 1000 with top_k 40 take 26 with it).
+    Descending(const float* l_, uint64_t n_, uint64_t want) : l(l_), n(n_) {
+        if (n <= want || n <= 384) {
+            order.resize(n);
+            for (uint64_t i = 0; i < n; i++) order[i] = {bits_of(l[i]) & 0x7FFFFFFFu, (uint32_t)i};
+            sort_from(0);
+            floor = 0;
+            return;
+        }
+        count.assign(BUCKETS, 0u);
         for (uint64_t i = 0; i < n; i++) count[(bits_of(l[i]) >> 16) & (BUCKETS - 1)]++;      // (-0.0 is a zero like the other)
+    }
+    void sort_from(size_t at) {
+        std::stable_sort(order.begin() + at, order.end(), [](const Entry& a, const Entry& b) { return a.bits > b.bits; });
     }
     // Appends a batch; false: everything is there already.
     bool extend(uint64_t want) {
@@ -98,10 +111,7 @@ struct Descending {
             if (k >= floor && k < above) order.push_back({b, (uint32_t)i});
         }
         // they came in index order: any stable sort by bits will do
-        if (m < 4096) {
-            std::stable_sort(order.begin() + at, order.end(), [](const Entry& a, const Entry& b) { return a.bits > b.bits; });
-            return true;
-        }
+        if (m < 4096) { sort_from(at); return true; }
         spare.resize(m);
         Entry *from = order.data() + at, *to = spare.data();
         for (int shift = 0; shift < 33; shift += 11) {
@@ -168,12 +178,12 @@ int32_t forge_hip_sample(float* logits_host, uint64_t n, float temperature, uint
         // Largest first, equal ones by index: what lies past the first top_k goes, and what follows once the sum so far (which takes every
         // entry, zeros included, and never falls) exceeds top_p -- the entry that crosses the threshold too (project.rs:535-540).
         try {
-            Descending d(l, n);
+            uint64_t batch = cut_k ? std::min<uint64_t>(top_k, 4096) : 1024;
+            Descending d(l, n, batch);
             const uint64_t most = cut_k ? top_k : n;
             uint64_t keep = 0;
             float cumsum = 0.0f;
             bool crossed = false;
-            uint64_t batch = cut_k ? std::min<uint64_t>(top_k, 4096) : 1024;
             while (!crossed && keep < most) {
                 if (keep == d.order.size()) {
                     if (!d.extend(batch)) break;

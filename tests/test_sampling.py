@@ -141,6 +141,13 @@ def test_cuts_at_the_edges_of_the_partial_order(fh, oracle, so, n, top_k, top_p,
         assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
 
 
+@pytest.mark.parametrize("n,top_k,top_p", [(2, 1, 0.9), (50, 0, 0.9), (384, 40, 0.95), (385, 40, 0.95), (1024, 0, 0.999), (1025, 0, 0.999)])
+@pytest.mark.parametrize("spread", [0.0, 0.3, 40.0])
+def test_cuts_of_few_entries(fh, oracle, so, n, top_k, top_p, spread):
+    """Up to 384 entries, or 1024 without top_k, are ordered at once and not batch by batch: both sides of those lines."""
+    test_cuts_at_the_edges_of_the_partial_order(fh, oracle, so, n, top_k, top_p, spread)
+
+
 def test_top_p_drops_the_entry_that_crosses_the_threshold(fh, oracle, so):
     """project.rs:535-540 zeroes every entry from the first whose running sum exceeds top_p, that entry included."""
     l = np.log(np.array([0.5, 0.3, 0.15, 0.05], np.float32))
