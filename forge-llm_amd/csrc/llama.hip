@@ -539,7 +539,9 @@ int32_t LlamaModel::resident_profile(float* stage_ms, uint32_t* stage_launches) 
 int32_t LlamaModel::decode_launches() const {
     if (pd) return (int32_t)pd_launches_per_step(pd);
     const bool exact = (cfg.flags & FORGE_HIP_FLAG_EXACT) != 0;
-    const int attn = exact ? 1 : 2;
+    // order-faithful: three where the step is spread over the chip (without a window, past the one-launch form's line)
+    const bool spread = exact && cfg.sliding_window == 0 && decode_form() != 0 && attn_exact_decode_workspace_bytes(cfg.heads, cfg.head_dim, cfg.max_seq) != 0;
+    const int attn = spread ? 3 : exact ? 1 : 2;
     if (mixed && mixed_plain_layers)
         return 1 + (int)cfg.layers * ((fuse_norm ? 1 : 3) + attn + 1 + (fuse_silu ? 1 : 3) + 1) + 4;
     if (mixed) {

@@ -62,6 +62,18 @@ def test_exact_mode_across_the_line_between_the_attention_forms(fh, oracle, torc
     gm.close()
 
 
+@pytest.mark.parametrize("flags,window,at", [(0, 0, 20), (EXACT, 0, 20), (EXACT, 0, 767), (EXACT, 0, 768), (EXACT, 100, 768)])
+def test_decode_launches_is_what_the_next_step_launches(fh, torch_gpu, monkeypatch, flags, window, at):
+    """On both sides of the line between the attention's forms, and for the forms that have none."""
+    monkeypatch.setenv("FORGE_HIP_PERSIST", "0")              # fast mode: the kernel sequence
+    cfg = dict(tiny_cfg(fh, Q8, flags), max_seq=1024, sliding_window=window)
+    gm = fh.HipModel(cfg, fh.synth.make_weights_blob(cfg, seed=2))
+    gm.forward_prefill_batch(fh.synth.uniform_ids(3, at, cfg["vocab"]))
+    want = gm.decode_launches
+    assert sum(n for _, n in gm.forward_profile(4).values()) == want
+    gm.close()
+
+
 @pytest.mark.parametrize("heads,kv_heads,head_dim,line", [(4, 2, 64, 768), (4, 4, 96, 256), (4, 2, 128, 256)])
 def test_exact_mode_across_the_line_with_a_changing_penalty(fh, oracle, torch_gpu, heads, kv_heads, head_dim, line):
     """Greedy steps across the line between the attention's forms with a repeat penalty: the graph of the form past the line is there before the
