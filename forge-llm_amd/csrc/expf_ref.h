@@ -24,6 +24,15 @@
 namespace fh {
 
 namespace expf_detail {
+// The numbers of the algorithm, for every form of it (sampling.cpp has one that works on four values at a time).
+constexpr double N = 32.0;
+constexpr double InvLn2N = 0x1.71547652b82fep+0 * N;
+constexpr double Shift = 0x1.8p+52;
+constexpr double C0 = 0x1.c6af84b912394p-5 / N / N / N;
+constexpr double C1 = 0x1.ebfce50fac4f3p-3 / N / N;
+constexpr double C2 = 0x1.62e42ff0c52d6p-1 / N;
+constexpr float Most = 0x1.62e42ep6f;          // log(2^128)
+constexpr float Least = -0x1.9fe368p6f;        // log(2^-150)
 FH_HD inline uint64_t tab(int i) {
     // asuint64(2^(i/32)) - (i << 47), i = 0..31
     constexpr uint64_t T[32] = {
@@ -57,15 +66,9 @@ FH_HD inline uint64_t double_as_u64(double d) {
 template <bool kFma, typename Lookup>
 FH_HD inline float expf_ref_with(float x, Lookup lookup) {
     using namespace expf_detail;
-    constexpr double N = 32.0;
-    constexpr double InvLn2N = 0x1.71547652b82fep+0 * N;
-    constexpr double Shift = 0x1.8p+52;
-    constexpr double C0 = 0x1.c6af84b912394p-5 / N / N / N;
-    constexpr double C1 = 0x1.ebfce50fac4f3p-3 / N / N;
-    constexpr double C2 = 0x1.62e42ff0c52d6p-1 / N;
     if (x != x) return x + x;
-    if (x > 0x1.62e42ep6f) return INFINITY;       // > log(2^128)
-    if (x < -0x1.9fe368p6f) return 0.0f;          // < log(2^-150); also -inf
+    if (x > Most) return INFINITY;
+    if (x < Least) return 0.0f;                   // also -inf
     const double xd = (double)x;
     double z = InvLn2N * xd;
     double kd = z + Shift;

@@ -4,8 +4,8 @@
 //
 // What bounds it: passes over the vocabulary on one core.  128 256 logits with top_p 0.9: 9.2 ms with a stable sort of every index
 // and a scalar exp, 0.71 ms here -- the order is worked out only down to where top_k or top_p cuts (a radix sort of the candidates), exp
-// runs four at a time, and the last two passes visit the entries that are left.  What remains is mostly the sequential sum of all
-// exponentials, one dependent addition per entry.
+// runs four at a time, and the last two passes visit the entries that are left.  What remains: the order down to the cut and its running
+// sum a good half, setting the rest to zero 15 %, the maximum and exp 10 % each, the sequential sum of all exponentials 5 %.
 #include <math.h>
 #include <string.h>
 
@@ -34,12 +34,11 @@ __attribute__((target("avx2,fma"))) void exp_avx2(float* l, uint64_t n, float sh
         uint64_t t[32];
         Table() { for (int i = 0; i < 32; i++) t[i] = fh::expf_detail::tab(i); }
     } table;
-    constexpr double N = 32.0;
-    const __m256d inv = _mm256_set1_pd(0x1.71547652b82fep+0 * N), round = _mm256_set1_pd(0x1.8p+52), one = _mm256_set1_pd(1.0);
-    const __m256d c0 = _mm256_set1_pd(0x1.c6af84b912394p-5 / N / N / N), c1 = _mm256_set1_pd(0x1.ebfce50fac4f3p-3 / N / N),
-                  c2 = _mm256_set1_pd(0x1.62e42ff0c52d6p-1 / N);
+    namespace ex = fh::expf_detail;
+    const __m256d inv = _mm256_set1_pd(ex::InvLn2N), round = _mm256_set1_pd(ex::Shift), one = _mm256_set1_pd(1.0);
+    const __m256d c0 = _mm256_set1_pd(ex::C0), c1 = _mm256_set1_pd(ex::C1), c2 = _mm256_set1_pd(ex::C2);
     const __m256i low5 = _mm256_set1_epi64x(31);
-    const __m128 sh = _mm_set1_ps(shift), least = _mm_set1_ps(-0x1.9fe368p6f), most = _mm_set1_ps(0x1.62e42ep6f), inf = _mm_set1_ps(INFINITY);
+    const __m128 sh = _mm_set1_ps(shift), least = _mm_set1_ps(ex::Least), most = _mm_set1_ps(ex::Most), inf = _mm_set1_ps(INFINITY);
     uint64_t i = 0;
     for (; i + 4 <= n; i += 4) {
         const __m128 x = _mm_sub_ps(_mm_loadu_ps(l + i), sh);
