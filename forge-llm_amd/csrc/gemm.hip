@@ -666,10 +666,10 @@ void launch_gemm(const QWeight& w, const int8_t* aq, const uint16_t* as, uint32_
             const uint64_t tiles64 = (uint64_t)((nc + BN - 1) / BN) * ((mc + 63) / 64);
             const bool small_tiles = tiles64 <= (uint64_t)cus && mc > 64;
             int tm = small_tiles ? 1 : 2;
-            // Fast mode with a workspace from the caller: tiles that fill the CUs a few times and a fraction have the tiles of
-            // the fraction cut along K, so that they spread over all CUs; a problem with fewer tiles than half the CUs is
-            // all fraction.  Which tile height then fills the CUs best is decided by a small cost model (microseconds per K
-            // stage of a workgroup that has a CU to itself, measured: 1.3 for a 128-row tile, 1.1 for a 64-row one).
+            // Fast mode: which tile height fills the CUs best is decided by a small cost model (microseconds per K stage of a
+            // workgroup that has a CU to itself, measured: 1.3 for a 128-row tile, 1.1 for a 64-row one).  With a workspace from
+            // the caller, tiles that fill the CUs a few times and a fraction have the tiles of the fraction cut along K, so that
+            // they spread over all CUs; a problem with fewer tiles than half the CUs is all fraction.
             GemmSplit fsp{};
             uint32_t items = 0;
             if (!exact && !isums && mc == M && nc == w.N) {
