@@ -13,8 +13,8 @@
 // - Operands that several XCDs fetch.  Tiles are dealt out in groups of a few rows of tiles, column by column, and an XCD works a run of
 //   them: at 902 rows each XCD reads a part of the weights where it used to read all of them.
 // - The latency of a stage's loads where a compute unit has one workgroup: 3 or 4 buffers, and the depth shared out to the waves.
-// Times in us, 32-bit results, before / now: 16384 x 2048 by 902 rows 109 / 64.5 (940 TFLOP/s), 2048 x 8192 by 902 73.6 / 48.0,
-// 2048 x 2048 by 902 24.2 / 15.7, 6144 x 2048 by 902 49.3 / 33.7, 3072 x 576 by 2502 30.6 / 18.2, 576 x 576 by 2502 10.1 / 6.5.
+// Times in us of a caller's loop, 32-bit results, before / now: 16384 x 2048 by 902 rows 110 / 66.5 (910 TFLOP/s), 2048 x 8192 by 902
+// 67.9 / 47.1, 2048 x 2048 by 902 22.9 / 15.3, 6144 x 2048 by 902 48.4 / 32.2, 3072 x 576 by 2502 29.5 / 17.7, 576 x 576 by 2502 9.3 / 7.2.
 // M = 1: dense_gemv.h.
 #include <hip/hip_runtime.h>
 
@@ -424,23 +424,25 @@ void go(const DenseWeight& w, const DenseIn& in, uint32_t M, const DenseEpiArgs&
         // The largest tile that keeps the chip busy (us, 256 x 256 / 128 x 128 / 128 x 64 / 64 x 64; gate: input products, up: gate and up,
         // res: residual products of a prompt):
         // - 256 x 256, one workgroup a compute unit, if its last round is at least 0.8 full on average: up 16384 x 2048 by 902 rows (256 tiles)
-        //   65.4 / 74.7 / 85 / 92, gate 6144 x 2048 by 2502 (240) 71.1 / 73.7 / 87 / 94, by 902 (96) 59.5 / 38.3 / 37.5 / 42.9.  Not for up to 128
-        //   rows, of which it would compute 256: 128256 x 2048 by 128 165 / 156 / 153 / 169, by 200 175 / 195 / 217 / 253.
-        // - 128 x 128, two workgroups a compute unit, from more than one on: res 2048 x 2048 by 2502 (320) 54 / 35.0 / 37.4 / 39.9, up
-        //   3072 x 576 by 2502 (480) 26.7 / 17.6 / 18.7 / 19.0; one on each, 16384 x 2048 by 130 (256): 46 / 29 / 21.7 / 20.9.
-        // - 64 x 64 where two a compute unit hold all of them: res 2048 x 8192 by 902 (480) 160 / 80 / 50.4 / 46.0, gate 6144 x 2048 by 300 (480)
-        //   57 / 31 / 17.4 / 16.5; and for up to 64 rows, of which the others would compute 128: 128256 x 2048 by 2 144 / 126 / 109 / 97, by 64
-        //   154 / 140 / 126 / 122, 49152 x 576 by 2 18.7 / 13.1 / 12.1 / 11.2.
+        //   66.0 / 70.6 / 83 / 92, gate 6144 x 2048 by 2502 (240) 70.1 / 70.5 / 85 / 92, by 902 (96) 59.2 / 35.1 / 37.3 / 42.9.  Not for up to 128
+        //   rows, of which it would compute 256: 128256 x 2048 by 128 148 / 138 / 148 / 164, by 200 162 / 182 / 211 / 243.
+        // - 128 x 128, two workgroups a compute unit, from more than one on: res 2048 x 2048 by 2502 (320) 54 / 31.4 / 36.9 / 39.8, up
+        //   3072 x 576 by 2502 (480) 25.7 / 16.3 / 19.2 / 18.8; one on each, 16384 x 2048 by 130 (256): 46 / 25.0 / 21.0 / 20.2.  Eight waves to a
+        //   tile: four, with two 32 x 32 tiles more each, do not cover the gate's exponentials and the stores (gate 3392 x 2048 by 2502 rows 62.0
+        //   with four, 57.1 with eight, res 2048 x 8192 by 2502 106.2 / 99.3, gate 9216 x 3072 by 2502 151.7 / 148.0).
+        // - 64 x 64 where two a compute unit hold all of them: res 2048 x 8192 by 902 (480) 159 / 76 / 49.7 / 46.6, gate 6144 x 2048 by 300 (480)
+        //   56 / 26 / 16.8 / 16.0; and for up to 64 rows, of which the others would compute 128: 128256 x 2048 by 2 118 / 103 / 96 / 91, by 64
+        //   135 / 122 / 117 / 119, 49152 x 576 by 2 16.6 / 11.0 / 11.0 / 9.9.
         //   Deep ones are a chain of stages: four buffers and a quarter of the depth for each wave against two buffers and a quarter of the tile:
-        //   res 2048 x 8192 by 130 rows 35.5 / 59.5, 2048 x 2048 by 520 14.5 / 18.4, but gate 1152 x 576 by 902 8.4 / 7.7.  The shallow form
-        //   has four and more to a compute unit: gate 928 x 576 by 2502 rows (600) 32 / 17 / 11.4 / 9.9, up 3072 x 576 by 1500 (1152)
-        //   24.6 / 15.7 / 14.9 / 13.8, but 2048 x 512 by 2502 (1280) 21 / 15.0 / 16.1 / 15.6.
+        //   res 2048 x 8192 by 130 rows 35.0 / 59.2, 2048 x 2048 by 520 14.3 / 18.1, but gate 1152 x 576 by 902 8.2 / 7.5.  The shallow form
+        //   wins up to four on a compute unit: gate 928 x 576 by 2502 rows (600) 33 / 12.9 / 10.7 / 9.2, up 3072 x 576 by 1344 (1008) - / 12.7 / 11.2 /
+        //   11.2, but gate 1728 x 576 by 2502 (1080) 33 / 14.9 / 17.0 / 15.6, up 3072 x 576 by 1500 (1152) 25 / 13.0 / 15.4 / 15.3.
         const uint64_t t64 = tiles(64, 64), t256 = tiles(256, 256), rounds = (t256 + CUS - 1) / CUS;
-        const bool deep = w.K >= 1024, small = M <= 64 || t64 <= 2 * CUS || (!deep && 2 * t64 <= 9 * CUS);
+        const bool deep = w.K >= 1024, small = M <= 64 || t64 <= 2 * CUS || (!deep && t64 <= 4 * CUS);
         if (small && deep) go_gemm<T, 1, 1, 4, 2, 2, 4, MODE>(w, a, lda, M, e, s);
         else if (small) go_gemm<T, 2, 2, 1, 1, 1, 2, MODE>(w, a, lda, M, e, s);
         else if (M > 128 && 5 * t256 >= 4 * CUS * rounds) go_gemm<T, 4, 2, 1, 2, 4, 2, MODE>(w, a, lda, M, e, s);
-        else if (tiles(128, 128) > CUS) go_gemm<T, 2, 2, 1, 2, 2, 2, MODE>(w, a, lda, M, e, s);
+        else if (tiles(128, 128) > CUS) go_gemm<T, 4, 2, 1, 1, 2, 2, MODE>(w, a, lda, M, e, s);
         else go_gemm<T, 2, 2, 2, 2, 1, 3, MODE>(w, a, lda, M, e, s);
     } else {
         // 32-bit: bound by the matrix unit's rate; the large tile when its tiles give most compute units work

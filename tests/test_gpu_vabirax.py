@@ -328,7 +328,7 @@ def test_dense_products_of_every_tile(fh, torch_gpu, M, N, K):
 
 
 @pytest.mark.parametrize("M,N,K", [(130, 16300, 1024), (150, 11905, 1088), (64, 40001, 192), (65, 40001, 64), (2, 33000, 1024), (64, 33003, 1088), (128, 33002, 128),
-                                   (129, 33002, 64), (2500, 1850, 64), (2500, 1860, 192)])
+                                   (129, 33002, 64), (2500, 1850, 64), (2500, 1860, 192), (2500, 1600, 128), (2500, 1602, 64)])
 def test_dense_products_at_the_lines_between_tiles(fh, torch_gpu, M, N, K):
     """Wide matrices by up to 64, up to 128 and more rows, the last product of the shallow 64 x 64 form, and 128 x 64 tiles of deep ones.
     A 32-bit sum of K products in any order is off by at most K 2^-24 times the sum of their magnitudes (one rounding an addition, one a product)."""
