@@ -58,7 +58,8 @@ void dense_gemm_kernel(const T* __restrict__ w, const T* __restrict__ a, uint32_
     // 128 x 128 tiles 3392 x 2048 by 2502 rows 69.0 / 71.8 / 68.0 / 73.9, 6144 x 2048 by 1500 69.7 / 63.5 / 62.7 / 68.2; 128 x 64 tiles
     // 6144 x 2048 by 902 55.8 / 42.3 / 40.9 / 40.9; 256 x 256 tiles 9216 x 3072 by 2502 187.9 / 183.5 / 184.3 / 195.1).
     constexpr uint32_t GROUP = 512 / BM;
-    const uint32_t tiles_m = (M + BM - 1) / BM, first = tile / (GROUP * tiles_n) * GROUP, rows = min(GROUP, tiles_m - first), in = tile - first * tiles_n;
+    // (One group is one division less ahead of the first loads: 32-bit [gate; up] 3072 x 576 by 65 rows 19.97 us with it, 19.58 without.)
+    const uint32_t tiles_m = (M + BM - 1) / BM, first = tiles_m <= GROUP ? 0u : tile / (GROUP * tiles_n) * GROUP, rows = min(GROUP, tiles_m - first), in = tile - first * tiles_n;
     const uint32_t n0 = in / rows * BN, m0 = (first + in % rows) * BM;
     const uint32_t stages = K / BK;
 
