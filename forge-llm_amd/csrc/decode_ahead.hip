@@ -1,0 +1,1082 @@
+// One decode token of a narrow model as ONE kernel whose waves hold their share of a layer's matrices in registers (model::forward, emit.rs:4029-4227).
+//
+// A step of a model of a few hundred channels is a chain of four short products and an attention per layer; neither bytes nor arithmetic bound it but what
+// lies between them.  As kernels a link of that chain is 4 to 6 us (a launch that does nothing takes 2.7); as phases of the kernel for wide models
+// (decode_persistent.hip) it is 5.  Here a layer of SmolLM2-135M takes 14 us: five hand-overs of 0.8 to 1.2, two norms of 1.1, attention 3.3, and the products.
+//   * A wave's rows of the four matrices are a few registers (a lane holds at most UQ + UO + UG + UD blocks of 32 weights), all requested while the attention
+//     is at work: no product waits for memory, and nothing that comes from far is on its way to a compute unit that waits for a vector.  (A compute unit's
+//     loads return in order: weights requested behind each product held the next hand-over up by 2 to 3 us.)
+//   * Eight waves hold weights, four fetch the vectors.  A wave forms and sums whole rows by itself; the workgroup's rows lie side by side and are handed over
+//     by ONE store.  (Element by element from eight waves a hand-over of 576 elements among 72 workgroups takes 1.9 us, by one store 1.2; among 144 workgroups 1.5, among 256
+//     1.8: hence no more workgroups than the rows need.)
+//   * A polling thread requests all its elements before it looks at one, without a condition around a load (behind which the compiler would wait for it).
+//   * Attention workgroups hold no weights: a head each, its cached rows requested a layer ahead.
+//   * Pointers come from a copy in LDS: a scalar load of a line that nobody has touched takes a microsecond.
+// Values travel between workgroups as tagged 8-byte elements (resident.h; every wait is bounded, as in decode_persistent.hip): a buffer is overwritten only by a
+// phase whose inputs transitively depend on every reader of what it held.
+//
+// The arithmetic is the reference's own order throughout (block products, row sums, norm, softmax over 64-key blocks, the C library's expf): bit-identical to
+// the order-faithful kernel sequence, so the kernel serves both modes.  Per token, SmolLM2-135M Q8_0, us: kernel sequence (order-faithful mode) / kernel for
+// wide models (fast mode) / this: 33 rows of context 781 / 880 / 426, 400 rows 837 / 878 / 489, 740 rows 907 / 876 / 587.
+#include <stddef.h>
+#include <string.h>
+
+#include <algorithm>
+#include <chrono>
+#include <memory>
+#include <vector>
+
+#include "common.h"
+#include "device_utils.h"
+#include "expf_ref.h"
+#include "gemv_order.h"
+#include "resident.h"
+
+namespace fh {
+
+namespace {
+
+constexpr uint32_t PA_POLL = 4, PA_COMP = 8, PA_WAVES = PA_POLL + PA_COMP, PA_THREADS = PA_WAVES * 64, PA_POLL_THREADS = PA_POLL * 64;
+constexpr uint32_t PA_B = 64;                 // FLASH_ATTN_BLOCK_SIZE, emit.rs:201; a wave takes one block of keys: at most PA_WAVES blocks
+constexpr uint32_t PA_MAX_ROWS = 8;           // rows of a product that one wave holds (not the lm_head)
+constexpr int PA_PN = 3;                      // elements a polling thread takes: vectors of up to 768
+constexpr uint32_t PA_SUM = 24, PA_SSQ = 12;  // a row's products, and an accumulator's elements of the norm, are read in groups of so many: LDS rows end in zeros up to there
+// blocks of 32 weights that a lane holds: q;k;v, o, gate;up, down, and each of two sets of the lm_head
+constexpr int UQ = 1, UO = 1, UG = 3, UD = 1, UL = 4;
+
+// magic: floor(2^32 / nblk) + 1; R: rows per wave; stride: words between two rows of products; prod: the first wave's area of them (LDS bytes)
+struct PaMat { uint32_t N, nblk, magic, R, stride, prod; };
+struct PaWeights { const uint8_t* qs; const uint16_t* ws; };
+struct PaLayer {
+    PaWeights w[4];                           // q;k;v, o, gate;up, down
+    const float* norm[2];
+    uint16_t* kc;
+    uint16_t* vc;
+};
+
+struct PaArgs {
+    PaMat m[5];                               // q;k;v, o, gate;up (N = 2 I; a workgroup holds 32 + 32 rows), down, lm_head
+    uint32_t L, H, I, QKS, KV, heads, kv_heads;
+    uint32_t G;                               // workgroups [0, G) hold the layers' matrices, the next `heads` a head each; all share the lm_head
+    float eps;
+    const PaLayer* layers;                    // [L + 1]: the last one's first norm is the final norm; its q;k;v is the first layer's (requested, not used)
+    PaWeights lm;
+    const float* embed;
+    const float* cos_t;
+    const float* sin_t;
+    // tagged exchange buffers
+    uint64_t* tx;      // [H]                residual stream
+    uint64_t* tq;      // [QKS]              rotated q
+    uint64_t* tkv;     // [2 KV]             this position's K row (rotated) and V row, fp16 bits
+    uint64_t* taq;     // [QKS/32][9]        attention output, a block of 32: int8 codes (4 per element), then the fp16 scale
+    uint64_t* taq2;    // [I/32][9]          silu(gate)*up, same format
+    uint64_t* tpart;   // [2 G]              per-workgroup argmax candidates
+    float* logits;
+    uint32_t* state;   // [0] position  [1] token  [2] next token  [3] abort flag  [4] number of the step that counted its token
+    uint32_t* counts;
+    float penalty;
+    uint32_t tag_base, spin_limit, token, step_seq;
+    unsigned long long* host_out;             // host-mapped {launch number, next token}: written last, or null
+    uint32_t host_seq;
+    unsigned long long* stamps;               // optional: wall clock at the start of every phase (workgroup 0)
+    uint32_t off_as, off_xs, off_out, off_nw, off_silu, off_prod, off_layers, off_attn, prod_words, lds_words, xstride;      // LDS byte offsets (activation codes at 0)
+};
+
+// A uniform base and a lane's 32-bit offset in bytes.
+template <typename T>
+__device__ __forceinline__ T pa_at(const void* base, uint32_t off) { return ldg(reinterpret_cast<const T*>(static_cast<const uint8_t*>(base) + off)); }
+
+// Pointers of a layer, from their copy in LDS (a scalar load of a line that nobody has touched takes a microsecond).
+template <typename T>
+__device__ __forceinline__ T pa_lds_ptr(const T& p) {
+    const uint64_t v = *reinterpret_cast<const uint64_t*>(&p);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v), hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
+    return reinterpret_cast<T>(((uint64_t)hi << 32) | lo);
+}
+__device__ __forceinline__ PaWeights pa_lds_ptr(const PaWeights& w) { return PaWeights{pa_lds_ptr(w.qs), pa_lds_ptr(w.ws)}; }
+
+struct PaCtx {
+    uint32_t tid, lane, wave, wg, G, spin_limit;
+    uint32_t* sh_abort;      // LDS
+    uint32_t* abort_flag;    // global
+};
+
+__host__ __device__ constexpr uint32_t pa_up(uint32_t v, uint32_t m) { return (v + m - 1) / m * m; }
+
+// N elements a thread takes, re-read together until all carry their tags; bounded.  Every load of a round trip is issued before any is looked at, and
+// without a condition: a branch around one of them would put a wait behind it.  (A thread without an element of its own takes one that another has.)
+template <int N, typename Addr, typename Tag>
+__device__ __forceinline__ void pa_poll(Addr addr, Tag tag, uint32_t* out, const PaCtx& cx) {
+    uint64_t w[N];
+    uint32_t spins = 0;
+    for (;;) {
+#pragma unroll
+        for (int i = 0; i < N; i++) w[i] = ldc64(addr(i));
+        uint32_t off = 0;
+#pragma unroll
+        for (int i = 0; i < N; i++) off |= (uint32_t)(w[i] >> 32) ^ tag(i);
+        if (!off) break;
+        ++spins;
+        if (spins > cx.spin_limit ||
+            ((spins & 1023u) == 0 && __hip_atomic_load(cx.abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
+            *cx.sh_abort = 1;
+            __hip_atomic_store(cx.abort_flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            break;
+        }
+        __builtin_amdgcn_s_sleep(1);
+    }
+#pragma unroll
+    for (int i = 0; i < N; i++) out[i] = (uint32_t)w[i];
+}
+
+// A wave's blocks of a matrix: n of them, row after row; from block `seg` on they lie `jump` blocks further (the up rows of gate;up).
+struct PaTask { uint32_t base, n, seg, jump; };
+__device__ __forceinline__ uint32_t pa_sgpr(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
+__device__ __forceinline__ uint32_t pa_rows(const PaMat& m, uint32_t wv) { return wv * m.R < m.N ? min(m.R, m.N - wv * m.R) : 0u; }
+__device__ __forceinline__ PaTask pa_task(const PaMat& m, uint32_t wv) {
+    const uint32_t rows = pa_rows(m, wv);
+    return PaTask{rows ? wv * m.R * m.nblk : 0u, rows * m.nblk, 0xFFFFFFFFu, 0u};
+}
+
+// Lane l of round j holds block 64 j + l (Q4_0), or halves of two blocks with Q8_0: of blocks 64 j + l / 2 and 64 j + 32 + l / 2 the half
+// l & 1, so that a load covers consecutive bytes; the sums of both halves meet by a move between neighbours.
+template <int U, bool Q4> struct PaSet { int4 v[Q4 ? U : 2 * U]; uint32_t s[U]; };
+template <bool Q4>
+__device__ __forceinline__ uint32_t pa_own(uint32_t j, uint32_t lane) { return Q4 ? 64 * j + lane : 64 * j + 32 * (lane & 1u) + (lane >> 1); }
+
+template <int U, bool Q4>
+__device__ __forceinline__ void pa_load(PaSet<U, Q4>& w, const PaWeights& mat, const PaTask& t, uint32_t lane) {
+    asm volatile("" : "+v"(lane));           // the addresses are worked out here: kept from layer to layer they would not fit the registers
+    // Blocks past the last one re-read it, and a wave without rows reads the matrix's first block: with no condition around them the loads in flight are
+    // known where a product waits for its own.
+    const uint32_t last = max(t.n, 1u) - 1;
+    auto at = [&](uint32_t unit) {
+        const uint32_t u = min(unit, last);
+        return t.base + u + (u >= t.seg ? t.jump : 0u);
+    };
+#pragma unroll
+    for (int j = 0; j < U; j++) {
+        if (Q4) {
+            w.v[j] = pa_at<int4>(mat.qs, at(64 * j + lane) * 16);
+        } else {
+#pragma unroll
+            for (int h = 0; h < 2; h++) w.v[2 * j + h] = pa_at<int4>(mat.qs, at(64 * j + 32 * h + (lane >> 1)) * 32 + (lane & 1u) * 16);
+        }
+        w.s[j] = pa_at<uint16_t>(mat.ws, at(pa_own<Q4>(j, lane)) * 2);
+    }
+}
+
+// Where a lane finds its blocks' activations and leaves their products (LDS bytes), worked out ahead of the wait for the vector.
+template <int U, bool Q4> struct PaIdx { uint32_t a[Q4 ? U : 2 * U], s[U], p[U]; };
+template <int U, bool Q4>
+__device__ __forceinline__ PaIdx<U, Q4> pa_index(const PaTask& t, const PaMat& m, uint32_t off_as, uint32_t prod, uint32_t lane) {
+    PaIdx<U, Q4> x;
+#pragma unroll
+    for (int j = 0; j < U; j++) {
+        const uint32_t u = pa_own<Q4>(j, lane), r = __umulhi(u, m.magic), b = u - r * m.nblk;      // b is a block of the row whatever u is
+        x.s[j] = off_as + b * 4;
+        x.p[j] = u < t.n ? prod + (r * m.stride + b) * 4 : prod + (m.R * m.stride) * 4;             // past the last block: a word that nobody reads
+        if (Q4) {
+            x.a[j] = b * 32;
+        } else {
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const uint32_t uh = 64 * j + 32 * h + (lane >> 1);
+                x.a[2 * j + h] = (uh - __umulhi(uh, m.magic) * m.nblk) * 32 + (lane & 1u) * 16;
+            }
+        }
+        asm volatile("" : "+v"(x.s[j]), "+v"(x.p[j]));
+    }
+#pragma unroll
+    for (int i = 0; i < (Q4 ? U : 2 * U); i++) asm volatile("" : "+v"(x.a[i]));
+    return x;
+}
+
+// The blocks' products (a_s * w_s) * f32(isum), exact int32 block sums, parked in the wave's LDS.
+template <int U, bool Q4>
+__device__ __forceinline__ void pa_products(const PaSet<U, Q4>& w, const PaIdx<U, Q4>& x, uint32_t n, uint8_t* smem) {
+#pragma unroll
+    for (int j = 0; j < U; j++) {
+        if (64u * j >= n) break;
+        int isum;
+        if (Q4) {
+            const int4 a0 = *reinterpret_cast<const int4*>(smem + x.a[j]);
+            const int4 a1 = *reinterpret_cast<const int4*>(smem + x.a[j] + 16);
+            const int4 v = w.v[j];
+            const int k = 0x0F0F0F0F;
+            const int4 lo = make_int4(v.x & k, v.y & k, v.z & k, v.w & k);
+            const int4 hi = make_int4((v.x >> 4) & k, (v.y >> 4) & k, (v.z >> 4) & k, (v.w >> 4) & k);
+            const int4 ones = make_int4(0x01010101, 0x01010101, 0x01010101, 0x01010101);
+            isum = dot16(hi, a1, dot16(lo, a0, 0)) - 8 * dot16(ones, a1, dot16(ones, a0, 0));
+        } else {
+            int d[2];
+#pragma unroll
+            for (int h = 0; h < 2; h++) d[h] = dot16(w.v[2 * j + h], *reinterpret_cast<const int4*>(smem + x.a[2 * j + h]), 0);
+#pragma unroll
+            for (int h = 0; h < 2; h++) d[h] += lane_xor<1>(d[h]);
+            isum = (__lane_id() & 1u) ? d[1] : d[0];
+        }
+        *reinterpret_cast<float*>(smem + x.p[j]) = (*reinterpret_cast<const float*>(smem + x.s[j]) * f16_bits_to_f32((uint16_t)w.s[j])) * (float)isum;
+    }
+}
+
+// Ordered sums of the wave's rows: lane r < rows returns row r's.  Products and sums are one wave's LDS operations, which execute in order.
+// The zeros behind a row's products change nothing: a sum that starts at +0 is never -0.
+__device__ __forceinline__ float pa_row_sum(const PaMat& m, uint32_t rows, const uint8_t* area, uint32_t lane) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    float r = 0.f;
+    if (lane < rows) {
+        const float4* p = reinterpret_cast<const float4*>(area) + lane * (m.stride / 4);
+        constexpr int N4 = PA_SUM / 4;
+        float4 v[N4], w[N4];
+#pragma unroll
+        for (int i = 0; i < N4; i++) v[i] = p[i];
+        for (uint32_t b = PA_SUM; b < m.nblk; b += PA_SUM) {
+            p += N4;
+#pragma unroll
+            for (int i = 0; i < N4; i++) w[i] = p[i];
+#pragma unroll
+            for (int i = 0; i < N4; i++) { r = r + v[i].x; r = r + v[i].y; r = r + v[i].z; r = r + v[i].w; }
+#pragma unroll
+            for (int i = 0; i < N4; i++) v[i] = w[i];
+        }
+#pragma unroll
+        for (int i = 0; i < N4; i++) { r = r + v[i].x; r = r + v[i].y; r = r + v[i].z; r = r + v[i].w; }
+    }
+    return r;
+}
+
+// int8 codes of 32 values, one per lane of a half wave, and their fp16 scale (emit.rs:1410-1440), as the nine elements of a block: side by side and by one
+// instruction.  (Elements of one line that arrive one by one, from eight waves or with the scales elsewhere, cost the hand-over 0.7 us.)
+__device__ __forceinline__ void pa_store_block(float o, uint64_t* block, uint32_t tag, uint32_t lane, bool on) {
+    const float amax = half_wave_max(fabsf(o));
+    float inv;
+    const float sc = act_scale(amax, inv);
+    const uint32_t code = (uint32_t)quant_code(o * inv) & 0xFFu;
+    const uint32_t pk = quad_broadcast<0>(code) | (quad_broadcast<1>(code) << 8) | (quad_broadcast<2>(code) << 16) | (quad_broadcast<3>(code) << 24);
+    const uint32_t l = lane & 31u;            // lanes 0, 4, .. 28: codes; lane 1: the scale
+    if (on && ((l & 3u) == 0 || l == 1)) stc64(block + (l == 1 ? 8u : l / 4), tag, l == 1 ? (uint32_t)f32_to_f16_bits(sc) : pk);
+}
+
+// Vectors, fetched by the polling waves.  The residual row lies in LDS accumulator by accumulator of the norm: element e in row e % 16.
+__device__ __forceinline__ uint32_t pa_xs(uint32_t e, uint32_t xstride) { return (e & 15u) * xstride + (e >> 4); }
+__device__ __forceinline__ void pa_fetch_x(const uint64_t* tx, uint32_t tag, const float* emb, uint32_t H, float* xs, uint32_t xstride, const PaCtx& cx) {
+    if (!tag) {                               // the layer ahead of the first: the embedding row
+        for (uint32_t i = cx.tid; i < H; i += PA_POLL_THREADS) xs[pa_xs(i, xstride)] = ldg(emb + i);
+        return;
+    }
+    uint32_t v[PA_PN];
+    pa_poll<PA_PN>([&](int i) { return tx + min(cx.tid + i * PA_POLL_THREADS, H - 1); }, [&](int) { return tag; }, v, cx);
+#pragma unroll
+    for (int i = 0; i < PA_PN; i++)
+        if (cx.tid + i * PA_POLL_THREADS < H) xs[pa_xs(cx.tid + i * PA_POLL_THREADS, xstride)] = __uint_as_float(v[i]);
+}
+
+// A quantised vector and, with it, the residual of the rows that this workgroup holds: element res_row of x in lane r of the first wave
+// (res_tag 0: the embedding row; threads without a row: anything).
+__device__ __forceinline__ float pa_fetch_aq(const uint64_t* t, uint32_t tag, uint32_t K, uint32_t* aq, float* as, bool has_res, uint32_t res_row, const uint64_t* tx,
+                                             uint32_t res_tag, const float* emb, const PaCtx& cx) {
+    const uint32_t ne = K / 32 * 9;
+    float re = 0.f;
+    if (has_res && !res_tag) re = ldg(emb + res_row);
+    // the residual is the last slot, with a tag of its own (it was final before the vector's phase began)
+    const bool poll_res = has_res && res_tag != 0;
+    const uint64_t* pr = poll_res ? tx + res_row : t;
+    const uint32_t tr = poll_res ? res_tag : tag;
+    auto fetch = [&](auto n) {
+        constexpr int N = decltype(n)::value;
+        uint32_t v[N + 1];
+        pa_poll<N + 1>([&](int i) { return i < N ? t + min(cx.tid + i * PA_POLL_THREADS, ne - 1) : pr; }, [&](int i) { return i < N ? tag : tr; }, v, cx);
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            const uint32_t e = cx.tid + i * PA_POLL_THREADS, b = e / 9, k = e - b * 9;
+            if (e < ne) {
+                if (k < 8) aq[b * 8 + k] = v[i];
+                else as[b] = f16_bits_to_f32((uint16_t)v[i]);
+            }
+        }
+        if (poll_res) re = __uint_as_float(v[N]);
+    };
+    if (ne <= PA_POLL_THREADS) fetch(std::integral_constant<int, 1>{});
+    else if (ne <= 2 * PA_POLL_THREADS) fetch(std::integral_constant<int, 2>{});
+    else fetch(std::integral_constant<int, PA_PN>{});
+    return re;
+}
+
+// rms_norm (emit.rs:327-334, the 16-accumulator order of emit.rs:272-295) + activation quantiser, an element a thread.  Every wave forms the
+// sum of squares for itself, so there is no barrier between the sum and the codes; zeros behind an accumulator's elements change nothing.
+// nw: the norm weight of element tid.
+__device__ __forceinline__ void pa_norm_quant(const float* xs, uint32_t xstride, float nw, float eps, uint32_t H, uint8_t* smem, uint32_t off_as, const PaCtx& cx) {
+    const float x = cx.tid < H ? xs[pa_xs(cx.tid, xstride)] : 0.f;
+    const float4* p = reinterpret_cast<const float4*>(xs + (cx.lane & 15u) * xstride);
+    float s = 0.f;
+    constexpr int N4 = PA_SSQ / 4;
+    float4 v[N4], w[N4];
+#pragma unroll
+    for (int i = 0; i < N4; i++) v[i] = p[i];
+    for (uint32_t c = PA_SSQ; c < H / 16; c += PA_SSQ) {
+        p += N4;
+#pragma unroll
+        for (int i = 0; i < N4; i++) w[i] = p[i];
+#pragma unroll
+        for (int i = 0; i < N4; i++) { s = fmaf(v[i].x, v[i].x, s); s = fmaf(v[i].y, v[i].y, s); s = fmaf(v[i].z, v[i].z, s); s = fmaf(v[i].w, v[i].w, s); }
+#pragma unroll
+        for (int i = 0; i < N4; i++) v[i] = w[i];
+    }
+#pragma unroll
+    for (int i = 0; i < N4; i++) { s = fmaf(v[i].x, v[i].x, s); s = fmaf(v[i].y, v[i].y, s); s = fmaf(v[i].z, v[i].z, s); s = fmaf(v[i].w, v[i].w, s); }
+    // (p[i] + p[4+i]) + (p[8+i] + p[12+i]) for i = 0..3, then (t0 + t1) + (t2 + t3): a pair's sum is the same in both of its lanes
+    s = lane_xor_add<4>(s);
+    s = lane_xor_add<8>(s);
+    s = lane_xor_add<1>(s);
+    s = lane_xor_add<2>(s);
+    const float inv_rms = 1.0f / sqrtf(s / (float)H + eps);
+    const float y = x * inv_rms * nw;
+    const float amax = half_wave_max(fabsf(y));
+    float inv;
+    const float sc = act_scale(amax, inv);
+    if (cx.tid < H) {
+        smem[cx.tid] = (uint8_t)quant_code(y * inv);
+        if ((cx.tid & 31u) == 0) *reinterpret_cast<float*>(smem + off_as + cx.tid / 8) = f16_bits_to_f32(f32_to_f16_bits(sc));
+    }
+}
+
+struct PaExpTab {
+    const uint64_t* p;
+    __device__ __forceinline__ uint64_t operator()(int i) const { return p[i]; }
+};
+
+// LDS of an attention workgroup.  pn: products of q and this position's K row, vn: its V row, es: exp(m of the block before - m).
+template <int HD>
+struct PaAttn {
+    float q[HD], pn[HD], vn[HD];
+    float e[PA_WAVES][PA_B];
+    float sums[PA_WAVES][HD];
+    float bmax[PA_WAVES], lblk[PA_WAVES], es[PA_WAVES], snew;
+};
+
+// A wave's 64-key block of the cache: lane = key of the K rows, lane = head dim of the V rows.  Heads of 64: all of it, in 32-bit; wider heads:
+// K rows as they are and KC of the V rows at a time.
+typedef _Float16 PaHalf2 __attribute__((ext_vector_type(2)));
+template <int HD>
+struct PaKv {
+    static constexpr int DPL = (HD + 63) / 64, KC = HD == 64 ? 64 : 16;
+    float k[HD == 64 ? 64 : 1];
+    uint4 kr[HD == 64 ? 1 : HD / 8];
+    PaHalf2 v[KC / 2][DPL];
+    __device__ __forceinline__ void set_keys(const uint4 (&raw)[HD / 8]) {
+#pragma unroll
+        for (int c = 0; c < HD / 8; c++) {
+            if constexpr (HD == 64) {
+                const uint32_t w[4] = {raw[c].x, raw[c].y, raw[c].z, raw[c].w};
+#pragma unroll
+                for (int j = 0; j < 8; j++) k[c * 8 + j] = f16_bits_to_f32((uint16_t)(j & 1 ? w[j / 2] >> 16 : w[j / 2] & 0xFFFFu));
+            } else {
+                kr[c] = raw[c];
+            }
+        }
+    }
+    __device__ __forceinline__ float key(int i) const {
+        if constexpr (HD == 64) {
+            return k[i];
+        } else {
+            const uint4 r = kr[i / 8];
+            const uint32_t w = i % 8 / 2 == 0 ? r.x : i % 8 / 2 == 1 ? r.y : i % 8 / 2 == 2 ? r.z : r.w;
+            return f16_bits_to_f32((uint16_t)(i & 1 ? w >> 16 : w & 0xFFFFu));
+        }
+    }
+};
+template <int HD>
+__device__ __forceinline__ void pa_load_values(PaKv<HD>& kv, const uint16_t* vb, uint32_t bs, uint32_t k0, uint32_t pos, uint32_t kv_stride, uint32_t lane) {
+#pragma unroll
+    for (int i = 0; i < PaKv<HD>::KC; i++)
+#pragma unroll
+        for (int t = 0; t < PaKv<HD>::DPL; t++) {
+            const uint32_t d = min(lane + 64 * t, (uint32_t)HD - 1), row = bs + k0 + i;      // rows past the last cached one: row 0
+            kv.v[i / 2][t][i % 2] = pa_at<_Float16>(vb + (row < pos ? row : 0u) * kv_stride, d * 2);
+        }
+}
+
+// attention_flash (emit.rs:656-715) of head h in every layer, a wave per block of 64 keys: attn_exact_decode_one_kernel's steps.  The cached rows of a
+// layer are requested as soon as the layer before it is done.
+template <int HD>
+__device__ __forceinline__ void pa_attention(const PaArgs& a, const PaLayer* layers, PaAttn<HD>* sh, const uint64_t* exp_tab, uint32_t pos, uint32_t h, PaCtx& cx) {
+    constexpr int DPL = PaKv<HD>::DPL, KC = PaKv<HD>::KC;
+    const uint32_t kvh = h / (a.heads / a.kv_heads), kv_stride = a.KV;
+    const uint32_t b = cx.wave, seq = pos + 1, nb = (seq + PA_B - 1) / PA_B, bs = b * PA_B;
+    const uint32_t bl = bs < seq ? min(PA_B, seq - bs) : 0u;
+    const bool has_new = bs <= pos && pos < bs + PA_B;            // this position is the last key of the last block
+    uint32_t nk = has_new ? bl - 1 : bl;                          // of which cached
+    // the score of this position and the blocks' exp_scale are the work of waves without a block, as long as there are such
+    const bool wave_new = b == nb % PA_WAVES, wave_es = nb > 1 && b == (nb + 1) % PA_WAVES;
+    const float scale = 1.0f / sqrtf((float)HD);
+    const PaExpTab tab{exp_tab};
+#pragma nounroll
+    for (uint32_t l = 0; l < a.L; l++) {
+        asm volatile("" : "+v"(cx.tid), "+v"(cx.lane), "+s"(nk));
+        const uint32_t lane = cx.lane, tag_in = a.tag_base + 6 * l + 1;
+        PaKv<HD> kv;
+        const uint16_t* vb = pa_lds_ptr(layers[l].vc) + kvh * HD;
+        if (bl) {
+            const uint16_t* kb = pa_lds_ptr(layers[l].kc) + kvh * HD;
+            const uint32_t row = bs + lane, at = (row < pos ? row : 0u) * kv_stride * 2;
+            uint4 kr[HD / 8];
+#pragma unroll
+            for (int c = 0; c < HD / 8; c++) kr[c] = pa_at<uint4>(kb, at + c * 16);
+            pa_load_values<HD>(kv, vb, bs, 0, pos, kv_stride, lane);
+            __builtin_amdgcn_sched_barrier(0);
+            kv.set_keys(kr);
+        }
+        if (cx.tid < pa_up(HD, 64)) {
+            uint32_t g[3];
+            const uint32_t e = min(cx.tid, (uint32_t)HD - 1);
+            pa_poll<3>([&](int i) { return i == 0 ? a.tq + (size_t)h * HD + e : a.tkv + (i == 1 ? 0u : a.KV) + kvh * HD + e; }, [&](int) { return tag_in; }, g, cx);
+            if (cx.tid < HD) {
+                sh->q[e] = __uint_as_float(g[0]);
+                sh->pn[e] = __uint_as_float(g[0]) * f16_bits_to_f32((uint16_t)g[1]);
+                sh->vn[e] = f16_bits_to_f32((uint16_t)g[2]);
+            }
+        }
+        __syncthreads();
+        if (*cx.sh_abort) return;
+        float sc = -INFINITY;
+        if (bl) {
+            float sum = 0.f;
+#pragma unroll
+            for (int i = 0; i < HD; i++) {
+                if (i % 16 == 0) __builtin_amdgcn_sched_barrier(0);      // all of q at once would not fit the registers
+                sum = sum + sh->q[i] * kv.key(i);
+            }
+            if (lane < nk) sc = sum * scale;
+            const float mb = wave_max(sc);
+            if (lane == 0) sh->bmax[b] = mb;
+        }
+        if (wave_new) {
+            float sum = 0.f;
+#pragma unroll
+            for (int i = 0; i < HD; i++) {
+                if (i % 32 == 0) __builtin_amdgcn_sched_barrier(0);
+                sum = sum + sh->pn[i];
+            }
+            if (lane == 0) sh->snew = sum * scale;
+        }
+        __syncthreads();
+        if (wave_es) {
+            // m after block i: the largest block maximum so far; es[0] = exp(-inf - m) is 0
+            float m = -INFINITY, before = -INFINITY;
+#pragma unroll
+            for (uint32_t i = 0; i < PA_WAVES; i++) {
+                const float v = i < nb ? (i == nb - 1 ? fmaxf(sh->bmax[i], sh->snew) : sh->bmax[i]) : -INFINITY;
+                if (i < lane) before = fmaxf(before, v);
+                if (i <= lane) m = fmaxf(m, v);
+            }
+            const float es = expf_ref_with<true>(before - m, tab);
+            if (lane < nb) sh->es[lane] = es;
+        }
+        if (bl) {
+            float m = wave_max(lane <= b ? sh->bmax[lane] : -INFINITY);
+            if (has_new) {
+                const float s = sh->snew;
+                m = fmaxf(m, s);
+                if (lane == nk) sc = s;
+            }
+            sh->e[b][lane] = lane < bl ? expf_ref_with<true>(sc - m, tab) : 0.f;       // LDS operations of one wave execute in order
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            float l_block = 0.f, sum[DPL];
+#pragma unroll
+            for (int t = 0; t < DPL; t++) sum[t] = 0.f;
+#pragma nounroll
+            for (uint32_t k0 = 0; k0 < PA_B; k0 += KC) {
+                if (k0 && k0 >= nk) break;
+                if (k0) pa_load_values<HD>(kv, vb, bs, k0, pos, kv_stride, lane);
+                // keys past the last one are left out, not given a weight of 0: 0 * v is not 0 for an infinite v
+#pragma unroll
+                for (int i16 = 0; i16 < KC; i16 += 16) {
+                    __builtin_amdgcn_sched_barrier(0);       // all weights at once would not fit the registers
+                    if (k0 + i16 < nk) {
+                        float w[16];
+#pragma unroll
+                        for (int i = 0; i < 16; i += 4) *reinterpret_cast<float4*>(w + i) = *reinterpret_cast<const float4*>(&sh->e[b][k0 + i16 + i]);
+                        auto add = [&](int i) {
+                            l_block = l_block + w[i];
+#pragma unroll
+                            for (int t = 0; t < DPL; t++) sum[t] = sum[t] + w[i] * (float)kv.v[(i16 + i) / 2][t][(i16 + i) % 2];
+                        };
+                        if (k0 + i16 + 16 <= nk) {
+#pragma unroll
+                            for (int i = 0; i < 16; i++) add(i);
+                        } else {
+#pragma unroll
+                            for (int i = 0; i < 16; i++)
+                                if (k0 + i16 + i < nk) add(i);
+                        }
+                    }
+                }
+            }
+            if (has_new) {
+                const float w = sh->e[b][nk];
+                l_block = l_block + w;
+#pragma unroll
+                for (int t = 0; t < DPL; t++) sum[t] = sum[t] + w * sh->vn[min(lane + 64 * t, (uint32_t)HD - 1)];
+            }
+#pragma unroll
+            for (int t = 0; t < DPL; t++)
+                if (lane + 64 * t < HD) sh->sums[b][lane + 64 * t] = sum[t];
+            if (lane == 0) sh->lblk[b] = l_block;
+        }
+        __syncthreads();
+        if (cx.tid < pa_up(HD, 64)) {
+            const uint32_t d = cx.tid < HD ? cx.tid : 0;
+            float l_i = 0.f + sh->lblk[0], acc = 0.f + sh->sums[0][d];               // es[0] = 0 times 0, then the sum
+            for (uint32_t i = 1; i < nb; i++) {
+                const float exp_scale = sh->es[i];
+                l_i = l_i * exp_scale;
+                acc = acc * exp_scale;
+                l_i = l_i + sh->lblk[i];
+                acc = acc + sh->sums[i][d];
+            }
+            const float inv_l = 1.0f / l_i;
+            const float o = acc * inv_l;
+            const uint32_t e = h * HD + cx.tid;
+            pa_store_block(cx.tid < HD ? o : 0.f, a.taq + e / 32 * 9, tag_in + 1, cx.lane, cx.tid < HD);
+        }
+    }
+}
+
+// One workgroup's part of an argmax: the LAST index among equal maxima (project.rs:501-503).
+__device__ __forceinline__ ArgPair pa_arg_wg(ArgPair v, ArgPair* sh, const PaCtx& cx) {
+    auto fold = [&](auto O) { v = arg_better(v, ArgPair{lane_xor<O.value>(v.v), lane_xor<O.value>(v.i)}); };
+    fold(std::integral_constant<int, 32>{}); fold(std::integral_constant<int, 16>{}); fold(std::integral_constant<int, 8>{});
+    fold(std::integral_constant<int, 4>{}); fold(std::integral_constant<int, 2>{}); fold(std::integral_constant<int, 1>{});
+    __syncthreads();
+    if (cx.lane == 0) sh[cx.wave] = v;
+    __syncthreads();
+    ArgPair r = sh[0];
+    for (uint32_t w = 1; w < PA_WAVES; w++) r = arg_better(r, sh[w]);
+    return r;
+}
+
+// The tag of a phase instance: tag_base + 6 layer + 1 q;k;v, 2 attention, 4 o, 5 gate;up, 6 down; the argmax's is behind the last layer's.
+template <int HD, bool Q4, bool LMQ4>
+__global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
+    extern __shared__ __align__(16) uint8_t smem[];
+    __shared__ uint32_t sh_abort;
+    __shared__ ArgPair sh_arg[PA_WAVES];
+    __shared__ uint64_t exp_tab[32];          // expf_ref's table
+    uint32_t* aq = reinterpret_cast<uint32_t*>(smem);
+    float* as = reinterpret_cast<float*>(smem + a.off_as);
+    float* xs = reinterpret_cast<float*>(smem + a.off_xs);
+    float* out = reinterpret_cast<float*>(smem + a.off_out);                     // the workgroup's row sums
+    float* nws = reinterpret_cast<float*>(smem + a.off_nw);
+    float* silu = reinterpret_cast<float*>(smem + a.off_silu);
+    const PaLayer* layers = reinterpret_cast<const PaLayer*>(smem + a.off_layers);
+    PaAttn<HD>* attn = reinterpret_cast<PaAttn<HD>*>(smem + a.off_attn);
+
+    PaCtx cx;
+    cx.tid = threadIdx.x;
+    cx.lane = threadIdx.x & 63u;
+    cx.wave = pa_sgpr(threadIdx.x >> 6);
+    cx.wg = blockIdx.x;
+    cx.G = a.G;
+    cx.spin_limit = a.spin_limit;
+    cx.sh_abort = &sh_abort;
+    cx.abort_flag = a.state + 3;
+    const bool comp = cx.wave >= PA_POLL;
+    const uint32_t c = comp ? cx.wave - PA_POLL : 0u, wv = cx.wg * PA_COMP + c;       // a workgroup's rows lie side by side: one store hands them over
+    if (cx.tid == 0) sh_abort = 0;
+    if (cx.tid < 32) exp_tab[cx.tid] = expf_detail::tab((int)cx.tid);
+    for (uint32_t i = cx.tid; i < a.lds_words; i += PA_THREADS) reinterpret_cast<uint32_t*>(smem)[i] = 0;      // the zeros behind products and accumulators
+    for (uint32_t i = cx.tid; i < (a.L + 1) * (uint32_t)(sizeof(PaLayer) / 4); i += PA_THREADS)
+        reinterpret_cast<uint32_t*>(smem + a.off_layers)[i] = ldg(reinterpret_cast<const uint32_t*>(a.layers) + i);
+    const uint32_t pos = a.state[0];
+    const float* emb = a.embed + (size_t)a.token * a.H;
+    __syncthreads();
+
+    const uint32_t ntid = cx.tid - PA_POLL_THREADS;                               // of a computing thread
+    const bool stamp = a.stamps && cx.wg == 0 && cx.tid == 0;
+    PaSet<UL, LMQ4> wl[2];
+    float n1 = 0.f, n1p = 0.f;                // norm weights of element tid, and of a polling thread's element, which gets them through LDS
+    const PaMat ml = a.m[4];
+    const uint32_t T = gridDim.x, W = PA_COMP * T, lwv = c * T + cx.wg;
+
+    if (cx.wg < cx.G) {
+        const PaMat mq = a.m[0], mo = a.m[1], mg = a.m[2], md = a.m[3];
+        const uint32_t per_wave = 32 / PA_COMP;                                  // gate;up: 4 gate and 4 up rows a wave
+        const uint32_t row_q = cx.wg * PA_COMP * mq.R, row_o = cx.wg * PA_COMP * mo.R, row_d = cx.wg * PA_COMP * md.R;
+        const bool on_q = row_q < mq.N, on_o = row_o < mo.N, on_g = cx.wg < a.I / 32, on_d = row_d < md.N;
+        const PaTask tq = pa_task(mq, wv), to = pa_task(mo, wv), td = pa_task(md, wv);
+        const PaTask tg{on_g ? (cx.wg * 32 + c * per_wave) * mg.nblk : 0u, on_g ? 2 * per_wave * mg.nblk : 0u, per_wave * mg.nblk, (a.I - per_wave) * mg.nblk};
+        const uint32_t pq = mq.prod + c * a.prod_words * 4, po = mo.prod + c * a.prod_words * 4, pg = mg.prod + c * a.prod_words * 4, pd = md.prod + c * a.prod_words * 4;
+        PaSet<UQ, Q4> wq;
+        PaSet<UO, Q4> wo;
+        PaSet<UG, Q4> wg;
+        PaSet<UD, Q4> wd;
+        float n2 = 0.f, n2p = 0.f;
+        // the first wave finishes rows: lane r the workgroup's r-th
+        float rc = 1.f, rs = 0.f;                                                // rotation of its row of q | k
+        const uint32_t qrow = row_q + cx.lane;
+        const bool mine_q = cx.wave == 0 && cx.lane < PA_COMP * mq.R && qrow < mq.N;
+        if (mine_q && qrow < a.QKS + a.KV) {
+            const uint32_t d = (qrow < a.QKS ? qrow : qrow - a.QKS) % HD;
+            rc = ldg(a.cos_t + (size_t)pos * (HD / 2) + d / 2);
+            rs = ldg(a.sin_t + (size_t)pos * (HD / 2) + d / 2);
+        }
+        auto load_norm = [&](const float* nw, float& own, float& other) {      // elements past the last one: it again
+            own = pa_at<float>(nw, min(cx.tid, a.H - 1) * 4);
+            other = pa_at<float>(nw, min(ntid, a.H - 1) * 4);
+        };
+        if (comp) {
+            const PaLayer& L = layers[0];
+            load_norm(pa_lds_ptr(L.norm[0]), n1, n1p);
+            pa_load(wq, pa_lds_ptr(L.w[0]), tq, cx.lane);
+        }
+
+#pragma nounroll
+        for (uint32_t l = 0; l < a.L; l++) {
+            // The thread's number is read afresh in every layer: addresses that follow from it would be kept from layer to layer and not fit the registers.
+            asm volatile("" : "+v"(cx.tid), "+v"(cx.lane));
+            const PaLayer& L = layers[l];
+            const PaLayer& N = layers[l + 1];
+            const uint32_t base = a.tag_base + 6 * l, x_in = l ? base : 0u;
+            // ---- norm | q;k;v | rotation, cache row
+            if (stamp) a.stamps[6 * l] = wall_clock64();
+            if (on_q) {
+                if (!comp) {
+                    uint16_t* kc = pa_lds_ptr(L.kc);
+                    uint16_t* vc = pa_lds_ptr(L.vc);
+                    pa_fetch_x(a.tx, x_in, emb, a.H, xs, a.xstride, cx);
+                    __syncthreads();
+                    if (sh_abort) return;
+                    pa_norm_quant(xs, a.xstride, nws[cx.tid], a.eps, a.H, smem, a.off_as, cx);
+                    __syncthreads();
+                    __syncthreads();
+                    if (cx.wave == 0) {
+                        const float v = out[cx.lane];
+                        const float other = lane_xor<1>(v);                      // rope (emit.rs:508-528): rows 2i, 2i + 1 of a head
+                        const float o = (qrow & 1u) ? other * rs + v * rc : v * rc - other * rs;
+                        const bool is_q = qrow < a.QKS, is_k = qrow < a.QKS + a.KV;
+                        const uint16_t hb = f32_to_f16_bits(is_k ? o : v);
+                        const uint32_t at = qrow - a.QKS;                        // of [K row | V row]
+                        if (mine_q) {
+                            stc64(is_q ? a.tq + qrow : a.tkv + at, base + 1, is_q ? __float_as_uint(o) : (uint32_t)hb);
+                            if (!is_q) stg((is_k ? kc + at : vc + (at - a.KV)) + (size_t)pos * a.KV, hb);
+                        }
+                    }
+                } else {
+                    const auto x = pa_index<UQ, Q4>(tq, mq, a.off_as, pq, cx.lane);
+                    if (ntid < PA_POLL_THREADS) nws[ntid] = n1p;
+                    __syncthreads();
+                    if (sh_abort) return;
+                    pa_norm_quant(xs, a.xstride, n1, a.eps, a.H, smem, a.off_as, cx);
+                    __syncthreads();
+                    pa_products(wq, x, tq.n, smem);
+                    const float v = pa_row_sum(mq, mq.R, smem + pq, cx.lane);
+                    if (cx.lane < mq.R) out[c * mq.R + cx.lane] = v;
+                    __syncthreads();
+                }
+            }
+            // While the attention is at work nothing else is on its way to this workgroup: now the matrices that follow are requested (a load that
+            // misses ahead of a poll holds the poll up, whichever wave it belongs to).
+            if (comp) {
+                pa_load(wo, pa_lds_ptr(L.w[1]), to, cx.lane);
+                load_norm(pa_lds_ptr(L.norm[1]), n2, n2p);
+                pa_load(wg, pa_lds_ptr(L.w[2]), tg, cx.lane);
+                pa_load(wd, pa_lds_ptr(L.w[3]), td, cx.lane);
+                load_norm(pa_lds_ptr(N.norm[0]), n1, n1p);
+                pa_load(wq, pa_lds_ptr(N.w[0]), tq, cx.lane);
+            }
+            // ---- (attention) o + residual
+            if (stamp) { const unsigned long long t = wall_clock64(); a.stamps[6 * l + 1] = t; a.stamps[6 * l + 2] = t; a.stamps[6 * l + 3] = t; }
+            if (on_o) {
+                const bool mine = cx.wave == 0 && cx.lane < PA_COMP * mo.R && row_o + cx.lane < mo.N;
+                if (!comp) {
+                    const float r = pa_fetch_aq(a.taq, base + 2, a.QKS, aq, as, mine, row_o + cx.lane, a.tx, x_in, emb, cx);
+                    __syncthreads();
+                    if (sh_abort) return;
+                    __syncthreads();
+                    if (mine) stc64(a.tx + row_o + cx.lane, base + 4, __float_as_uint(r + out[cx.lane]));     // residual_add, emit.rs:455-459
+                } else {
+                    const auto x = pa_index<UO, Q4>(to, mo, a.off_as, po, cx.lane);
+                    __syncthreads();
+                    if (sh_abort) return;
+                    pa_products(wo, x, to.n, smem);
+                    const float v = pa_row_sum(mo, mo.R, smem + po, cx.lane);
+                    if (cx.lane < mo.R) out[c * mo.R + cx.lane] = v;
+                    __syncthreads();
+                }
+            }
+            // ---- norm | gate;up | silu(gate) * up
+            if (stamp) a.stamps[6 * l + 4] = wall_clock64();
+            if (on_g) {
+                if (!comp) {
+                    pa_fetch_x(a.tx, base + 4, emb, a.H, xs, a.xstride, cx);
+                    __syncthreads();
+                    if (sh_abort) return;
+                    pa_norm_quant(xs, a.xstride, nws[cx.tid], a.eps, a.H, smem, a.off_as, cx);
+                    __syncthreads();
+                    __syncthreads();
+                    if (cx.wave == 0) pa_store_block(silu[cx.lane & 31u], a.taq2 + cx.wg * 9, base + 5, cx.lane, cx.lane < 32);
+                } else {
+                    const auto x = pa_index<UG, Q4>(tg, mg, a.off_as, pg, cx.lane);
+                    if (ntid < PA_POLL_THREADS) nws[ntid] = n2p;
+                    __syncthreads();
+                    if (sh_abort) return;
+                    pa_norm_quant(xs, a.xstride, n2, a.eps, a.H, smem, a.off_as, cx);
+                    __syncthreads();
+                    pa_products(wg, x, tg.n, smem);
+                    const float v = pa_row_sum(mg, 2 * per_wave, smem + pg, cx.lane);
+                    const float up = lane_xor<4>(v);
+                    if (cx.lane < per_wave) silu[c * per_wave + cx.lane] = (v / (1.0f + expf_ref_with<true>(-v, PaExpTab{exp_tab}))) * up;      // silu_mul, emit.rs:380-386
+                    __syncthreads();
+                }
+            }
+            // ---- down + residual
+            if (stamp) a.stamps[6 * l + 5] = wall_clock64();
+            if (on_d) {
+                const bool mine = cx.wave == 0 && cx.lane < PA_COMP * md.R && row_d + cx.lane < md.N;
+                if (!comp) {
+                    const float r = pa_fetch_aq(a.taq2, base + 5, a.I, aq, as, mine, row_d + cx.lane, a.tx, base + 4, emb, cx);
+                    __syncthreads();
+                    if (sh_abort) return;
+                    __syncthreads();
+                    if (mine) stc64(a.tx + row_d + cx.lane, base + 6, __float_as_uint(r + out[cx.lane]));
+                } else {
+                    const auto x = pa_index<UD, Q4>(td, md, a.off_as, pd, cx.lane);
+                    __syncthreads();
+                    if (sh_abort) return;
+                    pa_products(wd, x, td.n, smem);
+                    const float v = pa_row_sum(md, md.R, smem + pd, cx.lane);
+                    if (cx.lane < md.R) out[c * md.R + cx.lane] = v;
+                    __syncthreads();
+                }
+            }
+        }
+        if (comp) pa_load(wl[0], a.lm, pa_task(ml, lwv), cx.lane);
+    } else {
+        if (comp) {
+            const float* nw = pa_lds_ptr(layers[a.L].norm[0]);
+            n1 = pa_at<float>(nw, min(cx.tid, a.H - 1) * 4);
+            n1p = pa_at<float>(nw, min(ntid, a.H - 1) * 4);
+        }
+        if (cx.wg - cx.G < a.heads) {
+            pa_attention<HD>(a, layers, attn, exp_tab, pos, cx.wg - cx.G, cx);
+            if (sh_abort) return;
+        }
+        if (comp) pa_load(wl[0], a.lm, pa_task(ml, lwv), cx.lane);
+        // a workgroup without rows in the layers looks for the final row now and then only
+        if (cx.tid == 0) {
+            uint32_t spins = 0;
+            while ((uint32_t)(ldc64(a.tx + a.H - 1) >> 32) != a.tag_base + 6 * a.L && ++spins <= cx.spin_limit &&
+                   ((spins & 255u) != 0 || __hip_atomic_load(cx.abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0))
+                __builtin_amdgcn_s_sleep(16);
+        }
+        __syncthreads();
+    }
+
+    // ---- final norm | lm_head | argmax
+    asm volatile("" : "+v"(cx.tid), "+v"(cx.lane));
+    if (stamp) a.stamps[6 * a.L] = wall_clock64();
+    ArgPair best{-INFINITY, 0};
+    if (!comp) {
+        pa_fetch_x(a.tx, a.tag_base + 6 * a.L, emb, a.H, xs, a.xstride, cx);
+        __syncthreads();
+        if (sh_abort) return;
+        pa_norm_quant(xs, a.xstride, nws[cx.tid], a.eps, a.H, smem, a.off_as, cx);
+        __syncthreads();
+    } else {
+        const uint32_t pl = ml.prod + c * a.prod_words * 4;
+        if (ntid < PA_POLL_THREADS) nws[ntid] = n1p;
+        __syncthreads();
+        if (sh_abort) return;
+        pa_norm_quant(xs, a.xstride, n1, a.eps, a.H, smem, a.off_as, cx);
+        __syncthreads();
+        auto tile = [&](uint32_t t, const PaSet<UL, LMQ4>& w) {
+            const PaTask task = pa_task(ml, t);
+            pa_products(w, pa_index<UL, LMQ4>(task, ml, a.off_as, pl, cx.lane), task.n, smem);
+            const uint32_t rows = pa_rows(ml, t), row = t * ml.R + cx.lane;
+            float v = pa_row_sum(ml, rows, smem + pl, cx.lane);
+            if (cx.lane < rows) {
+                stg(a.logits + row, v);
+                // apply_repeat_penalty (project.rs:505-513) ahead of the argmax.  The lane that holds the row of the token being fed is the
+                // only one in the grid to touch that counter: it adds this step's occurrence.
+                if (a.penalty > 1.0f) {
+                    const bool fed = row == a.token;
+                    const uint32_t n = ldg(a.counts + row) + (fed ? 1u : 0u);
+                    if (fed) { stg(a.counts + row, n); stg(a.state + 4, a.step_seq); }      // so that a step that gives up later can be undone
+                    v = repeat_penalised(v, n, a.penalty);
+                }
+                best = arg_better(best, ArgPair{v, row});
+            }
+        };
+        for (uint32_t t = lwv; t * ml.R < ml.N; t += 2 * W) {
+            const bool second = (t + W) * ml.R < ml.N, third = (t + 2 * W) * ml.R < ml.N;
+            if (second) pa_load(wl[1], a.lm, pa_task(ml, t + W), cx.lane);
+            tile(t, wl[0]);
+            if (third) pa_load(wl[0], a.lm, pa_task(ml, t + 2 * W), cx.lane);
+            if (second) tile(t + W, wl[1]);
+        }
+    }
+    const uint32_t th = a.tag_base + 6 * a.L + 1;
+    best = pa_arg_wg(best, sh_arg, cx);
+    if (cx.tid == 0) {
+        stc64(a.tpart + 2 * cx.wg, th, __float_as_uint(best.v));
+        stc64(a.tpart + 2 * cx.wg + 1, th, best.i);
+    }
+    if (stamp) a.stamps[6 * a.L + 1] = wall_clock64();
+    if (cx.wg != 0) return;
+    ArgPair p{-INFINITY, 0};
+    for (uint32_t w = cx.tid; w < T; w += PA_THREADS) {
+        uint32_t v[2];
+        pa_poll<2>([&](int i) { return a.tpart + 2 * w + (uint32_t)i; }, [&](int) { return th; }, v, cx);
+        p = arg_better(p, ArgPair{__uint_as_float(v[0]), v[1]});
+    }
+    p = pa_arg_wg(p, sh_arg, cx);
+    if (sh_abort) return;
+    if (cx.tid == 0) {
+        a.state[2] = p.i;
+        a.state[1] = p.i;
+        a.state[0] = pos + 1;
+        if (!(a.penalty > 1.0f)) a.counts[a.token] += 1;          // nobody read the counters in this launch
+        if (stamp) a.stamps[6 * a.L + 2] = wall_clock64();
+        // the host may be spinning on this word instead of waiting for the stream
+        if (a.host_out) __hip_atomic_store(a.host_out, ((unsigned long long)a.host_seq << 32) | p.i, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
+template <int HD>
+const void* pa_kernel_hd(bool q4, bool lmq4) {
+    if (q4) return lmq4 ? reinterpret_cast<const void*>(decode_ahead_kernel<HD, true, true>) : reinterpret_cast<const void*>(decode_ahead_kernel<HD, true, false>);
+    return lmq4 ? reinterpret_cast<const void*>(decode_ahead_kernel<HD, false, true>) : reinterpret_cast<const void*>(decode_ahead_kernel<HD, false, false>);
+}
+template <int HD>
+uint32_t pa_attn_bytes() { return (uint32_t)sizeof(PaAttn<HD>); }
+
+}  // namespace
+
+struct PaState {
+    PaArgs args{};
+    std::vector<void*> owned;
+    const void* kernel = nullptr;
+    uint32_t grid = 0, lds = 0, n_stamps = 0;
+    uint64_t* tagged = nullptr;
+    size_t tagged_bytes = 0;
+    std::vector<unsigned long long> stamps_host;
+    int wall_khz = 0;
+    unsigned long long* host_out = nullptr;
+    unsigned long long* host_out_dev = nullptr;
+    uint32_t seq = 0;
+    ~PaState() {
+        for (void* p : owned) (void)hipFree(p);
+        if (host_out) (void)hipHostFree(host_out);
+    }
+    template <typename T>
+    T* dev(size_t n) {
+        void* p = nullptr;
+        if (hipMalloc(&p, n < 16 ? 16 : n) != hipSuccess) return nullptr;
+        owned.push_back(p);
+        return static_cast<T*>(p);
+    }
+};
+
+void pa_destroy(PaState* st) { delete st; }
+
+// Contexts of up to PA_WAVES blocks: a workgroup takes a head's whole context, and lanes without a key of their own read the cache's first row, which an
+// empty cache does not have yet.
+bool pa_covers(const PaState* st, int64_t pos) { return st && pos >= 1 && pos < (int64_t)(PA_WAVES * PA_B); }
+
+int32_t pa_create(const forge_hip_config& c, const std::vector<PdLayerIn>& layers, const QWeight& lm_head, const float* embed, const float* final_norm,
+                  const float* cos_t, const float* sin_t, float* logits, uint32_t* state, uint32_t* counts, PaState** out) {
+    *out = nullptr;
+    const uint32_t H = c.hidden, I = c.inter, hd = c.head_dim, QKS = c.heads * hd, KV = c.kv_heads * hd;
+    if (c.sliding_window != 0 || layers.empty() || !layers[0].qkv || lm_head.kquant()) return FORGE_HIP_OK;
+    if (hd != 64 && hd != 96 && hd != 128) return FORGE_HIP_OK;
+    if (H < 64 || I < 64 || QKS < 64) return FORGE_HIP_OK;
+    // what the polling threads fetch at once
+    if (H > PA_PN * PA_POLL_THREADS || I / 32 * 9 > PA_PN * PA_POLL_THREADS || QKS / 32 * 9 > PA_PN * PA_POLL_THREADS) return FORGE_HIP_OK;
+    // rows that the reference adds in its four-accumulator order (the last len % 4 of a chunk) are left to the other kernels
+    if (H % 4 || I % 4 || QKS % 4 || KV % 4 || c.vocab % 4) return FORGE_HIP_OK;
+    int dev = 0, cus = 0, khz = 0;
+    FH_HIP(hipGetDevice(&dev));
+    FH_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    FH_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev));
+
+    std::unique_ptr<PaState> st(new PaState());
+    PaArgs& a = st->args;
+    const uint32_t nq[5] = {QKS + 2 * KV, H, 2 * I, H, c.vocab}, kk[5] = {H, QKS, H, I, H};
+    const int units[5] = {UQ, UO, UG, UD, UL};
+    for (int i = 0; i < 5; i++) {
+        PaMat& m = a.m[i];
+        m.N = nq[i]; m.nblk = kk[i] / 32;
+        m.magic = (uint32_t)(0x100000000ull / m.nblk) + 1u;
+        m.R = 64u * units[i] / m.nblk;                             // the most a wave can hold
+        if (i == 0) m.R = std::min(m.R & ~1u, PA_MAX_ROWS);        // a rotation's pair in one wave
+        else if (i == 1 || i == 3) m.R = std::min(m.R, PA_MAX_ROWS);
+        else if (i == 2) { if (m.R < 64 / PA_COMP) return FORGE_HIP_OK; m.R = 64 / PA_COMP; }
+        else m.R = std::min(m.R, 32u);
+        if (m.R == 0) return FORGE_HIP_OK;
+    }
+    // The fewest workgroups that hold every row at the most per wave and gate;up by whole blocks of 32, a workgroup per head, and what is left of the
+    // device for the lm_head; then as few rows per wave as that many workgroups allow.
+    uint32_t g = I / 32;
+    for (int i : {0, 1, 3}) g = std::max(g, (a.m[i].N + a.m[i].R * PA_COMP - 1) / (a.m[i].R * PA_COMP));
+    if (g + c.heads > (uint32_t)cus) return FORGE_HIP_OK;
+    a.G = g;
+    st->grid = (uint32_t)cus;
+    for (int i : {0, 1, 3}) {
+        a.m[i].R = (a.m[i].N + g * PA_COMP - 1) / (g * PA_COMP);
+        if (i == 0) a.m[i].R = pa_up(a.m[i].R, 2);
+    }
+    a.L = (uint32_t)layers.size(); a.H = H; a.I = I; a.QKS = QKS; a.KV = KV; a.heads = c.heads; a.kv_heads = c.kv_heads;
+    a.eps = c.rms_eps;
+    const uint32_t kmax = std::max(std::max(H, I), QKS);
+    a.off_as = pa_up(kmax, 16);
+    a.off_xs = a.off_as + pa_up(kmax / 32 * 4, 16);
+    auto odd16 = [](uint32_t words) { return words % 8 ? words : words + 4; };      // rows an odd number of 16-byte units apart spread over the banks
+    a.xstride = odd16(pa_up(H / 16, PA_SSQ));
+    a.off_out = a.off_xs + 16 * a.xstride * 4;
+    a.off_nw = a.off_out + PA_COMP * PA_MAX_ROWS * 4;
+    a.off_silu = a.off_nw + PA_POLL_THREADS * 4;
+    a.off_prod = a.off_silu + 32 * 4;
+    a.prod_words = 0;
+    for (int i = 0; i < 5; i++) {
+        PaMat& m = a.m[i];
+        m.stride = odd16(pa_up(m.nblk, PA_SUM));
+        m.prod = a.off_prod + a.prod_words * 4;
+        a.prod_words += m.R * m.stride + 4;
+    }
+    a.off_layers = a.off_prod + PA_COMP * a.prod_words * 4;
+    a.lds_words = a.off_layers / 4;
+    a.off_attn = pa_up(a.off_layers + ((uint32_t)layers.size() + 1) * (uint32_t)sizeof(PaLayer), 16);
+    st->lds = a.off_attn + (hd == 64 ? pa_attn_bytes<64>() : hd == 96 ? pa_attn_bytes<96>() : pa_attn_bytes<128>());
+    if (st->lds > 64000) return FORGE_HIP_OK;
+    const bool q4 = c.wdtype == FORGE_HIP_Q4_0, lmq4 = c.lm_head_dtype == FORGE_HIP_Q4_0;
+    st->kernel = hd == 64 ? pa_kernel_hd<64>(q4, lmq4) : hd == 96 ? pa_kernel_hd<96>(q4, lmq4) : pa_kernel_hd<128>(q4, lmq4);
+    int per_cu = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, st->kernel, PA_THREADS, st->lds) != hipSuccess || per_cu < 1) { (void)hipGetLastError(); return FORGE_HIP_OK; }
+
+    std::vector<PaLayer> host(layers.size() + 1);
+    memset(host.data(), 0, host.size() * sizeof(PaLayer));
+    for (size_t l = 0; l < layers.size(); l++) {
+        const PdLayerIn& in = layers[l];
+        const QWeight* w[4] = {in.qkv, in.o, in.gate_up, in.down};
+        for (int k = 0; k < 4; k++) host[l].w[k] = PaWeights{w[k]->qs, w[k]->scales};
+        host[l].norm[0] = in.attn_norm; host[l].norm[1] = in.ffn_norm; host[l].kc = in.kc; host[l].vc = in.vc;
+    }
+    host.back() = host[0];
+    host.back().norm[0] = final_norm;
+    PaLayer* dl = st->dev<PaLayer>(host.size() * sizeof(PaLayer));
+    const size_t n_tagged = (size_t)H + QKS + 2 * KV + QKS / 32 * 9 + I / 32 * 9 + 2 * (size_t)st->grid;
+    uint64_t* t = st->dev<uint64_t>(n_tagged * 8);
+    if (!dl || !t) return fail(FORGE_HIP_ERR_HIP, "resident decode: out of device memory");
+    FH_HIP(hipMemcpy(dl, host.data(), host.size() * sizeof(PaLayer), hipMemcpyHostToDevice));
+    FH_HIP(hipMemset(t, 0, n_tagged * 8));                       // tag 0 is never expected
+    st->tagged = t; st->tagged_bytes = n_tagged * 8;
+    a.layers = dl;
+    a.tx = t; t += H;
+    a.tq = t; t += QKS;
+    a.tkv = t; t += 2 * KV;
+    a.taq = t; t += QKS / 32 * 9;
+    a.taq2 = t; t += I / 32 * 9;
+    a.tpart = t;
+    a.lm = PaWeights{lm_head.qs, lm_head.scales};
+    a.embed = embed; a.cos_t = cos_t; a.sin_t = sin_t;
+    a.logits = logits; a.state = state; a.counts = counts; a.penalty = 1.0f;
+    { const char* e = getenv("FORGE_HIP_PD_TAG_START"); if (e) a.tag_base = (uint32_t)strtoul(e, nullptr, 0); }
+    pa_set_poll_limit(st.get(), 0);
+    { const char* e = getenv("FORGE_HIP_PD_SPIN_LIMIT"); if (e && atoi(e) > 0) a.spin_limit = (uint32_t)atoi(e); }
+    if (!(getenv("FORGE_HIP_PD_HOSTWORD") && getenv("FORGE_HIP_PD_HOSTWORD")[0] == '0')) {
+        void *hp = nullptr, *dp = nullptr;
+        if (hipHostMalloc(&hp, 64, hipHostMallocMapped) == hipSuccess) {
+            if (hipHostGetDevicePointer(&dp, hp, 0) == hipSuccess) {
+                st->host_out = static_cast<unsigned long long*>(hp);
+                st->host_out_dev = static_cast<unsigned long long*>(dp);
+                st->host_out[0] = 0;
+            } else {
+                (void)hipHostFree(hp);
+            }
+        }
+        (void)hipGetLastError();
+    }
+    st->wall_khz = khz;
+    st->n_stamps = 6 * a.L + 3;
+    *out = st.release();
+    return FORGE_HIP_OK;
+}
+
+void pa_set_poll_limit(PaState* st, uint32_t n) { st->args.spin_limit = n ? n : 400000u; }
+void pa_set_repeat_penalty(PaState* st, float penalty) { st->args.penalty = penalty; }
+
+// Enqueues the step at the position in `state` for `token`.  With `profile` the kernel also records the clock at the start of every phase.
+int32_t pa_enqueue(PaState* st, bool profile, uint32_t token, hipStream_t s) {
+    PaArgs& a = st->args;
+    a.token = token;
+    a.step_seq = a.step_seq + 1 ? a.step_seq + 1 : 1;
+    a.host_out = st->host_out_dev;
+    if (a.host_out) a.host_seq = ++st->seq;
+    if (a.tag_base > 0xF0000000u) {      // tags are about to wrap: start again from zeroed buffers
+        FH_HIP(hipMemsetAsync(st->tagged, 0, st->tagged_bytes, s));
+        a.tag_base = 0;
+    }
+    if (profile && !a.stamps) {
+        a.stamps = st->dev<unsigned long long>(st->n_stamps * 8);
+        if (!a.stamps) return fail(FORGE_HIP_ERR_HIP, "resident decode: out of device memory");
+    }
+    unsigned long long* keep = a.stamps;
+    if (!profile) a.stamps = nullptr;
+    void* kargs[] = {&a};
+    const hipError_t e = hipLaunchKernel(st->kernel, dim3(st->grid), dim3(PA_THREADS), kargs, st->lds, s);
+    a.stamps = keep;
+    if (e != hipSuccess) return fail(FORGE_HIP_ERR_HIP, std::string("resident decode launch: ") + hipGetErrorString(e));
+    a.tag_base += 6 * a.L + 1;
+    return FORGE_HIP_OK;
+}
+
+// The next token, from the word that the kernel writes last; false: not in use or not in time, wait for the stream instead.
+bool pa_wait_token(PaState* st, uint32_t* next) {
+    if (!st->host_out || !st->args.host_out) return false;
+    const volatile unsigned long long* w = st->host_out;
+    const auto t0 = std::chrono::steady_clock::now();
+    for (uint32_t spin = 0;; spin++) {
+        const unsigned long long v = *w;
+        if ((uint32_t)(v >> 32) == st->seq) { *next = (uint32_t)v; return true; }
+        if ((spin & 1023u) == 1023u && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(200)) return false;
+    }
+}
+
+// After the stream has drained, with the abort flag: a step that gave up did not happen (the position advances last); what may have happened
+// is the count of its token, which is taken back.
+int32_t pa_after_sync(PaState* st, uint32_t abort_flag, hipStream_t s) {
+    if (!abort_flag) return FORGE_HIP_OK;
+    PaArgs& a = st->args;
+    uint32_t seq = 0, n = 0;
+    FH_HIP(hipMemcpyAsync(&seq, a.state + 4, 4, hipMemcpyDeviceToHost, s));
+    FH_HIP(hipMemcpyAsync(&n, a.counts + a.token, 4, hipMemcpyDeviceToHost, s));
+    FH_HIP(hipStreamSynchronize(s));
+    if (seq == a.step_seq && n) {
+        n -= 1;
+        FH_HIP(hipMemcpyAsync(a.counts + a.token, &n, 4, hipMemcpyHostToDevice, s));
+        FH_HIP(hipStreamSynchronize(s));
+    }
+    FH_HIP(hipMemsetAsync(st->tagged, 0, st->tagged_bytes, s));
+    FH_HIP(hipMemsetAsync(a.state + 3, 0, 4, s));
+    FH_HIP(hipStreamSynchronize(s));
+    a.tag_base = 0;
+    return fail(FORGE_HIP_ERR_HIP, "resident decode step gave up waiting for another workgroup's data (grid not co-resident?)");
+}
+
+// Milliseconds between the phase starts of the last profiled step, as pd_phase_ms reports them.
+int32_t pa_phase_ms(PaState* st, std::vector<float>* out, hipStream_t s) {
+    PaArgs& a = st->args;
+    out->clear();
+    if (!a.stamps) return FORGE_HIP_OK;
+    st->stamps_host.resize(st->n_stamps);
+    FH_HIP(hipMemcpyAsync(st->stamps_host.data(), a.stamps, st->n_stamps * 8, hipMemcpyDeviceToHost, s));
+    FH_HIP(hipStreamSynchronize(s));
+    for (uint32_t i = 0; i + 1 < st->n_stamps; i++)
+        out->push_back((float)((double)(st->stamps_host[i + 1] - st->stamps_host[i]) / (double)st->wall_khz));
+    return FORGE_HIP_OK;
+}
+
+}  // namespace fh

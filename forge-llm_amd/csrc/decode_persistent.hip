@@ -50,6 +50,7 @@
 #include "device_utils.h"
 #include "expf_ref.h"
 #include "gemv_order.h"
+#include "resident.h"
 
 namespace fh {
 
@@ -168,44 +169,6 @@ struct PdArgs {
 };
 static_assert(sizeof(PdArgs) <= 4096, "kernel arguments exceed 4 KB");
 
-// ---- plain global accesses -------------------------------------------------------------------------------
-// Pointers that reach the kernel through descriptors in memory have lost their address space; a load through
-// them would be a FLAT instruction, whose completion the compiler can only order with a full wait.  These
-// say "global" explicitly.
-typedef uint32_t pd_u32x4 __attribute__((ext_vector_type(4)));
-template <typename T>
-__device__ __forceinline__ T ldg(const T* p) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    if constexpr (sizeof(T) == 16) {
-        const pd_u32x4 v = *(const __attribute__((address_space(1))) pd_u32x4*)(uintptr_t)p;
-        T r;
-        __builtin_memcpy(&r, &v, 16);
-        return r;
-    } else {
-        static_assert(sizeof(T) <= 8, "ldg: scalar or 16-byte types only");
-        return *(const __attribute__((address_space(1))) T*)(uintptr_t)p;
-    }
-#else
-    return *p;
-#endif
-}
-template <typename T>
-__device__ __forceinline__ void stg(T* p, T v) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    *(__attribute__((address_space(1))) T*)(uintptr_t)p = v;
-#else
-    *p = v;
-#endif
-}
-
-// ---- coherent (agent-scope, L2-bypassing) accesses ----------------------------------------------------
-__device__ __forceinline__ uint64_t ldc64(const uint64_t* p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void stc64(uint64_t* p, uint32_t tag, uint32_t payload) {
-    __hip_atomic_store(p, ((uint64_t)tag << 32) | payload, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
 struct PdCtx {
     uint32_t tid, lane, wave, wg, G;
     uint32_t token;          // the token this step feeds
@@ -300,14 +263,6 @@ __device__ __forceinline__ void poll_vec(const uint64_t* base, uint32_t count, u
         for (int i = 0; i < N; i++)
             if (i0 + (uint32_t)i * nthreads < count) put(i0 + (uint32_t)i * nthreads, v[i]);
     }
-}
-
-__device__ __forceinline__ int dot16(int4 w, int4 a, int acc) {
-    acc = __builtin_amdgcn_sdot4(w.x, a.x, acc, false);
-    acc = __builtin_amdgcn_sdot4(w.y, a.y, acc, false);
-    acc = __builtin_amdgcn_sdot4(w.z, a.z, acc, false);
-    acc = __builtin_amdgcn_sdot4(w.w, a.w, acc, false);
-    return acc;
 }
 
 // ---- prologues: the activation vector of a GEMV phase, quantised, in LDS ------------------------------
@@ -1118,11 +1073,6 @@ __device__ __forceinline__ void pd_attn_exact_chain(const PxArgs& a, uint32_t po
 }
 
 // ---- argmax (project.rs:501-503): the LAST index among equal maxima --------------------------------------
-struct ArgPair { float v; uint32_t i; };
-__device__ __forceinline__ ArgPair arg_better(ArgPair a, ArgPair b) {
-    const bool take_b = (b.v > a.v) || (b.v == a.v && b.i > a.i);
-    return take_b ? b : a;
-}
 __device__ __forceinline__ ArgPair arg_wg(ArgPair a, float* misc, const PdCtx& cx) {
     auto fold = [&](auto O) { a = arg_better(a, ArgPair{lane_xor<O.value>(a.v), lane_xor<O.value>(a.i)}); };
     fold(std::integral_constant<int, 32>{}); fold(std::integral_constant<int, 16>{}); fold(std::integral_constant<int, 8>{});

@@ -60,6 +60,9 @@ struct LlamaModel : forge_hip_model {
     bool prefill_fuse_silu = false;              // fast mode: the gate/up GEMM writes silu(gate) * up quantised (FORGE_HIP_FUSE=0: separate kernel)
     bool fuse_norm = false, fuse_silu = false;   // fused GEMV prologue/epilogue variants fit LDS for this model
     PdState* pd = nullptr;               // the decode step as one resident kernel, when the shape is covered
+    PaState* pa = nullptr;               // the same for a narrow model, whatever the mode, over the short contexts that it covers
+    bool step_ahead = false;             // the step enqueued last is pa's
+    std::unique_ptr<ResidentSeat> seat;  // of a model that has either
     // ProjectionDTypes (ir.rs:410-421): q, k, v, o, gate, up, down each in its own storage format (GGML ids 8, 2, 12, 14).
     // `mixed`: they are not all cfg.wdtype, or the lm_head is a K-quant: every projection is then a GEMV launch of its own
     // and a prompt is walked token by token, as the reference does for such models (emit.rs:4530-4534, 4621-5040).
@@ -70,6 +73,7 @@ struct LlamaModel : forge_hip_model {
 
     ~LlamaModel() override {
         pd_destroy(pd);
+        pa_destroy(pa);
         for (auto& L : layers) {
             qweight_free(&L.qkv); qweight_free(&L.o); qweight_free(&L.gate_up); qweight_free(&L.down);
             qweight_free(&L.q); qweight_free(&L.k); qweight_free(&L.v); qweight_free(&L.gate); qweight_free(&L.up);
@@ -85,13 +89,26 @@ struct LlamaModel : forge_hip_model {
     void enqueue_row_logits(uint32_t row) override;
     bool keeps_rows() const override { return !mixed || mixed_batched; }
     int32_t decode_launches() const override;
-    bool resident() const override { return pd != nullptr; }
-    int32_t resident_enqueue(bool profile, uint32_t token) override { return pd_enqueue(pd, profile, token, stream); }
-    bool resident_wait_token(uint32_t* next) override { return pd_wait_token(pd, next); }
-    int32_t resident_after_sync(uint32_t abort_flag) override { return pd_after_sync(pd, abort_flag, stream); }
+    bool ahead() const { return pa && !pt.table && pa_covers(pa, pos); }
+    bool resident() const override { return ahead() || pd; }
+    int32_t resident_enqueue(bool profile, uint32_t token) override {
+        step_ahead = ahead();
+        return seat->turn(stream, [&] { return step_ahead ? pa_enqueue(pa, profile, token, stream) : pd_enqueue(pd, profile, token, stream); });
+    }
+    bool resident_wait_token(uint32_t* next) override { return step_ahead ? pa_wait_token(pa, next) : pd_wait_token(pd, next); }
+    int32_t resident_after_sync(uint32_t abort_flag) override {
+        return step_ahead ? pa_after_sync(pa, abort_flag, stream) : pd_after_sync(pd, abort_flag, stream);
+    }
     int32_t resident_profile(float* stage_ms, uint32_t* stage_launches) override;
-    int32_t repeat_penalty_changed(float penalty) override { return pd ? pd_set_repeat_penalty(pd, penalty) : FORGE_HIP_OK; }
-    void poll_limit_changed(uint32_t polls) override { if (pd) pd_set_poll_limit(pd, polls); }
+    int32_t repeat_penalty_changed(float penalty) override {
+        const int32_t rc = pd ? pd_set_repeat_penalty(pd, penalty) : FORGE_HIP_OK;
+        if (!rc && pa) pa_set_repeat_penalty(pa, penalty);
+        return rc;
+    }
+    void poll_limit_changed(uint32_t polls) override {
+        if (pd) pd_set_poll_limit(pd, polls);
+        if (pa) pa_set_poll_limit(pa, polls);
+    }
     int32_t set_kv_pages(uint32_t page_rows, const uint32_t* page_table_host, uint32_t n_pages) override;
     int32_t read_kv(uint32_t layer, uint32_t which, uint16_t* out_host) override;
 };
@@ -521,7 +538,7 @@ void LlamaModel::enqueue_row_logits(uint32_t row) {
 
 int32_t LlamaModel::resident_profile(float* stage_ms, uint32_t* stage_launches) {
     std::vector<float> ph;
-    const int32_t rc = pd_phase_ms(pd, &ph, stream);
+    const int32_t rc = step_ahead ? pa_phase_ms(pa, &ph, stream) : pd_phase_ms(pd, &ph, stream);
     if (rc) return rc;
     for (int i = 0; i < ST_COUNT; i++) { stage_ms[i] = 0.f; if (stage_launches) stage_launches[i] = 0; }
     // the second attention phase (merge of the splits, or the recurrence over the blocks, and the quantised row for the O
@@ -537,6 +554,7 @@ int32_t LlamaModel::resident_profile(float* stage_ms, uint32_t* stage_launches) 
 }
 
 int32_t LlamaModel::decode_launches() const {
+    if (ahead()) return 1;
     if (pd) return (int32_t)pd_launches_per_step(pd);
     const bool exact = (cfg.flags & FORGE_HIP_FLAG_EXACT) != 0;
     // order-faithful: three where the step is spread over the chip (without a window, past the one-launch form's line)
@@ -945,7 +963,16 @@ static int32_t model_create_impl(const forge_hip_config* cfg, const uint32_t* pd
                        m->sin_t.as<float>(), m->logits.as<float>(), m->state.as<uint32_t>(), m->counts.as<uint32_t>(),
                        has_bias ? m->biases.as<float>() : nullptr, &m->pd);
         if (rc) return rc;
+        // Narrow models over short contexts (decode_ahead.hip).  Where a variable asks for one of the other kernels' forms, it gets that.
+        auto set_to = [](const char* name, char v) { const char* e = getenv(name); return e && (v ? e[0] == v : true); };
+        if (!has_bias && !set_to("FORGE_HIP_PD_AHEAD", '0') && !set_to("FORGE_HIP_PD_ORDERED", '1') &&
+            !((cfg->flags & FORGE_HIP_FLAG_EXACT) && set_to("FORGE_HIP_PD_EXACT", 0))) {
+            rc = pa_create(*cfg, pl, m->lm_head, m->embed.as<float>(), m->final_norm.as<float>(), m->cos_t.as<float>(), m->sin_t.as<float>(),
+                           m->logits.as<float>(), m->state.as<uint32_t>(), m->counts.as<uint32_t>(), &m->pa);
+            if (rc) return rc;
+        }
     }
+    if (m->pd || m->pa) m->seat.reset(new ResidentSeat());
     FH_HIP(hipDeviceSynchronize());
     *out = m.release();
     return FORGE_HIP_OK;

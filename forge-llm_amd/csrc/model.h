@@ -45,6 +45,7 @@ struct forge_hip_model {
     float* h_logits = nullptr;           // pinned: logits come home at PCIe speed and are copied to the caller's (pageable) buffer from here
     int64_t pos = 0;
     bool use_graph = true;
+    bool step_resident = false;          // the step enqueued last is a resident kernel
     hipGraphExec_t decode_graph[2] = {nullptr, nullptr};      // by decode_form()
     // forward_profile / prefill_profile: one event pair per kernel launch, tagged with the stage of the
     // enclosing StageMark (ST_COUNT = outside any stage, not measured)
@@ -81,7 +82,8 @@ struct forge_hip_model {
     virtual int32_t decode_launches() const = 0;
 
     // ---- optional parts ------------------------------------------------------------------------------
-    // A step that is one resident kernel: it takes the token with the launch and hands the next one over through host memory.
+    // Whether the step at the host's position `pos` is one resident kernel: it takes the token with the launch and hands the next one over
+    // through host memory.
     virtual bool resident() const { return false; }
     virtual int32_t resident_enqueue(bool profile, uint32_t token) { (void)profile; (void)token; return FORGE_HIP_OK; }
     virtual bool resident_wait_token(uint32_t* next) { (void)next; return false; }

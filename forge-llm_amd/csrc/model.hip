@@ -8,7 +8,46 @@
 
 #include <string.h>
 
+#include <mutex>
+
 using namespace fh;
+
+namespace fh {
+
+namespace {
+std::mutex seat_mutex;
+uint32_t seats = 0;
+hipEvent_t seat_event = nullptr;          // behind the launch before; null until there was a second seat
+hipStream_t seat_stream = nullptr;
+}  // namespace
+
+ResidentSeat::Lock::Lock() { seat_mutex.lock(); }
+ResidentSeat::Lock::~Lock() { seat_mutex.unlock(); }
+ResidentSeat::ResidentSeat() {
+    const Lock lock;
+    // launches made while there was one seat left no event: they end here
+    if (++seats == 2) (void)hipDeviceSynchronize();
+}
+ResidentSeat::~ResidentSeat() {
+    const Lock lock;
+    if (--seats > 0) return;
+    if (seat_event) (void)hipEventDestroy(seat_event);
+    seat_event = nullptr;
+    seat_stream = nullptr;
+}
+int32_t ResidentSeat::before(hipStream_t s) {
+    if (seats > 1 && seat_event && seat_stream != s) FH_HIP(hipStreamWaitEvent(s, seat_event, 0));
+    return FORGE_HIP_OK;
+}
+int32_t ResidentSeat::after(hipStream_t s) {
+    if (seats < 2) return FORGE_HIP_OK;
+    if (!seat_event) FH_HIP(hipEventCreateWithFlags(&seat_event, hipEventDisableTiming));
+    seat_stream = s;
+    FH_HIP(hipEventRecord(seat_event, s));
+    return FORGE_HIP_OK;
+}
+
+}  // namespace fh
 
 void forge_hip_model::drop_decode_graphs() {
     for (hipGraphExec_t& g : decode_graph) {
@@ -115,7 +154,8 @@ int32_t capture_decode_step(forge_hip_model* m, hipGraphExec_t* graph) {
 }
 
 int32_t run_decode_step(forge_hip_model* m, uint32_t token) {
-    if (m->resident()) return m->resident_enqueue(false, token);   // the token rides with the launch
+    m->step_resident = m->resident();
+    if (m->step_resident) return m->resident_enqueue(false, token);   // the token rides with the launch
     m->h_stage[0] = token;
     FH_HIP(hipMemcpyAsync(m->d_token(), &m->h_stage[0], 4, hipMemcpyHostToDevice, m->stream));
     hipGraphExec_t& graph = m->decode_graph[m->decode_form()];
@@ -140,7 +180,7 @@ void capture_next_form(forge_hip_model* m) {
 int32_t finish_decode_step(forge_hip_model* m) {
     FH_HIP(hipMemcpyAsync(&m->h_stage[4], m->d_next(), 8, hipMemcpyDeviceToHost, m->stream));
     FH_HIP(hipStreamSynchronize(m->stream));
-    if (m->resident()) return m->resident_after_sync(m->h_stage[5]);
+    if (m->step_resident) return m->resident_after_sync(m->h_stage[5]);
     return FORGE_HIP_OK;
 }
 
@@ -245,7 +285,7 @@ int32_t forge_hip_forward_greedy(forge_hip_model* m, uint32_t token, uint32_t* n
     int32_t rc = forward_common(m, token);
     if (rc) return rc;
     // the resident kernel hands the token over through host memory as soon as it is final
-    if (m->resident() && m->resident_wait_token(next_token_host)) return FORGE_HIP_OK;
+    if (m->step_resident && m->resident_wait_token(next_token_host)) return FORGE_HIP_OK;
     rc = finish_or_undo(m);
     if (rc) return rc;
     *next_token_host = m->h_stage[4];
@@ -286,7 +326,8 @@ int32_t forge_hip_forward_profile(forge_hip_model* m, uint32_t token, float* sta
     FH_CHECK(m && stage_ms, "forward_profile: null pointer");
     if (m->pos >= (int64_t)m->cfg.max_seq) return fail(FORGE_HIP_ERR_POSITION, "KV cache is full (pos == max_seq)");
     if (token >= m->cfg.vocab) return fail(FORGE_HIP_ERR_POSITION, "token id out of range");
-    if (m->resident()) {
+    m->step_resident = m->resident();
+    if (m->step_resident) {
         // one kernel: the stages are its phases, timed by the kernel's own clock stamps
         int32_t rc = m->resident_enqueue(true, token);
         if (rc) return rc;

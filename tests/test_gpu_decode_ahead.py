@@ -1,0 +1,154 @@
+"""The resident decode kernel of narrow models (decode_ahead.hip) against the order-faithful kernel sequence, bit for bit."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+Q8, Q4, EXACT = 8, 2, 1
+
+
+def same_bits(got, want):
+    got, want = np.ascontiguousarray(got, np.float32), np.ascontiguousarray(want, np.float32)
+    diff = got.view(np.uint32) != want.view(np.uint32)
+    assert not diff.any(), f"{diff.sum()} of {diff.size} differ in bits; max abs err {np.max(np.abs(got - want)):.3e}"
+
+
+def pair(fh, monkeypatch, cfg, seed):
+    """(the kernel, the kernel sequence) over the same weights."""
+    blob = fh.synth.make_weights_blob(cfg, seed=seed, threads=16)
+    one = fh.HipModel(cfg, blob)
+    monkeypatch.setenv("FORGE_HIP_PD_AHEAD", "0")
+    seq = fh.HipModel(cfg, blob)
+    monkeypatch.delenv("FORGE_HIP_PD_AHEAD")
+    return one, seq
+
+
+def shape(fh, wd, hidden, inter, heads, kv_heads, head_dim, vocab, layers=3, lm=None, max_seq=1024):
+    cfg = fh.synth.tiny(wdtype=wd, max_seq=max_seq, hidden=hidden, inter=inter, layers=layers, heads=heads, kv_heads=kv_heads, head_dim=head_dim, vocab=vocab)
+    return dict(cfg, flags=EXACT, lm_head_dtype=lm or wd)
+
+
+# (format, hidden, inter, heads, kv heads, head dim, vocab, lm_head format): widths whose rows end inside a wave's and a workgroup's share, depths that are
+# no multiple of a group of products (24) or of a norm accumulator's (12), the widest and the narrowest vectors, one wave's rows per matrix, a vocabulary of a
+# few tiles and of a ragged number of them
+SHAPES = {
+    "smollm2": (Q8, 576, 1536, 9, 3, 64, 49152, None),
+    "narrow": (Q8, 64, 64, 1, 1, 64, 100, None),
+    "q4_ragged": (Q4, 608, 1056, 9, 1, 64, 4100, None),
+    "widest": (Q8, 768, 2048, 8, 2, 96, 3004, Q4),
+    "hd128": (Q4, 352, 736, 6, 2, 128, 1000, Q8),
+}
+
+
+@pytest.mark.parametrize("name", sorted(SHAPES))
+def test_equals_the_kernel_sequence(fh, torch_gpu, monkeypatch, name):
+    """Contexts that end inside a block of 64 keys, at its last key and at the first of the next, with one and with several blocks: logits, greedy tokens, cache."""
+    wd, *rest, lm = SHAPES[name]
+    cfg = shape(fh, wd, *rest, layers=2 if name == "smollm2" else 3, lm=lm)
+    one, seq = pair(fh, monkeypatch, cfg, 7)
+    toks = fh.synth.uniform_ids(8, 400, cfg["vocab"])
+    for n in (1, 60, 126, 380):
+        one.reset(); seq.reset()
+        same_bits(one.forward_prefill(toks[:n]), seq.forward_prefill(toks[:n]))
+        assert one.decode_launches == 1 and seq.decode_launches > 1
+        for t in toks[n:n + 4]:
+            assert one.forward_greedy(int(t)) == seq.forward_greedy(int(t))
+        for t in toks[n + 4:n + 7]:
+            same_bits(one.forward(int(t)), seq.forward(int(t)))
+    for layer in range(cfg["layers"]):
+        for which in (0, 1):
+            assert np.array_equal(one.read_kv(layer, which), seq.read_kv(layer, which))
+    one.close(); seq.close()
+
+
+@pytest.mark.parametrize("head_dim", [64, 128])
+def test_across_its_last_context_with_a_penalty(fh, torch_gpu, monkeypatch, head_dim):
+    """From the kernel to the sequence where the context outgrows a workgroup's blocks, and back after a reset, the repeat penalty's counts shared by both."""
+    cfg = shape(fh, Q8, 256, 512, 4, 2, head_dim, 1000)
+    one, seq = pair(fh, monkeypatch, cfg, 17)
+    toks = fh.synth.uniform_ids(18, 770, cfg["vocab"])
+    for turn in range(2):
+        for m in (one, seq):
+            m.reset()
+            m.set_repeat_penalty(1.3)
+            m.forward_prefill(toks[:764])
+        t = 5
+        for _ in range(8):
+            a, b = one.forward_greedy(t), seq.forward_greedy(t)
+            assert a == b
+            t = a
+        same_bits(one.forward(t), seq.forward(t))
+    one.close(); seq.close()
+
+
+def test_rewinds_its_tags_and_gives_up_instead_of_hanging(fh, torch_gpu, monkeypatch):
+    """Tags that are about to wrap, and a poll limit of 1: a step that gave up has not happened and can be fed again."""
+    cfg = shape(fh, Q8, 256, 512, 4, 2, 64, 1000)
+    monkeypatch.setenv("FORGE_HIP_PD_TAG_START", str(0xF0000000 - 40))
+    one, seq = pair(fh, monkeypatch, cfg, 27)
+    monkeypatch.delenv("FORGE_HIP_PD_TAG_START")
+    toks = [int(t) for t in fh.synth.uniform_ids(28, 24, cfg["vocab"])]
+    for m in (one, seq):
+        m.set_repeat_penalty(1.2)
+        m.forward_prefill(toks[:4])
+    for t in toks[4:12]:
+        assert one.forward_greedy(t) == seq.forward_greedy(t)
+    one.set_poll_limit(1)
+    failed = False
+    for t in toks[12:18]:
+        before = one.pos
+        try:
+            one.forward_greedy(t)
+        except fh.ForgeHipError as e:
+            assert e.code == fh.ERR_HIP and "gave up waiting" in str(e) and one.pos == before
+            failed = True
+            break
+        seq.forward_greedy(t)
+    assert failed, "no step gave up with a poll limit of 1"
+    one.set_poll_limit(0)
+    assert one.forward_greedy(t) == seq.forward_greedy(t)
+    for t in toks[18:]:
+        same_bits(one.forward(t), seq.forward(t))
+    one.close(); seq.close()
+
+
+def test_fast_mode_takes_it_too(fh, oracle, torch_gpu):
+    """Fast mode: from the same cache the kernel's step is the order-faithful one.  A prompt of one token leaves the cache that both modes' first step leaves."""
+    cfg = shape(fh, Q8, 256, 512, 4, 2, 64, 1000)
+    blob = fh.synth.make_weights_blob(cfg, seed=37)
+    fast, om = fh.HipModel(dict(cfg, flags=0), blob), oracle.Model(cfg, blob, 0, 1)
+    toks = fh.synth.uniform_ids(38, 70, cfg["vocab"])
+    fast.forward(int(toks[0])); om.forward(int(toks[0]))
+    assert fast.decode_launches == 1
+    for t in toks[1:]:
+        a, b = fast.forward(int(t)), om.forward(int(t))
+    assert np.corrcoef(a, b)[0, 1] > 0.999
+    fast.close()
+
+
+def test_models_of_several_threads_take_turns(fh, torch_gpu):
+    """Two models step at the same time: each kernel needs the whole device, so their launches follow one another, and the tokens are those of a model alone."""
+    import threading
+    cfg = shape(fh, Q8, 256, 512, 4, 2, 64, 1000)
+    blob = fh.synth.make_weights_blob(cfg, seed=47)
+    prompt = fh.synth.uniform_ids(48, 30, cfg["vocab"])
+
+    def generate(m):
+        m.reset()
+        return m.generate_greedy(prompt, 200)
+
+    models = [fh.HipModel(cfg, blob) for _ in range(2)]
+    want = generate(models[0])
+    got = [None, None]
+
+    def work(i):
+        got[i] = generate(models[i])
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert got[0] == want and got[1] == want
+    for m in models:
+        m.close()
