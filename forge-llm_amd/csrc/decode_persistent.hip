@@ -66,8 +66,8 @@ constexpr int PD_POLL_WAVES = 2;              // waves that fetch a phase's inpu
 constexpr int PD_POLL_THREADS = PD_POLL_WAVES * 64;
 constexpr int PD_STREAM_WAVES = PD_WAVES - PD_POLL_WAVES;
 constexpr int PD_POLL_N = 20;                 // tagged elements a poller thread takes per round trip
-// misc LDS (floats): [0,33) norm partial sums, [40] hint flag, [64,128) phase scratch
-constexpr int PD_MISC_HINT = 40, PD_MISC_SCRATCH = 64;
+// misc LDS (floats): [0,33) norm partial sums, [64,128) phase scratch
+constexpr int PD_MISC_SCRATCH = 64;
 // misc LDS words [PD_MISC_PT, 512): page-table entries of this workgroup's attention items, staged once per step (an item's
 // key range is the same in every layer); slot (round, wave group) holds pt_cap entries
 constexpr int PD_MISC_PT = 128, PD_MISC_PT_WORDS = 512 - PD_MISC_PT;
@@ -160,7 +160,6 @@ struct PdArgs {
     uint32_t window;                           // != 0: attention over the last `window` positions only (sliding window)
     PageTable pt;                              // paged KV cache (table == nullptr: flat); pt_cap: table entries an attention item may span
     uint32_t pt_cap;
-    uint32_t use_hint;                         // pollers wait for one watched element before re-reading a whole buffer
     uint32_t off_act_s, off_misc, off_big;     // LDS byte offsets (activation codes sit at 0)
     unsigned long long* stamps;                // optional: wall clock at the start of every phase (workgroup 0)
     // Kernel arguments are read with scalar loads, which have their own completion counter: a wave can
@@ -202,37 +201,20 @@ __device__ __forceinline__ uint32_t poll(const uint64_t* p, uint32_t tag, const 
     return (uint32_t)w;
 }
 
-// Thousands of threads re-reading a buffer that is not ready yet would flood the memory fabric the weight
-// stream needs.  After a first attempt that found something missing, the pollers of a workgroup therefore
-// wait (on an LDS flag) until thread 0 has seen one watched element of the buffer arrive, which in a
-// balanced phase is when the rest is about to.
-struct Hint { const uint64_t* sentinel; volatile uint32_t* flag; };
-
-// Up to N elements per thread: all loads are issued before any tag is looked at, so a hand-over costs one
-// memory round trip however many elements a thread takes; only elements still carrying another tag are re-read.
+// N elements per thread: all loads are issued before any tag is looked at, so a hand-over costs one memory round trip however many elements a thread
+// takes, and all are read again until the last has arrived.  No condition around a load: with one per element a thread's 16 elements cost 200 instructions a
+// pass (1B shape at a context of 2400: 687 us per step, 644 without).
 template <int N, typename Addr>
-__device__ __forceinline__ void poll_many(Addr addr, uint32_t n, uint32_t tag, uint32_t* out, const PdCtx& cx, Hint hint) {
+__device__ __forceinline__ void poll_many(Addr addr, uint32_t tag, uint32_t* out, const PdCtx& cx) {
     uint64_t w[N];
-#pragma unroll
-    for (int i = 0; i < N; i++) w[i] = (uint32_t)i < n ? ldc64(addr(i)) : ((uint64_t)tag << 32);
-    if (hint.flag && cx.tid == 0) {
-        (void)poll(hint.sentinel, tag, cx);
-        *hint.flag = tag;
-    }
     uint32_t spins = 0;
-    bool waited = hint.flag == nullptr;
     for (;;) {
-        bool ok = true;
 #pragma unroll
-        for (int i = 0; i < N; i++) ok = ok && (uint32_t)(w[i] >> 32) == tag;
-        if (ok) break;
-        if (!waited) {
-            uint32_t s2 = 0;
-            while (*hint.flag != tag && *cx.sh_abort == 0 && ++s2 < cx.spin_limit) __builtin_amdgcn_s_sleep(4);
-            waited = true;
-        } else {
-            __builtin_amdgcn_s_sleep(2);
-        }
+        for (int i = 0; i < N; i++) w[i] = ldc64(addr(i));
+        uint32_t off = 0;
+#pragma unroll
+        for (int i = 0; i < N; i++) off |= (uint32_t)(w[i] >> 32) ^ tag;
+        if (!off) break;
         ++spins;
         if (spins > cx.spin_limit ||
             ((spins & 1023u) == 0 && __hip_atomic_load(cx.abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
@@ -240,30 +222,33 @@ __device__ __forceinline__ void poll_many(Addr addr, uint32_t n, uint32_t tag, u
             __hip_atomic_store(cx.abort_flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             break;
         }
-#pragma unroll
-        for (int i = 0; i < N; i++)
-            if ((uint32_t)(w[i] >> 32) != tag) w[i] = ldc64(addr(i));
+        __builtin_amdgcn_s_sleep(1);
     }
 #pragma unroll
     for (int i = 0; i < N; i++) out[i] = (uint32_t)w[i];
 }
 
-// A whole vector of `count` elements fetched by the first `nthreads` threads of the workgroup, N per thread and
-// round trip; `put(index, payload)` stores each.  Threads past nthreads return at once.
-template <int N, typename Put>
-__device__ __forceinline__ void poll_vec(const uint64_t* base, uint32_t count, uint32_t tag, uint32_t nthreads, const PdCtx& cx,
-                                         Hint hint, Put put) {
-    if (cx.tid >= nthreads) return;
-    for (uint32_t i0 = cx.tid; i0 < count; i0 += N * nthreads) {
-        uint32_t v[N];
-        const uint32_t n = (count - i0 + nthreads - 1) / nthreads;
-        poll_many<N>([&](int i) { return base + i0 + (uint32_t)i * nthreads; }, n < (uint32_t)N ? n : (uint32_t)N, tag, v, cx, hint);
-        hint.flag = nullptr;      // later passes: the buffer is known to be arriving
-#pragma unroll
-        for (int i = 0; i < N; i++)
-            if (i0 + (uint32_t)i * nthreads < count) put(i0 + (uint32_t)i * nthreads, v[i]);
+// A whole vector of `count` elements fetched by the first NT threads of the workgroup, up to N (a multiple of 4) per thread and round trip;
+// `put(index, payload)` stores each.  Threads past NT return at once.  A slot past the last element re-reads that one.
+template <int N, uint32_t NT, typename Put>
+__device__ __forceinline__ void poll_slots(const uint64_t* base, uint32_t count, uint32_t tag, const PdCtx& cx, Put put) {
+    if constexpr (N > 4) {
+        if (count <= (N - 4) * NT) { poll_slots<N - 4, NT>(base, count, tag, cx, put); return; }
     }
+    uint32_t v[N];
+    poll_many<N>([&](int i) { return base + (i < N - 4 ? cx.tid + i * NT : min(cx.tid + i * NT, count - 1)); }, tag, v, cx);
+#pragma unroll
+    for (int i = 0; i < N; i++)
+        if (i < N - 4 || cx.tid + i * NT < count) put(cx.tid + i * NT, v[i]);
 }
+template <int N, uint32_t NT, typename Put>
+__device__ __forceinline__ void poll_vec(const uint64_t* base, uint32_t count, uint32_t tag, const PdCtx& cx, Put put) {
+    static_assert(N % 4 == 0, "poll_slots goes by fours");
+    if (cx.tid >= NT) return;
+#pragma nounroll
+    for (uint32_t at = 0; at < count; at += N * NT) poll_slots<N, NT>(base + at, min(count - at, N * NT), tag, cx, [&](uint32_t i, uint32_t p) { put(at + i, p); });
+}
+
 
 // ---- prologues: the activation vector of a GEMV phase, quantised, in LDS ------------------------------
 // rms_norm (emit.rs:327-334, 16-lane FMA order of emit.rs:272-295) + activation quantiser (emit.rs:1410-1440).
@@ -333,10 +318,9 @@ __device__ __forceinline__ void pd_norm_quant(float* xs, const float* __restrict
 
 // An already quantised vector (codes then scales, tagged) from another phase; fetched by the poller waves.
 __device__ __forceinline__ void pd_load_aq(const uint64_t* t, uint32_t tag, uint32_t K, uint32_t* aq_lds, float* as_lds,
-                                           float* misc, bool use_hint, const PdCtx& cx) {
+                                           const PdCtx& cx) {
     const uint32_t nq = K / 4, ns = K / 32;
-    const Hint hint{t + nq + ns - 1, use_hint ? reinterpret_cast<volatile uint32_t*>(misc + PD_MISC_HINT) : nullptr};
-    poll_vec<PD_POLL_N>(t, nq + ns, tag, PD_POLL_THREADS, cx, hint, [&](uint32_t i, uint32_t p) {
+    poll_vec<PD_POLL_N, PD_POLL_THREADS>(t, nq + ns, tag, cx, [&](uint32_t i, uint32_t p) {
         if (i < nq) aq_lds[i] = p;
         else as_lds[i - nq] = f16_bits_to_f32((uint16_t)p);
     });
@@ -344,10 +328,8 @@ __device__ __forceinline__ void pd_load_aq(const uint64_t* t, uint32_t tag, uint
 
 // The residual stream (tagged) into LDS as floats; fetched by the poller waves.
 // `ssq` collects the squares of what this thread fetched.
-__device__ __forceinline__ void pd_load_x(const uint64_t* tx, uint32_t tag, uint32_t H, float* xs, float* misc, bool use_hint,
-                                          const PdCtx& cx, float& ssq) {
-    const Hint hint{tx + H - 1, use_hint ? reinterpret_cast<volatile uint32_t*>(misc + PD_MISC_HINT) : nullptr};
-    poll_vec<PD_POLL_N>(tx, H, tag, PD_POLL_THREADS, cx, hint, [&](uint32_t i, uint32_t p) {
+__device__ __forceinline__ void pd_load_x(const uint64_t* tx, uint32_t tag, uint32_t H, float* xs, const PdCtx& cx, float& ssq) {
+    poll_vec<PD_POLL_N, PD_POLL_THREADS>(tx, H, tag, cx, [&](uint32_t i, uint32_t p) {
         const float v = __uint_as_float(p);
         xs[i] = v;
         ssq += v * v;
@@ -591,19 +573,25 @@ __device__ __forceinline__ void merge_state(float& m, float& l, float* a, float 
 
 // Key range [t0, t1) of attention work item number `round` of wave group `grp` of this workgroup (the items of
 // attn_decode_split_kernel: kv head group x split), and which item it is.  The same in every layer of a step.
-struct PdItem { uint32_t item, n_items, nbx, t0, t1, seq, start, chunk; bool on; };
-template <int HD>
+struct PdItem { uint32_t item, n_items, nbx, t0, t1, seq, start, chunk; bool on, one; };
+// Up to this many keys (and where nothing asks for the kernel sequence's bits or a page table) a kv head group is ONE item whose workgroup finishes the heads itself:
+// no merge phase behind the splits.  128 keys are what the waves request at once: 1B shape, us per step, with the merge / without: 33 keys 637 / 610, 100 keys 637 / 613;
+// a second round of keys costs more than the merge (200 keys 636 / 647).
+constexpr uint32_t PD_ONE_KEYS = 128;
+template <int HD, bool ORD>
 __device__ __forceinline__ PdItem pd_attn_item(const PdArgs& a, uint32_t pos, uint32_t round, uint32_t grp, const PdCtx& cx) {
     constexpr int LPK = HD <= 64 ? 8 : 16;
     constexpr int KPW = 64 / LPK;
     const bool dual = a.gt == 1;
     const uint32_t gsize = a.heads / a.kv_heads, gpk = gsize / a.gt;
     PdItem r;
-    r.nbx = a.kv_heads * gpk; r.n_items = r.nbx * DECODE_SPLITS;
+    r.nbx = a.kv_heads * gpk;
     r.seq = pos + 1;
     // attention_sliding (emit.rs:598-627): only the last `window` rows are keys (window 0: all of them)
     r.start = (a.window != 0 && r.seq > a.window) ? r.seq - a.window : 0;
-    r.chunk = (r.seq - r.start + DECODE_SPLITS - 1) / DECODE_SPLITS;
+    r.one = !ORD && !a.pt.table && r.seq - r.start <= PD_ONE_KEYS;
+    r.n_items = r.one ? r.nbx : r.nbx * DECODE_SPLITS;
+    r.chunk = r.one ? r.seq - r.start : (r.seq - r.start + DECODE_SPLITS - 1) / DECODE_SPLITS;
     r.chunk = (r.chunk + 4 * KPW - 1) / (4 * KPW) * (4 * KPW);
     r.item = cx.wg + (dual ? 2 * round + grp : round) * cx.G;
     r.on = r.item < r.n_items;
@@ -614,18 +602,29 @@ __device__ __forceinline__ PdItem pd_attn_item(const PdArgs& a, uint32_t pos, ui
 }
 
 // Paged cache: the table entries of every item of this workgroup, into LDS, once per step.
-template <int HD>
+template <int HD, bool ORD>
 __device__ __forceinline__ void pd_stage_pages(const PdArgs& a, uint32_t pos, uint32_t* pts, const PdCtx& cx) {
     if (!a.pt.table) return;
     const bool dual = a.gt == 1;
-    const PdItem any = pd_attn_item<HD>(a, pos, 0, 0, cx);
+    const PdItem any = pd_attn_item<HD, ORD>(a, pos, 0, 0, cx);
     const uint32_t per_round = dual ? 2 * cx.G : cx.G, rounds = (any.n_items + per_round - 1) / per_round;
     for (uint32_t s = 0; s < rounds * (dual ? 2u : 1u); s++) {
-        const PdItem it = pd_attn_item<HD>(a, pos, dual ? s >> 1 : s, dual ? s & 1u : 0u, cx);
+        const PdItem it = pd_attn_item<HD, ORD>(a, pos, dual ? s >> 1 : s, dual ? s & 1u : 0u, cx);
         if (it.t1 <= it.t0) continue;
         const uint32_t first = it.t0 >> a.pt.shift, n = ((it.t1 - 1) >> a.pt.shift) - first + 1;
         for (uint32_t i = cx.tid; i < n && i < a.pt_cap; i += PD_THREADS) pts[s * a.pt_cap + i] = a.pt.table[first + i];
     }
+}
+
+// Element e of the attention's output, one per lane of whole half waves: quantised for the O GEMV and handed over.
+__device__ __forceinline__ void pd_store_head(const PdArgs& a, uint32_t e, float o, uint32_t tag_out) {
+    const float amax = half_wave_max(fabsf(o));
+    float inv;
+    const float sc = act_scale(amax, inv);
+    const uint32_t code = (uint32_t)quant_code(o * inv) & 0xFFu;
+    const uint32_t pk = quad_broadcast<0>(code) | (quad_broadcast<1>(code) << 8) | (quad_broadcast<2>(code) << 16) | (quad_broadcast<3>(code) << 24);
+    if ((e & 3u) == 0) stc64(a.taq + e / 4, tag_out, pk);
+    if ((e & 31u) == 0) stc64(a.taq + a.QKS / 4 + e / 32, tag_out, f32_to_f16_bits(sc));
 }
 
 // P2: the work items of attn_decode_split_kernel (kv head group x split), one per workgroup at a time.  The
@@ -633,8 +632,9 @@ __device__ __forceinline__ void pd_stage_pages(const PdArgs& a, uint32_t pos, ui
 // 4 g + w carries head g over the keys wave w would take (same keys, same order, same merges), which
 // keeps the per-thread state small.  Keys before this position come from the cache, this position's K/V
 // row and q from the tagged buffers P1 filled.
-template <int HD>
-__device__ __forceinline__ void pd_attn_split(const PdArgs& a, const uint16_t* kc, const uint16_t* vc, uint32_t pos, uint32_t tag_in,
+// Returns whether the heads are finished (PdItem::one): the quantised rows are then on their way as pd_attn_combine would send them.
+template <int HD, bool ORD>
+__device__ __forceinline__ bool pd_attn_split(const PdArgs& a, const uint16_t* kc, const uint16_t* vc, uint32_t pos, uint32_t tag_in,
                                               uint32_t tag_out, float* big, const uint32_t* pts, const PdCtx& cx) {
     constexpr int LPK = HD <= 64 ? 8 : 16;
     constexpr int KPW = 64 / LPK;
@@ -650,7 +650,8 @@ __device__ __forceinline__ void pd_attn_split(const PdArgs& a, const uint16_t* k
     float* sh = big + grp * AREA;                                     // [4 waves][4][REC]
     float* q_lds = sh + 16 * REC;                                     // [gt][HD]
     uint32_t* kvn = reinterpret_cast<uint32_t*>(q_lds + 4 * HD);      // [2][HD] fp16 bits of this position's K and V
-    const uint32_t nbx = a.kv_heads * gpk, n_items = nbx * DECODE_SPLITS;
+    const PdItem any = pd_attn_item<HD, ORD>(a, pos, 0, 0, cx);
+    const uint32_t nbx = any.nbx, n_items = any.n_items;
     const uint32_t c = lane % LPK, slot = lane / LPK;
     const bool dvalid = c * 8 < HD;
     const float scale = 1.0f / sqrtf((float)HD);
@@ -662,7 +663,7 @@ __device__ __forceinline__ void pd_attn_split(const PdArgs& a, const uint16_t* k
     const uint32_t per_round = dual ? 2 * cx.G : cx.G;
     const uint32_t rounds = (n_items + per_round - 1) / per_round;
     for (uint32_t it = 0; it < rounds; it++) {
-        const PdItem itm = pd_attn_item<HD>(a, pos, it, grp, cx);
+        const PdItem itm = pd_attn_item<HD, ORD>(a, pos, it, grp, cx);
         const uint32_t item = itm.item;
         const bool on = itm.on;
         const uint32_t bx = item % nbx, split = item / nbx;
@@ -705,12 +706,12 @@ __device__ __forceinline__ void pd_attn_split(const PdArgs& a, const uint16_t* k
             const uint64_t* pkv = a.tkv + (e < HD ? kvh * HD + e : a.KV + kvh * HD + (e - HD));
             uint32_t v[2];
             // one batch: an element that is not needed re-reads the needed one
-            poll_many<2>([&](int i) { return (i == 0 ? need_q : !need_kv) ? pq : pkv; }, 2, tag_in, v, cx, Hint{nullptr, nullptr});
+            poll_many<2>([&](int i) { return (i == 0 ? need_q : !need_kv) ? pq : pkv; }, tag_in, v, cx);
             if (need_q) q_lds[e] = __uint_as_float(v[0]);
             if (need_kv) kvn[e] = v[1];
         }
         __syncthreads();
-        if (*cx.sh_abort) return;
+        if (*cx.sh_abort) return true;
 #pragma unroll
         for (int u = 0; u < UNR; u++) {                      // this position's row arrived with q
             const uint32_t t = tbw + u * 4 * KPW + slot;
@@ -809,12 +810,17 @@ __device__ __forceinline__ void pd_attn_split(const PdArgs& a, const uint16_t* k
                 float a2 = sh[(w * 4 + gg) * REC + d];
                 merge_state<1>(mm, ll, &av, sh[(w * 4 + gg) * REC + HD], sh[(w * 4 + gg) * REC + HD + 1], &a2);
             }
-            uint64_t* rec = a.tws + ((size_t)(h0 + gg) * DECODE_SPLITS + split) * REC;
-            stc64(rec + d, tag_out, __float_as_uint(av));
-            if (d == 0) { stc64(rec + HD, tag_out, __float_as_uint(mm)); stc64(rec + HD + 1, tag_out, __float_as_uint(ll)); }
+            if (any.one) {
+                pd_store_head(a, (h0 + gg) * HD + d, av * (1.0f / ll), tag_out + 1);
+            } else {
+                uint64_t* rec = a.tws + ((size_t)(h0 + gg) * DECODE_SPLITS + split) * REC;
+                stc64(rec + d, tag_out, __float_as_uint(av));
+                if (d == 0) { stc64(rec + HD, tag_out, __float_as_uint(mm)); stc64(rec + HD + 1, tag_out, __float_as_uint(ll)); }
+            }
         }
         __syncthreads();
     }
+    return any.one;
 }
 
 // P3: attn_decode_combine_kernel, one head per workgroup at a time; output quantised for the O GEMV.  All
@@ -828,7 +834,7 @@ __device__ __forceinline__ void pd_attn_combine(const PdArgs& a, uint32_t tag_in
     float* recs = big;                           // [DECODE_SPLITS][REC]
     for (uint32_t h = cx.wg; h < a.heads; h += cx.G) {
         const uint64_t* base = a.tws + (size_t)h * DECODE_SPLITS * REC;
-        poll_vec<(DECODE_SPLITS * REC + PD_THREADS - 1) / PD_THREADS>(base, DECODE_SPLITS * REC, tag_in, PD_THREADS, cx, Hint{nullptr, nullptr},
+        poll_vec<(DECODE_SPLITS * REC + 4 * PD_THREADS - 1) / (4 * PD_THREADS) * 4, PD_THREADS>(base, DECODE_SPLITS * REC, tag_in, cx,
                     [&](uint32_t i, uint32_t p) { recs[i] = __uint_as_float(p); });
         __syncthreads();
         if (*cx.sh_abort) return;
@@ -847,15 +853,7 @@ __device__ __forceinline__ void pd_attn_combine(const PdArgs& a, uint32_t tag_in
 #pragma unroll
             for (uint32_t s = 0; s < DECODE_SPLITS; s++) num = fmaf(wgt_s[s], recs[s * REC + d], num);
             const float o = num * (1.0f / wgt_s[DECODE_SPLITS]);
-            const float amax = half_wave_max(fabsf(o));
-            float inv;
-            const float sc = act_scale(amax, inv);
-            const uint32_t code = (uint32_t)quant_code(o * inv) & 0xFFu;
-            const uint32_t pk = quad_broadcast<0>(code) | (quad_broadcast<1>(code) << 8) | (quad_broadcast<2>(code) << 16) |
-                                (quad_broadcast<3>(code) << 24);
-            const uint32_t e = h * HD + d;
-            if ((d & 3u) == 0) stc64(a.taq + e / 4, tag_out, pk);
-            if ((d & 31u) == 0) stc64(a.taq + a.QKS / 4 + e / 32, tag_out, f32_to_f16_bits(sc));
+            pd_store_head(a, h * HD + d, o, tag_out);
         }
         __syncthreads();
     }
@@ -943,7 +941,7 @@ __device__ __forceinline__ void pd_attn_exact_blocks(const PxArgs& a, const uint
                 const uint32_t e = lane + 64u * (uint32_t)j < (uint32_t)HD ? lane + 64u * (uint32_t)j : lane % 32u;
                 return (i < NQ || !has_new) ? pq + e : (i < 2 * NQ ? pk + e : pv + e);
             };
-            poll_many<3 * NQ>(addr, 3 * NQ, tag_in, got, cx, Hint{nullptr, nullptr});
+            poll_many<3 * NQ>(addr, tag_in, got, cx);
         }
         // ---- scores (sequential q.k sums, lane = key) and the block maximum
         float sum = 0.f;
@@ -968,8 +966,7 @@ __device__ __forceinline__ void pd_attn_exact_blocks(const PxArgs& a, const uint
         float m = mb;
         for (uint32_t j0 = 0; j0 < b; j0 += 128) {
             uint32_t v[2];
-            poll_many<2>([&](int i) { return a.tbm + (size_t)h * a.nb_cap + min(j0 + lane + 64u * (uint32_t)i, b - 1); }, 2, tag_out, v, cx,
-                         Hint{nullptr, nullptr});
+            poll_many<2>([&](int i) { return a.tbm + (size_t)h * a.nb_cap + min(j0 + lane + 64u * (uint32_t)i, b - 1); }, tag_out, v, cx);
             m = fmaxf(m, fmaxf(__uint_as_float(v[0]), __uint_as_float(v[1])));
         }
         m = wave_max(m);
@@ -1019,7 +1016,7 @@ __device__ __forceinline__ void pd_attn_exact_chain(const PxArgs& a, uint32_t po
         for (uint32_t c0 = 0; c0 < nb; c0 += PX_CHUNK) {
             const uint32_t n = min(PX_CHUNK, nb - c0);
             const uint64_t* base = a.trec + ((size_t)h * a.nb_cap + c0) * REC;
-            poll_vec<(PX_CHUNK * REC + PD_THREADS - 1) / PD_THREADS>(base, n * REC, tag_in, PD_THREADS, cx, Hint{nullptr, nullptr},
+            poll_vec<(PX_CHUNK * REC + 4 * PD_THREADS - 1) / (4 * PD_THREADS) * 4, PD_THREADS>(base, n * REC, tag_in, cx,
                         [&](uint32_t i, uint32_t p) { recs[i] = __uint_as_float(p); });
             __syncthreads();
             if (*cx.sh_abort) return;
@@ -1129,8 +1126,8 @@ __device__ __forceinline__ void pd_gemv_phase(const PdArgs& a, const GemvJob& jo
         if (!early) load_round(t, 0, W);                                  // otherwise the previous phase's tail issued them
     } else {
         float ssq = 0.f;
-        if (job.pro == PRO_AQ) pd_load_aq(job.tin, job.tin_tag, K, aq_lds, as_lds, misc, a.use_hint != 0, cx);
-        else if (job.tin_tag) pd_load_x(job.tin, job.tin_tag, K, xs, misc, a.use_hint != 0, cx, ssq);
+        if (job.pro == PRO_AQ) pd_load_aq(job.tin, job.tin_tag, K, aq_lds, as_lds, cx);
+        else if (job.tin_tag) pd_load_x(job.tin, job.tin_tag, K, xs, cx, ssq);
         else for (uint32_t i = cx.tid; i < K; i += PD_POLL_THREADS) { const float v = emb[i]; xs[i] = v; ssq += v * v; }
         if (!ORDERED && job.pro == PRO_NORM) {
             // the pollers square what they fetched: the sum of squares needs no pass (and no barrier) of its own
@@ -1306,7 +1303,7 @@ __global__ __launch_bounds__(PD_THREADS) void decode_step_kernel(PdArgs a) {
     cx.spin_limit = a.spin_limit;
     cx.sh_abort = &sh_abort;
     cx.abort_flag = a.state + 3;
-    if (cx.tid == 0) { sh_abort = 0; reinterpret_cast<uint32_t*>(misc)[PD_MISC_HINT] = 0; }
+    if (cx.tid == 0) sh_abort = 0;
     cx.exp_tab = reinterpret_cast<const uint64_t*>(misc + PD_MISC_EXP);
     if (ORD && cx.tid < 32) reinterpret_cast<uint64_t*>(misc + PD_MISC_EXP)[cx.tid] = expf_detail::tab((int)cx.tid);
     __syncthreads();
@@ -1314,7 +1311,7 @@ __global__ __launch_bounds__(PD_THREADS) void decode_step_kernel(PdArgs a) {
     const uint32_t pos = a.state[0], token = a.token_from_arg ? a.token : a.state[1];
     const size_t crow = paged_row(a.pt, pos);        // row of the cache (pool) that this position's K and V go to
     uint32_t* pts = reinterpret_cast<uint32_t*>(misc) + PD_MISC_PT;
-    pd_stage_pages<HD>(a, pos, pts, cx);             // published by the first barrier of the first phase
+    pd_stage_pages<HD, ORD>(a, pos, pts, cx);             // published by the first barrier of the first phase
     const float* emb = a.embed + (size_t)token * a.H;
     cx.token = token;
     const uint32_t L = a.n_layers;
@@ -1345,10 +1342,10 @@ __global__ __launch_bounds__(PD_THREADS) void decode_step_kernel(PdArgs a) {
                 __syncthreads();
                 if (sh_abort) return;
             } else {
-                pd_attn_split<HD>(a, a.layers[l].kc, a.layers[l].vc, pos, base + 1, base + 2, big, pts, cx);
+                const bool done = pd_attn_split<HD, ORD>(a, a.layers[l].kc, a.layers[l].vc, pos, base + 1, base + 2, big, pts, cx);
                 if (sh_abort) return;
                 if (a.stamps && cx.wg == 0 && cx.tid == 0) a.stamps[6 * lg + 2] = wall_clock64();
-                pd_attn_combine<HD>(a, base + 2, base + 3, misc, big, cx);
+                if (!done) pd_attn_combine<HD>(a, base + 2, base + 3, misc, big, cx);
                 if (sh_abort) return;
             }
             pd_forget(W);          // the O projection loads its first round itself (`early` is false here)
@@ -1431,7 +1428,7 @@ __global__ __launch_bounds__(PD_THREADS) void decode_step_kernel(PdArgs a) {
         ArgPair p{-INFINITY, 0};
         for (uint32_t w = cx.tid; w < cx.G; w += PD_THREADS) {
             uint32_t v[2];
-            poll_many<2>([&](int i) { return a.tpart + 2 * w + (uint32_t)i; }, 2, th, v, cx, Hint{nullptr, nullptr});
+            poll_many<2>([&](int i) { return a.tpart + 2 * w + (uint32_t)i; }, th, v, cx);
             p = arg_better(p, ArgPair{__uint_as_float(v[0]), v[1]});
         }
         p = arg_wg(p, misc, cx);
@@ -1862,11 +1859,6 @@ int32_t pd_create(const forge_hip_config& c, const std::vector<PdLayerIn>& layer
     // FORGE_HIP_PD_SPIN_LIMIT: how often a wait re-reads before the workgroup gives up (a test sets it to 1 to walk the
     // give-up path: every wait in the kernel is bounded by it, so the kernel still ends normally)
     { const char* e = getenv("FORGE_HIP_PD_SPIN_LIMIT"); if (e && atoi(e) > 0) a.spin_limit = (uint32_t)atoi(e); }
-    // The watcher (one thread polls one element of a buffer, the other pollers wait for its word in LDS before they re-read
-    // what they missed) pays on narrow models, where a phase is nothing but its hand-over (hidden 576: +2 %); from a hidden
-    // size of 1024 up the pollers re-read on their own (1B +1.0 %, 3B +1.7 %, 8B +0.9 % over the watcher).
-    // FORGE_HIP_PD_HINT=0 / 1 forces either.
-    { const char* e = getenv("FORGE_HIP_PD_HINT"); a.use_hint = e ? (e[0] == '0' ? 0 : 1) : (a.H < 1024 ? 1 : 0); }
     a.token = 0; a.token_from_arg = 0; a.host_out = nullptr; a.host_seq = 0;
     // All workgroups are co-resident by construction (one per CU, checked above), and every wait in the kernel is
     // bounded, so an ordinary launch is enough; it costs ~7 us less per step than a cooperative one.
