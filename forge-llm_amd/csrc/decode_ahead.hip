@@ -1,23 +1,24 @@
-// One decode token of a narrow model as ONE kernel whose waves hold their share of a layer's matrices in registers (model::forward, emit.rs:4029-4227).
+// One decode token over a short context as ONE kernel whose waves hold their share of a layer's matrices in registers (model::forward, emit.rs:4029-4227).
 //
-// A step of a model of a few hundred channels is a chain of four short products and an attention per layer; neither bytes nor arithmetic bound it but what
-// lies between them.  As kernels a link of that chain is 4 to 6 us (a launch that does nothing takes 2.7); as phases of the kernel for wide models
-// (decode_persistent.hip) it is 5.  Here a layer of SmolLM2-135M takes 14 us: five hand-overs of 0.8 to 1.2, two norms of 1.1, attention 3.3, and the products.
-//   * A wave's rows of the four matrices are a few registers (a lane holds at most UQ + UO + UG + UD blocks of 32 weights), all requested while the attention
-//     is at work: no product waits for memory, and nothing that comes from far is on its way to a compute unit that waits for a vector.  (A compute unit's
-//     loads return in order: weights requested behind each product held the next hand-over up by 2 to 3 us.)
+// A step is a chain of four products and an attention per layer.  As kernels a link of that chain is 4 to 6 us however small (a launch that does nothing takes
+// 2.7); as phases of the kernel that streams weights of any size (decode_persistent.hip) it is 5.  Here a layer of SmolLM2-135M takes 13 us, one of the 1B shape 24
+// (its 65 MB alone take 14): five hand-overs of 0.8 to 1.2 (1.5 to 2.5 beside weights), two norms of 0.7, attention 3.2, and the products.
+//   * A wave's rows are a few registers, requested where nothing is on its way to the compute unit: while the attention is at work, and with wide models also right
+//     behind the products.  (A compute unit's loads return in order and its queue is short: a poll behind weights comes when they have come, and so does a store.)
 //   * Eight waves hold weights, four fetch the vectors.  A wave forms and sums whole rows by itself; the workgroup's rows lie side by side and are handed over
 //     by ONE store.  (Element by element from eight waves a hand-over of 576 elements among 72 workgroups takes 1.9 us, by one store 1.2; among 144 workgroups 1.5, among 256
 //     1.8: hence no more workgroups than the rows need.)
 //   * A polling thread requests all its elements before it looks at one, without a condition around a load (behind which the compiler would wait for it).
-//   * Attention workgroups hold no weights: a head each, its cached rows requested a layer ahead.
+//   * Attention workgroups request a head's cached rows a layer ahead.
 //   * Pointers come from a copy in LDS: a scalar load of a line that nobody has touched takes a microsecond.
 // Values travel between workgroups as tagged 8-byte elements (resident.h; every wait is bounded, as in decode_persistent.hip): a buffer is overwritten only by a
 // phase whose inputs transitively depend on every reader of what it held.
 //
-// The arithmetic is the reference's own order throughout (block products, row sums, norm, softmax over 64-key blocks, the C library's expf): bit-identical to
-// the order-faithful kernel sequence, so the kernel serves both modes.  Per token, SmolLM2-135M Q8_0, us: kernel sequence (order-faithful mode) / kernel for
-// wide models (fast mode) / this: 33 rows of context 781 / 880 / 426, 400 rows 837 / 878 / 489, 740 rows 907 / 876 / 587.
+// ORD: the arithmetic in the reference's own order (block products, row sums, norm, softmax over 64-key blocks, the C library's expf), bit-identical to the
+// order-faithful kernel sequence; narrow models, to which the order costs nothing, run it in both modes.  Otherwise row sums and the norm's sum add up as the lanes
+// have them.  Per token in us, kernel sequence (order-faithful mode) / decode_persistent.hip (fast mode) / this, by rows of context:
+//   SmolLM2-135M Q8_0   33: 781 / 880 / 384    300: 820 / 878 / 421    740: 907 / 876 / 466
+//   1B shape Q8_0       33: 754 / 610 / 466 and 427 (order-faithful, fast)    200: - / 636 / 473 and 439       Q4_0, fast: 33: 532 / 407
 #include <stddef.h>
 #include <string.h>
 
@@ -39,13 +40,18 @@ namespace {
 constexpr uint32_t PA_POLL = 4, PA_COMP = 8, PA_WAVES = PA_POLL + PA_COMP, PA_THREADS = PA_WAVES * 64, PA_POLL_THREADS = PA_POLL * 64;
 constexpr uint32_t PA_B = 64;                 // FLASH_ATTN_BLOCK_SIZE, emit.rs:201; a wave takes one block of keys: at most PA_WAVES blocks
 constexpr uint32_t PA_MAX_ROWS = 8;           // rows of a product that one wave holds (not the lm_head)
-constexpr int PA_PN = 3;                      // elements a polling thread takes: vectors of up to 768
 constexpr uint32_t PA_SUM = 24, PA_SSQ = 12;  // a row's products, and an accumulator's elements of the norm, are read in groups of so many: LDS rows end in zeros up to there
-// blocks of 32 weights that a lane holds: q;k;v, o, gate;up, down, and each of two sets of the lm_head
-constexpr int UQ = 1, UO = 1, UG = 3, UD = 1, UL = 4;
+// The two forms.  UQ .. UL: blocks of 32 weights that a lane holds of q;k;v, o, gate;up (two sets), down and each of two sets of the lm_head; NX, NV: elements
+// a polling thread takes of the residual row and of gate;up's quantised vector; AW: waves that attend to a head, each to 64 keys.
+//   Narrow (up to 768 channels): a layer in 54 registers of a few dozen workgroups; the heads have workgroups of their own, up to 768 rows of context.
+//   Wide (up to 2048 channels): every compute unit holds a block of 32 gate;up rows in two sets of registers, so heads and weights share workgroups: the last `heads` of
+//   them hold no rows of q;k;v and o, and their fetching waves attend, to up to 256 rows.  down takes the place of the second set when that is done.
+struct PaNarrow { static constexpr int UQ = 1, UO = 1, UG1 = 3, UG2 = 0, UD = 1, UL = 4, NX = 3, NV = 3; static constexpr uint32_t AW = PA_WAVES; static constexpr bool WIDE = false; };
+struct PaWide { static constexpr int UQ = 2, UO = 2, UG1 = 4, UG2 = 4, UD = 4, UL = 4, NX = 8, NV = 9; static constexpr uint32_t AW = PA_POLL; static constexpr bool WIDE = true; };
 
-// magic: floor(2^32 / nblk) + 1; R: rows per wave; stride: words between two rows of products; prod: the first wave's area of them (LDS bytes)
-struct PaMat { uint32_t N, nblk, magic, R, stride, prod; };
+// magic: floor(2^32 / nblk) + 1; R: rows per wave; wg0: the first workgroup with rows; stride: words between two rows of products; prod: the first wave's area of
+// them (LDS bytes), dump: a word behind it that nobody reads; fold: log2 of the lanes that add a row up where the order is free
+struct PaMat { uint32_t N, nblk, magic, R, wg0, stride, prod, dump, fold; };
 struct PaWeights { const uint8_t* qs; const uint16_t* ws; };
 struct PaLayer {
     PaWeights w[4];                           // q;k;v, o, gate;up, down
@@ -57,7 +63,7 @@ struct PaLayer {
 struct PaArgs {
     PaMat m[5];                               // q;k;v, o, gate;up (N = 2 I; a workgroup holds 32 + 32 rows), down, lm_head
     uint32_t L, H, I, QKS, KV, heads, kv_heads;
-    uint32_t G;                               // workgroups [0, G) hold the layers' matrices, the next `heads` a head each; all share the lm_head
+    uint32_t G, head0;                        // workgroups [0, G) hold the layers' matrices, [head0, head0 + heads) take a head each; all share the lm_head
     float eps;
     const PaLayer* layers;                    // [L + 1]: the last one's first norm is the final norm; its q;k;v is the first layer's (requested, not used)
     PaWeights lm;
@@ -79,7 +85,7 @@ struct PaArgs {
     unsigned long long* host_out;             // host-mapped {launch number, next token}: written last, or null
     uint32_t host_seq;
     unsigned long long* stamps;               // optional: wall clock at the start of every phase (workgroup 0)
-    uint32_t off_as, off_xs, off_out, off_nw, off_silu, off_prod, off_layers, off_attn, prod_words, lds_words, xstride;      // LDS byte offsets (activation codes at 0)
+    uint32_t off_as, off_xs, off_out, off_silu, off_prod, off_layers, off_attn, prod_words, lds_words, xstride;      // LDS byte offsets (activation codes at 0)
 };
 
 // A uniform base and a lane's 32-bit offset in bytes.
@@ -105,7 +111,8 @@ __host__ __device__ constexpr uint32_t pa_up(uint32_t v, uint32_t m) { return (v
 
 // N elements a thread takes, re-read together until all carry their tags; bounded.  Every load of a round trip is issued before any is looked at, and
 // without a condition: a branch around one of them would put a wait behind it.  (A thread without an element of its own takes one that another has.)
-template <int N, typename Addr, typename Tag>
+// LATER: an element of a later phase will do; nothing is handed out.
+template <int N, bool LATER = false, typename Addr, typename Tag>
 __device__ __forceinline__ void pa_poll(Addr addr, Tag tag, uint32_t* out, const PaCtx& cx) {
     uint64_t w[N];
     uint32_t spins = 0;
@@ -114,7 +121,7 @@ __device__ __forceinline__ void pa_poll(Addr addr, Tag tag, uint32_t* out, const
         for (int i = 0; i < N; i++) w[i] = ldc64(addr(i));
         uint32_t off = 0;
 #pragma unroll
-        for (int i = 0; i < N; i++) off |= (uint32_t)(w[i] >> 32) ^ tag(i);
+        for (int i = 0; i < N; i++) off |= LATER ? ((uint32_t)(w[i] >> 32) - tag(i)) >> 31 : (uint32_t)(w[i] >> 32) ^ tag(i);
         if (!off) break;
         ++spins;
         if (spins > cx.spin_limit ||
@@ -125,6 +132,7 @@ __device__ __forceinline__ void pa_poll(Addr addr, Tag tag, uint32_t* out, const
         }
         __builtin_amdgcn_s_sleep(1);
     }
+    if constexpr (LATER) return;
 #pragma unroll
     for (int i = 0; i < N; i++) out[i] = (uint32_t)w[i];
 }
@@ -144,7 +152,7 @@ template <int U, bool Q4> struct PaSet { int4 v[Q4 ? U : 2 * U]; uint32_t s[U]; 
 template <bool Q4>
 __device__ __forceinline__ uint32_t pa_own(uint32_t j, uint32_t lane) { return Q4 ? 64 * j + lane : 64 * j + 32 * (lane & 1u) + (lane >> 1); }
 
-template <int U, bool Q4>
+template <int J0 = 0, int U, bool Q4>
 __device__ __forceinline__ void pa_load(PaSet<U, Q4>& w, const PaWeights& mat, const PaTask& t, uint32_t lane) {
     asm volatile("" : "+v"(lane));           // the addresses are worked out here: kept from layer to layer they would not fit the registers
     // Blocks past the last one re-read it, and a wave without rows reads the matrix's first block: with no condition around them the loads in flight are
@@ -157,31 +165,31 @@ __device__ __forceinline__ void pa_load(PaSet<U, Q4>& w, const PaWeights& mat, c
 #pragma unroll
     for (int j = 0; j < U; j++) {
         if (Q4) {
-            w.v[j] = pa_at<int4>(mat.qs, at(64 * j + lane) * 16);
+            w.v[j] = pa_at<int4>(mat.qs, at(64 * (J0 + j) + lane) * 16);
         } else {
 #pragma unroll
-            for (int h = 0; h < 2; h++) w.v[2 * j + h] = pa_at<int4>(mat.qs, at(64 * j + 32 * h + (lane >> 1)) * 32 + (lane & 1u) * 16);
+            for (int h = 0; h < 2; h++) w.v[2 * j + h] = pa_at<int4>(mat.qs, at(64 * (J0 + j) + 32 * h + (lane >> 1)) * 32 + (lane & 1u) * 16);
         }
-        w.s[j] = pa_at<uint16_t>(mat.ws, at(pa_own<Q4>(j, lane)) * 2);
+        w.s[j] = pa_at<uint16_t>(mat.ws, at(pa_own<Q4>(J0 + j, lane)) * 2);
     }
 }
 
 // Where a lane finds its blocks' activations and leaves their products (LDS bytes), worked out ahead of the wait for the vector.
 template <int U, bool Q4> struct PaIdx { uint32_t a[Q4 ? U : 2 * U], s[U], p[U]; };
-template <int U, bool Q4>
+template <int U, bool Q4, int J0 = 0>
 __device__ __forceinline__ PaIdx<U, Q4> pa_index(const PaTask& t, const PaMat& m, uint32_t off_as, uint32_t prod, uint32_t lane) {
     PaIdx<U, Q4> x;
 #pragma unroll
     for (int j = 0; j < U; j++) {
-        const uint32_t u = pa_own<Q4>(j, lane), r = __umulhi(u, m.magic), b = u - r * m.nblk;      // b is a block of the row whatever u is
+        const uint32_t u = pa_own<Q4>(J0 + j, lane), r = __umulhi(u, m.magic), b = u - r * m.nblk;      // b is a block of the row whatever u is
         x.s[j] = off_as + b * 4;
-        x.p[j] = u < t.n ? prod + (r * m.stride + b) * 4 : prod + (m.R * m.stride) * 4;             // past the last block: a word that nobody reads
+        x.p[j] = u < t.n ? prod + (r * m.stride + b) * 4 : prod + m.dump;
         if (Q4) {
             x.a[j] = b * 32;
         } else {
 #pragma unroll
             for (int h = 0; h < 2; h++) {
-                const uint32_t uh = 64 * j + 32 * h + (lane >> 1);
+                const uint32_t uh = 64 * (J0 + j) + 32 * h + (lane >> 1);
                 x.a[2 * j + h] = (uh - __umulhi(uh, m.magic) * m.nblk) * 32 + (lane & 1u) * 16;
             }
         }
@@ -193,11 +201,11 @@ __device__ __forceinline__ PaIdx<U, Q4> pa_index(const PaTask& t, const PaMat& m
 }
 
 // The blocks' products (a_s * w_s) * f32(isum), exact int32 block sums, parked in the wave's LDS.
-template <int U, bool Q4>
+template <int J0 = 0, int U, bool Q4>
 __device__ __forceinline__ void pa_products(const PaSet<U, Q4>& w, const PaIdx<U, Q4>& x, uint32_t n, uint8_t* smem) {
 #pragma unroll
     for (int j = 0; j < U; j++) {
-        if (64u * j >= n) break;
+        if (64u * (J0 + j) >= n) break;
         int isum;
         if (Q4) {
             const int4 a0 = *reinterpret_cast<const int4*>(smem + x.a[j]);
@@ -220,11 +228,27 @@ __device__ __forceinline__ void pa_products(const PaSet<U, Q4>& w, const PaIdx<U
     }
 }
 
-// Ordered sums of the wave's rows: lane r < rows returns row r's.  Products and sums are one wave's LDS operations, which execute in order.
-// The zeros behind a row's products change nothing: a sum that starts at +0 is never -0.
-__device__ __forceinline__ float pa_row_sum(const PaMat& m, uint32_t rows, const uint8_t* area, uint32_t lane) {
+// Sums of the wave's rows.  Products and sums are one wave's LDS operations, which execute in order.
+//   ORD      in block order: lane r < rows holds row r's.  The zeros behind a row's products change nothing: a sum that starts at +0 is never -0.
+//   not ORD  2^fold lanes add a row up (as many as there are for m.R rows), the first of them holds it.
+struct PaSum { float v; uint32_t row; bool on; };
+template <bool ORD>
+__device__ __forceinline__ PaSum pa_row_sum(const PaMat& m, uint32_t rows, const uint8_t* area, uint32_t lane) {
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
+    if constexpr (!ORD) {
+        const uint32_t row = lane >> m.fold, part = lane & ((1u << m.fold) - 1);
+        const float* p = reinterpret_cast<const float*>(area) + row * m.stride;
+        float r = 0.f;
+        for (uint32_t b = part; b < m.nblk; b += 1u << m.fold) r += p[b];
+        if (m.fold > 0) r = lane_xor_add<1>(r);
+        if (m.fold > 1) r = lane_xor_add<2>(r);
+        if (m.fold > 2) r = lane_xor_add<4>(r);
+        if (m.fold > 3) r = lane_xor_add<8>(r);
+        if (m.fold > 4) r = lane_xor_add<16>(r);
+        if (m.fold > 5) r = lane_xor_add<32>(r);
+        return PaSum{r, row, part == 0 && row < rows};
+    }
     float r = 0.f;
     if (lane < rows) {
         const float4* p = reinterpret_cast<const float4*>(area) + lane * (m.stride / 4);
@@ -244,7 +268,7 @@ __device__ __forceinline__ float pa_row_sum(const PaMat& m, uint32_t rows, const
 #pragma unroll
         for (int i = 0; i < N4; i++) { r = r + v[i].x; r = r + v[i].y; r = r + v[i].z; r = r + v[i].w; }
     }
-    return r;
+    return PaSum{r, lane, lane < rows};
 }
 
 // int8 codes of 32 values, one per lane of a half wave, and their fp16 scale (emit.rs:1410-1440), as the nine elements of a block: side by side and by one
@@ -261,20 +285,35 @@ __device__ __forceinline__ void pa_store_block(float o, uint64_t* block, uint32_
 
 // Vectors, fetched by the polling waves.  The residual row lies in LDS accumulator by accumulator of the norm: element e in row e % 16.
 __device__ __forceinline__ uint32_t pa_xs(uint32_t e, uint32_t xstride) { return (e & 15u) * xstride + (e >> 4); }
-__device__ __forceinline__ void pa_fetch_x(const uint64_t* tx, uint32_t tag, const float* emb, uint32_t H, float* xs, uint32_t xstride, const PaCtx& cx) {
+// Where the order of the norm's sum is free, every wave leaves the sum of its elements' squares in `part`.
+template <int N, bool ORD>
+__device__ __forceinline__ void pa_fetch_x(const uint64_t* tx, uint32_t tag, const float* emb, uint32_t H, float* xs, uint32_t xstride, float* part, const PaCtx& cx) {
+    uint32_t v[N];
     if (!tag) {                               // the layer ahead of the first: the embedding row
-        for (uint32_t i = cx.tid; i < H; i += PA_POLL_THREADS) xs[pa_xs(i, xstride)] = ldg(emb + i);
-        return;
-    }
-    uint32_t v[PA_PN];
-    pa_poll<PA_PN>([&](int i) { return tx + min(cx.tid + i * PA_POLL_THREADS, H - 1); }, [&](int) { return tag; }, v, cx);
 #pragma unroll
-    for (int i = 0; i < PA_PN; i++)
-        if (cx.tid + i * PA_POLL_THREADS < H) xs[pa_xs(cx.tid + i * PA_POLL_THREADS, xstride)] = __uint_as_float(v[i]);
+        for (int i = 0; i < N; i++) v[i] = __float_as_uint(ldg(emb + min(cx.tid + i * PA_POLL_THREADS, H - 1)));
+    } else {
+        pa_poll<N>([&](int i) { return tx + min(cx.tid + i * PA_POLL_THREADS, H - 1); }, [&](int) { return tag; }, v, cx);
+    }
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        const uint32_t e = cx.tid + i * PA_POLL_THREADS;
+        const float x = __uint_as_float(v[i]);
+        if (e < H) {
+            xs[pa_xs(e, xstride)] = x;
+            ss = fmaf(x, x, ss);
+        }
+    }
+    if constexpr (!ORD) {
+        ss = wave_sum(ss);
+        if (cx.lane == 0) part[cx.wave] = ss;
+    }
 }
 
 // A quantised vector and, with it, the residual of the rows that this workgroup holds: element res_row of x in lane r of the first wave
 // (res_tag 0: the embedding row; threads without a row: anything).
+template <int NV>
 __device__ __forceinline__ float pa_fetch_aq(const uint64_t* t, uint32_t tag, uint32_t K, uint32_t* aq, float* as, bool has_res, uint32_t res_row, const uint64_t* tx,
                                              uint32_t res_tag, const float* emb, const PaCtx& cx) {
     const uint32_t ne = K / 32 * 9;
@@ -300,15 +339,15 @@ __device__ __forceinline__ float pa_fetch_aq(const uint64_t* t, uint32_t tag, ui
     };
     if (ne <= PA_POLL_THREADS) fetch(std::integral_constant<int, 1>{});
     else if (ne <= 2 * PA_POLL_THREADS) fetch(std::integral_constant<int, 2>{});
-    else fetch(std::integral_constant<int, PA_PN>{});
+    else if (NV == 3 || ne <= 3 * PA_POLL_THREADS) fetch(std::integral_constant<int, 3>{});
+    else fetch(std::integral_constant<int, NV>{});
     return re;
 }
 
-// rms_norm (emit.rs:327-334, the 16-accumulator order of emit.rs:272-295) + activation quantiser, an element a thread.  Every wave forms the
-// sum of squares for itself, so there is no barrier between the sum and the codes; zeros behind an accumulator's elements change nothing.
-// nw: the norm weight of element tid.
-__device__ __forceinline__ void pa_norm_quant(const float* xs, uint32_t xstride, float nw, float eps, uint32_t H, uint8_t* smem, uint32_t off_as, const PaCtx& cx) {
-    const float x = cx.tid < H ? xs[pa_xs(cx.tid, xstride)] : 0.f;
+// rms_norm (emit.rs:327-334) + activation quantiser.  In the reference's order (16 accumulators, emit.rs:272-295) each fetching wave walks the row and the first
+// leaves 1 / rms behind; zeros behind an accumulator's elements change nothing.  The computing waves, which have nothing else to do yet, quantise four elements a
+// thread, whose norm weights they hold.  (All twelve waves forming the sum for themselves and an element a thread: 1.1 us at 576 channels where this takes 0.7.)
+__device__ __forceinline__ void pa_norm_sum(const float* xs, uint32_t xstride, float eps, uint32_t H, float* part, const PaCtx& cx) {
     const float4* p = reinterpret_cast<const float4*>(xs + (cx.lane & 15u) * xstride);
     float s = 0.f;
     constexpr int N4 = PA_SSQ / 4;
@@ -331,15 +370,18 @@ __device__ __forceinline__ void pa_norm_quant(const float* xs, uint32_t xstride,
     s = lane_xor_add<8>(s);
     s = lane_xor_add<1>(s);
     s = lane_xor_add<2>(s);
-    const float inv_rms = 1.0f / sqrtf(s / (float)H + eps);
-    const float y = x * inv_rms * nw;
-    const float amax = half_wave_max(fabsf(y));
-    float inv;
-    const float sc = act_scale(amax, inv);
-    if (cx.tid < H) {
-        smem[cx.tid] = (uint8_t)quant_code(y * inv);
-        if ((cx.tid & 31u) == 0) *reinterpret_cast<float*>(smem + off_as + cx.tid / 8) = f16_bits_to_f32(f32_to_f16_bits(sc));
-    }
+    if (cx.tid == 0) part[0] = 1.0f / sqrtf(s / (float)H + eps);
+}
+template <bool ORD>
+__device__ __forceinline__ void pa_norm_quant(const float* xs, uint32_t xstride, float4 nw, float eps, uint32_t H, uint8_t* smem, uint32_t off_as, const float* part, uint32_t t) {
+    if (t * 4 >= H) return;
+    const float* p = xs + (t * 4 & 15u) * xstride + t / 4;        // four neighbours: rows t * 4 % 16 .. + 3
+    const float x0 = p[0], x1 = p[xstride], x2 = p[2 * xstride], x3 = p[3 * xstride];
+    const float inv_rms = ORD ? part[0] : 1.0f / sqrtf(((part[0] + part[1]) + (part[2] + part[3])) / (float)H + eps);
+    const float4 v = make_float4(x0 * inv_rms * nw.x, x1 * inv_rms * nw.y, x2 * inv_rms * nw.z, x3 * inv_rms * nw.w);
+    uint16_t sb;
+    reinterpret_cast<uint32_t*>(smem)[t] = quantize_block_part(v, sb);
+    if ((t & 7u) == 0) *reinterpret_cast<float*>(smem + off_as + t / 2) = f16_bits_to_f32(sb);
 }
 
 struct PaExpTab {
@@ -348,23 +390,22 @@ struct PaExpTab {
 };
 
 // LDS of an attention workgroup.  pn: products of q and this position's K row, vn: its V row, es: exp(m of the block before - m).
-template <int HD>
+template <int HD, uint32_t AW>
 struct PaAttn {
     float q[HD], pn[HD], vn[HD];
-    float e[PA_WAVES][PA_B];
-    float sums[PA_WAVES][HD];
-    float bmax[PA_WAVES], lblk[PA_WAVES], es[PA_WAVES], snew;
+    float e[AW][PA_B];
+    float sums[AW][HD];
+    float bmax[AW], lblk[AW], es[AW], snew;
 };
 
 // A wave's 64-key block of the cache: lane = key of the K rows, lane = head dim of the V rows.  Heads of 64: all of it, in 32-bit; wider heads:
 // K rows as they are and KC of the V rows at a time.
-typedef _Float16 PaHalf2 __attribute__((ext_vector_type(2)));
 template <int HD>
 struct PaKv {
     static constexpr int DPL = (HD + 63) / 64, KC = HD == 64 ? 64 : 16;
     float k[HD == 64 ? 64 : 1];
     uint4 kr[HD == 64 ? 1 : HD / 8];
-    PaHalf2 v[KC / 2][DPL];
+    uint32_t v[KC / 2][DPL];                  // two rows to a register
     __device__ __forceinline__ void set_keys(const uint4 (&raw)[HD / 8]) {
 #pragma unroll
         for (int c = 0; c < HD / 8; c++) {
@@ -377,6 +418,7 @@ struct PaKv {
             }
         }
     }
+    __device__ __forceinline__ float value(int i, int t) const { return f16_bits_to_f32((uint16_t)(i & 1 ? v[i / 2][t] >> 16 : v[i / 2][t] & 0xFFFFu)); }
     __device__ __forceinline__ float key(int i) const {
         if constexpr (HD == 64) {
             return k[i];
@@ -387,47 +429,69 @@ struct PaKv {
         }
     }
 };
+// KC rows of V from row bs + k0 on, as they arrive: 16 bits to a register.  (Loads into halves of registers wait for each other in pairs.)
+template <int HD> struct PaRaw { uint32_t v[PaKv<HD>::KC][PaKv<HD>::DPL]; };
 template <int HD>
-__device__ __forceinline__ void pa_load_values(PaKv<HD>& kv, const uint16_t* vb, uint32_t bs, uint32_t k0, uint32_t pos, uint32_t kv_stride, uint32_t lane) {
+__device__ __forceinline__ void pa_load_values(PaRaw<HD>& raw, const uint16_t* vb, uint32_t row0, uint32_t pos, uint32_t kv_stride, uint32_t lane) {
 #pragma unroll
     for (int i = 0; i < PaKv<HD>::KC; i++)
 #pragma unroll
         for (int t = 0; t < PaKv<HD>::DPL; t++) {
-            const uint32_t d = min(lane + 64 * t, (uint32_t)HD - 1), row = bs + k0 + i;      // rows past the last cached one: row 0
-            kv.v[i / 2][t][i % 2] = pa_at<_Float16>(vb + (row < pos ? row : 0u) * kv_stride, d * 2);
+            const uint32_t d = min(lane + 64 * t, (uint32_t)HD - 1), row = row0 + i;      // rows past the last cached one: row 0
+            raw.v[i][t] = pa_at<uint16_t>(vb + (row < pos ? row : 0u) * kv_stride, d * 2);
         }
+    __builtin_amdgcn_sched_barrier(0);                // all requested before the first is waited for
+}
+template <int HD>
+__device__ __forceinline__ void pa_pack_values(PaKv<HD>& kv, const PaRaw<HD>& raw) {
+#pragma unroll
+    for (int i = 0; i < PaKv<HD>::KC; i += 2)
+#pragma unroll
+        for (int t = 0; t < PaKv<HD>::DPL; t++) kv.v[i / 2][t] = raw.v[i][t] | (raw.v[i + 1][t] << 16);
+    __builtin_amdgcn_sched_barrier(0);
 }
 
-// attention_flash (emit.rs:656-715) of head h in every layer, a wave per block of 64 keys: attn_exact_decode_one_kernel's steps.  The cached rows of a
-// layer are requested as soon as the layer before it is done.
-template <int HD>
-__device__ __forceinline__ void pa_attention(const PaArgs& a, const PaLayer* layers, PaAttn<HD>* sh, const uint64_t* exp_tab, uint32_t pos, uint32_t h, PaCtx& cx) {
-    constexpr int DPL = PaKv<HD>::DPL, KC = PaKv<HD>::KC;
-    const uint32_t kvh = h / (a.heads / a.kv_heads), kv_stride = a.KV;
-    const uint32_t b = cx.wave, seq = pos + 1, nb = (seq + PA_B - 1) / PA_B, bs = b * PA_B;
-    const uint32_t bl = bs < seq ? min(PA_B, seq - bs) : 0u;
-    const bool has_new = bs <= pos && pos < bs + PA_B;            // this position is the last key of the last block
-    uint32_t nk = has_new ? bl - 1 : bl;                          // of which cached
-    // the score of this position and the blocks' exp_scale are the work of waves without a block, as long as there are such
-    const bool wave_new = b == nb % PA_WAVES, wave_es = nb > 1 && b == (nb + 1) % PA_WAVES;
-    const float scale = 1.0f / sqrtf((float)HD);
-    const PaExpTab tab{exp_tab};
-#pragma nounroll
-    for (uint32_t l = 0; l < a.L; l++) {
-        asm volatile("" : "+v"(cx.tid), "+v"(cx.lane), "+s"(nk));
-        const uint32_t lane = cx.lane, tag_in = a.tag_base + 6 * l + 1;
-        PaKv<HD> kv;
-        const uint16_t* vb = pa_lds_ptr(layers[l].vc) + kvh * HD;
-        if (bl) {
-            const uint16_t* kb = pa_lds_ptr(layers[l].kc) + kvh * HD;
-            const uint32_t row = bs + lane, at = (row < pos ? row : 0u) * kv_stride * 2;
-            uint4 kr[HD / 8];
+// attention_flash (emit.rs:656-715) of one head, a wave per block of 64 keys: attn_exact_decode_one_kernel's steps.  AW waves attend, the workgroup's others only take
+// part in the barriers.
+template <int HD, uint32_t AW>
+struct PaHead {
+    uint32_t h, kvh, b, nb, bs, bl, nk;           // the wave's block b: bl keys, nk of them cached
+    bool has_new;                                 // this position is the last key of the last block
+    __device__ __forceinline__ PaHead(const PaArgs& a, uint32_t head, uint32_t pos, uint32_t wave) {
+        h = head; kvh = head / (a.heads / a.kv_heads);
+        const uint32_t seq = pos + 1;
+        b = wave; nb = (seq + PA_B - 1) / PA_B; bs = b * PA_B;
+        bl = b < AW && bs < seq ? min(PA_B, seq - bs) : 0u;
+        has_new = b < AW && bs <= pos && pos < bs + PA_B;
+        nk = has_new ? bl - 1 : bl;
+    }
+    __device__ __forceinline__ void load(PaKv<HD>& kv, const PaArgs& a, const PaLayer& L, uint32_t pos, uint32_t lane) const {
+        if (!bl) return;
+        const uint16_t* kb = pa_lds_ptr(L.kc) + kvh * HD;
+        const uint32_t row = bs + lane, at = (row < pos ? row : 0u) * a.KV * 2;      // lanes without a cached key: row 0
+        uint4 kr[HD / 8];
 #pragma unroll
-            for (int c = 0; c < HD / 8; c++) kr[c] = pa_at<uint4>(kb, at + c * 16);
-            pa_load_values<HD>(kv, vb, bs, 0, pos, kv_stride, lane);
-            __builtin_amdgcn_sched_barrier(0);
-            kv.set_keys(kr);
-        }
+        for (int c = 0; c < HD / 8; c++) kr[c] = pa_at<uint4>(kb, at + c * 16);
+        PaRaw<HD> raw;
+        pa_load_values<HD>(raw, pa_lds_ptr(L.vc) + kvh * HD, bs, pos, a.KV, lane);
+        pa_pack_values<HD>(kv, raw);
+        kv.set_keys(kr);
+    }
+    __device__ __forceinline__ void step(PaKv<HD>& kv, const PaArgs& a, const PaLayer& L, PaAttn<HD, AW>* sh, const uint64_t* exp_tab, uint32_t pos, uint32_t tag_in, PaCtx& cx) const;
+};
+
+template <int HD, uint32_t AW>
+__device__ __forceinline__ void PaHead<HD, AW>::step(PaKv<HD>& kv, const PaArgs& a, const PaLayer& L, PaAttn<HD, AW>* sh, const uint64_t* exp_tab, uint32_t pos, uint32_t tag_in,
+                                                     PaCtx& cx) const {
+        constexpr int DPL = PaKv<HD>::DPL, KC = PaKv<HD>::KC;
+        const uint32_t kv_stride = a.KV, lane = cx.lane;
+        const float scale = 1.0f / sqrtf((float)HD);
+        const PaExpTab tab{exp_tab};
+        // the score of this position and the blocks' exp_scale are the work of waves without a block, as long as there are such
+        const bool wave_new = b == nb % AW, wave_es = nb > 1 && b == (nb + 1) % AW;
+        const uint16_t* vb = pa_lds_ptr(L.vc) + kvh * HD;
+        uint32_t nk = pa_sgpr(this->nk);
+        asm volatile("" : "+s"(nk));              // conditions on it are formed where they are used: kept from layer to layer they would not fit the registers
         if (cx.tid < pa_up(HD, 64)) {
             uint32_t g[3];
             const uint32_t e = min(cx.tid, (uint32_t)HD - 1);
@@ -466,7 +530,7 @@ __device__ __forceinline__ void pa_attention(const PaArgs& a, const PaLayer* lay
             // m after block i: the largest block maximum so far; es[0] = exp(-inf - m) is 0
             float m = -INFINITY, before = -INFINITY;
 #pragma unroll
-            for (uint32_t i = 0; i < PA_WAVES; i++) {
+            for (uint32_t i = 0; i < AW; i++) {
                 const float v = i < nb ? (i == nb - 1 ? fmaxf(sh->bmax[i], sh->snew) : sh->bmax[i]) : -INFINITY;
                 if (i < lane) before = fmaxf(before, v);
                 if (i <= lane) m = fmaxf(m, v);
@@ -490,7 +554,7 @@ __device__ __forceinline__ void pa_attention(const PaArgs& a, const PaLayer* lay
 #pragma nounroll
             for (uint32_t k0 = 0; k0 < PA_B; k0 += KC) {
                 if (k0 && k0 >= nk) break;
-                if (k0) pa_load_values<HD>(kv, vb, bs, k0, pos, kv_stride, lane);
+                if (k0) { PaRaw<HD> raw; pa_load_values<HD>(raw, vb, bs + k0, pos, kv_stride, lane); pa_pack_values<HD>(kv, raw); }
                 // keys past the last one are left out, not given a weight of 0: 0 * v is not 0 for an infinite v
 #pragma unroll
                 for (int i16 = 0; i16 < KC; i16 += 16) {
@@ -502,7 +566,7 @@ __device__ __forceinline__ void pa_attention(const PaArgs& a, const PaLayer* lay
                         auto add = [&](int i) {
                             l_block = l_block + w[i];
 #pragma unroll
-                            for (int t = 0; t < DPL; t++) sum[t] = sum[t] + w[i] * (float)kv.v[(i16 + i) / 2][t][(i16 + i) % 2];
+                            for (int t = 0; t < DPL; t++) sum[t] = sum[t] + w[i] * kv.value(i16 + i, t);
                         };
                         if (k0 + i16 + 16 <= nk) {
 #pragma unroll
@@ -542,7 +606,6 @@ __device__ __forceinline__ void pa_attention(const PaArgs& a, const PaLayer* lay
             const uint32_t e = h * HD + cx.tid;
             pa_store_block(cx.tid < HD ? o : 0.f, a.taq + e / 32 * 9, tag_in + 1, cx.lane, cx.tid < HD);
         }
-    }
 }
 
 // One workgroup's part of an argmax: the LAST index among equal maxima (project.rs:501-503).
@@ -559,20 +622,20 @@ __device__ __forceinline__ ArgPair pa_arg_wg(ArgPair v, ArgPair* sh, const PaCtx
 }
 
 // The tag of a phase instance: tag_base + 6 layer + 1 q;k;v, 2 attention, 4 o, 5 gate;up, 6 down; the argmax's is behind the last layer's.
-template <int HD, bool Q4, bool LMQ4>
+template <typename F, bool ORD, int HD, bool Q4, bool LMQ4>
 __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
     extern __shared__ __align__(16) uint8_t smem[];
     __shared__ uint32_t sh_abort;
     __shared__ ArgPair sh_arg[PA_WAVES];
+    __shared__ float norm_part[PA_POLL];
     __shared__ uint64_t exp_tab[32];          // expf_ref's table
     uint32_t* aq = reinterpret_cast<uint32_t*>(smem);
     float* as = reinterpret_cast<float*>(smem + a.off_as);
     float* xs = reinterpret_cast<float*>(smem + a.off_xs);
     float* out = reinterpret_cast<float*>(smem + a.off_out);                     // the workgroup's row sums
-    float* nws = reinterpret_cast<float*>(smem + a.off_nw);
     float* silu = reinterpret_cast<float*>(smem + a.off_silu);
     const PaLayer* layers = reinterpret_cast<const PaLayer*>(smem + a.off_layers);
-    PaAttn<HD>* attn = reinterpret_cast<PaAttn<HD>*>(smem + a.off_attn);
+    auto* attn = reinterpret_cast<PaAttn<HD, F::AW>*>(smem + a.off_attn);
 
     PaCtx cx;
     cx.tid = threadIdx.x;
@@ -584,36 +647,61 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
     cx.sh_abort = &sh_abort;
     cx.abort_flag = a.state + 3;
     const bool comp = cx.wave >= PA_POLL;
-    const uint32_t c = comp ? cx.wave - PA_POLL : 0u, wv = cx.wg * PA_COMP + c;       // a workgroup's rows lie side by side: one store hands them over
+    const uint32_t c = comp ? cx.wave - PA_POLL : 0u;
     if (cx.tid == 0) sh_abort = 0;
     if (cx.tid < 32) exp_tab[cx.tid] = expf_detail::tab((int)cx.tid);
     for (uint32_t i = cx.tid; i < a.lds_words; i += PA_THREADS) reinterpret_cast<uint32_t*>(smem)[i] = 0;      // the zeros behind products and accumulators
     for (uint32_t i = cx.tid; i < (a.L + 1) * (uint32_t)(sizeof(PaLayer) / 4); i += PA_THREADS)
         reinterpret_cast<uint32_t*>(smem + a.off_layers)[i] = ldg(reinterpret_cast<const uint32_t*>(a.layers) + i);
-    const uint32_t pos = a.state[0];
+    const uint32_t pos = pa_sgpr(a.state[0]);
     const float* emb = a.embed + (size_t)a.token * a.H;
     __syncthreads();
 
     const uint32_t ntid = cx.tid - PA_POLL_THREADS;                               // of a computing thread
     const bool stamp = a.stamps && cx.wg == 0 && cx.tid == 0;
-    PaSet<UL, LMQ4> wl[2];
-    float n1 = 0.f, n1p = 0.f;                // norm weights of element tid, and of a polling thread's element, which gets them through LDS
+    PaSet<F::UL, LMQ4> wl[2];
+    float4 n1;                                // norm weights of elements 4 ntid ..
     const PaMat ml = a.m[4];
     const uint32_t T = gridDim.x, W = PA_COMP * T, lwv = c * T + cx.wg;
+    auto load_norm = [&](const float* nw) { return pa_at<float4>(nw, min(ntid * 4, a.H - 4) * 4); };      // threads past the last one: it again
+    // the barriers and what lies between them from a fetched row to its codes, for fetching and computing waves; false: the step is given up
+    auto norm_fetching = [&]() {
+        __syncthreads();
+        if (sh_abort) return false;
+        if (ORD) { pa_norm_sum(xs, a.xstride, a.eps, a.H, norm_part, cx); __syncthreads(); }
+        __syncthreads();
+        return true;
+    };
+    // Wide: where weights would be requested while others wait for a hand-over, the workgroup waits for an element of it too (requested at once they fill the memory
+    // system in front of it: 545 us a token at the 1B shape, 451 so)
+    // (a workgroup on which nothing depends may come late and find a later phase's element there)
+    auto glance = [&](const uint64_t* p, uint32_t tag) {
+        if (cx.wave == 0) pa_poll<1, true>([&](int) { return p; }, [&](int) { return tag; }, nullptr, cx);
+        __syncthreads();
+        return sh_abort == 0;
+    };
+    auto norm_computing = [&](float4 n) {
+        __syncthreads();
+        if (sh_abort) return false;
+        if (ORD) __syncthreads();
+        pa_norm_quant<ORD>(xs, a.xstride, n, a.eps, a.H, smem, a.off_as, norm_part, ntid);
+        __syncthreads();
+        return true;
+    };
+    const uint32_t head = cx.wg - a.head0;
+    const bool on_a = head < a.heads;         // unsigned
 
     if (cx.wg < cx.G) {
         const PaMat mq = a.m[0], mo = a.m[1], mg = a.m[2], md = a.m[3];
         const uint32_t per_wave = 32 / PA_COMP;                                  // gate;up: 4 gate and 4 up rows a wave
-        const uint32_t row_q = cx.wg * PA_COMP * mq.R, row_o = cx.wg * PA_COMP * mo.R, row_d = cx.wg * PA_COMP * md.R;
+        // a workgroup's rows lie side by side: one store hands them over
+        auto rank = [&](const PaMat& m) { return cx.wg >= m.wg0 && (!F::WIDE || !on_a || &m == &md) ? cx.wg - m.wg0 : 0xFFFFFFu; };
+        const uint32_t kq = rank(mq), ko = rank(mo), kd = rank(md);
+        const uint32_t row_q = kq * PA_COMP * mq.R, row_o = ko * PA_COMP * mo.R, row_d = kd * PA_COMP * md.R;
         const bool on_q = row_q < mq.N, on_o = row_o < mo.N, on_g = cx.wg < a.I / 32, on_d = row_d < md.N;
-        const PaTask tq = pa_task(mq, wv), to = pa_task(mo, wv), td = pa_task(md, wv);
+        const PaTask tq = pa_task(mq, kq * PA_COMP + c), to = pa_task(mo, ko * PA_COMP + c), td = pa_task(md, kd * PA_COMP + c);
         const PaTask tg{on_g ? (cx.wg * 32 + c * per_wave) * mg.nblk : 0u, on_g ? 2 * per_wave * mg.nblk : 0u, per_wave * mg.nblk, (a.I - per_wave) * mg.nblk};
         const uint32_t pq = mq.prod + c * a.prod_words * 4, po = mo.prod + c * a.prod_words * 4, pg = mg.prod + c * a.prod_words * 4, pd = md.prod + c * a.prod_words * 4;
-        PaSet<UQ, Q4> wq;
-        PaSet<UO, Q4> wo;
-        PaSet<UG, Q4> wg;
-        PaSet<UD, Q4> wd;
-        float n2 = 0.f, n2p = 0.f;
         // the first wave finishes rows: lane r the workgroup's r-th
         float rc = 1.f, rs = 0.f;                                                // rotation of its row of q | k
         const uint32_t qrow = row_q + cx.lane;
@@ -623,34 +711,22 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
             rc = ldg(a.cos_t + (size_t)pos * (HD / 2) + d / 2);
             rs = ldg(a.sin_t + (size_t)pos * (HD / 2) + d / 2);
         }
-        auto load_norm = [&](const float* nw, float& own, float& other) {      // elements past the last one: it again
-            own = pa_at<float>(nw, min(cx.tid, a.H - 1) * 4);
-            other = pa_at<float>(nw, min(ntid, a.H - 1) * 4);
-        };
-        if (comp) {
-            const PaLayer& L = layers[0];
-            load_norm(pa_lds_ptr(L.norm[0]), n1, n1p);
-            pa_load(wq, pa_lds_ptr(L.w[0]), tq, cx.lane);
-        }
-
+        // Fetching and computing waves go through the layers in loops of their own (with the same barriers): neither keeps the other's registers.
+        if (!comp) {
+            const PaHead<HD, F::AW> ph(a, F::WIDE && on_a ? head : 0u, pos, cx.wave);
 #pragma nounroll
-        for (uint32_t l = 0; l < a.L; l++) {
-            // The thread's number is read afresh in every layer: addresses that follow from it would be kept from layer to layer and not fit the registers.
-            asm volatile("" : "+v"(cx.tid), "+v"(cx.lane));
-            const PaLayer& L = layers[l];
-            const PaLayer& N = layers[l + 1];
-            const uint32_t base = a.tag_base + 6 * l, x_in = l ? base : 0u;
-            // ---- norm | q;k;v | rotation, cache row
-            if (stamp) a.stamps[6 * l] = wall_clock64();
-            if (on_q) {
-                if (!comp) {
+            for (uint32_t l = 0; l < a.L; l++) {
+                // The thread's number is read afresh in every layer: addresses that follow from it would be kept from layer to layer and not fit the registers.
+                asm volatile("" : "+v"(cx.tid), "+v"(cx.lane));
+                const PaLayer& L = layers[l];
+                const uint32_t base = a.tag_base + 6 * l, x_in = l ? base : 0u;
+                // ---- norm | q;k;v | rotation, cache row
+                if (stamp) a.stamps[6 * l] = wall_clock64();
+                if (on_q) {
                     uint16_t* kc = pa_lds_ptr(L.kc);
                     uint16_t* vc = pa_lds_ptr(L.vc);
-                    pa_fetch_x(a.tx, x_in, emb, a.H, xs, a.xstride, cx);
-                    __syncthreads();
-                    if (sh_abort) return;
-                    pa_norm_quant(xs, a.xstride, nws[cx.tid], a.eps, a.H, smem, a.off_as, cx);
-                    __syncthreads();
+                    pa_fetch_x<F::NX, ORD>(a.tx, x_in, emb, a.H, xs, a.xstride, norm_part, cx);
+                    if (!norm_fetching()) return;
                     __syncthreads();
                     if (cx.wave == 0) {
                         const float v = out[cx.lane];
@@ -664,105 +740,143 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
                             if (!is_q) stg((is_k ? kc + at : vc + (at - a.KV)) + (size_t)pos * a.KV, hb);
                         }
                     }
-                } else {
-                    const auto x = pa_index<UQ, Q4>(tq, mq, a.off_as, pq, cx.lane);
-                    if (ntid < PA_POLL_THREADS) nws[ntid] = n1p;
-                    __syncthreads();
-                    if (sh_abort) return;
-                    pa_norm_quant(xs, a.xstride, n1, a.eps, a.H, smem, a.off_as, cx);
-                    __syncthreads();
-                    pa_products(wq, x, tq.n, smem);
-                    const float v = pa_row_sum(mq, mq.R, smem + pq, cx.lane);
-                    if (cx.lane < mq.R) out[c * mq.R + cx.lane] = v;
-                    __syncthreads();
                 }
-            }
-            // While the attention is at work nothing else is on its way to this workgroup: now the matrices that follow are requested (a load that
-            // misses ahead of a poll holds the poll up, whichever wave it belongs to).
-            if (comp) {
-                pa_load(wo, pa_lds_ptr(L.w[1]), to, cx.lane);
-                load_norm(pa_lds_ptr(L.norm[1]), n2, n2p);
-                pa_load(wg, pa_lds_ptr(L.w[2]), tg, cx.lane);
-                pa_load(wd, pa_lds_ptr(L.w[3]), td, cx.lane);
-                load_norm(pa_lds_ptr(N.norm[0]), n1, n1p);
-                pa_load(wq, pa_lds_ptr(N.w[0]), tq, cx.lane);
-            }
-            // ---- (attention) o + residual
-            if (stamp) { const unsigned long long t = wall_clock64(); a.stamps[6 * l + 1] = t; a.stamps[6 * l + 2] = t; a.stamps[6 * l + 3] = t; }
-            if (on_o) {
-                const bool mine = cx.wave == 0 && cx.lane < PA_COMP * mo.R && row_o + cx.lane < mo.N;
-                if (!comp) {
-                    const float r = pa_fetch_aq(a.taq, base + 2, a.QKS, aq, as, mine, row_o + cx.lane, a.tx, x_in, emb, cx);
+                // ---- attention
+                if (stamp) a.stamps[6 * l + 1] = wall_clock64();
+                if constexpr (F::WIDE) {
+                    if (on_a) {
+                        PaKv<HD> kv;
+                        ph.load(kv, a, L, pos, cx.lane);
+                        ph.step(kv, a, L, attn, exp_tab, pos, base + 1, cx);
+                    } else {
+                        if (!glance(a.tkv + 2 * a.KV - 1, base + 1)) return;
+                    }
+                    if (sh_abort) return;
+                    if (!on_o && !on_a && !glance(a.taq + a.QKS / 32 * 9 - 1, base + 2)) return;
+                }
+                // ---- o + residual
+                if (stamp) { const unsigned long long t = wall_clock64(); a.stamps[6 * l + 2] = t; a.stamps[6 * l + 3] = t; }
+                if (on_o) {
+                    const bool mine = cx.wave == 0 && cx.lane < PA_COMP * mo.R && row_o + cx.lane < mo.N;
+                    const float r = pa_fetch_aq<F::NV>(a.taq, base + 2, a.QKS, aq, as, mine, row_o + cx.lane, a.tx, x_in, emb, cx);
                     __syncthreads();
                     if (sh_abort) return;
                     __syncthreads();
                     if (mine) stc64(a.tx + row_o + cx.lane, base + 4, __float_as_uint(r + out[cx.lane]));     // residual_add, emit.rs:455-459
-                } else {
-                    const auto x = pa_index<UO, Q4>(to, mo, a.off_as, po, cx.lane);
-                    __syncthreads();
-                    if (sh_abort) return;
-                    pa_products(wo, x, to.n, smem);
-                    const float v = pa_row_sum(mo, mo.R, smem + po, cx.lane);
-                    if (cx.lane < mo.R) out[c * mo.R + cx.lane] = v;
-                    __syncthreads();
                 }
-            }
-            // ---- norm | gate;up | silu(gate) * up
-            if (stamp) a.stamps[6 * l + 4] = wall_clock64();
-            if (on_g) {
-                if (!comp) {
-                    pa_fetch_x(a.tx, base + 4, emb, a.H, xs, a.xstride, cx);
-                    __syncthreads();
-                    if (sh_abort) return;
-                    pa_norm_quant(xs, a.xstride, nws[cx.tid], a.eps, a.H, smem, a.off_as, cx);
-                    __syncthreads();
+                // ---- norm | gate;up | silu(gate) * up
+                if (stamp) a.stamps[6 * l + 4] = wall_clock64();
+                if (on_g) {
+                    pa_fetch_x<F::NX, ORD>(a.tx, base + 4, emb, a.H, xs, a.xstride, norm_part, cx);
+                    if (!norm_fetching()) return;
                     __syncthreads();
                     if (cx.wave == 0) pa_store_block(silu[cx.lane & 31u], a.taq2 + cx.wg * 9, base + 5, cx.lane, cx.lane < 32);
-                } else {
-                    const auto x = pa_index<UG, Q4>(tg, mg, a.off_as, pg, cx.lane);
-                    if (ntid < PA_POLL_THREADS) nws[ntid] = n2p;
-                    __syncthreads();
-                    if (sh_abort) return;
-                    pa_norm_quant(xs, a.xstride, n2, a.eps, a.H, smem, a.off_as, cx);
-                    __syncthreads();
-                    pa_products(wg, x, tg.n, smem);
-                    const float v = pa_row_sum(mg, 2 * per_wave, smem + pg, cx.lane);
-                    const float up = lane_xor<4>(v);
-                    if (cx.lane < per_wave) silu[c * per_wave + cx.lane] = (v / (1.0f + expf_ref_with<true>(-v, PaExpTab{exp_tab}))) * up;      // silu_mul, emit.rs:380-386
-                    __syncthreads();
                 }
-            }
-            // ---- down + residual
-            if (stamp) a.stamps[6 * l + 5] = wall_clock64();
-            if (on_d) {
-                const bool mine = cx.wave == 0 && cx.lane < PA_COMP * md.R && row_d + cx.lane < md.N;
-                if (!comp) {
-                    const float r = pa_fetch_aq(a.taq2, base + 5, a.I, aq, as, mine, row_d + cx.lane, a.tx, base + 4, emb, cx);
+                // ---- down + residual
+                if (stamp) a.stamps[6 * l + 5] = wall_clock64();
+                if (on_d) {
+                    const bool mine = cx.wave == 0 && cx.lane < PA_COMP * md.R && row_d + cx.lane < md.N;
+                    const float r = pa_fetch_aq<F::NV>(a.taq2, base + 5, a.I, aq, as, mine, row_d + cx.lane, a.tx, base + 4, emb, cx);
                     __syncthreads();
                     if (sh_abort) return;
                     __syncthreads();
                     if (mine) stc64(a.tx + row_d + cx.lane, base + 6, __float_as_uint(r + out[cx.lane]));
+                }
+            }
+        } else {
+            PaSet<F::UQ, Q4> wq;
+            PaSet<F::UO, Q4> wo;
+            PaSet<F::UG1, Q4> wg;
+            PaSet<F::WIDE ? F::UG2 : F::UD, Q4> wd;                              // Wide: first gate;up's second part, then down
+            float4 n2;
+            n1 = load_norm(pa_lds_ptr(layers[0].norm[0]));
+            pa_load(wq, pa_lds_ptr(layers[0].w[0]), tq, cx.lane);
+            if (F::WIDE && on_a) pa_load(wg, pa_lds_ptr(layers[0].w[2]), tg, cx.lane);
+#pragma nounroll
+            for (uint32_t l = 0; l < a.L; l++) {
+                asm volatile("" : "+v"(cx.tid), "+v"(cx.lane));
+                const PaLayer& L = layers[l];
+                const PaLayer& N = layers[l + 1];
+                if (on_q) {
+                    const auto x = pa_index<F::UQ, Q4>(tq, mq, a.off_as, pq, cx.lane);
+                    if (!norm_computing(n1)) return;
+                    pa_products(wq, x, tq.n, smem);
+                    const PaSum v = pa_row_sum<ORD>(mq, mq.R, smem + pq, cx.lane);
+                    if (v.on) out[c * mq.R + v.row] = v.v;
+                    __syncthreads();
+                }
+                if constexpr (F::WIDE) {
+                    __syncthreads();
+                    if (sh_abort) return;
+                    if (on_a) { __syncthreads(); __syncthreads(); }
+                }
+                // While the attention is at work nothing else is on its way to this workgroup: now the matrices that follow are requested (a load that
+                // misses ahead of a poll holds the poll up, whichever wave it belongs to).
+                n2 = load_norm(pa_lds_ptr(L.norm[1]));
+                n1 = load_norm(pa_lds_ptr(N.norm[0]));
+                pa_load(wo, pa_lds_ptr(L.w[1]), to, cx.lane);
+                if constexpr (F::WIDE) {
+                    if (!on_a) pa_load(wg, pa_lds_ptr(L.w[2]), tg, cx.lane);
+                    if (!on_o) {
+                        if (!on_a) { __syncthreads(); if (sh_abort) return; }
+                        pa_load<F::UG1>(wd, pa_lds_ptr(L.w[2]), tg, cx.lane);
+                    }
                 } else {
-                    const auto x = pa_index<UD, Q4>(td, md, a.off_as, pd, cx.lane);
+                    pa_load(wg, pa_lds_ptr(L.w[2]), tg, cx.lane);
+                    pa_load(wd, pa_lds_ptr(L.w[3]), td, cx.lane);
+                    pa_load(wq, pa_lds_ptr(N.w[0]), tq, cx.lane);
+                }
+                if (on_o) {
+                    const auto x = pa_index<F::UO, Q4>(to, mo, a.off_as, po, cx.lane);
+                    __syncthreads();
+                    if (sh_abort) return;
+                    pa_products(wo, x, to.n, smem);
+                    const PaSum v = pa_row_sum<ORD>(mo, mo.R, smem + po, cx.lane);
+                    if (v.on) out[c * mo.R + v.row] = v.v;
+                    __syncthreads();
+                    if constexpr (F::WIDE) pa_load<F::UG1>(wd, pa_lds_ptr(L.w[2]), tg, cx.lane);
+                }
+                if (on_g) {
+                    const auto x = pa_index<F::UG1, Q4>(tg, mg, a.off_as, pg, cx.lane);
+                    if (!norm_computing(n2)) return;
+                    pa_products(wg, x, tg.n, smem);
+                    if constexpr (F::WIDE) pa_products<F::UG1>(wd, pa_index<F::UG2, Q4, F::UG1>(tg, mg, a.off_as, pg, cx.lane), tg.n, smem);
+                    const PaSum v = pa_row_sum<ORD>(mg, 2 * per_wave, smem + pg, cx.lane);
+                    const float up = ORD ? lane_xor<4>(v.v) : lane_xor<32>(v.v);           // row r + 4 of 8
+                    if (v.on && v.row < per_wave) silu[c * per_wave + v.row] = (v.v / (1.0f + expf_ref_with<true>(-v.v, PaExpTab{exp_tab}))) * up;      // silu_mul, emit.rs:380-386
+                    __syncthreads();
+                }
+                if constexpr (F::WIDE) pa_load(wd, pa_lds_ptr(L.w[3]), td, cx.lane);
+                if (on_d) {
+                    const auto x = pa_index<F::UD, Q4>(td, md, a.off_as, pd, cx.lane);
                     __syncthreads();
                     if (sh_abort) return;
                     pa_products(wd, x, td.n, smem);
-                    const float v = pa_row_sum(md, md.R, smem + pd, cx.lane);
-                    if (cx.lane < md.R) out[c * md.R + cx.lane] = v;
+                    const PaSum v = pa_row_sum<ORD>(md, md.R, smem + pd, cx.lane);
+                    if (v.on) out[c * md.R + v.row] = v.v;
                     __syncthreads();
                 }
+                if constexpr (F::WIDE) {
+                    pa_load(wq, pa_lds_ptr(N.w[0]), tq, cx.lane);
+                    if (on_a) pa_load(wg, pa_lds_ptr(N.w[2]), tg, cx.lane);
+                }
             }
+            pa_load(wl[0], a.lm, pa_task(ml, lwv), cx.lane);
         }
-        if (comp) pa_load(wl[0], a.lm, pa_task(ml, lwv), cx.lane);
     } else {
-        if (comp) {
-            const float* nw = pa_lds_ptr(layers[a.L].norm[0]);
-            n1 = pa_at<float>(nw, min(cx.tid, a.H - 1) * 4);
-            n1p = pa_at<float>(nw, min(ntid, a.H - 1) * 4);
-        }
-        if (cx.wg - cx.G < a.heads) {
-            pa_attention<HD>(a, layers, attn, exp_tab, pos, cx.wg - cx.G, cx);
-            if (sh_abort) return;
+        if (comp) n1 = load_norm(pa_lds_ptr(layers[a.L].norm[0]));
+        if constexpr (!F::WIDE) {
+            if (on_a) {
+                const PaHead<HD, F::AW> ph(a, head, pos, cx.wave);
+#pragma nounroll
+                for (uint32_t l = 0; l < a.L; l++) {
+                    asm volatile("" : "+v"(cx.tid), "+v"(cx.lane));
+                    PaKv<HD> kv;
+                    ph.load(kv, a, layers[l], pos, cx.lane);                     // requested as soon as the layer before is done
+                    ph.step(kv, a, layers[l], attn, exp_tab, pos, a.tag_base + 6 * l + 1, cx);
+                    if (sh_abort) return;
+                }
+            }
         }
         if (comp) pa_load(wl[0], a.lm, pa_task(ml, lwv), cx.lane);
         // a workgroup without rows in the layers looks for the final row now and then only
@@ -780,24 +894,18 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
     if (stamp) a.stamps[6 * a.L] = wall_clock64();
     ArgPair best{-INFINITY, 0};
     if (!comp) {
-        pa_fetch_x(a.tx, a.tag_base + 6 * a.L, emb, a.H, xs, a.xstride, cx);
-        __syncthreads();
-        if (sh_abort) return;
-        pa_norm_quant(xs, a.xstride, nws[cx.tid], a.eps, a.H, smem, a.off_as, cx);
-        __syncthreads();
+        pa_fetch_x<F::NX, ORD>(a.tx, a.tag_base + 6 * a.L, emb, a.H, xs, a.xstride, norm_part, cx);
+        if (!norm_fetching()) return;
     } else {
         const uint32_t pl = ml.prod + c * a.prod_words * 4;
-        if (ntid < PA_POLL_THREADS) nws[ntid] = n1p;
-        __syncthreads();
-        if (sh_abort) return;
-        pa_norm_quant(xs, a.xstride, n1, a.eps, a.H, smem, a.off_as, cx);
-        __syncthreads();
-        auto tile = [&](uint32_t t, const PaSet<UL, LMQ4>& w) {
+        if (!norm_computing(n1)) return;
+        auto tile = [&](uint32_t t, const PaSet<F::UL, LMQ4>& w) {
             const PaTask task = pa_task(ml, t);
-            pa_products(w, pa_index<UL, LMQ4>(task, ml, a.off_as, pl, cx.lane), task.n, smem);
-            const uint32_t rows = pa_rows(ml, t), row = t * ml.R + cx.lane;
-            float v = pa_row_sum(ml, rows, smem + pl, cx.lane);
-            if (cx.lane < rows) {
+            pa_products(w, pa_index<F::UL, LMQ4>(task, ml, a.off_as, pl, cx.lane), task.n, smem);
+            const PaSum sum = pa_row_sum<ORD>(ml, pa_rows(ml, t), smem + pl, cx.lane);
+            const uint32_t row = t * ml.R + sum.row;
+            float v = sum.v;
+            if (sum.on) {
                 stg(a.logits + row, v);
                 // apply_repeat_penalty (project.rs:505-513) ahead of the argmax.  The lane that holds the row of the token being fed is the
                 // only one in the grid to touch that counter: it adds this step's occurrence.
@@ -845,13 +953,20 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
     }
 }
 
-template <int HD>
+template <typename F, bool ORD, int HD>
 const void* pa_kernel_hd(bool q4, bool lmq4) {
-    if (q4) return lmq4 ? reinterpret_cast<const void*>(decode_ahead_kernel<HD, true, true>) : reinterpret_cast<const void*>(decode_ahead_kernel<HD, true, false>);
-    return lmq4 ? reinterpret_cast<const void*>(decode_ahead_kernel<HD, false, true>) : reinterpret_cast<const void*>(decode_ahead_kernel<HD, false, false>);
+    if (q4) return lmq4 ? reinterpret_cast<const void*>(decode_ahead_kernel<F, ORD, HD, true, true>) : reinterpret_cast<const void*>(decode_ahead_kernel<F, ORD, HD, true, false>);
+    return lmq4 ? reinterpret_cast<const void*>(decode_ahead_kernel<F, ORD, HD, false, true>) : reinterpret_cast<const void*>(decode_ahead_kernel<F, ORD, HD, false, false>);
 }
-template <int HD>
-uint32_t pa_attn_bytes() { return (uint32_t)sizeof(PaAttn<HD>); }
+
+// What a form means for a shape.
+struct PaForm { int units[5]; uint32_t nx, nv, aw; bool wide; const void* kernel; uint32_t attn_bytes; };
+template <typename F, bool ORD>
+PaForm pa_form(uint32_t hd, bool q4, bool lmq4) {
+    return PaForm{{F::UQ, F::UO, F::UG1 + F::UG2, F::UD, F::UL}, F::NX, F::NV, F::AW, F::WIDE,
+                  hd == 64 ? pa_kernel_hd<F, ORD, 64>(q4, lmq4) : hd == 96 ? pa_kernel_hd<F, ORD, 96>(q4, lmq4) : pa_kernel_hd<F, ORD, 128>(q4, lmq4),
+                  (uint32_t)(hd == 64 ? sizeof(PaAttn<64, F::AW>) : hd == 96 ? sizeof(PaAttn<96, F::AW>) : sizeof(PaAttn<128, F::AW>))};
+}
 
 }  // namespace
 
@@ -859,7 +974,7 @@ struct PaState {
     PaArgs args{};
     std::vector<void*> owned;
     const void* kernel = nullptr;
-    uint32_t grid = 0, lds = 0, n_stamps = 0;
+    uint32_t grid = 0, lds = 0, n_stamps = 0, max_rows = 0;
     uint64_t* tagged = nullptr;
     size_t tagged_bytes = 0;
     std::vector<unsigned long long> stamps_host;
@@ -882,9 +997,8 @@ struct PaState {
 
 void pa_destroy(PaState* st) { delete st; }
 
-// Contexts of up to PA_WAVES blocks: a workgroup takes a head's whole context, and lanes without a key of their own read the cache's first row, which an
-// empty cache does not have yet.
-bool pa_covers(const PaState* st, int64_t pos) { return st && pos >= 1 && pos < (int64_t)(PA_WAVES * PA_B); }
+// A workgroup takes a head's whole context, a wave a block of 64 keys; lanes without a key of their own read the cache's first row, which an empty cache does not have yet.
+bool pa_covers(const PaState* st, int64_t pos) { return st && pos >= 1 && pos < (int64_t)st->max_rows; }
 
 int32_t pa_create(const forge_hip_config& c, const std::vector<PdLayerIn>& layers, const QWeight& lm_head, const float* embed, const float* final_norm,
                   const float* cos_t, const float* sin_t, float* logits, uint32_t* state, uint32_t* counts, PaState** out) {
@@ -893,8 +1007,11 @@ int32_t pa_create(const forge_hip_config& c, const std::vector<PdLayerIn>& layer
     if (c.sliding_window != 0 || layers.empty() || !layers[0].qkv || lm_head.kquant()) return FORGE_HIP_OK;
     if (hd != 64 && hd != 96 && hd != 128) return FORGE_HIP_OK;
     if (H < 64 || I < 64 || QKS < 64) return FORGE_HIP_OK;
+    const bool q4 = c.wdtype == FORGE_HIP_Q4_0, lmq4 = c.lm_head_dtype == FORGE_HIP_Q4_0;
+    const bool exact = (c.flags & FORGE_HIP_FLAG_EXACT) != 0;
+    const PaForm f = H <= PaNarrow::NX * PA_POLL_THREADS ? pa_form<PaNarrow, true>(hd, q4, lmq4) : exact ? pa_form<PaWide, true>(hd, q4, lmq4) : pa_form<PaWide, false>(hd, q4, lmq4);
     // what the polling threads fetch at once
-    if (H > PA_PN * PA_POLL_THREADS || I / 32 * 9 > PA_PN * PA_POLL_THREADS || QKS / 32 * 9 > PA_PN * PA_POLL_THREADS) return FORGE_HIP_OK;
+    if (H > f.nx * PA_POLL_THREADS || I / 32 * 9 > f.nv * PA_POLL_THREADS || QKS / 32 * 9 > f.nv * PA_POLL_THREADS) return FORGE_HIP_OK;
     // rows that the reference adds in its four-accumulator order (the last len % 4 of a chunk) are left to the other kernels
     if (H % 4 || I % 4 || QKS % 4 || KV % 4 || c.vocab % 4) return FORGE_HIP_OK;
     int dev = 0, cus = 0, khz = 0;
@@ -905,29 +1022,35 @@ int32_t pa_create(const forge_hip_config& c, const std::vector<PdLayerIn>& layer
     std::unique_ptr<PaState> st(new PaState());
     PaArgs& a = st->args;
     const uint32_t nq[5] = {QKS + 2 * KV, H, 2 * I, H, c.vocab}, kk[5] = {H, QKS, H, I, H};
-    const int units[5] = {UQ, UO, UG, UD, UL};
     for (int i = 0; i < 5; i++) {
         PaMat& m = a.m[i];
         m.N = nq[i]; m.nblk = kk[i] / 32;
         m.magic = (uint32_t)(0x100000000ull / m.nblk) + 1u;
-        m.R = 64u * units[i] / m.nblk;                             // the most a wave can hold
+        m.R = 64u * f.units[i] / m.nblk;                             // the most a wave can hold
         if (i == 0) m.R = std::min(m.R & ~1u, PA_MAX_ROWS);        // a rotation's pair in one wave
         else if (i == 1 || i == 3) m.R = std::min(m.R, PA_MAX_ROWS);
         else if (i == 2) { if (m.R < 64 / PA_COMP) return FORGE_HIP_OK; m.R = 64 / PA_COMP; }
         else m.R = std::min(m.R, 32u);
         if (m.R == 0) return FORGE_HIP_OK;
     }
-    // The fewest workgroups that hold every row at the most per wave and gate;up by whole blocks of 32, a workgroup per head, and what is left of the
-    // device for the lm_head; then as few rows per wave as that many workgroups allow.
+    // Narrow: the fewest workgroups that hold every row at the most per wave, gate;up by whole blocks of 32, then a workgroup per head, and what is left of the device
+    // for the lm_head; as few rows per wave as that many workgroups allow.
+    // Wide: every workgroup a block of gate;up and of down's rows; the last ones a head each in place of rows of q;k;v and o, which lie at either end of the others.
     uint32_t g = I / 32;
     for (int i : {0, 1, 3}) g = std::max(g, (a.m[i].N + a.m[i].R * PA_COMP - 1) / (a.m[i].R * PA_COMP));
-    if (g + c.heads > (uint32_t)cus) return FORGE_HIP_OK;
-    a.G = g;
+    if (g + (f.wide ? 0u : c.heads) > (uint32_t)cus || c.heads >= (uint32_t)cus) return FORGE_HIP_OK;
     st->grid = (uint32_t)cus;
+    a.G = f.wide ? st->grid : g;
+    a.head0 = f.wide ? st->grid - c.heads : g;
     for (int i : {0, 1, 3}) {
-        a.m[i].R = (a.m[i].N + g * PA_COMP - 1) / (g * PA_COMP);
-        if (i == 0) a.m[i].R = pa_up(a.m[i].R, 2);
+        const uint32_t n = f.wide && i != 3 ? a.head0 : a.G;             // workgroups that may hold rows
+        uint32_t r = (a.m[i].N + n * PA_COMP - 1) / (n * PA_COMP);
+        if (i == 0) r = pa_up(r, 2);
+        if (r > a.m[i].R) return FORGE_HIP_OK;
+        a.m[i].R = r;
+        a.m[i].wg0 = f.wide && i == 1 ? n - (a.m[i].N + r * PA_COMP - 1) / (r * PA_COMP) : 0u;
     }
+    st->max_rows = f.aw * PA_B;
     a.L = (uint32_t)layers.size(); a.H = H; a.I = I; a.QKS = QKS; a.KV = KV; a.heads = c.heads; a.kv_heads = c.kv_heads;
     a.eps = c.rms_eps;
     const uint32_t kmax = std::max(std::max(H, I), QKS);
@@ -936,23 +1059,34 @@ int32_t pa_create(const forge_hip_config& c, const std::vector<PdLayerIn>& layer
     auto odd16 = [](uint32_t words) { return words % 8 ? words : words + 4; };      // rows an odd number of 16-byte units apart spread over the banks
     a.xstride = odd16(pa_up(H / 16, PA_SSQ));
     a.off_out = a.off_xs + 16 * a.xstride * 4;
-    a.off_nw = a.off_out + PA_COMP * PA_MAX_ROWS * 4;
-    a.off_silu = a.off_nw + PA_POLL_THREADS * 4;
+    a.off_silu = a.off_out + PA_COMP * PA_MAX_ROWS * 4;
     a.off_prod = a.off_silu + 32 * 4;
     a.prod_words = 0;
     for (int i = 0; i < 5; i++) {
         PaMat& m = a.m[i];
         m.stride = odd16(pa_up(m.nblk, PA_SUM));
-        m.prod = a.off_prod + a.prod_words * 4;
-        a.prod_words += m.R * m.stride + 4;
+        while ((m.R << (m.fold + 1)) <= 64) m.fold++;
+        // matrices of one depth share an area: the zeros behind their rows are the same
+        int same = 0;
+        while (a.m[same].nblk != m.nblk) same++;
+        uint32_t rows = 0;
+        for (int k = i; same == i && k < 5; k++)
+            if (a.m[k].nblk == m.nblk) rows = std::max(rows, a.m[k].R);
+        if (same == i) {
+            m.prod = a.off_prod + a.prod_words * 4;
+            m.dump = rows * m.stride * 4;
+            a.prod_words += rows * m.stride + 4;
+        } else {
+            m.prod = a.m[same].prod;
+            m.dump = a.m[same].dump;
+        }
     }
     a.off_layers = a.off_prod + PA_COMP * a.prod_words * 4;
     a.lds_words = a.off_layers / 4;
     a.off_attn = pa_up(a.off_layers + ((uint32_t)layers.size() + 1) * (uint32_t)sizeof(PaLayer), 16);
-    st->lds = a.off_attn + (hd == 64 ? pa_attn_bytes<64>() : hd == 96 ? pa_attn_bytes<96>() : pa_attn_bytes<128>());
+    st->lds = a.off_attn + f.attn_bytes;
     if (st->lds > 64000) return FORGE_HIP_OK;
-    const bool q4 = c.wdtype == FORGE_HIP_Q4_0, lmq4 = c.lm_head_dtype == FORGE_HIP_Q4_0;
-    st->kernel = hd == 64 ? pa_kernel_hd<64>(q4, lmq4) : hd == 96 ? pa_kernel_hd<96>(q4, lmq4) : pa_kernel_hd<128>(q4, lmq4);
+    st->kernel = f.kernel;
     int per_cu = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, st->kernel, PA_THREADS, st->lds) != hipSuccess || per_cu < 1) { (void)hipGetLastError(); return FORGE_HIP_OK; }
 

@@ -1,4 +1,4 @@
-"""The resident decode kernel of narrow models (decode_ahead.hip) against the order-faithful kernel sequence, bit for bit."""
+"""The resident decode kernel of short contexts (decode_ahead.hip) against the order-faithful kernel sequence, bit for bit."""
 import numpy as np
 import pytest
 
@@ -37,6 +37,11 @@ SHAPES = {
     "q4_ragged": (Q4, 608, 1056, 9, 1, 64, 4100, None),
     "widest": (Q8, 768, 2048, 8, 2, 96, 3004, Q4),
     "hd128": (Q4, 352, 736, 6, 2, 128, 1000, Q8),
+    # the wide form: the 1B shape, one block of channels above the narrow form, ragged depths and few tiles
+    "wide_1b": (Q8, 2048, 8192, 32, 8, 64, 8000, None),
+    "wide_least": (Q4, 800, 1088, 12, 4, 64, 1000, Q8),
+    "wide_hd128": (Q8, 1184, 3040, 9, 3, 128, 2052, Q4),
+    "wide_hd96": (Q4, 1536, 4096, 16, 4, 96, 4000, None),
 }
 
 
@@ -47,7 +52,7 @@ def test_equals_the_kernel_sequence(fh, torch_gpu, monkeypatch, name):
     cfg = shape(fh, wd, *rest, layers=2 if name == "smollm2" else 3, lm=lm)
     one, seq = pair(fh, monkeypatch, cfg, 7)
     toks = fh.synth.uniform_ids(8, 400, cfg["vocab"])
-    for n in (1, 60, 126, 380):
+    for n in (1, 60, 126, 380 if cfg["hidden"] <= 768 else 188):
         one.reset(); seq.reset()
         same_bits(one.forward_prefill(toks[:n]), seq.forward_prefill(toks[:n]))
         assert one.decode_launches == 1 and seq.decode_launches > 1
@@ -61,17 +66,17 @@ def test_equals_the_kernel_sequence(fh, torch_gpu, monkeypatch, name):
     one.close(); seq.close()
 
 
-@pytest.mark.parametrize("head_dim", [64, 128])
-def test_across_its_last_context_with_a_penalty(fh, torch_gpu, monkeypatch, head_dim):
+@pytest.mark.parametrize("hidden,head_dim,line", [(256, 64, 768), (256, 128, 768), (800, 64, 256)])
+def test_across_its_last_context_with_a_penalty(fh, torch_gpu, monkeypatch, hidden, head_dim, line):
     """From the kernel to the sequence where the context outgrows a workgroup's blocks, and back after a reset, the repeat penalty's counts shared by both."""
-    cfg = shape(fh, Q8, 256, 512, 4, 2, head_dim, 1000)
+    cfg = shape(fh, Q8, hidden, 512, 4, 2, head_dim, 1000)
     one, seq = pair(fh, monkeypatch, cfg, 17)
     toks = fh.synth.uniform_ids(18, 770, cfg["vocab"])
     for turn in range(2):
         for m in (one, seq):
             m.reset()
             m.set_repeat_penalty(1.3)
-            m.forward_prefill(toks[:764])
+            m.forward_prefill(toks[:line - 4])
         t = 5
         for _ in range(8):
             a, b = one.forward_greedy(t), seq.forward_greedy(t)
@@ -81,9 +86,10 @@ def test_across_its_last_context_with_a_penalty(fh, torch_gpu, monkeypatch, head
     one.close(); seq.close()
 
 
-def test_rewinds_its_tags_and_gives_up_instead_of_hanging(fh, torch_gpu, monkeypatch):
+@pytest.mark.parametrize("hidden", [256, 800])
+def test_rewinds_its_tags_and_gives_up_instead_of_hanging(fh, torch_gpu, monkeypatch, hidden):
     """Tags that are about to wrap, and a poll limit of 1: a step that gave up has not happened and can be fed again."""
-    cfg = shape(fh, Q8, 256, 512, 4, 2, 64, 1000)
+    cfg = shape(fh, Q8, hidden, 512, 4, 2, 64, 1000)
     monkeypatch.setenv("FORGE_HIP_PD_TAG_START", str(0xF0000000 - 40))
     one, seq = pair(fh, monkeypatch, cfg, 27)
     monkeypatch.delenv("FORGE_HIP_PD_TAG_START")
@@ -112,17 +118,20 @@ def test_rewinds_its_tags_and_gives_up_instead_of_hanging(fh, torch_gpu, monkeyp
     one.close(); seq.close()
 
 
-def test_fast_mode_takes_it_too(fh, oracle, torch_gpu):
-    """Fast mode: from the same cache the kernel's step is the order-faithful one.  A prompt of one token leaves the cache that both modes' first step leaves."""
-    cfg = shape(fh, Q8, 256, 512, 4, 2, 64, 1000)
-    blob = fh.synth.make_weights_blob(cfg, seed=37)
+@pytest.mark.parametrize("name", ["narrow_form", "wide_1b", "wide_least", "wide_hd128"])
+def test_fast_mode_takes_it_too(fh, oracle, torch_gpu, name):
+    """Fast mode, token by token: the narrow form is the order-faithful one, the wide form adds up in another order.  Rounding moves single codes of the
+    8-bit activations, which random weights amplify from layer to layer: two layers, and the loose bound that the other kernels' fast mode is held to."""
+    wd, *rest, lm = SHAPES[name] if name in SHAPES else (Q8, 256, 512, 4, 2, 64, 1000, None)
+    cfg = shape(fh, wd, *rest, layers=2, lm=lm)
+    blob = fh.synth.make_weights_blob(cfg, seed=37, threads=16)
     fast, om = fh.HipModel(dict(cfg, flags=0), blob), oracle.Model(cfg, blob, 0, 1)
     toks = fh.synth.uniform_ids(38, 70, cfg["vocab"])
     fast.forward(int(toks[0])); om.forward(int(toks[0]))
     assert fast.decode_launches == 1
     for t in toks[1:]:
         a, b = fast.forward(int(t)), om.forward(int(t))
-    assert np.corrcoef(a, b)[0, 1] > 0.999
+    assert np.all(np.isfinite(a)) and np.corrcoef(a, b)[0, 1] > 0.99
     fast.close()
 
 
