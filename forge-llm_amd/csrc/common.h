@@ -499,7 +499,7 @@ int32_t pd_after_sync(PdState* st, uint32_t abort_flag, hipStream_t s);
 // Milliseconds between the phase starts of the last profiled step: six per layer, then head and argmax.
 int32_t pd_phase_ms(PdState* st, std::vector<float>* out, hipStream_t s);
 
-// decode_ahead.hip — the decode step of a narrow model over a short context as one resident kernel, either mode.  The functions are the pd_ ones' counterparts.
+// decode_ahead.hip — the decode step of a model of up to 2048 channels over a context that its registers hold as one resident kernel, either mode.  The functions are the pd_ ones' counterparts.
 struct PaState;
 int32_t pa_create(const forge_hip_config& c, const std::vector<PdLayerIn>& layers, const QWeight& lm_head, const float* embed, const float* final_norm,
                   const float* cos_t, const float* sin_t, float* logits, uint32_t* state, uint32_t* counts, PaState** out);
@@ -507,7 +507,7 @@ void pa_destroy(PaState* st);
 bool pa_covers(const PaState* st, int64_t pos);         // a step at this position can run so
 void pa_set_repeat_penalty(PaState* st, float penalty);
 void pa_set_poll_limit(PaState* st, uint32_t n);
-int32_t pa_enqueue(PaState* st, bool profile, uint32_t token, hipStream_t s);
+int32_t pa_enqueue(PaState* st, int64_t pos, bool profile, uint32_t token, hipStream_t s);
 bool pa_wait_token(PaState* st, uint32_t* next);
 int32_t pa_after_sync(PaState* st, uint32_t abort_flag, hipStream_t s);
 int32_t pa_phase_ms(PaState* st, std::vector<float>* out, hipStream_t s);

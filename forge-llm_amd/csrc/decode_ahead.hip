@@ -1,4 +1,4 @@
-// One decode token over a short context as ONE kernel whose waves hold their share of a layer's matrices in registers (model::forward, emit.rs:4029-4227).
+// One decode token as ONE kernel whose waves hold their share of a layer's matrices in registers (model::forward, emit.rs:4029-4227).
 //
 // A step is a chain of four products and an attention per layer.  As kernels a link of that chain is 4 to 6 us however small (a launch that does nothing takes
 // 2.7); as phases of the kernel that streams weights of any size (decode_persistent.hip) it is 5.  Here a layer of SmolLM2-135M takes 13 us, one of the 1B shape 24
@@ -19,6 +19,7 @@
 // have them.  Per token in us, kernel sequence (order-faithful mode) / decode_persistent.hip (fast mode) / this, by rows of context:
 //   SmolLM2-135M Q8_0   33: 781 / 880 / 384    300: 820 / 878 / 421    740: 907 / 876 / 466
 //   1B shape Q8_0       33: 754 / 610 / 466 and 427 (order-faithful, fast)    200: - / 636 / 473 and 439       Q4_0, fast: 33: 532 / 407
+//   and in fast mode (PaPart) 260: 637 / 470    1000: 642 / 475    2400: 644 / 483    Q4_0 2400: 570 / 439
 #include <stddef.h>
 #include <string.h>
 
@@ -27,6 +28,7 @@
 #include <memory>
 #include <vector>
 
+#include "attn_decode_math.h"
 #include "common.h"
 #include "device_utils.h"
 #include "expf_ref.h"
@@ -45,7 +47,7 @@ constexpr uint32_t PA_SUM = 24, PA_SSQ = 12;  // a row's products, and an accumu
 // a polling thread takes of the residual row and of gate;up's quantised vector; AW: waves that attend to a head, each to 64 keys.
 //   Narrow (up to 768 channels): a layer in 54 registers of a few dozen workgroups; the heads have workgroups of their own, up to 768 rows of context.
 //   Wide (up to 2048 channels): every compute unit holds a block of 32 gate;up rows in two sets of registers, so heads and weights share workgroups: the last `heads` of
-//   them hold no rows of q;k;v and o, and their fetching waves attend, to up to 256 rows.  down takes the place of the second set when that is done.
+//   them hold no rows of q;k;v and o, and their fetching waves attend, to up to 256 rows (longer contexts, order free: every workgroup's, PaPart).  down takes the place of the second set when that is done.
 struct PaNarrow { static constexpr int UQ = 1, UO = 1, UG1 = 3, UG2 = 0, UD = 1, UL = 4, NX = 3, NV = 3; static constexpr uint32_t AW = PA_WAVES; static constexpr bool WIDE = false; };
 struct PaWide { static constexpr int UQ = 2, UO = 2, UG1 = 4, UG2 = 4, UD = 4, UL = 4, NX = 8, NV = 9; static constexpr uint32_t AW = PA_POLL; static constexpr bool WIDE = true; };
 
@@ -63,6 +65,7 @@ struct PaLayer {
 struct PaArgs {
     PaMat m[5];                               // q;k;v, o, gate;up (N = 2 I; a workgroup holds 32 + 32 rows), down, lm_head
     uint32_t L, H, I, QKS, KV, heads, kv_heads;
+    uint32_t splits;                          // Wide, order free: parts that a long context is attended in (0: it is not)
     uint32_t G, head0;                        // workgroups [0, G) hold the layers' matrices, [head0, head0 + heads) take a head each; all share the lm_head
     float eps;
     const PaLayer* layers;                    // [L + 1]: the last one's first norm is the final norm; its q;k;v is the first layer's (requested, not used)
@@ -76,6 +79,7 @@ struct PaArgs {
     uint64_t* tkv;     // [2 KV]             this position's K row (rotated) and V row, fp16 bits
     uint64_t* taq;     // [QKS/32][9]        attention output, a block of 32: int8 codes (4 per element), then the fp16 scale
     uint64_t* taq2;    // [I/32][9]          silu(gate)*up, same format
+    uint64_t* trec;    // [heads][splits][HD + 2]  Wide, long contexts: a split's weighted sum, maximum and weight sum
     uint64_t* tpart;   // [2 G]              per-workgroup argmax candidates
     float* logits;
     uint32_t* state;   // [0] position  [1] token  [2] next token  [3] abort flag  [4] number of the step that counted its token
@@ -85,7 +89,7 @@ struct PaArgs {
     unsigned long long* host_out;             // host-mapped {launch number, next token}: written last, or null
     uint32_t host_seq;
     unsigned long long* stamps;               // optional: wall clock at the start of every phase (workgroup 0)
-    uint32_t off_as, off_xs, off_out, off_silu, off_prod, off_layers, off_attn, prod_words, lds_words, xstride;      // LDS byte offsets (activation codes at 0)
+    uint32_t off_as, off_xs, off_out, off_silu, off_prod, off_layers, off_attn, off_rec, prod_words, lds_words, xstride;      // LDS byte offsets (activation codes at 0)
 };
 
 // A uniform base and a lane's 32-bit offset in bytes.
@@ -608,6 +612,131 @@ __device__ __forceinline__ void PaHead<HD, AW>::step(PaKv<HD>& kv, const PaArgs&
         }
 }
 
+// Longer contexts where the order is free, a kernel of their own (beside the short form's registers neither has enough: 957 us a token at 2400 rows of the 1B
+// shape, 483 apart): workgroup (KV head, split) attends to its part of the keys, a fetching wave per query head of the group (and the next four heads behind
+// these); a head's workgroup merges the splits.  A pass is 8 keys (heads of 64; 4 of wider ones), 16 bytes of K and V a lane, and all passes of a split are
+// requested before the workgroup waits for the query: what the registers hold of them is where the form ends.  (With a second round of passes behind the first
+// it is the slower one soon after: 8 layers of the 1B shape at 5000 rows 343 us, decode_persistent.hip 324; at 2540 rows 230 against 309.)
+constexpr int PA_PASSES = 10;
+constexpr uint32_t PA_SPLITS = 32, PA_LDS = 64000;
+template <int HD>
+struct PaPart {
+    static constexpr int LPK = HD <= 64 ? 8 : 16, KPW = 64 / LPK, REC = HD + 2;
+    uint32_t kvh, split, t0, t1;              // keys [t0, t1)
+    bool on;
+    __device__ __forceinline__ PaPart(const PaArgs& a, uint32_t wg, uint32_t pos) {
+        kvh = wg % a.kv_heads; split = wg / a.kv_heads;
+        const uint32_t seq = pos + 1, chunk = pa_up((seq + a.splits - 1) / max(a.splits, 1u), KPW);
+        on = split < a.splits;
+        t0 = min(split * chunk, seq);
+        t1 = min(t0 + chunk, seq);
+    }
+    // rows that are not cached read row 0
+    __device__ __forceinline__ void load(Half8* k, Half8* v, const PaArgs& a, const PaLayer& L, uint32_t pos, uint32_t lane) const {
+        const uint16_t* kc = pa_lds_ptr(L.kc) + kvh * HD;
+        const uint16_t* vc = pa_lds_ptr(L.vc) + kvh * HD;
+        const uint32_t c = min(lane % LPK, (uint32_t)HD / 8 - 1);
+#pragma unroll
+        for (int p = 0; p < PA_PASSES; p++) {
+            const uint32_t t = t0 + p * KPW + lane / LPK;
+            const uint32_t at = ((t < pos ? t : 0u) * a.KV + c * 8) * 2;
+            k[p] = pa_at<Half8>(kc, at);
+            v[p] = pa_at<Half8>(vc, at);
+        }
+    }
+    // q_s: the group's heads in LDS, new_s: this position's K row and V row, fp16 pairs.  After the barrier that publishes them.
+    __device__ __forceinline__ void attend(Half8* k, Half8* v, const PaArgs& a, const PaLayer& L, const float* q_s, const Half8* new_s, uint32_t pos, uint32_t tag_out,
+                                           const PaCtx& cx) const {
+        const uint32_t gsize = a.heads / a.kv_heads, lane = cx.lane, slot = lane / LPK, c = lane % LPK;
+        const bool dvalid = c * 8 < (uint32_t)HD;
+        const float scale = 1.0f / sqrtf((float)HD);
+        const uint32_t cv = min(c, (uint32_t)HD / 8 - 1);
+        uint32_t nk[4], nv[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) { nk[i] = new_s[cv].w[i]; nv[i] = new_s[HD / 8 + cv].w[i]; }
+        for (uint32_t g = cx.wave; g < gsize; g += PA_POLL) {
+            float qf[8], acc[8], m = -INFINITY, l = 0.f;
+#pragma unroll
+            for (int i = 0; i < 8; i++) { qf[i] = dvalid ? q_s[g * HD + c * 8 + i] : 0.f; acc[i] = 0.f; }
+            if (g >= PA_POLL) load(k, v, a, L, pos, lane);
+#pragma unroll
+            for (int p0 = 0; p0 < PA_PASSES; p0 += 2) {
+                const uint32_t tp = t0 + p0 * KPW;
+                if (tp < t1) {
+                    float sc[2];
+                    Half8 vv[2];
+#pragma unroll
+                    for (int u = 0; u < 2; u++) {
+                        const uint32_t t = tp + u * KPW + slot;
+                        Half8 kk;
+#pragma unroll
+                        for (int i = 0; i < 4; i++) {
+                            kk.w[i] = t == pos ? nk[i] : k[p0 + u].w[i];
+                            vv[u].w[i] = t == pos ? nv[i] : v[p0 + u].w[i];
+                        }
+                        const float d = key_dot<LPK>(qf, kk);
+                        sc[u] = t < t1 ? d * scale : -INFINITY;
+                    }
+                    softmax_block_update<2>(m, l, acc, sc, vv);
+                }
+            }
+            // fold the key slots: every lane of a column ends with the same sums
+            auto fold = [&](auto O) {
+                const float m2 = lane_xor<O.value>(m), l2 = lane_xor<O.value>(l), mn = fmaxf(m, m2);
+                const float s1 = m == -INFINITY ? 0.f : __expf(m - mn), s2 = m2 == -INFINITY ? 0.f : __expf(m2 - mn);
+                l = l * s1 + l2 * s2;
+#pragma unroll
+                for (int i = 0; i < 8; i++) acc[i] = acc[i] * s1 + lane_xor<O.value>(acc[i]) * s2;
+                m = mn;
+            };
+            if (LPK == 8) fold(std::integral_constant<int, 8>{});
+            fold(std::integral_constant<int, 16>{});
+            fold(std::integral_constant<int, 32>{});
+            uint64_t* rec = a.trec + ((size_t)(kvh * gsize + g) * a.splits + split) * REC;
+#pragma unroll
+            for (int j = 0; j < 8 / KPW; j++) {               // lane (slot, column): element column 8 + slot + KPW j
+                float x = acc[KPW * j];
+#pragma unroll
+                for (int i = 1; i < KPW; i++) x = slot == (uint32_t)i ? acc[KPW * j + i] : x;
+                if (dvalid) stc64(rec + c * 8 + slot + KPW * j, tag_out, __float_as_uint(x));
+            }
+            if (lane < 2) stc64(rec + HD + lane, tag_out, __float_as_uint(lane ? l : m));
+        }
+    }
+};
+
+// The splits of head h into its quantised row; recs: splits records, wt: a weight per split.  Fetching waves; two barriers.
+template <int HD>
+__device__ __forceinline__ void pa_merge(const PaArgs& a, uint32_t h, uint32_t tag_in, uint32_t tag_out, float* recs, float* wt, const PaCtx& cx) {
+    constexpr uint32_t REC = HD + 2, N = (PA_SPLITS * REC + PA_POLL_THREADS - 1) / PA_POLL_THREADS;
+    const uint32_t ne = a.splits * REC;
+    const uint64_t* base = a.trec + (size_t)h * ne;
+    uint32_t v[N];
+    pa_poll<N>([&](int i) { return base + min(cx.tid + i * PA_POLL_THREADS, ne - 1); }, [&](int) { return tag_in; }, v, cx);
+#pragma unroll
+    for (uint32_t i = 0; i < N; i++)
+        if (cx.tid + i * PA_POLL_THREADS < ne) recs[cx.tid + i * PA_POLL_THREADS] = __uint_as_float(v[i]);
+    __syncthreads();
+    if (*cx.sh_abort) return;
+    if (cx.wave == 0) {
+        const bool in = cx.lane < a.splits;
+        const float m = in ? recs[cx.lane * REC + HD] : -INFINITY, l = in ? recs[cx.lane * REC + HD + 1] : 0.f;
+        const float mx = wave_max(m);
+        const float w = m == -INFINITY ? 0.f : __expf(m - mx);
+        const float den = wave_sum(w * l);
+        if (in) wt[cx.lane] = w / den;
+    }
+    __syncthreads();
+    if (cx.tid < pa_up(HD, 64)) {
+        const uint32_t d = min(cx.tid, (uint32_t)HD - 1);
+        float o = 0.f;
+#pragma unroll 8
+        for (uint32_t i = 0; i < a.splits; i++) o = fmaf(wt[i], recs[i * REC + d], o);
+        const uint32_t e = h * HD + cx.tid;
+        pa_store_block(cx.tid < HD ? o : 0.f, a.taq + e / 32 * 9, tag_out, cx.lane, cx.tid < HD);
+    }
+}
+
 // One workgroup's part of an argmax: the LAST index among equal maxima (project.rs:501-503).
 __device__ __forceinline__ ArgPair pa_arg_wg(ArgPair v, ArgPair* sh, const PaCtx& cx) {
     auto fold = [&](auto O) { v = arg_better(v, ArgPair{lane_xor<O.value>(v.v), lane_xor<O.value>(v.i)}); };
@@ -621,8 +750,9 @@ __device__ __forceinline__ ArgPair pa_arg_wg(ArgPair v, ArgPair* sh, const PaCtx
     return r;
 }
 
-// The tag of a phase instance: tag_base + 6 layer + 1 q;k;v, 2 attention, 4 o, 5 gate;up, 6 down; the argmax's is behind the last layer's.
-template <typename F, bool ORD, int HD, bool Q4, bool LMQ4>
+// The tag of a phase instance: tag_base + 6 layer + 1 q;k;v, 2 attention (long contexts: its parts, 3 their merge), 4 o, 5 gate;up, 6 down; the argmax's is behind
+// the last layer's.
+template <typename F, bool ORD, bool LONG, int HD, bool Q4, bool LMQ4>
 __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
     extern __shared__ __align__(16) uint8_t smem[];
     __shared__ uint32_t sh_abort;
@@ -714,6 +844,9 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
         // Fetching and computing waves go through the layers in loops of their own (with the same barriers): neither keeps the other's registers.
         if (!comp) {
             const PaHead<HD, F::AW> ph(a, F::WIDE && on_a ? head : 0u, pos, cx.wave);
+            const PaPart<HD> part(a, cx.wg, pos);
+            float* q_s = reinterpret_cast<float*>(attn);                         // long contexts: the group's heads, then this position's K and V row
+            Half8* new_s = reinterpret_cast<Half8*>(q_s + a.heads / a.kv_heads * HD);
 #pragma nounroll
             for (uint32_t l = 0; l < a.L; l++) {
                 // The thread's number is read afresh in every layer: addresses that follow from it would be kept from layer to layer and not fit the registers.
@@ -722,6 +855,10 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
                 const uint32_t base = a.tag_base + 6 * l, x_in = l ? base : 0u;
                 // ---- norm | q;k;v | rotation, cache row
                 if (stamp) a.stamps[6 * l] = wall_clock64();
+                Half8 pk[LONG ? PA_PASSES : 1], pv[LONG ? PA_PASSES : 1];
+                if constexpr (LONG) {
+                    if (part.on && cx.wave < a.heads / a.kv_heads) part.load(pk, pv, a, L, pos, cx.lane);
+                }
                 if (on_q) {
                     uint16_t* kc = pa_lds_ptr(L.kc);
                     uint16_t* vc = pa_lds_ptr(L.vc);
@@ -743,7 +880,36 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
                 }
                 // ---- attention
                 if (stamp) a.stamps[6 * l + 1] = wall_clock64();
-                if constexpr (F::WIDE) {
+                if constexpr (LONG) {
+                    if (part.on) {
+                        // the group's heads, this position's K row and V row
+                        const uint32_t gsize = a.heads / a.kv_heads, nq = gsize * HD, ne = nq + 2 * HD;
+                        constexpr int N = 4;
+                        uint32_t v[N];
+                        auto at = [&](uint32_t e) {
+                            e = min(e, ne - 1);
+                            return e < nq ? a.tq + (size_t)part.kvh * nq + e : a.tkv + (e - nq < HD ? part.kvh * HD + (e - nq) : a.KV + part.kvh * HD + (e - nq - HD));
+                        };
+                        pa_poll<N>([&](int i) { return at(cx.tid + i * PA_POLL_THREADS); }, [&](int) { return base + 1; }, v, cx);
+#pragma unroll
+                        for (int i = 0; i < N; i++) {
+                            const uint32_t e = cx.tid + i * PA_POLL_THREADS;
+                            if (e < nq) q_s[e] = __uint_as_float(v[i]);
+                            else if (e < ne) reinterpret_cast<uint16_t*>(new_s)[e - nq] = (uint16_t)v[i];
+                        }
+                        __syncthreads();
+                        if (sh_abort) return;
+                        part.attend(pk, pv, a, L, q_s, new_s, pos, base + 2, cx);
+                    } else if (!glance(a.tkv + 2 * a.KV - 1, base + 1)) {
+                        return;
+                    }
+                    if (on_a) {
+                        pa_merge<HD>(a, head, base + 2, base + 3, reinterpret_cast<float*>(smem + a.off_rec), silu, cx);
+                        if (sh_abort) return;
+                    } else if (!on_o && !glance(a.taq + a.QKS / 32 * 9 - 1, base + 3)) {
+                        return;
+                    }
+                } else if constexpr (F::WIDE) {
                     if (on_a) {
                         PaKv<HD> kv;
                         ph.load(kv, a, L, pos, cx.lane);
@@ -758,7 +924,7 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
                 if (stamp) { const unsigned long long t = wall_clock64(); a.stamps[6 * l + 2] = t; a.stamps[6 * l + 3] = t; }
                 if (on_o) {
                     const bool mine = cx.wave == 0 && cx.lane < PA_COMP * mo.R && row_o + cx.lane < mo.N;
-                    const float r = pa_fetch_aq<F::NV>(a.taq, base + 2, a.QKS, aq, as, mine, row_o + cx.lane, a.tx, x_in, emb, cx);
+                    const float r = pa_fetch_aq<F::NV>(a.taq, base + (LONG ? 3 : 2), a.QKS, aq, as, mine, row_o + cx.lane, a.tx, x_in, emb, cx);
                     __syncthreads();
                     if (sh_abort) return;
                     __syncthreads();
@@ -808,7 +974,7 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
                 if constexpr (F::WIDE) {
                     __syncthreads();
                     if (sh_abort) return;
-                    if (on_a) { __syncthreads(); __syncthreads(); }
+                    if (on_a) { __syncthreads(); if (LONG && sh_abort) return; __syncthreads(); }
                 }
                 // While the attention is at work nothing else is on its way to this workgroup: now the matrices that follow are requested (a load that
                 // misses ahead of a poll holds the poll up, whichever wave it belongs to).
@@ -953,18 +1119,22 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
     }
 }
 
-template <typename F, bool ORD, int HD>
+template <typename F, bool ORD, bool LONG, int HD>
 const void* pa_kernel_hd(bool q4, bool lmq4) {
-    if (q4) return lmq4 ? reinterpret_cast<const void*>(decode_ahead_kernel<F, ORD, HD, true, true>) : reinterpret_cast<const void*>(decode_ahead_kernel<F, ORD, HD, true, false>);
-    return lmq4 ? reinterpret_cast<const void*>(decode_ahead_kernel<F, ORD, HD, false, true>) : reinterpret_cast<const void*>(decode_ahead_kernel<F, ORD, HD, false, false>);
+    if (q4) return lmq4 ? reinterpret_cast<const void*>(decode_ahead_kernel<F, ORD, LONG, HD, true, true>) : reinterpret_cast<const void*>(decode_ahead_kernel<F, ORD, LONG, HD, true, false>);
+    return lmq4 ? reinterpret_cast<const void*>(decode_ahead_kernel<F, ORD, LONG, HD, false, true>) : reinterpret_cast<const void*>(decode_ahead_kernel<F, ORD, LONG, HD, false, false>);
 }
 
 // What a form means for a shape.
 struct PaForm { int units[5]; uint32_t nx, nv, aw; bool wide; const void* kernel; uint32_t attn_bytes; };
+template <typename F, bool ORD, bool LONG>
+const void* pa_kernel(uint32_t hd, bool q4, bool lmq4) {
+    return hd == 64 ? pa_kernel_hd<F, ORD, LONG, 64>(q4, lmq4) : hd == 96 ? pa_kernel_hd<F, ORD, LONG, 96>(q4, lmq4) : pa_kernel_hd<F, ORD, LONG, 128>(q4, lmq4);
+}
 template <typename F, bool ORD>
 PaForm pa_form(uint32_t hd, bool q4, bool lmq4) {
     return PaForm{{F::UQ, F::UO, F::UG1 + F::UG2, F::UD, F::UL}, F::NX, F::NV, F::AW, F::WIDE,
-                  hd == 64 ? pa_kernel_hd<F, ORD, 64>(q4, lmq4) : hd == 96 ? pa_kernel_hd<F, ORD, 96>(q4, lmq4) : pa_kernel_hd<F, ORD, 128>(q4, lmq4),
+                  pa_kernel<F, ORD, false>(hd, q4, lmq4),
                   (uint32_t)(hd == 64 ? sizeof(PaAttn<64, F::AW>) : hd == 96 ? sizeof(PaAttn<96, F::AW>) : sizeof(PaAttn<128, F::AW>))};
 }
 
@@ -974,7 +1144,8 @@ struct PaState {
     PaArgs args{};
     std::vector<void*> owned;
     const void* kernel = nullptr;
-    uint32_t grid = 0, lds = 0, n_stamps = 0, max_rows = 0;
+    const void* kernel_long = nullptr;
+    uint32_t grid = 0, lds = 0, n_stamps = 0, max_rows = 0, one_rows = 0;
     uint64_t* tagged = nullptr;
     size_t tagged_bytes = 0;
     std::vector<unsigned long long> stamps_host;
@@ -997,7 +1168,7 @@ struct PaState {
 
 void pa_destroy(PaState* st) { delete st; }
 
-// A workgroup takes a head's whole context, a wave a block of 64 keys; lanes without a key of their own read the cache's first row, which an empty cache does not have yet.
+// Lanes without a key of their own read the cache's first row, which an empty cache does not have yet.  The last context: what the attention's registers hold.
 bool pa_covers(const PaState* st, int64_t pos) { return st && pos >= 1 && pos < (int64_t)st->max_rows; }
 
 int32_t pa_create(const forge_hip_config& c, const std::vector<PdLayerIn>& layers, const QWeight& lm_head, const float* embed, const float* final_norm,
@@ -1050,7 +1221,6 @@ int32_t pa_create(const forge_hip_config& c, const std::vector<PdLayerIn>& layer
         a.m[i].R = r;
         a.m[i].wg0 = f.wide && i == 1 ? n - (a.m[i].N + r * PA_COMP - 1) / (r * PA_COMP) : 0u;
     }
-    st->max_rows = f.aw * PA_B;
     a.L = (uint32_t)layers.size(); a.H = H; a.I = I; a.QKS = QKS; a.KV = KV; a.heads = c.heads; a.kv_heads = c.kv_heads;
     a.eps = c.rms_eps;
     const uint32_t kmax = std::max(std::max(H, I), QKS);
@@ -1085,10 +1255,24 @@ int32_t pa_create(const forge_hip_config& c, const std::vector<PdLayerIn>& layer
     a.lds_words = a.off_layers / 4;
     a.off_attn = pa_up(a.off_layers + ((uint32_t)layers.size() + 1) * (uint32_t)sizeof(PaLayer), 16);
     st->lds = a.off_attn + f.attn_bytes;
-    if (st->lds > 64000) return FORGE_HIP_OK;
+    if (st->lds > PA_LDS) return FORGE_HIP_OK;
     st->kernel = f.kernel;
+    st->one_rows = st->max_rows = f.aw * PA_B;
+    // Long contexts: as many splits as there are workgroups and room for a head's records in LDS (the group's heads and this position's rows are in PaAttn's place)
+    const uint32_t gsize = c.heads / c.kv_heads, rec_bytes = (hd + 2) * 4;
+    if (f.wide && !exact && gsize * hd + 2 * hd <= 4 * PA_POLL_THREADS && (gsize * hd + hd) * 4 <= f.attn_bytes) {
+        const uint32_t n = std::min(std::min(PA_SPLITS, a.G / c.kv_heads), (PA_LDS - st->lds) / rec_bytes);
+        if (n >= 8) {
+            a.splits = n;
+            a.off_rec = st->lds;
+            st->lds += n * rec_bytes;
+            st->max_rows = std::min(c.max_seq, n * PA_PASSES * (hd <= 64 ? 8u : 4u));
+            st->kernel_long = pa_kernel<PaWide, false, true>(hd, q4, lmq4);
+        }
+    }
     int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, st->kernel, PA_THREADS, st->lds) != hipSuccess || per_cu < 1) { (void)hipGetLastError(); return FORGE_HIP_OK; }
+    for (const void* k : {st->kernel, st->kernel_long})
+        if (k && (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k, PA_THREADS, st->lds) != hipSuccess || per_cu < 1)) { (void)hipGetLastError(); return FORGE_HIP_OK; }
 
     std::vector<PaLayer> host(layers.size() + 1);
     memset(host.data(), 0, host.size() * sizeof(PaLayer));
@@ -1101,7 +1285,7 @@ int32_t pa_create(const forge_hip_config& c, const std::vector<PdLayerIn>& layer
     host.back() = host[0];
     host.back().norm[0] = final_norm;
     PaLayer* dl = st->dev<PaLayer>(host.size() * sizeof(PaLayer));
-    const size_t n_tagged = (size_t)H + QKS + 2 * KV + QKS / 32 * 9 + I / 32 * 9 + 2 * (size_t)st->grid;
+    const size_t n_tagged = (size_t)H + QKS + 2 * KV + QKS / 32 * 9 + I / 32 * 9 + 2 * (size_t)st->grid + (size_t)c.heads * a.splits * (hd + 2);
     uint64_t* t = st->dev<uint64_t>(n_tagged * 8);
     if (!dl || !t) return fail(FORGE_HIP_ERR_HIP, "resident decode: out of device memory");
     FH_HIP(hipMemcpy(dl, host.data(), host.size() * sizeof(PaLayer), hipMemcpyHostToDevice));
@@ -1113,7 +1297,8 @@ int32_t pa_create(const forge_hip_config& c, const std::vector<PdLayerIn>& layer
     a.tkv = t; t += 2 * KV;
     a.taq = t; t += QKS / 32 * 9;
     a.taq2 = t; t += I / 32 * 9;
-    a.tpart = t;
+    a.tpart = t; t += 2 * (size_t)st->grid;
+    a.trec = t;
     a.lm = PaWeights{lm_head.qs, lm_head.scales};
     a.embed = embed; a.cos_t = cos_t; a.sin_t = sin_t;
     a.logits = logits; a.state = state; a.counts = counts; a.penalty = 1.0f;
@@ -1142,8 +1327,8 @@ int32_t pa_create(const forge_hip_config& c, const std::vector<PdLayerIn>& layer
 void pa_set_poll_limit(PaState* st, uint32_t n) { st->args.spin_limit = n ? n : 400000u; }
 void pa_set_repeat_penalty(PaState* st, float penalty) { st->args.penalty = penalty; }
 
-// Enqueues the step at the position in `state` for `token`.  With `profile` the kernel also records the clock at the start of every phase.
-int32_t pa_enqueue(PaState* st, bool profile, uint32_t token, hipStream_t s) {
+// Enqueues the step at position `pos` (which the device has in `state`) for `token`.  With `profile` the kernel also records the clock at the start of every phase.
+int32_t pa_enqueue(PaState* st, int64_t pos, bool profile, uint32_t token, hipStream_t s) {
     PaArgs& a = st->args;
     a.token = token;
     a.step_seq = a.step_seq + 1 ? a.step_seq + 1 : 1;
@@ -1160,7 +1345,7 @@ int32_t pa_enqueue(PaState* st, bool profile, uint32_t token, hipStream_t s) {
     unsigned long long* keep = a.stamps;
     if (!profile) a.stamps = nullptr;
     void* kargs[] = {&a};
-    const hipError_t e = hipLaunchKernel(st->kernel, dim3(st->grid), dim3(PA_THREADS), kargs, st->lds, s);
+    const hipError_t e = hipLaunchKernel(pos < (int64_t)st->one_rows ? st->kernel : st->kernel_long, dim3(st->grid), dim3(PA_THREADS), kargs, st->lds, s);
     a.stamps = keep;
     if (e != hipSuccess) return fail(FORGE_HIP_ERR_HIP, std::string("resident decode launch: ") + hipGetErrorString(e));
     a.tag_base += 6 * a.L + 1;

@@ -60,7 +60,7 @@ struct LlamaModel : forge_hip_model {
     bool prefill_fuse_silu = false;              // fast mode: the gate/up GEMM writes silu(gate) * up quantised (FORGE_HIP_FUSE=0: separate kernel)
     bool fuse_norm = false, fuse_silu = false;   // fused GEMV prologue/epilogue variants fit LDS for this model
     PdState* pd = nullptr;               // the decode step as one resident kernel, when the shape is covered
-    PaState* pa = nullptr;               // the same for a narrow model, whatever the mode, over the short contexts that it covers
+    PaState* pa = nullptr;               // the same for a narrow model, whatever the mode, over the contexts that it covers
     bool step_ahead = false;             // the step enqueued last is pa's
     std::unique_ptr<ResidentSeat> seat;  // of a model that has either
     // ProjectionDTypes (ir.rs:410-421): q, k, v, o, gate, up, down each in its own storage format (GGML ids 8, 2, 12, 14).
@@ -93,7 +93,7 @@ struct LlamaModel : forge_hip_model {
     bool resident() const override { return ahead() || pd; }
     int32_t resident_enqueue(bool profile, uint32_t token) override {
         step_ahead = ahead();
-        return seat->turn(stream, [&] { return step_ahead ? pa_enqueue(pa, profile, token, stream) : pd_enqueue(pd, profile, token, stream); });
+        return seat->turn(stream, [&] { return step_ahead ? pa_enqueue(pa, pos, profile, token, stream) : pd_enqueue(pd, profile, token, stream); });
     }
     bool resident_wait_token(uint32_t* next) override { return step_ahead ? pa_wait_token(pa, next) : pd_wait_token(pd, next); }
     int32_t resident_after_sync(uint32_t abort_flag) override {
@@ -963,7 +963,7 @@ static int32_t model_create_impl(const forge_hip_config* cfg, const uint32_t* pd
                        m->sin_t.as<float>(), m->logits.as<float>(), m->state.as<uint32_t>(), m->counts.as<uint32_t>(),
                        has_bias ? m->biases.as<float>() : nullptr, &m->pd);
         if (rc) return rc;
-        // Narrow models over short contexts (decode_ahead.hip).  Where a variable asks for one of the other kernels' forms, it gets that.
+        // Models of up to 2048 channels over the contexts that it covers (decode_ahead.hip).  Where a variable asks for one of the other kernels' forms, it gets that.
         auto set_to = [](const char* name, char v) { const char* e = getenv(name); return e && (v ? e[0] == v : true); };
         if (!has_bias && !set_to("FORGE_HIP_PD_AHEAD", '0') && !set_to("FORGE_HIP_PD_ORDERED", '1') &&
             !((cfg->flags & FORGE_HIP_FLAG_EXACT) && set_to("FORGE_HIP_PD_EXACT", 0))) {

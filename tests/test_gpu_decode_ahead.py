@@ -1,4 +1,4 @@
-"""The resident decode kernel of short contexts (decode_ahead.hip) against the order-faithful kernel sequence, bit for bit."""
+"""The resident decode kernel of models of up to 2048 channels (decode_ahead.hip): order-faithful against the kernel sequence, bit for bit."""
 import numpy as np
 import pytest
 
@@ -133,6 +133,46 @@ def test_fast_mode_takes_it_too(fh, oracle, torch_gpu, name):
         a, b = fast.forward(int(t)), om.forward(int(t))
     assert np.all(np.isfinite(a)) and np.corrcoef(a, b)[0, 1] > 0.99
     fast.close()
+
+
+# (hidden, inter, heads, kv heads, head dim, the first context that is another kernel's): groups of 4, of 7 (waves with a second head) and of 3 heads, heads
+# that fill their lanes and heads that do not; fewer than 32 splits where LDS ends
+LONG = {"1b": (2048, 8192, 32, 8, 64, 2560), "groups_of_7": (896, 4864, 14, 2, 64, 2560), "hd96": (1536, 4096, 16, 4, 96, 1280), "hd128": (1024, 3072, 12, 4, 128, 1280)}
+
+
+@pytest.mark.parametrize("name", sorted(LONG))
+def test_longer_contexts_of_fast_mode(fh, torch_gpu, monkeypatch, name):
+    """Splits of the context, from the last short one to the first that another kernel takes: the same sums in another order, so outputs agree to rounding (a sum of
+    a few thousand terms: 1e-5) unless a code of an 8-bit vector falls to its neighbour; each of the four vectors carries a rounding of 1/127 of a block's
+    largest value, 0.6% of its norm, twice (both kernels'): under 2% of the output's."""
+    hidden, inter, heads, kv_heads, hd, end = LONG[name]
+    cfg = dict(shape(fh, Q8, hidden, inter, heads, kv_heads, hd, 1000, layers=1, max_seq=2700), flags=0)
+    one, streamed = pair(fh, monkeypatch, cfg, 57)
+    toks = fh.synth.uniform_ids(58, 2700, cfg["vocab"])
+    rel = []
+    for n in (254, 318, 800, end - 3):
+        for m in (one, streamed):
+            m.reset()
+            m.forward_prefill(toks[:n])
+        for t in toks[n:n + 5]:
+            a, b = one.forward(int(t)), streamed.forward(int(t))
+            assert one.decode_launches == 1 and np.all(np.isfinite(a))
+            rel.append(np.linalg.norm(a - b) / np.linalg.norm(b))
+    assert max(rel) < 2e-2 and np.median(rel) < 1e-5, rel
+    # a step that gives up has not happened
+    for m in (one, streamed):
+        m.reset()
+        m.forward_prefill(toks[:400])
+    one.set_poll_limit(1)
+    with pytest.raises(fh.ForgeHipError, match="gave up waiting"):
+        for t in toks[400:410]:
+            one.forward(int(t))
+            streamed.forward(int(t))
+    one.set_poll_limit(0)
+    assert one.pos == streamed.pos
+    a, b = one.forward(int(toks[420])), streamed.forward(int(toks[420]))
+    assert np.linalg.norm(a - b) < 2e-2 * np.linalg.norm(b)
+    one.close(); streamed.close()
 
 
 def test_models_of_several_threads_take_turns(fh, torch_gpu):
