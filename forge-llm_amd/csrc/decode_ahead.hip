@@ -19,7 +19,7 @@
 // have them.  Per token in us, kernel sequence (order-faithful mode) / decode_persistent.hip (fast mode) / this, by rows of context:
 //   SmolLM2-135M Q8_0   33: 781 / 880 / 384    300: 820 / 878 / 421    740: 907 / 876 / 466
 //   1B shape Q8_0       33: 754 / 610 / 466 and 427 (order-faithful, fast)    200: - / 636 / 473 and 439       Q4_0, fast: 33: 532 / 407
-//   and in fast mode (PaPart) 260: 637 / 470    1000: 642 / 475    2400: 644 / 483    Q4_0 2400: 570 / 439
+//   and in fast mode (PaPart) 260: 637 / 470    1000: 642 / 475    2400: 644 / 483    5000: 676 / 514    Q4_0 2400: 570 / 439
 #include <stddef.h>
 #include <string.h>
 
@@ -614,9 +614,8 @@ __device__ __forceinline__ void PaHead<HD, AW>::step(PaKv<HD>& kv, const PaArgs&
 
 // Longer contexts where the order is free, a kernel of their own (beside the short form's registers neither has enough: 957 us a token at 2400 rows of the 1B
 // shape, 483 apart): workgroup (KV head, split) attends to its part of the keys, a fetching wave per query head of the group (and the next four heads behind
-// these); a head's workgroup merges the splits.  A pass is 8 keys (heads of 64; 4 of wider ones), 16 bytes of K and V a lane, and all passes of a split are
-// requested before the workgroup waits for the query: what the registers hold of them is where the form ends.  (With a second round of passes behind the first
-// it is the slower one soon after: 8 layers of the 1B shape at 5000 rows 343 us, decode_persistent.hip 324; at 2540 rows 230 against 309.)
+// these); a head's workgroup merges the splits.  A pass is 8 keys (heads of 64; 4 of wider ones), 16 bytes of K and V a lane; a split's first PA_PASSES are
+// requested before the workgroup waits for the query, further rounds of them when those are done.
 constexpr int PA_PASSES = 10;
 constexpr uint32_t PA_SPLITS = 32, PA_LDS = 64000;
 template <int HD>
@@ -632,13 +631,13 @@ struct PaPart {
         t1 = min(t0 + chunk, seq);
     }
     // rows that are not cached read row 0
-    __device__ __forceinline__ void load(Half8* k, Half8* v, const PaArgs& a, const PaLayer& L, uint32_t pos, uint32_t lane) const {
+    __device__ __forceinline__ void load(Half8* k, Half8* v, const PaArgs& a, const PaLayer& L, uint32_t from, uint32_t pos, uint32_t lane) const {
         const uint16_t* kc = pa_lds_ptr(L.kc) + kvh * HD;
         const uint16_t* vc = pa_lds_ptr(L.vc) + kvh * HD;
         const uint32_t c = min(lane % LPK, (uint32_t)HD / 8 - 1);
 #pragma unroll
         for (int p = 0; p < PA_PASSES; p++) {
-            const uint32_t t = t0 + p * KPW + lane / LPK;
+            const uint32_t t = from + p * KPW + lane / LPK;
             const uint32_t at = ((t < pos ? t : 0u) * a.KV + c * 8) * 2;
             k[p] = pa_at<Half8>(kc, at);
             v[p] = pa_at<Half8>(vc, at);
@@ -658,26 +657,28 @@ struct PaPart {
             float qf[8], acc[8], m = -INFINITY, l = 0.f;
 #pragma unroll
             for (int i = 0; i < 8; i++) { qf[i] = dvalid ? q_s[g * HD + c * 8 + i] : 0.f; acc[i] = 0.f; }
-            if (g >= PA_POLL) load(k, v, a, L, pos, lane);
+            for (uint32_t from = t0; from < t1; from += PA_PASSES * KPW) {
+                if (from != t0 || g >= PA_POLL) load(k, v, a, L, from, pos, lane);
 #pragma unroll
-            for (int p0 = 0; p0 < PA_PASSES; p0 += 2) {
-                const uint32_t tp = t0 + p0 * KPW;
-                if (tp < t1) {
-                    float sc[2];
-                    Half8 vv[2];
+                for (int p0 = 0; p0 < PA_PASSES; p0 += 2) {
+                    const uint32_t tp = from + p0 * KPW;
+                    if (tp < t1) {
+                        float sc[2];
+                        Half8 vv[2];
 #pragma unroll
-                    for (int u = 0; u < 2; u++) {
-                        const uint32_t t = tp + u * KPW + slot;
-                        Half8 kk;
+                        for (int u = 0; u < 2; u++) {
+                            const uint32_t t = tp + u * KPW + slot;
+                            Half8 kk;
 #pragma unroll
-                        for (int i = 0; i < 4; i++) {
-                            kk.w[i] = t == pos ? nk[i] : k[p0 + u].w[i];
-                            vv[u].w[i] = t == pos ? nv[i] : v[p0 + u].w[i];
+                            for (int i = 0; i < 4; i++) {
+                                kk.w[i] = t == pos ? nk[i] : k[p0 + u].w[i];
+                                vv[u].w[i] = t == pos ? nv[i] : v[p0 + u].w[i];
+                            }
+                            const float d = key_dot<LPK>(qf, kk);
+                            sc[u] = t < t1 ? d * scale : -INFINITY;
                         }
-                        const float d = key_dot<LPK>(qf, kk);
-                        sc[u] = t < t1 ? d * scale : -INFINITY;
+                        softmax_block_update<2>(m, l, acc, sc, vv);
                     }
-                    softmax_block_update<2>(m, l, acc, sc, vv);
                 }
             }
             // fold the key slots: every lane of a column ends with the same sums
@@ -857,7 +858,7 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
                 if (stamp) a.stamps[6 * l] = wall_clock64();
                 Half8 pk[LONG ? PA_PASSES : 1], pv[LONG ? PA_PASSES : 1];
                 if constexpr (LONG) {
-                    if (part.on && cx.wave < a.heads / a.kv_heads) part.load(pk, pv, a, L, pos, cx.lane);
+                    if (part.on && cx.wave < a.heads / a.kv_heads) part.load(pk, pv, a, L, part.t0, pos, cx.lane);
                 }
                 if (on_q) {
                     uint16_t* kc = pa_lds_ptr(L.kc);
@@ -1266,7 +1267,11 @@ int32_t pa_create(const forge_hip_config& c, const std::vector<PdLayerIn>& layer
             a.splits = n;
             a.off_rec = st->lds;
             st->lds += n * rec_bytes;
-            st->max_rows = std::min(c.max_seq, n * PA_PASSES * (hd <= 64 ? 8u : 4u));
+            // Rounds.  With a second head a wave, a third round is no longer hidden (us per token, decode_persistent.hip / this: 12/2 heads of 128, 2540 rows 287 / 270,
+            // 3500: 286 / 293; 14/2 of 64, 5000: 241 / 210, 10000: 256 / 261); with few KV heads that kernel has more workgroups for the context.  Otherwise this
+            // one is ahead as far as was measured (8 layers of the 1B shape, 5000: 325 / 245, 20000: 377 / 337; 16/4 heads of 96, 10000: 372 / 299).
+            const uint32_t rounds = gsize <= PA_POLL && c.kv_heads >= 4 ? 8 : 2;
+            st->max_rows = std::min(c.max_seq, n * rounds * PA_PASSES * (hd <= 64 ? 8u : 4u));
             st->kernel_long = pa_kernel<PaWide, false, true>(hd, q4, lmq4);
         }
     }

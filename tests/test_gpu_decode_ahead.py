@@ -135,22 +135,23 @@ def test_fast_mode_takes_it_too(fh, oracle, torch_gpu, name):
     fast.close()
 
 
-# (hidden, inter, heads, kv heads, head dim, the first context that is another kernel's): groups of 4, of 7 (waves with a second head) and of 3 heads, heads
-# that fill their lanes and heads that do not; fewer than 32 splits where LDS ends
-LONG = {"1b": (2048, 8192, 32, 8, 64, 2560), "groups_of_7": (896, 4864, 14, 2, 64, 2560), "hd96": (1536, 4096, 16, 4, 96, 1280), "hd128": (1024, 3072, 12, 4, 128, 1280)}
+# (hidden, inter, heads, kv heads, head dim, contexts whose next steps cross a line): from the short form; from one round of requested keys to two and to three; from
+# two rounds to the other kernel.  Groups of 4, of 7 (waves with a second head) and of 3 heads, heads that fill their lanes and heads that do not
+LONG = {"1b": (2048, 8192, 32, 8, 64, (254, 800, 2557, 5117)), "groups_of_7": (896, 4864, 14, 2, 64, (254, 318, 2557, 5117)),
+        "hd96": (1536, 4096, 16, 4, 96, (254, 800, 1277, 2557)), "hd128": (1024, 3072, 12, 4, 128, (254, 318, 1277, 2557))}
 
 
 @pytest.mark.parametrize("name", sorted(LONG))
 def test_longer_contexts_of_fast_mode(fh, torch_gpu, monkeypatch, name):
-    """Splits of the context, from the last short one to the first that another kernel takes: the same sums in another order, so outputs agree to rounding (a sum of
+    """Splits of the context: the same sums in another order, so outputs agree to rounding (a sum of
     a few thousand terms: 1e-5) unless a code of an 8-bit vector falls to its neighbour; each of the four vectors carries a rounding of 1/127 of a block's
     largest value, 0.6% of its norm, twice (both kernels'): under 2% of the output's."""
-    hidden, inter, heads, kv_heads, hd, end = LONG[name]
-    cfg = dict(shape(fh, Q8, hidden, inter, heads, kv_heads, hd, 1000, layers=1, max_seq=2700), flags=0)
+    hidden, inter, heads, kv_heads, hd, contexts = LONG[name]
+    cfg = dict(shape(fh, Q8, hidden, inter, heads, kv_heads, hd, 1000, layers=1, max_seq=5200), flags=0)
     one, streamed = pair(fh, monkeypatch, cfg, 57)
-    toks = fh.synth.uniform_ids(58, 2700, cfg["vocab"])
+    toks = fh.synth.uniform_ids(58, 5200, cfg["vocab"])
     rel = []
-    for n in (254, 318, 800, end - 3):
+    for n in contexts:
         for m in (one, streamed):
             m.reset()
             m.forward_prefill(toks[:n])
