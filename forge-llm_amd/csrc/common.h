@@ -506,6 +506,7 @@ int32_t pa_create(const forge_hip_config& c, const std::vector<PdLayerIn>& layer
 void pa_destroy(PaState* st);
 bool pa_covers(const PaState* st, int64_t pos);         // a step at this position can run so
 void pa_set_repeat_penalty(PaState* st, float penalty);
+void pa_set_kv_pages(PaState* st, const PageTable& pt, uint32_t max_seq);
 void pa_set_poll_limit(PaState* st, uint32_t n);
 int32_t pa_enqueue(PaState* st, int64_t pos, bool profile, uint32_t token, hipStream_t s);
 bool pa_wait_token(PaState* st, uint32_t* next);

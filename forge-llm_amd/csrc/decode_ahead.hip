@@ -65,6 +65,8 @@ struct PaLayer {
 struct PaArgs {
     PaMat m[5];                               // q;k;v, o, gate;up (N = 2 I; a workgroup holds 32 + 32 rows), down, lm_head
     uint32_t L, H, I, QKS, KV, heads, kv_heads;
+    const uint32_t* pages;                    // paged cache: pool page of each page of the sequence (null: rows lie in order); a page has at least PA_B rows
+    uint32_t page_shift, n_pages;
     uint32_t splits;                          // Wide, order free: parts that a long context is attended in (0: it is not)
     uint32_t G, head0;                        // workgroups [0, G) hold the layers' matrices, [head0, head0 + heads) take a head each; all share the lm_head
     float eps;
@@ -433,16 +435,20 @@ struct PaKv {
         }
     }
 };
+// Where row t of the cache lies.
+__device__ __forceinline__ uint32_t pa_row(const PaArgs& a, uint32_t t) {
+    return a.pages ? (a.pages[t >> a.page_shift] << a.page_shift) + (t & ((1u << a.page_shift) - 1u)) : t;
+}
 // KC rows of V from row bs + k0 on, as they arrive: 16 bits to a register.  (Loads into halves of registers wait for each other in pairs.)
 template <int HD> struct PaRaw { uint32_t v[PaKv<HD>::KC][PaKv<HD>::DPL]; };
 template <int HD>
-__device__ __forceinline__ void pa_load_values(PaRaw<HD>& raw, const uint16_t* vb, uint32_t row0, uint32_t pos, uint32_t kv_stride, uint32_t lane) {
+__device__ __forceinline__ void pa_load_values(PaRaw<HD>& raw, const uint16_t* vb, uint32_t row0, uint32_t pos, uint32_t delta, uint32_t zero, uint32_t kv_stride, uint32_t lane) {
 #pragma unroll
     for (int i = 0; i < PaKv<HD>::KC; i++)
 #pragma unroll
         for (int t = 0; t < PaKv<HD>::DPL; t++) {
-            const uint32_t d = min(lane + 64 * t, (uint32_t)HD - 1), row = row0 + i;      // rows past the last cached one: row 0
-            raw.v[i][t] = pa_at<uint16_t>(vb + (row < pos ? row : 0u) * kv_stride, d * 2);
+            const uint32_t d = min(lane + 64 * t, (uint32_t)HD - 1), row = row0 + i;      // rows past the last cached one: the first
+            raw.v[i][t] = pa_at<uint16_t>(vb + (row < pos ? row + delta : zero) * kv_stride, d * 2);
         }
     __builtin_amdgcn_sched_barrier(0);                // all requested before the first is waited for
 }
@@ -460,6 +466,7 @@ __device__ __forceinline__ void pa_pack_values(PaKv<HD>& kv, const PaRaw<HD>& ra
 template <int HD, uint32_t AW>
 struct PaHead {
     uint32_t h, kvh, b, nb, bs, bl, nk;           // the wave's block b: bl keys, nk of them cached
+    uint32_t delta, zero;                         // from a row of the block to where it lies; where the first row lies
     bool has_new;                                 // this position is the last key of the last block
     __device__ __forceinline__ PaHead(const PaArgs& a, uint32_t head, uint32_t pos, uint32_t wave) {
         h = head; kvh = head / (a.heads / a.kv_heads);
@@ -468,16 +475,18 @@ struct PaHead {
         bl = b < AW && bs < seq ? min(PA_B, seq - bs) : 0u;
         has_new = b < AW && bs <= pos && pos < bs + PA_B;
         nk = has_new ? bl - 1 : bl;
+        delta = pa_sgpr(bl ? pa_row(a, bs) - bs : 0u);
+        zero = pa_sgpr(pa_row(a, 0));
     }
     __device__ __forceinline__ void load(PaKv<HD>& kv, const PaArgs& a, const PaLayer& L, uint32_t pos, uint32_t lane) const {
         if (!bl) return;
         const uint16_t* kb = pa_lds_ptr(L.kc) + kvh * HD;
-        const uint32_t row = bs + lane, at = (row < pos ? row : 0u) * a.KV * 2;      // lanes without a cached key: row 0
+        const uint32_t row = bs + lane, at = (row < pos ? row + delta : zero) * a.KV * 2;      // lanes without a cached key: the first row
         uint4 kr[HD / 8];
 #pragma unroll
         for (int c = 0; c < HD / 8; c++) kr[c] = pa_at<uint4>(kb, at + c * 16);
         PaRaw<HD> raw;
-        pa_load_values<HD>(raw, pa_lds_ptr(L.vc) + kvh * HD, bs, pos, a.KV, lane);
+        pa_load_values<HD>(raw, pa_lds_ptr(L.vc) + kvh * HD, bs, pos, delta, zero, a.KV, lane);
         pa_pack_values<HD>(kv, raw);
         kv.set_keys(kr);
     }
@@ -558,7 +567,7 @@ __device__ __forceinline__ void PaHead<HD, AW>::step(PaKv<HD>& kv, const PaArgs&
 #pragma nounroll
             for (uint32_t k0 = 0; k0 < PA_B; k0 += KC) {
                 if (k0 && k0 >= nk) break;
-                if (k0) { PaRaw<HD> raw; pa_load_values<HD>(raw, vb, bs + k0, pos, kv_stride, lane); pa_pack_values<HD>(kv, raw); }
+                if (k0) { PaRaw<HD> raw; pa_load_values<HD>(raw, vb, bs + k0, pos, delta, zero, kv_stride, lane); pa_pack_values<HD>(kv, raw); }
                 // keys past the last one are left out, not given a weight of 0: 0 * v is not 0 for an infinite v
 #pragma unroll
                 for (int i16 = 0; i16 < KC; i16 += 16) {
@@ -617,11 +626,12 @@ __device__ __forceinline__ void PaHead<HD, AW>::step(PaKv<HD>& kv, const PaArgs&
 // these); a head's workgroup merges the splits.  A pass is 8 keys (heads of 64; 4 of wider ones), 16 bytes of K and V a lane; a split's first PA_PASSES are
 // requested before the workgroup waits for the query, further rounds of them when those are done.
 constexpr int PA_PASSES = 10;
-constexpr uint32_t PA_SPLITS = 32, PA_LDS = 64000;
+constexpr uint32_t PA_SPLITS = 32, PA_LDS = 64000, PA_ROUNDS = 8;
+constexpr uint32_t PA_PAGES = PA_ROUNDS * PA_PASSES * 8 / PA_B + 2;       // pages that a split's rows lie in
 template <int HD>
 struct PaPart {
     static constexpr int LPK = HD <= 64 ? 8 : 16, KPW = 64 / LPK, REC = HD + 2;
-    uint32_t kvh, split, t0, t1;              // keys [t0, t1)
+    uint32_t kvh, split, t0, t1, zero;        // keys [t0, t1); where the first row lies
     bool on;
     __device__ __forceinline__ PaPart(const PaArgs& a, uint32_t wg, uint32_t pos) {
         kvh = wg % a.kv_heads; split = wg / a.kv_heads;
@@ -629,22 +639,25 @@ struct PaPart {
         on = split < a.splits;
         t0 = min(split * chunk, seq);
         t1 = min(t0 + chunk, seq);
+        zero = pa_sgpr(pa_row(a, 0));
     }
-    // rows that are not cached read row 0
-    __device__ __forceinline__ void load(Half8* k, Half8* v, const PaArgs& a, const PaLayer& L, uint32_t from, uint32_t pos, uint32_t lane) const {
+    // pages: the pool pages from t0's on, in LDS; rows that are not cached or another split's: the first row
+    __device__ __forceinline__ void load(Half8* k, Half8* v, const PaArgs& a, const PaLayer& L, uint32_t from, const uint32_t* pages, uint32_t pos, uint32_t lane) const {
         const uint16_t* kc = pa_lds_ptr(L.kc) + kvh * HD;
         const uint16_t* vc = pa_lds_ptr(L.vc) + kvh * HD;
         const uint32_t c = min(lane % LPK, (uint32_t)HD / 8 - 1);
 #pragma unroll
         for (int p = 0; p < PA_PASSES; p++) {
             const uint32_t t = from + p * KPW + lane / LPK;
-            const uint32_t at = ((t < pos ? t : 0u) * a.KV + c * 8) * 2;
+            uint32_t row = t;
+            if (a.pages) row = (pages[min((t >> a.page_shift) - (t0 >> a.page_shift), PA_PAGES - 1)] << a.page_shift) + (t & ((1u << a.page_shift) - 1u));
+            const uint32_t at = ((t < min(t1, pos) ? row : zero) * a.KV + c * 8) * 2;
             k[p] = pa_at<Half8>(kc, at);
             v[p] = pa_at<Half8>(vc, at);
         }
     }
     // q_s: the group's heads in LDS, new_s: this position's K row and V row, fp16 pairs.  After the barrier that publishes them.
-    __device__ __forceinline__ void attend(Half8* k, Half8* v, const PaArgs& a, const PaLayer& L, const float* q_s, const Half8* new_s, uint32_t pos, uint32_t tag_out,
+    __device__ __forceinline__ void attend(Half8* k, Half8* v, const PaArgs& a, const PaLayer& L, const float* q_s, const Half8* new_s, const uint32_t* pages, uint32_t pos, uint32_t tag_out,
                                            const PaCtx& cx) const {
         const uint32_t gsize = a.heads / a.kv_heads, lane = cx.lane, slot = lane / LPK, c = lane % LPK;
         const bool dvalid = c * 8 < (uint32_t)HD;
@@ -658,7 +671,7 @@ struct PaPart {
 #pragma unroll
             for (int i = 0; i < 8; i++) { qf[i] = dvalid ? q_s[g * HD + c * 8 + i] : 0.f; acc[i] = 0.f; }
             for (uint32_t from = t0; from < t1; from += PA_PASSES * KPW) {
-                if (from != t0 || g >= PA_POLL) load(k, v, a, L, from, pos, lane);
+                if (from != t0 || g >= PA_POLL) load(k, v, a, L, from, pages, pos, lane);
 #pragma unroll
                 for (int p0 = 0; p0 < PA_PASSES; p0 += 2) {
                     const uint32_t tp = from + p0 * KPW;
@@ -759,6 +772,7 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
     __shared__ uint32_t sh_abort;
     __shared__ ArgPair sh_arg[PA_WAVES];
     __shared__ float norm_part[PA_POLL];
+    __shared__ uint32_t sh_pages[LONG ? PA_PAGES : 1];
     __shared__ uint64_t exp_tab[32];          // expf_ref's table
     uint32_t* aq = reinterpret_cast<uint32_t*>(smem);
     float* as = reinterpret_cast<float*>(smem + a.off_as);
@@ -786,6 +800,9 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
         reinterpret_cast<uint32_t*>(smem + a.off_layers)[i] = ldg(reinterpret_cast<const uint32_t*>(a.layers) + i);
     const uint32_t pos = pa_sgpr(a.state[0]);
     const float* emb = a.embed + (size_t)a.token * a.H;
+    if constexpr (LONG) {
+        if (a.pages && cx.tid < PA_PAGES) sh_pages[cx.tid] = ldg(a.pages + min((PaPart<HD>(a, cx.wg, pos).t0 >> a.page_shift) + cx.tid, a.n_pages - 1));
+    }
     __syncthreads();
 
     const uint32_t ntid = cx.tid - PA_POLL_THREADS;                               // of a computing thread
@@ -819,6 +836,7 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
         __syncthreads();
         return true;
     };
+    const uint32_t pos_row = pa_sgpr(pa_row(a, pos));
     const uint32_t head = cx.wg - a.head0;
     const bool on_a = head < a.heads;         // unsigned
 
@@ -858,7 +876,7 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
                 if (stamp) a.stamps[6 * l] = wall_clock64();
                 Half8 pk[LONG ? PA_PASSES : 1], pv[LONG ? PA_PASSES : 1];
                 if constexpr (LONG) {
-                    if (part.on && cx.wave < a.heads / a.kv_heads) part.load(pk, pv, a, L, part.t0, pos, cx.lane);
+                    if (part.on && cx.wave < a.heads / a.kv_heads) part.load(pk, pv, a, L, part.t0, sh_pages, pos, cx.lane);
                 }
                 if (on_q) {
                     uint16_t* kc = pa_lds_ptr(L.kc);
@@ -875,7 +893,7 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
                         const uint32_t at = qrow - a.QKS;                        // of [K row | V row]
                         if (mine_q) {
                             stc64(is_q ? a.tq + qrow : a.tkv + at, base + 1, is_q ? __float_as_uint(o) : (uint32_t)hb);
-                            if (!is_q) stg((is_k ? kc + at : vc + (at - a.KV)) + (size_t)pos * a.KV, hb);
+                            if (!is_q) stg((is_k ? kc + at : vc + (at - a.KV)) + (size_t)pos_row * a.KV, hb);
                         }
                     }
                 }
@@ -900,7 +918,7 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
                         }
                         __syncthreads();
                         if (sh_abort) return;
-                        part.attend(pk, pv, a, L, q_s, new_s, pos, base + 2, cx);
+                        part.attend(pk, pv, a, L, q_s, new_s, sh_pages, pos, base + 2, cx);
                     } else if (!glance(a.tkv + 2 * a.KV - 1, base + 1)) {
                         return;
                     }
@@ -1178,7 +1196,7 @@ int32_t pa_create(const forge_hip_config& c, const std::vector<PdLayerIn>& layer
     const uint32_t H = c.hidden, I = c.inter, hd = c.head_dim, QKS = c.heads * hd, KV = c.kv_heads * hd;
     if (c.sliding_window != 0 || layers.empty() || !layers[0].qkv || lm_head.kquant()) return FORGE_HIP_OK;
     if (hd != 64 && hd != 96 && hd != 128) return FORGE_HIP_OK;
-    if (H < 64 || I < 64 || QKS < 64) return FORGE_HIP_OK;
+    if (H < 64 || I < 64 || QKS < 64 || (uint64_t)c.max_seq * KV * 2 > 0xFFFFFFFFull) return FORGE_HIP_OK;      // a row's place: 32 bits
     const bool q4 = c.wdtype == FORGE_HIP_Q4_0, lmq4 = c.lm_head_dtype == FORGE_HIP_Q4_0;
     const bool exact = (c.flags & FORGE_HIP_FLAG_EXACT) != 0;
     const PaForm f = H <= PaNarrow::NX * PA_POLL_THREADS ? pa_form<PaNarrow, true>(hd, q4, lmq4) : exact ? pa_form<PaWide, true>(hd, q4, lmq4) : pa_form<PaWide, false>(hd, q4, lmq4);
@@ -1270,7 +1288,7 @@ int32_t pa_create(const forge_hip_config& c, const std::vector<PdLayerIn>& layer
             // Rounds.  With a second head a wave, a third round is no longer hidden (us per token, decode_persistent.hip / this: 12/2 heads of 128, 2540 rows 287 / 270,
             // 3500: 286 / 293; 14/2 of 64, 5000: 241 / 210, 10000: 256 / 261); with few KV heads that kernel has more workgroups for the context.  Otherwise this
             // one is ahead as far as was measured (8 layers of the 1B shape, 5000: 325 / 245, 20000: 377 / 337; 16/4 heads of 96, 10000: 372 / 299).
-            const uint32_t rounds = gsize <= PA_POLL && c.kv_heads >= 4 ? 8 : 2;
+            const uint32_t rounds = gsize <= PA_POLL && c.kv_heads >= 4 ? PA_ROUNDS : 2;
             st->max_rows = std::min(c.max_seq, n * rounds * PA_PASSES * (hd <= 64 ? 8u : 4u));
             st->kernel_long = pa_kernel<PaWide, false, true>(hd, q4, lmq4);
         }
@@ -1330,6 +1348,11 @@ int32_t pa_create(const forge_hip_config& c, const std::vector<PdLayerIn>& layer
 }
 
 void pa_set_poll_limit(PaState* st, uint32_t n) { st->args.spin_limit = n ? n : 400000u; }
+void pa_set_kv_pages(PaState* st, const PageTable& pt, uint32_t max_seq) {
+    st->args.pages = pt.table;
+    st->args.page_shift = pt.shift;
+    st->args.n_pages = pt.table ? max_seq >> pt.shift : 0u;
+}
 void pa_set_repeat_penalty(PaState* st, float penalty) { st->args.penalty = penalty; }
 
 // Enqueues the step at position `pos` (which the device has in `state`) for `token`.  With `profile` the kernel also records the clock at the start of every phase.

@@ -89,7 +89,7 @@ struct LlamaModel : forge_hip_model {
     void enqueue_row_logits(uint32_t row) override;
     bool keeps_rows() const override { return !mixed || mixed_batched; }
     int32_t decode_launches() const override;
-    bool ahead() const { return pa && !pt.table && pa_covers(pa, pos); }
+    bool ahead() const { return pa && pa_covers(pa, pos); }
     bool resident() const override { return ahead() || pd; }
     int32_t resident_enqueue(bool profile, uint32_t token) override {
         step_ahead = ahead();
@@ -605,6 +605,7 @@ int32_t LlamaModel::set_kv_pages(uint32_t page_rows, const uint32_t* page_table_
         const int32_t rc = pd_set_kv_pages(pd, npt, cfg.max_seq);
         if (rc) return rc;
     }
+    if (pa) pa_set_kv_pages(pa, npt, cfg.max_seq);
     pt = npt;
     page_table_host_copy.swap(table);
     return FORGE_HIP_OK;

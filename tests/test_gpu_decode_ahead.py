@@ -147,7 +147,7 @@ def test_longer_contexts_of_fast_mode(fh, torch_gpu, monkeypatch, name):
     a few thousand terms: 1e-5) unless a code of an 8-bit vector falls to its neighbour; each of the four vectors carries a rounding of 1/127 of a block's
     largest value, 0.6% of its norm, twice (both kernels'): under 2% of the output's."""
     hidden, inter, heads, kv_heads, hd, contexts = LONG[name]
-    cfg = dict(shape(fh, Q8, hidden, inter, heads, kv_heads, hd, 1000, layers=1, max_seq=5200), flags=0)
+    cfg = dict(shape(fh, Q8, hidden, inter, heads, kv_heads, hd, 1000, layers=1, max_seq=5248), flags=0)
     one, streamed = pair(fh, monkeypatch, cfg, 57)
     toks = fh.synth.uniform_ids(58, 5200, cfg["vocab"])
     rel = []
@@ -160,6 +160,16 @@ def test_longer_contexts_of_fast_mode(fh, torch_gpu, monkeypatch, name):
             assert one.decode_launches == 1 and np.all(np.isfinite(a))
             rel.append(np.linalg.norm(a - b) / np.linalg.norm(b))
     assert max(rel) < 2e-2 and np.median(rel) < 1e-5, rel
+    # the same rows in pages all over the pool: the same bits
+    paged = fh.HipModel(cfg, fh.synth.make_weights_blob(cfg, seed=57, threads=16))
+    paged.set_kv_pages(64, np.random.default_rng(59).permutation(cfg["max_seq"] // 64).astype(np.uint32))
+    for n in (200, contexts[-1]):
+        for m in (one, paged):
+            m.reset()
+            m.forward_prefill(toks[:n])
+        for t in toks[n:n + 3]:
+            same_bits(paged.forward(int(t)), one.forward(int(t)))
+    paged.close()
     # a step that gives up has not happened
     for m in (one, streamed):
         m.reset()
