@@ -6,7 +6,7 @@ decode steps at that context, and prints ONE JSON line.  Weights, KV cache and a
 resident in HBM when the timed regions start.
 
 roofline: the decode step's dominant kernel.  By default the whole step is ONE resident kernel
-(decode_step_kernel): `achieved` = algorithmic bytes of one token (GGUF block bytes of every matrix + the
+(decode_ahead_kernel; decode_step_kernel above 2048 channels): `achieved` = algorithmic bytes of one token (GGUF block bytes of every matrix + the
 f32 input and output vectors of each GEMV + the fp16 K/V rows attention reads) / the kernel's duration,
 measured live by the library's forward_profile from the kernel's own clock stamps (one per phase, summed).
 With FORGE_HIP_PERSIST=0 the step is a sequence of kernels and the figure is that of the quantised GEMV
@@ -47,7 +47,7 @@ DIVERGENCE_STEPS = 128         # greedy steps over which the fast mode's tokens 
 # WRITE_SIZE counters of two profiler runs of this script, each scaled by what the same counter reads for the 1 GiB
 # copy of --calibrate-copy (FETCH_SIZE x2.000, WRITE_SIZE x1.000).  Summary: profiles/gemv_hbm_traffic_pmc.md.
 GEMV_HBM_BYTES_PER_LAUNCH = 20.46e6 + 0.02e6      # fetched + written
-# The same for one launch of the resident decode kernel (the whole step) at this context: 1 436.9 MB fetched + 13.8 MB
+# The same for one launch of decode_step_kernel (the whole step; not counted again for decode_ahead_kernel, which reads the same planes once) at this context: 1 436.9 MB fetched + 13.8 MB
 # written.  Summary: profiles/decode_step_kernel_hbm_traffic_pmc.md.
 STEP_KERNEL_HBM_BYTES_PER_LAUNCH = 1450.7e6
 
@@ -137,7 +137,7 @@ def decode_profile(fh, model, cfg, tok, context, prof_steps=8):
         total = gemv_bytes_total + kv_bytes
         kernel_ms = sum(stage_ms.values())
         achieved = total / (kernel_ms * 1e-3) / 1e9
-        roof = {"kernel": "decode_step_kernel (the whole decode step: every quantised GEMV, decode attention, norms, argmax)",
+        roof = {"kernel": "the resident decode kernel (decode_ahead_kernel or decode_step_kernel; the whole decode step: every quantised GEMV, decode attention, norms, argmax)",
                 "bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS,
                 "traffic": STEP_KERNEL_HBM_BYTES_PER_LAUNCH, "bytes_per_launch": total / n_launch, "us_per_launch": kernel_ms * 1e3 / n_launch,
                 "launches_per_step": n_launch, "weights_and_vectors_bytes": gemv_bytes_total, "kv_cache_bytes": kv_bytes,
