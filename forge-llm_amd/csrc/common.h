@@ -491,7 +491,7 @@ int32_t pd_set_repeat_penalty(PdState* st, float penalty);
 void pd_set_poll_limit(PdState* st, uint32_t n);
 int32_t pd_set_kv_pages(PdState* st, PageTable pt, uint32_t max_seq);
 void pd_destroy(PdState* st);
-int32_t pd_enqueue(PdState* st, bool profile, uint32_t token, hipStream_t s);
+int32_t pd_enqueue(PdState* st, bool profile, uint32_t token, uint32_t step_seq, hipStream_t s);
 // Spins on the host word the kernel writes last; false = not available, wait for the stream instead.
 bool pd_wait_token(PdState* st, uint32_t* next);
 // Call with the abort flag read back after the stream drained; resets the exchange buffers and fails if it is set.
@@ -508,7 +508,7 @@ bool pa_covers(const PaState* st, int64_t pos);         // a step at this positi
 void pa_set_repeat_penalty(PaState* st, float penalty);
 void pa_set_kv_pages(PaState* st, const PageTable& pt, uint32_t max_seq);
 void pa_set_poll_limit(PaState* st, uint32_t n);
-int32_t pa_enqueue(PaState* st, int64_t pos, bool profile, uint32_t token, hipStream_t s);
+int32_t pa_enqueue(PaState* st, int64_t pos, bool profile, uint32_t token, uint32_t step_seq, hipStream_t s);
 bool pa_wait_token(PaState* st, uint32_t* next);
 int32_t pa_after_sync(PaState* st, uint32_t abort_flag, hipStream_t s);
 int32_t pa_phase_ms(PaState* st, std::vector<float>* out, hipStream_t s);

@@ -1355,11 +1355,11 @@ void pa_set_kv_pages(PaState* st, const PageTable& pt, uint32_t max_seq) {
 }
 void pa_set_repeat_penalty(PaState* st, float penalty) { st->args.penalty = penalty; }
 
-// Enqueues the step at position `pos` (which the device has in `state`) for `token`.  With `profile` the kernel also records the clock at the start of every phase.
-int32_t pa_enqueue(PaState* st, int64_t pos, bool profile, uint32_t token, hipStream_t s) {
+// Enqueues the step at position `pos` (which the device has in `state`) for `token`; `step_seq`: its number, not 0.  With `profile` the kernel also records the clock at the start of every phase.
+int32_t pa_enqueue(PaState* st, int64_t pos, bool profile, uint32_t token, uint32_t step_seq, hipStream_t s) {
     PaArgs& a = st->args;
     a.token = token;
-    a.step_seq = a.step_seq + 1 ? a.step_seq + 1 : 1;
+    a.step_seq = step_seq;
     a.host_out = st->host_out_dev;
     if (a.host_out) a.host_seq = ++st->seq;
     if (a.tag_base > 0xF0000000u) {      // tags are about to wrap: start again from zeroed buffers

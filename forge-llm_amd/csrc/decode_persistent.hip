@@ -1921,13 +1921,13 @@ int32_t pd_set_repeat_penalty(PdState* st, float penalty) {
     return FORGE_HIP_OK;
 }
 
-// Enqueue one decode step at the position in `state` for `token` (travels as a kernel argument).  With `profile`
-// the kernel also records the wall clock at the start of every phase.
-int32_t pd_enqueue(PdState* st, bool profile, uint32_t token, hipStream_t s) {
+// Enqueue one decode step at the position in `state` for `token` (travels as a kernel argument); `step_seq`: its number, not 0.
+// With `profile` the kernel also records the wall clock at the start of every phase.
+int32_t pd_enqueue(PdState* st, bool profile, uint32_t token, uint32_t step_seq, hipStream_t s) {
     PdArgs& a = st->args;
     a.token = token;
     a.token_from_arg = 1;
-    a.step_seq = a.step_seq + 1 ? a.step_seq + 1 : 1;
+    a.step_seq = step_seq;
     a.host_out = st->host_out_dev;
     if (a.host_out) a.host_seq = ++st->seq;
     if (a.tag_base > 0xF0000000u) {      // tags are about to wrap: start again from zeroed buffers

@@ -62,6 +62,7 @@ struct LlamaModel : forge_hip_model {
     PdState* pd = nullptr;               // the decode step as one resident kernel, when the shape is covered
     PaState* pa = nullptr;               // the same for a narrow model, whatever the mode, over the contexts that it covers
     bool step_ahead = false;             // the step enqueued last is pa's
+    uint32_t step_seq = 0;               // its number.  One count for both kernels: they mark a counted token in the same word of the device's state
     std::unique_ptr<ResidentSeat> seat;  // of a model that has either
     // ProjectionDTypes (ir.rs:410-421): q, k, v, o, gate, up, down each in its own storage format (GGML ids 8, 2, 12, 14).
     // `mixed`: they are not all cfg.wdtype, or the lm_head is a K-quant: every projection is then a GEMV launch of its own
@@ -93,7 +94,8 @@ struct LlamaModel : forge_hip_model {
     bool resident() const override { return ahead() || pd; }
     int32_t resident_enqueue(bool profile, uint32_t token) override {
         step_ahead = ahead();
-        return seat->turn(stream, [&] { return step_ahead ? pa_enqueue(pa, pos, profile, token, stream) : pd_enqueue(pd, profile, token, stream); });
+        step_seq = step_seq + 1 ? step_seq + 1 : 1;
+        return seat->turn(stream, [&] { return step_ahead ? pa_enqueue(pa, pos, profile, token, step_seq, stream) : pd_enqueue(pd, profile, token, step_seq, stream); });
     }
     bool resident_wait_token(uint32_t* next) override { return step_ahead ? pa_wait_token(pa, next) : pd_wait_token(pd, next); }
     int32_t resident_after_sync(uint32_t abort_flag) override {

@@ -118,6 +118,43 @@ def test_rewinds_its_tags_and_gives_up_instead_of_hanging(fh, torch_gpu, monkeyp
     one.close(); seq.close()
 
 
+@pytest.mark.parametrize("hidden", [256, 800])
+def test_a_failed_step_keeps_the_count_that_the_other_kernel_made(fh, torch_gpu, monkeypatch, hidden):
+    """Fast mode, a penalty: the token at position 0 is counted by decode_step_kernel's step, the one at position 1 is the first of decode_ahead_kernel, which gives up.
+    The first count stays: without it the token, whose row of the output matrix is 64 times the others, would be the next one."""
+    cfg = dict(shape(fh, Q8, hidden, 512, 4, 2, 64, 1000), flags=0)
+    blob = fh.synth.make_weights_blob(cfg, seed=67)
+    often, row = 7, hidden // 32 * 34
+    blocks = blob[len(blob) - 1000 * row:][often * row:(often + 1) * row].reshape(-1, 34)
+    blocks[:, :2] = (np.ascontiguousarray(blocks[:, :2]).view(np.float16) * np.float16(64)).view(np.uint8)
+    one = fh.HipModel(cfg, blob)
+    assert one.decode_launches == 1
+
+    def after(x):
+        one.reset()
+        one.forward_greedy(often)
+        return one.forward_greedy(x)
+
+    x = next(x for x in range(500, 600) if after(x) == often)
+    one.set_repeat_penalty(1000.0)
+    want = after(x)
+    assert want != often
+    for _ in range(8):                                       # a step may get through if every hand-over is on time
+        one.reset()
+        one.forward_greedy(often)
+        one.set_poll_limit(1)
+        try:
+            one.forward_greedy(often)
+        except fh.ForgeHipError as e:
+            assert "gave up waiting" in str(e) and one.pos == 1
+            break
+        finally:
+            one.set_poll_limit(0)
+    assert one.pos == 1, "no step gave up with a poll limit of 1"
+    assert one.forward_greedy(x) == want
+    one.close()
+
+
 @pytest.mark.parametrize("name", ["narrow_form", "wide_1b", "wide_least", "wide_hd128"])
 def test_fast_mode_takes_it_too(fh, oracle, torch_gpu, name):
     """Fast mode, token by token: the narrow form is the order-faithful one, the wide form adds up in another order.  Rounding moves single codes of the
