@@ -12,7 +12,7 @@ LIB = os.path.join(HERE, "libforge_hip.so")
 
 SOURCES = ["format.hip", "elementwise.hip", "gemv.hip", "gemv_f32.hip", "gemv_kquant.hip", "kquant_prefill.hip", "gemm.hip", "gemm_rows.hip", "attn_decode.hip", "attn_prefill.hip",
            "attn_exact.hip", "decode_persistent.hip", "decode_ahead.hip", "api.hip", "model.hip", "llama.hip", "block_model.hip", "block_mixers.hip", "dense.hip",
-           "attn_prompt.hip", "attn_latent.hip", "attn_grouped.hip", "linear_attn.hip", "checkpoint.cpp", "gguf.cpp", "sampling.cpp"]
+           "attn_prompt.hip", "attn_latent.hip", "attn_grouped.hip", "linear_attn.hip", "checkpoint.cpp", "gguf.cpp", "sampling.cpp", "resident_seat.cpp"]
 
 # The trace replay program holds the dense networks only.
 TRACE_RUN = os.path.join(BUILD, "trace_run")

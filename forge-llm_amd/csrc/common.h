@@ -513,29 +513,4 @@ bool pa_wait_token(PaState* st, uint32_t* next);
 int32_t pa_after_sync(PaState* st, uint32_t abort_flag, hipStream_t s);
 int32_t pa_phase_ms(PaState* st, std::vector<float>* out, hipStream_t s);
 
-// The workgroups of a resident kernel wait for each other, so all of them have to be on the device at once.  One such kernel takes every compute unit; were two launched
-// side by side (models of two threads), each could get a part and wait for the rest until its polls run out.  A model that launches one holds a seat: while there are
-// several seats in the process, a launch on another stream than the one before it waits for that one to end.  With a single seat nothing is recorded.
-class ResidentSeat {
-public:
-    ResidentSeat();
-    ~ResidentSeat();
-    ResidentSeat(const ResidentSeat&) = delete;
-    ResidentSeat& operator=(const ResidentSeat&) = delete;
-    // launch(): enqueues on s
-    template <typename F>
-    int32_t turn(hipStream_t s, F launch) {
-        const Lock lock;
-        int32_t rc = before(s);
-        if (!rc) rc = launch();
-        return rc ? rc : after(s);
-    }
-
-private:
-    struct Lock { Lock(); ~Lock(); };
-    static int32_t before(hipStream_t s);
-    static int32_t after(hipStream_t s);
-};
-
-
 }  // namespace fh

@@ -15,6 +15,7 @@
 #include <vector>
 
 #include "model.h"
+#include "resident_seat.h"
 
 namespace fh {
 

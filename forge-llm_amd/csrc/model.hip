@@ -8,46 +8,7 @@
 
 #include <string.h>
 
-#include <mutex>
-
 using namespace fh;
-
-namespace fh {
-
-namespace {
-std::mutex seat_mutex;
-uint32_t seats = 0;
-hipEvent_t seat_event = nullptr;          // behind the launch before; null until there was a second seat
-hipStream_t seat_stream = nullptr;
-}  // namespace
-
-ResidentSeat::Lock::Lock() { seat_mutex.lock(); }
-ResidentSeat::Lock::~Lock() { seat_mutex.unlock(); }
-ResidentSeat::ResidentSeat() {
-    const Lock lock;
-    // launches made while there was one seat left no event: they end here
-    if (++seats == 2) (void)hipDeviceSynchronize();
-}
-ResidentSeat::~ResidentSeat() {
-    const Lock lock;
-    if (--seats > 0) return;
-    if (seat_event) (void)hipEventDestroy(seat_event);
-    seat_event = nullptr;
-    seat_stream = nullptr;
-}
-int32_t ResidentSeat::before(hipStream_t s) {
-    if (seats > 1 && seat_event && seat_stream != s) FH_HIP(hipStreamWaitEvent(s, seat_event, 0));
-    return FORGE_HIP_OK;
-}
-int32_t ResidentSeat::after(hipStream_t s) {
-    if (seats < 2) return FORGE_HIP_OK;
-    if (!seat_event) FH_HIP(hipEventCreateWithFlags(&seat_event, hipEventDisableTiming));
-    seat_stream = s;
-    FH_HIP(hipEventRecord(seat_event, s));
-    return FORGE_HIP_OK;
-}
-
-}  // namespace fh
 
 void forge_hip_model::drop_decode_graphs() {
     for (hipGraphExec_t& g : decode_graph) {

@@ -1,0 +1,81 @@
+// The turns of resident kernels over a stand-in for the runtime: what is called is printed, and an event is recorded on, and waited for by, streams as HIP has it
+// (recording: only on a stream of the event's own device).  Argument: the scenario.
+#include <hip/hip_runtime_api.h>
+#include <stdio.h>
+#include <string.h>
+
+#include <memory>
+#include <string>
+#include <vector>
+
+#include "forge_hip.h"
+#include "resident_seat.h"
+
+namespace {
+struct Stream { int device; const char* name; };
+struct Event { int device; };
+int current = 0;
+bool record_fails = false, wait_fails = false;
+hipStream_t handle(Stream& s) { return reinterpret_cast<hipStream_t>(&s); }
+const char* name(hipStream_t s) { return reinterpret_cast<Stream*>(s)->name; }
+}  // namespace
+
+extern "C" {
+hipError_t hipGetDevice(int* d) { *d = current; return hipSuccess; }
+hipError_t hipDeviceSynchronize() { printf("sync device %d\n", current); return hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { *e = reinterpret_cast<hipEvent_t>(new Event{current}); return hipSuccess; }
+hipError_t hipEventDestroy(hipEvent_t e) { delete reinterpret_cast<Event*>(e); return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
+    if (record_fails) return hipErrorOutOfMemory;
+    if (reinterpret_cast<Event*>(e)->device != reinterpret_cast<Stream*>(s)->device) return hipErrorInvalidHandle;
+    printf("record %s\n", name(s));
+    return hipSuccess;
+}
+hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t, unsigned) {
+    if (wait_fails) return hipErrorUnknown;
+    printf("wait %s\n", name(s));
+    return hipSuccess;
+}
+hipError_t hipStreamSynchronize(hipStream_t s) { printf("sync %s\n", name(s)); return hipSuccess; }
+hipError_t hipGetLastError() { return hipSuccess; }
+const char* hipGetErrorString(hipError_t) { return "error"; }
+}
+
+namespace fh {
+int32_t fail(int32_t code, const std::string&) { return code; }
+}  // namespace fh
+
+int main(int argc, char** argv) {
+    const std::string what = argc > 1 ? argv[1] : "";
+    Stream a{0, "a"}, b{0, "b"};
+    auto step = [](fh::ResidentSeat& seat, Stream& s) {
+        const int32_t rc = seat.turn(handle(s), [&] { printf("launch %s\n", s.name); return (int32_t)FORGE_HIP_OK; });
+        printf("-> %d\n", rc);
+    };
+    if (what == "one") {
+        fh::ResidentSeat seat;
+        step(seat, a);
+        step(seat, a);
+    } else if (what == "two") {
+        fh::ResidentSeat one, other;
+        step(one, a);
+        step(one, a);
+        step(other, b);
+        step(one, a);
+    } else if (what == "record fails") {
+        fh::ResidentSeat one, other;
+        record_fails = true;
+        step(one, a);
+        record_fails = false;
+        step(other, b);
+        step(one, a);
+    } else if (what == "wait fails") {
+        fh::ResidentSeat one, other;
+        step(one, a);
+        wait_fails = true;
+        step(other, b);
+    } else {
+        return 2;
+    }
+    return 0;
+}
