@@ -1,5 +1,6 @@
 #include "resident_seat.h"
 
+#include <map>
 #include <mutex>
 #include <string>
 
@@ -9,41 +10,51 @@ namespace fh {
 
 int32_t fail(int32_t code, const std::string& msg);       // common.h, which a host compiler does not take
 
-namespace {
-std::mutex seat_mutex;
-uint32_t seats = 0;
-hipEvent_t seat_event = nullptr;          // behind the launch before; null until there was a second seat
-hipStream_t seat_stream = nullptr;        // that launch's, or null if it has ended
-}  // namespace
+struct ResidentSeat::Device {
+    std::mutex mutex;
+    uint32_t seats = 0;
+    hipEvent_t event = nullptr;               // behind the launch before; null until there was a second seat
+    hipStream_t stream = nullptr;             // that launch's, or null if it has ended
+};
 
-ResidentSeat::Lock::Lock() { seat_mutex.lock(); }
-ResidentSeat::Lock::~Lock() { seat_mutex.unlock(); }
+ResidentSeat::Lock::Lock(Device* device) : d(device) { d->mutex.lock(); }
+ResidentSeat::Lock::~Lock() { d->mutex.unlock(); }
 ResidentSeat::ResidentSeat() {
-    const Lock lock;
-    // launches made while there was one seat left no event: they end here
-    if (++seats == 2) (void)hipDeviceSynchronize();
+    // never destroyed: a model may outlive the statics of its process
+    static std::mutex* mutex = new std::mutex;
+    static auto* devices = new std::map<int, Device>;
+    int id = 0;
+    (void)hipGetDevice(&id);
+    {
+        const std::lock_guard<std::mutex> one(*mutex);
+        dev = &(*devices)[id];
+    }
+    const Lock lock(dev);
+    if (++dev->seats != 2) return;
+    // launches made while there was one seat left no event: they end here.  An event belongs to the device that is current when it is made.
+    (void)hipDeviceSynchronize();
+    if (!dev->event && hipEventCreateWithFlags(&dev->event, hipEventDisableTiming) != hipSuccess) { dev->event = nullptr; (void)hipGetLastError(); }
 }
 ResidentSeat::~ResidentSeat() {
-    const Lock lock;
-    if (--seats > 0) return;
-    if (seat_event) (void)hipEventDestroy(seat_event);
-    seat_event = nullptr;
-    seat_stream = nullptr;
+    const Lock lock(dev);
+    if (--dev->seats > 0) return;
+    if (dev->event) (void)hipEventDestroy(dev->event);
+    dev->event = nullptr;
+    dev->stream = nullptr;
 }
 int32_t ResidentSeat::before(hipStream_t s) {
-    if (seats < 2 || !seat_stream || seat_stream == s) return FORGE_HIP_OK;
-    const hipError_t e = hipStreamWaitEvent(s, seat_event, 0);
+    if (dev->seats < 2 || !dev->stream || dev->stream == s) return FORGE_HIP_OK;
+    const hipError_t e = hipStreamWaitEvent(s, dev->event, 0);
     return e == hipSuccess ? FORGE_HIP_OK : fail(FORGE_HIP_ERR_HIP, std::string("resident decode: the wait for another model's step: ") + hipGetErrorString(e));
 }
 // The step is on its way, whatever happens here: where nothing can be left for the next launch to wait for, this one is waited for at once.
 void ResidentSeat::after(hipStream_t s) {
-    if (seats < 2) return;
-    seat_stream = s;
-    if (!seat_event && hipEventCreateWithFlags(&seat_event, hipEventDisableTiming) != hipSuccess) seat_event = nullptr;
-    if (seat_event && hipEventRecord(seat_event, s) == hipSuccess) return;
+    if (dev->seats < 2) return;
+    dev->stream = s;
+    if (dev->event && hipEventRecord(dev->event, s) == hipSuccess) return;
     (void)hipGetLastError();
     (void)hipStreamSynchronize(s);
-    seat_stream = nullptr;
+    dev->stream = nullptr;
 }
 
 }  // namespace fh

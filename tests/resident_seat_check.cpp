@@ -2,11 +2,8 @@
 // (recording: only on a stream of the event's own device).  Argument: the scenario.
 #include <hip/hip_runtime_api.h>
 #include <stdio.h>
-#include <string.h>
 
-#include <memory>
 #include <string>
-#include <vector>
 
 #include "forge_hip.h"
 #include "resident_seat.h"
@@ -62,6 +59,22 @@ int main(int argc, char** argv) {
         step(one, a);
         step(other, b);
         step(one, a);
+    } else if (what == "devices") {
+        // a model on each of two devices, then a second one on the second; steps come while the first device is current
+        Stream c{1, "c"}, d{1, "d"};
+        fh::ResidentSeat one;
+        current = 1;
+        fh::ResidentSeat other;
+        current = 0;
+        step(one, a);
+        step(other, c);
+        step(one, a);
+        current = 1;
+        fh::ResidentSeat third;
+        current = 0;
+        step(other, c);
+        step(one, a);
+        step(third, d);
     } else if (what == "record fails") {
         fh::ResidentSeat one, other;
         record_fails = true;

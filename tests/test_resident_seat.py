@@ -38,6 +38,11 @@ def test_launches_on_two_streams_follow_one_another(seats):
     assert seats("two") == ["sync device 0", "launch a", "record a", OK, "launch a", "record a", OK, "wait b", "launch b", "record b", OK, "wait a", "launch a", "record a", OK]
 
 
+def test_devices_do_not_wait_for_one_another(seats):
+    """An event belongs to a device and is recorded on that device's streams only."""
+    assert seats("devices") == ["launch a", OK, "launch c", OK, "launch a", OK, "sync device 1", "launch c", "record c", OK, "launch a", OK, "wait d", "launch d", "record d", OK]
+
+
 def test_a_step_that_was_launched_is_not_reported_as_failed(seats):
     """The device advances position and counts: an error behind the launch would let the caller feed the token again."""
     assert seats("record fails") == ["sync device 0", "launch a", "sync a", OK, "launch b", "record b", OK, "wait a", "launch a", "record a", OK]
