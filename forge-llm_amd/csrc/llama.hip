@@ -65,6 +65,9 @@ struct LlamaModel : forge_hip_model {
     bool step_ahead = false;             // the step enqueued last is pa's
     uint32_t step_seq = 0;               // its number.  One count for both kernels: they mark a counted token in the same word of the device's state
     std::unique_ptr<ResidentSeat> seat;  // of a model that has either
+    // Where there is no pd, the kernel sequence, which asks nothing of the rest of the GPU, takes the steps that pa does not: also from the step on that pa could
+    // not end because another process held compute units.  A caller that has set a poll limit gets that step's error instead.
+    bool pa_left = false, polls_set = false;
     // ProjectionDTypes (ir.rs:410-421): q, k, v, o, gate, up, down each in its own storage format (GGML ids 8, 2, 12, 14).
     // `mixed`: they are not all cfg.wdtype, or the lm_head is a K-quant: every projection is then a GEMV launch of its own
     // and a prompt is walked token by token, as the reference does for such models (emit.rs:4530-4534, 4621-5040).
@@ -91,7 +94,7 @@ struct LlamaModel : forge_hip_model {
     void enqueue_row_logits(uint32_t row) override;
     bool keeps_rows() const override { return !mixed || mixed_batched; }
     int32_t decode_launches() const override;
-    bool ahead() const { return pa && pa_covers(pa, pos); }
+    bool ahead() const { return pa && !pa_left && pa_covers(pa, pos); }
     bool resident() const override { return ahead() || pd; }
     int32_t resident_enqueue(bool profile, uint32_t token) override {
         step_ahead = ahead();
@@ -100,7 +103,9 @@ struct LlamaModel : forge_hip_model {
     }
     bool resident_wait_token(uint32_t* next) override { return step_ahead ? pa_wait_token(pa, next) : pd_wait_token(pd, next); }
     int32_t resident_after_sync(uint32_t abort_flag) override {
-        return step_ahead ? pa_after_sync(pa, abort_flag, stream) : pd_after_sync(pd, abort_flag, stream);
+        if (!step_ahead) return pd_after_sync(pd, abort_flag, stream);
+        pa_left = abort_flag && !pd && !polls_set;
+        return pa_after_sync(pa, abort_flag, stream);
     }
     int32_t resident_profile(float* stage_ms, uint32_t* stage_launches) override;
     int32_t repeat_penalty_changed(float penalty) override {
@@ -109,6 +114,8 @@ struct LlamaModel : forge_hip_model {
         return rc;
     }
     void poll_limit_changed(uint32_t polls) override {
+        polls_set = polls != 0;
+        pa_left = false;
         if (pd) pd_set_poll_limit(pd, polls);
         if (pa) pa_set_poll_limit(pa, polls);
     }

@@ -166,6 +166,9 @@ int32_t finish_or_undo(forge_hip_model* m) {
     return rc;
 }
 
+// Whether the step that failed with rc was a resident kernel's and the model takes it as the kernel sequence from now on.
+bool left_resident(const forge_hip_model* m, int32_t rc) { return rc && m->step_resident && !m->resident(); }
+
 // A prompt of n tokens in chunks; logits of the rows want[0..n_want) into logits_host [n_want][vocab].
 int32_t prefill_rows(forge_hip_model* m, const uint32_t* tokens, uint64_t n, const uint64_t* want, uint64_t n_want, float* logits_host) {
     FH_CHECK(m && tokens, "prefill_batch: null pointer");
@@ -234,8 +237,15 @@ int32_t forge_hip_forward(forge_hip_model* m, uint32_t token, float* logits_host
     FH_CHECK(logits_host, "forward: null logits");
     int32_t rc = forward_common(m, token);
     if (rc) return rc;
-    FH_HIP(hipMemcpyAsync(m->h_logits, m->logits.p, (size_t)m->cfg.vocab * 4, hipMemcpyDeviceToHost, m->stream));
-    rc = finish_or_undo(m);
+    auto finish = [&]() -> int32_t {
+        FH_HIP(hipMemcpyAsync(m->h_logits, m->logits.p, (size_t)m->cfg.vocab * 4, hipMemcpyDeviceToHost, m->stream));
+        return finish_or_undo(m);
+    };
+    rc = finish();
+    if (left_resident(m, rc)) {
+        rc = forward_common(m, token);
+        if (!rc) rc = finish();
+    }
     if (rc) return rc;
     memcpy(logits_host, m->h_logits, (size_t)m->cfg.vocab * 4);
     return FORGE_HIP_OK;
@@ -248,6 +258,10 @@ int32_t forge_hip_forward_greedy(forge_hip_model* m, uint32_t token, uint32_t* n
     // the resident kernel hands the token over through host memory as soon as it is final
     if (m->step_resident && m->resident_wait_token(next_token_host)) return FORGE_HIP_OK;
     rc = finish_or_undo(m);
+    if (left_resident(m, rc)) {
+        rc = forward_common(m, token);
+        if (!rc) rc = finish_or_undo(m);
+    }
     if (rc) return rc;
     *next_token_host = m->h_stage[4];
     return FORGE_HIP_OK;
@@ -293,9 +307,11 @@ int32_t forge_hip_forward_profile(forge_hip_model* m, uint32_t token, float* sta
         int32_t rc = m->resident_enqueue(true, token);
         if (rc) return rc;
         rc = finish_decode_step(m);
-        if (rc) return rc;
-        m->pos += 1;
-        return m->resident_profile(stage_ms, stage_launches);
+        if (!rc) {
+            m->pos += 1;
+            return m->resident_profile(stage_ms, stage_launches);
+        }
+        if (!left_resident(m, rc)) return rc;
     }
     m->h_stage[0] = token;
     FH_HIP(hipMemcpyAsync(m->d_token(), &m->h_stage[0], 4, hipMemcpyHostToDevice, m->stream));

@@ -185,7 +185,8 @@ class HipModel:
 
     def set_poll_limit(self, polls: int) -> None:
         """Polls a workgroup of the resident decode kernel spends on one hand-over before the step gives up (0: default).
-        A step that gives up raises ForgeHipError(ERR_HIP) and leaves position, token counts and context as they were."""
+        A step that gives up raises ForgeHipError(ERR_HIP) and leaves position, token counts and context as they were; under the default
+        limit an order-faithful model of Q8_0 / Q4_0 matrices runs it, and those behind it, as the kernel sequence instead."""
         self._check(self._lib.forge_hip_model_set_poll_limit(self._h, int(polls)))
 
     def set_repeat_penalty(self, penalty: float) -> None:

@@ -47,7 +47,8 @@
  *    stream of this process holds compute units for long enough, the kernel's bounded wait expires,
  *    the call returns FORGE_HIP_ERR_HIP with the model's position and repeat counts unchanged, and the
  *    caller may repeat it or set FORGE_HIP_PERSIST=0 before model_create to use the kernel sequence,
- *    which has no such requirement.
+ *    which has no such requirement.  An order-faithful model of Q8_0 / Q4_0 matrices needs neither: it takes that step
+ *    and those behind it as the kernel sequence by itself (see forge_hip_model_set_poll_limit).
  */
 #ifndef FORGE_HIP_H
 #define FORGE_HIP_H
@@ -201,7 +202,9 @@ int64_t forge_hip_model_pos(const forge_hip_model* m);
  * (0: the default, 400000 polls, far beyond any wait of a healthy step).  A step that gives up returns
  * FORGE_HIP_ERR_HIP from forge_hip_forward / forge_hip_forward_greedy and has not happened: the position, the token
  * counts of the repeat penalty and the context in the cache are what they were before the call, and the same token can
- * be fed again.  No counterpart in the reference (its CPU loop has nothing to wait for); a no-op for a model that runs
+ * be fed again.  Where the kernel sequence is a model's other way of taking a step (order-faithful models of Q8_0 / Q4_0
+ * matrices, unless FORGE_HIP_PD_EXACT is set), a step that gives up under the default limit is run again that way within the call, and so are
+ * all steps until this function is called again; under a limit set here (polls > 0) it returns the error.  No counterpart in the reference (its CPU loop has nothing to wait for); a no-op for a model that runs
  * the kernel sequence. */
 int32_t forge_hip_model_set_poll_limit(forge_hip_model* m, uint32_t polls);
 /* A PAGED KV cache for the model: the cache memory of every layer is taken as a pool of n_pages = max_seq / page_rows pages

@@ -119,6 +119,44 @@ def test_rewinds_its_tags_and_gives_up_instead_of_hanging(fh, torch_gpu, monkeyp
 
 
 @pytest.mark.parametrize("hidden", [256, 800])
+def test_order_faithful_steps_that_give_up_run_as_the_sequence(fh, torch_gpu, monkeypatch, hidden):
+    """Other users of the GPU do not make a step of the order-faithful mode fail: what gives up is the kernel sequence's, with its bits, until a poll limit is set."""
+    cfg = shape(fh, Q8, hidden, 512, 4, 2, 64, 1000)
+    monkeypatch.setenv("FORGE_HIP_PD_SPIN_LIMIT", "1")
+    left = []
+    toks = [int(t) for t in fh.synth.uniform_ids(78, 40, cfg["vocab"])]
+    for first in ("greedy", "logits", "profile"):
+        one, seq = pair(fh, monkeypatch, cfg, 77)
+        for m in (one, seq):
+            m.set_repeat_penalty(1.2)
+            m.forward_prefill(toks[:6])
+        assert one.decode_launches == 1
+        at = 6
+        for t in toks[6:12]:                                 # a step may get through if every hand-over is on time
+            if first == "greedy":
+                assert one.forward_greedy(t) == seq.forward_greedy(t)
+            elif first == "logits":
+                same_bits(one.forward(t), seq.forward(t))
+            else:
+                a, b = one.forward_profile(t), seq.forward_profile(t)
+                if one.decode_launches > 1:
+                    assert [n for _, n in a.values()] == [n for _, n in b.values()]
+            at += 1
+            if one.decode_launches > 1:
+                break
+        left.append(one.decode_launches)
+        for t in toks[at:at + 6]:
+            assert one.forward_greedy(t) == seq.forward_greedy(t) and one.pos == seq.pos
+        one.set_poll_limit(0)
+        assert one.decode_launches == 1
+        for t in toks[at + 6:at + 10]:
+            same_bits(one.forward(t), seq.forward(t))
+        assert one.decode_launches == 1
+        one.close(); seq.close()
+    assert min(left) > 1, "no step gave up with a poll limit of 1"
+
+
+@pytest.mark.parametrize("hidden", [256, 800])
 def test_a_failed_step_keeps_the_count_that_the_other_kernel_made(fh, torch_gpu, monkeypatch, hidden):
     """Fast mode, a penalty: the token at position 0 is counted by decode_step_kernel's step, the one at position 1 is the first of decode_ahead_kernel, which gives up.
     The first count stays: without it the token, whose row of the output matrix is 64 times the others, would be the next one."""
