@@ -34,6 +34,7 @@
 #include "expf_ref.h"
 #include "gemv_order.h"
 #include "resident.h"
+#include "resident_seat.h"
 
 namespace fh {
 
@@ -1165,6 +1166,7 @@ struct PaState {
     const void* kernel = nullptr;
     const void* kernel_long = nullptr;
     uint32_t grid = 0, lds = 0, n_stamps = 0, max_rows = 0, one_rows = 0;
+    bool cooperative = false;
     uint64_t* tagged = nullptr;
     size_t tagged_bytes = 0;
     std::vector<unsigned long long> stamps_host;
@@ -1204,12 +1206,15 @@ int32_t pa_create(const forge_hip_config& c, const std::vector<PdLayerIn>& layer
     if (H > f.nx * PA_POLL_THREADS || I / 32 * 9 > f.nv * PA_POLL_THREADS || QKS / 32 * 9 > f.nv * PA_POLL_THREADS) return FORGE_HIP_OK;
     // rows that the reference adds in its four-accumulator order (the last len % 4 of a chunk) are left to the other kernels
     if (H % 4 || I % 4 || QKS % 4 || KV % 4 || c.vocab % 4) return FORGE_HIP_OK;
-    int dev = 0, cus = 0, khz = 0;
+    int dev = 0, coop = 0, cus = 0, khz = 0;
     FH_HIP(hipGetDevice(&dev));
+    FH_HIP(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev));
     FH_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
     FH_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev));
 
     std::unique_ptr<PaState> st(new PaState());
+    st->cooperative = resident_cooperative();
+    if (st->cooperative && !coop) return FORGE_HIP_OK;
     PaArgs& a = st->args;
     const uint32_t nq[5] = {QKS + 2 * KV, H, 2 * I, H, c.vocab}, kk[5] = {H, QKS, H, I, H};
     for (int i = 0; i < 5; i++) {
@@ -1373,7 +1378,7 @@ int32_t pa_enqueue(PaState* st, int64_t pos, bool profile, uint32_t token, uint3
     unsigned long long* keep = a.stamps;
     if (!profile) a.stamps = nullptr;
     void* kargs[] = {&a};
-    const hipError_t e = hipLaunchKernel(pos < (int64_t)st->one_rows ? st->kernel : st->kernel_long, dim3(st->grid), dim3(PA_THREADS), kargs, st->lds, s);
+    const hipError_t e = resident_launch(pos < (int64_t)st->one_rows ? st->kernel : st->kernel_long, st->grid, PA_THREADS, kargs, st->lds, st->cooperative, s);
     a.stamps = keep;
     if (e != hipSuccess) return fail(FORGE_HIP_ERR_HIP, std::string("resident decode launch: ") + hipGetErrorString(e));
     a.tag_base += 6 * a.L + 1;

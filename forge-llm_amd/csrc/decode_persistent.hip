@@ -51,6 +51,7 @@
 #include "expf_ref.h"
 #include "gemv_order.h"
 #include "resident.h"
+#include "resident_seat.h"
 
 namespace fh {
 
@@ -1604,8 +1605,7 @@ const void* pd_kernel(const PdState* st) {
 template <int HD>
 hipError_t launch_pd_hd(const PdState* st, hipStream_t s) {
     void* kargs[] = {const_cast<PdArgs*>(&st->args)};
-    if (!st->cooperative) return hipLaunchKernel(pd_kernel<HD>(st), dim3(st->grid), dim3(PD_THREADS), kargs, st->lds, s);
-    return hipLaunchCooperativeKernel(pd_kernel<HD>(st), dim3(st->grid), dim3(PD_THREADS), kargs, st->lds, s);
+    return resident_launch(pd_kernel<HD>(st), st->grid, PD_THREADS, kargs, st->lds, st->cooperative, s);
 }
 
 const void* pd_kernel_for(const PdState* st) {
@@ -1860,10 +1860,7 @@ int32_t pd_create(const forge_hip_config& c, const std::vector<PdLayerIn>& layer
     // give-up path: every wait in the kernel is bounded by it, so the kernel still ends normally)
     { const char* e = getenv("FORGE_HIP_PD_SPIN_LIMIT"); if (e && atoi(e) > 0) a.spin_limit = (uint32_t)atoi(e); }
     a.token = 0; a.token_from_arg = 0; a.host_out = nullptr; a.host_seq = 0;
-    // All workgroups are co-resident by construction (one per CU, checked above), and every wait in the kernel is
-    // bounded, so an ordinary launch is enough; it costs ~7 us less per step than a cooperative one.
-    // FORGE_HIP_PD_COOP=1 asks for the cooperative launch (which re-checks residency on every launch).
-    { const char* e = getenv("FORGE_HIP_PD_COOP"); st->cooperative = e && e[0] == '1'; }
+    st->cooperative = resident_cooperative();
     if (!(getenv("FORGE_HIP_PD_HOSTWORD") && getenv("FORGE_HIP_PD_HOSTWORD")[0] == '0')) {
         void* hp = nullptr;
         if (hipHostMalloc(&hp, 64, hipHostMallocMapped) == hipSuccess) {

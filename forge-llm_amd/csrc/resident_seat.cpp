@@ -1,5 +1,7 @@
 #include "resident_seat.h"
 
+#include <stdlib.h>
+
 #include <map>
 #include <mutex>
 #include <string>
@@ -9,6 +11,14 @@
 namespace fh {
 
 int32_t fail(int32_t code, const std::string& msg);       // common.h, which a host compiler does not take
+
+bool resident_cooperative() {
+    const char* e = getenv("FORGE_HIP_PD_COOP");
+    return e && e[0] == '1';
+}
+hipError_t resident_launch(const void* kernel, uint32_t grid, uint32_t threads, void** args, uint32_t lds, bool cooperative, hipStream_t s) {
+    return cooperative ? hipLaunchCooperativeKernel(kernel, dim3(grid), dim3(threads), args, lds, s) : hipLaunchKernel(kernel, dim3(grid), dim3(threads), args, lds, s);
+}
 
 struct ResidentSeat::Device {
     std::mutex mutex;

@@ -1,10 +1,15 @@
-// Whose turn it is to launch a resident kernel.
+// How a resident kernel is launched, and whose turn it is.
 #pragma once
 
 #include <hip/hip_runtime_api.h>
 #include <stdint.h>
 
 namespace fh {
+
+// All workgroups are co-resident by construction (one per compute unit, checked when the model is created) and every wait in the kernel is bounded, so an ordinary launch
+// is enough; it costs ~7 us less per step than a cooperative one, which checks again.  FORGE_HIP_PD_COOP=1 asks for that one.
+bool resident_cooperative();
+hipError_t resident_launch(const void* kernel, uint32_t grid, uint32_t threads, void** args, uint32_t lds, bool cooperative, hipStream_t s);
 
 // The workgroups of a resident kernel wait for each other, so all of them have to be on the device at once.  One such kernel takes every compute unit; were two launched
 // side by side (models of two threads), each could get a part and wait for the rest until its polls run out.  A model that launches one holds a seat of its device: while

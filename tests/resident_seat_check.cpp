@@ -1,4 +1,4 @@
-// The turns of resident kernels over a stand-in for the runtime: what is called is printed, and an event is recorded on, and waited for by, streams as HIP has it
+// Launches and turns of resident kernels over a stand-in for the runtime: what is called is printed, and an event is recorded on, and waited for by, streams as HIP has it
 // (recording: only on a stream of the event's own device).  Argument: the scenario.
 #include <hip/hip_runtime_api.h>
 #include <stdio.h>
@@ -34,6 +34,14 @@ hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t, unsigned) {
     return hipSuccess;
 }
 hipError_t hipStreamSynchronize(hipStream_t s) { printf("sync %s\n", name(s)); return hipSuccess; }
+hipError_t hipLaunchKernel(const void*, dim3 grid, dim3 block, void**, size_t lds, hipStream_t s) {
+    printf("ordinary %s %u %u %zu\n", name(s), grid.x, block.x, lds);
+    return hipSuccess;
+}
+hipError_t hipLaunchCooperativeKernel(const void*, dim3 grid, dim3 block, void**, unsigned lds, hipStream_t s) {
+    printf("cooperative %s %u %u %u\n", name(s), grid.x, block.x, lds);
+    return hipSuccess;
+}
 hipError_t hipGetLastError() { return hipSuccess; }
 const char* hipGetErrorString(hipError_t) { return "error"; }
 }
@@ -49,7 +57,9 @@ int main(int argc, char** argv) {
         const int32_t rc = seat.turn(handle(s), [&] { printf("launch %s\n", s.name); return (int32_t)FORGE_HIP_OK; });
         printf("-> %d\n", rc);
     };
-    if (what == "one") {
+    if (what == "launch") {
+        (void)fh::resident_launch(nullptr, 256, 768, nullptr, 1000, fh::resident_cooperative(), handle(a));
+    } else if (what == "one") {
         fh::ResidentSeat seat;
         step(seat, a);
         step(seat, a);

@@ -118,6 +118,21 @@ def test_rewinds_its_tags_and_gives_up_instead_of_hanging(fh, torch_gpu, monkeyp
     one.close(); seq.close()
 
 
+@pytest.mark.parametrize("hidden,flags,prompt", [(256, EXACT, 30), (800, EXACT, 30), (800, 0, 300)])
+def test_cooperative_launches(fh, torch_gpu, monkeypatch, hidden, flags, prompt):
+    """FORGE_HIP_PD_COOP=1: the same tokens from launches that check residency."""
+    cfg = dict(shape(fh, Q8, hidden, 512, 4, 4, 64, 1000), flags=flags)
+    blob = fh.synth.make_weights_blob(cfg, seed=87)
+    toks = fh.synth.uniform_ids(88, prompt, cfg["vocab"])
+    plain = fh.HipModel(cfg, blob)
+    monkeypatch.setenv("FORGE_HIP_PD_COOP", "1")
+    coop = fh.HipModel(cfg, blob)
+    assert coop.generate_greedy(toks, 12) == plain.generate_greedy(toks, 12)
+    assert coop.decode_launches == plain.decode_launches == 1
+    same_bits(coop.forward(3), plain.forward(3))
+    coop.close(); plain.close()
+
+
 @pytest.mark.parametrize("hidden", [256, 800])
 def test_order_faithful_steps_that_give_up_run_as_the_sequence(fh, torch_gpu, monkeypatch, hidden):
     """Other users of the GPU do not make a step of the order-faithful mode fail: what gives up is the kernel sequence's, with its bits, until a poll limit is set."""

@@ -1,4 +1,4 @@
-"""ResidentSeat (csrc/resident_seat.h) over a stand-in for the HIP runtime: which calls the launches of several models' resident kernels are surrounded by."""
+"""csrc/resident_seat.h over a stand-in for the HIP runtime: how a resident kernel is launched, and which calls the launches of several models are surrounded by."""
 import os
 import shutil
 import subprocess
@@ -20,14 +20,27 @@ def seats(tmp_path_factory):
                         os.path.join(ROOT, "tests", "resident_seat_check.cpp"), os.path.join(csrc, "resident_seat.cpp"), "-o", exe], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stderr
 
-    def run(scenario):
-        out = subprocess.run([exe, scenario], capture_output=True, text=True, timeout=60)
+    def run(scenario, **env):
+        out = subprocess.run([exe, scenario], capture_output=True, text=True, timeout=60, env=dict(os.environ, **env))
         assert out.returncode == 0, out
         return out.stdout.split("\n")[:-1]
     return run
 
 
 OK, HIP_ERROR = "-> 0", "-> -5"
+
+
+@pytest.mark.parametrize("value,want", [("0", "ordinary"), ("1", "cooperative")])
+def test_the_variable_asks_for_cooperative_launches(seats, value, want):
+    assert seats("launch", FORGE_HIP_PD_COOP=value) == [f"{want} a 256 768 1000"]
+
+
+def test_no_kernel_is_launched_past_it():
+    """Both resident kernels go through resident_launch."""
+    for name in ("decode_ahead.hip", "decode_persistent.hip"):
+        with open(os.path.join(ROOT, "forge-llm_amd", "csrc", name)) as f:
+            text = f.read()
+        assert "resident_launch(" in text and "hipLaunchKernel(" not in text and "hipLaunchCooperativeKernel(" not in text, name
 
 
 def test_a_model_alone_pays_for_nothing(seats):
