@@ -91,7 +91,7 @@ struct PaArgs {
     uint32_t tag_base, spin_limit, token, step_seq;
     unsigned long long* host_out;             // host-mapped {launch number, next token}: written last, or null
     uint32_t host_seq;
-    unsigned long long* stamps;               // optional: wall clock at the start of every phase (workgroup 0)
+    unsigned long long* stamps;               // optional: wall clock between the phases, each from a workgroup that has done the phase before
     uint32_t off_as, off_xs, off_out, off_silu, off_prod, off_layers, off_attn, off_rec, prod_words, lds_words, xstride;      // LDS byte offsets (activation codes at 0)
 };
 
@@ -807,7 +807,13 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
     __syncthreads();
 
     const uint32_t ntid = cx.tid - PA_POLL_THREADS;                               // of a computing thread
-    const bool stamp = a.stamps && cx.wg == 0 && cx.tid == 0;
+    // A phase ends, and the next one begins, where the first workgroup with a part of it has handed that on: a wait for the others' parts is the next phase's.
+    auto stamp = [&](uint32_t wg, uint32_t slot, uint32_t slots = 1) {
+        if (a.stamps && cx.wg == wg && cx.tid == 0) {
+            const unsigned long long t = wall_clock64();
+            for (uint32_t i = 0; i < slots; i++) a.stamps[slot + i] = t;
+        }
+    };
     PaSet<F::UL, LMQ4> wl[2];
     float4 n1;                                // norm weights of elements 4 ntid ..
     const PaMat ml = a.m[4];
@@ -874,7 +880,7 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
                 const PaLayer& L = layers[l];
                 const uint32_t base = a.tag_base + 6 * l, x_in = l ? base : 0u;
                 // ---- norm | q;k;v | rotation, cache row
-                if (stamp) a.stamps[6 * l] = wall_clock64();
+                stamp(0, 6 * l);
                 Half8 pk[LONG ? PA_PASSES : 1], pv[LONG ? PA_PASSES : 1];
                 if constexpr (LONG) {
                     if (part.on && cx.wave < a.heads / a.kv_heads) part.load(pk, pv, a, L, part.t0, sh_pages, pos, cx.lane);
@@ -899,7 +905,7 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
                     }
                 }
                 // ---- attention
-                if (stamp) a.stamps[6 * l + 1] = wall_clock64();
+                stamp(0, 6 * l + 1);
                 if constexpr (LONG) {
                     if (part.on) {
                         // the group's heads, this position's K row and V row
@@ -920,12 +926,14 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
                         __syncthreads();
                         if (sh_abort) return;
                         part.attend(pk, pv, a, L, q_s, new_s, sh_pages, pos, base + 2, cx);
+                        stamp(0, 6 * l + 2);
                     } else if (!glance(a.tkv + 2 * a.KV - 1, base + 1)) {
                         return;
                     }
                     if (on_a) {
                         pa_merge<HD>(a, head, base + 2, base + 3, reinterpret_cast<float*>(smem + a.off_rec), silu, cx);
                         if (sh_abort) return;
+                        stamp(a.head0, 6 * l + 3);
                     } else if (!on_o && !glance(a.taq + a.QKS / 32 * 9 - 1, base + 3)) {
                         return;
                     }
@@ -934,6 +942,7 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
                         PaKv<HD> kv;
                         ph.load(kv, a, L, pos, cx.lane);
                         ph.step(kv, a, L, attn, exp_tab, pos, base + 1, cx);
+                        stamp(a.head0, 6 * l + 2, 2);                            // no merge phase
                     } else {
                         if (!glance(a.tkv + 2 * a.KV - 1, base + 1)) return;
                     }
@@ -941,7 +950,6 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
                     if (!on_o && !on_a && !glance(a.taq + a.QKS / 32 * 9 - 1, base + 2)) return;
                 }
                 // ---- o + residual
-                if (stamp) { const unsigned long long t = wall_clock64(); a.stamps[6 * l + 2] = t; a.stamps[6 * l + 3] = t; }
                 if (on_o) {
                     const bool mine = cx.wave == 0 && cx.lane < PA_COMP * mo.R && row_o + cx.lane < mo.N;
                     const float r = pa_fetch_aq<F::NV>(a.taq, base + (LONG ? 3 : 2), a.QKS, aq, as, mine, row_o + cx.lane, a.tx, x_in, emb, cx);
@@ -951,7 +959,7 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
                     if (mine) stc64(a.tx + row_o + cx.lane, base + 4, __float_as_uint(r + out[cx.lane]));     // residual_add, emit.rs:455-459
                 }
                 // ---- norm | gate;up | silu(gate) * up
-                if (stamp) a.stamps[6 * l + 4] = wall_clock64();
+                stamp(mo.wg0, 6 * l + 4);
                 if (on_g) {
                     pa_fetch_x<F::NX, ORD>(a.tx, base + 4, emb, a.H, xs, a.xstride, norm_part, cx);
                     if (!norm_fetching()) return;
@@ -959,7 +967,7 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
                     if (cx.wave == 0) pa_store_block(silu[cx.lane & 31u], a.taq2 + cx.wg * 9, base + 5, cx.lane, cx.lane < 32);
                 }
                 // ---- down + residual
-                if (stamp) a.stamps[6 * l + 5] = wall_clock64();
+                stamp(0, 6 * l + 5);
                 if (on_d) {
                     const bool mine = cx.wave == 0 && cx.lane < PA_COMP * md.R && row_d + cx.lane < md.N;
                     const float r = pa_fetch_aq<F::NV>(a.taq2, base + 5, a.I, aq, as, mine, row_d + cx.lane, a.tx, base + 4, emb, cx);
@@ -1061,6 +1069,7 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
                     ph.load(kv, a, layers[l], pos, cx.lane);                     // requested as soon as the layer before is done
                     ph.step(kv, a, layers[l], attn, exp_tab, pos, a.tag_base + 6 * l + 1, cx);
                     if (sh_abort) return;
+                    stamp(a.head0, 6 * l + 2, 2);
                 }
             }
         }
@@ -1077,7 +1086,7 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
 
     // ---- final norm | lm_head | argmax
     asm volatile("" : "+v"(cx.tid), "+v"(cx.lane));
-    if (stamp) a.stamps[6 * a.L] = wall_clock64();
+    stamp(0, 6 * a.L);
     ArgPair best{-INFINITY, 0};
     if (!comp) {
         pa_fetch_x<F::NX, ORD>(a.tx, a.tag_base + 6 * a.L, emb, a.H, xs, a.xstride, norm_part, cx);
@@ -1118,7 +1127,7 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
         stc64(a.tpart + 2 * cx.wg, th, __float_as_uint(best.v));
         stc64(a.tpart + 2 * cx.wg + 1, th, best.i);
     }
-    if (stamp) a.stamps[6 * a.L + 1] = wall_clock64();
+    stamp(0, 6 * a.L + 1);
     if (cx.wg != 0) return;
     ArgPair p{-INFINITY, 0};
     for (uint32_t w = cx.tid; w < T; w += PA_THREADS) {
@@ -1133,7 +1142,7 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
         a.state[1] = p.i;
         a.state[0] = pos + 1;
         if (!(a.penalty > 1.0f)) a.counts[a.token] += 1;          // nobody read the counters in this launch
-        if (stamp) a.stamps[6 * a.L + 2] = wall_clock64();
+        stamp(0, 6 * a.L + 2);
         // the host may be spinning on this word instead of waiting for the stream
         if (a.host_out) __hip_atomic_store(a.host_out, ((unsigned long long)a.host_seq << 32) | p.i, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     }
@@ -1427,7 +1436,7 @@ int32_t pa_phase_ms(PaState* st, std::vector<float>* out, hipStream_t s) {
     FH_HIP(hipMemcpyAsync(st->stamps_host.data(), a.stamps, st->n_stamps * 8, hipMemcpyDeviceToHost, s));
     FH_HIP(hipStreamSynchronize(s));
     for (uint32_t i = 0; i + 1 < st->n_stamps; i++)
-        out->push_back((float)((double)(st->stamps_host[i + 1] - st->stamps_host[i]) / (double)st->wall_khz));
+        out->push_back((float)((double)(int64_t)(st->stamps_host[i + 1] - st->stamps_host[i]) / (double)st->wall_khz));
     return FORGE_HIP_OK;
 }
 

@@ -177,8 +177,9 @@ int32_t forge_hip_prefill_logits(forge_hip_model* m, const uint32_t* tokens_host
  * stage_launches_host (may be NULL) the number of kernel launches.  The position advances
  * like forward(); no logits are returned.  prefill_profile does the same for a batched prefill.
  * When the decode step is one resident kernel (forge_hip_model_decode_launches() == 1) its phases are the
- * stages: the kernel stamps the device wall clock at the start of each phase and the differences are
- * reported ("attention" = split + merge phases; "launches" then counts phases). */
+ * stages: the kernel stamps the device wall clock between its phases and the differences are reported ("quantize_act" = the
+ * attention's second phase, where it has one: the merge of its parts and the quantised row; "launches" then counts phases).  A phase's time holds
+ * the wait for the phase before it, and not what was requested of its weights earlier. */
 #define FORGE_HIP_NUM_STAGES 12
 #define FORGE_HIP_STAGE_NAMES                                                                                  \
     "embedding", "rms_norm", "qkv_matmul", "rope_kv_store", "attention", "quantize_act", "o_matmul", "gate_up_matmul", \

@@ -276,6 +276,27 @@ def test_longer_contexts_of_fast_mode(fh, torch_gpu, monkeypatch, name):
     one.close(); streamed.close()
 
 
+@pytest.mark.parametrize("name,flags,prompt", [("smollm2", EXACT, 100), ("wide_1b", EXACT, 100), ("wide_1b", 0, 100), ("wide_1b", 0, 600), ("wide_hd128", 0, 600)])
+def test_profile_gives_every_phase_its_time(fh, torch_gpu, name, flags, prompt):
+    """The phases' times: none is shorter than a hand-over between workgroups takes (0.7 us measured; half of it is asked for), the merge of a long context
+    is the quantise stage's, and they add up to what the kernel takes."""
+    wd, *rest, lm = SHAPES[name]
+    cfg = dict(shape(fh, wd, *rest, layers=4, lm=lm), flags=flags)
+    m = fh.HipModel(cfg, fh.synth.make_weights_blob(cfg, seed=97, threads=16))
+    m.forward_prefill_batch(fh.synth.uniform_ids(98, prompt, cfg["vocab"]))
+    m.forward_profile(1)
+    assert m.decode_launches == 1
+    stages = {k: v for k, v in m.forward_profile(2).items() if v[1]}
+    print({k: f"{1e3 * ms / n:.2f} us" for k, (ms, n) in stages.items()})
+    for stage, (ms, n) in stages.items():
+        if stage == "quantize_act" and prompt < 256:
+            assert ms == 0
+        elif stage != "argmax":
+            assert ms / n > 0.35e-3, (stage, ms, n)
+    assert sum(ms for ms, _ in stages.values()) < 1.0
+    m.close()
+
+
 def test_models_of_several_threads_take_turns(fh, torch_gpu):
     """Two models step at the same time: each kernel needs the whole device, so their launches follow one another, and the tokens are those of a model alone."""
     import threading
