@@ -1207,8 +1207,8 @@ int32_t pa_create(const forge_hip_config& c, const std::vector<PdLayerIn>& layer
     const uint32_t H = c.hidden, I = c.inter, hd = c.head_dim, QKS = c.heads * hd, KV = c.kv_heads * hd;
     if (c.sliding_window != 0 || layers.empty() || !layers[0].qkv || lm_head.kquant()) return FORGE_HIP_OK;
     if (hd != 64 && hd != 96 && hd != 128) return FORGE_HIP_OK;
-    if (H < 64 || I < 64 || QKS < 64 || (uint64_t)c.max_seq * KV * 2 > 0xFFFFFFFFull) return FORGE_HIP_OK;      // a row's place: 32 bits
     const bool q4 = c.wdtype == FORGE_HIP_Q4_0, lmq4 = c.lm_head_dtype == FORGE_HIP_Q4_0;
+    if (H < 64 || I < 64 || QKS < 64 || !decode_ahead_offsets_fit(c.max_seq, KV, c.vocab, H, lmq4)) return FORGE_HIP_OK;
     const bool exact = (c.flags & FORGE_HIP_FLAG_EXACT) != 0;
     const PaForm f = H <= PaNarrow::NX * PA_POLL_THREADS ? pa_form<PaNarrow, true>(hd, q4, lmq4) : exact ? pa_form<PaWide, true>(hd, q4, lmq4) : pa_form<PaWide, false>(hd, q4, lmq4);
     // what the polling threads fetch at once

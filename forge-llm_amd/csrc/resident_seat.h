@@ -1,10 +1,16 @@
-// How a resident kernel is launched, and whose turn it is.
+// The host's side of the resident kernels: what they can reach, how they are launched, and whose turn it is.
 #pragma once
 
 #include <hip/hip_runtime_api.h>
 #include <stdint.h>
 
 namespace fh {
+
+// decode_ahead_kernel finds a layer's cached rows and the blocks of a matrix by 32-bit byte offsets.  (Its other matrices are smaller than the output matrix can be:
+// at most 8192 by 2048 twice.)
+constexpr bool decode_ahead_offsets_fit(uint64_t max_seq, uint64_t kv_channels, uint64_t vocab, uint64_t hidden, bool lm_head_q4) {
+    return max_seq * kv_channels * 2 <= 0xFFFFFFFFull && vocab * hidden / (lm_head_q4 ? 2 : 1) <= 0xFFFFFFFFull;
+}
 
 // All workgroups are co-resident by construction (one per compute unit, checked when the model is created) and every wait in the kernel is bounded, so an ordinary launch
 // is enough; it costs ~7 us less per step than a cooperative one, which checks again.  FORGE_HIP_PD_COOP=1 asks for that one.

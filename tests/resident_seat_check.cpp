@@ -57,7 +57,12 @@ int main(int argc, char** argv) {
         const int32_t rc = seat.turn(handle(s), [&] { printf("launch %s\n", s.name); return (int32_t)FORGE_HIP_OK; });
         printf("-> %d\n", rc);
     };
-    if (what == "launch") {
+    if (what == "offsets") {
+        // the last row of a cache and of an output matrix that 32 bits reach, and the first that they do not
+        printf("%d %d %d %d %d %d\n", fh::decode_ahead_offsets_fit((1u << 21) - 1, 1024, 128256, 2048, false), fh::decode_ahead_offsets_fit(1u << 21, 1024, 128256, 2048, false),
+               fh::decode_ahead_offsets_fit(4096, 512, (1u << 21) - 1, 2048, false), fh::decode_ahead_offsets_fit(4096, 512, 1u << 21, 2048, false),
+               fh::decode_ahead_offsets_fit(4096, 512, (1u << 22) - 1, 2048, true), fh::decode_ahead_offsets_fit(4096, 512, 1u << 22, 2048, true));
+    } else if (what == "launch") {
         (void)fh::resident_launch(nullptr, 256, 768, nullptr, 1000, fh::resident_cooperative(), handle(a));
     } else if (what == "one") {
         fh::ResidentSeat seat;

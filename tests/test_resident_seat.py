@@ -30,6 +30,11 @@ def seats(tmp_path_factory):
 OK, HIP_ERROR = "-> 0", "-> -5"
 
 
+def test_offsets_of_32_bits(seats):
+    """A cache or an output matrix (Q8_0, Q4_0) of 4 GiB is left to the other kernels: the blocks behind would be read from its beginning."""
+    assert seats("offsets") == ["1 0 1 0 1 0"]
+
+
 @pytest.mark.parametrize("value,want", [("0", "ordinary"), ("1", "cooperative")])
 def test_the_variable_asks_for_cooperative_launches(seats, value, want):
     assert seats("launch", FORGE_HIP_PD_COOP=value) == [f"{want} a 256 768 1000"]
