@@ -683,10 +683,11 @@ struct PaPart {
                         for (int u = 0; u < 2; u++) {
                             const uint32_t t = tp + u * KPW + slot;
                             Half8 kk;
+                            // what is read in place of a key that is not there, or past a row's end, counts as 0: a weight of 0 times an infinite value would not
 #pragma unroll
                             for (int i = 0; i < 4; i++) {
-                                kk.w[i] = t == pos ? nk[i] : k[p0 + u].w[i];
-                                vv[u].w[i] = t == pos ? nv[i] : v[p0 + u].w[i];
+                                kk.w[i] = !dvalid ? 0u : t == pos ? nk[i] : k[p0 + u].w[i];
+                                vv[u].w[i] = t >= t1 ? 0u : t == pos ? nv[i] : v[p0 + u].w[i];
                             }
                             const float d = key_dot<LPK>(qf, kk);
                             sc[u] = t < t1 ? d * scale : -INFINITY;

@@ -276,6 +276,43 @@ def test_longer_contexts_of_fast_mode(fh, torch_gpu, monkeypatch, name):
     one.close(); streamed.close()
 
 
+@pytest.mark.parametrize("head_dim,which,channel", [(64, "v", 5), (96, "v", 5), (128, "v", 127), (96, "k", 95), (128, "k", 127)])
+def test_an_infinite_value_in_the_first_row_of_a_long_context(fh, torch_gpu, monkeypatch, head_dim, which, channel):
+    """The first row stands in for keys that are not there and its last channels for those past a head's: neither may count.  The first token's embedding has one channel, and
+    one row of k or v is that channel alone, by a factor that takes it past what the 16-bit cache holds and leaves every other token's there."""
+    hidden, heads, kv = 800, 4, 2
+    cfg = dict(shape(fh, Q8, hidden, 512, heads, kv, head_dim, 1000, layers=1), flags=0)
+    blob = fh.synth.make_weights_blob(cfg, seed=107)
+    row, first, at = hidden // 32 * 34, 11, 3
+    embed = blob[:1000 * hidden * 4].view(np.float32).reshape(1000, hidden)
+    embed[first] = 0
+    embed[first, at] = 1
+    norm = blob[1000 * hidden * 4:][:hidden * 4].view(np.float32)
+    matrix = 1001 * hidden * 4 + (heads * head_dim + (kv * head_dim if which == "v" else 0)) * row
+    blocks = blob[matrix + channel * row:matrix + (channel + 1) * row].reshape(-1, 34)
+    blocks[:] = 0
+    blocks[0, :2] = np.array([1.4e5 / (127 * hidden ** 0.5 * abs(norm[at]))], np.float16).view(np.uint8)
+    blocks[0, 2 + at] = 127
+    one = fh.HipModel(cfg, blob)
+    monkeypatch.setenv("FORGE_HIP_PD_AHEAD", "0")
+    streamed = fh.HipModel(cfg, blob)
+    toks = fh.synth.uniform_ids(108, 340, 1000)
+    toks[toks == first] = 12
+    toks[0] = first
+    for m in (one, streamed):
+        m.forward_prefill_batch(toks[:300])
+    cached = one.read_kv(0, 0 if which == "k" else 1)
+    cached = cached.view(np.float16).reshape(300, kv * head_dim)
+    assert np.isinf(cached[0, channel]) and np.isfinite(cached[1:]).all()
+    for t in toks[300:310]:
+        a, b = one.forward(int(t)), streamed.forward(int(t))
+        assert one.decode_launches == 1
+        assert np.array_equal(np.isfinite(a), np.isfinite(b))
+        if np.isfinite(b).all():
+            assert np.linalg.norm(a - b) < 2e-2 * np.linalg.norm(b)
+    one.close(); streamed.close()
+
+
 @pytest.mark.parametrize("name,flags,prompt", [("smollm2", EXACT, 100), ("wide_1b", EXACT, 100), ("wide_1b", 0, 100), ("wide_1b", 0, 600), ("wide_hd128", 0, 600)])
 def test_profile_gives_every_phase_its_time(fh, torch_gpu, name, flags, prompt):
     """The phases' times: none is shorter than a hand-over between workgroups takes (0.7 us measured; half of it is asked for), the merge of a long context
