@@ -1302,8 +1302,11 @@ int32_t pa_create(const forge_hip_config& c, const std::vector<PdLayerIn>& layer
             st->lds += n * rec_bytes;
             // Rounds.  With a second head a wave, a third round is no longer hidden (us per token, decode_persistent.hip / this: 12/2 heads of 128, 2540 rows 287 / 270,
             // 3500: 286 / 293; 14/2 of 64, 5000: 241 / 210, 10000: 256 / 261); with few KV heads that kernel has more workgroups for the context.  Otherwise this
-            // one is ahead as far as was measured (8 layers of the 1B shape, 5000: 325 / 245, 20000: 377 / 337; 16/4 heads of 96, 10000: 372 / 299).
-            const uint32_t rounds = gsize <= PA_POLL && c.kv_heads >= 4 ? PA_ROUNDS : 2;
+            // one is ahead up to the eighth round (8 layers of the 1B shape, 5000: 325 / 245, 20000: 377 / 337; 16/4 heads of 96, 10000: 368 / 308), but with heads of 128 not
+            // past the sixth (16/8, 7000: 274 / 261, 10000: 289 / 296; 16/16, 3500: 270 / 264, 5000: 286 / 295), and with fewer than 16 splits, whose contexts are short, not
+            // past the fifth (8 splits of 12/4 heads of 128, 1000: 226 / 201, 2400: 237 / 258; of 16/4 heads of 96, 1000: 261 / 217, 2400: 276 / 284; 4 splits of the 1B
+            // shape, 1000: 307 / 257, 2400: 311 / 321).  Below 8 splits (more than 32 KV heads, or no LDS for more) there is little context left to cover.
+            const uint32_t rounds = gsize > PA_POLL || c.kv_heads < 4 ? 2 : n < 16 ? 5 : hd > 96 ? 6 : PA_ROUNDS;
             st->max_rows = std::min(c.max_seq, n * rounds * PA_PASSES * (hd <= 64 ? 8u : 4u));
             st->kernel_long = pa_kernel<PaWide, false, true>(hd, q4, lmq4);
         }

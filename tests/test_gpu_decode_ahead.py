@@ -226,9 +226,9 @@ def test_fast_mode_takes_it_too(fh, oracle, torch_gpu, name):
 
 
 # (hidden, inter, heads, kv heads, head dim, contexts whose next steps cross a line): from the short form; from one round of requested keys to two and to three; from
-# two rounds to the other kernel.  Groups of 4, of 7 (waves with a second head) and of 3 heads, heads that fill their lanes and heads that do not
+# two rounds (two KV heads), five (10 splits) and six (heads of 128) to the other kernel.  Groups of 4, of 7 (waves with a second head) and of 3 heads, heads that fill their lanes and heads that do not
 LONG = {"1b": (2048, 8192, 32, 8, 64, (254, 800, 2557, 5117)), "groups_of_7": (896, 4864, 14, 2, 64, (254, 318, 2557, 5117)),
-        "hd96": (1536, 4096, 16, 4, 96, (254, 800, 1277, 2557)), "hd128": (1024, 3072, 12, 4, 128, (254, 318, 1277, 2557))}
+        "hd96": (1536, 4096, 16, 4, 96, (254, 800, 1277, 2557)), "hd128": (1024, 3072, 12, 4, 128, (254, 318, 1277, 2557, 7677)), "splits_10": (800, 512, 24, 24, 64, (254, 798, 3997))}
 
 
 @pytest.mark.parametrize("name", sorted(LONG))
@@ -237,9 +237,9 @@ def test_longer_contexts_of_fast_mode(fh, torch_gpu, monkeypatch, name):
     a few thousand terms: 1e-5) unless a code of an 8-bit vector falls to its neighbour; each of the four vectors carries a rounding of 1/127 of a block's
     largest value, 0.6% of its norm, twice (both kernels'): under 2% of the output's."""
     hidden, inter, heads, kv_heads, hd, contexts = LONG[name]
-    cfg = dict(shape(fh, Q8, hidden, inter, heads, kv_heads, hd, 1000, layers=1, max_seq=5248), flags=0)
+    cfg = dict(shape(fh, Q8, hidden, inter, heads, kv_heads, hd, 1000, layers=1, max_seq=5248 if contexts[-1] < 5200 else 7808), flags=0)
     one, streamed = pair(fh, monkeypatch, cfg, 57)
-    toks = fh.synth.uniform_ids(58, 5200, cfg["vocab"])
+    toks = fh.synth.uniform_ids(58, cfg["max_seq"] - 48, cfg["vocab"])
     rel = []
     for n in contexts:
         for m in (one, streamed):
