@@ -222,7 +222,49 @@ def test_fast_mode_takes_it_too(fh, oracle, torch_gpu, name):
     for t in toks[1:]:
         a, b = fast.forward(int(t)), om.forward(int(t))
     assert np.all(np.isfinite(a)) and np.corrcoef(a, b)[0, 1] > 0.99
+    # correlation sees neither scale nor offset.  Eight 8-bit vectors, 0.6% of the norm each and twice, over caches that differ as much
+    assert np.linalg.norm(a - b) < 0.1 * np.linalg.norm(b)
     fast.close()
+
+
+@pytest.mark.parametrize("name", ["narrow_form", "wide_1b", "wide_least", "wide_hd96", "wide_hd128"])
+def test_short_contexts_of_fast_mode(fh, torch_gpu, monkeypatch, name):
+    """Single steps from identical state, one layer, against decode_step_kernel: the bounds of test_longer_contexts_of_fast_mode."""
+    wd, *rest, lm = SHAPES[name] if name in SHAPES else (Q8, 256, 512, 4, 2, 64, 1000, None)
+    cfg = dict(shape(fh, wd, *rest, layers=1, lm=lm), flags=0)
+    one, streamed = pair(fh, monkeypatch, cfg, 117)
+    toks = fh.synth.uniform_ids(118, 260, cfg["vocab"])
+    rel = []
+    for n in (1, 2, 62, 63, 64, 126, 127, 128, 190, 191, 192, 253, 254):
+        for m in (one, streamed):
+            m.reset()
+            m.forward_prefill_batch(toks[:n])
+        a, b = one.forward(int(toks[n])), streamed.forward(int(toks[n]))
+        assert one.decode_launches == 1 and np.all(np.isfinite(a))
+        rel.append(np.linalg.norm(a - b) / np.linalg.norm(b))
+    assert max(rel) < 2e-2 and np.median(rel) < 1e-5, rel
+    one.close(); streamed.close()
+
+
+@pytest.mark.parametrize("head_dim", [64, 96, 128])
+@pytest.mark.parametrize("page_rows", [64, 256])
+def test_narrow_models_over_pages(fh, torch_gpu, head_dim, page_rows):
+    """Contexts across the edges of blocks and pages, up to the narrow form's last and past it: the flat cache's bits."""
+    cfg = dict(shape(fh, Q8, 256, 512, 4, 2, head_dim, 1000), flags=0)
+    blob = fh.synth.make_weights_blob(cfg, seed=127)
+    flat, paged = fh.HipModel(cfg, blob), fh.HipModel(cfg, blob)
+    paged.set_kv_pages(page_rows, np.random.default_rng(128).permutation(cfg["max_seq"] // page_rows).astype(np.uint32))
+    toks = fh.synth.uniform_ids(129, 780, cfg["vocab"])
+    for n in (1, 62, 127, 254, 510, 700, 764):
+        for m in (flat, paged):
+            m.reset()
+            m.forward_prefill_batch(toks[:n])
+        for t in toks[n:n + 6]:
+            same_bits(paged.forward(int(t)), flat.forward(int(t)))
+    for layer in range(cfg["layers"]):
+        for which in (0, 1):
+            assert np.array_equal(paged.read_kv(layer, which), flat.read_kv(layer, which))
+    flat.close(); paged.close()
 
 
 # (hidden, inter, heads, kv heads, head dim, contexts whose next steps cross a line): from the short form; from one round of requested keys to two and to three; from
@@ -252,13 +294,15 @@ def test_longer_contexts_of_fast_mode(fh, torch_gpu, monkeypatch, name):
     assert max(rel) < 2e-2 and np.median(rel) < 1e-5, rel
     # the same rows in pages all over the pool: the same bits
     paged = fh.HipModel(cfg, fh.synth.make_weights_blob(cfg, seed=57, threads=16))
-    paged.set_kv_pages(64, np.random.default_rng(59).permutation(cfg["max_seq"] // 64).astype(np.uint32))
-    for n in (200, contexts[-1]):
-        for m in (one, paged):
-            m.reset()
-            m.forward_prefill(toks[:n])
-        for t in toks[n:n + 3]:
-            same_bits(paged.forward(int(t)), one.forward(int(t)))
+    for page_rows, starts in ((64, (200, contexts[-1])), (128, (254, contexts[-2]))):
+        paged.reset()
+        paged.set_kv_pages(page_rows, np.random.default_rng(59).permutation(cfg["max_seq"] // page_rows).astype(np.uint32))
+        for n in starts:
+            for m in (one, paged):
+                m.reset()
+                m.forward_prefill(toks[:n])
+            for t in toks[n:n + 3]:
+                same_bits(paged.forward(int(t)), one.forward(int(t)))
     paged.close()
     # a step that gives up has not happened
     for m in (one, streamed):
@@ -324,7 +368,6 @@ def test_profile_gives_every_phase_its_time(fh, torch_gpu, name, flags, prompt):
     m.forward_profile(1)
     assert m.decode_launches == 1
     stages = {k: v for k, v in m.forward_profile(2).items() if v[1]}
-    print({k: f"{1e3 * ms / n:.2f} us" for k, (ms, n) in stages.items()})
     for stage, (ms, n) in stages.items():
         if stage == "quantize_act" and prompt < 256:
             assert ms == 0

@@ -293,8 +293,10 @@ def test_prefill_attention_with_quantising_epilogue_equals_separate_kernels(fh, 
 
 
 def persistent_pair(fh, cfg, blob, monkeypatch, ordered=True):
-    """The kernel-sequence model and the one-kernel model.  ordered: the one-kernel step sums GEMV rows in the
-    reference's block order (then it is bit-identical to the sequence) instead of as the products come."""
+    """The kernel-sequence model and the one-kernel model (decode_step_kernel, which runs these sizes only where decode_ahead_kernel is
+    switched off).  ordered: the one-kernel step sums GEMV rows in the reference's block order (then it is bit-identical to the
+    sequence) instead of as the products come."""
+    monkeypatch.setenv("FORGE_HIP_PD_AHEAD", "0")
     monkeypatch.setenv("FORGE_HIP_PERSIST", "0")
     seq = fh.HipModel(cfg, blob)
     monkeypatch.setenv("FORGE_HIP_PERSIST", "1")
@@ -448,6 +450,30 @@ def test_persistent_decode_kernel_default_summation(fh, oracle, torch_gpu, monke
     seq.close(); one.close()
 
 
+@pytest.mark.parametrize("head_dim", [64, 96, 128])
+@pytest.mark.parametrize("heads,kv_heads", [(4, 4), (4, 2), (6, 2), (8, 2)])
+def test_persistent_decode_kernel_without_a_merge(fh, torch_gpu, monkeypatch, heads, kv_heads, head_dim):
+    """Default sums: up to 128 keys a group of heads is one item whose workgroup finishes it, from 129 on its splits are merged.  Steps over 1, 2 and over 127 to
+    130 keys from identical state, one layer: the kernel sequence's sums in another order (a few hundred terms: 1e-5), unless a code of one of the four 8-bit vectors falls to its
+    neighbour, 1/127 of a block's largest value, 0.6% of the vector's norm, in either: under 2% of the output's."""
+    cfg = fh.synth.tiny(Q8, max_seq=640, hidden=256, inter=512, layers=1, heads=heads, kv_heads=kv_heads, head_dim=head_dim, vocab=1000)
+    blob = fh.synth.make_weights_blob(cfg, seed=47)
+    toks = fh.synth.uniform_ids(48, 140, cfg["vocab"])
+    seq, one = persistent_pair(fh, cfg, blob, monkeypatch, ordered=False)
+    rel = []
+    for n, steps in ((0, 2), (126, 4)):
+        for m in (seq, one):
+            m.reset()
+            if n:
+                m.forward_prefill_batch(toks[:n])
+        for t in toks[n:n + steps]:
+            a, b = one.forward(int(t)), seq.forward(int(t))
+            assert np.all(np.isfinite(a))
+            rel.append(np.linalg.norm(a - b) / np.linalg.norm(b))
+    assert max(rel) < 2e-2 and np.median(rel) < 1e-5, rel
+    seq.close(); one.close()
+
+
 @pytest.mark.parametrize("shape", ["smollm2_135m", "llama_1b_2layers", "llama_3b_2layers", "phi3_mini_2layers", "hd96_gqa", "mha_12_heads"])
 def test_persistent_decode_kernel_real_shapes(fh, torch_gpu, monkeypatch, shape):
     """Same check on the shapes that matter: SmolLM2-135M (hidden 576, 9 heads over 3 KV heads: partial weight
@@ -513,7 +539,8 @@ def test_order_faithful_mode_on_the_resident_kernel(fh, oracle, torch_gpu, monke
     }
     cfg, prompts = cfgs[shape]()
     blob = fh.synth.make_weights_blob(cfg, seed=91, threads=16)
-    seq = fh.HipModel(cfg, blob)                             # the default of the order-faithful mode: the kernel sequence
+    monkeypatch.setenv("FORGE_HIP_PD_AHEAD", "0")
+    seq = fh.HipModel(cfg, blob)                             # the order-faithful mode's kernel sequence
     monkeypatch.setenv("FORGE_HIP_PD_EXACT", "1")
     one = fh.HipModel(cfg, blob)
     assert one.decode_launches == 1 and seq.decode_launches > 1
@@ -610,6 +637,12 @@ def test_paged_kv_cache_equals_flat_cache(fh, torch_gpu, monkeypatch, shape, per
     paged.set_kv_pages(0)                                        # back to the flat cache
     same_bits(paged.forward_prefill(toks[:70]), flat.forward_prefill(toks[:70]))
     flat.close(); paged.close()
+
+
+def test_paged_kv_cache_equals_flat_cache_in_decode_step_kernel(fh, torch_gpu, monkeypatch):
+    """The 1B layer shape again, in the kernel that runs it without decode_ahead_kernel."""
+    monkeypatch.setenv("FORGE_HIP_PD_AHEAD", "0")
+    test_paged_kv_cache_equals_flat_cache(fh, torch_gpu, monkeypatch, "llama_1b_2layers", "1")
 
 
 def test_paged_kv_cache_refusals(fh, torch_gpu):

@@ -224,6 +224,14 @@ def test_greedy_with_repeat_penalty_on_the_device_equals_the_host_path(fh, so, t
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("wd", [Q8, Q4])
+def test_greedy_with_repeat_penalty_in_decode_step_kernel(fh, so, torch_gpu, monkeypatch, wd):
+    """The same with decode_ahead_kernel switched off, which runs models of this size by default."""
+    monkeypatch.setenv("FORGE_HIP_PD_AHEAD", "0")
+    test_greedy_with_repeat_penalty_on_the_device_equals_the_host_path(fh, so, torch_gpu, monkeypatch, wd, 0)
+
+
+@pytest.mark.gpu
 def test_generate_loop_equals_the_oracle_loop(fh, oracle, so, torch_gpu):
     """HipModel.generate (project.rs:714-751 with its defaults: greedy, repeat penalty 1.1) in exact mode against the same
     loop over the CPU oracle: identical tokens; and with a temperature, host sampler on GPU logits against the oracle's."""
