@@ -47,9 +47,9 @@ DIVERGENCE_STEPS = 128         # greedy steps over which the fast mode's tokens 
 # WRITE_SIZE counters of two profiler runs of this script, each scaled by what the same counter reads for the 1 GiB
 # copy of --calibrate-copy (FETCH_SIZE x2.000, WRITE_SIZE x1.000).  Summary: profiles/gemv_hbm_traffic_pmc.md.
 GEMV_HBM_BYTES_PER_LAUNCH = 20.46e6 + 0.02e6      # fetched + written
-# The same for one launch of decode_step_kernel (the whole step; not counted again for decode_ahead_kernel, which reads the same planes once) at this context: 1 436.9 MB fetched + 13.8 MB
-# written.  Summary: profiles/decode_step_kernel_hbm_traffic_pmc.md.
-STEP_KERNEL_HBM_BYTES_PER_LAUNCH = 1450.7e6
+# The same for one launch of the headline's decode_ahead_kernel (the whole step) at this context: 1 434.6 MB fetched + 11.6 MB
+# written.  Summary: profiles/decode_ahead_kernel_hbm_traffic_pmc.md.
+STEP_KERNEL_HBM_BYTES_PER_LAUNCH = 1434.6e6 + 11.6e6
 
 
 def gemv_launch_bytes(fh, cfg):
@@ -127,7 +127,9 @@ def decode_profile(fh, model, cfg, tok, context, prof_steps=8):
             stage_n[s] = stage_n.get(s, 0) + n
     gbytes = gemv_launch_bytes(fh, cfg)
     gemv_bytes_total = sum(gbytes.values())
-    per_stage = {s: {"GB/s": round(gbytes[s] / (stage_ms[s] * 1e-3) / 1e9, 1), "us_per_token": round(stage_ms[s] * 1e3, 1)} for s in gbytes}
+    rate = {s: gbytes[s] / (stage_ms[s] * 1e-3) / 1e9 for s in gbytes}
+    # no rate for a phase whose weights were for the most part requested during the one before it
+    per_stage = {s: {"GB/s": round(rate[s], 1) if rate[s] <= HBM_PEAK_GBS else None, "us_per_token": round(stage_ms[s] * 1e3, 1)} for s in gbytes}
     stage_us = {s: round(v * 1e3, 1) for s, v in stage_ms.items() if v > 0}
     n_launch = model.decode_launches
     if n_launch <= (cfg["layers"] + 33) // 34:
@@ -137,9 +139,11 @@ def decode_profile(fh, model, cfg, tok, context, prof_steps=8):
         total = gemv_bytes_total + kv_bytes
         kernel_ms = sum(stage_ms.values())
         achieved = total / (kernel_ms * 1e-3) / 1e9
+        counted = (cfg["hidden"], cfg["inter"], cfg["layers"], cfg["vocab"], cfg["wdtype"]) == (2048, 8192, 16, 128256, fh.Q8_0) and \
+            PROMPT_TOKENS <= context < PROMPT_TOKENS + 256 and os.environ.get("FORGE_HIP_PD_AHEAD", "1") != "0"
         roof = {"kernel": "the resident decode kernel (decode_ahead_kernel or decode_step_kernel; the whole decode step: every quantised GEMV, decode attention, norms, argmax)",
                 "bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS,
-                "traffic": STEP_KERNEL_HBM_BYTES_PER_LAUNCH, "bytes_per_launch": total / n_launch, "us_per_launch": kernel_ms * 1e3 / n_launch,
+                "traffic": STEP_KERNEL_HBM_BYTES_PER_LAUNCH if counted else None, "bytes_per_launch": total / n_launch, "us_per_launch": kernel_ms * 1e3 / n_launch,
                 "launches_per_step": n_launch, "weights_and_vectors_bytes": gemv_bytes_total, "kv_cache_bytes": kv_bytes,
                 "per_phase": per_stage}
     else:
