@@ -1,7 +1,7 @@
 // One decode token as ONE kernel whose waves hold their share of a layer's matrices in registers (model::forward, emit.rs:4029-4227).
 //
 // A step is a chain of four products and an attention per layer.  As kernels a link of that chain is 4 to 6 us however small (a launch that does nothing takes
-// 2.7); as phases of the kernel that streams weights of any size (decode_persistent.hip) it is 5.  Here a layer of SmolLM2-135M takes 13 us, one of the 1B shape 24
+// 2.7); as phases of the kernel that streams weights of any size (decode_persistent.hip) it is 5.  Here a layer of SmolLM2-135M takes 12 us, one of the 1B shape 23
 // (its 65 MB alone take 14): five hand-overs of 0.8 to 1.2 (1.5 to 2.5 beside weights), two norms of 0.7, attention 3.2, and the products.
 //   * A wave's rows are a few registers, requested where nothing is on its way to the compute unit: while the attention is at work, and with wide models also right
 //     behind the products.  (A compute unit's loads return in order and its queue is short: a poll behind weights comes when they have come, and so does a store.)
@@ -18,8 +18,10 @@
 // order-faithful kernel sequence; narrow models, to which the order costs nothing, run it in both modes.  Otherwise row sums and the norm's sum add up as the lanes
 // have them.  Per token in us, kernel sequence (order-faithful mode) / decode_persistent.hip (fast mode) / this, by rows of context:
 //   SmolLM2-135M Q8_0   33: 781 / 880 / 384    300: 820 / 878 / 421    740: 907 / 876 / 466
-//   1B shape Q8_0       33: 754 / 610 / 466 and 427 (order-faithful, fast)    200: - / 636 / 473 and 439       Q4_0, fast: 33: 532 / 407
-//   and in fast mode (PaPart) 260: 637 / 470    1000: 642 / 475    2400: 644 / 483    5000: 676 / 514    Q4_0 2400: 570 / 439
+//   1B shape Q8_0       33: 754 / 610 / 469 and 433 (order-faithful, fast)    200: - / 636 / 476 and 441       Q4_0, fast: 33: 532 / 403
+//   and in fast mode (PaPart) 300: 637 / 464    1000: 642 / 471    2400: 644 / 479    5000: 676 / 515    Q4_0 2400: 570 / 442
+// Heads of 96 and 128 gain as much though those of 128 spill (8 layers, 33 rows, fast: 8/2 of 96 at 768 channels 213 / 136, 6/2 of 128 207 / 138, 16/4 of 96 at 1536 246 / 174,
+// 12/4 of 128 at 1024 212 / 168).  A layer's weights hardly count (1B shape, us: Q8_0 23, Q4_0 22): it is the chain that takes the time.
 #include <stddef.h>
 #include <string.h>
 
@@ -83,7 +85,7 @@ struct PaArgs {
     uint64_t* taq;     // [QKS/32][9]        attention output, a block of 32: int8 codes (4 per element), then the fp16 scale
     uint64_t* taq2;    // [I/32][9]          silu(gate)*up, same format
     uint64_t* trec;    // [heads][splits][HD + 2]  Wide, long contexts: a split's weighted sum, maximum and weight sum
-    uint64_t* tpart;   // [2 G]              per-workgroup argmax candidates
+    uint64_t* tpart;   // [2 workgroups of the grid]  argmax candidates
     float* logits;
     uint32_t* state;   // [0] position  [1] token  [2] next token  [3] abort flag  [4] number of the step that counted its token
     uint32_t* counts;

@@ -61,7 +61,7 @@ struct LlamaModel : forge_hip_model {
     bool prefill_fuse_silu = false;              // fast mode: the gate/up GEMM writes silu(gate) * up quantised (FORGE_HIP_FUSE=0: separate kernel)
     bool fuse_norm = false, fuse_silu = false;   // fused GEMV prologue/epilogue variants fit LDS for this model
     PdState* pd = nullptr;               // the decode step as one resident kernel, when the shape is covered
-    PaState* pa = nullptr;               // the same for a narrow model, whatever the mode, over the contexts that it covers
+    PaState* pa = nullptr;               // the same for a model of up to 2048 channels, whatever the mode, over the contexts that it covers
     bool step_ahead = false;             // the step enqueued last is pa's
     uint32_t step_seq = 0;               // its number.  One count for both kernels: they mark a counted token in the same word of the device's state
     std::unique_ptr<ResidentSeat> seat;  // of a model that has either

@@ -191,7 +191,7 @@ int32_t forge_hip_prefill_profile(forge_hip_model* m, const uint32_t* tokens_hos
 
 /* Kernel launches the next decode step costs on this model (an order-faithful one has three for attention past a context of 768 rows,
  * or 256 with heads wider than 64, and one up to it): 1 when the whole step runs as one resident kernel
- * (fast mode, covered shapes; one launch per 34 layers for a deeper model), otherwise the length of the kernel sequence.  The Metal backend's counterpart
+ * (covered shapes, in the order-faithful mode over short contexts; one launch per 34 layers for a deeper model of more than 2048 channels), otherwise the length of the kernel sequence.  The Metal backend's counterpart
  * is the fixed encoder sequence of MetalModel::forward (metal:5070-5300). */
 int32_t forge_hip_model_decode_launches(const forge_hip_model* m);
 
