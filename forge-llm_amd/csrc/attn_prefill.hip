@@ -2,15 +2,23 @@
 // cache, with both matrix products on fp16 MFMA (v_mfma_f32_32x32x16_f16) and the online
 // softmax in f32.
 //
-// Workgroup = 8 waves = 128 consecutive queries of one head: four groups of 32 queries, each shared by two
-// waves that take one half (32 keys) of every key tile and merge their (max, sum, output) once at the end, so
-// that the longest chain of dependent tile steps (the last query tile's) is worked on by twice the waves.
-// K/V are streamed in tiles of 64 keys through two LDS buffers (K row-major, V transposed so that
-// the contraction index of P.V is contiguous per lane; a thread fetches 4 head dims of two
-// consecutive keys and writes the pairs as dwords).  Scores stay in the base-2 domain
-// (s * scale * log2 e) so that the exponential is one v_exp_f32 after one FMA; keys are masked only in
-// tiles that reach past the wave's first query, and the accumulators are rescaled only when some
-// query of the wave saw a new maximum.
+// Workgroup = 128 consecutive queries of one head in four groups of 32; four waves, one to a group, or eight, two to a group, which take one
+// half (32 keys) of every key tile and merge their (max, sum, output) once at the end, so that the longest chain of dependent tile steps
+// (the last query tile's) is worked on by twice the waves.
+// K/V are streamed in tiles of 64 keys through two LDS buffers, both as rows, by loads that go straight into LDS: no registers, one offset per
+// lane that every tile reuses behind a new descriptor, one wait and one barrier per step.  P.V wants V with the keys contiguous per lane:
+// ds_read_b64_tr_b16 transposes on the way out.  (Through registers, with V transposed on the way in, a third of a step went into issuing the
+// loads and writing them to LDS, and the registers they took left two waves per SIMD where three fit now.)
+// Scores stay in the base-2 domain (s * scale * log2 e) so that the exponential is one v_exp_f32 after one FMA; keys are masked only in
+// tiles that reach past the wave's first query; the maximum that scores are taken against, and the accumulators with it, move only when
+// some query of the wave has risen above it by more than 2^SLACK (before: whenever it rose, which with 32 queries to a wave is most steps
+// of a prompt of a few thousand tokens, 50 multiplications of about 190 VALU instructions each time).
+// What bounds it: full, the matrix unit, the VALU (32 exp, 32 FMA, 32 additions, 16 conversions, 16 maxima per 32 x 64 scores) and LDS reads
+// take about 800 cycles each and overlap to 1800 (heads of 96, 3072 queries behind 8192 keys 390 us = 0.94 PFLOP/s, 128 1.0, 64 0.9; the
+// library's large bf16 product is at 1.2); causal, the uneven length of the query tiles on top.  3001 tokens: 32/32 heads of 96 95.4 -> 75.1 us,
+// 32/8 of 128 124 -> 89, 2502 tokens of 32/8 of 64 52.5 -> 42.7, 1000 of 32/8 of 128 38.2 -> 24.0.
+// Measured and not kept: waits of our own around the transposing reads (the compiler waits for the next tiles ahead of the first of them):
+// no faster; query tiles of every other round in ascending order: within 2 %.
 //
 // Both products are computed transposed, S^T = K Q^T and O^T = V^T P^T.  In the 32x32 MFMA
 // result layout a lane then owns ONE query (column = lane%32) and 16 keys (or 16 head dims),
@@ -24,12 +32,30 @@ namespace fh {
 
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef _Float16 v4h __attribute__((ext_vector_type(4)));
+typedef short v4s __attribute__((ext_vector_type(4)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 
 constexpr int QW = 32;        // queries per wave pair
 constexpr int QB = 128;       // queries per workgroup
 constexpr int KT = 64;        // keys per tile
 constexpr int AP_THREADS = 512;   // the 8-wave form; the 4-wave form runs 256
+constexpr uint32_t AP_RSRC_FLAGS = 0x00020000;   // raw buffer, 32-bit data format
+constexpr float SLACK = 8.f;      // base-2 exponent
+
+#define FH_LDS3(p) ((__attribute__((address_space(3))) void*)(p))
+
+// Where piece p (16 bytes) of row r of a tile lies in its row of LDS, and which piece lies at p: eight consecutive rows of K at one piece
+// (a fragment's reads), and two neighbouring pieces of four consecutive rows of V, touch all banks.  Rows are as long in LDS as they are: a load
+// into LDS fills 1 KB in lane order.
+template <int HD>
+__device__ __forceinline__ uint32_t piece_of(uint32_t r, uint32_t p) {
+    if constexpr (HD == 96) return p ^ ((r & 2) | ((r >> 2) & 1));       // rows alternate between two halves of the banks as they are
+    else return p ^ (((r & 3) << 1) | ((r >> 2) & 1));
+}
+
+__device__ __forceinline__ v4h read_transposed(const uint8_t* at) {
+    return __builtin_bit_cast(v4h, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s*)at));
+}
 
 // QUANT: instead of f32 rows the kernel writes what the o projection's GEMM reads, the activation quantiser's int8
 // codes oq[M][heads*HD] and fp16 scales osc[M][heads*HD/32] of the same values (a 32-element block is one 32-wide
@@ -46,24 +72,20 @@ void attn_prefill_kernel(const float* __restrict__ q, const uint16_t* __restrict
                          float* __restrict__ out, uint32_t q_stride, uint32_t out_stride, uint32_t M, uint32_t base_pos,
                          uint32_t heads, uint32_t kv_heads, int8_t* __restrict__ oq, uint16_t* __restrict__ osc, uint32_t window,
                          PageTable pt) {
-    constexpr int KS = HD + 8;    // K tile row stride (halfs): 16-byte pad
-    constexpr int VS = KT + 4;    // V^T tile row stride (halfs): 8-byte pad
-    constexpr int KTOTAL = KT * HD / 8;          // 16-byte pieces of K per tile
-    constexpr int VTOTAL = KT * HD / 8;          // (key pair, 4 dims) items of V per tile
-    constexpr int NT = AP_THREADS / KH;           // threads of the workgroup
-    constexpr int KPIECES = (KTOTAL + NT - 1) / NT, VITEMS = (VTOTAL + NT - 1) / NT;
-    constexpr int DG = HD / 4;    // groups of 4 head dims
+    constexpr uint32_t ROW = HD * 2, PIECES = HD / 8;     // bytes and 16-byte pieces of a row of a tile
+    constexpr uint32_t TILE = KT * ROW;                   // bytes of a tile of K, and of V
+    constexpr uint32_t WAVES = AP_THREADS / KH / 64;
+    constexpr uint32_t LOADS = 2 * PIECES / WAVES;        // loads of 1 KB into LDS per wave and tile pair: K's come first
+    constexpr bool EVEN = PIECES % WAVES == 0;            // then a wave's loads of V repeat those of K
+    constexpr uint32_t OFFS = EVEN ? LOADS / 2 : LOADS;
     constexpr int NS = HD / 16;   // MFMA k-steps over head_dim
     constexpr int ND = HD / 32;   // 32-wide head_dim tiles of the output
-    constexpr int KBYTES = KT * KS * 2, VBYTES = HD * VS * 2;
     constexpr int MERGE_FLOATS = 2 + ND * 16;    // per lane: m, l and the output accumulators
-    static_assert(KH == 2 || 2 * (KBYTES + VBYTES) >= 4 * 64 * MERGE_FLOATS * 4, "the merge reuses the tile buffers");
-    // two tiles each: the loads of tile t+1 are written while tile t is read, one barrier per tile
-    __shared__ __attribute__((aligned(16))) uint8_t smem[2 * (KBYTES + VBYTES)];
-    auto Ks = [&](uint32_t buf) { return reinterpret_cast<_Float16*>(smem + buf * KBYTES); };
-    auto Vt = [&](uint32_t buf) { return reinterpret_cast<_Float16*>(smem + 2 * KBYTES + buf * VBYTES); };
+    // two pairs of tiles: those of step t+1 arrive while the ones of step t are read, one barrier per step
+    constexpr uint32_t LDS = KH == 1 && 4 * 64 * MERGE_FLOATS * 4 > 4 * TILE ? 4 * 64 * MERGE_FLOATS * 4 : 4 * TILE;
+    __shared__ __attribute__((aligned(16))) uint8_t smem[LDS];
 
-    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
     const uint32_t qg = KH == 1 ? wave >> 1 : wave, kh = KH == 1 ? (wave & 1) : 0;   // query group of 32, (first) half of every key tile
     const uint32_t lq = lane & 31, lh = lane >> 5;
     // tile-major order, heaviest (latest) query tiles first: they stream the most keys, and whatever does not fit the
@@ -110,61 +132,50 @@ void attn_prefill_kernel(const float* __restrict__ q, const uint16_t* __restrict
     const uint32_t wave_lo = (WIN && wave_min_pos + 1 > window) ? wave_min_pos + 1 - window : 0;
     const uint32_t tile0 = wg_lo / KT;
 
-    int4 kreg[KPIECES];
-    uint2 va[VITEMS], vb[VITEMS];
-    auto load_tile = [&](uint32_t kt) {
-        // a paged cache: a tile of 64 keys lies within one page (pages are multiples of 64 rows), `shift` rows further on
-        const ptrdiff_t shift = pt.table ? (ptrdiff_t)paged_row(pt, kt * KT) - (ptrdiff_t)(kt * KT) : 0;
-        const uint16_t* kc = kc_flat + shift * (ptrdiff_t)kv_stride;
-        const uint16_t* vc = vc_flat + shift * (ptrdiff_t)kv_stride;
+    // Load j of a step (a wave's are wave, wave + WAVES, ...) fills 1 KB of K (j < PIECES) or V, lane -> 16-byte piece; which piece of its row
+    // that is follows from the swizzle.  Rows past the last key read 0.
+    uint32_t off[OFFS];
 #pragma unroll
-        for (int i = 0; i < KPIECES; i++) {
-            const uint32_t idx = tid + NT * i, key = idx / (HD / 8), dc = idx % (HD / 8);
-            const uint32_t t = kt * KT + key;
-            kreg[i] = (idx < KTOTAL && t < seq_total) ? *reinterpret_cast<const int4*>(kc + (size_t)t * kv_stride + kvh * HD + dc * 8)
-                                                     : make_int4(0, 0, 0, 0);
-        }
-        // V: an item is 4 head dims of two consecutive keys (seq rows t, t+1)
+    for (uint32_t i = 0; i < OFFS; i++) {
+        const uint32_t p = (wave + WAVES * i) % PIECES * 64 + lane, row = p / PIECES;
+        off[i] = row * kv_stride * 2 + piece_of<HD>(row, p % PIECES) * 16;
+    }
+    auto load_tiles = [&](uint32_t kt, uint32_t buf) {
+        // a paged cache: a tile of 64 keys lies within one page (pages are multiples of 64 rows)
+        const size_t at = paged_row(pt, kt * KT) * kv_stride + kvh * HD;
+        const uint32_t records = (uint32_t)__builtin_amdgcn_readfirstlane((int)((min(seq_total - kt * KT, (uint32_t)KT) - 1) * kv_stride * 2 + ROW));
 #pragma unroll
-        for (int i = 0; i < VITEMS; i++) {
-            const uint32_t idx = tid + NT * i, kp = idx / DG, dg = idx % DG;
-            const uint32_t t = kt * KT + 2 * kp;
-            const uint16_t* src = vc + (size_t)t * kv_stride + kvh * HD + dg * 4;
-            va[i] = (idx < VTOTAL && t < seq_total) ? *reinterpret_cast<const uint2*>(src) : make_uint2(0, 0);
-            vb[i] = (idx < VTOTAL && t + 1 < seq_total) ? *reinterpret_cast<const uint2*>(src + kv_stride) : make_uint2(0, 0);
+        for (uint32_t i = 0; i < LOADS; i++) {
+            const uint32_t j = wave + WAVES * i;
+            const bool of_k = EVEN ? i < PIECES / WAVES : j < PIECES;
+            const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)((of_k ? kc_flat : vc_flat) + at), 0, records, AP_RSRC_FLAGS);
+            const uint32_t at_lane = off[i % OFFS];
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(r, FH_LDS3(smem + buf * 2 * TILE + j * 1024), 16, at_lane, 0, 0, 0);
         }
     };
-    auto store_tile = [&](uint32_t buf) {
-#pragma unroll
-        for (int i = 0; i < KPIECES; i++) {
-            const uint32_t idx = tid + NT * i, key = idx / (HD / 8), dc = idx % (HD / 8);
-            if (idx < KTOTAL) *reinterpret_cast<int4*>(Ks(buf) + key * KS + dc * 8) = kreg[i];
-        }
-        // V^T[d][key]: the two keys' values of one head dim side by side in a dword
-#pragma unroll
-        for (int i = 0; i < VITEMS; i++) {
-            const uint32_t idx = tid + NT * i, kp = idx / DG, dg = idx % DG;
-            if (idx < VTOTAL) {
-                uint32_t* vt = reinterpret_cast<uint32_t*>(Vt(buf) + (dg * 4) * VS + 2 * kp);
-                vt[0 * (VS / 2)] = __builtin_amdgcn_perm(vb[i].x, va[i].x, 0x05040100u);
-                vt[1 * (VS / 2)] = __builtin_amdgcn_perm(vb[i].x, va[i].x, 0x07060302u);
-                vt[2 * (VS / 2)] = __builtin_amdgcn_perm(vb[i].y, va[i].y, 0x05040100u);
-                vt[3 * (VS / 2)] = __builtin_amdgcn_perm(vb[i].y, va[i].y, 0x07060302u);
-            }
-        }
+    // Addresses of the fragments in LDS.  K (A operand): row lq, pieces 2 s + lh.  V (transposed while it is read: sixteen lanes fetch 4 keys x 16
+    // head dims and each ends up with the 4 keys of one dim): key 4 lh + (lane % 16) / 4, dims 16 ((lane / 16) % 2) + 4 (lane % 4) .. + 3.
+    auto k_frag = [&](const uint8_t* tile, int h, int s) {
+        return *reinterpret_cast<const v8h*>(tile + ((kh + h) * 32 + lq) * ROW + piece_of<HD>(lq, 2 * s + lh) * 16);
+    };
+    const uint32_t vrow = 4 * lh + ((lane & 15) >> 2), vpiece = 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1);
+    auto v_frag = [&](const uint8_t* tile, int key, int d) {       // keys key + 4 lh .. + 3 and key + 8 + 4 lh .. + 3
+        const uint8_t* at = tile + vrow * ROW + piece_of<HD>(vrow, 4 * d + vpiece) * 16 + (lane & 1) * 8 + key * ROW;
+        const v4h v0 = read_transposed(at), v1 = read_transposed(at + 8 * ROW);
+        return (v8h){v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
     };
 
-    load_tile(tile0);
-    store_tile(tile0 & 1);
-    __syncthreads();
+    load_tiles(tile0, tile0 & 1);
     for (uint32_t kt = tile0; kt < ntiles; kt++) {
         const uint32_t buf = kt & 1;
-        if (kt + 1 < ntiles) load_tile(kt + 1);          // in flight while this tile is computed
+        __builtin_amdgcn_s_waitcnt(0);       // this wave's share of the step's tiles is in LDS,
+        __syncthreads();                     // and so is everyone's; nobody reads the other buffer any more
+        if (kt + 1 < ntiles) load_tiles(kt + 1, buf ^ 1);
         const uint32_t k0 = kt * KT + kh * 32;            // this wave's first 32 keys of the tile
         constexpr uint32_t KW = 32 * KH;                  // keys of the tile this wave works
         if (wave_active && k0 <= wave_max_pos && k0 + KW > wave_lo) {   // else they lie entirely in the group's future, or before every window
-            const _Float16* Kb = Ks(buf);
-            const _Float16* Vb = Vt(buf);
+            const uint8_t* Kb = smem + buf * 2 * TILE;
+            const uint8_t* Vb = Kb + TILE;
             // ---- S^T tiles: sacc[h][r] = q . k for key k0 + 32 h + 8(r/4) + 4 lh + r%4, query lq
             v16f sacc[KH];
 #pragma unroll
@@ -175,8 +186,7 @@ void attn_prefill_kernel(const float* __restrict__ q, const uint16_t* __restrict
             for (int s = 0; s < NS; s++)
 #pragma unroll
                 for (int h = 0; h < KH; h++) {
-                    v8h kf = *reinterpret_cast<const v8h*>(Kb + ((kh + h) * 32 + lq) * KS + 16 * s + 8 * lh);
-                    sacc[h] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf, qf[s], sacc[h], 0, 0, 0);
+                    sacc[h] = __builtin_amdgcn_mfma_f32_32x32x16_f16(k_frag(Kb, h, s), qf[s], sacc[h], 0, 0, 0);
                 }
             // ---- causal mask: only keys past the group's first query can be masked for some query
             // with a window, also keys that the group's last query no longer sees
@@ -203,12 +213,22 @@ void attn_prefill_kernel(const float* __restrict__ q, const uint16_t* __restrict
             for (int h = 0; h < KH; h++)
 #pragma unroll
                 for (int r = 0; r < 16; r++) m_tile = fmaxf(m_tile, sacc[h][r]);
-            m_tile = lane_xor_max<32>(m_tile) * c2;      // c2 > 0: max commutes with the scaling
-            const float m_new = fmaxf(m_run, m_tile);
+            m_tile *= c2;                                // c2 > 0: max commutes with the scaling
+            // The maximum that scores are taken against follows only where some query of the wave has risen above it by more than SLACK: p stays
+            // below 2^SLACK, and l and O are relative to the same number whatever it is.
+            if (__builtin_amdgcn_ballot_w64(m_tile > m_run + SLACK) != 0) {
+                const float m_new = fmaxf(m_run, lane_xor_max<32>(m_tile));
+                const float alpha = m_run == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run - m_new);
+                l_run *= alpha;
+#pragma unroll
+                for (int d = 0; d < ND; d++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) oacc[d][r] *= alpha;
+                m_run = m_new;
+            }
             // a query that has seen no key yet (all of these keys masked for it) keeps m = -inf: exponentiate
             // against 0 instead, every p is then 2^-inf = 0
-            const float m_exp = m_new == -INFINITY ? 0.f : m_new;
-            float l_tile = 0.f;
+            const float m_exp = m_run == -INFINITY ? 0.f : m_run;
             v8h pb[KH][2];
 #pragma unroll
             for (int h = 0; h < KH; h++)
@@ -217,41 +237,24 @@ void attn_prefill_kernel(const float* __restrict__ q, const uint16_t* __restrict
 #pragma unroll
                     for (int e = 0; e < 8; e++) {
                         const float p = __builtin_amdgcn_exp2f(fmaf(sacc[h][8 * j + e], c2, -m_exp));   // 2^-inf = 0 for masked keys
-                        l_tile += p;
+                        l_run += p;
                         pb[h][j][e] = (_Float16)p;
                     }
-            // rescale what has been accumulated, unless no query of the wave saw a new maximum
-            if (__builtin_amdgcn_ballot_w64(m_new > m_run) != 0) {
-                const float alpha = m_run == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run - m_new);
-                l_run *= alpha;
-#pragma unroll
-                for (int d = 0; d < ND; d++)
-#pragma unroll
-                    for (int r = 0; r < 16; r++) oacc[d][r] *= alpha;
-            }
-            l_run += l_tile;
-            m_run = m_new;
             // ---- O^T += V^T P^T over this wave's keys
 #pragma unroll
             for (int h = 0; h < KH; h++)
 #pragma unroll
                 for (int j = 0; j < 2; j++)
 #pragma unroll
-                    for (int d = 0; d < ND; d++) {
-                        const _Float16* vrow = Vb + (d * 32 + lq) * VS + (kh + h) * 32 + 16 * j + 4 * lh;
-                        v4h v0 = *reinterpret_cast<const v4h*>(vrow);
-                        v4h v1 = *reinterpret_cast<const v4h*>(vrow + 8);
-                        v8h vf = (v8h){v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
-                        oacc[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, pb[h][j], oacc[d], 0, 0, 0);
-                    }
+                    for (int d = 0; d < ND; d++)
+                        oacc[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v_frag(Vb, (kh + h) * 32 + 16 * j, d), pb[h][j], oacc[d], 0, 0, 0);
         }
-        if (kt + 1 < ntiles) store_tile(buf ^ 1);   // nobody reads that buffer: its tile was finished before the last barrier
-        __syncthreads();
     }
 
     // ---- the two waves of a query group merge their halves: the odd one hands (m, l, O) over through LDS
     float* mg = reinterpret_cast<float*>(smem) + (qg * 64 + lane) * MERGE_FLOATS;
     if (KH == 1) {
+    __syncthreads();          // the tile buffers are free
     if (kh == 1) {
         mg[0] = m_run;
         mg[1] = l_run;
@@ -321,19 +324,18 @@ template <int HD, bool QUANT>
 void launch_win(dim3 grid, hipStream_t s, const float* q, const uint16_t* kc, const uint16_t* vc, float* out, uint32_t q_stride,
                 uint32_t out_stride, uint32_t M, uint32_t base_pos, uint32_t heads, uint32_t kv_heads, int8_t* oq, uint16_t* osc,
                 uint32_t window, PageTable pt) {
-    // The 4-wave form when there are clearly more workgroups than the machine holds at once (three per CU at head_dim 64,
-    // two above: then throughput decides, and a wave with two score tiles per step does 15-30 % more of it); the 8-wave form
-    // when they all fit (then the longest workgroup's chain of tile steps decides, and twice the waves halve its steps).
-    // Measured, 32 heads: 3001 tokens of head_dim 96 143 -> 108 us, 8192 tokens of head_dim 128 978 -> 842 us; 2502 tokens of
-    // head_dim 64 59 -> 67 us, which is why the count decides.  FORGE_HIP_ATTN_WAVES=8 / 4 forces one.
+    // The 4-wave form from two workgroups per CU on (then throughput decides, and a wave with two score tiles per step does more of it); the
+    // 8-wave form below (then the longest workgroup's chain of tile steps decides, and twice the waves halve its steps).  us, 4 waves / 8 waves:
+    // 256 workgroups 1000 rows of 32/8 heads of 128 27.1 / 25.2, 1024 behind 8192 of 32/32 of 96 176 / 161, of 32/8 of 64 117 / 108;
+    // 480 24/8 of 128 62.3 / 60.3, 32/32 of 96 38.8 / 39.4; 512 2048 behind 8192 of 64 192 / 197, of 96 269 / 264, of 128 321 / 334;
+    // 640 2502 rows of 64 44.0 / 44.6; 768 3001 rows of 96 75.0 / 79.1, of 128 89.8 / 105.  FORGE_HIP_ATTN_WAVES=8 / 4 forces one.
     static const int forced = [] { const char* e = getenv("FORGE_HIP_ATTN_WAVES"); return e ? atoi(e) : 0; }();
     static const int cus = [] {
         int dev = 0, n = 0;
         if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) n = 256;
         return n > 0 ? n : 256;
     }();
-    const uint32_t slots = (uint32_t)cus * (HD == 64 ? 3 : 2);
-    const bool four = forced == 4 || (forced != 8 && grid.x * 4 >= slots * 5);
+    const bool four = forced == 4 || (forced != 8 && grid.x >= 2 * (uint32_t)cus);
     // a window that covers every key of the call is plain causal attention
     const bool win = window != 0 && window < base_pos + M;
 #define FH_AP(WIN_, KH_) \

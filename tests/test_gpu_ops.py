@@ -588,6 +588,33 @@ def test_attention_prefill_parity(fh, oracle, torch_gpu, heads, kv_heads, hd, M,
     close(fh.ops.attention_flash_batch(qd, kd, vd, base, heads, kv_heads, hd, 0).cpu().numpy(), want, rtol=2e-3, atol=2e-3)
 
 
+@pytest.mark.parametrize("hd", [64, 96, 128])
+@pytest.mark.parametrize("heads,M,base,window,ramp", [
+    (64, 1025, 0, 0, 0.0), (64, 960, 37, 0, 0.06), (64, 1000, 0, 150, -0.06),      # four waves to a workgroup: 512 workgroups and more
+    (2, 129, 0, 0, 0.06), (2, 200, 63, 0, 3.0), (2, 191, 5, 70, -3.0),              # eight
+])
+def test_attention_prefill_running_maximum(fh, torch_gpu, hd, heads, M, base, window, ramp):
+    """Both forms of the prompt kernel, with scores that rise or fall along the keys (`ramp`: by how much per key, in powers of two): the maximum
+    that they are taken against follows late.  p is rounded to fp16 (2^-11), scores and sums are 32-bit: 2^-10 of the largest value is enough."""
+    torch = torch_gpu
+    g = torch.Generator(device="cuda").manual_seed(M + hd)
+    seq = base + M
+    q = torch.randn(M, heads, hd, generator=g, device="cuda").half().float()
+    k = torch.randn(seq, 2, hd, generator=g, device="cuda").half()
+    v = torch.randn(seq, 2, hd, generator=g, device="cuda").half()
+    q[..., 0] = 8.0
+    k[..., 0] = (torch.arange(seq, device="cuda")[:, None] * (ramp * hd ** 0.5 / 8.0 / 1.4426950408889634)).half()
+    args = (q.reshape(M, -1), k.reshape(seq, -1).view(torch.int16), v.reshape(seq, -1).view(torch.int16), base)
+    got = (fh.ops.attention_sliding_batch(*args, window, heads, 2, hd) if window else fh.ops.attention_flash_batch(*args, heads, 2, hd)).view(M, heads, hd)
+    pos, key = torch.arange(base, seq, device="cuda")[:, None], torch.arange(seq, device="cuda")[None, :]
+    hidden = (key > pos) | (key + window <= pos) if window else key > pos
+    for h in range(0, heads, 9):
+        kv = h * 2 // heads
+        sc = (q[:, h].double() @ k[:, kv].double().T) * hd ** -0.5
+        want = torch.softmax(sc.masked_fill(hidden, float("-inf")), -1) @ v[:, kv].double()
+        assert (got[:, h].double() - want).abs().max().item() <= 2.0 ** -10 * v.abs().max().item()
+
+
 @pytest.mark.parametrize("heads,kv_heads,hd", [(32, 8, 64), (9, 3, 64), (6, 6, 96), (24, 8, 128)])
 @pytest.mark.parametrize("seq,window", [(1, 1), (5, 3), (70, 1), (70, 64), (70, 70), (70, 4096), (900, 17), (900, 256), (900, 899)])
 def test_attention_sliding_decode_parity(fh, oracle, torch_gpu, heads, kv_heads, hd, seq, window):
