@@ -15,10 +15,9 @@
 // of a prompt of a few thousand tokens, 50 multiplications of about 190 VALU instructions each time).
 // What bounds it: full, the matrix unit, the VALU (32 exp, 32 FMA, 32 additions, 16 conversions, 16 maxima per 32 x 64 scores) and LDS reads
 // take about 800 cycles each and overlap to 1800 (heads of 96, 3072 queries behind 8192 keys 390 us = 0.94 PFLOP/s, 128 1.0, 64 0.9; the
-// library's large bf16 product is at 1.2); causal, the uneven length of the query tiles on top.  3001 tokens: 32/32 heads of 96 95.4 -> 75.1 us,
+// library's large bf16 product is at 1.2); causal, the uneven length of the query tiles on top.  3001 tokens: 32/32 heads of 96 97.7 -> 74.5 us,
 // 32/8 of 128 124 -> 89, 2502 tokens of 32/8 of 64 52.5 -> 42.7, 1000 of 32/8 of 128 38.2 -> 24.0.
-// Measured and not kept: waits of our own around the transposing reads (the compiler waits for the next tiles ahead of the first of them):
-// no faster; query tiles of every other round in ascending order: within 2 %.
+// Measured and not kept: query tiles of every other round in ascending order: within 2 %.
 //
 // Both products are computed transposed, S^T = K Q^T and O^T = V^T P^T.  In the 32x32 MFMA
 // result layout a lane then owns ONE query (column = lane%32) and 16 keys (or 16 head dims),
@@ -56,6 +55,28 @@ __device__ __forceinline__ uint32_t piece_of(uint32_t r, uint32_t p) {
 __device__ __forceinline__ v4h read_transposed(const uint8_t* at) {
     return __builtin_bit_cast(v4h, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s*)at));
 }
+
+// V fragments of 32 keys x 96 head dims in two rows of LDS `at`: f[j][d] = keys 16 j + 4 lh .. + 3 and + 8 of dim 32 d + lane % 32.  The compiler
+// waits for everything that is on its way into LDS ahead of a transposing read of its own, that is for the next tiles in the middle of a step.
+// Where K and V come from HBM, as they do with as many KV heads as heads (3001 tokens of 32/32 heads of 96, 110 MB), the step has to be given to
+// them whole: 82.8 us behind the compiler's waits, 77.8 behind these.  With shared heads they come out of a cache in time, and these waits,
+// which keep the reads from running ahead of the products, cost more (32/8 heads of 128 91.7 / 93.4, 12/2 49.1 / 53.3; of 64 43.0 / 43.4).
+#define FH_TR(dst, off) "ds_read_b64_tr_b16 " dst ", %[at] offset:" off "\n"
+#define FH_TR4(a, b, c, d, off) FH_TR(a, off) FH_TR(b, off "+%[k8]") FH_TR(c, off "+%[k8]*2") FH_TR(d, off "+%[k8]*3")
+__device__ __forceinline__ void read_v96(v8h (&f)[2][3], uint32_t at) {
+    v4h r[3][4];
+    asm volatile(FH_TR4("%[x00]", "%[x01]", "%[x02]", "%[x03]", "0") FH_TR4("%[x10]", "%[x11]", "%[x12]", "%[x13]", "64")
+                 FH_TR4("%[x20]", "%[x21]", "%[x22]", "%[x23]", "128") "s_waitcnt lgkmcnt(0)"
+                 : [x00] "=&v"(r[0][0]), [x01] "=&v"(r[0][1]), [x02] "=&v"(r[0][2]), [x03] "=&v"(r[0][3]), [x10] "=&v"(r[1][0]), [x11] "=&v"(r[1][1]),
+                   [x12] "=&v"(r[1][2]), [x13] "=&v"(r[1][3]), [x20] "=&v"(r[2][0]), [x21] "=&v"(r[2][1]), [x22] "=&v"(r[2][2]), [x23] "=&v"(r[2][3])
+                 : [at] "v"(at), [k8] "n"(8 * 192));
+#pragma unroll
+    for (int d = 0; d < 3; d++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) f[j][d] = __builtin_shufflevector(r[d][2 * j], r[d][2 * j + 1], 0, 1, 2, 3, 4, 5, 6, 7);
+}
+#undef FH_TR4
+#undef FH_TR
 
 // QUANT: instead of f32 rows the kernel writes what the o projection's GEMM reads, the activation quantiser's int8
 // codes oq[M][heads*HD] and fp16 scales osc[M][heads*HD/32] of the same values (a 32-element block is one 32-wide
@@ -99,22 +120,8 @@ void attn_prefill_kernel(const float* __restrict__ q, const uint16_t* __restrict
     // scores are kept in the base-2 domain: s * (scale * log2 e), so that exp is the bare v_exp_f32
     const float c2 = (1.0f / sqrtf((float)HD)) * 1.4426950408889634f;
 
-    // ---- Q fragment (B operand of S^T = K Q^T): lane (lq, lh) holds q[row][16 s + 8 lh + 0..7]
     const uint32_t qrow = q0 + qg * QW + lq;
     const uint32_t qpos = base_pos + qrow;
-    v8h qf[NS];
-#pragma unroll
-    for (int s = 0; s < NS; s++) {
-        if (qrow < M) {
-            const float4* p = reinterpret_cast<const float4*>(q + (size_t)qrow * q_stride + head * HD + 16 * s + 8 * lh);
-            float4 a = p[0], b = p[1];
-            qf[s] = (v8h){(_Float16)a.x, (_Float16)a.y, (_Float16)a.z, (_Float16)a.w,
-                          (_Float16)b.x, (_Float16)b.y, (_Float16)b.z, (_Float16)b.w};
-        } else {
-            qf[s] = (v8h){0, 0, 0, 0, 0, 0, 0, 0};
-        }
-    }
-
     v16f oacc[ND];
 #pragma unroll
     for (int d = 0; d < ND; d++)
@@ -159,13 +166,27 @@ void attn_prefill_kernel(const float* __restrict__ q, const uint16_t* __restrict
         return *reinterpret_cast<const v8h*>(tile + ((kh + h) * 32 + lq) * ROW + piece_of<HD>(lq, 2 * s + lh) * 16);
     };
     const uint32_t vrow = 4 * lh + ((lane & 15) >> 2), vpiece = 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1);
+    auto v_at = [&](const uint8_t* tile, int key, int d) { return tile + vrow * ROW + piece_of<HD>(vrow, 4 * d + vpiece) * 16 + (lane & 1) * 8 + key * ROW; };
     auto v_frag = [&](const uint8_t* tile, int key, int d) {       // keys key + 4 lh .. + 3 and key + 8 + 4 lh .. + 3
-        const uint8_t* at = tile + vrow * ROW + piece_of<HD>(vrow, 4 * d + vpiece) * 16 + (lane & 1) * 8 + key * ROW;
+        const uint8_t* at = v_at(tile, key, d);
         const v4h v0 = read_transposed(at), v1 = read_transposed(at + 8 * ROW);
         return (v8h){v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
     };
 
     load_tiles(tile0, tile0 & 1);
+    // ---- Q fragment (B operand of S^T = K Q^T): lane (lq, lh) holds q[row][16 s + 8 lh + 0..7].  All of it is requested at once (a row past the
+    // last takes the last one's): with a condition around each load they waited for one another (3001 tokens of 32/32 heads of 96 76.3 us, now 74.5).
+    v8h qf[NS];
+    {
+        const float4* p = reinterpret_cast<const float4*>(q + (size_t)min(qrow, M - 1) * q_stride + head * HD + 8 * lh);
+        float4 f[NS][2];
+#pragma unroll
+        for (int s = 0; s < NS; s++) { f[s][0] = p[4 * s]; f[s][1] = p[4 * s + 1]; }
+#pragma unroll
+        for (int s = 0; s < NS; s++)
+            qf[s] = (v8h){(_Float16)f[s][0].x, (_Float16)f[s][0].y, (_Float16)f[s][0].z, (_Float16)f[s][0].w,
+                          (_Float16)f[s][1].x, (_Float16)f[s][1].y, (_Float16)f[s][1].z, (_Float16)f[s][1].w};
+    }
     for (uint32_t kt = tile0; kt < ntiles; kt++) {
         const uint32_t buf = kt & 1;
         __builtin_amdgcn_s_waitcnt(0);       // this wave's share of the step's tiles is in LDS,
@@ -242,12 +263,17 @@ void attn_prefill_kernel(const float* __restrict__ q, const uint16_t* __restrict
                     }
             // ---- O^T += V^T P^T over this wave's keys
 #pragma unroll
-            for (int h = 0; h < KH; h++)
+            for (int h = 0; h < KH; h++) {
+                v8h vf[2][ND];
+                if constexpr (HD == 96) read_v96(vf, (uint32_t)(uintptr_t)FH_LDS3(v_at(Vb, (kh + h) * 32, 0)));
 #pragma unroll
                 for (int j = 0; j < 2; j++)
 #pragma unroll
-                    for (int d = 0; d < ND; d++)
-                        oacc[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v_frag(Vb, (kh + h) * 32 + 16 * j, d), pb[h][j], oacc[d], 0, 0, 0);
+                    for (int d = 0; d < ND; d++) {
+                        if constexpr (HD != 96) vf[j][d] = v_frag(Vb, (kh + h) * 32 + 16 * j, d);
+                        oacc[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[j][d], pb[h][j], oacc[d], 0, 0, 0);
+                    }
+            }
         }
     }
 
