@@ -98,6 +98,30 @@ def test_greedy_and_degenerate_settings(fh, oracle, so, n):
         assert tok == (first if n > 1 else 0)
 
 
+@pytest.mark.parametrize("n", [1, 31, 33, 511, 530, 4111, 60000])
+@pytest.mark.parametrize("kind", ["normal", "ties", "steps", "minus_inf"])
+def test_sample_equals_oracle_over_sizes(fh, oracle, so, n, kind):
+    """Blocks of 32 and 16 entries, both ways of sorting, equal numbers across the cut, a histogram that promises more than its entries hold
+    (steps: whole buckets of numbers at their lower edge), entries of probability zero."""
+    l = logits_of(fh, n, n)
+    if kind == "ties":
+        l = np.round(l)
+    elif kind == "steps":
+        l = (-np.float32(np.log(2.0)) * np.minimum(np.arange(n) % 4, np.arange(n))).astype(np.float32)
+        l[fh.synth.uniform_ids(5, n // 4 + 1, n)] = -np.inf
+        l[0] = 0.0
+    elif kind == "minus_inf":
+        l[fh.synth.uniform_ids(5, n // 2 + 1, n)] = -np.inf
+        l[n // 3] = 1.0
+    state_l = state_o = 0x1234567 + n
+    for temp, top_k, top_p in [(0.8, 0, 0.9), (1.0, 0, 0.67), (1.0, 0, 0.535), (1.0, 0, 0.8), (1.2, 0, 0.999), (0.9, 40, 1.0), (1.0, n // 2, 0.99), (1.1, n - 1, 1.0), (0.3, 0, 1.0), (0.6, 600, 0.5)]:
+        a, b = l.copy(), l.copy()
+        tok_l, state_l = fh.ops.sample(a, temp, top_k, top_p, state_l)
+        tok_o, state_o = so.sample(oracle, b, temp, top_k, top_p, state_o)
+        assert (tok_l, state_l) == (tok_o, state_o)
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
 @pytest.mark.parametrize("temp,top_k,top_p", [(1.0, 0, 1.0), (0.7, 0, 1.0), (0.8, 40, 1.0), (1.0, 0, 0.9), (0.7, 40, 0.9), (1.3, 5, 0.5),
                                                (0.5, 0, 0.3), (2.0, 1000, 0.99)])
 def test_sample_equals_oracle_and_brackets_r(fh, oracle, so, temp, top_k, top_p):
