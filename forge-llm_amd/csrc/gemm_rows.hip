@@ -3,7 +3,7 @@
 //
 // What bounds it: the weights' way from memory (each byte is used for a few rows only) and latency.  The tile kernel (gemm.hip) walks
 // the whole of K in one workgroup of 128 columns, about 1.1 us per 128-deep stage however few rows there are, on N / 128 workgroups.
-// Here a workgroup takes a 32 x 32 tile (two with the SiLU epilogue) and its waves share out K, each through a strip of LDS of its own:
+// Here a workgroup takes a 32 x 32 tile, or two of the same columns (twice that with the SiLU epilogue), and its waves share out K, each through a strip of LDS of its own:
 // no barrier until the waves' partial tiles meet at the end, where they are added in the order of K.
 // Block sums are exact (v_mfma_i32_32x32x32_i8, one quant block per instruction); the scales' products come from a rank-1
 // v_mfma_f32_32x32x8_f16, exact in f32.  Up to a depth of 4096 a block's sum is converted and added with one FMA: an error of 2e-7 of the
@@ -43,21 +43,21 @@ struct FewArgs {
     uint32_t inter;
 };
 
-// One workgroup: 32 rows of activations x 32 columns.  SILU: the matrix is [gate; up], a workgroup takes 32 gate columns and the up
+// One workgroup: 32 MT rows of activations x 32 columns.  SILU: the matrix is [gate; up], a workgroup takes 32 gate columns and the up
 // columns of the same indices and writes quantize(silu(gate) * up) as gemm.hip's epilogue does.
-template <bool Q4, int WAVES, bool SILU, bool BIASED>
+template <bool Q4, int WAVES, bool SILU, bool BIASED, int MT>
 __global__ __launch_bounds__(WAVES * 64) void gemm_rows_kernel(FewArgs a) {
     constexpr int NT = SILU ? 2 : 1, KW = WAVES / NT;         // column tiles; waves that share K of one
-    constexpr int THREADS = WAVES * 64, TILE = 1024;
+    constexpr int THREADS = WAVES * 64, TILE = 1024 * MT;
     constexpr int WB = Q4 ? 64 : 128;                         // bytes of a weight row in a step
-    constexpr int LA = 32 * 128, LB = 32 * WB;                // LDS bytes of a step's activation tile / weight tile
+    constexpr int LA = MT * 32 * 128, LB = 32 * WB;           // LDS bytes of a step's activation tiles / weight tile
     constexpr int WAVE_LDS = LA + LB;
     static_assert(WAVE_LDS >= TILE * 4, "a wave's strip holds its partial tile");
     __shared__ __attribute__((aligned(16))) uint8_t lds[WAVES * WAVE_LDS];
     const uint32_t tid = threadIdx.x, lane = tid & 63;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
     const uint32_t c = lane & 31, h = lane >> 5;
-    const uint32_t nblk = a.K / 32, n0 = blockIdx.x * 32, m0 = blockIdx.y * 32;
+    const uint32_t nblk = a.K / 32, n0 = blockIdx.x * 32, m0 = blockIdx.y * 32 * MT;
     const uint32_t steps = (nblk + FR_U - 1) / FR_U, each = (steps + KW - 1) / KW, per = BIASED ? (each + 1) & ~1u : each;
     const uint32_t s0 = min(steps, wave % KW * per), s1 = min(steps, s0 + per);
     const uint32_t col0 = n0 + (SILU ? wave / KW * a.inter : 0u);        // this wave's columns: rows col0 .. + 32 of the matrix
@@ -72,10 +72,10 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_rows_kernel(FewArgs a) {
     const __amdgpu_buffer_rsrc_t rws = __builtin_amdgcn_make_buffer_rsrc((void*)a.wsc, 0, a.N * nblk * 2, FR_RSRC);
     const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)a.aq, 0, a.M * a.K, FR_RSRC);
     const __amdgpu_buffer_rsrc_t ras = __builtin_amdgcn_make_buffer_rsrc((void*)a.asc, 0, a.M * nblk * 2, FR_RSRC);
-    constexpr int NLA = 4, NLB = Q4 ? 2 : 4;                  // loads of a step per tile: 8 rows (Q4_0 weights: 16) each
+    constexpr int NLA = 4 * MT, NLB = Q4 ? 2 : 4;                  // loads of a step per tile: 8 rows (Q4_0 weights: 16) each
     const uint32_t ar = lane >> 3, ap = lane & 7;
     const uint32_t br = Q4 ? lane >> 2 : lane >> 3, bp = Q4 ? lane & 3 : lane & 7;
-    struct Step { v4i A[NLA], B[NLB]; uint2 sa, sb; };
+    struct Step { v4i A[NLA], B[NLB]; uint2 sa[MT], sb; };
     // A row's four scales.  An even number of blocks to a row keeps them on 4-byte boundaries and the matrix's end on one; otherwise they
     // are fetched one by one (a word that reaches past the end reads as zero altogether).
     const bool odd_row = (nblk & 1u) != 0;
@@ -93,12 +93,15 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_rows_kernel(FewArgs a) {
         g.sb = load_scales(rws, (col0 + c) * nblk * 2 + st * 8);
 #pragma unroll
         for (int i = 0; i < NLA; i++) g.A[i] = __builtin_amdgcn_raw_buffer_load_b128(ra, (m0 + i * 8 + ar) * a.K + st * 128 + ap * 16, 0, 0);
-        g.sa = load_scales(ras, (m0 + c) * nblk * 2 + st * 8);
+#pragma unroll
+        for (int t = 0; t < MT; t++) g.sa[t] = load_scales(ras, (m0 + 32 * t + c) * nblk * 2 + st * 8);
     };
 
-    float acc[16];
+    float acc[MT][16];
 #pragma unroll
-    for (int r = 0; r < 16; r++) acc[r] = 0.f;
+    for (int t = 0; t < MT; t++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[t][r] = 0.f;
     v16i c_in;
 #pragma unroll
     for (int r = 0; r < 16; r++) c_in[r] = BIASED ? (int)FR_MAGIC : 0;
@@ -119,7 +122,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_rows_kernel(FewArgs a) {
     };
 
     auto compute = [&](Step& g, uint32_t st) {
-        g.sa = valid_scales(g.sa, st, false);
+#pragma unroll
+        for (int t = 0; t < MT; t++) g.sa[t] = valid_scales(g.sa[t], st, false);
         g.sb = valid_scales(g.sb, st, true);
 #pragma unroll
         for (int i = 0; i < NLA; i++) {
@@ -133,8 +137,6 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_rows_kernel(FewArgs a) {
         }
 #pragma unroll
         for (int u = 0; u < FR_U; u++) {
-            const v4i A = *reinterpret_cast<const v4i*>(la + c * 128 + (((2 * u + h) ^ ((c >> 1) & 7)) * 16));
-            const v4h fa = scale_operand(scale_of(g.sa, u));
             v4i B;
             if (Q4) {
                 const v4i p = *reinterpret_cast<const v4i*>(lb + c * WB + ((u ^ ((c >> 2) & 3)) * 16));
@@ -146,29 +148,38 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_rows_kernel(FewArgs a) {
                 B = *reinterpret_cast<const v4i*>(lb + c * WB + (((2 * u + h) ^ ((c >> 1) & 7)) * 16));
             }
             const v4h fb = scale_operand(scale_of(g.sb, u));
-            const v16i isum = __builtin_amdgcn_mfma_i32_32x32x32_i8(A, B, c_in, 0, 0, 0);
-            const v16f S = __builtin_amdgcn_mfma_f32_32x32x8f16(fa, fb, zero_f, 0, 0, 0);
-            const v16f biased = __builtin_bit_cast(v16f, isum);          // 12582912 +- block sum
 #pragma unroll
-            for (int r = 0; r < 16; r++) acc[r] = fmaf(S[r], BIASED ? biased[r] : (float)isum[r], acc[r]);
+            for (int t = 0; t < MT; t++) {
+                const v4i A = *reinterpret_cast<const v4i*>(la + (32 * t + c) * 128 + (((2 * u + h) ^ ((c >> 1) & 7)) * 16));
+                const v16i isum = __builtin_amdgcn_mfma_i32_32x32x32_i8(A, B, c_in, 0, 0, 0);
+                const v16f S = __builtin_amdgcn_mfma_f32_32x32x8f16(scale_operand(scale_of(g.sa[t], u)), fb, zero_f, 0, 0, 0);
+                const v16f biased = __builtin_bit_cast(v16f, isum);          // 12582912 +- block sum
+#pragma unroll
+                for (int r = 0; r < 16; r++) acc[t][r] = fmaf(S[r], BIASED ? biased[r] : (float)isum[r], acc[t][r]);
+            }
         }
         // the sums are final here: left alone, the compiler works on two steps' products at once and has no registers for them
 #pragma unroll
-        for (int r = 0; r < 16; r++) asm volatile("" : "+v"(acc[r]));
+        for (int t = 0; t < MT; t++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) asm volatile("" : "+v"(acc[t][r]));
     };
     // What eight blocks left of the bias, 1.5 * 2^23 * sum_b a_s[b] * (+-w_s[b]), off the sums: gemm.hip's f16 MFMA over the same eight
     // blocks (most of the biased sums' rounding is made here, and the same eight blocks make the same).
-    auto unbias = [&](uint2 a0, uint2 a1, uint2 w0, uint2 w1) {
+    auto unbias = [&](const uint2 (&a0)[MT], const uint2 (&a1)[MT], uint2 w0, uint2 w1) {
         const _Float16 af = (_Float16)(float)(1 << FR_A_LOG2);
         const _Float16 bf = h ? (_Float16)(-(float)(1 << (22 - FR_A_LOG2))) : (_Float16)(-(float)(1 << (23 - FR_A_LOG2)));
-        const v8h ta = __builtin_bit_cast(v8h, make_uint4(a0.x, a0.y, a1.x, a1.y)) * (v8h){af, af, af, af, af, af, af, af};
         const v8h tb = __builtin_bit_cast(v8h, make_uint4(w0.x, w0.y, w1.x, w1.y)) * (v8h){bf, bf, bf, bf, bf, bf, bf, bf};
-        v16f d;
 #pragma unroll
-        for (int r = 0; r < 16; r++) d[r] = acc[r];
-        d = __builtin_amdgcn_mfma_f32_32x32x16_f16(ta, tb, d, 0, 0, 0);
+        for (int t = 0; t < MT; t++) {
+            const v8h ta = __builtin_bit_cast(v8h, make_uint4(a0[t].x, a0[t].y, a1[t].x, a1[t].y)) * (v8h){af, af, af, af, af, af, af, af};
+            v16f d;
 #pragma unroll
-        for (int r = 0; r < 16; r++) acc[r] = d[r];
+            for (int r = 0; r < 16; r++) d[r] = acc[t][r];
+            d = __builtin_amdgcn_mfma_f32_32x32x16_f16(ta, tb, d, 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[t][r] = d[r];
+        }
     };
     // two steps in flight
     Step x0, x1;
@@ -176,22 +187,27 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_rows_kernel(FewArgs a) {
     if (s0 + 1 < s1) load(x1, s0 + 1);
     for (uint32_t st = s0; st < s1; st += 2) {
         compute(x0, st);
-        const uint2 a0 = x0.sa, w0 = x0.sb;
-        uint2 a1 = make_uint2(0u, 0u), w1 = a1;
+        uint2 a0[MT], a1[MT], w0 = x0.sb, w1 = make_uint2(0u, 0u);
+#pragma unroll
+        for (int t = 0; t < MT; t++) { a0[t] = x0.sa[t]; a1[t] = w1; }
         if (st + 2 < s1) load(x0, st + 2);
         if (st + 1 < s1) {
             compute(x1, st + 1);
-            a1 = x1.sa; w1 = x1.sb;
+#pragma unroll
+            for (int t = 0; t < MT; t++) a1[t] = x1.sa[t];
+            w1 = x1.sb;
         }
         if (st + 3 < s1) load(x1, st + 3);
         if (BIASED) unbias(a0, a1, w0, w1);
     }
 
-    // lane: column c, rows 8 (r / 4) + 4 h + r % 4 of the tile.  Element e = r * 64 + lane of a partial tile; the waves' partial tiles are
+    // lane: column c, rows 8 (r / 4) + 4 h + r % 4 of a tile of 32.  Element e = (16 t + r) * 64 + lane of a partial tile; the waves' partial tiles are
     // added in the order of K.
     float* red = reinterpret_cast<float*>(la);
 #pragma unroll
-    for (int r = 0; r < 16; r++) red[r * 64 + lane] = acc[r];
+    for (int t = 0; t < MT; t++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) red[(16 * t + r) * 64 + lane] = acc[t][r];
     __syncthreads();
     for (uint32_t e = tid; e < TILE; e += THREADS) {
         float v[NT];
@@ -206,7 +222,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_rows_kernel(FewArgs a) {
             if (Q4) v[j] *= 0.0625f;
         }
         const uint32_t r = e >> 6, el = e & 63, col = el & 31;
-        const uint32_t m = m0 + 8 * (r >> 2) + 4 * (el >> 5) + (r & 3);
+        const uint32_t m = m0 + 8 * (r >> 2) + 4 * (el >> 5) + (r & 3);       // (32 rows further on every 16 r)
         if (SILU) {
             // gemm.hip's epilogue: the 32 lanes of a half-wave are one block of one row
             const float o = v[0] * __builtin_amdgcn_rcpf(1.0f + __expf(-v[0])) * v[NT - 1];
@@ -227,12 +243,12 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_rows_kernel(FewArgs a) {
     }
 }
 
-template <bool Q4, bool SILU>
+template <bool Q4, bool SILU, int MT>
 void launch_rows(const FewArgs& a, hipStream_t s) {
     constexpr int WAVES = 8;       // sixteen leave a wave 128 registers, and two steps in flight do not fit them
-    const dim3 grid(((SILU ? a.inter : a.N) + 31) / 32, (a.M + 31) / 32);
-    if (a.K > 4096) fh::launch(gemm_rows_kernel<Q4, WAVES, SILU, true>, grid, WAVES * 64, 0, s, a);
-    else fh::launch(gemm_rows_kernel<Q4, WAVES, SILU, false>, grid, WAVES * 64, 0, s, a);
+    const dim3 grid(((SILU ? a.inter : a.N) + 31) / 32, (a.M + 32 * MT - 1) / (32 * MT));
+    if (a.K > 4096) fh::launch(gemm_rows_kernel<Q4, WAVES, SILU, true, MT>, grid, WAVES * 64, 0, s, a);
+    else fh::launch(gemm_rows_kernel<Q4, WAVES, SILU, false, MT>, grid, WAVES * 64, 0, s, a);
 }
 
 }  // namespace
@@ -242,24 +258,38 @@ bool gemm_rows_supported(const QWeight& w, uint32_t M, bool silu) {
     return (!silu || w.N % 64 == 0) && M <= 65535u * 32u && (uint64_t)M * w.K <= 0x7FFFFFFFull && (uint64_t)w.N * std::max<uint64_t>(w.qs_row_bytes(), w.K / 16) <= 0x7FFFFFFFull;
 }
 
+// Rounds of 256 tiles of 32 columns by 32 `mt` rows, one to a compute unit (a SiLU workgroup works two columns of them).
+static uint32_t rounds(const QWeight& w, uint32_t M, uint32_t mt) { return (uint32_t)(((uint64_t)((w.N + 31) / 32) * ((M + 32 * mt - 1) / (32 * mt)) + 255) / 256); }
+
+// Rows of tiles to a workgroup.  Two share the weights, their way through LDS and the nibbles' arithmetic: a round takes 1.6 times as long
+// (1.4 to 1.7; 1.8 where the sums are biased), so they pay where they save more than that in rounds.  us with the quantiser, one row of tiles / two, Q4_0: 2048 -> 8192 by 33
+// rows 12.4 / 10.6, 64 13.1 / 11.4, 65 (3 rounds against 2) 17.2 / 17.6, 100 21.9 / 18.5; 8192 -> 2048 by 128 17.4 / 22.6, by 256 31.5 / 27.1; 3072 -> 1024
+// by 300 15.5 / 13.9.  The same bits either way.
+static double two_rows_take(const QWeight& w) { return w.K > 4096 ? 1.8 : 1.6; }
+static uint32_t tile_rows(const QWeight& w, uint32_t M) { return two_rows_take(w) * rounds(w, M, 2) < rounds(w, M, 1) ? 2 : 1; }
+
 // Microseconds of a launch, for the choice between the kernels.  Tiles come in rounds of one to a compute unit; a round takes 1.8 plus 2.7 per
 // 2048 of depth, or what its columns take from memory at 4.8 TB/s (with the quantiser, 1 / 2 / 3 / 4 rounds: K = 2048 9.9 / 14.2 / 18.8 / 23.5,
-// K = 4096 13 / 20 / 27 / 34, K = 8192 17.5 / 29 / 40 / 52).  1422 products of 2 to 1300 rows were timed both ways: the kernel that the estimates
-// prefer is within 3 % of the faster one in all but 9, within 8 % in all.  A SiLU workgroup works two tiles.
+// K = 4096 13 / 20 / 27 / 34, K = 8192 17.5 / 29 / 40 / 52).  1422 products of 2 to 1300 rows were timed both ways, with one row of tiles to a
+// workgroup: the kernel that the estimates prefer is within 3 % of the faster one in all but 9, within 8 % in all.
 double gemm_rows_cost(const QWeight& w, uint32_t M) {
-    const uint64_t tiles = (uint64_t)((w.N + 31) / 32) * ((M + 31) / 32);
+    const uint32_t mt = tile_rows(w, M);
     const double columns = std::min<uint32_t>(w.N, 256 * 32), row_bytes = (double)w.qs_row_bytes() + w.K / 16;
-    return 2.0 + (double)((tiles + 255) / 256) * std::max(1.8 + 2.7 * w.K / 2048.0, columns * row_bytes / 4.8e6);
+    return 2.0 + (double)rounds(w, M, mt) * std::max((mt == 2 ? two_rows_take(w) : 1.0) * (1.8 + 2.7 * w.K / 2048.0), columns * row_bytes / 4.8e6);
 }
 
 void launch_gemm_rows(const QWeight& w, const int8_t* aq, const uint16_t* as, uint32_t M, float* y, uint32_t ldy, bool accumulate, hipStream_t s,
                       int8_t* silu_q, uint16_t* silu_sc) {
     const FewArgs a{w.qs, w.scales, aq, as, y, M, w.N, w.K, ldy, accumulate ? 1u : 0u, silu_q, silu_sc, w.N / 2};
     const bool q4 = w.wdtype == FORGE_HIP_Q4_0, silu = silu_q != nullptr;
-    if (q4 && silu) launch_rows<true, true>(a, s);
-    else if (q4) launch_rows<true, false>(a, s);
-    else if (silu) launch_rows<false, true>(a, s);
-    else launch_rows<false, false>(a, s);
+    auto go = [&](auto q4_, auto silu_) {
+        if (tile_rows(w, M) == 2) launch_rows<decltype(q4_)::value, decltype(silu_)::value, 2>(a, s);
+        else launch_rows<decltype(q4_)::value, decltype(silu_)::value, 1>(a, s);
+    };
+    if (q4 && silu) go(std::true_type{}, std::true_type{});
+    else if (q4) go(std::true_type{}, std::false_type{});
+    else if (silu) go(std::false_type{}, std::true_type{});
+    else go(std::false_type{}, std::false_type{});
 }
 
 }  // namespace fh

@@ -258,7 +258,8 @@ def test_matmul_mat_tiles_at_their_edges(fh, torch_gpu, wd, M, K, N):
 
 
 @pytest.mark.parametrize("wd", [Q8, Q4])
-@pytest.mark.parametrize("M,K,N", [(1, 288, 5), (2, 416, 32), (31, 544, 33), (32, 576, 64), (33, 2048, 100), (64, 1120, 31), (70, 4096, 512), (33, 4128, 40), (5, 8192, 96)])
+@pytest.mark.parametrize("M,K,N", [(1, 288, 5), (2, 416, 32), (31, 544, 33), (32, 576, 64), (33, 2048, 100), (64, 1120, 31), (70, 4096, 512), (33, 4128, 40), (5, 8192, 96),
+                                   (33, 2048, 4100), (64, 288, 4127), (70, 4128, 2750), (97, 416, 2100)])      # two rows of tiles to a workgroup
 def test_matmul_mat_few_rows(fh, torch_gpu, wd, M, K, N):
     """Few rows (32 x 32 tiles, K shared out to the waves): edges of the tiles, depths that are no multiple of a step or of the
     waves, against the order-faithful product.  Both add the same exact block terms t_b; sums of n terms differ by at most
@@ -278,6 +279,7 @@ def test_matmul_mat_few_rows(fh, torch_gpu, wd, M, K, N):
         bound += 3.0 * 2.0 ** -24 * 13.1e6 * (a_s @ w_s.T)
     assert (np.abs(fast.cpu().numpy().astype(np.float64) - exact.cpu().numpy()) <= bound).all()
     same_bits(fh.ops.matmul_mat_q(w, x).cpu().numpy(), fast.cpu().numpy())
+    same_bits(fh.ops.matmul_mat_q(w, x[M // 2:].contiguous()).cpu().numpy(), fast[M // 2:].cpu().numpy())      # whichever rows a workgroup has
 
 
 @pytest.mark.parametrize("ty", [Q8, Q4, 12, 14])
@@ -387,7 +389,7 @@ def test_matmul_mat_k_ranges_of_leftover_tiles(fh, torch_gpu, wd, M, K, N):
 
 
 @pytest.mark.parametrize("wd", [Q8, Q4])
-@pytest.mark.parametrize("M,K,I", [(2502, 2048, 8192), (37, 576, 1536), (300, 256, 64), (700, 3072, 1024), (65, 8192, 128), (515, 576, 1472), (1000, 288, 2112)])
+@pytest.mark.parametrize("M,K,I", [(2502, 2048, 8192), (37, 576, 1536), (300, 256, 64), (700, 3072, 1024), (65, 8192, 128), (515, 576, 1472), (1000, 288, 2112), (40, 288, 2112)])
 def test_gate_up_matmul_with_silu_and_quantiser_in_the_epilogue(fh, oracle, torch_gpu, wd, M, K, I):
     """forge_hip_gemm_silu_q: gate / up matmuls (fast arithmetic), silu(gate) * up and the activation quantiser in one kernel.
     Checked against the order-faithful matmul (bit-identical to the CPU path, see above) followed by silu_mul and the
