@@ -214,6 +214,9 @@ bool gemm_rows_supported(const QWeight& w, uint32_t M, bool silu);
 double gemm_rows_cost(const QWeight& w, uint32_t M);
 void launch_gemm_rows(const QWeight& w, const int8_t* aq, const uint16_t* as, uint32_t M, float* y, uint32_t ldy, bool accumulate, hipStream_t s,
                       int8_t* silu_q, uint16_t* silu_sc);
+// gemm_order.hip -- the same for the order-faithful mode
+bool gemm_order_pays(const QWeight& w, uint32_t M);
+void launch_gemm_order(const QWeight& w, const int8_t* aq, const uint16_t* as, uint32_t M, float* y, uint32_t ldy, bool accumulate, hipStream_t s);
 
 // llama.hip — the part of forge_hip_model_create's checks that sizes depend on (formats, dimensions the kernels cover);
 // sets the error message.

@@ -624,6 +624,10 @@ void launch_gemm(const QWeight& w, const int8_t* aq, const uint16_t* as, uint32_
     const bool silu = silu_q != nullptr;      // caller: gemm_silu_supported, fast mode, no block-sum dump
     const int accf = accumulate ? 1 : 0;
     const bool q4 = w.wdtype == FORGE_HIP_Q4_0;
+    if (exact && !isums && gemm_order_pays(w, M)) {
+        launch_gemm_order(w, aq, as, M, y, ldy, accumulate, s);
+        return;
+    }
     const uint64_t LIMIT = 0x7FFFFFFFull - 2 * BK;
     const uint64_t nblk = w.K / 32;
     const uint64_t per_m = std::max<uint64_t>(w.K, (uint64_t)ldy * 4);

@@ -239,6 +239,23 @@ def test_matmul_mat_parity(fh, oracle, torch_gpu, wd, M, K, N):
 
 
 @pytest.mark.parametrize("wd", [Q8, Q4])
+@pytest.mark.parametrize("M,K,N", [(1, 32, 4), (2, 96, 12), (15, 128, 64), (16, 160, 16), (17, 288, 68), (33, 416, 132), (32, 576, 576), (31, 1088, 100), (20, 1120, 20),
+                                   (50, 2048, 60), (5, 4128, 36), (150, 8192, 24), (300, 64, 48), (300, 576, 1532), (64, 2048, 4100)])
+def test_matmul_mat_order_of_few_rows(fh, oracle, torch_gpu, wd, M, K, N):
+    """Order-faithful products of few rows (16 x 16 results to a wave, steps of four blocks): edges of the tiles, depths of less than a step and of
+    a step and a part, rows whose scales lie between two words.  The oracle's bits, whatever lies behind the operands."""
+    torch = torch_gpu
+    wraw = make_weight(fh, wd, N, K, seed=3 * N + K + M)
+    x = fh.synth.normal(29 + K, M * K, 1.0).reshape(M, K)
+    x[M // 2, :32] = 0.0
+    w = fh.ops.QWeight(wd, wraw, K, N)
+    xd = torch.from_numpy(x).cuda()
+    got = fh.ops.matmul_mat_q(w, xd, EXACT)
+    same_bits(got.cpu().numpy(), oracle.matmul_mat(wd, 0, x, wraw, M, K, N))
+    w.close()
+
+
+@pytest.mark.parametrize("wd", [Q8, Q4])
 @pytest.mark.parametrize("M,K,N", [(1000, 1088, 2100), (515, 576, 2060), (330, 8256, 2100), (2050, 1152, 3073)])
 def test_matmul_mat_tiles_at_their_edges(fh, torch_gpu, wd, M, K, N):
     """Fast mode, products that stay on the tile kernel (128- and 64-row tiles, without and with K ranges): rows and columns that are no multiple of
