@@ -644,6 +644,27 @@ uint32_t attn_exact_one_launch_rows(uint32_t hd) { return hd <= 64 ? 768u : 256u
 // Longest window (rows whose scores one workgroup keeps in LDS) the order-faithful decode attention takes.
 uint32_t attn_exact_max_window() { return 12288; }
 
+// Rows of a workgroup of attn_exact_batch_group_kernel, whose one wave carries up to 16 queries.  Fewer of them make its walk over the key blocks
+// shorter (a block takes about 110 + 10 per four queries + 8 per query with heads of 64, 190 + 40 + 20 with wider ones, in units of 65 ns) and
+// the walks more: the cheapest estimate of the longest walk, of the shortest one times the rounds of what the chip holds, and of all walks
+// together.  us, as many rows as fit / what this takes: 9/3 heads of 64 by 32 rows 33.2 / 17.2, by 902 333 / 184, 24/8 of 128 by 64 73.6 / 35.0,
+// 32/32 of 96 by 32 65.9 / 24.1, 32/8 of 64 by 500 behind 700 444 / 318 (one row: 365).
+static uint32_t group_rows(bool batch_order, uint32_t M, uint32_t base_pos, uint32_t heads, uint32_t kv_heads, uint32_t hd) {
+    const uint32_t G = heads / kv_heads, most = 16 / G;
+    const double fixed = hd == 64 ? 110 : 190, four = hd == 64 ? 10 : 40, one = hd == 64 ? 8 : 20;
+    const double room = hd == 64 ? 2800 : batch_order ? 2048 : 1024;      // waves the chip holds (by their registers)
+    const double longest = (double)base_pos + M, mean = base_pos + 0.5 * M;
+    uint32_t best = most;
+    double least = INFINITY;
+    for (uint32_t r = most; r >= 1; r--) {
+        const double waves = (double)kv_heads * ((M + r - 1) / r);
+        const double keys = std::max(longest, std::max(base_pos * ceil(waves / room), 1.2 * waves * mean / room));
+        const double cost = keys * (fixed + four * ((r * G + 3) / 4) + one * r * G);
+        if (cost < least) { least = cost; best = r; }
+    }
+    return best;
+}
+
 void launch_attn_exact(bool batch_order, const float* q, uint32_t q_stride, const uint16_t* kc, const uint16_t* vc,
                        float* out, uint32_t out_stride, int8_t* oq, uint16_t* osc, uint32_t M, uint32_t base_pos,
                        const uint32_t* pos_dev, uint32_t heads, uint32_t kv_heads, uint32_t hd, uint32_t window, uint32_t max_rows,
@@ -679,7 +700,7 @@ void launch_attn_exact(bool batch_order, const float* q, uint32_t q_stride, cons
     // 16 heads per KV head; FORGE_HIP_EXACT_GROUP=0: the one-query kernel)
     static const bool group_ok = [] { const char* e = getenv("FORGE_HIP_EXACT_GROUP"); return !(e && e[0] == '0'); }();
     if (group_ok && window == 0 && M > 1 && out && !oq && !pos_dev && heads / kv_heads <= 16) {
-        const uint32_t rows_per_wg = 16 / (heads / kv_heads);
+        const uint32_t rows_per_wg = group_rows(batch_order, M, base_pos, heads, kv_heads, hd);
         dim3 gg(kv_heads, (M + rows_per_wg - 1) / rows_per_wg);
 #define FH_AXG(HD_, B_) \
     fh::launch(attn_exact_batch_group_kernel<HD_, B_>, gg, 64, 0, s, q, q_stride, kc, vc, out, out_stride, base_pos, M, heads, kv_heads, rows_per_wg)
