@@ -20,6 +20,66 @@ template <typename T> constexpr uint32_t gemv_unroll() { return sizeof(T) == 2 ?
 // matrix columns that the waves of a row group work in one step
 template <typename T, int KS> constexpr uint32_t gemv_step() { return gemv_unroll<T>() * KS * 512; }
 
+// The epilogue of a wave's four rows, an element to a lane (lanes 0 to 3; pairs: 0 and 1).  What it reads is requested ahead of the weights: at
+// the end it is a round trip of its own, two where the position stands between (rotations), and one lane working all four elements takes four
+// times as long over their exponentials.  The operations are dense_epilogue's.
+template <typename T, DenseEpi MODE>
+struct RowEpilogue {
+    float pw = 0.f, pb = 0.f, nw = 0.f, nb = 0.f, x = 0.f;      // Residual: the norms' weights, the stream; Rope: cosine and sine in pw, pb
+    T gate = (T)0.0f;
+    uint32_t n0, i, pair = 0, pos = 0;
+    bool rotates = false;
+
+    __device__ __forceinline__ RowEpilogue(const DenseEpiArgs& e, uint32_t n0_, uint32_t N, uint32_t lane) : n0(n0_), i(lane & 3) {
+        const uint32_t n = min(n0 + i, N - 1);
+        if constexpr (MODE == DenseEpi::Residual) {
+            if (e.post.w) { pw = e.post.w[n]; pb = e.post.b[n]; }
+            if (e.next.w) { nw = e.next.w[n]; nb = e.next.b[n]; }
+            if (e.add) x = e.f32[n];
+        }
+        if constexpr (MODE == DenseEpi::GateMul) gate = ((const T*)e.gate)[n];
+        if constexpr (MODE == DenseEpi::Rope) {
+            const uint32_t j = n0 % e.head_stride;
+            pair = (j - e.rot_off) / 2 + (i >> 1);
+            rotates = j >= e.rot_off && pair < e.rot_pairs;
+            pos = e.pos_dev ? *e.pos_dev : e.base_pos;
+        }
+    }
+    // behind the weights' requests: what an address had to be waited for
+    __device__ __forceinline__ void late(const DenseEpiArgs& e) {
+        if constexpr (MODE == DenseEpi::Rope) {
+            if (rotates) { pw = e.cos_t[(size_t)pos * e.rot_pairs + pair]; pb = e.sin_t[(size_t)pos * e.rot_pairs + pair]; }
+        }
+    }
+    __device__ __forceinline__ void store(const DenseEpiArgs& e, uint32_t N, uint32_t lane, const float (&v)[4]) const {
+        if (lane >= 4) return;
+        const uint32_t n = n0 + i;
+        float a = i == 0 ? v[0] : i == 1 ? v[1] : i == 2 ? v[2] : v[3];
+        if constexpr (MODE == DenseEpi::F32) {
+            if (n < N) e.f32[n] = e.cap > 0.f ? e.cap * tanhf(a / e.cap) : a;
+        } else if constexpr (MODE == DenseEpi::RawGate) {
+            if (n0 < e.split) e.f32[n] = a;
+            else ((T*)e.out)[n - e.split] = (T)act_f(e.act, a);
+        } else if constexpr (MODE == DenseEpi::Rope) {
+            const float b = i == 0 ? v[1] : i == 1 ? v[0] : i == 2 ? v[3] : v[2];
+            if (rotates) a = i & 1 ? a * pw + b * pb : a * pw - b * pb;
+            ((T*)e.out)[n] = (T)a;
+        } else if constexpr (MODE == DenseEpi::GateMul) {
+            ((T*)e.out)[n] = (T)(a * (float)gate);
+        } else if constexpr (MODE == DenseEpi::ActPair) {
+            if (i < 2) ((T*)e.out)[n0 / 2 + i] = (T)(act_f(e.act, i ? v[2] : v[0]) * (i ? v[3] : v[1]));
+        } else {
+            static_assert(MODE == DenseEpi::Residual, "the modes of a row");
+            if (e.post.w) a = tanhf(e.post.alpha * a) * pw + pb;
+            a += x;
+            e.f32[n] = a;
+            if (!e.out) return;
+            if (e.next.w) a = tanhf(e.next.alpha * a) * nw + nb;
+            ((T*)e.out)[n] = (T)a;
+        }
+    }
+};
+
 // xs: LDS, K floats, filled by `prologue`; red: LDS, 16 floats.  STEPS = 1: K <= gemv_step.
 template <typename T, int KS, DenseEpi MODE, int STEPS, typename Prologue>
 __device__ __forceinline__ void gemv_body(const T* __restrict__ w, uint32_t N, uint32_t K, uint32_t row0, float* xs, float* red,
@@ -58,10 +118,12 @@ __device__ __forceinline__ void gemv_body(const T* __restrict__ w, uint32_t N, u
     };
     x8 va[U][4], vb[U][4];
     constexpr uint32_t D = U * STEP;
+    RowEpilogue<T, MODE> epilogue(e, n0, N, lane);
     __builtin_amdgcn_sched_barrier(0);
     fetch(va, k_lane);
     if constexpr (STEPS > 1) fetch(vb, k_lane + D);
     __builtin_amdgcn_sched_barrier(0);
+    epilogue.late(e);
     prologue();
     __syncthreads();
     if constexpr (STEPS == 1) add(va, k_lane);
@@ -87,7 +149,7 @@ __device__ __forceinline__ void gemv_body(const T* __restrict__ w, uint32_t N, u
             for (int i = 0; i < 4; i++)
                 if (part == 0) acc[i] += red[(wave + p) * 4 + i];
     }
-    if (part == 0 && lane == 0 && n0 < N) dense_epilogue<T, MODE>(e, 0, n0, N, acc, epilogue_cols<MODE>(e, n0), epilogue_row<T, MODE>(e, 0, n0));
+    if (part == 0 && n0 < N) epilogue.store(e, N, lane, acc);
 }
 
 // Depth split of an N-row matrix: as many waves per row group as it takes to have a few workgroups on every compute unit.
