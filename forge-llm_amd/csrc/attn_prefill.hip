@@ -10,8 +10,8 @@
 // ds_read_b64_tr_b16 transposes on the way out.  (Through registers, with V transposed on the way in, a third of a step went into issuing the
 // loads and writing them to LDS, and the registers they took left two waves per SIMD where three fit now.)
 // Scores stay in the base-2 domain (s * scale * log2 e) so that the exponential is one v_exp_f32 after one FMA; keys are masked only in
-// tiles that reach past the wave's first query; the maximum that scores are taken against, and the accumulators with it, move only when
-// some query of the wave has risen above it by more than 2^SLACK (before: whenever it rose, which with 32 queries to a wave is most steps
+// tiles that reach past the wave's first query; the maximum that a query's scores are taken against, and its accumulators with it, move only
+// when one rises above it by more than 2^SLACK (before: whenever it rose, which with 32 queries to a wave is most steps
 // of a prompt of a few thousand tokens, 50 multiplications of about 190 VALU instructions each time).
 // What bounds it: full, the matrix unit, the VALU (32 exp, 32 FMA, 32 additions, 16 conversions, 16 maxima per 32 x 64 scores) and LDS reads
 // take about 800 cycles each and overlap to 1800 (heads of 96, 3072 queries behind 8192 keys 390 us = 0.94 PFLOP/s, 128 1.0, 64 0.9; the
@@ -234,11 +234,12 @@ void attn_prefill_kernel(const float* __restrict__ q, const uint16_t* __restrict
             for (int h = 0; h < KH; h++)
 #pragma unroll
                 for (int r = 0; r < 16; r++) m_tile = fmaxf(m_tile, sacc[h][r]);
-            m_tile *= c2;                                // c2 > 0: max commutes with the scaling
-            // The maximum that scores are taken against follows only where some query of the wave has risen above it by more than SLACK: p stays
-            // below 2^SLACK, and l and O are relative to the same number whatever it is.
-            if (__builtin_amdgcn_ballot_w64(m_tile > m_run + SLACK) != 0) {
-                const float m_new = fmaxf(m_run, lane_xor_max<32>(m_tile));
+            m_tile = lane_xor_max<32>(m_tile) * c2;      // c2 > 0: max commutes with the scaling
+            // The maximum that a query's scores are taken against follows only where one has risen above it by more than SLACK: p stays below 2^SLACK,
+            // and l and O are relative to the same number whatever it is.  (Each query by itself: its result does not depend on its neighbours.)
+            const bool risen = m_tile > m_run + SLACK;
+            if (__builtin_amdgcn_ballot_w64(risen) != 0) {
+                const float m_new = risen ? m_tile : m_run;
                 const float alpha = m_run == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run - m_new);
                 l_run *= alpha;
 #pragma unroll
