@@ -20,6 +20,7 @@
 //   SmolLM2-135M Q8_0   33: 781 / 880 / 384    300: 820 / 878 / 421    740: 907 / 876 / 466
 //   1B shape Q8_0       33: 754 / 610 / 469 and 433 (order-faithful, fast)    200: - / 636 / 476 and 441       Q4_0, fast: 33: 532 / 403
 //   and in fast mode (PaPart) 300: 637 / 464    1000: 642 / 471    2400: 644 / 479    5000: 676 / 515    Q4_0 2400: 570 / 442
+//   and of Q4_K / Q6_K matrices (llama.cpp's Q4_K_M recipe), 1B shape 33: 623 / 489    300: 646 / 527    2400: 655 / 543    5000: 688 / 580
 // Heads of 96 and 128 gain as much though those of 128 spill (8 layers, 33 rows, fast: 8/2 of 96 at 768 channels 213 / 136, 6/2 of 128 207 / 138, 16/4 of 96 at 1536 246 / 174,
 // 12/4 of 128 at 1024 212 / 168).  A layer's weights hardly count (1B shape, us: Q8_0 23, Q4_0 22): it is the chain that takes the time.
 #include <stddef.h>
@@ -53,6 +54,11 @@ constexpr uint32_t PA_SUM = 24, PA_SSQ = 12;  // a row's products, and an accumu
 //   them hold no rows of q;k;v and o, and their fetching waves attend, to up to 256 rows (longer contexts, order free: every workgroup's, PaPart).  down takes the place of the second set when that is done.
 struct PaNarrow { static constexpr int UQ = 1, UO = 1, UG1 = 3, UG2 = 0, UD = 1, UL = 4, NX = 3, NV = 3; static constexpr uint32_t AW = PA_WAVES; static constexpr bool WIDE = false; };
 struct PaWide { static constexpr int UQ = 2, UO = 2, UG1 = 4, UG2 = 4, UD = 4, UL = 4, NX = 8, NV = 9; static constexpr uint32_t AW = PA_POLL; static constexpr bool WIDE = true; };
+
+// How a matrix's blocks of 32 weights lie in memory.  Q8, Q4: as for every other kernel.  KQ: Q4_K and Q6_K alike, made by pa_create: the codes as int8 in order
+// (0 .. 15 and -32 .. 31) and a word: fp16 bits of d (Q4_K, odd blocks: of dmin) | an int8 scale << 16 | Q6_K: the second half's << 24, Q4_K: the minimum << 24.
+// (Codes of 4 bits would be half the bytes and no faster: a layer's weights hardly count here.)
+enum PaFmt : int { PA_Q8, PA_Q4, PA_KQ };
 
 // magic: floor(2^32 / nblk) + 1; R: rows per wave; wg0: the first workgroup with rows; stride: words between two rows of products; prod: the first wave's area of
 // them (LDS bytes), dump: a word behind it that nobody reads; fold: log2 of the lanes that add a row up where the order is free
@@ -95,6 +101,8 @@ struct PaArgs {
     uint32_t host_seq;
     unsigned long long* stamps;               // optional: wall clock between the phases, each from a workgroup that has done the phase before
     uint32_t off_as, off_xs, off_out, off_silu, off_prod, off_layers, off_attn, off_rec, prod_words, lds_words, xstride;      // LDS byte offsets (activation codes at 0)
+    uint32_t to_sums;                         // KQ: from the activation scales to the blocks' sums of codes
+    uint32_t six[5], six_v;                   // KQ: which matrices are Q6_K; the v rows of q;k;v have a format of their own
 };
 
 // A uniform base and a lane's 32-bit offset in bytes.
@@ -147,22 +155,23 @@ __device__ __forceinline__ void pa_poll(Addr addr, Tag tag, uint32_t* out, const
 }
 
 // A wave's blocks of a matrix: n of them, row after row; from block `seg` on they lie `jump` blocks further (the up rows of gate;up).
-struct PaTask { uint32_t base, n, seg, jump; };
+// six: KQ, 1 for Q6_K.
+struct PaTask { uint32_t base, n, seg, jump, six; };
 __device__ __forceinline__ uint32_t pa_sgpr(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
 __device__ __forceinline__ uint32_t pa_rows(const PaMat& m, uint32_t wv) { return wv * m.R < m.N ? min(m.R, m.N - wv * m.R) : 0u; }
-__device__ __forceinline__ PaTask pa_task(const PaMat& m, uint32_t wv) {
+__device__ __forceinline__ PaTask pa_task(const PaMat& m, uint32_t wv, uint32_t six = 0) {
     const uint32_t rows = pa_rows(m, wv);
-    return PaTask{rows ? wv * m.R * m.nblk : 0u, rows * m.nblk, 0xFFFFFFFFu, 0u};
+    return PaTask{rows ? wv * m.R * m.nblk : 0u, rows * m.nblk, 0xFFFFFFFFu, 0u, six};
 }
 
-// Lane l of round j holds block 64 j + l (Q4_0), or halves of two blocks with Q8_0: of blocks 64 j + l / 2 and 64 j + 32 + l / 2 the half
+// Lane l of round j holds block 64 j + l (Q4), or halves of two blocks (Q8, KQ): of blocks 64 j + l / 2 and 64 j + 32 + l / 2 the half
 // l & 1, so that a load covers consecutive bytes; the sums of both halves meet by a move between neighbours.
-template <int U, bool Q4> struct PaSet { int4 v[Q4 ? U : 2 * U]; uint32_t s[U]; };
-template <bool Q4>
-__device__ __forceinline__ uint32_t pa_own(uint32_t j, uint32_t lane) { return Q4 ? 64 * j + lane : 64 * j + 32 * (lane & 1u) + (lane >> 1); }
+template <int U, PaFmt W> struct PaSet { int4 v[W == PA_Q4 ? U : 2 * U]; uint32_t s[U]; };
+template <PaFmt W>
+__device__ __forceinline__ uint32_t pa_own(uint32_t j, uint32_t lane) { return W == PA_Q4 ? 64 * j + lane : 64 * j + 32 * (lane & 1u) + (lane >> 1); }
 
-template <int J0 = 0, int U, bool Q4>
-__device__ __forceinline__ void pa_load(PaSet<U, Q4>& w, const PaWeights& mat, const PaTask& t, uint32_t lane) {
+template <int J0 = 0, int U, PaFmt W>
+__device__ __forceinline__ void pa_load(PaSet<U, W>& w, const PaWeights& mat, const PaTask& t, uint32_t lane) {
     asm volatile("" : "+v"(lane));           // the addresses are worked out here: kept from layer to layer they would not fit the registers
     // Blocks past the last one re-read it, and a wave without rows reads the matrix's first block: with no condition around them the loads in flight are
     // known where a product waits for its own.
@@ -173,27 +182,28 @@ __device__ __forceinline__ void pa_load(PaSet<U, Q4>& w, const PaWeights& mat, c
     };
 #pragma unroll
     for (int j = 0; j < U; j++) {
-        if (Q4) {
+        if (W == PA_Q4) {
             w.v[j] = pa_at<int4>(mat.qs, at(64 * (J0 + j) + lane) * 16);
         } else {
 #pragma unroll
             for (int h = 0; h < 2; h++) w.v[2 * j + h] = pa_at<int4>(mat.qs, at(64 * (J0 + j) + 32 * h + (lane >> 1)) * 32 + (lane & 1u) * 16);
         }
-        w.s[j] = pa_at<uint16_t>(mat.ws, at(pa_own<Q4>(J0 + j, lane)) * 2);
+        if constexpr (W == PA_KQ) w.s[j] = pa_at<uint32_t>(mat.ws, at(pa_own<W>(J0 + j, lane)) * 4);
+        else w.s[j] = pa_at<uint16_t>(mat.ws, at(pa_own<W>(J0 + j, lane)) * 2);
     }
 }
 
 // Where a lane finds its blocks' activations and leaves their products (LDS bytes), worked out ahead of the wait for the vector.
-template <int U, bool Q4> struct PaIdx { uint32_t a[Q4 ? U : 2 * U], s[U], p[U]; };
-template <int U, bool Q4, int J0 = 0>
-__device__ __forceinline__ PaIdx<U, Q4> pa_index(const PaTask& t, const PaMat& m, uint32_t off_as, uint32_t prod, uint32_t lane) {
-    PaIdx<U, Q4> x;
+template <int U, PaFmt W> struct PaIdx { uint32_t a[W == PA_Q4 ? U : 2 * U], s[U], p[U]; };
+template <int U, PaFmt W, int J0 = 0>
+__device__ __forceinline__ PaIdx<U, W> pa_index(const PaTask& t, const PaMat& m, uint32_t off_as, uint32_t prod, uint32_t lane) {
+    PaIdx<U, W> x;
 #pragma unroll
     for (int j = 0; j < U; j++) {
-        const uint32_t u = pa_own<Q4>(J0 + j, lane), r = __umulhi(u, m.magic), b = u - r * m.nblk;      // b is a block of the row whatever u is
+        const uint32_t u = pa_own<W>(J0 + j, lane), r = __umulhi(u, m.magic), b = u - r * m.nblk;      // b is a block of the row whatever u is
         x.s[j] = off_as + b * 4;
         x.p[j] = u < t.n ? prod + (r * m.stride + b) * 4 : prod + m.dump;
-        if (Q4) {
+        if (W == PA_Q4) {
             x.a[j] = b * 32;
         } else {
 #pragma unroll
@@ -205,18 +215,20 @@ __device__ __forceinline__ PaIdx<U, Q4> pa_index(const PaTask& t, const PaMat& m
         asm volatile("" : "+v"(x.s[j]), "+v"(x.p[j]));
     }
 #pragma unroll
-    for (int i = 0; i < (Q4 ? U : 2 * U); i++) asm volatile("" : "+v"(x.a[i]));
+    for (int i = 0; i < (W == PA_Q4 ? U : 2 * U); i++) asm volatile("" : "+v"(x.a[i]));
     return x;
 }
 
-// The blocks' products (a_s * w_s) * f32(isum), exact int32 block sums, parked in the wave's LDS.
-template <int J0 = 0, int U, bool Q4>
-__device__ __forceinline__ void pa_products(const PaSet<U, Q4>& w, const PaIdx<U, Q4>& x, uint32_t n, uint8_t* smem) {
+// The blocks' products, parked in the wave's LDS: (a_s * w_s) * f32(isum) of an exact int32 block sum, or the block's term of dot_q4_k_q8_0 / dot_q6_k_q8_0
+// (emit.rs:3035-3306, 3553-3612), a_s * (d * f32(sum of scale * isum over the halves) - (dmin * minimum) * f32(sum of the codes)): both sums whole numbers of less than
+// 2^24.  sums: KQ, from a block's activation scale to the sum of its codes (LDS bytes).
+template <int J0 = 0, int U, PaFmt W>
+__device__ __forceinline__ void pa_products(const PaSet<U, W>& w, const PaIdx<U, W>& x, const PaTask& t, uint8_t* smem, uint32_t sums) {
 #pragma unroll
     for (int j = 0; j < U; j++) {
-        if (64u * (J0 + j) >= n) break;
+        if (64u * (J0 + j) >= t.n) break;
         int isum;
-        if (Q4) {
+        if (W == PA_Q4) {
             const int4 a0 = *reinterpret_cast<const int4*>(smem + x.a[j]);
             const int4 a1 = *reinterpret_cast<const int4*>(smem + x.a[j] + 16);
             const int4 v = w.v[j];
@@ -229,11 +241,29 @@ __device__ __forceinline__ void pa_products(const PaSet<U, Q4>& w, const PaIdx<U
             int d[2];
 #pragma unroll
             for (int h = 0; h < 2; h++) d[h] = dot16(w.v[2 * j + h], *reinterpret_cast<const int4*>(smem + x.a[2 * j + h]), 0);
+            if constexpr (W == PA_KQ) {
+                // this lane's half of either block times its scale: its own block's word and its neighbour's
+                const bool odd = __lane_id() & 1u;
+                const uint32_t own = w.s[j], far = lane_xor<1>(own), up = odd && t.six ? 0u : 8u;
+                d[0] = __mul24(d[0], (int)((odd ? far : own) << up) >> 24);
+                d[1] = __mul24(d[1], (int)((odd ? own : far) << up) >> 24);
+            }
 #pragma unroll
             for (int h = 0; h < 2; h++) d[h] += lane_xor<1>(d[h]);
             isum = (__lane_id() & 1u) ? d[1] : d[0];
         }
-        *reinterpret_cast<float*>(smem + x.p[j]) = (*reinterpret_cast<const float*>(smem + x.s[j]) * f16_bits_to_f32((uint16_t)w.s[j])) * (float)isum;
+        const float as = *reinterpret_cast<const float*>(smem + x.s[j]);
+        float* p = reinterpret_cast<float*>(smem + x.p[j]);
+        if constexpr (W == PA_KQ) {
+            // d and dmin of a super-block lie in its even and odd blocks
+            const uint32_t own = w.s[j], mate = lane_xor<2>(own);
+            const bool second = __lane_id() & 2u;
+            const float d = f16_bits_to_f32((uint16_t)(second ? mate : own)), dmin = f16_bits_to_f32((uint16_t)(second ? own : mate));
+            const float asum = *reinterpret_cast<const float*>(smem + x.s[j] + sums);
+            *p = as * (d * (float)isum - (t.six ? 0.f : dmin * (float)(own >> 24)) * asum);
+        } else {
+            *p = (as * f16_bits_to_f32((uint16_t)w.s[j])) * (float)isum;
+        }
     }
 }
 
@@ -282,6 +312,8 @@ __device__ __forceinline__ PaSum pa_row_sum(const PaMat& m, uint32_t rows, const
 
 // int8 codes of 32 values, one per lane of a half wave, and their fp16 scale (emit.rs:1410-1440), as the nine elements of a block: side by side and by one
 // instruction.  (Elements of one line that arrive one by one, from eight waves or with the scales elsewhere, cost the hand-over 0.7 us.)
+// SUMS: the sum of the codes above the scale.
+template <bool SUMS>
 __device__ __forceinline__ void pa_store_block(float o, uint64_t* block, uint32_t tag, uint32_t lane, bool on) {
     const float amax = half_wave_max(fabsf(o));
     float inv;
@@ -289,7 +321,13 @@ __device__ __forceinline__ void pa_store_block(float o, uint64_t* block, uint32_
     const uint32_t code = (uint32_t)quant_code(o * inv) & 0xFFu;
     const uint32_t pk = quad_broadcast<0>(code) | (quad_broadcast<1>(code) << 8) | (quad_broadcast<2>(code) << 16) | (quad_broadcast<3>(code) << 24);
     const uint32_t l = lane & 31u;            // lanes 0, 4, .. 28: codes; lane 1: the scale
-    if (on && ((l & 3u) == 0 || l == 1)) stc64(block + (l == 1 ? 8u : l / 4), tag, l == 1 ? (uint32_t)f32_to_f16_bits(sc) : pk);
+    uint32_t last = f32_to_f16_bits(sc);
+    if constexpr (SUMS) {
+        int sum = __builtin_amdgcn_sdot4((int)pk, 0x01010101, 0, false);
+        sum += lane_xor<4>(sum); sum += lane_xor<8>(sum); sum += lane_xor<16>(sum);
+        last |= (uint32_t)sum << 16;
+    }
+    if (on && ((l & 3u) == 0 || l == 1)) stc64(block + (l == 1 ? 8u : l / 4), tag, l == 1 ? last : pk);
 }
 
 // Vectors, fetched by the polling waves.  The residual row lies in LDS accumulator by accumulator of the norm: element e in row e % 16.
@@ -322,8 +360,8 @@ __device__ __forceinline__ void pa_fetch_x(const uint64_t* tx, uint32_t tag, con
 
 // A quantised vector and, with it, the residual of the rows that this workgroup holds: element res_row of x in lane r of the first wave
 // (res_tag 0: the embedding row; threads without a row: anything).
-template <int NV>
-__device__ __forceinline__ float pa_fetch_aq(const uint64_t* t, uint32_t tag, uint32_t K, uint32_t* aq, float* as, bool has_res, uint32_t res_row, const uint64_t* tx,
+template <int NV, bool SUMS>
+__device__ __forceinline__ float pa_fetch_aq(const uint64_t* t, uint32_t tag, uint32_t K, uint32_t* aq, float* as, float* sums, bool has_res, uint32_t res_row, const uint64_t* tx,
                                              uint32_t res_tag, const float* emb, const PaCtx& cx) {
     const uint32_t ne = K / 32 * 9;
     float re = 0.f;
@@ -342,6 +380,7 @@ __device__ __forceinline__ float pa_fetch_aq(const uint64_t* t, uint32_t tag, ui
             if (e < ne) {
                 if (k < 8) aq[b * 8 + k] = v[i];
                 else as[b] = f16_bits_to_f32((uint16_t)v[i]);
+                if (SUMS && k == 8) sums[b] = (float)((int)v[i] >> 16);
             }
         }
         if (poll_res) re = __uint_as_float(v[N]);
@@ -381,16 +420,23 @@ __device__ __forceinline__ void pa_norm_sum(const float* xs, uint32_t xstride, f
     s = lane_xor_add<2>(s);
     if (cx.tid == 0) part[0] = 1.0f / sqrtf(s / (float)H + eps);
 }
-template <bool ORD>
-__device__ __forceinline__ void pa_norm_quant(const float* xs, uint32_t xstride, float4 nw, float eps, uint32_t H, uint8_t* smem, uint32_t off_as, const float* part, uint32_t t) {
+template <bool ORD, bool SUMS>
+__device__ __forceinline__ void pa_norm_quant(const float* xs, uint32_t xstride, float4 nw, float eps, uint32_t H, uint8_t* smem, uint32_t off_as, uint32_t to_sums, const float* part,
+                                              uint32_t t) {
     if (t * 4 >= H) return;
     const float* p = xs + (t * 4 & 15u) * xstride + t / 4;        // four neighbours: rows t * 4 % 16 .. + 3
     const float x0 = p[0], x1 = p[xstride], x2 = p[2 * xstride], x3 = p[3 * xstride];
     const float inv_rms = ORD ? part[0] : 1.0f / sqrtf(((part[0] + part[1]) + (part[2] + part[3])) / (float)H + eps);
     const float4 v = make_float4(x0 * inv_rms * nw.x, x1 * inv_rms * nw.y, x2 * inv_rms * nw.z, x3 * inv_rms * nw.w);
     uint16_t sb;
-    reinterpret_cast<uint32_t*>(smem)[t] = quantize_block_part(v, sb);
+    const uint32_t codes = quantize_block_part(v, sb);
+    reinterpret_cast<uint32_t*>(smem)[t] = codes;
     if ((t & 7u) == 0) *reinterpret_cast<float*>(smem + off_as + t / 2) = f16_bits_to_f32(sb);
+    if constexpr (SUMS) {
+        int sum = __builtin_amdgcn_sdot4((int)codes, 0x01010101, 0, false);
+        sum += lane_xor<1>(sum); sum += lane_xor<2>(sum); sum += lane_xor<4>(sum);
+        if ((t & 7u) == 0) *reinterpret_cast<float*>(smem + off_as + t / 2 + to_sums) = (float)sum;
+    }
 }
 
 struct PaExpTab {
@@ -493,10 +539,12 @@ struct PaHead {
         pa_pack_values<HD>(kv, raw);
         kv.set_keys(kr);
     }
+    template <bool SUMS>
     __device__ __forceinline__ void step(PaKv<HD>& kv, const PaArgs& a, const PaLayer& L, PaAttn<HD, AW>* sh, const uint64_t* exp_tab, uint32_t pos, uint32_t tag_in, PaCtx& cx) const;
 };
 
 template <int HD, uint32_t AW>
+template <bool SUMS>
 __device__ __forceinline__ void PaHead<HD, AW>::step(PaKv<HD>& kv, const PaArgs& a, const PaLayer& L, PaAttn<HD, AW>* sh, const uint64_t* exp_tab, uint32_t pos, uint32_t tag_in,
                                                      PaCtx& cx) const {
         constexpr int DPL = PaKv<HD>::DPL, KC = PaKv<HD>::KC;
@@ -620,7 +668,7 @@ __device__ __forceinline__ void PaHead<HD, AW>::step(PaKv<HD>& kv, const PaArgs&
             const float inv_l = 1.0f / l_i;
             const float o = acc * inv_l;
             const uint32_t e = h * HD + cx.tid;
-            pa_store_block(cx.tid < HD ? o : 0.f, a.taq + e / 32 * 9, tag_in + 1, cx.lane, cx.tid < HD);
+            pa_store_block<SUMS>(cx.tid < HD ? o : 0.f, a.taq + e / 32 * 9, tag_in + 1, cx.lane, cx.tid < HD);
         }
 }
 
@@ -724,7 +772,7 @@ struct PaPart {
 };
 
 // The splits of head h into its quantised row; recs: splits records, wt: a weight per split.  Fetching waves; two barriers.
-template <int HD>
+template <int HD, bool SUMS>
 __device__ __forceinline__ void pa_merge(const PaArgs& a, uint32_t h, uint32_t tag_in, uint32_t tag_out, float* recs, float* wt, const PaCtx& cx) {
     constexpr uint32_t REC = HD + 2, N = (PA_SPLITS * REC + PA_POLL_THREADS - 1) / PA_POLL_THREADS;
     const uint32_t ne = a.splits * REC;
@@ -751,7 +799,7 @@ __device__ __forceinline__ void pa_merge(const PaArgs& a, uint32_t h, uint32_t t
 #pragma unroll 8
         for (uint32_t i = 0; i < a.splits; i++) o = fmaf(wt[i], recs[i * REC + d], o);
         const uint32_t e = h * HD + cx.tid;
-        pa_store_block(cx.tid < HD ? o : 0.f, a.taq + e / 32 * 9, tag_out, cx.lane, cx.tid < HD);
+        pa_store_block<SUMS>(cx.tid < HD ? o : 0.f, a.taq + e / 32 * 9, tag_out, cx.lane, cx.tid < HD);
     }
 }
 
@@ -770,8 +818,10 @@ __device__ __forceinline__ ArgPair pa_arg_wg(ArgPair v, ArgPair* sh, const PaCtx
 
 // The tag of a phase instance: tag_base + 6 layer + 1 q;k;v, 2 attention (long contexts: its parts, 3 their merge), 4 o, 5 gate;up, 6 down; the argmax's is behind
 // the last layer's.
-template <typename F, bool ORD, bool LONG, int HD, bool Q4, bool LMQ4>
+template <typename F, bool ORD, bool LONG, int HD, PaFmt W, PaFmt LMW>
 __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
+    constexpr bool SUMS = W == PA_KQ;
+    static_assert(!SUMS || (!ORD && LMW == PA_KQ), "models of K-quant matrices: all of them, where the order is free");
     extern __shared__ __align__(16) uint8_t smem[];
     __shared__ uint32_t sh_abort;
     __shared__ ArgPair sh_arg[PA_WAVES];
@@ -780,6 +830,7 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
     __shared__ uint64_t exp_tab[32];          // expf_ref's table
     uint32_t* aq = reinterpret_cast<uint32_t*>(smem);
     float* as = reinterpret_cast<float*>(smem + a.off_as);
+    float* code_sums = reinterpret_cast<float*>(smem + a.off_as + a.to_sums);
     float* xs = reinterpret_cast<float*>(smem + a.off_xs);
     float* out = reinterpret_cast<float*>(smem + a.off_out);                     // the workgroup's row sums
     float* silu = reinterpret_cast<float*>(smem + a.off_silu);
@@ -817,10 +868,10 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
             for (uint32_t i = 0; i < slots; i++) a.stamps[slot + i] = t;
         }
     };
-    PaSet<F::UL, LMQ4> wl[2];
+    PaSet<F::UL, LMW> wl[2];
     float4 n1;                                // norm weights of elements 4 ntid ..
     const PaMat ml = a.m[4];
-    const uint32_t T = gridDim.x, W = PA_COMP * T, lwv = c * T + cx.wg;
+    const uint32_t T = gridDim.x, WAVES = PA_COMP * T, lwv = c * T + cx.wg;
     auto load_norm = [&](const float* nw) { return pa_at<float4>(nw, min(ntid * 4, a.H - 4) * 4); };      // threads past the last one: it again
     // the barriers and what lies between them from a fetched row to its codes, for fetching and computing waves; false: the step is given up
     auto norm_fetching = [&]() {
@@ -842,7 +893,7 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
         __syncthreads();
         if (sh_abort) return false;
         if (ORD) __syncthreads();
-        pa_norm_quant<ORD>(xs, a.xstride, n, a.eps, a.H, smem, a.off_as, norm_part, ntid);
+        pa_norm_quant<ORD, SUMS>(xs, a.xstride, n, a.eps, a.H, smem, a.off_as, a.to_sums, norm_part, ntid);
         __syncthreads();
         return true;
     };
@@ -858,8 +909,9 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
         const uint32_t kq = rank(mq), ko = rank(mo), kd = rank(md);
         const uint32_t row_q = kq * PA_COMP * mq.R, row_o = ko * PA_COMP * mo.R, row_d = kd * PA_COMP * md.R;
         const bool on_q = row_q < mq.N, on_o = row_o < mo.N, on_g = cx.wg < a.I / 32, on_d = row_d < md.N;
-        const PaTask tq = pa_task(mq, kq * PA_COMP + c), to = pa_task(mo, ko * PA_COMP + c), td = pa_task(md, kd * PA_COMP + c);
-        const PaTask tg{on_g ? (cx.wg * 32 + c * per_wave) * mg.nblk : 0u, on_g ? 2 * per_wave * mg.nblk : 0u, per_wave * mg.nblk, (a.I - per_wave) * mg.nblk};
+        const PaTask tq = pa_task(mq, kq * PA_COMP + c, (kq * PA_COMP + c) * mq.R < a.QKS + a.KV ? a.six[0] : a.six_v), to = pa_task(mo, ko * PA_COMP + c, a.six[1]),
+                     td = pa_task(md, kd * PA_COMP + c, a.six[3]);
+        const PaTask tg{on_g ? (cx.wg * 32 + c * per_wave) * mg.nblk : 0u, on_g ? 2 * per_wave * mg.nblk : 0u, per_wave * mg.nblk, (a.I - per_wave) * mg.nblk, a.six[2]};
         const uint32_t pq = mq.prod + c * a.prod_words * 4, po = mo.prod + c * a.prod_words * 4, pg = mg.prod + c * a.prod_words * 4, pd = md.prod + c * a.prod_words * 4;
         // the first wave finishes rows: lane r the workgroup's r-th
         float rc = 1.f, rs = 0.f;                                                // rotation of its row of q | k
@@ -934,7 +986,7 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
                         return;
                     }
                     if (on_a) {
-                        pa_merge<HD>(a, head, base + 2, base + 3, reinterpret_cast<float*>(smem + a.off_rec), silu, cx);
+                        pa_merge<HD, SUMS>(a, head, base + 2, base + 3, reinterpret_cast<float*>(smem + a.off_rec), silu, cx);
                         if (sh_abort) return;
                         stamp(a.head0, 6 * l + 3);
                     } else if (!on_o && !glance(a.taq + a.QKS / 32 * 9 - 1, base + 3)) {
@@ -944,7 +996,7 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
                     if (on_a) {
                         PaKv<HD> kv;
                         ph.load(kv, a, L, pos, cx.lane);
-                        ph.step(kv, a, L, attn, exp_tab, pos, base + 1, cx);
+                        ph.template step<SUMS>(kv, a, L, attn, exp_tab, pos, base + 1, cx);
                         stamp(a.head0, 6 * l + 2, 2);                            // no merge phase
                     } else {
                         if (!glance(a.tkv + 2 * a.KV - 1, base + 1)) return;
@@ -955,7 +1007,7 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
                 // ---- o + residual
                 if (on_o) {
                     const bool mine = cx.wave == 0 && cx.lane < PA_COMP * mo.R && row_o + cx.lane < mo.N;
-                    const float r = pa_fetch_aq<F::NV>(a.taq, base + (LONG ? 3 : 2), a.QKS, aq, as, mine, row_o + cx.lane, a.tx, x_in, emb, cx);
+                    const float r = pa_fetch_aq<F::NV, SUMS>(a.taq, base + (LONG ? 3 : 2), a.QKS, aq, as, code_sums, mine, row_o + cx.lane, a.tx, x_in, emb, cx);
                     __syncthreads();
                     if (sh_abort) return;
                     __syncthreads();
@@ -967,13 +1019,13 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
                     pa_fetch_x<F::NX, ORD>(a.tx, base + 4, emb, a.H, xs, a.xstride, norm_part, cx);
                     if (!norm_fetching()) return;
                     __syncthreads();
-                    if (cx.wave == 0) pa_store_block(silu[cx.lane & 31u], a.taq2 + cx.wg * 9, base + 5, cx.lane, cx.lane < 32);
+                    if (cx.wave == 0) pa_store_block<SUMS>(silu[cx.lane & 31u], a.taq2 + cx.wg * 9, base + 5, cx.lane, cx.lane < 32);
                 }
                 // ---- down + residual
                 stamp(0, 6 * l + 5);
                 if (on_d) {
                     const bool mine = cx.wave == 0 && cx.lane < PA_COMP * md.R && row_d + cx.lane < md.N;
-                    const float r = pa_fetch_aq<F::NV>(a.taq2, base + 5, a.I, aq, as, mine, row_d + cx.lane, a.tx, base + 4, emb, cx);
+                    const float r = pa_fetch_aq<F::NV, SUMS>(a.taq2, base + 5, a.I, aq, as, code_sums, mine, row_d + cx.lane, a.tx, base + 4, emb, cx);
                     __syncthreads();
                     if (sh_abort) return;
                     __syncthreads();
@@ -981,10 +1033,10 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
                 }
             }
         } else {
-            PaSet<F::UQ, Q4> wq;
-            PaSet<F::UO, Q4> wo;
-            PaSet<F::UG1, Q4> wg;
-            PaSet<F::WIDE ? F::UG2 : F::UD, Q4> wd;                              // Wide: first gate;up's second part, then down
+            PaSet<F::UQ, W> wq;
+            PaSet<F::UO, W> wo;
+            PaSet<F::UG1, W> wg;
+            PaSet<F::WIDE ? F::UG2 : F::UD, W> wd;                              // Wide: first gate;up's second part, then down
             float4 n2;
             n1 = load_norm(pa_lds_ptr(layers[0].norm[0]));
             pa_load(wq, pa_lds_ptr(layers[0].w[0]), tq, cx.lane);
@@ -995,9 +1047,9 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
                 const PaLayer& L = layers[l];
                 const PaLayer& N = layers[l + 1];
                 if (on_q) {
-                    const auto x = pa_index<F::UQ, Q4>(tq, mq, a.off_as, pq, cx.lane);
+                    const auto x = pa_index<F::UQ, W>(tq, mq, a.off_as, pq, cx.lane);
                     if (!norm_computing(n1)) return;
-                    pa_products(wq, x, tq.n, smem);
+                    pa_products(wq, x, tq, smem, a.to_sums);
                     const PaSum v = pa_row_sum<ORD>(mq, mq.R, smem + pq, cx.lane);
                     if (v.on) out[c * mq.R + v.row] = v.v;
                     __syncthreads();
@@ -1024,20 +1076,20 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
                     pa_load(wq, pa_lds_ptr(N.w[0]), tq, cx.lane);
                 }
                 if (on_o) {
-                    const auto x = pa_index<F::UO, Q4>(to, mo, a.off_as, po, cx.lane);
+                    const auto x = pa_index<F::UO, W>(to, mo, a.off_as, po, cx.lane);
                     __syncthreads();
                     if (sh_abort) return;
-                    pa_products(wo, x, to.n, smem);
+                    pa_products(wo, x, to, smem, a.to_sums);
                     const PaSum v = pa_row_sum<ORD>(mo, mo.R, smem + po, cx.lane);
                     if (v.on) out[c * mo.R + v.row] = v.v;
                     __syncthreads();
                     if constexpr (F::WIDE) pa_load<F::UG1>(wd, pa_lds_ptr(L.w[2]), tg, cx.lane);
                 }
                 if (on_g) {
-                    const auto x = pa_index<F::UG1, Q4>(tg, mg, a.off_as, pg, cx.lane);
+                    const auto x = pa_index<F::UG1, W>(tg, mg, a.off_as, pg, cx.lane);
                     if (!norm_computing(n2)) return;
-                    pa_products(wg, x, tg.n, smem);
-                    if constexpr (F::WIDE) pa_products<F::UG1>(wd, pa_index<F::UG2, Q4, F::UG1>(tg, mg, a.off_as, pg, cx.lane), tg.n, smem);
+                    pa_products(wg, x, tg, smem, a.to_sums);
+                    if constexpr (F::WIDE) pa_products<F::UG1>(wd, pa_index<F::UG2, W, F::UG1>(tg, mg, a.off_as, pg, cx.lane), tg, smem, a.to_sums);
                     const PaSum v = pa_row_sum<ORD>(mg, 2 * per_wave, smem + pg, cx.lane);
                     const float up = ORD ? lane_xor<4>(v.v) : lane_xor<32>(v.v);           // row r + 4 of 8
                     if (v.on && v.row < per_wave) silu[c * per_wave + v.row] = (v.v / (1.0f + expf_ref_with<true>(-v.v, PaExpTab{exp_tab}))) * up;      // silu_mul, emit.rs:380-386
@@ -1045,10 +1097,10 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
                 }
                 if constexpr (F::WIDE) pa_load(wd, pa_lds_ptr(L.w[3]), td, cx.lane);
                 if (on_d) {
-                    const auto x = pa_index<F::UD, Q4>(td, md, a.off_as, pd, cx.lane);
+                    const auto x = pa_index<F::UD, W>(td, md, a.off_as, pd, cx.lane);
                     __syncthreads();
                     if (sh_abort) return;
-                    pa_products(wd, x, td.n, smem);
+                    pa_products(wd, x, td, smem, a.to_sums);
                     const PaSum v = pa_row_sum<ORD>(md, md.R, smem + pd, cx.lane);
                     if (v.on) out[c * md.R + v.row] = v.v;
                     __syncthreads();
@@ -1058,7 +1110,7 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
                     if (on_a) pa_load(wg, pa_lds_ptr(N.w[2]), tg, cx.lane);
                 }
             }
-            pa_load(wl[0], a.lm, pa_task(ml, lwv), cx.lane);
+            pa_load(wl[0], a.lm, pa_task(ml, lwv, a.six[4]), cx.lane);
         }
     } else {
         if (comp) n1 = load_norm(pa_lds_ptr(layers[a.L].norm[0]));
@@ -1070,13 +1122,13 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
                     asm volatile("" : "+v"(cx.tid), "+v"(cx.lane));
                     PaKv<HD> kv;
                     ph.load(kv, a, layers[l], pos, cx.lane);                     // requested as soon as the layer before is done
-                    ph.step(kv, a, layers[l], attn, exp_tab, pos, a.tag_base + 6 * l + 1, cx);
+                    ph.template step<SUMS>(kv, a, layers[l], attn, exp_tab, pos, a.tag_base + 6 * l + 1, cx);
                     if (sh_abort) return;
                     stamp(a.head0, 6 * l + 2, 2);
                 }
             }
         }
-        if (comp) pa_load(wl[0], a.lm, pa_task(ml, lwv), cx.lane);
+        if (comp) pa_load(wl[0], a.lm, pa_task(ml, lwv, a.six[4]), cx.lane);
         // a workgroup without rows in the layers looks for the final row now and then only
         if (cx.tid == 0) {
             uint32_t spins = 0;
@@ -1097,9 +1149,9 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
     } else {
         const uint32_t pl = ml.prod + c * a.prod_words * 4;
         if (!norm_computing(n1)) return;
-        auto tile = [&](uint32_t t, const PaSet<F::UL, LMQ4>& w) {
-            const PaTask task = pa_task(ml, t);
-            pa_products(w, pa_index<F::UL, LMQ4>(task, ml, a.off_as, pl, cx.lane), task.n, smem);
+        auto tile = [&](uint32_t t, const PaSet<F::UL, LMW>& w) {
+            const PaTask task = pa_task(ml, t, a.six[4]);
+            pa_products(w, pa_index<F::UL, LMW>(task, ml, a.off_as, pl, cx.lane), task, smem, a.to_sums);
             const PaSum sum = pa_row_sum<ORD>(ml, pa_rows(ml, t), smem + pl, cx.lane);
             const uint32_t row = t * ml.R + sum.row;
             float v = sum.v;
@@ -1116,12 +1168,12 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
                 best = arg_better(best, ArgPair{v, row});
             }
         };
-        for (uint32_t t = lwv; t * ml.R < ml.N; t += 2 * W) {
-            const bool second = (t + W) * ml.R < ml.N, third = (t + 2 * W) * ml.R < ml.N;
-            if (second) pa_load(wl[1], a.lm, pa_task(ml, t + W), cx.lane);
+        for (uint32_t t = lwv; t * ml.R < ml.N; t += 2 * WAVES) {
+            const bool second = (t + WAVES) * ml.R < ml.N, third = (t + 2 * WAVES) * ml.R < ml.N;
+            if (second) pa_load(wl[1], a.lm, pa_task(ml, t + WAVES, a.six[4]), cx.lane);
             tile(t, wl[0]);
-            if (third) pa_load(wl[0], a.lm, pa_task(ml, t + 2 * W), cx.lane);
-            if (second) tile(t + W, wl[1]);
+            if (third) pa_load(wl[0], a.lm, pa_task(ml, t + 2 * WAVES, a.six[4]), cx.lane);
+            if (second) tile(t + WAVES, wl[1]);
         }
     }
     const uint32_t th = a.tag_base + 6 * a.L + 1;
@@ -1152,22 +1204,61 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
 }
 
 template <typename F, bool ORD, bool LONG, int HD>
-const void* pa_kernel_hd(bool q4, bool lmq4) {
-    if (q4) return lmq4 ? reinterpret_cast<const void*>(decode_ahead_kernel<F, ORD, LONG, HD, true, true>) : reinterpret_cast<const void*>(decode_ahead_kernel<F, ORD, LONG, HD, true, false>);
-    return lmq4 ? reinterpret_cast<const void*>(decode_ahead_kernel<F, ORD, LONG, HD, false, true>) : reinterpret_cast<const void*>(decode_ahead_kernel<F, ORD, LONG, HD, false, false>);
+const void* pa_kernel_hd(PaFmt w, PaFmt lm) {
+    if constexpr (F::WIDE && !ORD) {
+        if (w == PA_KQ) return reinterpret_cast<const void*>(decode_ahead_kernel<F, ORD, LONG, HD, PA_KQ, PA_KQ>);
+    }
+    if (w == PA_Q4)
+        return lm == PA_Q4 ? reinterpret_cast<const void*>(decode_ahead_kernel<F, ORD, LONG, HD, PA_Q4, PA_Q4>) : reinterpret_cast<const void*>(decode_ahead_kernel<F, ORD, LONG, HD, PA_Q4, PA_Q8>);
+    return lm == PA_Q4 ? reinterpret_cast<const void*>(decode_ahead_kernel<F, ORD, LONG, HD, PA_Q8, PA_Q4>) : reinterpret_cast<const void*>(decode_ahead_kernel<F, ORD, LONG, HD, PA_Q8, PA_Q8>);
 }
 
 // What a form means for a shape.
 struct PaForm { int units[5]; uint32_t nx, nv, aw; bool wide; const void* kernel; uint32_t attn_bytes; };
 template <typename F, bool ORD, bool LONG>
-const void* pa_kernel(uint32_t hd, bool q4, bool lmq4) {
-    return hd == 64 ? pa_kernel_hd<F, ORD, LONG, 64>(q4, lmq4) : hd == 96 ? pa_kernel_hd<F, ORD, LONG, 96>(q4, lmq4) : pa_kernel_hd<F, ORD, LONG, 128>(q4, lmq4);
+const void* pa_kernel(uint32_t hd, PaFmt w, PaFmt lm) {
+    return hd == 64 ? pa_kernel_hd<F, ORD, LONG, 64>(w, lm) : hd == 96 ? pa_kernel_hd<F, ORD, LONG, 96>(w, lm) : pa_kernel_hd<F, ORD, LONG, 128>(w, lm);
 }
 template <typename F, bool ORD>
-PaForm pa_form(uint32_t hd, bool q4, bool lmq4) {
+PaForm pa_form(uint32_t hd, PaFmt w, PaFmt lm) {
     return PaForm{{F::UQ, F::UO, F::UG1 + F::UG2, F::UD, F::UL}, F::NX, F::NV, F::AW, F::WIDE,
-                  pa_kernel<F, ORD, false>(hd, q4, lmq4),
+                  pa_kernel<F, ORD, false>(hd, w, lm),
                   (uint32_t)(hd == 64 ? sizeof(PaAttn<64, F::AW>) : hd == 96 ? sizeof(PaAttn<96, F::AW>) : sizeof(PaAttn<128, F::AW>))};
+}
+
+// A K-quant matrix as PA_KQ blocks, from the planes gemv_kquant.hip keeps.  One thread per (row, block).
+__global__ __launch_bounds__(256) void pa_repack_kernel(bool q6, const uint8_t* __restrict__ qs, const uint8_t* __restrict__ meta, uint32_t K, uint64_t total, uint8_t* __restrict__ codes,
+                                                        uint32_t* __restrict__ words) {
+    const uint64_t id = (uint64_t)blockIdx.x * 256 + threadIdx.x;       // n * nblk + b
+    if (id >= total) return;
+    const uint32_t nblk = K / 32;
+    const uint64_t n = id / nblk;
+    const uint32_t b = (uint32_t)(id % nblk), j = b & 7;
+    const uint64_t super = n * (K / 256) + b / 8;
+    uint8_t* dst = codes + id * 32;
+    if (q6) {
+        // block 4 h + r: r = 0, 1 the low nibbles of ql[64 h + 32 r ..], r = 2, 3 the high nibbles of ql[64 h + 32 (r - 2) ..]; bit pair r of qh[32 h ..]
+        const uint8_t *sp = qs + super * 192, *mp = meta + super * 32;
+        const uint32_t h = j >> 2, r = j & 3;
+        const uint8_t *ql = sp + 64 * h + 32 * (r & 1), *qh = sp + 128 + 32 * h;
+        for (uint32_t e = 0; e < 32; e++) dst[e] = (uint8_t)(int8_t)((int)(((ql[e] >> (r >> 1) * 4) & 15u) | (((qh[e] >> 2 * r) & 3u) << 4)) - 32);
+        words[id] = (uint32_t)mp[16] | ((uint32_t)mp[17] << 8) | ((uint32_t)mp[2 * j] << 16) | ((uint32_t)mp[2 * j + 1] << 24);
+    } else {
+        const uint8_t *mp = meta + super * 16, *s12 = mp + 4;
+        uint32_t sc, mn;                                                 // get_scale_min_k4, emit.rs:3013-3021
+        if (j < 4) { sc = s12[j] & 63u; mn = s12[j + 4] & 63u; }
+        else {
+            sc = (s12[j + 4] & 0x0Fu) | ((s12[j - 4] >> 6) << 4);
+            mn = (s12[j + 4] >> 4) | ((s12[j] >> 6) << 4);
+        }
+        const uint8_t* src = qs + super * 128 + 32 * (j >> 1);           // the low nibbles (j even) or the high ones
+        for (uint32_t e = 0; e < 32; e++) dst[e] = (uint8_t)((src[e] >> (j & 1) * 4) & 15u);
+        words[id] = ((uint32_t)mp[2 * (j & 1)] | ((uint32_t)mp[2 * (j & 1) + 1] << 8)) | (sc << 16) | (mn << 24);
+    }
+}
+void pa_repack(const QWeight& w, uint8_t* codes, uint32_t* words) {
+    const uint64_t total = (uint64_t)w.N * (w.K / 32);
+    fh::launch(pa_repack_kernel, dim3((uint32_t)((total + 255) / 256)), 256, 0, nullptr, w.wdtype == FORGE_HIP_Q6_K, w.qs, reinterpret_cast<const uint8_t*>(w.scales), w.K, total, codes, words);
 }
 
 }  // namespace
@@ -1208,12 +1299,24 @@ int32_t pa_create(const forge_hip_config& c, const std::vector<PdLayerIn>& layer
                   const float* cos_t, const float* sin_t, float* logits, uint32_t* state, uint32_t* counts, PaState** out) {
     *out = nullptr;
     const uint32_t H = c.hidden, I = c.inter, hd = c.head_dim, QKS = c.heads * hd, KV = c.kv_heads * hd;
-    if (c.sliding_window != 0 || layers.empty() || !layers[0].qkv || lm_head.kquant()) return FORGE_HIP_OK;
+    if (c.sliding_window != 0 || layers.empty()) return FORGE_HIP_OK;
+    const bool kq = layers[0].q != nullptr;
+    if (kq != lm_head.kquant() || (!kq && !layers[0].qkv)) return FORGE_HIP_OK;
     if (hd != 64 && hd != 96 && hd != 128) return FORGE_HIP_OK;
     const bool q4 = c.wdtype == FORGE_HIP_Q4_0, lmq4 = c.lm_head_dtype == FORGE_HIP_Q4_0;
     if (H < 64 || I < 64 || QKS < 64 || !decode_ahead_offsets_fit(c.max_seq, KV, c.vocab, H, lmq4)) return FORGE_HIP_OK;
     const bool exact = (c.flags & FORGE_HIP_FLAG_EXACT) != 0;
-    const PaForm f = H <= PaNarrow::NX * PA_POLL_THREADS ? pa_form<PaNarrow, true>(hd, q4, lmq4) : exact ? pa_form<PaWide, true>(hd, q4, lmq4) : pa_form<PaWide, false>(hd, q4, lmq4);
+    // Matrices of K-quants: the wide form where the order is free, formats that are the same in every layer.
+    const PaFmt fw = kq ? PA_KQ : q4 ? PA_Q4 : PA_Q8, fl = kq ? PA_KQ : lmq4 ? PA_Q4 : PA_Q8;
+    if (kq) {
+        if (exact || H <= PaNarrow::NX * PA_POLL_THREADS) return FORGE_HIP_OK;
+        for (const PdLayerIn& in : layers) {
+            const QWeight *now[7] = {in.q, in.k, in.v, in.o, in.gate, in.up, in.down}, *first[7] = {layers[0].q, layers[0].q, layers[0].v, layers[0].o, layers[0].gate, layers[0].gate, layers[0].down};
+            for (int i = 0; i < 7; i++)
+                if (!now[i] || !now[i]->kquant() || now[i]->wdtype != first[i]->wdtype) return FORGE_HIP_OK;
+        }
+    }
+    const PaForm f = H <= PaNarrow::NX * PA_POLL_THREADS ? pa_form<PaNarrow, true>(hd, fw, fl) : exact ? pa_form<PaWide, true>(hd, fw, fl) : pa_form<PaWide, false>(hd, fw, fl);
     // what the polling threads fetch at once
     if (H > f.nx * PA_POLL_THREADS || I / 32 * 9 > f.nv * PA_POLL_THREADS || QKS / 32 * 9 > f.nv * PA_POLL_THREADS) return FORGE_HIP_OK;
     // rows that the reference adds in its four-accumulator order (the last len % 4 of a chunk) are left to the other kernels
@@ -1257,11 +1360,18 @@ int32_t pa_create(const forge_hip_config& c, const std::vector<PdLayerIn>& layer
         a.m[i].R = r;
         a.m[i].wg0 = f.wide && i == 1 ? n - (a.m[i].N + r * PA_COMP - 1) / (r * PA_COMP) : 0u;
     }
+    if (kq) {
+        auto six = [](const QWeight* w) { return w->wdtype == FORGE_HIP_Q6_K ? 1u : 0u; };
+        const PdLayerIn& in = layers[0];
+        a.six[0] = six(in.q); a.six_v = six(in.v); a.six[1] = six(in.o); a.six[2] = six(in.gate); a.six[3] = six(in.down); a.six[4] = six(&lm_head);
+        if (a.six[0] != a.six_v && (QKS + KV) % a.m[0].R) return FORGE_HIP_OK;      // a wave's rows are of one format
+    }
     a.L = (uint32_t)layers.size(); a.H = H; a.I = I; a.QKS = QKS; a.KV = KV; a.heads = c.heads; a.kv_heads = c.kv_heads;
     a.eps = c.rms_eps;
     const uint32_t kmax = std::max(std::max(H, I), QKS);
     a.off_as = pa_up(kmax, 16);
-    a.off_xs = a.off_as + pa_up(kmax / 32 * 4, 16);
+    a.to_sums = kq ? pa_up(kmax / 32 * 4, 16) : 0u;
+    a.off_xs = a.off_as + pa_up(kmax / 32 * 4, 16) + a.to_sums;
     auto odd16 = [](uint32_t words) { return words % 8 ? words : words + 4; };      // rows an odd number of 16-byte units apart spread over the banks
     a.xstride = odd16(pa_up(H / 16, PA_SSQ));
     a.off_out = a.off_xs + 16 * a.xstride * 4;
@@ -1308,9 +1418,10 @@ int32_t pa_create(const forge_hip_config& c, const std::vector<PdLayerIn>& layer
             // past the sixth (16/8, 7000: 274 / 261, 10000: 289 / 296; 16/16, 3500: 270 / 264, 5000: 286 / 295), and with fewer than 16 splits, whose contexts are short, not
             // past the fifth (8 splits of 12/4 heads of 128, 1000: 226 / 201, 2400: 237 / 258; of 16/4 heads of 96, 1000: 261 / 217, 2400: 276 / 284; 4 splits of the 1B
             // shape, 1000: 307 / 257, 2400: 311 / 321).  Below 8 splits (more than 32 KV heads, or no LDS for more) there is little context left to cover.
-            const uint32_t rounds = gsize > PA_POLL || c.kv_heads < 4 ? 2 : n < 16 ? 5 : hd > 96 ? 6 : PA_ROUNDS;
+            // Where two rounds are the line, K-quants, whose streamed matrices are fewer bytes, take one (12/2 heads of 128, 8192 wide, 1000: 274 / 275, 2400: 286 / 307).
+            const uint32_t rounds = gsize > PA_POLL || c.kv_heads < 4 ? (kq ? 1 : 2) : n < 16 ? 5 : hd > 96 ? 6 : PA_ROUNDS;
             st->max_rows = std::min(c.max_seq, n * rounds * PA_PASSES * (hd <= 64 ? 8u : 4u));
-            st->kernel_long = pa_kernel<PaWide, false, true>(hd, q4, lmq4);
+            st->kernel_long = pa_kernel<PaWide, false, true>(hd, fw, fl);
         }
     }
     int per_cu = 0;
@@ -1319,10 +1430,31 @@ int32_t pa_create(const forge_hip_config& c, const std::vector<PdLayerIn>& layer
 
     std::vector<PaLayer> host(layers.size() + 1);
     memset(host.data(), 0, host.size() * sizeof(PaLayer));
+    // matrices of one depth, one behind the other, as PA_KQ blocks; false: no memory for them, and the other kernel takes the steps
+    auto units = [&](const std::vector<const QWeight*>& ws, PaWeights* to) {
+        size_t blocks = 0;
+        for (const QWeight* w : ws) blocks += (size_t)w->N * (w->K / 32);
+        uint8_t* codes = st->dev<uint8_t>(blocks * 32);
+        uint32_t* words = codes ? st->dev<uint32_t>(blocks * 4) : nullptr;
+        if (!words) { (void)hipGetLastError(); return false; }
+        *to = PaWeights{codes, reinterpret_cast<const uint16_t*>(words)};
+        for (const QWeight* w : ws) {
+            pa_repack(*w, codes, words);
+            codes += (size_t)w->N * w->K;
+            words += (size_t)w->N * (w->K / 32);
+        }
+        return true;
+    };
     for (size_t l = 0; l < layers.size(); l++) {
         const PdLayerIn& in = layers[l];
-        const QWeight* w[4] = {in.qkv, in.o, in.gate_up, in.down};
-        for (int k = 0; k < 4; k++) host[l].w[k] = PaWeights{w[k]->qs, w[k]->scales};
+        if (kq) {
+            const std::vector<const QWeight*> parts[4] = {{in.q, in.k, in.v}, {in.o}, {in.gate, in.up}, {in.down}};
+            for (int k = 0; k < 4; k++)
+                if (!units(parts[k], &host[l].w[k])) return FORGE_HIP_OK;
+        } else {
+            const QWeight* w[4] = {in.qkv, in.o, in.gate_up, in.down};
+            for (int k = 0; k < 4; k++) host[l].w[k] = PaWeights{w[k]->qs, w[k]->scales};
+        }
         host[l].norm[0] = in.attn_norm; host[l].norm[1] = in.ffn_norm; host[l].kc = in.kc; host[l].vc = in.vc;
     }
     host.back() = host[0];
@@ -1343,6 +1475,11 @@ int32_t pa_create(const forge_hip_config& c, const std::vector<PdLayerIn>& layer
     a.tpart = t; t += 2 * (size_t)st->grid;
     a.trec = t;
     a.lm = PaWeights{lm_head.qs, lm_head.scales};
+    if (kq) {
+        if (!units({&lm_head}, &a.lm)) return FORGE_HIP_OK;
+        FH_HIP(hipDeviceSynchronize());
+        FH_HIP(hipGetLastError());
+    }
     a.embed = embed; a.cos_t = cos_t; a.sin_t = sin_t;
     a.logits = logits; a.state = state; a.counts = counts; a.penalty = 1.0f;
     { const char* e = getenv("FORGE_HIP_PD_TAG_START"); if (e) a.tag_base = (uint32_t)strtoul(e, nullptr, 0); }

@@ -924,6 +924,7 @@ static int32_t model_create_impl(const forge_hip_config* cfg, const uint32_t* pd
             if ((rc = m->paq2.alloc((size_t)R * I)) || (rc = m->pasc2.alloc((size_t)R * (I / 32) * 2))) return rc;
         }
     }
+    auto set_to = [](const char* name, char v) { const char* e = getenv(name); return e && (v ? e[0] == v : true); };
     const char* penv = getenv("FORGE_HIP_PERSIST");
     const char* kenv = getenv("FORGE_HIP_PD_KQUANT");
     if (pd && !(penv && penv[0] == '0') && !(kenv && kenv[0] == '0')) {
@@ -943,6 +944,12 @@ static int32_t model_create_impl(const forge_hip_config* cfg, const uint32_t* pd
                            m->sin_t.as<float>(), m->logits.as<float>(), m->state.as<uint32_t>(), m->counts.as<uint32_t>(),
                            has_bias ? m->biases.as<float>() : nullptr, &m->pd);
             if (rc) return rc;
+            // (beside the other kernel, which takes the steps that this one does not: decode_ahead.hip)
+            if (m->pd && !has_bias && !set_to("FORGE_HIP_PD_AHEAD", '0') && !set_to("FORGE_HIP_PD_ORDERED", '1')) {
+                rc = pa_create(*cfg, pl, m->lm_head, m->embed.as<float>(), m->final_norm.as<float>(), m->cos_t.as<float>(), m->sin_t.as<float>(),
+                               m->logits.as<float>(), m->state.as<uint32_t>(), m->counts.as<uint32_t>(), &m->pa);
+                if (rc) return rc;
+            }
         }
     }
     if (pd && !m->pd && !(penv && penv[0] == '0') && !(kenv && kenv[0] == '0') && cfg->lm_head_dtype == FORGE_HIP_Q6_K && !is_kquant(pd[0])) {
@@ -975,7 +982,6 @@ static int32_t model_create_impl(const forge_hip_config* cfg, const uint32_t* pd
                        has_bias ? m->biases.as<float>() : nullptr, &m->pd);
         if (rc) return rc;
         // Models of up to 2048 channels over the contexts that it covers (decode_ahead.hip).  Where a variable asks for one of the other kernels' forms, it gets that.
-        auto set_to = [](const char* name, char v) { const char* e = getenv(name); return e && (v ? e[0] == v : true); };
         if (!has_bias && !set_to("FORGE_HIP_PD_AHEAD", '0') && !set_to("FORGE_HIP_PD_ORDERED", '1') &&
             !((cfg->flags & FORGE_HIP_FLAG_EXACT) && set_to("FORGE_HIP_PD_EXACT", 0))) {
             rc = pa_create(*cfg, pl, m->lm_head, m->embed.as<float>(), m->final_norm.as<float>(), m->cos_t.as<float>(), m->sin_t.as<float>(),

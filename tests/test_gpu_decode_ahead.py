@@ -320,6 +320,45 @@ def test_longer_contexts_of_fast_mode(fh, torch_gpu, monkeypatch, name):
     one.close(); streamed.close()
 
 
+# formats of q, k, v, o, gate, up, down and the lm_head, then hidden, inter, heads, kv heads, head dim: v of its own format at the edge of a wave's rows, all of one
+# format, each format everywhere; depths whose last round of blocks is half a wave's
+Q4K, Q6K = 12, 14
+KQ = {"1b": ((Q4K, Q4K, Q6K, Q4K, Q4K, Q4K, Q6K), Q6K, 2048, 8192, 32, 8, 64), "all_q6": ((Q6K,) * 7, Q6K, 1024, 2048, 8, 4, 128), "all_q4": ((Q4K,) * 7, Q4K, 1536, 4096, 16, 4, 96),
+      "turned": ((Q6K, Q6K, Q4K, Q6K, Q6K, Q6K, Q4K), Q4K, 1280, 2304, 20, 4, 64)}
+
+
+@pytest.mark.parametrize("name", sorted(KQ))
+def test_kquant_models_of_fast_mode(fh, torch_gpu, monkeypatch, name):
+    """Single steps from identical state, one layer, against decode_step_kernel: the same whole sums and products of them, added up in another order, so the bounds of
+    test_longer_contexts_of_fast_mode; over pages the same bits; a penalty's counts are both kernels'."""
+    formats, lm, hidden, inter, heads, kv_heads, hd = KQ[name]
+    cfg = dict(shape(fh, Q8, hidden, inter, heads, kv_heads, hd, 1004, layers=1, lm=lm, max_seq=2048), flags=0)
+    blob = fh.synth.make_weights_blob_mixed(cfg, formats, seed=67, std=0.05)
+    one = fh.HipModel(cfg, blob, proj_dtypes=formats)
+    paged = fh.HipModel(cfg, blob, proj_dtypes=formats)
+    monkeypatch.setenv("FORGE_HIP_PD_AHEAD", "0")
+    streamed = fh.HipModel(cfg, blob, proj_dtypes=formats)
+    monkeypatch.delenv("FORGE_HIP_PD_AHEAD")
+    paged.set_kv_pages(128, np.random.default_rng(69).permutation(cfg["max_seq"] // 128).astype(np.uint32))
+    toks = fh.synth.uniform_ids(68, 2000, cfg["vocab"])
+    rel, differ = [], 0
+    for n in (1, 63, 64, 190, 254, 255, 700, 1990):
+        for m in (one, streamed, paged):
+            m.reset()
+            m.set_repeat_penalty(1.1)
+            m.forward_prefill(toks[:n])
+        for t in toks[n:n + 3]:
+            a, b = one.forward(int(t)), streamed.forward(int(t))
+            same_bits(paged.forward(int(t)), a)
+            assert one.decode_launches == 1 and np.all(np.isfinite(a))
+            rel.append(np.linalg.norm(a - b) / np.linalg.norm(b))
+            differ += not np.array_equal(a, b)
+        assert one.forward_greedy(5) == streamed.forward_greedy(5)
+    assert max(rel) < 2e-2 and np.median(rel) < 1e-5, rel
+    assert differ, "the same bits throughout: both ran the same kernel"
+    one.close(); streamed.close(); paged.close()
+
+
 @pytest.mark.parametrize("head_dim,which,channel", [(64, "v", 5), (96, "v", 5), (128, "v", 127), (96, "k", 95), (128, "k", 127)])
 def test_an_infinite_value_in_the_first_row_of_a_long_context(fh, torch_gpu, monkeypatch, head_dim, which, channel):
     """The first row stands in for keys that are not there and its last channels for those past a head's: neither may count.  The first token's embedding has one channel, and
