@@ -81,6 +81,88 @@ __global__ __launch_bounds__(GEMV_THREADS) void latent_query_kernel(LatentShape 
     });
 }
 
+// The two products of the query in one launch, a workgroup per head: [RMS norm of the query latent | W_uq | rotation | W_uk^T]; the last workgroup writes the
+// position's cache row.  For small heads, whose matrices a compute unit fetches while it norms the latent; operations and their order are those of
+// latent_query_kernel and latent_absorb_kernel.  What bounds it: a launch, one trip to memory and the steps from the norm on, 4.4 us where the two
+// launches took 6.9 (9 heads of 64 + 32, latents of 192 and 128).
+constexpr uint32_t LQ_THREADS = 1024, LQ_ROWS = 128, LQ_RANK = 256;      // rows (dim + rot) and ranks that registers and LDS are made for
+template <typename T>
+__global__ __launch_bounds__(LQ_THREADS) void latent_query_absorb_kernel(LatentShape sh, const float* __restrict__ raw, const float* __restrict__ q_norm, const float* __restrict__ kv_norm,
+                                                                         const T* __restrict__ uq, const T* __restrict__ uk, DenseEpiArgs e, T* __restrict__ ql, T* __restrict__ cache) {
+    typedef typename Vec<T>::x8 x8;
+    __shared__ float xs[LQ_RANK], red[LQ_THREADS / 64], qs[LQ_ROWS], part[32][LQ_RANK];
+    const uint32_t tid = threadIdx.x, K = sh.q_rank, head = blockIdx.x, lane = tid & 31;
+    if (head == sh.heads) {
+        store_cache_row<T>(sh, raw, kv_norm, e.cos_t, e.sin_t, e.pos_dev ? *e.pos_dev : e.base_pos, cache, red, tid, LQ_THREADS);
+        return;
+    }
+    // everything is requested here: the latent, the position, 32 lanes' pieces of a row of W_uq for four rows, and of W_uk
+    const float x = tid < K ? raw[tid] : 0.f, nw = tid < K ? q_norm[tid] : 0.f;
+    const uint32_t pos = e.pos_dev ? *e.pos_dev : e.base_pos;
+    constexpr uint32_t RP = LQ_ROWS / 32;
+    const uint32_t rows = sh.dim + sh.rot, r0 = tid >> 5, k = lane * 8;       // neighbouring rows, a rotation's pair, in one wave
+    const T* w = uq + (size_t)head * rows * K + k;
+    x8 wq[RP];
+#pragma unroll
+    for (uint32_t p = 0; p < RP; p++) wq[p] = p * 32 < rows && k < K ? load8(w + (size_t)(p * 32 + r0) * K) : zero8<T>();
+    const uint32_t groups = sh.rank / 8, drow = tid / groups, c8 = tid % groups * 8;
+    const T* wk = uk + (size_t)head * sh.dim * sh.rank + c8;
+    x8 wu[RP];
+#pragma unroll
+    for (uint32_t p = 0; p < RP; p++) wu[p] = drow < 32 && p * 32 < sh.dim ? load8(wk + (size_t)(p * 32 + drow) * sh.rank) : zero8<T>();
+    float cs[RP], sn[RP];
+#pragma unroll
+    for (uint32_t p = 0; p < RP; p++) {
+        const uint32_t j = p * 32 + r0, i = (j - sh.dim) / 2;
+        const bool rotates = j < rows && j >= sh.dim && i < sh.rot_pairs;
+        cs[p] = rotates ? e.cos_t[(size_t)pos * sh.rot_pairs + i] : 1.f;
+        sn[p] = rotates ? e.sin_t[(size_t)pos * sh.rot_pairs + i] : 0.f;
+    }
+    const float inv = 1.0f / sqrtf(block_sum(fmaf(x, x, 0.f), red, tid, LQ_THREADS) / (float)sh.q_rank_n + sh.eps);
+    if (tid < K) xs[tid] = x * inv * nw;
+    __syncthreads();
+    T* q = (T*)e.out + head * rows;
+#pragma unroll
+    for (uint32_t p = 0; p < RP; p++) {
+        if (p * 32 >= rows) break;
+        float acc = 0.f;
+        if (k < K) {
+#pragma unroll
+            for (int j = 0; j < 8; j++) acc = fmaf((float)wq[p][j], xs[k + j], acc);
+        }
+        acc = lane_xor_add<16>(acc); acc = lane_xor_add<8>(acc); acc = lane_xor_add<4>(acc); acc = lane_xor_add<2>(acc); acc = lane_xor_add<1>(acc);
+        const float other = lane_xor<32>(acc);
+        const uint32_t row = p * 32 + r0;
+        if (row >= sh.dim && (row - sh.dim) / 2 < sh.rot_pairs) acc = row & 1 ? acc * cs[p] + other * sn[p] : acc * cs[p] - other * sn[p];
+        if (lane == 0) {
+            q[row] = (T)acc;
+            qs[row] = (float)(T)acc;
+        }
+    }
+    __syncthreads();
+    if (drow < 32) {
+        float acc[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) acc[j] = 0.f;
+#pragma unroll
+        for (uint32_t p = 0; p < RP; p++) {
+            if (p * 32 >= sh.dim) break;
+            const float y = qs[p * 32 + drow];
+#pragma unroll
+            for (int j = 0; j < 8; j++) acc[j] = fmaf((float)wu[p][j], y, acc[j]);
+        }
+#pragma unroll
+        for (int j = 0; j < 8; j++) part[drow][c8 + j] = acc[j];
+    }
+    __syncthreads();
+    if (tid < sh.rank) {
+        float s = 0.f;
+#pragma unroll
+        for (int i = 0; i < 32; i++) s += part[i][tid];
+        ql[(size_t)head * sh.rank + tid] = (T)s;
+    }
+}
+
 // ql[head][r] = sum_d q[head][d] W_uk[head dim + d][r].  Workgroup = (64 columns, head): a wave reads 8 rows of 64 columns at a time.
 template <typename T>
 __global__ __launch_bounds__(256) void latent_absorb_kernel(LatentShape sh, const T* __restrict__ q, const T* __restrict__ uk, T* __restrict__ ql) {
@@ -269,6 +351,10 @@ __global__ __launch_bounds__(GEMV_THREADS) void latent_value_kernel(LatentShape 
     });
 }
 
+// Small heads: their query's products are one launch, a request of 30 layers with 9 heads of 64 + 32 11.0 ms instead of 11.4.  Up to what a
+// workgroup has in registers and LDS; past it a head's matrices are too much for one compute unit, and the launches over parts of them spread wider.
+bool latent_query_absorbs(const LatentShape& sh) { return sh.dim + sh.rot <= LQ_ROWS && sh.q_rank <= LQ_RANK && sh.rank <= LQ_RANK; }
+
 namespace {
 
 template <typename T, int NW, int MAXT>
@@ -307,6 +393,10 @@ void query(const LatentShape& sh, const LatentDecodeIo& io, hipStream_t s) {
     e.head_stride = sh.dim + sh.rot;
     e.rot_off = sh.dim;
     e.rot_pairs = sh.rot_pairs;
+    if (latent_query_absorbs(sh)) {
+        fh::launch(latent_query_absorb_kernel<T>, dim3(sh.heads + 1), LQ_THREADS, 0, s, sh, io.raw, io.q_norm, io.kv_norm, (const T*)io.uq.p, (const T*)io.ukv.p, e, (T*)io.ql, (T*)io.cache);
+        return;
+    }
     switch (gemv_depth_split(sh.q_row(), sh.q_rank)) {
         case 1: go_query<T, 1>(sh, io, e, s); break;
         case 2: go_query<T, 2>(sh, io, e, s); break;
@@ -316,7 +406,7 @@ void query(const LatentShape& sh, const LatentDecodeIo& io, hipStream_t s) {
 
 template <typename T>
 void decode(const LatentShape& sh, const LatentDecodeIo& io, hipStream_t s) {
-    fh::launch(latent_absorb_kernel<T>, dim3(sh.rank / 64, sh.heads), 256, 0, s, sh, (const T*)io.q, (const T*)io.ukv.p, (T*)io.ql);
+    if (!latent_query_absorbs(sh)) fh::launch(latent_absorb_kernel<T>, dim3(sh.rank / 64, sh.heads), 256, 0, s, sh, (const T*)io.q, (const T*)io.ukv.p, (T*)io.ql);
     if constexpr (sizeof(T) == 2) {
         if (sh.rank <= 128) go_decode<T, 4, 2>(sh, io, s);
         else if (sh.rank <= 512) go_decode<T, 4, 8>(sh, io, s);

@@ -116,7 +116,8 @@ void enqueue_raw_gate(const MixerCall& c, DType t, const DenseWeight& w, uint32_
 
 // ---- latent attention ------------------------------------------------------------------------------------------------------
 // prompt: [W_dq; W_dkv; W_g], norms + cache rows, W_uq + rotation, [W_uk; W_uv] over the visible cache rows, attention * gate;
-// decode: [W_dq; W_dkv; W_g], norm + W_uq + rotation beside the cache row, W_uk^T q, attention over latents, merge + W_uv * gate.
+// decode: [W_dq; W_dkv; W_g], norm + W_uq + rotation beside the cache row, W_uk^T q (small heads: with
+// the launch before), attention over latents, merge + W_uv * gate.
 struct LatentMixer : Mixer {
     LatentShape sh;
     DenseWeight in, uq, ukv;                 // in: [W_dq; W_dkv; W_g]
@@ -253,7 +254,7 @@ struct LatentMixer : Mixer {
         launch_attn_prompt(t, p, c.M, c.base_pos, stream);
         return dense_rows(out, hv);
     }
-    int decode_launches() const override { return 5; }
+    int decode_launches() const override { return latent_query_absorbs(sh) ? 4 : 5; }
 };
 
 // ---- grouped-query attention -----------------------------------------------------------------------------------------------

@@ -447,7 +447,7 @@ void launch_latent_norm_store(DType t, const LatentShape& sh, const float* raw, 
                               const float* sin_t, uint32_t M, uint32_t base_pos, void* cq, void* cache, hipStream_t s);
 // One row at pos_dev ? *pos_dev : base_pos, four launches: [norm of the query latent | W_uq | rotation] beside the new cache row,
 // queries taken to the latent space (W_uk^T q per head), attention over the cached latents in up to latent_splits() parts, and
-// [merge of the parts | W_uv | gate].
+// [merge of the parts | W_uv | gate].  Three where latent_query_absorbs(): the first does the second's work too.
 struct LatentDecodeIo {
     const float* raw;                  // [raw_row()]
     const float* q_norm;
@@ -466,6 +466,7 @@ struct LatentDecodeIo {
 };
 uint32_t latent_splits(const LatentShape& sh, uint32_t max_seq);
 size_t latent_parts_bytes(const LatentShape& sh, uint32_t max_seq);
+bool latent_query_absorbs(const LatentShape& sh);
 void launch_latent_query(DType t, const LatentShape& sh, const LatentDecodeIo& io, hipStream_t s);
 void launch_latent_attn_decode(DType t, const LatentShape& sh, const LatentDecodeIo& io, hipStream_t s);
 

@@ -12,7 +12,7 @@ from vabirax_cases import cases
 
 pytestmark = pytest.mark.gpu
 
-NAMES = ["uneven", "many_heads", "wide_head", "large_rank", "ones", "no_window", "part_rotation"]
+NAMES = ["uneven", "many_heads", "wide_head", "large_rank", "ones", "no_window", "query_edges", "part_rotation"]
 
 
 @pytest.fixture(scope="module")

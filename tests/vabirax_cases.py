@@ -20,6 +20,8 @@ def cases(fh):
         "ones": conf(33, 11, [lay(1, 1, 2, 1, 4, 5, 1, 1), lay(1, 3, 2, 2, 3, 4, 6, 2)], loop=(1, 2, 1)),
         # no mask: every earlier position is visible
         "no_window": conf(64, 150, [lay(4, 16, 16, 16, 32, 96, 64, None)] * 2, loop=(0, 2, 2)),
+        # the largest head and ranks whose query products are one launch, and one past each of them
+        "query_edges": conf(64, 80, [lay(3, 96, 32, 32, 256, 256, 64, 40), lay(2, 97, 32, 32, 256, 256, None, 40), lay(2, 96, 32, 32, 257, 256, 64, 40), lay(2, 64, 32, 32, 256, 257, None, 40)]),
         # part of the rotated dimensions turns
         "part_rotation": conf(72, 90, [lay(2, 24, 20, 16, 24, 32, 40, 17, rot_dims=12)]),
     }
