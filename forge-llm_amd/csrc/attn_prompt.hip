@@ -11,20 +11,76 @@ namespace fh {
 constexpr float LOG2E = 1.4426950408889634f;
 
 // Workgroup = 8 waves: 8 / KG groups of 32 consecutive queries of one head, each shared by KG waves that take 32 keys each of every tile
-// of 32 KG and merge their (maximum, sum, output) at the end, which cuts the longest chain of dependent tile steps to a KG-th.  Keys
-// and values stream through LDS (K row-major: the head's own part, the shared part; V transposed), the
-// next tile's loads in registers while this one is worked.  Both products are computed transposed (S^T = K Q^T, O^T = V^T P^T):
-// a lane owns one query, so the softmax statistics are per-lane scalars, and the exponentiated scores are already the second
-// product's operand.  Scores stay in the base-2 domain.
+// of 32 KG and merge their (maximum, sum, output) at the end, which cuts the longest chain of dependent tile steps to a KG-th.  Both products are
+// computed transposed (S^T = K Q^T, O^T = V^T P^T): a lane owns one query, so the softmax statistics are per-lane scalars, and the exponentiated
+// scores are already the second product's operand.  Scores stay in the base-2 domain.
+//   bfloat16  Tiles go straight into one of two pairs of LDS buffers while the other is worked, one barrier a step, 32 columns (64 bytes) of 16 rows at a time,
+//             so that a load is all of K's own part, or of the shared part, or of V.  V is transposed on its way out of LDS (ds_read_b64_tr_b16).
+//   32-bit    Through registers into one buffer (K row-major: the head's own part, the shared part; V transposed), two barriers a step.
+// What bounds it: up to a few hundred workgroups the chain of steps, each a trip through LDS, two products and the exponentials between them; then the VALU (exponentials,
+// maxima, conversions) beside the matrix unit.  In bfloat16 a step through registers took 1.8 us, half of it the loads' issue and the writes to LDS, and its registers left
+// one workgroup to a compute unit; now 1.1, and two.  us, before / now: 9 heads of 64 + 32 with a window of 1024, 902 tokens 18.4 / 14.7, 2502 36.0 / 22.2, 4000 47.1 /
+// 28.3; 32/8 heads of 64 902 23.2 / 15.2, 2502 92.7 / 48.5; 24/8 of 128 2502 101.9 / 76.7; 16 of 128 + 64 902 40.1 / 30.9, 4000 169 / 135; 33 tokens the same.
 // DQ >= dim + rot and DV >= vdim: the register tiles' sizes; columns past the real ones are zero.
 constexpr uint32_t LP_THREADS = 512;
+constexpr uint32_t LP_RSRC_FLAGS = 0x00020000;   // raw buffer, 32-bit data format
+constexpr float LP_SLACK = 8.f;                  // base-2 exponent
+template <typename T, int DQ> constexpr bool prompt_four() { return sizeof(T) == 2 && DQ <= 96; }      // four waves to a SIMD
 template <typename T, int DQ, int DV, int KG> constexpr uint32_t prompt_lds() {
-    const uint32_t tiles = (32 * KG * (DQ + 16 / sizeof(T)) + DV * (32 * KG + 8 / sizeof(T))) * sizeof(T), merge = 8 / KG * (KG - 1) * 64 * 18 * 4;
+    const uint32_t tiles = sizeof(T) == 2 ? 2 * 32 * KG * (DQ + DV) * 2 : (32 * KG * (DQ + 16 / sizeof(T)) + DV * (32 * KG + 8 / sizeof(T))) * sizeof(T),
+                   merge = 8 / KG * (KG - 1) * 64 * 18 * 4;
     return tiles > merge ? tiles : merge;
 }
 
+#define FH_LDS3(p) ((__attribute__((address_space(3))) void*)(p))
+
+// V fragments of 32 keys x 32 N columns: f[j][d] = keys 16 j + 4 lh .. + 3 and + 8 of column 32 d + lane % 32, from rows of 64 bytes, CHUNK bytes from one 32
+// columns to the next; at0, at1: LDS addresses of this lane's part of the first keys and of those 8 further on.  Its own waits: ahead of a transposing read of its
+// own the compiler waits for everything that is on its way into LDS, that is for the next tiles in the middle of a step.
+#define FH_TR(dst, at, off) "ds_read_b64_tr_b16 " dst ", " at " offset:" off "\n"
+template <int N, int CHUNK>
+__device__ __forceinline__ void read_v(v8bf (&f)[2][N], uint32_t at0, uint32_t at1) {
+    v4bf r[4 * N];
+    if constexpr (N == 1)
+        asm volatile(FH_TR("%0", "%4", "0") FH_TR("%1", "%5", "0") FH_TR("%2", "%4", "1024") FH_TR("%3", "%5", "1024") "s_waitcnt lgkmcnt(0)"
+                     : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3]) : "v"(at0), "v"(at1));
+    else
+        asm volatile(FH_TR("%0", "%8", "0") FH_TR("%1", "%9", "0") FH_TR("%2", "%8", "1024") FH_TR("%3", "%9", "1024")
+                     FH_TR("%4", "%8", "%10") FH_TR("%5", "%9", "%10") FH_TR("%6", "%8", "%10+1024") FH_TR("%7", "%9", "%10+1024") "s_waitcnt lgkmcnt(0)"
+                     : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3]), "=&v"(r[4]), "=&v"(r[5]), "=&v"(r[6]), "=&v"(r[7])
+                     : "v"(at0), "v"(at1), "n"(CHUNK));
+#pragma unroll
+    for (int d = 0; d < N; d++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) f[j][d] = __builtin_shufflevector(r[4 * d + 2 * j], r[4 * d + 2 * j + 1], 0, 1, 2, 3, 4, 5, 6, 7);
+}
+#undef FH_TR
+
+// Chunks [C0, C1) of a tile, each 16 RG rows of 32 columns, into LDS: load j (a wave's are wave, wave + 8, ...) fills 1 KB with 16 rows; lane -> 16-byte piece.  Columns
+// [0, n) come from `a`, those from there to `all` from `b`, columns past that and rows past the last read 0.  Piece c of row r lies at c ^ (r / 4 % 4) of its 64 bytes:
+// sixteen rows at one piece (fragments of K) touch all banks, and four rows (V) do as they are.
+template <uint32_t RG, uint32_t C0, uint32_t C1, typename T>
+__device__ __forceinline__ void direct_rows(const T* a, uint32_t a_row, uint32_t n, const T* b, uint32_t b_row, uint32_t all, uint32_t rows, uint32_t a_lane, uint32_t b_lane,
+                                            uint8_t* lds, uint32_t wave) {
+#pragma unroll
+    for (uint32_t j0 = C0 * RG / 8 * 8; j0 < C1 * RG; j0 += 8) {
+        const uint32_t j = j0 + wave;
+        if ((j0 < C0 * RG && j < C0 * RG) || (j0 + 8 > C1 * RG && j >= C1 * RG)) continue;
+        const uint32_t col = (j / RG - C0) * 32, r = j % RG * 16;
+        const bool of_a = col < n;
+        const uint32_t st = of_a ? a_row : b_row, at_lane = of_a ? a_lane : b_lane;
+        const uint64_t from = (uint64_t)((of_a ? a + col : b + (col - n)) + r * st);
+        const uint32_t records = r < rows && col < all ? (min(rows - r, 16u) - 1) * st * 2 + 64 : 0u;
+        // (readfirstlane: all of it is uniform, and a descriptor word in a vector register would cost a loop over its values around the load)
+        const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)from), hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(from >> 32));
+        const __amdgpu_buffer_rsrc_t rsrc =
+            __builtin_amdgcn_make_buffer_rsrc((void*)(((uint64_t)hi << 32) | lo), 0, (uint32_t)__builtin_amdgcn_readfirstlane((int)records), LP_RSRC_FLAGS);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, FH_LDS3(lds + j * 1024), 16, at_lane, 0, 0, 0);
+    }
+}
+
 template <typename T, int DQ, int DV, int KG>
-__global__ __launch_bounds__(LP_THREADS) __attribute__((amdgpu_waves_per_eu(2)))
+__global__ __launch_bounds__(LP_THREADS) __attribute__((amdgpu_waves_per_eu(prompt_four<T, DQ>() ? 4 : 2)))
 void attn_prompt_kernel(PromptAttn sh, const T* __restrict__ q, const T* __restrict__ kbuf, const T* __restrict__ vbuf, const T* __restrict__ shared,
                         const T* __restrict__ gate, T* __restrict__ out, uint32_t M, uint32_t base_pos) {
     typedef typename Vec<T>::x4 x4;
@@ -34,11 +90,13 @@ void attn_prompt_kernel(PromptAttn sh, const T* __restrict__ q, const T* __restr
     constexpr uint32_t NS = DQ / 16, ND = DV / 32;
     constexpr uint32_t KTOTAL = KT * DQ / 8, VTOTAL = (KT / 2) * (DV / 4);       // pieces of a tile
     constexpr uint32_t KP = (KTOTAL + NT - 1) / NT, VP = (VTOTAL + NT - 1) / NT;
+    constexpr bool DIRECT = sizeof(T) == 2, FOUR = prompt_four<T, DQ>();
+    constexpr uint32_t CHUNK = KT * 64, NCK = DQ / 32, NC = NCK + DV / 32, PAIR = NC * CHUNK;      // DIRECT: 32 columns of a tile, such chunks of K, of K and V, their bytes
     extern __shared__ __attribute__((aligned(16))) uint8_t ap_lds[];
     T* Ks = reinterpret_cast<T*>(ap_lds);
     T* Vt = Ks + KT * KS;
 
-    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, lq = lane & 31, lh = lane >> 5;
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6)), lq = lane & 31, lh = lane >> 5;
     const uint32_t qg = wave / KG, kh = wave % KG;       // query group, 32 keys of every key tile
     // latest (longest) query tiles first
     const uint32_t head = blockIdx.x % sh.heads, ntq = gridDim.x / sh.heads;
@@ -48,12 +106,16 @@ void attn_prompt_kernel(PromptAttn sh, const T* __restrict__ q, const T* __restr
     const float c2 = sh.scale * LOG2E;
     const uint32_t qrow = q0 + qg * 32 + lq, qpos = base_pos + qrow;
 
+    // requested at once: a row past the last takes the last one's, columns past dq any of the row's
     x8 qf[NS];
+    auto load_q = [&]() {
+        const T* row = q + ((size_t)min(qrow, M - 1) * sh.heads + head) * dq;
 #pragma unroll
-    for (uint32_t s = 0; s < NS; s++) {
-        const uint32_t d = 16 * s + 8 * lh;
-        qf[s] = (qrow < M && d < dq) ? load8(q + ((size_t)qrow * sh.heads + head) * dq + d) : zero8<T>();
-    }
+        for (uint32_t s = 0; s < NS; s++) qf[s] = load8(row + (16 * s < dq ? 16 * s : 0u) + 8 * lh);
+#pragma unroll
+        for (uint32_t s = 0; s < NS; s++)
+            if (16 * s >= dq) qf[s] = zero8<T>();
+    };
     v16f oacc[ND];
 #pragma unroll
     for (uint32_t d = 0; d < ND; d++)
@@ -112,65 +174,110 @@ void attn_prompt_kernel(PromptAttn sh, const T* __restrict__ q, const T* __restr
         }
     };
 
-    load_tile(tile0);
+    const uint32_t l_row = lane >> 2, l_col = ((lane & 3) ^ ((lane >> 4) & 3)) * 16;
+    const uint32_t k_lane = l_row * kst * 2 + l_col, c_lane = l_row * cst * 2 + l_col, v_lane = l_row * vst * 2 + l_col;
+    auto direct_tile = [&](uint32_t kt, uint32_t buf) {
+        const uint32_t r0 = kt * KT;
+        direct_rows<KT / 16, 0, NCK>(kbuf + (size_t)r0 * kst + kvh * sh.dim, kst, sh.dim, shared + (size_t)(kv_lo + r0) * cst, cst, dq, total - kv_lo - r0, k_lane, c_lane,
+                                     ap_lds + buf * PAIR, wave);
+        direct_rows<KT / 16, NCK, NC>(vbuf + (size_t)r0 * vst + kvh * sh.vdim, vst, sh.vdim, vbuf, 0, sh.vdim, total - kv_lo - r0, v_lane, 0, ap_lds + buf * PAIR, wave);
+    };
+    const uint32_t k_at = (kh * 32 + lq) * 64 + ((lh ^ ((lq >> 2) & 3)) * 16);       // odd steps of 16 columns: ^ 32
+    const uint32_t v_row = 4 * lh + ((lane & 15) >> 2), v_piece = 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1);
+    const uint32_t v_at = NCK * CHUNK + (kh * 32 + v_row) * 64 + ((v_piece ^ lh) * 16) + (lane & 1) * 8;      // 8 keys further on: + 512, ^ 32
+
+    if constexpr (DIRECT) direct_tile(tile0, tile0 & 1);
+    else load_tile(tile0);
+    load_q();
     for (uint32_t kt = tile0; kt < ntiles; kt++) {
-        __syncthreads();                      // the previous tile has been read
-        store_tile();
-        __syncthreads();
-        if (kt + 1 < ntiles) load_tile(kt + 1);
+        const uint8_t* pair = ap_lds + (kt & 1) * PAIR;
+        if constexpr (DIRECT) {
+            __builtin_amdgcn_s_waitcnt(0);        // this wave's share of the step's tiles is in LDS,
+            __syncthreads();                      // and so is everyone's; nobody reads the other pair any more
+            if (kt + 1 < ntiles) direct_tile(kt + 1, (kt + 1) & 1);
+        } else {
+            __syncthreads();                      // the previous tile has been read
+            store_tile();
+            __syncthreads();
+            if (kt + 1 < ntiles) load_tile(kt + 1);
+        }
         const uint32_t k0 = kv_lo + kt * KT + kh * 32;                                     // the wave's 32 keys
         if (!(wave_active && k0 <= wave_max && k0 + 32 > wave_lo)) continue;       // all in the wave's future, or before its windows
-        // two accumulators: a product waits for the one before the last
+        auto k_frag = [&](uint32_t s) {
+            if constexpr (DIRECT) return *reinterpret_cast<const x8*>(pair + (k_at ^ ((s & 1) * 32)) + (s >> 1) * CHUNK);
+            else return load8(Ks + (kh * 32 + lq) * KS + 16 * s + 8 * lh);
+        };
+        // two accumulators, where there are registers for them: a product waits for the one before the last
         v16f sacc, sodd;
 #pragma unroll
         for (int r = 0; r < 16; r++) sacc[r] = sodd[r] = 0.f;
 #pragma unroll
         for (uint32_t s = 0; s < NS; s += 2) {
-            sacc = mma32(load8(Ks + (kh * 32 + lq) * KS + 16 * s + 8 * lh), qf[s], sacc);
-            sodd = mma32(load8(Ks + (kh * 32 + lq) * KS + 16 * (s + 1) + 8 * lh), qf[s + 1], sodd);
+            sacc = mma32(k_frag(s), qf[s], sacc);
+            if constexpr (FOUR) sacc = mma32(k_frag(s + 1), qf[s + 1], sacc);
+            else sodd = mma32(k_frag(s + 1), qf[s + 1], sodd);
+        }
+        if constexpr (!FOUR) {
+#pragma unroll
+            for (int r = 0; r < 16; r++) sacc[r] += sodd[r];
         }
         if (k0 + 31 > wave_min || k0 < last_lo) {
 #pragma unroll
             for (int r = 0; r < 16; r++) {
                 const uint32_t t = k0 + 8 * (r >> 2) + 4 * lh + (r & 3);
-                sacc[r] = (t <= qpos && qpos - t < window) ? (sacc[r] + sodd[r]) * c2 : -INFINITY;
+                sacc[r] = (t <= qpos && qpos - t < window) ? sacc[r] : -INFINITY;
             }
-        } else {
-#pragma unroll
-            for (int r = 0; r < 16; r++) sacc[r] = (sacc[r] + sodd[r]) * c2;
         }
         float m_tile = sacc[0];
 #pragma unroll
         for (int r = 1; r < 16; r++) m_tile = fmaxf(m_tile, sacc[r]);
-        const float m_new = fmaxf(m_run, lane_xor_max<32>(m_tile));
-        const float m_exp = m_new == -INFINITY ? 0.f : m_new;            // no key seen yet: every weight is 2^-inf = 0
-        if (__builtin_amdgcn_ballot_w64(m_new > m_run) != 0) {
+        m_tile = lane_xor_max<32>(m_tile) * c2;      // c2 > 0
+        // A query's maximum follows only where a score has risen above it by more than SLACK: weights stay below 2^SLACK, and sums and output are relative to the
+        // same number whatever it is.
+        const bool risen = m_tile > m_run + LP_SLACK;
+        if (__builtin_amdgcn_ballot_w64(risen) != 0) {
+            const float m_new = risen ? m_tile : m_run;
             const float alpha = m_run == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run - m_new);
             l_run *= alpha;
 #pragma unroll
             for (uint32_t d = 0; d < ND; d++)
 #pragma unroll
                 for (int r = 0; r < 16; r++) oacc[d][r] *= alpha;
+            m_run = m_new;
         }
-        m_run = m_new;
+        const float m_exp = m_run == -INFINITY ? 0.f : m_run;            // no key seen yet: every weight is 2^-inf = 0
         x8 pb[2];
 #pragma unroll
         for (int j = 0; j < 2; j++)
 #pragma unroll
             for (int e = 0; e < 8; e++) {
-                const float p = __builtin_amdgcn_exp2f(sacc[8 * j + e] - m_exp);
+                const float p = __builtin_amdgcn_exp2f(fmaf(sacc[8 * j + e], c2, -m_exp));
                 l_run += p;
                 pb[j][e] = (T)p;
             }
         // element e of lane half lh is key 16 j + 8 (e / 4) + 4 lh + e % 4 of the wave's half
+        if constexpr (DIRECT) {
+            constexpr int N = ND > 1 ? 2 : 1;
+            const uint32_t base = (uint32_t)(uintptr_t)FH_LDS3(pair);
 #pragma unroll
-        for (int j = 0; j < 2; j++)
+            for (uint32_t d = 0; d < ND; d += N) {
+                v8bf vf[2][N];
+                read_v<N, CHUNK>(vf, base + v_at + d * CHUNK, base + (v_at ^ 32) + 512 + d * CHUNK);
 #pragma unroll
-            for (uint32_t d = 0; d < ND; d++) {
-                const T* vr = Vt + (d * 32 + lq) * VS + kh * 32 + 16 * j + 4 * lh;
-                const x4 v0 = *reinterpret_cast<const x4*>(vr), v1 = *reinterpret_cast<const x4*>(vr + 8);
-                oacc[d] = mma32((x8){v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]}, pb[j], oacc[d]);
+                for (int j = 0; j < 2; j++)
+#pragma unroll
+                    for (int i = 0; i < N; i++) oacc[d + i] = mma32(vf[j][i], pb[j], oacc[d + i]);
             }
+        } else {
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+#pragma unroll
+                for (uint32_t d = 0; d < ND; d++) {
+                    const T* vr = Vt + (d * 32 + lq) * VS + kh * 32 + 16 * j + 4 * lh;
+                    const x4 v0 = *reinterpret_cast<const x4*>(vr), v1 = *reinterpret_cast<const x4*>(vr + 8);
+                    oacc[d] = mma32((x8){v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]}, pb[j], oacc[d]);
+                }
+        }
     }
 
     // ---- merge: the first wave of a group takes the states of the others through LDS, 32 output columns at a time
@@ -234,15 +341,17 @@ void go_keys(const PromptAttn& a, uint32_t M, uint32_t base_pos, hipStream_t s) 
 
 template <typename T, int DQ, int DV>
 void go(const PromptAttn& a, uint32_t M, uint32_t base_pos, hipStream_t s) {
-    // Bound by the chain of tile steps (about 1.8 us each), not by work, as long as the workgroups are few: four waves to a query group while
-    // the workgroups of 64 queries are at most one a compute unit (that is how many run at a time) under a window, which makes them all equally
-    // long, and at most two without, where the short ones fill the gaps.  Whole prompts in ms, two / four: 9 heads with a window
-    // of 1024, 902 tokens (135 workgroups) 2.77 / 2.48, 1500 (216) 3.24 / 2.87, 2502 (360) 3.60 / 3.58; 9 heads without, 2502 3.69 / 3.51; 32
-    // heads without, 902 (480) 4.06 / 4.03, 2502 (1280) 8.79 / 8.82.  Shapes whose tiles of 128 keys fill LDS stay with two, and so do up to 64 keys,
-    // one tile for two waves: four would only load and merge more (30 layers of 9 heads, 2 tokens 0.16 / 0.19 ms, 64 tokens 0.19 / 0.22).
+    // Bound by the chain of tile steps (about 1.1 us each), not by work, as long as the workgroups are few: four waves to a query group while the workgroups of
+    // 64 queries are a few rounds of the chip, fewer under a window, which makes them all equally long, than without, where the short ones fill the gaps.  us, two /
+    // four, by workgroups of 64 queries.  bfloat16, up to 96 columns (two workgroups run on a compute unit): window, 9 heads 135 21.2 / 14.9, 360 26.4 / 22.2, 567
+    // 28.2 / 32.4; none, 9 to 32 heads 360 39.5 / 27.8, 480 47.3 / 32.9, 567 59.9 / 42.1, 756 72.5 / 61.1, 768 27.7 / 28.8, 1280 49.0 / 57.5.  128 columns (tiles of
+    // 128 keys are 128 KB, one workgroup to a compute unit), 24 heads 240 21.5 / 17.8, 360 28.2 / 28.1, 576 40.8 / 52.5.  32-bit (one to a compute unit as well), whole
+    // prompts of 9 heads in ms: window 135 2.77 / 2.48, 216 3.24 / 2.87, 360 3.60 / 3.58; none 360 3.69 / 3.51; 32 heads 480 4.06 / 4.03, 1280 8.79 / 8.82.  Shapes
+    // whose tiles of 128 keys do not fit stay with two, and so do up to 64 keys, one tile for two waves: four would only load and merge more (2 tokens 6.2 / 6.5 us).
     constexpr uint32_t CUS = 256;
-    const uint32_t at_most = a.window && a.window < base_pos + M ? CUS : 2 * CUS;
-    if constexpr (prompt_lds<T, DQ, DV, 4>() <= 80 * 1024)
+    const bool windowed = a.window && a.window < base_pos + M;
+    const uint32_t at_most = prompt_four<T, DQ>() ? (windowed ? 2 * CUS : 3 * CUS - 1) : sizeof(T) == 2 ? (windowed ? CUS : CUS * 3 / 2) : (windowed ? CUS : 2 * CUS);
+    if constexpr (sizeof(T) == 2 ? DQ <= 128 : prompt_lds<T, DQ, DV, 4>() <= 80 * 1024)
         if (base_pos + M > 64 && (uint64_t)((M + 63) / 64) * a.heads <= at_most) { go_keys<T, DQ, DV, 4>(a, M, base_pos, s); return; }
     go_keys<T, DQ, DV, 2>(a, M, base_pos, s);
 }

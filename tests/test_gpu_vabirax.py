@@ -359,6 +359,22 @@ def test_prompt_attention_forms(fh, vo, torch_gpu, tmp_path, heads, window):
         m.close()
 
 
+@pytest.mark.parametrize("heads,dim,rot,vdim,scale,window", [(90, 40, 8, 24, None, None), (34, 40, 8, 24, 6.0, 70), (62, 40, 8, 64, 2.0, 70), (45, 100, 20, 100, 2.0, None),
+                                                            (4, 100, 20, 100, None, 129), (3, 130, 60, 128, 2.0, None), (2, 190, 56, 256, 1.0, 300)])
+def test_prompt_attention_of_every_head_size(fh, vo, torch_gpu, tmp_path, heads, dim, rot, vdim, scale, window):
+    """The bfloat16 tiles of every size and both numbers of waves to a query group (90 heads, 530 rows: past 767 workgroups of 64 queries; 62 under a window: past 512;
+    45 of 128 columns: past 384), portions that begin anywhere in a tile, and scores whose maximum moves by more than the kernel lets it stand."""
+    c = Case(fh, vo, tmp_path, fh.synth.vabirax_config(48, 61, [fh.synth.vabirax_layer(heads, dim, rot, vdim, 32, 32, None, window, scale=scale)], embedding_scale=3.0))
+    ids = c.ids(700)
+    want = c.oracle.forward(ids)[0]
+    m = c.model(max_seq=700, dtype="bfloat16")
+    at = 0
+    for n in (70, 530, 100):
+        check(m.prefill_logits(ids[at:at + n], np.arange(n)), want[at:at + n], "bfloat16", np.sqrt((want ** 2).mean()))
+        at += n
+    m.close()
+
+
 # ---- generation, loading, replay --------------------------------------------------------------------------------------------------
 
 def test_greedy_generation(get):
