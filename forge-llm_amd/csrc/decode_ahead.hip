@@ -51,7 +51,7 @@ constexpr uint32_t PA_SUM = 24, PA_SSQ = 12;  // a row's products, and an accumu
 // a polling thread takes of the residual row and of gate;up's quantised vector; AW: waves that attend to a head, each to 64 keys.
 //   Narrow (up to 768 channels): a layer in 54 registers of a few dozen workgroups; the heads have workgroups of their own, up to 768 rows of context.
 //   Wide (up to 2048 channels): every compute unit holds a block of 32 gate;up rows in two sets of registers, so heads and weights share workgroups: the last `heads` of
-//   them hold no rows of q;k;v and o, and their fetching waves attend, to up to 256 rows (longer contexts, order free: every workgroup's, PaPart).  down takes the place of the second set when that is done.
+//   them hold no rows of q;k;v and o, and their fetching waves attend, to up to 256 rows (longer contexts, order free: every workgroup's, PaPart).  down takes the place of one of them when that is done.
 struct PaNarrow { static constexpr int UQ = 1, UO = 1, UG1 = 3, UG2 = 0, UD = 1, UL = 4, NX = 3, NV = 3; static constexpr uint32_t AW = PA_WAVES; static constexpr bool WIDE = false; };
 struct PaWide { static constexpr int UQ = 2, UO = 2, UG1 = 4, UG2 = 4, UD = 4, UL = 4, NX = 8, NV = 9; static constexpr uint32_t AW = PA_POLL; static constexpr bool WIDE = true; };
 
@@ -170,7 +170,8 @@ template <int U, PaFmt W> struct PaSet { int4 v[W == PA_Q4 ? U : 2 * U]; uint32_
 template <PaFmt W>
 __device__ __forceinline__ uint32_t pa_own(uint32_t j, uint32_t lane) { return W == PA_Q4 ? 64 * j + lane : 64 * j + 32 * (lane & 1u) + (lane >> 1); }
 
-template <int J0 = 0, int U, PaFmt W>
+// [A, B): the rounds of the set that are requested (B = -1: up to its last).
+template <int J0 = 0, int A = 0, int B = -1, int U, PaFmt W>
 __device__ __forceinline__ void pa_load(PaSet<U, W>& w, const PaWeights& mat, const PaTask& t, uint32_t lane) {
     asm volatile("" : "+v"(lane));           // the addresses are worked out here: kept from layer to layer they would not fit the registers
     // Blocks past the last one re-read it, and a wave without rows reads the matrix's first block: with no condition around them the loads in flight are
@@ -181,7 +182,7 @@ __device__ __forceinline__ void pa_load(PaSet<U, W>& w, const PaWeights& mat, co
         return t.base + u + (u >= t.seg ? t.jump : 0u);
     };
 #pragma unroll
-    for (int j = 0; j < U; j++) {
+    for (int j = A; j < (B < 0 ? U : B); j++) {
         if (W == PA_Q4) {
             w.v[j] = pa_at<int4>(mat.qs, at(64 * (J0 + j) + lane) * 16);
         } else {
@@ -1036,7 +1037,16 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
             PaSet<F::UQ, W> wq;
             PaSet<F::UO, W> wo;
             PaSet<F::UG1, W> wg;
-            PaSet<F::WIDE ? F::UG2 : F::UD, W> wd;                              // Wide: first gate;up's second part, then down
+            PaSet<F::WIDE ? F::UG2 : F::UD, W> wd;                              // Wide: first gate;up's second part, then (unless EARLY) down
+            // EARLY: down's weights take the place of gate;up's first part, half of them requested ahead of the second part's products and half behind: the memory has work
+            // while a workgroup computes, and what the result's store and the next poll wait behind is on its way by then.  (All of down behind the results' barrier / this, 1B
+            // shape, us a token by rows of context: Q8_0 33 430 / 400, 300 463 / 432, 2400 477 / 448, order-faithful 33 471 / 442; Q4_K and Q6_K 33 487 / 460, 2400 539 / 504;
+            // 8 layers of 1024 channels Q8_0 151 / 151, of 1280 163 / 160.  All of down ahead of the second part's products 472 for the first of these, none of it 412, its second
+            // half behind the row sums' barrier 418.)  Not Q4_0: half the bytes to wait for; 403 / 386, but models of 1024 channels 150 / 153.  The other sets gain little or
+            // nothing from an earlier place: q;k;v ahead of down's products 1 % (1024 channels 2 % slower), gate;up's second part ahead of o's products 2 to 6 us slower.
+            constexpr bool EARLY = F::WIDE && W != PA_Q4;
+            static_assert(!EARLY || F::UG1 == F::UD, "down takes the place of gate;up's first part");
+            constexpr int HALF = F::UD / 2;
             float4 n2;
             n1 = load_norm(pa_lds_ptr(layers[0].norm[0]));
             pa_load(wq, pa_lds_ptr(layers[0].w[0]), tq, cx.lane);
@@ -1089,18 +1099,25 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
                     const auto x = pa_index<F::UG1, W>(tg, mg, a.off_as, pg, cx.lane);
                     if (!norm_computing(n2)) return;
                     pa_products(wg, x, tg, smem, a.to_sums);
-                    if constexpr (F::WIDE) pa_products<F::UG1>(wd, pa_index<F::UG2, W, F::UG1>(tg, mg, a.off_as, pg, cx.lane), tg, smem, a.to_sums);
+                    if constexpr (F::WIDE) {
+                        if constexpr (EARLY) pa_load<0, 0, HALF>(wg, pa_lds_ptr(L.w[3]), td, cx.lane);
+                        pa_products<F::UG1>(wd, pa_index<F::UG2, W, F::UG1>(tg, mg, a.off_as, pg, cx.lane), tg, smem, a.to_sums);
+                        if constexpr (EARLY) pa_load<0, HALF>(wg, pa_lds_ptr(L.w[3]), td, cx.lane);
+                    }
                     const PaSum v = pa_row_sum<ORD>(mg, 2 * per_wave, smem + pg, cx.lane);
                     const float up = ORD ? lane_xor<4>(v.v) : lane_xor<32>(v.v);           // row r + 4 of 8
                     if (v.on && v.row < per_wave) silu[c * per_wave + v.row] = (v.v / (1.0f + expf_ref_with<true>(-v.v, PaExpTab{exp_tab}))) * up;      // silu_mul, emit.rs:380-386
                     __syncthreads();
+                } else if constexpr (EARLY) {
+                    pa_load(wg, pa_lds_ptr(L.w[3]), td, cx.lane);
                 }
-                if constexpr (F::WIDE) pa_load(wd, pa_lds_ptr(L.w[3]), td, cx.lane);
+                if constexpr (F::WIDE && !EARLY) pa_load(wd, pa_lds_ptr(L.w[3]), td, cx.lane);
                 if (on_d) {
                     const auto x = pa_index<F::UD, W>(td, md, a.off_as, pd, cx.lane);
                     __syncthreads();
                     if (sh_abort) return;
-                    pa_products(wd, x, td, smem, a.to_sums);
+                    if constexpr (EARLY) pa_products(wg, x, td, smem, a.to_sums);
+                    else pa_products(wd, x, td, smem, a.to_sums);
                     const PaSum v = pa_row_sum<ORD>(md, md.R, smem + pd, cx.lane);
                     if (v.on) out[c * md.R + v.row] = v.v;
                     __syncthreads();
