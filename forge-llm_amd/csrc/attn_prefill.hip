@@ -10,13 +10,12 @@
 // ds_read_b64_tr_b16 transposes on the way out.  (Through registers, with V transposed on the way in, a third of a step went into issuing the
 // loads and writing them to LDS, and the registers they took left two waves per SIMD where three fit now.)
 // Scores stay in the base-2 domain (s * scale * log2 e) so that the exponential is one v_exp_f32 after one FMA; keys are masked only in
-// tiles that reach past the wave's first query; the maximum that a query's scores are taken against, and its accumulators with it, move only
-// when one rises above it by more than 2^SLACK (before: whenever it rose, which with 32 queries to a wave is most steps
-// of a prompt of a few thousand tokens, 50 multiplications of about 190 VALU instructions each time).
+// tiles that reach past the wave's first query; accumulators are rescaled only when some query's maximum rises.  (Letting a maximum stand until a score passes
+// it by 2^8 saves 3 of 80 us at 3001 tokens, but the largest weight is then no longer exactly 1 in fp16: error against 64 bits 2.45e-4 instead of 2.35e-4.  Not kept.)
 // What bounds it: full, the matrix unit, the VALU (32 exp, 32 FMA, 32 additions, 16 conversions, 16 maxima per 32 x 64 scores) and LDS reads
-// take about 800 cycles each and overlap to 1800 (heads of 96, 3072 queries behind 8192 keys 390 us = 0.94 PFLOP/s, 128 1.0, 64 0.9; the
-// library's large bf16 product is at 1.2); causal, the uneven length of the query tiles on top.  3001 tokens: 32/32 heads of 96 97.7 -> 74.5 us,
-// 32/8 of 128 124 -> 89, 2502 tokens of 32/8 of 64 52.5 -> 42.7, 1000 of 32/8 of 128 38.2 -> 24.0.
+// take about 800 cycles each and overlap to 1800 (heads of 96, 3072 queries behind 8192 keys 408 us = 0.90 PFLOP/s, 128 0.93, 64 0.81; the
+// library's large bf16 product is at 1.2); causal, the uneven length of the query tiles on top.  3001 tokens: 32/32 heads of 96 97.7 -> 82 us,
+// 32/8 of 128 124 -> 95, 2502 tokens of 32/8 of 64 52.5 -> 45.1, 1000 of 32/8 of 128 38.2 -> 26.7.
 // Measured and not kept: query tiles of every other round in ascending order: within 2 %.
 //
 // Both products are computed transposed, S^T = K Q^T and O^T = V^T P^T.  In the 32x32 MFMA
@@ -39,7 +38,6 @@ constexpr int QB = 128;       // queries per workgroup
 constexpr int KT = 64;        // keys per tile
 constexpr int AP_THREADS = 512;   // the 8-wave form; the 4-wave form runs 256
 constexpr uint32_t AP_RSRC_FLAGS = 0x00020000;   // raw buffer, 32-bit data format
-constexpr float SLACK = 8.f;      // base-2 exponent
 
 #define FH_LDS3(p) ((__attribute__((address_space(3))) void*)(p))
 
@@ -175,7 +173,7 @@ void attn_prefill_kernel(const float* __restrict__ q, const uint16_t* __restrict
 
     load_tiles(tile0, tile0 & 1);
     // ---- Q fragment (B operand of S^T = K Q^T): lane (lq, lh) holds q[row][16 s + 8 lh + 0..7].  All of it is requested at once (a row past the
-    // last takes the last one's): with a condition around each load they waited for one another (3001 tokens of 32/32 heads of 96 76.3 us, now 74.5).
+    // last takes the last one's): with a condition around each load they waited for one another (3001 tokens of 32/32 heads of 96: 1.8 us more).
     v8h qf[NS];
     {
         const float4* p = reinterpret_cast<const float4*>(q + (size_t)min(qrow, M - 1) * q_stride + head * HD + 8 * lh);
@@ -235,9 +233,7 @@ void attn_prefill_kernel(const float* __restrict__ q, const uint16_t* __restrict
 #pragma unroll
                 for (int r = 0; r < 16; r++) m_tile = fmaxf(m_tile, sacc[h][r]);
             m_tile = lane_xor_max<32>(m_tile) * c2;      // c2 > 0: max commutes with the scaling
-            // The maximum that a query's scores are taken against follows only where one has risen above it by more than SLACK: p stays below 2^SLACK,
-            // and l and O are relative to the same number whatever it is.  (Each query by itself: its result does not depend on its neighbours.)
-            const bool risen = m_tile > m_run + SLACK;
+            const bool risen = m_tile > m_run;
             if (__builtin_amdgcn_ballot_w64(risen) != 0) {
                 const float m_new = risen ? m_tile : m_run;
                 const float alpha = m_run == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run - m_new);

@@ -19,12 +19,11 @@ constexpr float LOG2E = 1.4426950408889634f;
 //   32-bit    Through registers into one buffer (K row-major: the head's own part, the shared part; V transposed), two barriers a step.
 // What bounds it: up to a few hundred workgroups the chain of steps, each a trip through LDS, two products and the exponentials between them; then the VALU (exponentials,
 // maxima, conversions) beside the matrix unit.  In bfloat16 a step through registers took 1.8 us, half of it the loads' issue and the writes to LDS, and its registers left
-// one workgroup to a compute unit; now 1.1, and two.  us, before / now: 9 heads of 64 + 32 with a window of 1024, 902 tokens 18.4 / 14.7, 2502 36.0 / 22.2, 4000 47.1 /
-// 28.3; 32/8 heads of 64 902 23.2 / 15.2, 2502 92.7 / 48.5; 24/8 of 128 2502 101.9 / 76.7; 16 of 128 + 64 902 40.1 / 30.9, 4000 169 / 135; 33 tokens the same.
+// one workgroup to a compute unit; now 1.1, and two.  us, before / now: 9 heads of 64 + 32 with a window of 1024, 902 tokens 18.4 / 14.9, 2502 36.0 / 22.4, 4000 47.1 /
+// 29.5; 32/8 heads of 64 902 23.2 / 15.7, 2502 92.7 / 51.8; 24/8 of 128 2502 101.9 / 85; 16 of 128 + 64 902 40.1 / 33.1, 4000 169 / 141; 33 tokens the same.
 // DQ >= dim + rot and DV >= vdim: the register tiles' sizes; columns past the real ones are zero.
 constexpr uint32_t LP_THREADS = 512;
 constexpr uint32_t LP_RSRC_FLAGS = 0x00020000;   // raw buffer, 32-bit data format
-constexpr float LP_SLACK = 8.f;                  // base-2 exponent
 template <typename T, int DQ> constexpr bool prompt_four() { return sizeof(T) == 2 && DQ <= 96; }      // four waves to a SIMD
 template <typename T, int DQ, int DV, int KG> constexpr uint32_t prompt_lds() {
     const uint32_t tiles = sizeof(T) == 2 ? 2 * 32 * KG * (DQ + DV) * 2 : (32 * KG * (DQ + 16 / sizeof(T)) + DV * (32 * KG + 8 / sizeof(T))) * sizeof(T),
@@ -232,9 +231,7 @@ void attn_prompt_kernel(PromptAttn sh, const T* __restrict__ q, const T* __restr
 #pragma unroll
         for (int r = 1; r < 16; r++) m_tile = fmaxf(m_tile, sacc[r]);
         m_tile = lane_xor_max<32>(m_tile) * c2;      // c2 > 0
-        // A query's maximum follows only where a score has risen above it by more than SLACK: weights stay below 2^SLACK, and sums and output are relative to the
-        // same number whatever it is.
-        const bool risen = m_tile > m_run + LP_SLACK;
+        const bool risen = m_tile > m_run;
         if (__builtin_amdgcn_ballot_w64(risen) != 0) {
             const float m_new = risen ? m_tile : m_run;
             const float alpha = m_run == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run - m_new);

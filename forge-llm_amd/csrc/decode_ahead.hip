@@ -1,7 +1,7 @@
 // One decode token as ONE kernel whose waves hold their share of a layer's matrices in registers (model::forward, emit.rs:4029-4227).
 //
 // A step is a chain of four products and an attention per layer.  As kernels a link of that chain is 4 to 6 us however small (a launch that does nothing takes
-// 2.7); as phases of the kernel that streams weights of any size (decode_persistent.hip) it is 5.  Here a layer of SmolLM2-135M takes 12 us, one of the 1B shape 23
+// 2.7); as phases of the kernel that streams weights of any size (decode_persistent.hip) it is 5.  Here a layer of SmolLM2-135M takes 12 us, one of the 1B shape 21
 // (its 65 MB alone take 14): five hand-overs of 0.8 to 1.2 (1.5 to 2.5 beside weights), two norms of 0.7, attention 3.2, and the products.
 //   * A wave's rows are a few registers, requested where nothing is on its way to the compute unit: while the attention is at work, and with wide models also right
 //     behind the products.  (A compute unit's loads return in order and its queue is short: a poll behind weights comes when they have come, and so does a store.)
@@ -18,11 +18,11 @@
 // order-faithful kernel sequence; narrow models, to which the order costs nothing, run it in both modes.  Otherwise row sums and the norm's sum add up as the lanes
 // have them.  Per token in us, kernel sequence (order-faithful mode) / decode_persistent.hip (fast mode) / this, by rows of context:
 //   SmolLM2-135M Q8_0   33: 781 / 880 / 384    300: 820 / 878 / 421    740: 907 / 876 / 466
-//   1B shape Q8_0       33: 754 / 610 / 469 and 433 (order-faithful, fast)    200: - / 636 / 476 and 441       Q4_0, fast: 33: 532 / 403
-//   and in fast mode (PaPart) 300: 637 / 464    1000: 642 / 471    2400: 644 / 479    5000: 676 / 515    Q4_0 2400: 570 / 442
-//   and of Q4_K / Q6_K matrices (llama.cpp's Q4_K_M recipe), 1B shape 33: 623 / 489    300: 646 / 527    2400: 655 / 543    5000: 688 / 580
+//   1B shape Q8_0       33: 754 / 610 / 450 and 400 (order-faithful, fast)    200: - / 636 / 458 and 420       Q4_0, fast: 33: 532 / 403
+//   and in fast mode (PaPart) 300: 637 / 442    1000: 642 / 447    2400: 644 / 459    5000: 676 / 495    Q4_0 2400: 570 / 441
+//   and of Q4_K / Q6_K matrices (llama.cpp's Q4_K_M recipe), 1B shape 33: 623 / 457    300: 646 / 495    2400: 655 / 511    5000: 688 / 548
 // Heads of 96 and 128 gain as much though those of 128 spill (8 layers, 33 rows, fast: 8/2 of 96 at 768 channels 213 / 136, 6/2 of 128 207 / 138, 16/4 of 96 at 1536 246 / 174,
-// 12/4 of 128 at 1024 212 / 168).  A layer's weights hardly count (1B shape, us: Q8_0 23, Q4_0 22): it is the chain that takes the time.
+// 12/4 of 128 at 1024 212 / 168).  A layer's weights hardly count (1B shape, us: Q8_0 21, Q4_0 21): it is the chain that takes the time.
 #include <stddef.h>
 #include <string.h>
 
@@ -1040,7 +1040,7 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
             PaSet<F::WIDE ? F::UG2 : F::UD, W> wd;                              // Wide: first gate;up's second part, then (unless EARLY) down
             // EARLY: down's weights take the place of gate;up's first part, half of them requested ahead of the second part's products and half behind: the memory has work
             // while a workgroup computes, and what the result's store and the next poll wait behind is on its way by then.  (All of down behind the results' barrier / this, 1B
-            // shape, us a token by rows of context: Q8_0 33 430 / 400, 300 463 / 432, 2400 477 / 448, order-faithful 33 471 / 442; Q4_K and Q6_K 33 487 / 460, 2400 539 / 504;
+            // shape, us a token by rows of context: Q8_0 33 430 / 400, 300 463 / 440, 2400 477 / 457, order-faithful 33 471 / 450; Q4_K and Q6_K 33 487 / 457, 2400 539 / 511;
             // 8 layers of 1024 channels Q8_0 151 / 151, of 1280 163 / 160.  All of down ahead of the second part's products 472 for the first of these, none of it 412, its second
             // half behind the row sums' barrier 418.)  Not Q4_0: half the bytes to wait for; 403 / 386, but models of 1024 channels 150 / 153.  The other sets gain little or
             // nothing from an earlier place: q;k;v ahead of down's products 1 % (1024 channels 2 % slower), gate;up's second part ahead of o's products 2 to 6 us slower.
