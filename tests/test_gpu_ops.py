@@ -614,7 +614,7 @@ def test_attention_prefill_parity(fh, oracle, torch_gpu, heads, kv_heads, hd, M,
 ])
 def test_attention_prefill_running_maximum(fh, torch_gpu, hd, heads, M, base, window, ramp):
     """Both forms of the prompt kernel, with scores that rise or fall along the keys (`ramp`: by how much per key, in powers of two): the maximum
-    that they are taken against follows late.  p is rounded to fp16 (2^-11), scores and sums are 32-bit: 2^-10 of the largest value is enough."""
+    that they are taken against moves in every tile or in none.  p is rounded to fp16 (2^-11), scores and sums are 32-bit: 2^-10 of the largest value is enough."""
     torch = torch_gpu
     g = torch.Generator(device="cuda").manual_seed(M + hd)
     seq = base + M

@@ -363,7 +363,7 @@ def test_prompt_attention_forms(fh, vo, torch_gpu, tmp_path, heads, window):
                                                             (4, 100, 20, 100, None, 129), (3, 130, 60, 128, 2.0, None), (2, 190, 56, 256, 1.0, 300)])
 def test_prompt_attention_of_every_head_size(fh, vo, torch_gpu, tmp_path, heads, dim, rot, vdim, scale, window):
     """The bfloat16 tiles of every size and both numbers of waves to a query group (90 heads, 530 rows: past 767 workgroups of 64 queries; 62 under a window: past 512;
-    45 of 128 columns: past 384), portions that begin anywhere in a tile, and scores whose maximum moves by more than the kernel lets it stand."""
+    45 of 128 columns: past 384), portions that begin anywhere in a tile, and scores of a wide range."""
     c = Case(fh, vo, tmp_path, fh.synth.vabirax_config(48, 61, [fh.synth.vabirax_layer(heads, dim, rot, vdim, 32, 32, None, window, scale=scale)], embedding_scale=3.0))
     ids = c.ids(700)
     want = c.oracle.forward(ids)[0]
