@@ -202,9 +202,22 @@ void cut(const float* l, uint64_t n, float sum, const uint32_t* count, uint64_t 
             m += count[floor];
             if (count[floor]) mass += (double)count[floor] * float_of((floor << BUCKET_SHIFT) | (1u << (BUCKET_SHIFT - 1)));
         }
+        // The order is that of the quotients, and numbers that differ may have the same: what has the quotient of the least number of the last
+        // bucket stands beside it, whichever bucket it is in (a bit pattern or two below; many where quotients are denormal).
+        uint32_t least = floor << BUCKET_SHIFT;
+        if (least > 0) {
+            const float p = float_of(least) / sum;
+            uint32_t below = 0;                                    // float_of(below - 1) / sum < p <= float_of(least) / sum
+            while (below < least) {
+                const uint32_t mid = below + (least - below) / 2;
+                if (float_of(mid) / sum < p) below = mid + 1;
+                else least = mid;
+            }
+            for (uint32_t b = least >> BUCKET_SHIFT; b < floor; b++) m += count[b];      // room for as many
+        }
         room.resize(3 * (m + 16));
         uint32_t *key = room.data(), *index = key + m + 16, *spare = index + m + 16;
-        forms().collect(l, 0, n, floor << BUCKET_SHIFT, key, index);
+        m = forms().collect(l, 0, n, least, key, index);
         std::vector<uint32_t> sorted(m);
         for (uint64_t i = 0; i < m; i++) key[i] = bits_of(float_of(key[i]) / sum);
         uint32_t hi = 0, lo = UINT32_MAX;
@@ -221,7 +234,7 @@ void cut(const float* l, uint64_t n, float sum, const uint32_t* count, uint64_t 
                 if (cumsum > top_p) { crossed = true; break; }
             }
         } else keep = end;
-        if (!crossed && keep < most && floor > 0) continue;
+        if (!crossed && keep < most && least > 0) continue;
         if (!crossed && keep == n) { out->all = true; return; }
         out->index.resize(keep + 1);
         out->p.resize(keep + 1);

@@ -122,6 +122,43 @@ def test_sample_equals_oracle_over_sizes(fh, oracle, so, n, kind):
         assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
 
 
+@pytest.mark.parametrize("kind", ["maximum", "edges", "hot", "small"])
+def test_sample_equals_oracle_among_equal_quotients(fh, oracle, so, kind):
+    """Exponentials that differ and have the same quotient by their sum: equal probabilities, of which the lower index comes first.  They lie on either side of every line a
+    selection by exponentials can draw: next to the maximum, around the sixteenths of a power of two, all within a few units (hot), and where quotients are denormal (small)."""
+    rng = np.random.default_rng(19)
+    differ = 0
+    for trial in range(120):
+        n = int(rng.integers(3, 700)) if trial % 10 else 4111
+        temp = 1.0
+        l = (rng.normal(size=n) * 0.1 - 2.0).astype(np.float32)
+        if kind == "maximum":
+            top = np.float32(rng.uniform(-1.9, 1.0))
+            l = np.minimum(l, top - np.float32(0.1))
+            l[rng.integers(0, n, 4)] = np.nextafter(top, np.float32(-9))
+            l[n - 1] = top
+        elif kind == "edges":
+            edge = (16 + rng.integers(0, 16)) / 16 * 2.0 ** -rng.integers(1, 9)
+            near = rng.random(n) < 0.5
+            l[near] = (np.float32(np.log(edge)) * (1 + rng.integers(-4, 5, near.sum()) * 2.0 ** -23)).astype(np.float32)
+            l[n - 1] = 0.0
+        elif kind == "hot":
+            temp = float(np.float32(10.0 ** rng.uniform(5, 8)))
+        else:
+            edge = int(rng.integers(1, 40)) * 2.0 ** (19 - 149)
+            l[:] = (np.float32(np.log(edge)) * (1 + rng.integers(-1, 2, n) * 2.0 ** -23)).astype(np.float32)
+            l[rng.integers(0, n, max(1, n // 8))] = 0.0
+            l[n - 1] = 0.0
+        top_k, top_p = [(1, 1.0), (int(rng.integers(1, n)), 1.0), (0, float(rng.uniform(0.05, 0.999))), (int(rng.integers(1, n)), float(rng.uniform(0.3, 0.999)))][trial % 4]
+        if kind == "small" and trial % 4 < 2:
+            top_k, top_p = max(1, int((np.exp(l) >= np.float32(edge)).sum())), 1.0
+        a, b = l.copy(), l.copy()
+        tok_l, state_l = fh.ops.sample(a, temp, top_k, top_p, 0x1234567 + trial)
+        tok_o, state_o = so.sample(oracle, b, temp, top_k, top_p, 0x1234567 + trial)
+        differ += (tok_l, state_l) != (tok_o, state_o) or not np.array_equal(a.view(np.uint32), b.view(np.uint32))
+    assert differ == 0
+
+
 @pytest.mark.parametrize("temp,top_k,top_p", [(1.0, 0, 1.0), (0.7, 0, 1.0), (0.8, 40, 1.0), (1.0, 0, 0.9), (0.7, 40, 0.9), (1.3, 5, 0.5),
                                                (0.5, 0, 0.3), (2.0, 1000, 0.99)])
 def test_sample_equals_oracle_and_brackets_r(fh, oracle, so, temp, top_k, top_p):
