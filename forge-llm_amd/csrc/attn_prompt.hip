@@ -102,7 +102,10 @@ void attn_prompt_kernel(PromptAttn sh, const T* __restrict__ q, const T* __restr
     const uint32_t q0 = (ntq - 1 - blockIdx.x / sh.heads) * QB;
     const uint32_t kvh = head / sh.group, kv_lo = sh.kv_lo, ld_out = sh.ld_out;
     const uint32_t dq = sh.dim + sh.rot, window = sh.window ? sh.window : 0xFFFFFFFFu;
-    const float c2 = sh.scale * LOG2E;
+    // A folder may give any scale.  32-bit: scores are scaled, then masked.  bfloat16: they are masked and compared ahead of their scale, which wants it above 0: a negative one
+    // turns the query's sign, and where it is less than the least normal number (or 0) that number stands in, by which the weights of all finite products are alike.
+    const bool turned = DIRECT && sh.scale < 0.f;
+    const float c2 = DIRECT ? fmaxf(fabsf(sh.scale * LOG2E), 0x1p-126f) : sh.scale * LOG2E, later = DIRECT ? c2 : 1.f;
     const uint32_t qrow = q0 + qg * 32 + lq, qpos = base_pos + qrow;
 
     // requested at once: a row past the last takes the last one's, columns past dq any of the row's
@@ -114,6 +117,10 @@ void attn_prompt_kernel(PromptAttn sh, const T* __restrict__ q, const T* __restr
 #pragma unroll
         for (uint32_t s = 0; s < NS; s++)
             if (16 * s >= dq) qf[s] = zero8<T>();
+        if (turned) {
+#pragma unroll
+            for (uint32_t s = 0; s < NS; s++) qf[s] = -qf[s];
+        }
     };
     v16f oacc[ND];
 #pragma unroll
@@ -218,7 +225,7 @@ void attn_prompt_kernel(PromptAttn sh, const T* __restrict__ q, const T* __restr
         }
         if constexpr (!FOUR) {
 #pragma unroll
-            for (int r = 0; r < 16; r++) sacc[r] += sodd[r];
+            for (int r = 0; r < 16; r++) sacc[r] = DIRECT ? sacc[r] + sodd[r] : (sacc[r] + sodd[r]) * c2;
         }
         if (k0 + 31 > wave_min || k0 < last_lo) {
 #pragma unroll
@@ -230,7 +237,7 @@ void attn_prompt_kernel(PromptAttn sh, const T* __restrict__ q, const T* __restr
         float m_tile = sacc[0];
 #pragma unroll
         for (int r = 1; r < 16; r++) m_tile = fmaxf(m_tile, sacc[r]);
-        m_tile = lane_xor_max<32>(m_tile) * c2;      // c2 > 0
+        m_tile = lane_xor_max<32>(m_tile) * later;
         const bool risen = m_tile > m_run;
         if (__builtin_amdgcn_ballot_w64(risen) != 0) {
             const float m_new = risen ? m_tile : m_run;
@@ -248,7 +255,7 @@ void attn_prompt_kernel(PromptAttn sh, const T* __restrict__ q, const T* __restr
         for (int j = 0; j < 2; j++)
 #pragma unroll
             for (int e = 0; e < 8; e++) {
-                const float p = __builtin_amdgcn_exp2f(fmaf(sacc[8 * j + e], c2, -m_exp));
+                const float p = __builtin_amdgcn_exp2f(fmaf(sacc[8 * j + e], later, -m_exp));
                 l_run += p;
                 pb[j][e] = (T)p;
             }

@@ -100,6 +100,21 @@ def test_prompts_of_every_length_around_the_tiles(get, name, dtype):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("scale", [0.0, -0.3])
+def test_scores_scaled_by_zero_and_less(fh, ko, torch_gpu, tmp_path, scale, dtype):
+    """A folder may give any finite scale: every earlier key alike, or the least product first."""
+    cfg = fh.synth.kakirax_config(48, 61, [fh.synth.kakirax_attention(4, 2, 40, 24, None, scale=scale)], embedding_scale=3.0)
+    c = Case(fh, ko, tmp_path, cfg, fh.synth.folder_tensors(cfg, 5, fh.synth.kakirax_shapes(cfg)))
+    ids = c.ids(200)
+    want = c.oracle.forward(ids)[0]
+    rms = np.sqrt((want ** 2).mean())
+    m = c.model(dtype=dtype)
+    check(m.prefill_logits(ids[:180], np.arange(180)), want[:180], dtype, rms)
+    check(decode_all(m, ids[180:]), want[180:], dtype, rms)
+    m.close()
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 def test_requests_one_after_the_other(get, dtype):
     """What an earlier, longer request left in the cache, in the states and in the scratch areas does not show: the bits of a fresh
     model, whether a request begins with a prompt or with a decoded token."""

@@ -375,6 +375,22 @@ def test_prompt_attention_of_every_head_size(fh, vo, torch_gpu, tmp_path, heads,
     m.close()
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("scale", [0.0, -0.3, -2.0])
+@pytest.mark.parametrize("dim,rot,window", [(40, 8, None), (40, 8, 70), (130, 60, None)])
+def test_scores_scaled_by_zero_and_less(fh, vo, torch_gpu, tmp_path, dim, rot, window, scale, dtype):
+    """A folder may give any finite scale: every visible key alike, or the least product first.  Prompts, with rows behind a mask in every tile, and decoded tokens."""
+    c = Case(fh, vo, tmp_path, fh.synth.vabirax_config(48, 61, [fh.synth.vabirax_layer(3, dim, rot, 24, 32, 32, None, window, scale=scale)], embedding_scale=3.0))
+    ids = c.ids(240)
+    want = c.oracle.forward(ids)[0]
+    rms = np.sqrt((want ** 2).mean())
+    m = c.model(dtype=dtype)
+    check(m.prefill_logits(ids[:50], np.arange(50)), want[:50], dtype, rms)
+    check(m.prefill_logits(ids[50:220], np.arange(170)), want[50:220], dtype, rms)
+    check(decode_all(m, ids[220:]), want[220:], dtype, rms)
+    m.close()
+
+
 # ---- generation, loading, replay --------------------------------------------------------------------------------------------------
 
 def test_greedy_generation(get):
