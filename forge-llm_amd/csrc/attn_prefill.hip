@@ -247,6 +247,7 @@ void attn_prefill_kernel(const float* __restrict__ q, const uint16_t* __restrict
             // a query that has seen no key yet (all of these keys masked for it) keeps m = -inf: exponentiate
             // against 0 instead, every p is then 2^-inf = 0
             const float m_exp = m_run == -INFINITY ? 0.f : m_run;
+            float l_tile = 0.f;      // a tile's own: one by one onto the sum of thousands, weights that are alike are rounded alike
             v8h pb[KH][2];
 #pragma unroll
             for (int h = 0; h < KH; h++)
@@ -255,9 +256,10 @@ void attn_prefill_kernel(const float* __restrict__ q, const uint16_t* __restrict
 #pragma unroll
                     for (int e = 0; e < 8; e++) {
                         const float p = __builtin_amdgcn_exp2f(fmaf(sacc[h][8 * j + e], c2, -m_exp));   // 2^-inf = 0 for masked keys
-                        l_run += p;
+                        l_tile += p;
                         pb[h][j][e] = (_Float16)p;
                     }
+            l_run += l_tile;
             // ---- O^T += V^T P^T over this wave's keys
 #pragma unroll
             for (int h = 0; h < KH; h++) {

@@ -634,6 +634,28 @@ def test_attention_prefill_running_maximum(fh, torch_gpu, hd, heads, M, base, wi
         assert (got[:, h].double() - want).abs().max().item() <= 2.0 ** -10 * v.abs().max().item()
 
 
+@pytest.mark.parametrize("hd,heads,M", [(64, 2, 64), (96, 2, 64), (128, 2, 64), (64, 128, 512), (96, 128, 512), (128, 128, 512)])      # eight waves to a workgroup, four
+def test_attention_prefill_sum_of_many_like_weights(fh, torch_gpu, hd, heads, M):
+    """32768 keys of one weight, about 0.15 to 0.02 by the query, behind two of weight 1, and values of 1: the quotient of two sums, of the weights in fp16 and in 32 bits.  A lane adds
+    up 16 or 32 of them at a time: its sums of up to 512 such parts are off by 512 2^-24 at most, those of the products, 16 keys at a time, by twice that."""
+    torch = torch_gpu
+    seq = 32768
+    base = seq - M
+    t = -1.9 * (1 + torch.arange(M * heads, device="cuda").double() / (M * heads)).reshape(M, heads)
+    q = torch.zeros(M, heads, hd, device="cuda")
+    q[..., 0] = (t * hd ** 0.5).half().float()
+    k = torch.zeros(seq, 1, hd, device="cuda").half()
+    k[:, :, 0] = 1.0
+    k[[0, 32], :, 0] = 0.0                                  # in either half of a tile
+    v = torch.ones(seq, hd, device="cuda").half()
+    got = fh.ops.attention_flash_batch(q.reshape(M, -1), k.reshape(seq, -1).view(torch.int16), v.view(torch.int16), base, heads, 1, hd).view(M, heads, hd)
+    p = (q[..., 0].double() * hd ** -0.5).exp()
+    p16, n = p.half().double(), torch.arange(M, device="cuda").double()[:, None] + base - 1
+    off = (got[..., 0].double() / ((2 + n * p16) / (2 + n * p)) - 1).abs()
+    off = off[(p16 / p - 1).abs() < 0.9 * 2.0 ** -12]       # (next to the middle between two fp16 numbers the last bit of p decides)
+    assert off.numel() > 40 and off.max().item() <= 3 * 512 * 2.0 ** -24 + 2.0 ** -20
+
+
 @pytest.mark.parametrize("heads,kv_heads,hd", [(32, 8, 64), (9, 3, 64), (6, 6, 96), (24, 8, 128)])
 @pytest.mark.parametrize("seq,window", [(1, 1), (5, 3), (70, 1), (70, 64), (70, 70), (70, 4096), (900, 17), (900, 256), (900, 899)])
 def test_attention_sliding_decode_parity(fh, oracle, torch_gpu, heads, kv_heads, hd, seq, window):
