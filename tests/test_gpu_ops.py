@@ -634,6 +634,27 @@ def test_attention_prefill_running_maximum(fh, torch_gpu, hd, heads, M, base, wi
         assert (got[:, h].double() - want).abs().max().item() <= 2.0 ** -10 * v.abs().max().item()
 
 
+@pytest.mark.parametrize("heads,kv_heads,hd", [(4, 2, 64), (3, 3, 96), (2, 1, 128), (40, 8, 64)])
+@pytest.mark.parametrize("off_k,off_v", [(4, 0), (0, 4), (1, 3), (8, 2)])
+def test_attention_prefill_of_caches_that_begin_anywhere(fh, torch_gpu, heads, kv_heads, hd, off_k, off_v):
+    """A cache that is a part of a larger allocation need not begin on a 16-byte boundary: the same bits as of a copy that does."""
+    torch = torch_gpu
+    for M, base, window in ((1, 0, 0), (77, 130, 0), (200, 63, 50), (1700, 5, 0)):
+        g = torch.Generator(device="cuda").manual_seed(M + hd)
+        n, width = base + M, kv_heads * hd
+        q = torch.randn(M, heads * hd, generator=g, device="cuda")
+        k, v = (torch.randn(n, width, generator=g, device="cuda").half().view(torch.int16) for _ in range(2))
+        held = [torch.full((n * width + 16,), 0x7C00, dtype=torch.int16, device="cuda") for _ in range(2)]
+        parts = []
+        for whole, off, x in ((held[0], off_k, k), (held[1], off_v, v)):
+            part = whole[off:off + n * width].view(n, width)
+            part.copy_(x)
+            parts.append(part)
+        call = (lambda a, b: fh.ops.attention_sliding_batch(q, a, b, base, window, heads, kv_heads, hd)) if window else (lambda a, b: fh.ops.attention_flash_batch(q, a, b, base, heads, kv_heads, hd))
+        want, got = call(k, v).cpu().numpy(), call(*parts).cpu().numpy()
+        same_bits(got, want)
+
+
 @pytest.mark.parametrize("hd,heads,M", [(64, 2, 64), (96, 2, 64), (128, 2, 64), (64, 128, 512), (96, 128, 512), (128, 128, 512)])      # eight waves to a workgroup, four
 def test_attention_prefill_sum_of_many_like_weights(fh, torch_gpu, hd, heads, M):
     """32768 keys of one weight, about 0.15 to 0.02 by the query, behind two of weight 1, and values of 1: the quotient of two sums, of the weights in fp16 and in 32 bits.  A lane adds
