@@ -54,22 +54,35 @@ __device__ __forceinline__ v4h read_transposed(const uint8_t* at) {
     return __builtin_bit_cast(v4h, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s*)at));
 }
 
-// V fragments of 32 keys x 96 head dims in two rows of LDS `at`: f[j][d] = keys 16 j + 4 lh .. + 3 and + 8 of dim 32 d + lane % 32.  The compiler
-// waits for everything that is on its way into LDS ahead of a transposing read of its own, that is for the next tiles in the middle of a step.
-// Where K and V come from HBM, as they do with as many KV heads as heads (3001 tokens of 32/32 heads of 96, 110 MB), the step has to be given to
-// them whole: 82.8 us behind the compiler's waits, 77.8 behind these.  With shared heads they come out of a cache in time, and these waits,
-// which keep the reads from running ahead of the products, cost more (32/8 heads of 128 91.7 / 93.4, 12/2 49.1 / 53.3; of 64 43.0 / 43.4).
-#define FH_TR(dst, off) "ds_read_b64_tr_b16 " dst ", %[at] offset:" off "\n"
-#define FH_TR4(a, b, c, d, off) FH_TR(a, off) FH_TR(b, off "+%[k8]") FH_TR(c, off "+%[k8]*2") FH_TR(d, off "+%[k8]*3")
-__device__ __forceinline__ void read_v96(v8h (&f)[2][3], uint32_t at) {
+// The compiler waits for everything that is on its way into LDS ahead of a transposing read of its own, that is for the next tiles in the middle of a step; reads in
+// assembly have waits of their own, which keep them from running ahead of the products.  What is the better differs by form and head, hardly by whether heads share K and V.
+// us, the compiler's waits / own, 32/32 and 32/8 heads:
+//   eight waves, 1000 rows         64 21.3 / 20.5, 20.1 / 19.3    96 24.4 / 23.5, 24.6 / 23.4    128 27.1 / 27.9, 26.9 / 27.7
+//   1024 behind 4096               64 76.0 / 70.8, 73.6 / 68.7    96 111.8 / 96.0, 90.8 / 85.1    128 113.8 / 106.2, 102.1 / 105.2
+//   four waves, 3001               64 68.3 / 69.2, 58.2 / 58.5    96 85.4 / 84.7, 77.6 / 77.3    128 100.1 / 102.4, 93.9 / 95.9
+//   2048 behind 8192               64 209.9 / 217.3, 202.7 / 208.3    96 283.9 / 279.7, 277.4 / 278.9    128 340.4 / 346.3, 334.1 / 342.6
+template <int HD, int KH> constexpr bool own_waits() { return HD == 96 || (HD == 64 && KH == 1); }
+
+// V fragments of 32 keys: f[j][d] = keys 16 j + 4 lh .. + 3 and + 8 of dim 32 d + lane % 32.  at0, at1: LDS addresses of this lane's part of the first dims and of those 32 further on
+// (a row's swizzle is the same again 64 further; with heads of 96 it is the same everywhere).
+#define FH_TR(dst, at, off) "ds_read_b64_tr_b16 " dst ", " at " offset:" off "\n"
+#define FH_TR4(a, b, c, d, at, off) FH_TR(a, at, off) FH_TR(b, at, off "+%[k8]") FH_TR(c, at, off "+%[k8]*2") FH_TR(d, at, off "+%[k8]*3")
+template <int HD>
+__device__ __forceinline__ void read_v(v8h (&f)[2][HD / 32], uint32_t at0, uint32_t at1) {
     v4h r[3][4];
-    asm volatile(FH_TR4("%[x00]", "%[x01]", "%[x02]", "%[x03]", "0") FH_TR4("%[x10]", "%[x11]", "%[x12]", "%[x13]", "64")
-                 FH_TR4("%[x20]", "%[x21]", "%[x22]", "%[x23]", "128") "s_waitcnt lgkmcnt(0)"
-                 : [x00] "=&v"(r[0][0]), [x01] "=&v"(r[0][1]), [x02] "=&v"(r[0][2]), [x03] "=&v"(r[0][3]), [x10] "=&v"(r[1][0]), [x11] "=&v"(r[1][1]),
-                   [x12] "=&v"(r[1][2]), [x13] "=&v"(r[1][3]), [x20] "=&v"(r[2][0]), [x21] "=&v"(r[2][1]), [x22] "=&v"(r[2][2]), [x23] "=&v"(r[2][3])
-                 : [at] "v"(at), [k8] "n"(8 * 192));
+    if constexpr (HD == 96)
+        asm volatile(FH_TR4("%[x00]", "%[x01]", "%[x02]", "%[x03]", "%[at0]", "0") FH_TR4("%[x10]", "%[x11]", "%[x12]", "%[x13]", "%[at0]", "64")
+                     FH_TR4("%[x20]", "%[x21]", "%[x22]", "%[x23]", "%[at0]", "128") "s_waitcnt lgkmcnt(0)"
+                     : [x00] "=&v"(r[0][0]), [x01] "=&v"(r[0][1]), [x02] "=&v"(r[0][2]), [x03] "=&v"(r[0][3]), [x10] "=&v"(r[1][0]), [x11] "=&v"(r[1][1]),
+                       [x12] "=&v"(r[1][2]), [x13] "=&v"(r[1][3]), [x20] "=&v"(r[2][0]), [x21] "=&v"(r[2][1]), [x22] "=&v"(r[2][2]), [x23] "=&v"(r[2][3])
+                     : [at0] "v"(at0), [k8] "n"(8 * 2 * HD));
+    else
+        asm volatile(FH_TR4("%[x00]", "%[x01]", "%[x02]", "%[x03]", "%[at0]", "0") FH_TR4("%[x10]", "%[x11]", "%[x12]", "%[x13]", "%[at1]", "0") "s_waitcnt lgkmcnt(0)"
+                     : [x00] "=&v"(r[0][0]), [x01] "=&v"(r[0][1]), [x02] "=&v"(r[0][2]), [x03] "=&v"(r[0][3]), [x10] "=&v"(r[1][0]), [x11] "=&v"(r[1][1]),
+                       [x12] "=&v"(r[1][2]), [x13] "=&v"(r[1][3])
+                     : [at0] "v"(at0), [at1] "v"(at1), [k8] "n"(8 * 2 * HD));
 #pragma unroll
-    for (int d = 0; d < 3; d++)
+    for (int d = 0; d < HD / 32; d++)
 #pragma unroll
         for (int j = 0; j < 2; j++) f[j][d] = __builtin_shufflevector(r[d][2 * j], r[d][2 * j + 1], 0, 1, 2, 3, 4, 5, 6, 7);
 }
@@ -98,6 +111,7 @@ void attn_prefill_kernel(const float* __restrict__ q, const uint16_t* __restrict
     constexpr uint32_t LOADS = 2 * PIECES / WAVES;        // loads of 1 KB into LDS per wave and tile pair: K's come first
     constexpr bool EVEN = PIECES % WAVES == 0;            // then a wave's loads of V repeat those of K
     constexpr uint32_t OFFS = EVEN ? LOADS / 2 : LOADS;
+    constexpr bool OWN = own_waits<HD, KH>();
     constexpr int NS = HD / 16;   // MFMA k-steps over head_dim
     constexpr int ND = HD / 32;   // 32-wide head_dim tiles of the output
     constexpr int MERGE_FLOATS = 2 + ND * 16;    // per lane: m, l and the output accumulators
@@ -280,12 +294,12 @@ void attn_prefill_kernel(const float* __restrict__ q, const uint16_t* __restrict
 #pragma unroll
             for (int h = 0; h < KH; h++) {
                 v8h vf[2][ND];
-                if constexpr (HD == 96) read_v96(vf, (uint32_t)(uintptr_t)FH_LDS3(v_at(Vb, (kh + h) * 32, 0)));
+                if constexpr (OWN) read_v<HD>(vf, (uint32_t)(uintptr_t)FH_LDS3(v_at(Vb, (kh + h) * 32, 0)), (uint32_t)(uintptr_t)FH_LDS3(v_at(Vb, (kh + h) * 32, 1)));
 #pragma unroll
                 for (int j = 0; j < 2; j++)
 #pragma unroll
                     for (int d = 0; d < ND; d++) {
-                        if constexpr (HD != 96) vf[j][d] = v_frag(Vb, (kh + h) * 32 + 16 * j, d);
+                        if constexpr (!OWN) vf[j][d] = v_frag(Vb, (kh + h) * 32 + 16 * j, d);
                         oacc[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[j][d], pb[h][j], oacc[d], 0, 0, 0);
                     }
             }
@@ -368,20 +382,25 @@ template <int HD, bool QUANT>
 void launch_win(dim3 grid, hipStream_t s, const float* q, const uint16_t* kc, const uint16_t* vc, float* out, uint32_t q_stride,
                 uint32_t out_stride, uint32_t M, uint32_t base_pos, uint32_t heads, uint32_t kv_heads, int8_t* oq, uint16_t* osc,
                 uint32_t window, PageTable pt) {
-    // The 4-wave form from two workgroups per CU on (then throughput decides, and a wave with two score tiles per step does more of it); the
-    // 8-wave form below (then the longest workgroup's chain of tile steps decides, and twice the waves halve its steps).  us, 4 waves / 8 waves:
-    // 256 workgroups 1000 rows of 32/8 heads of 128 27.1 / 25.2, 1024 behind 8192 of 32/32 of 96 176 / 161, of 32/8 of 64 117 / 108;
-    // 480 24/8 of 128 62.3 / 60.3, 32/32 of 96 38.8 / 39.4; 512 2048 behind 8192 of 64 192 / 197, of 96 269 / 264, of 128 321 / 334;
-    // 640 2502 rows of 64 44.0 / 44.6; 768 3001 rows of 96 75.0 / 79.1, of 128 89.8 / 105.  FORGE_HIP_ATTN_WAVES=8 / 4 forces one.
+    // The four-wave form where there are many workgroups: then throughput decides, and a wave with two score tiles per step does more of it; the eight-wave form below: then the
+    // longest workgroup's chain of tile steps decides, and twice the waves halve its steps.  us, four waves / eight, heads of 64, 96, 128 (as they are taken: see own_waits):
+    //   workgroups      384 (2000 rows of 24/8) 33.3 / 32.7, 40.9 / 40.0, 50.6 / 47.9    480 (2500) 41.0 / 41.2, 51.9 / 54.8, 64.2 / 65.7    768 (4000) 74.7 / 80.2, 97.7 / 121, 120 / 147
+    //   under a window  180 (2500 rows of 9/3, 1500) 29.1 / 28.6, 35.5 / 34.2, 42.6 / 38.7    288 (1500 behind 1500 of 24/8, 700) 27.6 / 28.9, 35.3 / 44.4, 41.0 / 51.7
+    //                   480 (2500 of 24/8, 256) 17.1 / 18.0, 22.5 / 29.5, 26.0 / 35.5    (2000) 38.3 / 39.2, 49.3 / 56.4, 60.1 / 66.0    320 (2500 of 16/16, 2000) 36.9 / 35.9,
+    //                   45.6 / 42.6, 54.9 / 48.4
+    // Short prompts would gain from four waves as well (300 rows of 24/8 7.8 / 9.4, 9.8 / 11.8, 11.4 / 14.0, 1000 18.4 / 19.5, 22.9 / 23.5, 27.5 / 27.5), unless they have few rows behind
+    // many (33 behind 1400 of 9/3 23.0 / 18.8, 27.9 / 22.5, 33.8 / 23.4); but then the parts of one prompt would be worked on in different orders.  FORGE_HIP_ATTN_WAVES=8 / 4 forces one.
     static const int forced = [] { const char* e = getenv("FORGE_HIP_ATTN_WAVES"); return e ? atoi(e) : 0; }();
     static const int cus = [] {
         int dev = 0, n = 0;
         if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) n = 256;
         return n > 0 ? n : 256;
     }();
-    const bool four = forced == 4 || (forced != 8 && grid.x >= 2 * (uint32_t)cus);
     // a window that covers every key of the call is plain causal attention
     const bool win = window != 0 && window < base_pos + M;
+    const bool alike = win && window <= (base_pos + M) / 2;      // a narrow window makes nearly all workgroups equally long
+    const bool many = alike ? grid.x > (uint32_t)cus : grid.x >= (uint32_t)cus * 7 / 4;
+    const bool four = forced == 4 || (forced != 8 && many);
     // A model's caches are its own allocations; an operation's caller can have one that begins off a 16-byte boundary.  us, on one / 8 bytes off: 3001 rows of 32/32 heads of 96
     // 87.9 / 93.4, of 32/8 of 128 101 / 110, 2502 of 32/8 of 64 45.9 / 51.6.
     const bool direct = QUANT || ((reinterpret_cast<uintptr_t>(kc) | reinterpret_cast<uintptr_t>(vc)) & 15) == 0;
