@@ -19,8 +19,8 @@ constexpr float LOG2E = 1.4426950408889634f;
 //   32-bit    Through registers into one buffer (K row-major: the head's own part, the shared part; V transposed), two barriers a step.
 // What bounds it: up to a few hundred workgroups the chain of steps, each a trip through LDS, two products and the exponentials between them; then the VALU (exponentials,
 // maxima, conversions) beside the matrix unit.  In bfloat16 a step through registers took 1.8 us, half of it the loads' issue and the writes to LDS, and its registers left
-// one workgroup to a compute unit; now 1.1, and two.  us, before / now: 9 heads of 64 + 32 with a window of 1024, 902 tokens 18.4 / 14.9, 2502 36.0 / 22.4, 4000 47.1 /
-// 29.5; 32/8 heads of 64 902 23.2 / 15.7, 2502 92.7 / 51.8; 24/8 of 128 2502 101.9 / 85; 16 of 128 + 64 902 40.1 / 33.1, 4000 169 / 141; 33 tokens the same.
+// one workgroup to a compute unit; now 1.1, and two.  us, before / now: 9 heads of 64 + 32 with a window of 1024, 902 tokens 18.4 / 15.2, 2502 36.0 / 23.3, 4000 47.1 /
+// 29.7; 32/8 heads of 64 902 23.2 / 16.0, 2502 92.7 / 54.0; 24/8 of 128 2502 101.9 / 90.1; 16 of 128 + 64 902 40.1 / 33.0, 4000 169 / 147; 33 tokens the same.
 // DQ >= dim + rot and DV >= vdim: the register tiles' sizes; columns past the real ones are zero.
 constexpr uint32_t LP_THREADS = 512;
 constexpr uint32_t LP_RSRC_FLAGS = 0x00020000;   // raw buffer, 32-bit data format
@@ -346,12 +346,13 @@ void go_keys(const PromptAttn& a, uint32_t M, uint32_t base_pos, hipStream_t s) 
 template <typename T, int DQ, int DV>
 void go(const PromptAttn& a, uint32_t M, uint32_t base_pos, hipStream_t s) {
     // Bound by the chain of tile steps (about 1.1 us each), not by work, as long as the workgroups are few: four waves to a query group while the workgroups of
-    // 64 queries are a few rounds of the chip, fewer under a window, which makes them all equally long, than without, where the short ones fill the gaps.  us, two /
-    // four, by workgroups of 64 queries.  bfloat16, up to 96 columns (two workgroups run on a compute unit): window, 9 heads 135 21.2 / 14.9, 360 26.4 / 22.2, 567
-    // 28.2 / 32.4; none, 9 to 32 heads 360 39.5 / 27.8, 480 47.3 / 32.9, 567 59.9 / 42.1, 756 72.5 / 61.1, 768 27.7 / 28.8, 1280 49.0 / 57.5.  128 columns (tiles of
-    // 128 keys are 128 KB, one workgroup to a compute unit), 24 heads 240 21.5 / 17.8, 360 28.2 / 28.1, 576 40.8 / 52.5.  32-bit (one to a compute unit as well), whole
-    // prompts of 9 heads in ms: window 135 2.77 / 2.48, 216 3.24 / 2.87, 360 3.60 / 3.58; none 360 3.69 / 3.51; 32 heads 480 4.06 / 4.03, 1280 8.79 / 8.82.  Shapes
-    // whose tiles of 128 keys do not fit stay with two, and so do up to 64 keys, one tile for two waves: four would only load and merge more (2 tokens 6.2 / 6.5 us).
+    // 64 queries are a few rounds of the chip, fewer under a window, which makes them all equally long, than without, where the short ones fill the gaps.  us, two / four, by workgroups
+    // of 64 queries:
+    //   bfloat16, up to 96 columns (two workgroups run on a compute unit)    window 135 21.8 / 15.2, 360 27.4 / 23.3, 480 23.5 / 24.0, 567 29.7 / 32.9, 640 26.2 / 29.0; none 360 40.2 / 29.1, 480
+    //                         49.6 / 34.4, 608 24.3 / 23.7, 756 78.0 / 65.7, 768 30.2 / 30.6, 1280 54.0 / 63.2
+    //   128 columns (tiles of 128 keys are 128 KB, one workgroup)            window 240 22.6 / 19.3, 360 30.2 / 29.6, 576 37.7 / 50.9; none 240 22.7 / 18.9, 360 29.9 / 29.7, 456 36.6 / 38.2
+    //   32-bit, 64 columns (one as well)                                     window 192 31.6 / 24.1, 256 31.3 / 24.6, 320 32.3 / 45.4; none 360 57.0 / 37.3, 480 77.5 / 60.4, 608 98.7 / 102
+    // Shapes whose tiles of 128 keys do not fit stay with two, and so do up to 64 keys, one tile for two waves: four would only load and merge more (2 tokens 6.1 / 6.6 us).
     constexpr uint32_t CUS = 256;
     const bool windowed = a.window && a.window < base_pos + M;
     const uint32_t at_most = prompt_four<T, DQ>() ? (windowed ? 2 * CUS : 3 * CUS - 1) : sizeof(T) == 2 ? (windowed ? CUS : CUS * 3 / 2) : (windowed ? CUS : 2 * CUS);
