@@ -351,8 +351,9 @@ __global__ __launch_bounds__(GEMV_THREADS) void latent_value_kernel(LatentShape 
     });
 }
 
-// Small heads: their query's products are one launch, a request of 30 layers with 9 heads of 64 + 32 11.0 ms instead of 11.4.  Up to what a
-// workgroup has in registers and LDS; past it a head's matrices are too much for one compute unit, and the launches over parts of them spread wider.
+// Small heads: their query's products are one launch.  Up to what a workgroup has in registers and LDS.  us of a whole layer of width 256 without feed-forward, two launches / one, 9 and 250
+// heads: bfloat16 64 + 32, ranks 192 and 128 19.9 / 18.9, 31.9 / 27.0; 96 + 32, ranks of 256 23.1 / 22.6, 37.6 / 33.2; 32-bit 64 + 32, 192 and 128 23.4 / 22.6, 38.0 / 34.0; 96 + 32, ranks of 256
+// (229 KB to a compute unit) 26.9 / 26.8, 46.9 / 43.4.  Of 126 shapes of 2 to 250 heads the seven that lose (by 0.1 to 1.0) have two.
 bool latent_query_absorbs(const LatentShape& sh) { return sh.dim + sh.rot <= LQ_ROWS && sh.q_rank <= LQ_RANK && sh.rank <= LQ_RANK; }
 
 namespace {
