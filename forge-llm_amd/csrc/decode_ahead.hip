@@ -1447,6 +1447,13 @@ int32_t pa_create(const forge_hip_config& c, const std::vector<PdLayerIn>& layer
 
     std::vector<PaLayer> host(layers.size() + 1);
     memset(host.data(), 0, host.size() * sizeof(PaLayer));
+    if (kq) {
+        uint64_t blocks = (uint64_t)lm_head.N * (lm_head.K / 32);
+        for (const PdLayerIn& in : layers)
+            for (const QWeight* w : {in.q, in.k, in.v, in.o, in.gate, in.up, in.down}) blocks += (uint64_t)w->N * (w->K / 32);
+        size_t free_bytes = 0, all = 0;
+        if (hipMemGetInfo(&free_bytes, &all) != hipSuccess || !decode_ahead_copy_fits(blocks, free_bytes)) { (void)hipGetLastError(); return FORGE_HIP_OK; }
+    }
     // matrices of one depth, one behind the other, as PA_KQ blocks; false: no memory for them, and the other kernel takes the steps
     auto units = [&](const std::vector<const QWeight*>& ws, PaWeights* to) {
         size_t blocks = 0;

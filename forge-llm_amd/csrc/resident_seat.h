@@ -12,6 +12,11 @@ constexpr bool decode_ahead_offsets_fit(uint64_t max_seq, uint64_t kv_channels, 
     return max_seq * kv_channels * 2 <= 0xFFFFFFFFull && vocab * hidden / (lm_head_q4 ? 2 : 1) <= 0xFFFFFFFFull;
 }
 
+// A K-quant model's matrices as decode_ahead_kernel reads them are a copy of `blocks` blocks of 36 bytes.  It buys time only (decode_persistent_kernel runs the same models), so
+// it takes an eighth of the free memory at most: a model of up to 2048 channels next to others finds room for what it cannot do without.
+constexpr uint64_t decode_ahead_copy_bytes(uint64_t blocks) { return blocks * 36; }
+constexpr bool decode_ahead_copy_fits(uint64_t blocks, uint64_t free_bytes) { return decode_ahead_copy_bytes(blocks) <= free_bytes / 8; }
+
 // All workgroups are co-resident by construction (one per compute unit, checked when the model is created) and every wait in the kernel is bounded, so an ordinary launch
 // is enough; it costs ~7 us less per step than a cooperative one, which checks again.  FORGE_HIP_PD_COOP=1 asks for that one.
 bool resident_cooperative();

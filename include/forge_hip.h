@@ -33,7 +33,10 @@
  * Device memory and threads
  *  - A model allocates all its device buffers in forge_hip_model_create (weights, KV cache for max_seq,
  *    activations for one prefill chunk); later calls allocate no device memory (the kernel-sequence
- *    decode path instantiates its HIP graph at the first decode step).
+ *    decode path instantiates its HIP graph at the first decode step).  A model of Q4_K / Q6_K matrices also holds them as its decode
+ *    and prompt kernels read them: for the one-kernel decode step 36 bytes per 32 weights (FORGE_HIP_PD_AHEAD=0 does without; not
+ *    made where that is more than an eighth of the free memory) beside the units of the kernel that takes the other steps
+ *    (FORGE_HIP_PD_KQUANT=0: neither), for prompts in fast mode what forge_hip_gemm_q says below.
  *  - The op-level calls keep a few scratch areas per device (quantised activations, attention / argmax
  *    partial results, RoPE tables, 16 MB of partial GEMM tiles, K-quant operands) that GROW ON DEMAND: a call that needs more
  *    than any earlier call on that device did frees the old area, which waits for the device, and allocates one at least half

@@ -62,6 +62,10 @@ int main(int argc, char** argv) {
         printf("%d %d %d %d %d %d\n", fh::decode_ahead_offsets_fit((1u << 21) - 1, 1024, 128256, 2048, false), fh::decode_ahead_offsets_fit(1u << 21, 1024, 128256, 2048, false),
                fh::decode_ahead_offsets_fit(4096, 512, (1u << 21) - 1, 2048, false), fh::decode_ahead_offsets_fit(4096, 512, 1u << 21, 2048, false),
                fh::decode_ahead_offsets_fit(4096, 512, (1u << 22) - 1, 2048, true), fh::decode_ahead_offsets_fit(4096, 512, 1u << 22, 2048, true));
+    } else if (what == "copy") {
+        // the 1B shape: 1.236e9 weights, 1.39 GB; free memory that just suffices, and a byte less
+        const uint64_t blocks = 1235746816ull / 32, need = fh::decode_ahead_copy_bytes(blocks) * 8;
+        printf("%d %d %d\n", fh::decode_ahead_copy_fits(blocks, need), fh::decode_ahead_copy_fits(blocks, need - 1), fh::decode_ahead_copy_fits(blocks, 0));
     } else if (what == "launch") {
         (void)fh::resident_launch(nullptr, 256, 768, nullptr, 1000, fh::resident_cooperative(), handle(a));
     } else if (what == "one") {

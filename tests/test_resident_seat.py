@@ -35,6 +35,11 @@ def test_offsets_of_32_bits(seats):
     assert seats("offsets") == ["1 0 1 0 1 0"]
 
 
+def test_a_copy_for_speed_leaves_memory(seats):
+    """The copy of a K-quant model's matrices is made where it takes an eighth of the free memory at most."""
+    assert seats("copy") == ["1 0 0"]
+
+
 @pytest.mark.parametrize("value,want", [("0", "ordinary"), ("1", "cooperative")])
 def test_the_variable_asks_for_cooperative_launches(seats, value, want):
     assert seats("launch", FORGE_HIP_PD_COOP=value) == [f"{want} a 256 768 1000"]
