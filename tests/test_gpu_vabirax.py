@@ -360,10 +360,13 @@ def test_prompt_attention_forms(fh, vo, torch_gpu, tmp_path, heads, window):
 
 
 @pytest.mark.parametrize("heads,dim,rot,vdim,scale,window", [(90, 40, 8, 24, None, None), (34, 40, 8, 24, 6.0, 70), (62, 40, 8, 64, 2.0, 70), (45, 100, 20, 100, 2.0, None),
-                                                            (4, 100, 20, 100, None, 129), (3, 130, 60, 128, 2.0, None), (2, 190, 56, 256, 1.0, 300)])
+                                                            (4, 100, 20, 100, None, 129), (3, 130, 60, 128, 2.0, None), (2, 190, 56, 256, 1.0, 300),
+                                                            (90, 20, 8, 24, 2.0, None), (60, 20, 8, 60, 2.0, 70), (4, 20, 8, 24, 2.0, 129), (4, 20, 8, 60, 2.0, None),
+                                                            (45, 90, 20, 100, 2.0, None), (30, 90, 20, 100, 2.0, 300), (30, 90, 20, 100, 2.0, None), (4, 90, 20, 100, None, 129)])
 def test_prompt_attention_of_every_head_size(fh, vo, torch_gpu, tmp_path, heads, dim, rot, vdim, scale, window):
-    """The bfloat16 tiles of every size and both numbers of waves to a query group (90 heads, 530 rows: past 767 workgroups of 64 queries; 62 under a window: past 512;
-    45 of 128 columns: past 384), portions that begin anywhere in a tile, and scores of a wide range."""
+    """The bfloat16 tiles of every size (dim, rot and vdim are each padded to a multiple of 32: keys of 64, 96, 128, 160, 224 and 256 columns) and, of up to 128 columns, both numbers of waves to a
+    query group by 530 rows: 9 workgroups of 64 queries a head, two waves past 767 of them (90 heads), under a window past 512 (60), with 128 columns past 384 (45) and 256 (30).  Portions
+    that begin anywhere in a tile, and scores of a wide range."""
     c = Case(fh, vo, tmp_path, fh.synth.vabirax_config(48, 61, [fh.synth.vabirax_layer(heads, dim, rot, vdim, 32, 32, None, window, scale=scale)], embedding_scale=3.0))
     ids = c.ids(700)
     want = c.oracle.forward(ids)[0]
