@@ -190,17 +190,29 @@ struct Kept {
 // included, and never falls) exceeds top_p -- the entry that crosses the threshold too (project.rs:535-540).
 void cut(const float* l, uint64_t n, float sum, const uint32_t* count, uint64_t most, bool cut_p, float top_p, Kept* out) {
     std::vector<uint32_t> room;
-    // Buckets from the top until they hold `most` entries, or (by the middle of each bucket) a little more than top_p of the sum; where that
-    // turns out to be too few, a little more than that, and in the end all.
-    for (double more = 1.0 / 512;; more *= 16) {
+    auto middle = [&](uint32_t b) { return (double)count[b] * float_of((b << BUCKET_SHIFT) | (1u << (BUCKET_SHIFT - 1))); };      // of a bucket's numbers, off by 1/33 at most
+    // Little is left out: what the buckets hold from the top says too little about it, being off by as much when one entry has most of the sum; what the others hold does.  (Nothing of
+    // note lies below the first that is looked at.)  By the former alone all entries were sorted as soon as one had most of the sum: 128 256 of a spread of 8, top_p 0.99, 1.95 ms, this way 0.34.
+    const bool by_rest = cut_p && top_p > 0.96f;
+    const double out_of = (1.0 - (double)top_p) * sum;
+    double others = 0.0;
+    if (by_rest)
+        for (uint32_t b = bits_of((float)(out_of / (1024.0 * n))) >> BUCKET_SHIFT; b < BUCKETS; b++)
+            if (count[b]) others += middle(b);
+    // Buckets from the top until they hold `most` entries, or a little more than top_p of the sum; where that turns out to be too few, a little more than that, and in the end all.
+    const double more[3] = {1.0 + 1.0 / 512, 1.0 + 1.0 / 32, INFINITY}, less[3] = {15.0 / 16, 1.0 / 4, -INFINITY};
+    for (int attempt = 0;; attempt++) {
         uint32_t floor = BUCKETS;
         uint64_t m = 0;
-        double mass = 0.0;
-        const double enough = cut_p && more < 0.5 ? (double)top_p * sum * (1.0 + more) : INFINITY;
-        while (floor > 0 && m < most && mass < enough) {
+        double mass = 0.0, rest = others;
+        const double enough = cut_p ? (double)top_p * sum * more[attempt] : INFINITY, few = out_of * less[attempt];
+        while (floor > 0 && m < most && (by_rest ? rest > few : mass < enough)) {
             floor--;
             m += count[floor];
-            if (count[floor]) mass += (double)count[floor] * float_of((floor << BUCKET_SHIFT) | (1u << (BUCKET_SHIFT - 1)));
+            if (count[floor]) {
+                mass += middle(floor);
+                rest -= middle(floor);
+            }
         }
         // The order is that of the quotients, and numbers that differ may have the same: what has the quotient of the least number of the last
         // bucket stands beside it, whichever bucket it is in (a bit pattern or two below; many where quotients are denormal).
@@ -234,7 +246,10 @@ void cut(const float* l, uint64_t n, float sum, const uint32_t* count, uint64_t 
                 if (cumsum > top_p) { crossed = true; break; }
             }
         } else keep = end;
-        if (!crossed && keep < most && least > 0) continue;
+        if (!crossed && keep < most && least > 0) {
+            if (m > n / 2) attempt = 1;      // most of them anyway: all
+            continue;
+        }
         if (!crossed && keep == n) { out->all = true; return; }
         out->index.resize(keep + 1);
         out->p.resize(keep + 1);

@@ -122,6 +122,21 @@ def test_sample_equals_oracle_over_sizes(fh, oracle, so, n, kind):
         assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
 
 
+@pytest.mark.parametrize("n", [2, 50, 700, 60000])
+@pytest.mark.parametrize("spread", [0.0, 1.0, 5.0, 12.0])
+def test_sample_equals_oracle_where_little_is_left_out(fh, oracle, so, n, spread):
+    """Candidates chosen by what the others hold (top_p above 0.96): one entry that has nearly all of the sum, a 32-bit sum that says less than its entries hold together (60000 of a spread
+    of 0 or 1, where the first choice is too few), with top_k as well."""
+    l = logits_of(fh, 77 + n, n, spread)
+    state_l = state_o = 0x7654321 + n
+    for temp, top_k, top_p in [(1.0, 0, 0.9601), (1.0, 0, 0.98), (0.7, 0, 0.995), (1.0, 0, 0.9999), (1.0, 0, 1.0 - 2.0 ** -24), (1.0, max(1, n // 3), 0.99)]:
+        a, b = l.copy(), l.copy()
+        tok_l, state_l = fh.ops.sample(a, temp, top_k, top_p, state_l)
+        tok_o, state_o = so.sample(oracle, b, temp, top_k, top_p, state_o)
+        assert (tok_l, state_l) == (tok_o, state_o)
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
 @pytest.mark.parametrize("kind", ["maximum", "edges", "hot", "small"])
 def test_sample_equals_oracle_among_equal_quotients(fh, oracle, so, kind):
     """Exponentials that differ and have the same quotient by their sum: equal probabilities, of which the lower index comes first.  They lie on either side of every line a
