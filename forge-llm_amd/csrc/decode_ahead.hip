@@ -2,7 +2,7 @@
 //
 // A step is a chain of four products and an attention per layer.  As kernels a link of that chain is 4 to 6 us however small (a launch that does nothing takes
 // 2.7); as phases of the kernel that streams weights of any size (decode_persistent.hip) it is 5.  Here a layer of SmolLM2-135M takes 12 us, one of the 1B shape 21
-// (its 65 MB alone take 14): five hand-overs of 0.8 to 1.2 (1.5 to 2.5 beside weights), two norms of 0.7, attention 3.2, and the products.
+// (its 65 MB alone take 13): five hand-overs of 0.8 to 1.2 (1.5 to 2.5 beside weights), two norms of 0.7, attention 3.2, and the products.
 //   * A wave's rows are a few registers, requested where nothing is on its way to the compute unit: while the attention is at work, and with wide models also right
 //     behind the products.  (A compute unit's loads return in order and its queue is short: a poll behind weights comes when they have come, and so does a store.)
 //   * Eight waves hold weights, four fetch the vectors.  A wave forms and sums whole rows by itself; the workgroup's rows lie side by side and are handed over
@@ -22,7 +22,8 @@
 //   and in fast mode (PaPart) 300: 637 / 442    1000: 642 / 447    2400: 644 / 459    5000: 676 / 495    Q4_0 2400: 570 / 441
 //   and of Q4_K / Q6_K matrices (llama.cpp's Q4_K_M recipe), 1B shape 33: 623 / 457    300: 646 / 495    2400: 655 / 511    5000: 688 / 548
 // Heads of 96 and 128 gain as much though those of 128 spill (8 layers, 33 rows, fast: 8/2 of 96 at 768 channels 213 / 136, 6/2 of 128 207 / 138, 16/4 of 96 at 1536 246 / 174,
-// 12/4 of 128 at 1024 212 / 168).  A layer's weights hardly count (1B shape, us: Q8_0 21, Q4_0 21): it is the chain that takes the time.
+// 12/4 of 128 at 1024 212 / 168).  The chain takes the time, as far as a layer's weights arrive
+// beside it: half the bytes make no layer shorter (1B shape, us: Q8_0 21, Q4_0 21), an earlier request for those that were waited for did (Q8_0 23 -> 21: EARLY).
 #include <stddef.h>
 #include <string.h>
 
@@ -57,7 +58,7 @@ struct PaWide { static constexpr int UQ = 2, UO = 2, UG1 = 4, UG2 = 4, UD = 4, U
 
 // How a matrix's blocks of 32 weights lie in memory.  Q8, Q4: as for every other kernel.  KQ: Q4_K and Q6_K alike, made by pa_create: the codes as int8 in order
 // (0 .. 15 and -32 .. 31) and a word: fp16 bits of d (Q4_K, odd blocks: of dmin) | an int8 scale << 16 | Q6_K: the second half's << 24, Q4_K: the minimum << 24.
-// (Codes of 4 bits would be half the bytes and no faster: a layer's weights hardly count here.)
+// (One form for both, twice the bytes that Q4_K's codes need.  4 bits in a form of their own were not measured.)
 enum PaFmt : int { PA_Q8, PA_Q4, PA_KQ };
 
 // magic: floor(2^32 / nblk) + 1; R: rows per wave; wg0: the first workgroup with rows; stride: words between two rows of products; prod: the first wave's area of
@@ -1042,7 +1043,8 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
             // while a workgroup computes, and what the result's store and the next poll wait behind is on its way by then.  (All of down behind the results' barrier / this, 1B
             // shape, us a token by rows of context: Q8_0 33 430 / 400, 300 463 / 440, 2400 477 / 457, order-faithful 33 471 / 450; Q4_K and Q6_K 33 487 / 457, 2400 539 / 511;
             // 8 layers of 1024 channels Q8_0 151 / 151, of 1280 163 / 160.  All of down ahead of the second part's products 472 for the first of these, none of it 412, its second
-            // half behind the row sums' barrier 418.)  Not Q4_0: half the bytes to wait for; 403 / 386, but models of 1024 channels 150 / 153.  The other sets gain little or
+            // half behind the row sums' barrier 418.)  Not Q4_0, half the bytes to wait for: 403 / 386 there,
+            // but models of 1024 channels 150 / 153; one form for all its sizes, the one that costs none of them.  The other sets gain little or
             // nothing from an earlier place: q;k;v ahead of down's products 1 % (1024 channels 2 % slower), gate;up's second part ahead of o's products 2 to 6 us slower.
             constexpr bool EARLY = F::WIDE && W != PA_Q4;
             static_assert(!EARLY || F::UG1 == F::UD, "down takes the place of gate;up's first part");
