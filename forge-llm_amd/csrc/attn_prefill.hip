@@ -12,10 +12,10 @@
 // Scores stay in the base-2 domain (s * scale * log2 e) so that the exponential is one v_exp_f32 after one FMA; keys are masked only in
 // tiles that reach past the wave's first query; accumulators are rescaled only when some query's maximum rises.  (Letting a maximum stand until a score passes
 // it by 2^8 saves 3 of 80 us at 3001 tokens, but the largest weight is then no longer exactly 1 in fp16: error against 64 bits 2.45e-4 instead of 2.35e-4.  Not kept.)
-// What bounds it: full, the matrix unit, the VALU (32 exp, 32 FMA, 32 additions, 16 conversions, 16 maxima per 32 x 64 scores) and LDS reads
-// take about 800 cycles each and overlap to 1800 (heads of 96, 3072 queries behind 8192 keys 408 us = 0.90 PFLOP/s, 128 0.93, 64 0.81; the
-// library's large bf16 product is at 1.2); causal, the uneven length of the query tiles on top.  3001 tokens: 32/32 heads of 96 97.7 -> 82 us,
-// 32/8 of 128 124 -> 95, 2502 tokens of 32/8 of 64 52.5 -> 45.1, 1000 of 32/8 of 128 38.2 -> 26.7.
+// What bounds it: full, 768 cycles of the matrix unit and about 860 of the VALU (32 exp, 32 FMA, 32 additions, 16 conversions, 16 maxima per 32 x 64 scores, heads of 96), hardly
+// any of them beside one another, in about 1620; LDS is busy a third of the time, of 128 nearly half (heads of 96, 3072 queries behind 8192 keys 410 us = 0.89 PFLOP/s, 128 0.93, 64
+// 0.80; the library's large bf16 product is at 1.2); causal, the uneven length of the query tiles on top.  3001 tokens: 32/32 heads of 96 97.7 -> 80 us,
+// 32/8 of 128 124 -> 96, 2502 tokens of 32/8 of 64 52.5 -> 46.9, 1000 of 32/8 of 128 38.2 -> 28.
 // Measured and not kept: query tiles of every other round in ascending order: within 2 %.
 //
 // Both products are computed transposed, S^T = K Q^T and O^T = V^T P^T.  In the 32x32 MFMA
@@ -42,7 +42,8 @@ constexpr uint32_t AP_RSRC_FLAGS = 0x00020000;   // raw buffer, 32-bit data form
 #define FH_LDS3(p) ((__attribute__((address_space(3))) void*)(p))
 
 // Where piece p (16 bytes) of row r of a tile lies in its row of LDS, and which piece lies at p: eight consecutive rows of K at one piece
-// (a fragment's reads), and two neighbouring pieces of four consecutive rows of V, touch all banks.  Rows are as long in LDS as they are: a load
+// (a fragment's reads), and two neighbouring pieces of four consecutive rows of V, touch 128 bytes' worth of banks once.  By the counters that is half of what LDS serves at once: a third (heads of
+// 64 and 96) to a half (128) of its active cycles are conflicts, of a unit that is busy 29 to 44 % of the time.  Rows are as long in LDS as they are: a load
 // into LDS fills 1 KB in lane order.
 template <int HD>
 __device__ __forceinline__ uint32_t piece_of(uint32_t r, uint32_t p) {
