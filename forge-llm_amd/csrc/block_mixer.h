@@ -9,6 +9,7 @@
 #include <vector>
 
 #include "checkpoint.h"
+#include "decode_block.h"
 #include "model.h"
 
 namespace fh {
@@ -82,6 +83,8 @@ struct Mixer {
     // Everything up to the output product; returns that product's input.
     virtual DenseIn enqueue(const MixerCall& c) const = 0;
     virtual int decode_launches() const = 0;
+    // What the resident decode kernel needs of it.
+    virtual PbMixer parts() const = 0;
 
     // W_o [width][heads * vdim] with each head's columns padded to `head` and their number to a multiple of 64
     int32_t load_output(const BlockLoad& l, const std::string& name, uint32_t heads, uint32_t vdim, uint32_t head);

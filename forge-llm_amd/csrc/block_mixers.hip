@@ -255,6 +255,13 @@ struct LatentMixer : Mixer {
         return dense_rows(out, hv);
     }
     int decode_launches() const override { return latent_query_absorbs(sh) ? 4 : 5; }
+    PbMixer parts() const override {
+        PbMixer m{MixerKind::LatentAttention};
+        m.latent = sh;
+        m.in = in; m.o = o; m.uq = uq; m.ukv = ukv;
+        m.wa = q_norm; m.wb = kv_norm; m.cos_t = cos_t; m.sin_t = sin_t;
+        return m;
+    }
 };
 
 // ---- grouped-query attention -----------------------------------------------------------------------------------------------
@@ -339,6 +346,14 @@ struct GroupedMixer : Mixer {
         return dense_rows(out, hv);
     }
     int decode_launches() const override { return 3; }
+    PbMixer parts() const override {
+        PbMixer m{MixerKind::GroupedAttention};
+        m.grouped = sh;
+        m.in = in; m.o = o;
+        m.wa = q_norm; m.wb = k_norm; m.cos_t = cos_t; m.sin_t = sin_t;
+        m.values_at = k_bytes();
+        return m;
+    }
 };
 
 // ---- gated linear attention --------------------------------------------------------------------------------------------------
@@ -390,7 +405,7 @@ struct LinearMixer : Mixer {
         norm = b2 + sh.qk();
         return FORGE_HIP_OK;
     }
-    size_t cache_bytes() const override { return sh.state() * 4; }
+    size_t cache_bytes() const override { return 2 * sh.state() * 4; }
     void plan(BlockScratch* s, uint32_t R) const override {
         s->need(BlockScratch::RAW, (size_t)R * sh.raw_row() * 4);
         s->need(BlockScratch::GATE, (size_t)R * hv * dtype_size(t));
@@ -419,6 +434,13 @@ struct LinearMixer : Mixer {
         return dense_rows(sc.p(BlockScratch::OUT), hv);
     }
     int decode_launches() const override { return 2; }
+    PbMixer parts() const override {
+        PbMixer m{MixerKind::LinearAttention};
+        m.linear = sh;
+        m.in = in; m.o = o;
+        m.wa = w2; m.wb = b2; m.wc = norm;
+        return m;
+    }
 };
 
 template <typename M, typename S>

@@ -14,6 +14,7 @@
 #include <string.h>
 
 #include "block_mixer.h"
+#include "resident_seat.h"
 
 using namespace fh;
 
@@ -71,6 +72,34 @@ struct BlockModel : forge_hip_model {
     DevBuf b_embed, b_loop, b_head, b_final, b_cache;
     DevBuf x, h, xcat, act, rows_sel, h_sel; // of one prompt chunk
     BlockScratch scratch;
+    PbState* pb = nullptr;                   // the decode step as one resident kernel, when the model is covered
+    std::unique_ptr<ResidentSeat> seat;      // of a model that has it
+    // A step that gave up (another process on the GPU) runs again as the kernel sequence, and so do those behind it; not where a caller set the kernel's poll limit.
+    bool pb_left = false, polls_set = false;
+    uint32_t step_seq = 0;
+
+    ~BlockModel() override { pb_destroy(pb); }
+    bool resident() const override { return pb && !pb_left && pb_covers(pb, pos); }
+    int32_t resident_enqueue(bool profile, uint32_t token) override {
+        step_seq = step_seq + 1 ? step_seq + 1 : 1;
+        return seat->turn(stream, [&] { return pb_enqueue(pb, pos, profile, token, step_seq, stream); });
+    }
+    bool resident_wait_token(uint32_t* next) override { return pb_wait_token(pb, next); }
+    int32_t resident_after_sync(uint32_t abort_flag) override {
+        pb_left = abort_flag && !polls_set;
+        return pb_after_sync(pb, abort_flag, stream);
+    }
+    int32_t resident_profile(float* stage_ms, uint32_t* stage_launches) override;
+    int32_t repeat_penalty_changed(float penalty) override {
+        if (pb) pb_set_repeat_penalty(pb, penalty);
+        return FORGE_HIP_OK;
+    }
+    void poll_limit_changed(uint32_t polls) override {
+        polls_set = polls != 0;
+        pb_left = false;
+        if (pb) pb_set_poll_limit(pb, polls);
+    }
+    int32_t make_resident();
 
     uint32_t logits_rows_max() const override { return HEAD_ROWS; }
     uint32_t layer_runs() const override { return (uint32_t)runs.size(); }
@@ -145,6 +174,7 @@ struct BlockModel : forge_hip_model {
         enqueue_logits(h_sel.p, n);
     }
     int32_t decode_launches() const override {
+        if (resident()) return 1;
         int n = 1 + (elementwise_norms() ? 0 : 1) + 1 + 2;       // embedding, final norm, lm_head, argmax
         for (const LayerRun& r : runs) n += (r.pass_start ? 1 : 0) + layers[r.layer]->mixer->decode_launches() + 1 + (layers[r.layer]->ff ? 2 : 0);
         return n;
@@ -316,8 +346,48 @@ int32_t BlockModel::load(const std::string& dir, uint32_t max_seq, uint32_t flag
         if ((rc = m.upload(&b_loop, &loop_in))) return rc;
     }
     if ((rc = b_final.alloc((size_t)2 * width * 4)) || (rc = load_norm(st, "final.norm", &b_final, 0, &final_norm))) return rc;
-    if ((rc = alloc_scratch())) return rc;
+    if ((rc = alloc_scratch()) || (rc = make_resident())) return rc;
     FH_HIP(hipDeviceSynchronize());
+    return FORGE_HIP_OK;
+}
+
+int32_t BlockModel::make_resident() {
+    const char* e = getenv("FORGE_HIP_PERSIST");
+    if (t != DType::BF16 || (e && e[0] == '0')) return FORGE_HIP_OK;
+    std::vector<PbMixer> mixers(runs.size());
+    PbModelIn m{};
+    for (size_t i = 0; i < runs.size(); i++) {
+        const LayerRun& r = runs[i];
+        const BlockLayer& L = *layers[r.layer];
+        mixers[i] = L.mixer->parts();
+        m.layers.push_back(PbLayerIn{&mixers[i], L.gate_up, L.down, L.norm1.tanh, L.norm2.tanh, L.norm1b.tanh, L.norm2b.tanh, L.norm1.ln, L.norm2.ln,
+                                     b_cache.as<uint8_t>() + r.cache, r.pass_start, L.act, L.ff});
+    }
+    m.elementwise = elementwise_norms();
+    m.width = width; m.ln_n = spec.width; m.max_seq = cfg.max_seq;
+    m.head = head; m.loop = loop_in;
+    m.final_norm = final_norm.tanh;
+    m.ln_final = final_norm.ln.w;
+    m.ln_eps = (float)spec.eps; m.embed_scale = (float)spec.embedding_scale; m.cap = (float)spec.logit_cap;
+    m.table = table; m.table_ld = table_ld; m.table_n = spec.width;
+    m.logits = logits.as<float>(); m.state = state.as<uint32_t>(); m.counts = counts.as<uint32_t>();
+    const int32_t rc = pb_create(m, &pb);
+    if (pb) seat.reset(new ResidentSeat());
+    return rc;
+}
+
+int32_t BlockModel::resident_profile(float* stage_ms, uint32_t* stage_launches) {
+    std::vector<float> ph;
+    const int32_t rc = pb_phase_ms(pb, &ph, stream);
+    if (rc) return rc;
+    for (int i = 0; i < ST_COUNT; i++) { stage_ms[i] = 0.f; if (stage_launches) stage_launches[i] = 0; }
+    static const int phase_stage[5] = {ST_QKV, ST_ATTN, ST_O, ST_GATE_UP, ST_DOWN};
+    for (size_t i = 0; i < ph.size(); i++) {
+        const size_t n = 5 * runs.size();
+        const int st = i < n ? phase_stage[i % 5] : i == n ? ST_LM_HEAD : ST_ARGMAX;
+        stage_ms[st] += ph[i];
+        if (stage_launches) stage_launches[st] += 1;
+    }
     return FORGE_HIP_OK;
 }
 

@@ -417,7 +417,7 @@ struct LinearIo {
     const float* raw;                        // [M][q | k | v | low]
     const float* w2;                         // [rank][heads * dim]
     const float* b2;                         // [heads * dim]
-    float* state;                            // [heads][dim][vdim]; what it holds at position 0 is not looked at
+    float* state;                            // [2][heads][dim][vdim]: ahead of position p in half p % 2 (a step that does not come to its end leaves its own); at position 0 not looked at
     uint32_t base_pos;
     const uint32_t* pos_dev;                 // one row only
 };

@@ -119,41 +119,7 @@ __device__ __forceinline__ T pa_lds_ptr(const T& p) {
 }
 __device__ __forceinline__ PaWeights pa_lds_ptr(const PaWeights& w) { return PaWeights{pa_lds_ptr(w.qs), pa_lds_ptr(w.ws)}; }
 
-struct PaCtx {
-    uint32_t tid, lane, wave, wg, G, spin_limit;
-    uint32_t* sh_abort;      // LDS
-    uint32_t* abort_flag;    // global
-};
-
 __host__ __device__ constexpr uint32_t pa_up(uint32_t v, uint32_t m) { return (v + m - 1) / m * m; }
-
-// N elements a thread takes, re-read together until all carry their tags; bounded.  Every load of a round trip is issued before any is looked at, and
-// without a condition: a branch around one of them would put a wait behind it.  (A thread without an element of its own takes one that another has.)
-// LATER: an element of a later phase will do; nothing is handed out.
-template <int N, bool LATER = false, typename Addr, typename Tag>
-__device__ __forceinline__ void pa_poll(Addr addr, Tag tag, uint32_t* out, const PaCtx& cx) {
-    uint64_t w[N];
-    uint32_t spins = 0;
-    for (;;) {
-#pragma unroll
-        for (int i = 0; i < N; i++) w[i] = ldc64(addr(i));
-        uint32_t off = 0;
-#pragma unroll
-        for (int i = 0; i < N; i++) off |= LATER ? ((uint32_t)(w[i] >> 32) - tag(i)) >> 31 : (uint32_t)(w[i] >> 32) ^ tag(i);
-        if (!off) break;
-        ++spins;
-        if (spins > cx.spin_limit ||
-            ((spins & 1023u) == 0 && __hip_atomic_load(cx.abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
-            *cx.sh_abort = 1;
-            __hip_atomic_store(cx.abort_flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            break;
-        }
-        __builtin_amdgcn_s_sleep(1);
-    }
-    if constexpr (LATER) return;
-#pragma unroll
-    for (int i = 0; i < N; i++) out[i] = (uint32_t)w[i];
-}
 
 // A wave's blocks of a matrix: n of them, row after row; from block `seg` on they lie `jump` blocks further (the up rows of gate;up).
 // six: KQ, 1 for Q6_K.
@@ -336,13 +302,13 @@ __device__ __forceinline__ void pa_store_block(float o, uint64_t* block, uint32_
 __device__ __forceinline__ uint32_t pa_xs(uint32_t e, uint32_t xstride) { return (e & 15u) * xstride + (e >> 4); }
 // Where the order of the norm's sum is free, every wave leaves the sum of its elements' squares in `part`.
 template <int N, bool ORD>
-__device__ __forceinline__ void pa_fetch_x(const uint64_t* tx, uint32_t tag, const float* emb, uint32_t H, float* xs, uint32_t xstride, float* part, const PaCtx& cx) {
+__device__ __forceinline__ void pa_fetch_x(const uint64_t* tx, uint32_t tag, const float* emb, uint32_t H, float* xs, uint32_t xstride, float* part, const PollCtx& cx) {
     uint32_t v[N];
     if (!tag) {                               // the layer ahead of the first: the embedding row
 #pragma unroll
         for (int i = 0; i < N; i++) v[i] = __float_as_uint(ldg(emb + min(cx.tid + i * PA_POLL_THREADS, H - 1)));
     } else {
-        pa_poll<N>([&](int i) { return tx + min(cx.tid + i * PA_POLL_THREADS, H - 1); }, [&](int) { return tag; }, v, cx);
+        poll_tagged<N>([&](int i) { return tx + min(cx.tid + i * PA_POLL_THREADS, H - 1); }, [&](int) { return tag; }, v, cx);
     }
     float ss = 0.f;
 #pragma unroll
@@ -364,7 +330,7 @@ __device__ __forceinline__ void pa_fetch_x(const uint64_t* tx, uint32_t tag, con
 // (res_tag 0: the embedding row; threads without a row: anything).
 template <int NV, bool SUMS>
 __device__ __forceinline__ float pa_fetch_aq(const uint64_t* t, uint32_t tag, uint32_t K, uint32_t* aq, float* as, float* sums, bool has_res, uint32_t res_row, const uint64_t* tx,
-                                             uint32_t res_tag, const float* emb, const PaCtx& cx) {
+                                             uint32_t res_tag, const float* emb, const PollCtx& cx) {
     const uint32_t ne = K / 32 * 9;
     float re = 0.f;
     if (has_res && !res_tag) re = ldg(emb + res_row);
@@ -375,7 +341,7 @@ __device__ __forceinline__ float pa_fetch_aq(const uint64_t* t, uint32_t tag, ui
     auto fetch = [&](auto n) {
         constexpr int N = decltype(n)::value;
         uint32_t v[N + 1];
-        pa_poll<N + 1>([&](int i) { return i < N ? t + min(cx.tid + i * PA_POLL_THREADS, ne - 1) : pr; }, [&](int i) { return i < N ? tag : tr; }, v, cx);
+        poll_tagged<N + 1>([&](int i) { return i < N ? t + min(cx.tid + i * PA_POLL_THREADS, ne - 1) : pr; }, [&](int i) { return i < N ? tag : tr; }, v, cx);
 #pragma unroll
         for (int i = 0; i < N; i++) {
             const uint32_t e = cx.tid + i * PA_POLL_THREADS, b = e / 9, k = e - b * 9;
@@ -397,7 +363,7 @@ __device__ __forceinline__ float pa_fetch_aq(const uint64_t* t, uint32_t tag, ui
 // rms_norm (emit.rs:327-334) + activation quantiser.  In the reference's order (16 accumulators, emit.rs:272-295) each fetching wave walks the row and the first
 // leaves 1 / rms behind; zeros behind an accumulator's elements change nothing.  The computing waves, which have nothing else to do yet, quantise four elements a
 // thread, whose norm weights they hold.  (All twelve waves forming the sum for themselves and an element a thread: 1.1 us at 576 channels where this takes 0.7.)
-__device__ __forceinline__ void pa_norm_sum(const float* xs, uint32_t xstride, float eps, uint32_t H, float* part, const PaCtx& cx) {
+__device__ __forceinline__ void pa_norm_sum(const float* xs, uint32_t xstride, float eps, uint32_t H, float* part, const PollCtx& cx) {
     const float4* p = reinterpret_cast<const float4*>(xs + (cx.lane & 15u) * xstride);
     float s = 0.f;
     constexpr int N4 = PA_SSQ / 4;
@@ -542,13 +508,13 @@ struct PaHead {
         kv.set_keys(kr);
     }
     template <bool SUMS>
-    __device__ __forceinline__ void step(PaKv<HD>& kv, const PaArgs& a, const PaLayer& L, PaAttn<HD, AW>* sh, const uint64_t* exp_tab, uint32_t pos, uint32_t tag_in, PaCtx& cx) const;
+    __device__ __forceinline__ void step(PaKv<HD>& kv, const PaArgs& a, const PaLayer& L, PaAttn<HD, AW>* sh, const uint64_t* exp_tab, uint32_t pos, uint32_t tag_in, PollCtx& cx) const;
 };
 
 template <int HD, uint32_t AW>
 template <bool SUMS>
 __device__ __forceinline__ void PaHead<HD, AW>::step(PaKv<HD>& kv, const PaArgs& a, const PaLayer& L, PaAttn<HD, AW>* sh, const uint64_t* exp_tab, uint32_t pos, uint32_t tag_in,
-                                                     PaCtx& cx) const {
+                                                     PollCtx& cx) const {
         constexpr int DPL = PaKv<HD>::DPL, KC = PaKv<HD>::KC;
         const uint32_t kv_stride = a.KV, lane = cx.lane;
         const float scale = 1.0f / sqrtf((float)HD);
@@ -561,7 +527,7 @@ __device__ __forceinline__ void PaHead<HD, AW>::step(PaKv<HD>& kv, const PaArgs&
         if (cx.tid < pa_up(HD, 64)) {
             uint32_t g[3];
             const uint32_t e = min(cx.tid, (uint32_t)HD - 1);
-            pa_poll<3>([&](int i) { return i == 0 ? a.tq + (size_t)h * HD + e : a.tkv + (i == 1 ? 0u : a.KV) + kvh * HD + e; }, [&](int) { return tag_in; }, g, cx);
+            poll_tagged<3>([&](int i) { return i == 0 ? a.tq + (size_t)h * HD + e : a.tkv + (i == 1 ? 0u : a.KV) + kvh * HD + e; }, [&](int) { return tag_in; }, g, cx);
             if (cx.tid < HD) {
                 sh->q[e] = __uint_as_float(g[0]);
                 sh->pn[e] = __uint_as_float(g[0]) * f16_bits_to_f32((uint16_t)g[1]);
@@ -711,7 +677,7 @@ struct PaPart {
     }
     // q_s: the group's heads in LDS, new_s: this position's K row and V row, fp16 pairs.  After the barrier that publishes them.
     __device__ __forceinline__ void attend(Half8* k, Half8* v, const PaArgs& a, const PaLayer& L, const float* q_s, const Half8* new_s, const uint32_t* pages, uint32_t pos, uint32_t tag_out,
-                                           const PaCtx& cx) const {
+                                           const PollCtx& cx) const {
         const uint32_t gsize = a.heads / a.kv_heads, lane = cx.lane, slot = lane / LPK, c = lane % LPK;
         const bool dvalid = c * 8 < (uint32_t)HD;
         const float scale = 1.0f / sqrtf((float)HD);
@@ -775,12 +741,12 @@ struct PaPart {
 
 // The splits of head h into its quantised row; recs: splits records, wt: a weight per split.  Fetching waves; two barriers.
 template <int HD, bool SUMS>
-__device__ __forceinline__ void pa_merge(const PaArgs& a, uint32_t h, uint32_t tag_in, uint32_t tag_out, float* recs, float* wt, const PaCtx& cx) {
+__device__ __forceinline__ void pa_merge(const PaArgs& a, uint32_t h, uint32_t tag_in, uint32_t tag_out, float* recs, float* wt, const PollCtx& cx) {
     constexpr uint32_t REC = HD + 2, N = (PA_SPLITS * REC + PA_POLL_THREADS - 1) / PA_POLL_THREADS;
     const uint32_t ne = a.splits * REC;
     const uint64_t* base = a.trec + (size_t)h * ne;
     uint32_t v[N];
-    pa_poll<N>([&](int i) { return base + min(cx.tid + i * PA_POLL_THREADS, ne - 1); }, [&](int) { return tag_in; }, v, cx);
+    poll_tagged<N>([&](int i) { return base + min(cx.tid + i * PA_POLL_THREADS, ne - 1); }, [&](int) { return tag_in; }, v, cx);
 #pragma unroll
     for (uint32_t i = 0; i < N; i++)
         if (cx.tid + i * PA_POLL_THREADS < ne) recs[cx.tid + i * PA_POLL_THREADS] = __uint_as_float(v[i]);
@@ -805,19 +771,6 @@ __device__ __forceinline__ void pa_merge(const PaArgs& a, uint32_t h, uint32_t t
     }
 }
 
-// One workgroup's part of an argmax: the LAST index among equal maxima (project.rs:501-503).
-__device__ __forceinline__ ArgPair pa_arg_wg(ArgPair v, ArgPair* sh, const PaCtx& cx) {
-    auto fold = [&](auto O) { v = arg_better(v, ArgPair{lane_xor<O.value>(v.v), lane_xor<O.value>(v.i)}); };
-    fold(std::integral_constant<int, 32>{}); fold(std::integral_constant<int, 16>{}); fold(std::integral_constant<int, 8>{});
-    fold(std::integral_constant<int, 4>{}); fold(std::integral_constant<int, 2>{}); fold(std::integral_constant<int, 1>{});
-    __syncthreads();
-    if (cx.lane == 0) sh[cx.wave] = v;
-    __syncthreads();
-    ArgPair r = sh[0];
-    for (uint32_t w = 1; w < PA_WAVES; w++) r = arg_better(r, sh[w]);
-    return r;
-}
-
 // The tag of a phase instance: tag_base + 6 layer + 1 q;k;v, 2 attention (long contexts: its parts, 3 their merge), 4 o, 5 gate;up, 6 down; the argmax's is behind
 // the last layer's.
 template <typename F, bool ORD, bool LONG, int HD, PaFmt W, PaFmt LMW>
@@ -839,7 +792,7 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
     const PaLayer* layers = reinterpret_cast<const PaLayer*>(smem + a.off_layers);
     auto* attn = reinterpret_cast<PaAttn<HD, F::AW>*>(smem + a.off_attn);
 
-    PaCtx cx;
+    PollCtx cx;
     cx.tid = threadIdx.x;
     cx.lane = threadIdx.x & 63u;
     cx.wave = pa_sgpr(threadIdx.x >> 6);
@@ -887,7 +840,7 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
     // system in front of it: 545 us a token at the 1B shape, 451 so)
     // (a workgroup on which nothing depends may come late and find a later phase's element there)
     auto glance = [&](const uint64_t* p, uint32_t tag) {
-        if (cx.wave == 0) pa_poll<1, true>([&](int) { return p; }, [&](int) { return tag; }, nullptr, cx);
+        if (cx.wave == 0) poll_tagged<1, true>([&](int) { return p; }, [&](int) { return tag; }, nullptr, cx);
         __syncthreads();
         return sh_abort == 0;
     };
@@ -973,7 +926,7 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
                             e = min(e, ne - 1);
                             return e < nq ? a.tq + (size_t)part.kvh * nq + e : a.tkv + (e - nq < HD ? part.kvh * HD + (e - nq) : a.KV + part.kvh * HD + (e - nq - HD));
                         };
-                        pa_poll<N>([&](int i) { return at(cx.tid + i * PA_POLL_THREADS); }, [&](int) { return base + 1; }, v, cx);
+                        poll_tagged<N>([&](int i) { return at(cx.tid + i * PA_POLL_THREADS); }, [&](int) { return base + 1; }, v, cx);
 #pragma unroll
                         for (int i = 0; i < N; i++) {
                             const uint32_t e = cx.tid + i * PA_POLL_THREADS;
@@ -1196,7 +1149,7 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
         }
     }
     const uint32_t th = a.tag_base + 6 * a.L + 1;
-    best = pa_arg_wg(best, sh_arg, cx);
+    best = best_of_workgroup<PA_WAVES>(best, sh_arg, cx);
     if (cx.tid == 0) {
         stc64(a.tpart + 2 * cx.wg, th, __float_as_uint(best.v));
         stc64(a.tpart + 2 * cx.wg + 1, th, best.i);
@@ -1206,10 +1159,10 @@ __global__ __launch_bounds__(PA_THREADS) void decode_ahead_kernel(PaArgs a) {
     ArgPair p{-INFINITY, 0};
     for (uint32_t w = cx.tid; w < T; w += PA_THREADS) {
         uint32_t v[2];
-        pa_poll<2>([&](int i) { return a.tpart + 2 * w + (uint32_t)i; }, [&](int) { return th; }, v, cx);
+        poll_tagged<2>([&](int i) { return a.tpart + 2 * w + (uint32_t)i; }, [&](int) { return th; }, v, cx);
         p = arg_better(p, ArgPair{__uint_as_float(v[0]), v[1]});
     }
-    p = pa_arg_wg(p, sh_arg, cx);
+    p = best_of_workgroup<PA_WAVES>(p, sh_arg, cx);
     if (sh_abort) return;
     if (cx.tid == 0) {
         a.state[2] = p.i;

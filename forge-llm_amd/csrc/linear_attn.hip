@@ -37,7 +37,9 @@ __global__ __launch_bounds__(256) void linear_step_kernel(LinearShape sh, const 
     __shared__ v4f part[4][8];
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, head = blockIdx.x, c0 = blockIdx.y * 32 + (tid & 7) * 4, rg = tid >> 3;
     const uint32_t pos = pos_dev ? *pos_dev : base_pos;
-    float* S = state + (size_t)head * sh.dim * sh.vdim + c0;
+    const size_t at = (size_t)head * sh.dim * sh.vdim + c0;
+    const float* S = state + (size_t)(pos & 1u) * sh.state() + at;
+    float* next = state + (size_t)((pos + 1) & 1u) * sh.state() + at;
     v4f s[R];
 #pragma unroll
     for (int i = 0; i < R; i++) {
@@ -67,7 +69,7 @@ __global__ __launch_bounds__(256) void linear_step_kernel(LinearShape sh, const 
             s[i][j] = fmaf(a, s[i][j], k * v[j]);
             acc[j] = fmaf(q, s[i][j], acc[j]);
         }
-        *reinterpret_cast<v4f*>(S + (size_t)d * sh.vdim) = s[i];
+        *reinterpret_cast<v4f*>(next + (size_t)d * sh.vdim) = s[i];
     }
 #pragma unroll
     for (int j = 0; j < 4; j++) acc[j] = lane_xor_add<32>(lane_xor_add<16>(lane_xor_add<8>(acc[j])));
@@ -190,8 +192,8 @@ __global__ __launch_bounds__(256) void linear_chunk_kernel(LinearShape sh, const
     }
 }
 
-// add[chunk] <- the state ahead of the chunk; state <- the one behind the last.  A thread owns one element.
-__global__ __launch_bounds__(256) void linear_scan_kernel(LinearShape sh, uint32_t chunks, const float* __restrict__ total, float* add, float* state, uint32_t base_pos) {
+// add[chunk] <- the state ahead of the chunk; next <- the one behind the last.  A thread owns one element.
+__global__ __launch_bounds__(256) void linear_scan_kernel(LinearShape sh, uint32_t chunks, const float* __restrict__ total, float* add, const float* state, float* next, uint32_t base_pos) {
     const size_t n = sh.state(), i = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= n) return;
     const float* d = total + i / sh.vdim;
@@ -212,7 +214,7 @@ __global__ __launch_bounds__(256) void linear_scan_kernel(LinearShape sh, uint32
             s = fmaf(f[b], s, x[b]);
         }
     }
-    state[i] = s;
+    next[i] = s;
 }
 
 // Workgroup = (chunk, head), key channels 64 at a time.  A wave owns one piece of 16 tokens (loading, its own pairs, the running
@@ -455,7 +457,8 @@ void launch_linear_prompt(DType t, const LinearShape& sh, const LinearIo& io, ui
     static const hipError_t ok = hipFuncSetAttribute((const void*)linear_chunk_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     (void)ok;
     fh::launch(linear_chunk_kernel, dim3(chunks, sh.heads), 256, chunk_lds(sh), s, sh, io.raw, io.w2, io.b2, M, decay, add, total);
-    fh::launch(linear_scan_kernel, dim3((uint32_t)((sh.state() + 255) / 256)), 256, 0, s, sh, chunks, total, add, io.state, io.base_pos);
+    fh::launch(linear_scan_kernel, dim3((uint32_t)((sh.state() + 255) / 256)), 256, 0, s, sh, chunks, total, add, io.state + (io.base_pos & 1u) * sh.state(),
+               io.state + ((io.base_pos + M) & 1u) * sh.state(), io.base_pos);
     if (t == DType::BF16) output<__bf16>(sh, io, M, decay, add, norm, gate, out, ld_out, s);
     else output<float>(sh, io, M, decay, add, norm, gate, out, ld_out, s);
 }
