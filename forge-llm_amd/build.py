@@ -10,7 +10,7 @@ INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 BUILD = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "libforge_hip.so")
 
-SOURCES = ["format.hip", "elementwise.hip", "gemv.hip", "gemv_f32.hip", "gemv_kquant.hip", "kquant_prefill.hip", "gemm.hip", "gemm_rows.hip", "gemm_order.hip", "attn_decode.hip", "attn_prefill.hip",
+SOURCES = ["format.hip", "elementwise.hip", "gemv.hip", "gemv_f32.hip", "gemv_kquant.hip", "kquant_prefill.hip", "gemm.hip", "gemm_rows.hip", "gemm_order.hip", "attn_decode.hip", "attn_step.hip", "attn_prefill.hip",
            "attn_exact.hip", "decode_persistent.hip", "decode_ahead.hip", "decode_block.hip", "api.hip", "model.hip", "llama.hip", "block_model.hip", "block_mixers.hip", "dense.hip",
            "attn_prompt.hip", "attn_latent.hip", "attn_grouped.hip", "linear_attn.hip", "checkpoint.cpp", "gguf.cpp", "sampling.cpp", "resident_seat.cpp"]
 

@@ -414,8 +414,7 @@ int32_t forge_hip_attn_decode_f16kv(const float* q_dev, const uint16_t* k_cache_
     } else {
         rc = g_attn.reserve(attn_decode_workspace_bytes(heads, head_dim));
         if (rc) return rc;
-        launch_attn_decode(q_dev, k_cache_dev, v_cache_dev, out_dev, nullptr, nullptr, seq_len, nullptr, heads, kv_heads,
-                           head_dim, 0u, g_attn.ptr(), (hipStream_t)stream);
+        launch_attn_step(q_dev, k_cache_dev, v_cache_dev, out_dev, seq_len, heads, kv_heads, head_dim, 0u, g_attn.ptr(), (hipStream_t)stream);
     }
     FH_HIP(hipGetLastError());
     return FORGE_HIP_OK;
@@ -432,8 +431,8 @@ int32_t forge_hip_attn_decode_f16kv_paged(const float* q_dev, const uint16_t* k_
     FH_CHECK(attn_decode_paged_supported(seq_len, page_rows), "attn_decode_paged: pages too small for a sequence this long (more than 2048 table entries per split)");
     rc = g_attn.reserve(attn_decode_workspace_bytes(heads, head_dim));
     if (rc) return rc;
-    launch_attn_decode_paged(q_dev, k_pool_dev, v_pool_dev, page_table_dev, page_rows, out_dev, seq_len, heads, kv_heads, head_dim,
-                             g_attn.ptr(), (hipStream_t)stream);
+    launch_attn_step(q_dev, k_pool_dev, v_pool_dev, out_dev, seq_len, heads, kv_heads, head_dim, 0u, g_attn.ptr(), (hipStream_t)stream,
+                     PageTable{page_table_dev, (uint32_t)__builtin_ctz(page_rows)});
     FH_HIP(hipGetLastError());
     return FORGE_HIP_OK;
 }
@@ -454,8 +453,7 @@ int32_t forge_hip_attn_decode_sliding_f16kv(const float* q_dev, const uint16_t* 
     } else {
         rc = g_attn.reserve(attn_decode_workspace_bytes(heads, head_dim));
         if (rc) return rc;
-        launch_attn_decode(q_dev, k_cache_dev, v_cache_dev, out_dev, nullptr, nullptr, seq_len, nullptr, heads, kv_heads, head_dim,
-                           window, g_attn.ptr(), (hipStream_t)stream);
+        launch_attn_step(q_dev, k_cache_dev, v_cache_dev, out_dev, seq_len, heads, kv_heads, head_dim, window, g_attn.ptr(), (hipStream_t)stream);
     }
     FH_HIP(hipGetLastError());
     return FORGE_HIP_OK;

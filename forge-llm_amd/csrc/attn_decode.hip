@@ -30,8 +30,6 @@ __device__ __forceinline__ void merge_state(float& m, float& l, float* a, float 
 // A paged cache (PAGED): kc / vc are pools of pages of 2^page_shift rows, and row t of the sequence is row t % page of
 // pool page page_table[t / page].  A split's table entries are copied into LDS first (they are few), so the address of
 // a key costs one LDS read more than in the flat cache; nothing else changes, the bits included.
-constexpr uint32_t PAGE_ENTRIES_MAX = 2048;   // table entries one split may span (else: contiguous-only)
-
 // workspace record per (kv group, split, head-in-group): [HD acc][m][l]
 template <int HD, int GT, bool PAGED = false>
 __global__ __launch_bounds__(256) void attn_decode_split_kernel(const float* __restrict__ q,
@@ -238,16 +236,6 @@ bool attn_decode_paged_supported(uint32_t seq_len, uint32_t page_rows) {
     return per_split / page_rows + 2 <= PAGE_ENTRIES_MAX;
 }
 
-void launch_attn_decode_paged(const float* q, const uint16_t* k_pool, const uint16_t* v_pool, const uint32_t* page_table,
-                              uint32_t page_rows, float* out, uint32_t seq_len, uint32_t heads, uint32_t kv_heads, uint32_t hd,
-                              void* workspace, hipStream_t s) {
-    float* ws = reinterpret_cast<float*>(workspace);
-    PageTable pt{page_table, (uint32_t)__builtin_ctz(page_rows)};
-    if (hd == 64) launch_hd<64>(q, k_pool, v_pool, out, nullptr, nullptr, seq_len, nullptr, heads, kv_heads, 0u, ws, pt, s);
-    else if (hd == 96) launch_hd<96>(q, k_pool, v_pool, out, nullptr, nullptr, seq_len, nullptr, heads, kv_heads, 0u, ws, pt, s);
-    else launch_hd<128>(q, k_pool, v_pool, out, nullptr, nullptr, seq_len, nullptr, heads, kv_heads, 0u, ws, pt, s);
-}
-
 void launch_attn_decode(const float* q, const uint16_t* kc, const uint16_t* vc, float* out, int8_t* oq, uint16_t* osc,
                         uint32_t seq_len, const uint32_t* pos_dev, uint32_t heads, uint32_t kv_heads, uint32_t hd,
                         uint32_t window, void* workspace, hipStream_t s, PageTable pt) {
@@ -312,10 +300,8 @@ extern "C" int32_t forge_hip_attn_decode_f16kv_noalloc(const float* q_dev, const
     void* ws = nullptr;
     int32_t rc = scratch_on_current_device(&ws);
     if (rc) return rc;
-    // every (head, split) record is written by the split kernel before the merge kernel reads it, empty splits
-    // included, so nothing of the previous call's contents has to be cleared
-    fh::launch_attn_decode(q_dev, k_cache_dev, v_cache_dev, out_dev, nullptr, nullptr, seq_len, nullptr, heads, kv_heads, head_dim, 0u,
-                           ws, (hipStream_t)stream);
+    // every (head, part) record is written before the merge kernel reads it, so nothing of the previous call's contents has to be cleared
+    fh::launch_attn_step(q_dev, k_cache_dev, v_cache_dev, out_dev, seq_len, heads, kv_heads, head_dim, 0u, ws, (hipStream_t)stream);
     FH_HIP(hipGetLastError());
     return FORGE_HIP_OK;
 }

@@ -230,13 +230,13 @@ size_t attn_decode_workspace_bytes(uint32_t heads, uint32_t hd);
 void launch_attn_decode(const float* q, const uint16_t* kc, const uint16_t* vc, float* out, int8_t* oq, uint16_t* osc,
                         uint32_t seq_len, const uint32_t* pos_dev, uint32_t heads, uint32_t kv_heads, uint32_t hd,
                         uint32_t window, void* workspace, hipStream_t s, PageTable pt = PageTable{});
-// The same over a paged cache: k_pool / v_pool fp16 [pages][page_rows][kv_heads*hd], row t of the sequence is row
-// t % page_rows of pool page page_table[t / page_rows].  f32 output, no window.
+// A paged cache: k_pool / v_pool fp16 [pages][page_rows][kv_heads*hd], row t of the sequence is row t % page_rows of pool page page_table[t / page_rows].
 bool attn_decode_paged_supported(uint32_t seq_len, uint32_t page_rows);
-void launch_attn_decode_paged(const float* q, const uint16_t* k_pool, const uint16_t* v_pool, const uint32_t* page_table,
-                              uint32_t page_rows, float* out, uint32_t seq_len, uint32_t heads, uint32_t kv_heads, uint32_t hd,
-                              void* workspace, hipStream_t s);
+constexpr uint32_t PAGE_ENTRIES_MAX = 2048;   // table entries one part of a paged context may span
 
+// attn_step.hip — the same attention for a caller's own loop.  workspace: attn_decode_workspace_bytes(heads, hd).
+void launch_attn_step(const float* q, const uint16_t* kc, const uint16_t* vc, float* out, uint32_t seq, uint32_t heads, uint32_t kv_heads, uint32_t hd, uint32_t window, void* workspace,
+                      hipStream_t s, PageTable pt = PageTable{});
 // Looks up, once per device, the address of the fixed scratch array of forge_hip_attn_decode_f16kv_noalloc on the current
 // device; called from the library's set-up entry points.
 void attn_decode_noalloc_prepare();
