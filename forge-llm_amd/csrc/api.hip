@@ -82,13 +82,19 @@ bool scratch_at_hand(uint32_t K, hipStream_t s) {
     return hipStreamIsCapturing(s, &st) == hipSuccess && st == hipStreamCaptureStatusNone;
 }
 
-// Quantise x[M][K] into the shared scratch; returns pointers.
-int32_t quantise_into_scratch(const float* x, uint32_t M, uint32_t K, int8_t** q, uint16_t** sc, hipStream_t s, bool neg_odd = false) {
+// Room for quantised x[M][K] in the shared scratch; returns pointers.
+int32_t act_scratch(uint32_t M, uint32_t K, int8_t** q, uint16_t** sc) {
     const size_t qbytes = align256((size_t)M * K);
     int32_t rc = g_act.reserve(act_bytes(M, K));
     if (rc) return rc;
     *q = reinterpret_cast<int8_t*>(g_act.ptr());
     *sc = reinterpret_cast<uint16_t*>(reinterpret_cast<uint8_t*>(g_act.ptr()) + qbytes);
+    return FORGE_HIP_OK;
+}
+// Quantise x[M][K] into it.
+int32_t quantise_into_scratch(const float* x, uint32_t M, uint32_t K, int8_t** q, uint16_t** sc, hipStream_t s, bool neg_odd = false) {
+    int32_t rc = act_scratch(M, K, q, sc);
+    if (rc) return rc;
     launch_quantize_act(x, M, K, *q, *sc, s, neg_odd);
     return FORGE_HIP_OK;
 }
@@ -231,7 +237,7 @@ int32_t forge_hip_gemm_q(const forge_hip_qweight* w, const float* x_dev, uint32_
         FH_HIP(hipGetLastError());
         return FORGE_HIP_OK;
     }
-    int32_t rc = quantise_into_scratch(x_dev, M, w->w.K, &q, &sc, (hipStream_t)stream, !exact);   // the fast kernel takes odd blocks negated
+    int32_t rc = act_scratch(M, w->w.K, &q, &sc);
     if (rc) return rc;
     // fast mode may cut tiles along K to fill the CUs: that kernel parks partial tiles in a workspace
     void* split_ws = nullptr;
@@ -244,7 +250,7 @@ int32_t forge_hip_gemm_q(const forge_hip_qweight* w, const float* x_dev, uint32_
         if (fresh) FH_HIP(hipMemsetAsync(g_gemm.ptr(), 0, gemm_split_workspace_bytes(), (hipStream_t)stream));
         split_ws = g_gemm.ptr();
     }
-    launch_gemm(w->w, q, sc, M, y_dev, w->w.N, false, exact, nullptr, (hipStream_t)stream, split_ws);
+    launch_gemm(w->w, q, sc, M, y_dev, w->w.N, false, exact, nullptr, (hipStream_t)stream, split_ws, nullptr, nullptr, nullptr, nullptr, x_dev);
     FH_HIP(hipGetLastError());
     return FORGE_HIP_OK;
 }

@@ -206,14 +206,16 @@ bool gemm_silu_supported(const QWeight& w, uint32_t inter, uint32_t M);
 // mt_a / mt_w (fast mode, Q8_0-layout matrices, no isums): [M][K/32] and [N][K/32] slots of 4 bytes, each a hi | lo pair of
 // fp16 numbers (launch_act_block_sums, kquant_twin_create write them); every element of the result additionally receives
 // sum_b mt_a[m][b] * mt_w[n][b] (before the SiLU epilogue, if any).
+// raw: the activations [M][K] are there and aq, as are not yet.
 void launch_gemm(const QWeight& w, const int8_t* aq, const uint16_t* as, uint32_t M, float* y, uint32_t ldy,
                  bool accumulate, bool exact, int32_t* isums, hipStream_t s, void* split_ws = nullptr, int8_t* silu_q = nullptr,
-                 uint16_t* silu_sc = nullptr, const float* mt_a = nullptr, const float* mt_w = nullptr);
+                 uint16_t* silu_sc = nullptr, const float* mt_a = nullptr, const float* mt_w = nullptr, const float* raw = nullptr);
 // gemm_rows.hip -- the fast mode's product for few rows (the arguments of launch_gemm): launch_gemm goes there itself
 bool gemm_rows_supported(const QWeight& w, uint32_t M, bool silu);
+bool gemm_rows_raw(const QWeight& w, uint32_t M, hipStream_t s);
 double gemm_rows_cost(const QWeight& w, uint32_t M);
 void launch_gemm_rows(const QWeight& w, const int8_t* aq, const uint16_t* as, uint32_t M, float* y, uint32_t ldy, bool accumulate, hipStream_t s,
-                      int8_t* silu_q, uint16_t* silu_sc);
+                      int8_t* silu_q, uint16_t* silu_sc, const float* raw = nullptr);
 // gemm_order.hip -- the same for the order-faithful mode
 bool gemm_order_pays(const QWeight& w, uint32_t M);
 void launch_gemm_order(const QWeight& w, const int8_t* aq, const uint16_t* as, uint32_t M, float* y, uint32_t ldy, bool accumulate, hipStream_t s);

@@ -619,11 +619,16 @@ bool gemm_silu_supported(const QWeight& w, uint32_t inter, uint32_t M) {
 
 void launch_gemm(const QWeight& w, const int8_t* aq, const uint16_t* as, uint32_t M, float* y, uint32_t ldy,
                  bool accumulate, bool exact, int32_t* isums, hipStream_t s, void* split_ws, int8_t* silu_q, uint16_t* silu_sc,
-                 const float* mt_a, const float* mt_w) {
+                 const float* mt_a, const float* mt_w, const float* raw) {
     if (M == 0 || w.N == 0) return;
+    auto quantise = [&]() {
+        if (raw) launch_quantize_act(raw, M, w.K, const_cast<int8_t*>(aq), const_cast<uint16_t*>(as), s, !exact);
+        raw = nullptr;
+    };
     const bool silu = silu_q != nullptr;      // caller: gemm_silu_supported, fast mode, no block-sum dump
     const int accf = accumulate ? 1 : 0;
     const bool q4 = w.wdtype == FORGE_HIP_Q4_0;
+    if (exact) quantise();
     if (exact && !isums && gemm_order_pays(w, M)) {
         launch_gemm_order(w, aq, as, M, y, ldy, accumulate, s);
         return;
@@ -707,12 +712,14 @@ void launch_gemm(const QWeight& w, const int8_t* aq, const uint16_t* as, uint32_
                 // 4 us (1024 -> 8192 by 200 rows: 8.8 planned, 15.5 without and 19.0 with it).  The other kernel has no extra f32 term (MINT).
                 const double tiles_cost = best.cost + (best.items ? 0.0 : 5.0) + (silu ? 4.0 : 0.0);
                 if (!mt_a && gemm_rows_supported(w, M, silu) && gemm_rows_cost(w, M) < tiles_cost) {
-                    launch_gemm_rows(w, aq, as, M, y, ldy, accumulate, s, silu_q, silu_sc);
+                    if (raw && (silu || overlap(raw, (size_t)M * w.K * 4, y, ((size_t)(M - 1) * ldy + w.N) * 4) || !gemm_rows_raw(w, M, s))) quantise();
+                    launch_gemm_rows(w, aq, as, M, y, ldy, accumulate, s, silu_q, silu_sc, raw);
                     return;
                 }
                 tm = best.tm;
                 if (best.items) { fsp = best.sp; items = best.items; }
             }
+            quantise();
             if (items || silu || mt_a) {
                 // the fast kernel's variants: tiles cut along K, the SiLU epilogue, the extra f32 term
                 if (silu) { fsp.silu_q = silu_q; fsp.silu_sc = silu_sc; fsp.inter = w.N / 2; }

@@ -11,7 +11,13 @@
 // that kernel's own rounding reaches 1e-4 of a result, and a row would differ by all of it between a small and a large batch.
 // 32 rows of 2048 -> 8192: 6.2 us (2.7 TB/s of weights) against the tile kernel's 22; 8192 -> 2048: 12.5 against 76 (22 with K ranges);
 // [gate; up] with its epilogue, 2048 -> 16384: 10.5 against 29.5.  Operands fetched straight into registers took 10 and 31 us.
+// The scales' arithmetic is half of a wave's work (16 conversions and FMAs a block and tile), so rows of padding are left out by groups of 8: 2048 -> 8192 by 37 rows 10.7 -> 10.3 us with the
+// quantiser, Q8_0 11.5 -> 10.9, 3072 -> 8192 13.5 -> 12.8, 8192 -> 2048 by 8 Q8_0 15.0 -> 14.0.
+#include <stdlib.h>
+
 #include <algorithm>
+#include <atomic>
+#include <type_traits>
 
 #include "common.h"
 #include "device_utils.h"
@@ -27,6 +33,7 @@ typedef _Float16 v4h __attribute__((ext_vector_type(4)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 
 constexpr int FR_U = 4;                      // blocks of a step: 128 bytes of a Q8_0 or activation row, 64 of a Q4_0 row
+constexpr int FR_AGENT = 16;                 // a load past this XCD's L2 (SC1)
 constexpr uint32_t FR_RSRC = 0x00020000;     // raw buffer, 32-bit data format
 constexpr uint32_t FR_MAGIC = 0x4B400000u;   // 12582912.0f: the bias that makes a block sum a float (gemm.hip)
 constexpr int FR_A_LOG2 = 8;                 // its removal: activation scales times 2^8, weight scales times 2^15 and 2^14
@@ -41,14 +48,34 @@ struct FewArgs {
     int8_t* silu_q;              // SILU: [M][inter] codes (odd blocks negated), [M][inter / 32] scales
     uint16_t* silu_sc;
     uint32_t inter;
+    // RAW: the activations as they come; a workgroup's waves quantise pieces of 64 * 4 elements of them into aq and asc, which are the launch's own until it ends
+    const float* x;
+    unsigned long long *flags, id;   // a piece's flag holds the launch's number when the piece is there
+    uint32_t spin_limit;
 };
+constexpr uint32_t FR_PIECES = 2048;         // flags
+__host__ __device__ inline uint32_t fr_pieces(uint32_t M, uint32_t K) { return (uint32_t)(((uint64_t)M * K / 4 + 63) / 64); }
+__device__ unsigned long long fr_flags[FR_PIECES];
+
+// Piece i of the activations, by one wave.  Other workgroups read it within the launch: stores, and their loads, that say so.
+__device__ __forceinline__ void quantise_piece(const FewArgs& a, uint32_t i, uint32_t lane) {
+    const uint32_t at = i * 64 + lane, n4 = a.M * a.K / 4;
+    const float4 v = at < n4 ? reinterpret_cast<const float4*>(a.x)[at] : make_float4(0.f, 0.f, 0.f, 0.f);
+    uint16_t sb;
+    const uint32_t packed = quantize_block_part(v, sb, ((at >> 3) % (a.K / 32)) & 1u, true);
+    if (at < n4) {
+        __hip_atomic_store(reinterpret_cast<uint32_t*>(const_cast<int8_t*>(a.aq)) + at, packed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if ((at & 7u) == 0) __hip_atomic_store(const_cast<uint16_t*>(a.asc) + (at >> 3), sb, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+}
 
 // One workgroup: 32 MT rows of activations x 32 columns.  SILU: the matrix is [gate; up], a workgroup takes 32 gate columns and the up
 // columns of the same indices and writes quantize(silu(gate) * up) as gemm.hip's epilogue does.
-template <bool Q4, int WAVES, bool SILU, bool BIASED, int MT>
+// G: groups of 8 rows that are worked out of the last tile of 32 (register r of a tile: rows 8 (r / 4) + 4 h + r % 4); the rest is padding.
+template <bool Q4, int WAVES, bool SILU, bool BIASED, int MT, int G, bool RAW>
 __global__ __launch_bounds__(WAVES * 64) void gemm_rows_kernel(FewArgs a) {
     constexpr int NT = SILU ? 2 : 1, KW = WAVES / NT;         // column tiles; waves that share K of one
-    constexpr int THREADS = WAVES * 64, TILE = 1024 * MT;
+    constexpr int THREADS = WAVES * 64, TILE = 1024 * (MT - 1) + 256 * G;
     constexpr int WB = Q4 ? 64 : 128;                         // bytes of a weight row in a step
     constexpr int LA = MT * 32 * 128, LB = 32 * WB;           // LDS bytes of a step's activation tiles / weight tile
     constexpr int WAVE_LDS = LA + LB;
@@ -79,25 +106,29 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_rows_kernel(FewArgs a) {
     // A row's four scales.  An even number of blocks to a row keeps them on 4-byte boundaries and the matrix's end on one; otherwise they
     // are fetched one by one (a word that reaches past the end reads as zero altogether).
     const bool odd_row = (nblk & 1u) != 0;
-    auto load_scales = [&](const __amdgpu_buffer_rsrc_t& rsrc, uint32_t at) {
-        if (!odd_row) return __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(rsrc, at, 0, 0));
+    auto load_scales = [&](const __amdgpu_buffer_rsrc_t& rsrc, uint32_t at, auto aux) {
+        if (!odd_row) return __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(rsrc, at, 0, aux.value));
         uint32_t v[FR_U];
 #pragma unroll
-        for (int u = 0; u < FR_U; u++) v[u] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(rsrc, at + 2 * u, 0, 0) & 0xFFFFu;
+        for (int u = 0; u < FR_U; u++) v[u] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(rsrc, at + 2 * u, 0, aux.value) & 0xFFFFu;
         return make_uint2(v[0] | (v[1] << 16), v[2] | (v[3] << 16));
     };
-    auto load = [&](Step& g, uint32_t st) {
+    auto load_b = [&](Step& g, uint32_t st) {
 #pragma unroll
         for (int i = 0; i < NLB; i++)
             g.B[i] = __builtin_amdgcn_raw_buffer_load_b128(rw, (col0 + i * (Q4 ? 16 : 8) + br) * nblk * (Q4 ? 16 : 32) + st * WB + bp * 16, 0, 0);
-        g.sb = load_scales(rws, (col0 + c) * nblk * 2 + st * 8);
-#pragma unroll
-        for (int i = 0; i < NLA; i++) g.A[i] = __builtin_amdgcn_raw_buffer_load_b128(ra, (m0 + i * 8 + ar) * a.K + st * 128 + ap * 16, 0, 0);
-#pragma unroll
-        for (int t = 0; t < MT; t++) g.sa[t] = load_scales(ras, (m0 + 32 * t + c) * nblk * 2 + st * 8);
+        g.sb = load_scales(rws, (col0 + c) * nblk * 2 + st * 8, std::integral_constant<int, 0>{});
     };
+    auto load_a = [&](Step& g, uint32_t st) {
+#pragma unroll
+        for (int i = 0; i < NLA; i++) g.A[i] = __builtin_amdgcn_raw_buffer_load_b128(ra, (m0 + i * 8 + ar) * a.K + st * 128 + ap * 16, 0, RAW ? FR_AGENT : 0);
+#pragma unroll
+        for (int t = 0; t < MT; t++) g.sa[t] = load_scales(ras, (m0 + 32 * t + c) * nblk * 2 + st * 8, std::integral_constant<int, RAW ? FR_AGENT : 0>{});
+    };
+    auto load = [&](Step& g, uint32_t st) { load_b(g, st); load_a(g, st); };
 
     float acc[MT][16];
+    auto regs = [](int t) { return t < MT - 1 ? 16 : 4 * G; };
 #pragma unroll
     for (int t = 0; t < MT; t++)
 #pragma unroll
@@ -155,14 +186,14 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_rows_kernel(FewArgs a) {
                 const v16f S = __builtin_amdgcn_mfma_f32_32x32x8f16(scale_operand(scale_of(g.sa[t], u)), fb, zero_f, 0, 0, 0);
                 const v16f biased = __builtin_bit_cast(v16f, isum);          // 12582912 +- block sum
 #pragma unroll
-                for (int r = 0; r < 16; r++) acc[t][r] = fmaf(S[r], BIASED ? biased[r] : (float)isum[r], acc[t][r]);
+                for (int r = 0; r < regs(t); r++) acc[t][r] = fmaf(S[r], BIASED ? biased[r] : (float)isum[r], acc[t][r]);
             }
         }
         // the sums are final here: left alone, the compiler works on two steps' products at once and has no registers for them
 #pragma unroll
         for (int t = 0; t < MT; t++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) asm volatile("" : "+v"(acc[t][r]));
+            for (int r = 0; r < regs(t); r++) asm volatile("" : "+v"(acc[t][r]));
     };
     // What eight blocks left of the bias, 1.5 * 2^23 * sum_b a_s[b] * (+-w_s[b]), off the sums: gemm.hip's f16 MFMA over the same eight
     // blocks (most of the biased sums' rounding is made here, and the same eight blocks make the same).
@@ -183,8 +214,36 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_rows_kernel(FewArgs a) {
     };
     // two steps in flight
     Step x0, x1;
-    if (s0 < s1) load(x0, s0);
-    if (s0 + 1 < s1) load(x1, s0 + 1);
+    if constexpr (RAW) {
+        // A wave's pieces first, then its weights, which are on their way while everybody's pieces are waited for.
+        const uint32_t n = fr_pieces(a.M, a.K), grid = gridDim.x * gridDim.y;
+        __shared__ uint32_t late;
+        if (tid == 0) late = 0;
+        for (uint32_t i = blockIdx.y * gridDim.x + blockIdx.x + wave * grid; i < n; i += WAVES * grid) {
+            quantise_piece(a, i, lane);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");         // acknowledged
+            if (lane == 0) __hip_atomic_store(a.flags + i, a.id, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        if (s0 < s1) load_b(x0, s0);
+        if (s0 + 1 < s1) load_b(x1, s0 + 1);
+        __syncthreads();
+        for (uint32_t p = tid; p < n; p += THREADS) {
+            uint32_t rounds = 0;
+            while (__hip_atomic_load(a.flags + p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != a.id)
+                if (++rounds >= a.spin_limit) { late = 1; break; }
+        }
+        __syncthreads();
+        if (late) {                                                  // somebody is not there: the same codes once more
+            for (uint32_t j = wave; j < n; j += WAVES) quantise_piece(a, j, lane);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
+        }
+        if (s0 < s1) load_a(x0, s0);
+        if (s0 + 1 < s1) load_a(x1, s0 + 1);
+    } else {
+        if (s0 < s1) load(x0, s0);
+        if (s0 + 1 < s1) load(x1, s0 + 1);
+    }
     for (uint32_t st = s0; st < s1; st += 2) {
         compute(x0, st);
         uint2 a0[MT], a1[MT], w0 = x0.sb, w1 = make_uint2(0u, 0u);
@@ -207,7 +266,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_rows_kernel(FewArgs a) {
 #pragma unroll
     for (int t = 0; t < MT; t++)
 #pragma unroll
-        for (int r = 0; r < 16; r++) red[(16 * t + r) * 64 + lane] = acc[t][r];
+        for (int r = 0; r < regs(t); r++) red[(16 * t + r) * 64 + lane] = acc[t][r];
     __syncthreads();
     for (uint32_t e = tid; e < TILE; e += THREADS) {
         float v[NT];
@@ -243,15 +302,37 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_rows_kernel(FewArgs a) {
     }
 }
 
-template <bool Q4, bool SILU, int MT>
-void launch_rows(const FewArgs& a, hipStream_t s) {
+template <bool Q4, bool SILU, int MT, int G, bool RAW>
+void launch_groups(const FewArgs& a, hipStream_t s) {
     constexpr int WAVES = 8;       // sixteen leave a wave 128 registers, and two steps in flight do not fit them
     const dim3 grid(((SILU ? a.inter : a.N) + 31) / 32, (a.M + 32 * MT - 1) / (32 * MT));
-    if (a.K > 4096) fh::launch(gemm_rows_kernel<Q4, WAVES, SILU, true, MT>, grid, WAVES * 64, 0, s, a);
-    else fh::launch(gemm_rows_kernel<Q4, WAVES, SILU, false, MT>, grid, WAVES * 64, 0, s, a);
+    if (a.K > 4096) fh::launch(gemm_rows_kernel<Q4, WAVES, SILU, true, MT, G, RAW>, grid, WAVES * 64, 0, s, a);
+    else fh::launch(gemm_rows_kernel<Q4, WAVES, SILU, false, MT, G, RAW>, grid, WAVES * 64, 0, s, a);
+}
+template <bool Q4, bool SILU, int MT, bool RAW>
+void launch_rows(const FewArgs& a, hipStream_t s) {
+    // one row of workgroups: its last tile's rows are known here
+    const uint32_t left = a.M > 32 * (MT - 1) && a.M <= 32 * MT ? a.M - 32 * (MT - 1) : 32;
+    if (left <= 8) launch_groups<Q4, SILU, MT, 1, RAW>(a, s);
+    else if (left <= 16) launch_groups<Q4, SILU, MT, 2, RAW>(a, s);
+    else launch_groups<Q4, SILU, MT, 4, RAW>(a, s);
 }
 
 }  // namespace
+
+static unsigned long long* fr_flags_of_device() {
+    constexpr int MAX = 16;
+    static std::atomic<unsigned long long*> of[MAX] = {};
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= MAX) return nullptr;
+    unsigned long long* p = of[dev].load(std::memory_order_relaxed);
+    if (!p) {
+        void* v = nullptr;
+        if (hipGetSymbolAddress(&v, HIP_SYMBOL(fr_flags)) != hipSuccess) { (void)hipGetLastError(); return nullptr; }
+        of[dev].store(p = static_cast<unsigned long long*>(v), std::memory_order_relaxed);
+    }
+    return p;
+}
 
 // 32-bit byte offsets, and a grid's second dimension ends at 65535 (2.1 million rows, which its estimate would take for narrow, shallow matrices).
 bool gemm_rows_supported(const QWeight& w, uint32_t M, bool silu) {
@@ -268,6 +349,19 @@ static uint32_t rounds(const QWeight& w, uint32_t M, uint32_t mt) { return (uint
 static double two_rows_take(const QWeight& w) { return w.K > 4096 ? 1.8 : 1.6; }
 static uint32_t tile_rows(const QWeight& w, uint32_t M) { return two_rows_take(w) * rounds(w, M, 2) < rounds(w, M, 1) ? 2 : 1; }
 
+// Whether one launch quantises the activations too.  The hand-over of the codes inside it (2 us) hides where a caller's loop waits for the host's launches (9.6 us for two, 6.5 for
+// one), or where they are few.  us, two launches / one, Q4_0: 576 -> 1536 by 2 .. 200 rows 9.7 / 7.4, 2048 -> 2048 by 2 .. 64 9.5 / 7.3, by 128 9.5 / 8.1, 2048 -> 512 by 16 9.6 / 7.4,
+// 128 (two pieces a wave) 9.7 / 9.1, 2048 -> 8192 by 2 9.7 / 7.8, 32 9.6 / 8.7, 64 (two tiles) 11.2 / 11.2, 8192 -> 2048 by 8 13.4 / 12.0, 32 14.4 / 15.3, 3072 -> 8192 by 2 9.6 / 9.2,
+// 16 9.9 / 10.8, 3072 -> 1024 by 16 9.4 / 7.4, 64 9.4 / 9.5; Q8_0 2048 -> 8192 by 16 9.8 / 9.4, 32 9.5 / 9.7.
+// The whole grid has to be at work at a time (512 workgroups: those at work wait until they give up).  Recorded into a graph the launch would find its number from the replay before.
+bool gemm_rows_raw(const QWeight& w, uint32_t M, hipStream_t s) {
+    const uint64_t grid = (w.N + 31) / 32 * (((uint64_t)M + 31) / 32), bytes = (uint64_t)w.N * w.qs_row_bytes();
+    const bool pays = M <= 8 ? bytes <= (20u << 20) : M <= 16 ? w.K <= 2048 || bytes <= (4u << 20) : w.K <= 2048 && bytes <= (10u << 20);
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    return pays && tile_rows(w, M) == 1 && grid <= 256 && fr_pieces(M, w.K) <= std::min<uint64_t>(FR_PIECES, 16 * grid) && fr_flags_of_device() &&
+           hipStreamIsCapturing(s, &st) == hipSuccess && st == hipStreamCaptureStatusNone;
+}
+
 // Microseconds of a launch, for the choice between the kernels.  Tiles come in rounds of one to a compute unit; a round takes 1.8 plus 2.7 per
 // 2048 of depth, or what its columns take from memory at 4.8 TB/s (with the quantiser, 1 / 2 / 3 / 4 rounds: K = 2048 9.9 / 14.2 / 18.8 / 23.5,
 // K = 4096 13 / 20 / 27 / 34, K = 8192 17.5 / 29 / 40 / 52).  1422 products of 2 to 1300 rows were timed both ways, with one row of tiles to a
@@ -279,14 +373,23 @@ double gemm_rows_cost(const QWeight& w, uint32_t M) {
 }
 
 void launch_gemm_rows(const QWeight& w, const int8_t* aq, const uint16_t* as, uint32_t M, float* y, uint32_t ldy, bool accumulate, hipStream_t s,
-                      int8_t* silu_q, uint16_t* silu_sc) {
-    const FewArgs a{w.qs, w.scales, aq, as, y, M, w.N, w.K, ldy, accumulate ? 1u : 0u, silu_q, silu_sc, w.N / 2};
+                      int8_t* silu_q, uint16_t* silu_sc, const float* raw) {
+    FewArgs a{w.qs, w.scales, aq, as, y, M, w.N, w.K, ldy, accumulate ? 1u : 0u, silu_q, silu_sc, w.N / 2, raw, nullptr, 0, 0};
+    if (raw) {
+        static const uint32_t limit = [] { const char* e = getenv("FORGE_HIP_PD_SPIN_LIMIT"); return e && atoi(e) > 0 ? (uint32_t)atoi(e) : 64u; }();
+        a.spin_limit = limit;
+        static std::atomic<unsigned long long> number{0};
+        a.id = ++number;
+        a.flags = fr_flags_of_device();
+    }
     const bool q4 = w.wdtype == FORGE_HIP_Q4_0, silu = silu_q != nullptr;
     auto go = [&](auto q4_, auto silu_) {
-        if (tile_rows(w, M) == 2) launch_rows<decltype(q4_)::value, decltype(silu_)::value, 2>(a, s);
-        else launch_rows<decltype(q4_)::value, decltype(silu_)::value, 1>(a, s);
+        if (tile_rows(w, M) == 2) launch_rows<decltype(q4_)::value, decltype(silu_)::value, 2, false>(a, s);
+        else launch_rows<decltype(q4_)::value, decltype(silu_)::value, 1, false>(a, s);
     };
-    if (q4 && silu) go(std::true_type{}, std::true_type{});
+    if (raw && q4) launch_rows<true, false, 1, true>(a, s);
+    else if (raw) launch_rows<false, false, 1, true>(a, s);
+    else if (q4 && silu) go(std::true_type{}, std::true_type{});
     else if (q4) go(std::true_type{}, std::false_type{});
     else if (silu) go(std::false_type{}, std::true_type{});
     else go(std::false_type{}, std::false_type{});
