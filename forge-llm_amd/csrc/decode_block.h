@@ -8,7 +8,7 @@
 
 namespace fh {
 
-// decode_block.hip — the decode step of a small bfloat16 block network as one resident kernel.  The functions are the pd_ ones' counterparts.
+// decode_block.hip — the decode step of a bfloat16 block network as one resident kernel.  The functions are the pd_ ones' counterparts.
 struct PbMixer {
     MixerKind kind;
     LatentShape latent;                      // the kind's own is filled, the others are as constructed

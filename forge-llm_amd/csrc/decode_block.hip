@@ -1,5 +1,5 @@
-// One decode token of a block network (block_model.hip) as ONE kernel: small bfloat16 models, whose step is a chain of 150 to 210 products and attentions that read almost
-// nothing each.
+// One decode token of a block network (block_model.hip) as ONE kernel: bfloat16 models, whose step is a chain of 90 to 210 products and attentions.  First small ones, that read almost
+// nothing each; the wide form at the end is for layers that registers do not hold.
 //
 // As kernels in a graph a link of that chain is 2.4 to 6 us however small; here it is a hand-over of 1.2 us and what it computes (resident.h: tagged elements, bounded waits,
 // a buffer is overwritten only by a phase whose inputs transitively depend on every reader of what it held).  The form is decode_ahead.hip's:
@@ -104,7 +104,7 @@ struct PbArgs {
     unsigned long long* host_out;
     uint32_t host_seq;
     unsigned long long* stamps;
-    uint32_t plane, off_red, off_stats, off_layers, off_attn;      // plane: elements of a vector's plane (bytes 0 .. 4 planes); LDS byte offsets
+    uint32_t plane, off_red, off_stats, off_layers, off_attn, off_in;      // plane: elements of a vector's plane (bytes 0 .. 4 planes); LDS byte offsets
 };
 // Tags of a layer run, behind its base.
 enum PbTag : uint32_t { PB_T_LOOP = 1, PB_T_RAW, PB_T_REC, PB_T_OUT, PB_T_O, PB_T_ACT, PB_T_DOWN, PB_TAGS };
@@ -289,9 +289,9 @@ __device__ __forceinline__ void pb_attend(PbKeys<CK, VK, LATENT>& kv, PbRun<VK>&
 }
 
 // LDS of a workgroup that attends, VD values for each of H heads.
-template <uint32_t VD, uint32_t H>
+template <uint32_t VD, uint32_t H, uint32_t WAVES>
 struct PbMerge {
-    float o[PB_WAVES][H][VD], m[PB_WAVES][H], l[PB_WAVES][H];
+    float o[WAVES][H][VD], m[WAVES][H], l[WAVES][H];
 };
 struct PbLatentLds {
     alignas(16) __bf16 ct[PB_WAVES][PB_RANK * PB_CT];
@@ -301,30 +301,33 @@ struct PbLatentLds {
     alignas(16) __bf16 q[PB_DIM], row[PB_ROW], fresh[PB_ROW];      // unrotated query; the query against a cached row; this position's row
     float raw[PB_QR + PB_ROW + PB_VDIM];
     float out[PB_VDIM];
-    PbMerge<PB_RANK, 1> merge;
+    PbMerge<PB_RANK, 1, PB_WAVES> merge;
 };
+template <uint32_t WAVES>
 struct PbGroupedLds {
-    alignas(16) __bf16 ct[PB_WAVES][64 * PB_CT];
-    alignas(16) __bf16 p[PB_WAVES][16 * PB_CT];
+    alignas(16) __bf16 ct[WAVES][64 * PB_CT];
+    alignas(16) __bf16 p[WAVES][16 * PB_CT];
     alignas(16) __bf16 q[16][64 + 8];
     alignas(16) __bf16 k[64], v[64];
     float raw[(PB_GROUP + 2) * 64 + PB_GROUP * 64];
-    PbMerge<64, PB_GROUP> merge;
+    PbMerge<64, PB_GROUP, WAVES> merge;
 };
+template <uint32_t WAVES>
 struct PbLinearLds {
     float raw[2 * 64 + 2 * PB_LVDIM + PB_LOW];
     float a[64];
-    alignas(16) v4f part[PB_WAVES][PB_LVDIM / 4];
+    alignas(16) v4f part[WAVES][PB_LVDIM / 4];
 };
+template <uint32_t WAVES>
 struct PbKakiraxLds {
-    PbGroupedLds grouped;
-    PbLinearLds linear;
+    PbGroupedLds<WAVES> grouped;
+    PbLinearLds<WAVES> linear;
 };
 
 // The waves' sums as the workgroup's part, thread t: head t / VD, value t % VD.  w: the part's weight sum.
 struct PbPart { float o, m, l; };
-template <uint32_t VD, uint32_t H>
-__device__ __forceinline__ PbPart pb_waves(const PbMerge<VD, H>& sh, uint32_t waves, uint32_t head, uint32_t d) {
+template <uint32_t VD, uint32_t H, uint32_t WAVES>
+__device__ __forceinline__ PbPart pb_waves(const PbMerge<VD, H, WAVES>& sh, uint32_t waves, uint32_t head, uint32_t d) {
     PbPart p{0.f, PB_NO_KEYS, 0.f};
 #pragma unroll 4
     for (uint32_t w = 0; w < waves; w++) p.m = fmaxf(p.m, sh.m[w][head]);
@@ -336,8 +339,8 @@ __device__ __forceinline__ PbPart pb_waves(const PbMerge<VD, H>& sh, uint32_t wa
     }
     return p;
 }
-template <int VK, uint32_t VD, uint32_t H>
-__device__ __forceinline__ void pb_leave(PbMerge<VD, H>& sh, const PbRun<VK>& run, uint32_t heads, uint32_t wave, uint32_t lane) {
+template <int VK, uint32_t VD, uint32_t H, uint32_t WAVES>
+__device__ __forceinline__ void pb_leave(PbMerge<VD, H, WAVES>& sh, const PbRun<VK>& run, uint32_t heads, uint32_t wave, uint32_t lane) {
     const uint32_t l16 = lane & 15u, lg = lane >> 4;
     const float l = lane_xor_add<32>(lane_xor_add<16>(run.l));
     if (l16 >= heads) return;
@@ -352,8 +355,8 @@ __device__ __forceinline__ void pb_leave(PbMerge<VD, H>& sh, const PbRun<VK>& ru
 
 // The parts of `heads` heads: everybody but the first hands its part over, the first adds all up.  Thread t < heads * vd: head t / vd, value t % vd; returns its
 // weighted mean (first only).  False: the step is given up.
-template <uint32_t VD, uint32_t H>
-__device__ __forceinline__ bool pb_parts(const PbArgs& a, const PbMerge<VD, H>& sh, uint32_t owner, uint32_t split, uint32_t heads, uint32_t vd, uint32_t tag, float* recs, float& mean,
+template <uint32_t VD, uint32_t H, uint32_t WAVES>
+__device__ __forceinline__ bool pb_parts(const PbArgs& a, const PbMerge<VD, H, WAVES>& sh, uint32_t owner, uint32_t split, uint32_t heads, uint32_t vd, uint32_t tag, float* recs, float& mean,
                                          const PollCtx& cx) {
     const uint32_t n = heads * vd, rec = heads * (vd + 2), head = cx.tid / vd, d = cx.tid - head * vd;
     PbPart p{0.f, PB_NO_KEYS, 1.f};
@@ -577,9 +580,10 @@ __device__ __forceinline__ bool pb_latent_layers(const PbArgs& a, const PbLayer*
 
 // ---- grouped attention: a workgroup per (key / value head, part) -------------------------------------------------------------------
 // [norms, rotation, cache row | attention | merge * gate]
-__device__ __forceinline__ bool pb_grouped_layer(const PbArgs& a, const PbLayer& L, PbGroupedLds* sh, float* recs, uint32_t l, uint32_t pos, PollCtx& cx) {
+template <uint32_t WAVES>
+__device__ __forceinline__ bool pb_grouped_layer(const PbArgs& a, const PbLayer& L, PbGroupedLds<WAVES>* sh, float* recs, uint32_t role, uint32_t l, uint32_t pos, PollCtx& cx) {
     const GroupedShape& s = a.gs;
-    const uint32_t role = cx.wg - a.G, kvh = role / a.splits, split = role - kvh * a.splits, group = s.group();
+    const uint32_t kvh = role / a.splits, split = role - kvh * a.splits, group = s.group();
     const uint32_t lane = cx.lane, l16 = lane & 15u, lg = lane >> 4, wave = cx.wave, tid = cx.tid, base = a.tag_base + l * PB_TAGS;
     const uint32_t nk = s.dim / 32, nv = s.vdim / 32, span = PB_KEYS * a.attend, first0 = wave < a.attend ? split * span + wave * PB_KEYS : 0xFFFFFFFFu, step = a.splits * span;
     uint8_t *kc = pb_ptr(L.cache), *vc = pb_ptr(L.cache_v);
@@ -638,7 +642,7 @@ __device__ __forceinline__ bool pb_grouped_layer(const PbArgs& a, const PbLayer&
                 stg(reinterpret_cast<uint64_t*>(kc + ((size_t)pos * s.k_row() + kvh * s.dim) * 2) + sub, ((uint64_t)b.y << 32) | b.x);
             }
         }
-    } else if (wave == PB_POLL) {
+    } else if (wave == (WAVES > PB_POLL ? PB_POLL : WAVES - 1)) {
         for (uint32_t i = lane; i < s.vdim; i += 64) {
             const __bf16 b = (__bf16)sh->raw[ge + i];
             sh->v[i] = b;
@@ -672,28 +676,39 @@ __device__ __forceinline__ bool pb_grouped_layer(const PbArgs& a, const PbLayer&
 
 // ---- linear attention: a workgroup per head -------------------------------------------------------------------------------------------
 // [decay | state, read-out | norm * gate].  The state of position p is in half p % 2 of the buffer: a step that is given up leaves its own untouched.
-__device__ __forceinline__ bool pb_linear_layer(const PbArgs& a, const PbLayer& L, PbLinearLds* sh, uint32_t l, uint32_t pos, PollCtx& cx) {
-    const LinearShape& s = a.ns;
-    const uint32_t head = cx.wg - a.G, lane = cx.lane, wave = cx.wave, tid = cx.tid, base = a.tag_base + l * PB_TAGS;
-    const uint32_t cols = s.vdim / 4, groups = PB_THREADS / cols, rg = tid / cols, c = tid - rg * cols;      // cols divides the wave
-    float* state = reinterpret_cast<float*>(pb_ptr(L.cache));
-    const float* from = state + (size_t)(pos & 1u) * s.state() + (size_t)head * s.dim * s.vdim;
-    float* to = state + (size_t)((pos + 1) & 1u) * s.state() + (size_t)head * s.dim * s.vdim;
-    v4f st[PB_STATE];
+template <uint32_t WAVES>
+struct PbLinear {
+    static constexpr int STATE = PB_STATE * PB_WAVES / WAVES <= 8 ? PB_STATE * PB_WAVES / WAVES : 8;
+    static constexpr uint32_t THREADS = WAVES * 64;
+    v4f st[STATE];
+    float w2[PB_LOW], b2, nw[PB_LVDIM / 64];
+    // what a head's step reads that no other workgroup makes
+    __device__ __forceinline__ void load(const PbArgs& a, const PbLayer& L, uint32_t head, uint32_t pos, uint32_t tid, uint32_t lane) {
+        const LinearShape& s = a.ns;
+        const uint32_t cols = s.vdim / 4, groups = THREADS / cols, rg = tid / cols, c = tid - rg * cols;
+        const float* from = reinterpret_cast<float*>(pb_ptr(L.cache)) + (size_t)(pos & 1u) * s.state() + (size_t)head * s.dim * s.vdim;
 #pragma unroll
-    for (uint32_t i = 0; i < (uint32_t)PB_STATE; i++)
-        st[i] = __builtin_bit_cast(v4f, ldg(reinterpret_cast<const uint4*>(from + min(rg + i * groups, s.dim - 1) * s.vdim + 4 * c)));
-    float w2[PB_LOW], b2;
-    {
+        for (uint32_t i = 0; i < (uint32_t)STATE; i++)
+            st[i] = __builtin_bit_cast(v4f, ldg(reinterpret_cast<const uint4*>(from + min(rg + i * groups, s.dim - 1) * s.vdim + 4 * c)));
         const float* w = pb_ptr(L.wa);
         const uint32_t ch = head * s.dim + min(tid, s.dim - 1);
         b2 = pb_f32(pb_ptr(L.wb), ch);
 #pragma unroll
         for (uint32_t r = 0; r < PB_LOW; r++) w2[r] = pb_f32(w, min(r, s.rank - 1) * s.qk() + ch);
-    }
-    float nw[PB_LVDIM / 64];
 #pragma unroll
-    for (uint32_t i = 0; i < PB_LVDIM / 64; i++) nw[i] = pb_f32(pb_ptr(L.wc), min(lane + 64 * i, s.vdim - 1));
+        for (uint32_t i = 0; i < PB_LVDIM / 64; i++) nw[i] = pb_f32(pb_ptr(L.wc), min(lane + 64 * i, s.vdim - 1));
+    }
+};
+template <uint32_t WAVES>
+__device__ __forceinline__ bool pb_linear_layer(const PbArgs& a, const PbLayer& L, PbLinear<WAVES>& in, PbLinearLds<WAVES>* sh, uint32_t head, uint32_t l, uint32_t pos, PollCtx& cx) {
+    constexpr int STATE = PbLinear<WAVES>::STATE;
+    const LinearShape& s = a.ns;
+    const uint32_t lane = cx.lane, wave = cx.wave, tid = cx.tid, base = a.tag_base + l * PB_TAGS;
+    const uint32_t cols = s.vdim / 4, groups = PbLinear<WAVES>::THREADS / cols, rg = tid / cols, c = tid - rg * cols;      // cols divides the wave
+    float* to = reinterpret_cast<float*>(pb_ptr(L.cache)) + (size_t)((pos + 1) & 1u) * s.state() + (size_t)head * s.dim * s.vdim;
+    v4f (&st)[STATE] = in.st;
+    float (&w2)[PB_LOW] = in.w2, (&nw)[PB_LVDIM / 64] = in.nw;
+    const float b2 = in.b2;
     // q, k, v, gate, low
     const uint32_t e1 = s.dim, e2 = 2 * s.dim, e3 = e2 + s.vdim, e4 = e3 + s.vdim, ne = e4 + s.rank;
     if (wave < PB_POLL) {
@@ -723,7 +738,7 @@ __device__ __forceinline__ bool pb_linear_layer(const PbArgs& a, const PbLayer& 
     v4f acc = (v4f){0.f, 0.f, 0.f, 0.f};
     const v4f v = *reinterpret_cast<const v4f*>(sh->raw + e2 + 4 * c);
 #pragma unroll
-    for (uint32_t i = 0; i < (uint32_t)PB_STATE; i++) {
+    for (uint32_t i = 0; i < (uint32_t)STATE; i++) {
         const uint32_t d = rg + i * groups;
         if (d < s.dim) {
             const float dec = sh->a[d], k = sh->raw[e1 + d], q = sh->raw[d] * s.q_scale;
@@ -751,7 +766,7 @@ __device__ __forceinline__ bool pb_linear_layer(const PbArgs& a, const PbLayer& 
             o[i] = 0.f;
             if (e < s.vdim) {
 #pragma unroll
-                for (uint32_t w = 0; w < PB_WAVES; w++) o[i] += reinterpret_cast<const float*>(sh->part[w])[e];
+                for (uint32_t w = 0; w < WAVES; w++) o[i] += reinterpret_cast<const float*>(sh->part[w])[e];
             }
             ss = fmaf(o[i], o[i], ss);                                // zero past vdim_n
         }
@@ -765,11 +780,63 @@ __device__ __forceinline__ bool pb_linear_layer(const PbArgs& a, const PbLayer& 
     }
     // the state is the next step's
 #pragma unroll
-    for (uint32_t i = 0; i < (uint32_t)PB_STATE; i++) {
+    for (uint32_t i = 0; i < (uint32_t)STATE; i++) {
         const uint32_t d = rg + i * groups;
         if (d < s.dim) stg(reinterpret_cast<uint4*>(to + d * s.vdim + 4 * c), __builtin_bit_cast(uint4, st[i]));
     }
     return true;
+}
+
+// The logits of a tile of 16 rows and the best of them; every column is the same: lane l holds rows 4 (l / 16) .. + 3.
+__device__ __forceinline__ void pb_logits(const PbArgs& a, uint32_t tile, const v4f& acc, uint32_t lane, ArgPair& best) {
+#pragma unroll
+    for (uint32_t r = 0; r < 4; r++) {
+        const uint32_t row = tile * 16 + 4 * (lane >> 4) + r;
+        if (row >= a.head.N || (lane & 15u) != r) continue;
+        float v = acc[r];
+        if (a.cap > 0.f) v = a.cap * tanhf(v / a.cap);
+        stg(a.logits + row, v);
+        // apply_repeat_penalty (project.rs:505-513) ahead of the argmax.  The lane that holds the row of the token being fed is the only one in the grid to touch
+        // that counter: it adds this step's occurrence.
+        if (a.penalty > 1.0f) {
+            const bool fed = row == a.token;
+            const uint32_t n = ldg(a.counts + row) + (fed ? 1u : 0u);
+            if (fed) { stg(a.counts + row, n); stg(a.state + 4, a.step_seq); }      // so that a step that gives up later can be undone
+            v = repeat_penalised(v, n, a.penalty);
+        }
+        best = arg_better(best, ArgPair{v, row});
+    }
+}
+// The grid's best, by its first workgroup; the step's end.
+__device__ __forceinline__ void pb_choose(const PbArgs& a, ArgPair best, ArgPair* sh_arg, uint32_t pos, PollCtx& cx) {
+    const uint32_t th = a.tag_base + a.L * PB_TAGS, T = gridDim.x;
+    auto stamp = [&](uint32_t slot) {
+        if (a.stamps && cx.wg == 0 && cx.tid == 0) a.stamps[slot] = wall_clock64();
+    };
+    best = best_of_workgroup<PB_WAVES>(best, sh_arg, cx);
+    if (cx.tid == 0) {
+        stc64(a.tpart + 2 * cx.wg, th, __float_as_uint(best.v));
+        stc64(a.tpart + 2 * cx.wg + 1, th, best.i);
+    }
+    stamp(5 * a.L + 1);
+    if (cx.wg != 0) return;
+    ArgPair p{-INFINITY, 0};
+    for (uint32_t w = cx.tid; w < T; w += PB_THREADS) {
+        uint32_t v[2];
+        poll_tagged<2>([&](int i) { return a.tpart + 2 * w + (uint32_t)i; }, [&](int) { return th; }, v, cx);
+        p = arg_better(p, ArgPair{__uint_as_float(v[0]), v[1]});
+    }
+    p = best_of_workgroup<PB_WAVES>(p, sh_arg, cx);
+    if (*cx.sh_abort) return;
+    if (cx.tid == 0) {
+        a.state[2] = p.i;
+        a.state[1] = p.i;
+        a.state[0] = pos + 1;
+        if (!(a.penalty > 1.0f)) a.counts[a.token] += 1;          // nobody read the counters in this launch
+        stamp(5 * a.L + 2);
+        // the host may be spinning on this word instead of waiting for the stream
+        if (a.host_out) __hip_atomic_store(a.host_out, ((unsigned long long)a.host_seq << 32) | p.i, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
 }
 
 // ---- the kernel ---------------------------------------------------------------------------------------------------------------------------
@@ -783,7 +850,7 @@ __global__ __launch_bounds__(PB_THREADS) void decode_block_kernel(PbArgs a) {
     float* const red = reinterpret_cast<float*>(smem + a.off_red);                // [tile][wave][16 rows]
     float* const stats = reinterpret_cast<float*>(smem + a.off_stats);            // [wave][mean, sum of squares around it]
     const PbLayer* layers = reinterpret_cast<const PbLayer*>(smem + a.off_layers);
-    typedef std::conditional_t<LATENT, PbLatentLds, PbKakiraxLds> AttnLds;
+    typedef std::conditional_t<LATENT, PbLatentLds, PbKakiraxLds<PB_WAVES>> AttnLds;
     AttnLds* attn = reinterpret_cast<AttnLds*>(smem + a.off_attn);
     float* recs;                              // parts of other workgroups: where the transposed values are, when those are done with
     if constexpr (LATENT) recs = reinterpret_cast<float*>(attn->ct);
@@ -1108,8 +1175,10 @@ __global__ __launch_bounds__(PB_THREADS) void decode_block_kernel(PbArgs a) {
             for (uint32_t l = 0; (on_n || on_g) && l < a.L; l++) {
                 asm volatile("" : "+v"(cx.tid), "+v"(cx.lane));
                 if (pb_sgpr(layers[l].kind) == PB_FIRST) {
-                    if (on_n && !pb_linear_layer(a, layers[l], &attn->linear, l, pos, cx)) return;
-                } else if (on_g && !pb_grouped_layer(a, layers[l], &attn->grouped, recs, l, pos, cx)) {
+                    PbLinear<PB_WAVES> in;
+                    if (on_n) in.load(a, layers[l], role, pos, cx.tid, cx.lane);
+                    if (on_n && !pb_linear_layer(a, layers[l], in, &attn->linear, role, l, pos, cx)) return;
+                } else if (on_g && !pb_grouped_layer<PB_WAVES>(a, layers[l], &attn->grouped, recs, role, l, pos, cx)) {
                     return;
                 }
             }
@@ -1148,24 +1217,7 @@ __global__ __launch_bounds__(PB_THREADS) void decode_block_kernel(PbArgs a) {
                 acc = mma16(w.f[0][i], load8(k < mh.K / 32 ? x1 + 32 * k : zeros), acc);
             }
             if (u.chunk + 1 < chunks) return;
-            // every column is the same: lane l holds rows 4 (l / 16) .. + 3
-#pragma unroll
-            for (uint32_t r = 0; r < 4; r++) {
-                const uint32_t row = u.tile * 16 + 4 * (cx.lane >> 4) + r;
-                if (row >= mh.N || (cx.lane & 15u) != r) continue;
-                float v = acc[r];
-                if (a.cap > 0.f) v = a.cap * tanhf(v / a.cap);
-                stg(a.logits + row, v);
-                // apply_repeat_penalty (project.rs:505-513) ahead of the argmax.  The lane that holds the row of the token being fed is the only one in the grid to touch
-                // that counter: it adds this step's occurrence.
-                if (a.penalty > 1.0f) {
-                    const bool fed = row == a.token;
-                    const uint32_t n = ldg(a.counts + row) + (fed ? 1u : 0u);
-                    if (fed) { stg(a.counts + row, n); stg(a.state + 4, a.step_seq); }      // so that a step that gives up later can be undone
-                    v = repeat_penalised(v, n, a.penalty);
-                }
-                best = arg_better(best, ArgPair{v, row});
-            }
+            pb_logits(a, u.tile, acc, cx.lane, best);
             acc = (v4f){0.f, 0.f, 0.f, 0.f};
         };
         head_load(wh[1], u1);
@@ -1179,31 +1231,409 @@ __global__ __launch_bounds__(PB_THREADS) void decode_block_kernel(PbArgs a) {
             head_load(wh[1], v);
         }
     }
-    const uint32_t th = a.tag_base + a.L * PB_TAGS;
-    best = best_of_workgroup<PB_WAVES>(best, sh_arg, cx);
-    if (cx.tid == 0) {
-        stc64(a.tpart + 2 * cx.wg, th, __float_as_uint(best.v));
-        stc64(a.tpart + 2 * cx.wg + 1, th, best.i);
+    pb_choose(a, best, sh_arg, pos, cx);
+}
+
+// ---- the wide form ------------------------------------------------------------------------------------------------------------------------
+// Layers that registers cannot hold (linear and grouped attention): every workgroup streams its rows of every matrix, and the heads are the polling waves' of as many workgroups.  A tile is
+// 8 rows by two halves of the depth (row r of the product: row r % 8, half r / 8), tile t of a workgroup the grid's tile t G + wg: no row of a 2048-row matrix is left over on 256 workgroups.  A
+// column of the vector is a plane of one half.
+//
+// Per token in us, kernel sequence / this, kakirax_1b (width 2048, feed-forward 8192, three layers of linear attention to one of grouped): 20 rows 849 / 705, 902 855 / 718, 2400 859 / 735,
+// 6000 869 / 748.  What bounds it: the weights (134 MB a layer, 24 us of its 38) and the hand-overs while nothing is on its way (8 us between down's vector and the next input product's, 5 in
+// the others).  A compute unit takes about 64 KB of requests and a wave that has more to ask for stands still, so what decided the form is what stands in front of a barrier (us a token):
+//   * a head's workgroup asks for its next input product only when it has its output product (its polls would wait behind 260 KB): 760 -> 753, and its barriers come first: 753 -> 722;
+//   * down is requested behind the barrier that ends gate;up, not ahead of it: 753 -> 721;
+//   * the next layer's input product goes into LDS while the heads are at work, for which registers have no room: the same time, but no spills with half of gate;up early as well.
+// Without effect: at most 4, 8 or 12 KB of a wave under way, output product and a quarter of gate;up requested a phase earlier (720).  Spilled registers cost more than anything: a spill waits for
+// all loads (28 of them: 758 -> 840).
+constexpr uint32_t PW_WIDTH = 2048, PW_FF = 8192;
+constexpr int PW_U = 4, PW_UD = 16;          // pieces of a wave in a half: depth PW_WIDTH, PW_FF
+constexpr int PW_TI = 4, PW_TIL = 3, PW_TG = 8, PW_TGA = 4;      // tiles of a workgroup: input product (the first PW_TIL of them in LDS), gate;up (the first PW_TGA of them requested early)
+static_assert(PW_TGA % 2 == 0 && PW_TG % 2 == 0, "tiles are worked in pairs");
+constexpr uint32_t PW_SLOT = PW_TIL * PW_U * 1024;                   // LDS of a wave's pieces of an input product
+constexpr int PW_HEAD_U = 8;
+
+typedef __amdgpu_buffer_rsrc_t PwRsrc;
+__device__ __forceinline__ PwRsrc pw_rsrc(const __bf16* w, const PbMat& m) { return __builtin_amdgcn_make_buffer_rsrc((void*)w, 0, m.N * m.K * 2, 0x00020000); }
+// Tiles t0 .. t0 + T of a workgroup; rows past the matrix read as zero.
+template <int T, int U>
+__device__ __forceinline__ void pw_load(PbSet<T, U>& s, const __bf16* w, const PbMat& m, uint32_t t0, uint32_t G, uint32_t wg, uint32_t c, uint32_t lane) {
+    asm volatile("" : "+v"(lane));
+    __builtin_amdgcn_sched_barrier(0);
+    const PwRsrc rsrc = pw_rsrc(w, m);
+    const uint32_t last = m.K / 64 - 1;
+#pragma unroll
+    for (int t = 0; t < T; t++) {
+        const uint32_t at = (((t0 + t) * G + wg) * 8 + (lane & 7u)) * m.K * 2 + ((lane >> 3) & 1u) * m.K + (lane >> 4) * 16;
+#pragma unroll
+        for (int i = 0; i < U; i++) s.f[t][i] = __builtin_bit_cast(v8bf, __builtin_amdgcn_raw_buffer_load_b128(rsrc, at, min(c * m.per + min((uint32_t)i, m.per - 1), last) * 64, 0));
     }
-    stamp(5 * a.L + 1);
-    if (cx.wg != 0) return;
-    ArgPair p{-INFINITY, 0};
-    for (uint32_t w = cx.tid; w < T; w += PB_THREADS) {
-        uint32_t v[2];
-        poll_tagged<2>([&](int i) { return a.tpart + 2 * w + (uint32_t)i; }, [&](int) { return th; }, v, cx);
-        p = arg_better(p, ArgPair{__uint_as_float(v[0]), v[1]});
+    __builtin_amdgcn_sched_barrier(0);
+}
+// The first PW_TIL tiles into the wave's LDS, a lane's 16 bytes of a piece where it reads them.
+__device__ __forceinline__ void pw_load_lds(uint8_t* slot, const __bf16* w, const PbMat& m, uint32_t G, uint32_t wg, uint32_t c, uint32_t lane) {
+    asm volatile("" : "+v"(lane));
+    __builtin_amdgcn_sched_barrier(0);
+    const PwRsrc rsrc = pw_rsrc(w, m);
+    const uint32_t last = m.K / 64 - 1;
+#pragma unroll
+    for (int t = 0; t < PW_TIL; t++) {
+        const uint32_t at = ((t * G + wg) * 8 + (lane & 7u)) * m.K * 2 + ((lane >> 3) & 1u) * m.K + (lane >> 4) * 16;
+#pragma unroll
+        for (int i = 0; i < PW_U; i++)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void*)(slot + (t * PW_U + i) * 1024), 16, at, min(c * m.per + min((uint32_t)i, m.per - 1), last) * 64, 0, 0);
     }
-    p = best_of_workgroup<PB_WAVES>(p, sh_arg, cx);
-    if (sh_abort) return;
-    if (cx.tid == 0) {
-        a.state[2] = p.i;
-        a.state[1] = p.i;
-        a.state[0] = pos + 1;
-        if (!(a.penalty > 1.0f)) a.counts[a.token] += 1;          // nobody read the counters in this launch
-        stamp(5 * a.L + 2);
-        // the host may be spinning on this word instead of waiting for the stream
-        if (a.host_out) __hip_atomic_store(a.host_out, ((unsigned long long)a.host_seq << 32) | p.i, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    __builtin_amdgcn_sched_barrier(0);
+}
+template <int T, int U>
+__device__ __forceinline__ void pw_mul(const PbSet<T, U>& s, const PbMat& m, uint32_t c, const __bf16* x, const __bf16* zeros, v4f (&acc)[T]) {
+#pragma unroll
+    for (int t = 0; t < T; t++) acc[t] = (v4f){0.f, 0.f, 0.f, 0.f};
+    constexpr int B = T > 1 ? 2 : U < 8 ? U : 8;
+#pragma unroll
+    for (int i0 = 0; i0 < U; i0 += B) {
+        v8bf b[B];
+#pragma unroll
+        for (int i = 0; i < B; i++) {
+            const uint32_t k = c * m.per + i0 + i;
+            b[i] = load8((uint32_t)(i0 + i) < m.per && k < m.K / 64 ? x + 32 * k : zeros);
+        }
+#pragma unroll
+        for (int i = 0; i < B; i++)
+#pragma unroll
+            for (int t = 0; t < T; t++) acc[t] = mma16(s.f[t][i0 + i], b[i], acc[t]);
     }
+}
+
+typedef PbKakiraxLds<PB_POLL> PwAttnLds;
+
+__global__ __launch_bounds__(PB_THREADS) void decode_block_wide_kernel(PbArgs a) {
+    extern __shared__ __align__(16) uint8_t smem[];
+    __shared__ uint32_t sh_abort;
+    __shared__ ArgPair sh_arg[PB_WAVES];
+    __bf16* const vec = reinterpret_cast<__bf16*>(smem);
+    float* const red = reinterpret_cast<float*>(smem + a.off_red);                // [tile][wave][16 rows]
+    float* const stats = reinterpret_cast<float*>(smem + a.off_stats);
+    const PbLayer* layers = reinterpret_cast<const PbLayer*>(smem + a.off_layers);
+    PwAttnLds* attn = reinterpret_cast<PwAttnLds*>(smem + a.off_attn);
+    float* recs = reinterpret_cast<float*>(attn->grouped.ct);
+
+    PollCtx cx;
+    cx.tid = threadIdx.x;
+    cx.lane = threadIdx.x & 63u;
+    cx.wave = pb_sgpr(threadIdx.x >> 6);
+    cx.wg = blockIdx.x;
+    cx.G = a.G;
+    cx.spin_limit = a.spin_limit;
+    cx.sh_abort = &sh_abort;
+    cx.abort_flag = a.state + 3;
+    const bool comp = cx.wave >= PB_POLL;
+    const uint32_t c = comp ? cx.wave - PB_POLL : 0u, G = a.G;
+    if (cx.tid == 0) sh_abort = 0;
+    for (uint32_t i = cx.tid; i < sizeof(attn->grouped.q) / 4; i += PB_THREADS) reinterpret_cast<uint32_t*>(attn->grouped.q)[i] = 0;
+    __shared__ __align__(16) __bf16 sh_zeros[32];
+    if (cx.tid < 32) sh_zeros[cx.tid] = (__bf16)0.0f;
+    uint8_t* const slot = smem + a.off_in + c * PW_SLOT;
+    for (uint32_t i = cx.tid; i < a.L * (uint32_t)(sizeof(PbLayer) / 4); i += PB_THREADS) reinterpret_cast<uint32_t*>(smem + a.off_layers)[i] = ldg(reinterpret_cast<const uint32_t*>(a.layers) + i);
+    const uint32_t pos = pb_sgpr(a.state[0]);
+    __syncthreads();
+
+    auto stamp = [&](uint32_t slot) {
+        if (a.stamps && cx.wg == 0 && cx.tid == 0) a.stamps[slot] = wall_clock64();
+    };
+    // this lane's column of a vector of K elements: a half of a plane
+    auto column = [&](uint32_t K, bool planes) { return vec + (planes ? min((cx.lane >> 1) & 3u, 2u) * a.plane : 0u) + (cx.lane & 1u) * (K / 2) + 8 * (cx.lane >> 4); };
+    const __bf16* const zeros = sh_zeros + 8 * (cx.lane >> 4);
+    const PbMat mh = a.head;
+    const uint32_t T = gridDim.x, WAVES = PB_COMP * T, lwv = c * T + cx.wg, chunks = (mh.K / 32 + PW_HEAD_U - 1) / PW_HEAD_U;
+    struct Cur { uint32_t tile, chunk; };
+    auto next_of = [&](Cur u) { return u.chunk + 1 < chunks ? Cur{u.tile, u.chunk + 1} : Cur{u.tile + WAVES, 0u}; };
+    auto head_load = [&](PbSet<1, PW_HEAD_U>& w, Cur u) {
+        if (u.tile >= mh.tiles) return;
+        const uint32_t at = min(u.tile * 16 + (cx.lane & 15u), mh.N - 1) * mh.K * 2 + (cx.lane >> 4) * 16, last = mh.K / 32 - 1;
+#pragma unroll
+        for (int i = 0; i < PW_HEAD_U; i++) w.f[0][i] = pb_load8(a.head_w, at + min(u.chunk * PW_HEAD_U + i, last) * 64);
+    };
+
+    // As in the narrow form, twice: a wave's mean and squares around it, then the workgroup's.
+    constexpr int NX = PW_WIDTH / PB_POLL_THREADS;
+    auto layer_norm_fetch = [&](const uint64_t* t, uint32_t tag, const float* w, bool planes) {
+        float nw[NX], nb[NX], x[NX];
+#pragma unroll
+        for (int i = 0; i < NX; i++) {
+            const uint32_t e = min(cx.tid + i * PB_POLL_THREADS, a.W - 1);
+            nw[i] = pb_f32(w, e);
+            nb[i] = pb_f32(w, a.W + e);
+        }
+        if (!tag) {
+#pragma unroll
+            for (int i = 0; i < NX; i++) x[i] = pb_embed(a, min(cx.tid + i * PB_POLL_THREADS, a.W - 1));
+        } else {
+            uint32_t v[NX];
+            poll_tagged<NX>([&](int i) { return t + min(cx.tid + i * PB_POLL_THREADS, a.W - 1); }, [&](int) { return tag; }, v, cx);
+#pragma unroll
+            for (int i = 0; i < NX; i++) x[i] = __uint_as_float(v[i]);
+        }
+        float sum = 0.f;
+        uint32_t mine = 0;
+#pragma unroll
+        for (int i = 0; i < NX; i++) {
+            const uint32_t e0 = 64 * cx.wave + i * PB_POLL_THREADS;
+            if (e0 + cx.lane < a.Wn) sum += x[i];
+            mine += e0 < a.Wn ? min(64u, a.Wn - e0) : 0u;
+        }
+        const float n = (float)mine, mean_w = n > 0.f ? wave_sum(sum) / n : 0.f;
+        float ss = 0.f;
+#pragma unroll
+        for (int i = 0; i < NX; i++) {
+            const float d = x[i] - mean_w;
+            if (cx.tid + i * PB_POLL_THREADS < a.Wn) ss = fmaf(d, d, ss);
+        }
+        ss = wave_sum(ss);
+        if (cx.lane == 0) { stats[3 * cx.wave] = n; stats[3 * cx.wave + 1] = mean_w; stats[3 * cx.wave + 2] = ss; }
+        __syncthreads();
+        float mean = 0.f, sq = 0.f;
+#pragma unroll
+        for (uint32_t i = 0; i < PB_POLL; i++) mean = fmaf(stats[3 * i], stats[3 * i + 1], mean);
+        mean /= (float)a.Wn;
+#pragma unroll
+        for (uint32_t i = 0; i < PB_POLL; i++) { const float d = stats[3 * i + 1] - mean; sq += fmaf(stats[3 * i] * d, d, stats[3 * i + 2]); }
+        const float inv = 1.0f / sqrtf(sq / (float)a.Wn + a.eps);
+#pragma unroll
+        for (int i = 0; i < NX; i++) {
+            const uint32_t e = cx.tid + i * PB_POLL_THREADS;
+            if (e >= a.W) continue;
+            const float y = (x[i] - mean) * inv * nw[i] + nb[i];
+            if (planes) pb_put(vec, a.plane, e, y);
+            else vec[e] = (__bf16)y;
+        }
+    };
+    auto leave = [&](v4f v, uint32_t t, bool planes) {
+        const uint32_t lg = cx.lane >> 4;
+        if (planes) {
+#pragma unroll
+            for (int r = 0; r < 4; r++) v[r] = lane_xor_add<4>(lane_xor_add<2>((cx.lane & 6u) == 6u ? 0.f : v[r]));      // there is no fourth plane
+        }
+        if ((cx.lane & 15u) == lg >> 1) *reinterpret_cast<v4f*>(red + (t * PB_COMP + c) * 16 + 4 * lg) = v;
+    };
+    auto row_sum = [&](uint32_t t, uint32_t r) {
+        const float* p = red + t * PB_COMP * 16 + r;
+        float s = 0.f;
+#pragma unroll
+        for (uint32_t i = 0; i < PB_COMP; i++) s += p[16 * i] + p[16 * i + 8];
+        return s;
+    };
+    const bool on_o = cx.wg * 8 < a.W, on_g = cx.wg < a.gate_up.tiles;
+    const uint32_t grouped_roles = a.gs.kv_heads * a.splits;
+    if (!comp) {
+        const uint32_t sub = cx.lane & 7u, xrow = min(cx.wg * 8 + sub, a.W - 1);
+        const bool mine = on_o && cx.lane < 8;
+        float x = pb_embed(a, xrow);
+        auto hand_on = [&](uint32_t tag, float v) {
+            if (mine) stc64(a.th + xrow, tag, __float_as_uint(v));
+        };
+#pragma nounroll
+        for (uint32_t l = 0; l < a.L; l++) {
+            asm volatile("" : "+v"(cx.tid), "+v"(cx.lane));
+            const PbLayer& L = layers[l];
+            const uint32_t base = a.tag_base + l * PB_TAGS, kind = pb_sgpr(L.kind), x_in = l ? base - PB_TAGS + PB_T_DOWN : 0u;
+            const PbMat mi = pb_of(a.in, kind), mo = pb_of(a.o, kind);
+            stamp(5 * l);
+            PbLinear<PB_POLL> lin;
+            const bool on_n = kind == PB_FIRST && cx.wg < a.ns.heads, on_k = kind == PB_GROUPED && cx.wg < grouped_roles;
+            if (on_n) lin.load(a, L, cx.wg, pos, cx.tid, cx.lane);
+            if (cx.wg < mi.tiles) {
+                layer_norm_fetch(a.th, x_in, pb_ptr(L.norm1), true);
+                __syncthreads();
+                if (sh_abort) return;
+                __syncthreads();
+                if (cx.wave == 0) {
+                    const uint32_t t = cx.lane >> 3, row = (t * G + cx.wg) * 8 + sub, raw = kind == PB_FIRST ? a.ns.raw_row() : a.gs.raw_row();
+                    float v = row_sum(min(t, mi.T - 1), sub);
+                    const float g = kind == PB_FIRST ? silu_f(v) : sigmoid_f(v);
+                    if (row >= raw) v = (float)(__bf16)g;
+                    if (t < mi.T && row < mi.N) stc64(a.traw + row, base + PB_T_RAW, __float_as_uint(v));
+                }
+            }
+            stamp(5 * l + 1);
+            if (on_n) {
+                if (!pb_linear_layer(a, L, lin, &attn->linear, cx.wg, l, pos, cx)) return;
+            } else if (on_k) {
+                if (!pb_grouped_layer<PB_POLL>(a, L, &attn->grouped, recs, cx.wg, l, pos, cx)) return;
+            }
+            // ---- output product
+            if (on_o) {
+                uint32_t* plane = reinterpret_cast<uint32_t*>(vec);
+                if (kind == PB_GROUPED) pb_fetch_pairs<NX / 2>(a.tout, base + PB_T_OUT, a.gs.heads * a.gs.vdim / 2, mo.K / 2, plane, cx);
+                else pb_fetch_floats<NX>(a.tout, base + PB_T_OUT, a.ns.heads * a.ns.vdim, mo.K, vec, a.plane, cx);
+                __syncthreads();
+                if (sh_abort) return;
+                __syncthreads();
+                if (cx.wave == 0) {
+                    x += row_sum(0, sub);
+                    hand_on(base + PB_T_O, x);
+                }
+            }
+            stamp(5 * l + 3);
+            // ---- gate;up
+            if (on_g) {
+                layer_norm_fetch(a.th, base + PB_T_O, pb_ptr(L.norm2), true);
+                __syncthreads();
+                if (sh_abort) return;
+                __syncthreads();
+                if (cx.wave == 0) {
+                    // rows 2 i and 2 i + 1 are gate and up of element i; four rows to a pair
+                    const uint32_t t = cx.lane >> 3, row = (t * G + cx.wg) * 8 + sub;
+                    const float v = row_sum(min(t, a.gate_up.T - 1), sub), up = lane_xor<1>(v);
+                    const float y = act_f((Act)a.act, v) * up, y1 = lane_xor<2>(y);
+                    if (t < a.gate_up.T && !(cx.lane & 3u) && row < a.gate_up.N) stc64(a.tact + row / 4, base + PB_T_ACT, pb_pack(y, y1));
+                }
+            }
+            stamp(5 * l + 4);
+            // ---- down
+            if (on_o) {
+                constexpr int N = PW_FF / 2 / PB_POLL_THREADS;
+                pb_fetch_pairs<N>(a.tact, base + PB_T_ACT, a.ff / 2, a.ff / 2, reinterpret_cast<uint32_t*>(vec), cx);
+                __syncthreads();
+                if (sh_abort) return;
+                __syncthreads();
+                if (cx.wave == 0) {
+                    x += row_sum(0, sub);
+                    hand_on(base + PB_T_DOWN, x);
+                }
+            }
+        }
+    } else {
+        PbSet<PW_TI - PW_TIL, PW_U> wi;      // the input product's tiles behind those in LDS
+        pw_load_lds(slot, pb_ptr(layers[0].in), pb_of(a.in, pb_sgpr(layers[0].kind)), G, cx.wg, c, cx.lane);
+        pw_load(wi, pb_ptr(layers[0].in), pb_of(a.in, pb_sgpr(layers[0].kind)), PW_TIL, G, cx.wg, c, cx.lane);
+#pragma nounroll
+        for (uint32_t l = 0; l < a.L; l++) {
+            asm volatile("" : "+v"(cx.tid), "+v"(cx.lane));
+            const PbLayer& L = layers[l];
+            const uint32_t kind = pb_sgpr(L.kind);
+            const PbMat mi = pb_of(a.in, kind), mo = pb_of(a.o, kind);
+            if (cx.wg < mi.tiles) {
+                __syncthreads();
+                __syncthreads();
+                if (sh_abort) return;
+                v4f acc[PW_TI - PW_TIL];
+                pw_mul(wi, mi, c, column(a.W, true), zeros, acc);
+#pragma unroll
+                for (int t = 0; t < PW_TI - PW_TIL; t++) leave(acc[t], PW_TIL + t, true);
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                PbSet<PW_TIL, PW_U> wl;
+#pragma unroll
+                for (int t = 0; t < PW_TIL; t++)
+#pragma unroll
+                    for (int i = 0; i < PW_U; i++) wl.f[t][i] = *reinterpret_cast<const v8bf*>(slot + (t * PW_U + i) * 1024 + cx.lane * 16);
+                v4f acl[PW_TIL];
+                pw_mul(wl, mi, c, column(a.W, true), zeros, acl);
+#pragma unroll
+                for (int t = 0; t < PW_TIL; t++) leave(acl[t], t, true);
+                __syncthreads();
+            }
+            // A head's workgroup: the barriers of what its polling waves do.
+            const uint32_t joins = kind == PB_FIRST ? (cx.wg < a.ns.heads ? 3u : 0u) : cx.wg < grouped_roles ? (a.splits > 1 && cx.wg % a.splits == 0 ? 4u : 3u) : 0u;
+            const PbLayer& N = layers[min(l + 1, a.L - 1)];
+            PbSet<1, PW_U> wo;
+            PbSet<PW_TGA, PW_U> wga;
+            pw_load(wo, pb_ptr(L.o), mo, 0, G, cx.wg, c, cx.lane);
+            pw_load(wga, pb_ptr(L.gate_up), a.gate_up, 0, G, cx.wg, c, cx.lane);
+            for (uint32_t j = 0; j < joins; j++) {
+                __syncthreads();
+                if (sh_abort) return;
+            }
+            if (!joins) pw_load_lds(slot, pb_ptr(N.in), pb_of(a.in, pb_sgpr(N.kind)), G, cx.wg, c, cx.lane);
+            if (on_o) {
+                __syncthreads();
+                if (sh_abort) return;
+                const bool planes = kind == PB_FIRST;
+                v4f acc[1];
+                pw_mul(wo, mo, c, column(mo.K, planes), zeros, acc);
+                leave(acc[0], 0, planes);
+                __syncthreads();
+            }
+            PbSet<PW_TG - PW_TGA, PW_U> wgb;
+            if (joins) pw_load_lds(slot, pb_ptr(N.in), pb_of(a.in, pb_sgpr(N.kind)), G, cx.wg, c, cx.lane);
+            pw_load(wgb, pb_ptr(L.gate_up), a.gate_up, PW_TGA, G, cx.wg, c, cx.lane);
+            if (on_g) {
+                __syncthreads();
+                __syncthreads();
+                if (sh_abort) return;
+                const __bf16* xc = column(a.W, true);
+                auto some = [&](const auto& w, auto n, int t0) {
+#pragma unroll
+                    for (int t = 0; t < n.value; t += 2) {
+                        PbSet<2, PW_U> two;
+#pragma unroll
+                        for (int i = 0; i < PW_U; i++) { two.f[0][i] = w.f[t][i]; two.f[1][i] = w.f[t + 1][i]; }
+                        v4f acc[2];
+                        pw_mul(two, a.gate_up, c, xc, zeros, acc);
+                        leave(acc[0], t0 + t, true);
+                        leave(acc[1], t0 + t + 1, true);
+                    }
+                };
+                some(wga, std::integral_constant<int, PW_TGA>{}, 0);
+                some(wgb, std::integral_constant<int, PW_TG - PW_TGA>{}, PW_TGA);
+            }
+            if (on_g) __syncthreads();
+            PbSet<1, PW_UD> wd;
+            pw_load(wd, pb_ptr(L.down), a.down, 0, G, cx.wg, c, cx.lane);
+            if (on_o) {
+                __syncthreads();
+                if (sh_abort) return;
+            }
+            pw_load(wi, pb_ptr(N.in), pb_of(a.in, pb_sgpr(N.kind)), PW_TIL, G, cx.wg, c, cx.lane);
+            if (on_o) {
+                v4f acc[1];
+                pw_mul(wd, a.down, c, column(a.ff, false), zeros, acc);
+                leave(acc[0], 0, false);
+                __syncthreads();
+            }
+        }
+    }
+
+    // ---- final norm | output matrix | argmax
+    asm volatile("" : "+v"(cx.tid), "+v"(cx.lane));
+    stamp(5 * a.L);
+    ArgPair best{-INFINITY, 0};
+    if (!comp) {
+        layer_norm_fetch(a.th, a.tag_base + (a.L - 1) * PB_TAGS + PB_T_DOWN, a.final_norm, false);
+        __syncthreads();
+        if (sh_abort) return;
+    } else {
+        PbSet<1, PW_HEAD_U> wh[2];
+        const Cur u0{lwv, 0}, u1 = next_of(u0);
+        head_load(wh[0], u0);
+        head_load(wh[1], u1);
+        __syncthreads();
+        __syncthreads();
+        if (sh_abort) return;
+        const __bf16* const x1 = vec + 8 * (cx.lane >> 4);
+        v4f acc = (v4f){0.f, 0.f, 0.f, 0.f};
+        auto work = [&](const PbSet<1, PW_HEAD_U>& w, Cur u) {
+#pragma unroll
+            for (int i = 0; i < PW_HEAD_U; i++) {
+                const uint32_t k = u.chunk * PW_HEAD_U + i;
+                acc = mma16(w.f[0][i], load8(k < mh.K / 32 ? x1 + 32 * k : zeros), acc);
+            }
+            if (u.chunk + 1 < chunks) return;
+            pb_logits(a, u.tile, acc, cx.lane, best);
+            acc = (v4f){0.f, 0.f, 0.f, 0.f};
+        };
+        for (Cur u = u0, v = u1; u.tile < mh.tiles;) {
+            work(wh[0], u);
+            u = next_of(v);
+            head_load(wh[0], u);
+            if (v.tile >= mh.tiles) break;
+            work(wh[1], v);
+            v = next_of(u);
+            head_load(wh[1], v);
+        }
+    }
+    pb_choose(a, best, sh_arg, pos, cx);
 }
 
 // uk [head][dim][rank] -> [head][rank][dim]
@@ -1223,7 +1653,7 @@ struct PbState {
     std::vector<void*> owned;
     const void* kernel = nullptr;
     uint32_t grid = 0, lds = 0, n_stamps = 0, heads = 0, window = 0;
-    bool cooperative = false;
+    bool cooperative = false, wide = false;
     uint64_t* tagged = nullptr;
     size_t tagged_bytes = 0;
     std::vector<unsigned long long> stamps_host;
@@ -1255,7 +1685,7 @@ int32_t pb_create(const PbModelIn& in, PbState** out) {
     *out = nullptr;
     const std::vector<PbLayerIn>& layers = in.layers;
     const bool latent = in.elementwise;
-    if (layers.empty() || in.width > PB_WIDTH) return FORGE_HIP_OK;
+    if (layers.empty() || in.width > (latent ? PB_WIDTH : PW_WIDTH)) return FORGE_HIP_OK;
     const PbLayerIn* of[2] = {nullptr, nullptr};                     // the first layer of each kind
     for (const PbLayerIn& l : layers) {
         const PbMixer& m = *l.mixer;
@@ -1294,38 +1724,49 @@ int32_t pb_create(const PbModelIn& in, PbState** out) {
         if (l) need(l->mixer->in.N, PB_TI);
     need(layers[0].gate_up.N, PB_TG);
     need(a.W, 1);
+    // ... or, what registers do not hold, all workgroups
+    bool& wide = st->wide;
+    wide = !latent && (a.W > PB_WIDTH || a.ff > PB_FF || g + std::max({gs.kv_heads, ns.heads, 1u}) > (uint32_t)cus);
+    if (wide) g = (uint32_t)cus;
     a.G = g;
     st->heads = latent ? ls.heads : gs.kv_heads;
-    if (g + std::max({st->heads, ns.heads, 1u}) > (uint32_t)cus) return FORGE_HIP_OK;
-    a.splits_max = st->heads ? std::min(PB_SPLITS, ((uint32_t)cus - g) / st->heads) : 1u;
+    if ((wide ? 0u : g) + std::max({st->heads, ns.heads, 1u}) > (uint32_t)cus) return FORGE_HIP_OK;
+    if (wide && ns.dim * ns.vdim > (uint32_t)PbLinear<PB_POLL>::STATE * 4 * PB_POLL_THREADS) return FORGE_HIP_OK;
+    a.splits_max = st->heads ? std::min(PB_SPLITS, ((uint32_t)cus - (wide ? 0u : g)) / st->heads) : 1u;
     bool fits = true;
     auto mat = [&](const DenseWeight& w, uint32_t tiles_each, uint32_t pieces) {
-        PbMat m{w.N, w.K, (w.N + 15) / 16, 1, (w.K / 32 + PB_COMP - 1) / PB_COMP};
+        const uint32_t rows = wide ? 8 : 16, depth = wide ? 64 : 32;      // of a tile, of a piece (wide: of both halves)
+        PbMat m{w.N, w.K, (w.N + rows - 1) / rows, 1, (w.K / depth + PB_COMP - 1) / PB_COMP};
         m.T = (m.tiles + g - 1) / g;
-        fits = fits && m.T <= tiles_each && m.per <= pieces && w.K % 32 == 0 && w.N % 4 == 0;
+        fits = fits && m.T <= tiles_each && m.per <= pieces && w.K % depth == 0 && w.N % (wide ? 8 : 4) == 0 && (uint64_t)w.N * w.K * 2 <= 0x7FFFFFFFull;
         return m;
     };
     for (int k = 0; k < 2; k++)
-        if (of[k]) { a.in[k] = mat(of[k]->mixer->in, PB_TI, PB_UI); a.o[k] = mat(of[k]->mixer->o, 1, PB_UO); }
-    a.gate_up = mat(layers[0].gate_up, PB_TG, PB_UI);
-    a.down = mat(layers[0].down, 1, PB_UD);
+        if (of[k]) { a.in[k] = mat(of[k]->mixer->in, wide ? PW_TI : PB_TI, wide ? PW_U : PB_UI); a.o[k] = mat(of[k]->mixer->o, 1, wide ? PW_U : PB_UO); }
+    a.gate_up = mat(layers[0].gate_up, wide ? PW_TG : PB_TG, wide ? PW_U : PB_UI);
+    a.down = mat(layers[0].down, 1, wide ? PW_UD : PB_UD);
     if (in.loop.p) a.loop = mat(in.loop, 1, PB_UL);
     a.head = PbMat{in.head.N, in.head.K, (in.head.N + 15) / 16, 1, 1};
     if (!fits || a.in[0].N % 16 || a.in[1].N % 16 || a.gate_up.N % 16) return FORGE_HIP_OK;
 
     auto up = [](size_t v, size_t m) { return (uint32_t)((v + m - 1) / m * m); };
     a.plane = up(std::max({in.loop.p ? 2 * a.W : a.W, a.ff, a.o[0].K, a.o[1].K}), 32);
-    a.off_red = a.plane * 8;
-    a.off_stats = a.off_red + std::max(PB_TI, PB_TG) * PB_COMP * 16 * 4;
+    // Planes a quarter of the banks apart (us a token, 135M linear and grouped: 413 -> 410).  Wide: three of the longest vector that comes in planes; longer ones lie over them.
+    const uint32_t longest = a.plane;
+    a.plane = up(wide ? std::max({a.W, a.o[0].K, a.o[1].K}) : a.plane, 128) + 32;
+    a.off_red = wide ? up(std::max(a.plane * 6, longest * 2), 16) : a.plane * 8;
+    a.off_stats = a.off_red + (wide ? PW_TG : std::max(PB_TI, PB_TG)) * PB_COMP * 16 * 4;
     a.off_layers = a.off_stats + PB_POLL * 3 * 4;
     a.off_attn = up(a.off_layers + layers.size() * sizeof(PbLayer), 16);
-    const size_t attn = latent ? sizeof(PbLatentLds) : sizeof(PbKakiraxLds), recs = latent ? sizeof(PbLatentLds::ct) : sizeof(PbGroupedLds::ct);
-    st->lds = a.off_attn + (uint32_t)attn;
+    const size_t attn = latent ? sizeof(PbLatentLds) : wide ? sizeof(PwAttnLds) : sizeof(PbKakiraxLds<PB_WAVES>),
+                 recs = latent ? sizeof(PbLatentLds::ct) : wide ? sizeof(PbGroupedLds<PB_POLL>::ct) : sizeof(PbGroupedLds<PB_WAVES>::ct);
+    a.off_in = up(a.off_attn + attn, 1024);
+    st->lds = wide ? a.off_in + PB_COMP * PW_SLOT : a.off_attn + (uint32_t)attn;
     const uint32_t rec = latent ? ls.rank + 2 : gs.heads ? gs.group() * (gs.vdim + 2) : 0u;
     if (rec) a.splits_max = std::min<uint32_t>(a.splits_max, (uint32_t)(recs / 4 / rec) + 1);
     if (st->lds > PB_LDS) return FORGE_HIP_OK;
     st->window = ls.window;
-    st->kernel = latent ? reinterpret_cast<const void*>(decode_block_kernel<true>) : reinterpret_cast<const void*>(decode_block_kernel<false>);
+    st->kernel = wide ? reinterpret_cast<const void*>(decode_block_wide_kernel) : latent ? reinterpret_cast<const void*>(decode_block_kernel<true>) : reinterpret_cast<const void*>(decode_block_kernel<false>);
     FH_HIP(hipFuncSetAttribute(st->kernel, hipFuncAttributeMaxDynamicSharedMemorySize, PB_LDS));
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, st->kernel, PB_THREADS, st->lds) != hipSuccess || per_cu < 1) { (void)hipGetLastError(); return FORGE_HIP_OK; }
     st->grid = (uint32_t)cus;
@@ -1420,7 +1861,7 @@ int32_t pb_enqueue(PbState* st, int64_t pos, bool profile, uint32_t token, uint3
     // Up to 384 keys one workgroup, which saves the hand-over of parts; from there on four waves a workgroup attend, one to a SIMD, as long as there are workgroups for the keys (1024 keys,
     // us a token: 453 with twelve waves in three parts, 419 with four in eight); then eight, then all, and rounds of those.
     const uint64_t parts = keys <= PB_WAVES * PB_KEYS ? 1 : a.splits_max;
-    for (a.attend = 4; a.attend < PB_WAVES && parts * a.attend * PB_KEYS < keys; a.attend += 4) {}
+    for (a.attend = 4; !st->wide && a.attend < PB_WAVES && parts * a.attend * PB_KEYS < keys; a.attend += 4) {}
     a.splits = (uint32_t)std::min<uint64_t>(a.splits_max, (keys + a.attend * PB_KEYS - 1) / (a.attend * PB_KEYS));
     if (a.tag_base > 0xF0000000u) {      // tags are about to wrap: start again from zeroed buffers
         FH_HIP(hipMemsetAsync(st->tagged, 0, st->tagged_bytes, s));

@@ -21,6 +21,10 @@ def configs(fh):
         "mixed_largest": ("kakirax_oracle", kak(768, 70, [gla(6, 64, 128, 1536), att(12, 3, 64, 64, 1536), 0], embedding_scale=20.0)),
         "mixed_ragged": ("kakirax_oracle", kak(90, 203, [gla(5, 20, 60, 77, tau=3.0), att(6, 2, 20, 44, 77, rot_dims=12), 0, 1], embedding_scale=9.5, eps=3e-3, cap=7.0)),
         "grouped_many_heads": ("kakirax_oracle", kak(64, 80, [att(24, 24, 32, 32, 51)] * 2, embedding_scale=8.0)),
+        # layers that registers do not hold: the wide form
+        "wide_largest": ("kakirax_oracle", kak(2048, 70, [gla(16, 64, 128, 8192), att(32, 8, 64, 64, 8192)], embedding_scale=45.0)),
+        "wide_ragged": ("kakirax_oracle", kak(1000, 203, [gla(5, 20, 60, 2077, tau=3.0), att(6, 2, 20, 44, 2077, rot_dims=12), 0, 1], embedding_scale=9.5, eps=3e-3, cap=7.0)),
+        "wide_deep": ("kakirax_oracle", kak(90, 80, [att(24, 24, 32, 32, 1601), gla(48, 16, 32, 1601), 0], embedding_scale=8.0)),
         "linear_only": ("kakirax_oracle", kak(70, 61, [gla(3, 16, 32, 40), 0], embedding_scale=8.0)),
     }
 
@@ -41,7 +45,7 @@ def get(fh, torch_gpu, tmp_path_factory):
     return case
 
 
-@pytest.mark.parametrize("name", ["latent_largest", "latent_ragged", "latent_many_heads", "mixed_largest", "mixed_ragged", "grouped_many_heads", "linear_only"])
+@pytest.mark.parametrize("name", ["latent_largest", "latent_ragged", "latent_many_heads", "mixed_largest", "mixed_ragged", "grouped_many_heads", "linear_only", "wide_largest", "wide_ragged", "wide_deep"])
 def test_against_the_oracle(get, name):
     """Token by token over the first tiles of keys, the window's edge and the change from one workgroup a head to parts (384 keys)."""
     c = get(name)
@@ -59,9 +63,9 @@ def test_against_the_oracle(get, name):
     m.close()
 
 
-@pytest.mark.parametrize("name", ["latent_many_heads", "grouped_many_heads"])
+@pytest.mark.parametrize("name", ["latent_many_heads", "grouped_many_heads", "wide_deep"])
 def test_contexts_of_several_rounds(get, name, monkeypatch):
-    """24 heads leave each eight or nine workgroups of twelve waves of 32 keys: four waves, eight, twelve, and a second round."""
+    """24 heads leave each eight or nine workgroups of twelve waves of 32 keys: four waves, eight, twelve, and a second round.  The wide form: ten of four waves, up to three rounds."""
     c = get(name)
     ids = c.ids(3700, seed=4)
     m = c.model(max_seq=3700, dtype="bfloat16")
@@ -83,7 +87,7 @@ def bits(x):
     return x.view(np.uint32)
 
 
-@pytest.mark.parametrize("name", ["latent_ragged", "mixed_ragged"])
+@pytest.mark.parametrize("name", ["latent_ragged", "mixed_ragged", "wide_ragged"])
 def test_a_step_that_is_given_up(get, fh, name, monkeypatch):
     """With a poll limit of 1 a step that gives up has not happened, states of linear layers included; with the library's own limit it runs as the kernel sequence.  Tags wrap."""
     c = get(name)
@@ -129,7 +133,7 @@ def test_a_step_that_is_given_up(get, fh, name, monkeypatch):
         x.close()
 
 
-@pytest.mark.parametrize("name", ["latent_ragged", "mixed_ragged"])
+@pytest.mark.parametrize("name", ["latent_ragged", "mixed_ragged", "wide_ragged"])
 def test_greedy_with_a_repeat_penalty(get, fh, name):
     """The token that a greedy step returns is the last maximum of the penalised logits of the same step."""
     c = get(name)
