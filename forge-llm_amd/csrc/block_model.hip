@@ -71,6 +71,7 @@ struct BlockModel : forge_hip_model {
     uint32_t table_ld = 0;
     DevBuf b_embed, b_loop, b_head, b_final, b_cache;
     DevBuf x, h, xcat, act, rows_sel, h_sel; // of one prompt chunk
+    DevBuf sums, arrivals;                   // of a residual product in ranges of its depth
     BlockScratch scratch;
     PbState* pb = nullptr;                   // the decode step as one resident kernel, when the model is covered
     std::unique_ptr<ResidentSeat> seat;      // of a model that has it
@@ -214,6 +215,8 @@ void BlockModel::enqueue_run(size_t i, uint32_t M, uint32_t base_pos, const uint
         e.next = nx.norm;
         e.out = nx.out;
         e.ld_out = nx.ld;
+        e.sums = sums.as<uint64_t>();
+        e.arrivals = arrivals.as<uint32_t>();
         launch_dense(t, w, in, M, DenseEpi::Residual, e, stream);
     };
     if (r.pass_start) residual(loop_in, dense_rows(xcat.p, 2 * width), DynTanh{}, false, Next{L.norm1.tanh, h.p, width}, ST_QKV);
@@ -296,6 +299,10 @@ int32_t BlockModel::alloc_scratch() {
         (rc = rows_sel.alloc(HEAD_ROWS * 4)) || (rc = h_sel.alloc(HEAD_ROWS * width * es)) || (rc = scratch.alloc()))
         return rc;
     if (loop_in.p && (rc = xcat.alloc(R * 2 * width * es))) return rc;
+    if (t == DType::BF16) {
+        if ((rc = sums.alloc(dense_sums_bytes())) || (rc = arrivals.alloc(dense_arrivals_bytes()))) return rc;
+        FH_HIP(hipMemset(arrivals.p, 0, dense_arrivals_bytes()));
+    }
     return FORGE_HIP_OK;
 }
 

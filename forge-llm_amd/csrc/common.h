@@ -325,6 +325,10 @@ struct DenseEpiArgs {
     uint32_t base_pos = 0;
     const uint32_t* pos_dev = nullptr;
     uint32_t head_stride = 1, rot_off = 0, rot_pairs = 0;
+    // Residual: memory in which ranges of the depth meet (dense_sums_bytes()), and a counter a tile, zero between launches; null: products stay whole.
+    uint64_t* sums = nullptr;
+    uint32_t* arrivals = nullptr;
+    uint32_t parts = 1;              // set by the launch
 };
 // What a product multiplies: stored rows, or (one row only) something its kernel makes from 32-bit values on the way in.
 struct DenseIn {
@@ -346,6 +350,7 @@ inline DenseIn dense_rows(const void* rows, uint32_t lda) { DenseIn in; in.rows 
 // y = a W^T over M rows, then the epilogue.  One row runs as a matrix-vector kernel.
 void launch_dense(DType t, const DenseWeight& w, const DenseIn& in, uint32_t M, DenseEpi mode, const DenseEpiArgs& e, hipStream_t s);
 uint32_t dense_k_max();
+size_t dense_sums_bytes(), dense_arrivals_bytes();
 // out[m] = layer norm of x[m]; rows of `width` elements (a multiple of 64, at most 16384), those past ln.n come out zero
 void launch_layer_norm(DType t, const float* x, uint32_t ldx, const LayerNorm& ln, uint32_t width, uint32_t M, void* out, uint32_t ld_out, hipStream_t s);
 // x[m] = table[token[m]] * scale (f32, rows of ldx, zero past `width`), out (optional) = next(x), out2 (optional) = x; the table's rows

@@ -15,9 +15,13 @@
 // - The latency of a stage's loads where a compute unit has one workgroup: 3 or 4 buffers, and the depth shared out to the waves.
 // Times in us of a caller's loop, 32-bit results, before / now: 16384 x 2048 by 902 rows 110 / 66.5 (910 TFLOP/s), 2048 x 8192 by 902
 // 67.9 / 47.1, 2048 x 2048 by 902 22.9 / 15.3, 6144 x 2048 by 902 48.4 / 32.2, 3072 x 576 by 2502 29.5 / 17.7, 576 x 576 by 2502 9.3 / 7.2.
+// - The chain of a tile where there are few: launch, first loads, stages, epilogue one behind the other while most compute units have nothing.
+//   Tiles of 32 x 32 to 64 x 32 whose waves share out the depth give every unit a part, and a residual product of 4096 or more columns is cut along its depth
+//   over workgroups (`parts`), whose 32-bit sums meet in memory: the one that arrives last adds them up in the order of the ranges.
 // M = 1: dense_gemv.h.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "common.h"
@@ -44,6 +48,7 @@ void dense_gemm_kernel(const T* __restrict__ w, const T* __restrict__ a, uint32_
     extern __shared__ __attribute__((aligned(16))) uint8_t dense_lds[];
     constexpr uint32_t WAVES = WN * WM * KG, BN = 32 * TN * WN, BM = 32 * TM * WM, BK = ROW_BYTES / sizeof(T), ES = sizeof(T), LR = 8 * WAVES;
     constexpr uint32_t BUF = (BN + BM) * ROW_BYTES;
+    static_assert(BN % LR == 0 && BM % LR == 0, "every wave has a part of each load");
     const uint32_t tid = threadIdx.x, lane = tid & 63;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
     const uint32_t wn = wave % WN, wm = wave / WN % WM, kg = wave / (WN * WM), lrow = lane & 31, lh = lane >> 5;
@@ -53,6 +58,15 @@ void dense_gemm_kernel(const T* __restrict__ w, const T* __restrict__ a, uint32_
         const uint32_t total = gridDim.x, per = total / 8, x = tile % 8, i = tile / 8;
         if (i < per) tile = x * per + i;          // the last total % 8 tiles stay where they are
     }
+    // All tiles of one range of the depth ahead of those of the next: an XCD reads the columns of one or two ranges.
+    uint32_t part = 0, st0 = 0, stages = K / BK;
+    if (MODE == DenseEpi::Residual && e.parts > 1) {
+        const uint32_t tiles = gridDim.x / e.parts, all = stages;
+        part = tile / tiles;
+        tile -= part * tiles;
+        st0 = part * all / e.parts;
+        stages = (part + 1) * all / e.parts - st0;
+    }
     // Tiles are counted in groups of GROUP rows of tiles, down the column first: the tiles that run at a time share both operands.  512 rows
     // of activations to a group, which an XCD's L2 holds beside the weights (products with a gate, bfloat16, us by 1 / 2 / 4 / 8 rows of tiles:
     // 128 x 128 tiles 3392 x 2048 by 2502 rows 69.0 / 71.8 / 68.0 / 73.9, 6144 x 2048 by 1500 69.7 / 63.5 / 62.7 / 68.2; 128 x 64 tiles
@@ -61,7 +75,6 @@ void dense_gemm_kernel(const T* __restrict__ w, const T* __restrict__ a, uint32_
     // (One group is one division less ahead of the first loads: 32-bit [gate; up] 3072 x 576 by 65 rows 19.97 us with it, 19.58 without.)
     const uint32_t tiles_m = (M + BM - 1) / BM, first = tiles_m <= GROUP ? 0u : tile / (GROUP * tiles_n) * GROUP, rows = min(GROUP, tiles_m - first), in = tile - first * tiles_n;
     const uint32_t n0 = in / rows * BN, m0 = (first + in % rows) * BM;
-    const uint32_t stages = K / BK;
 
     const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void*)(w + (size_t)n0 * K), 0, min(N - n0, BN) * K * ES, DENSE_RSRC_FLAGS);
     const __amdgpu_buffer_rsrc_t ra =
@@ -73,7 +86,7 @@ void dense_gemm_kernel(const T* __restrict__ w, const T* __restrict__ a, uint32_
     constexpr uint32_t LOADS = (BN + BM) / LR;
     auto issue = [&](uint32_t stage, uint32_t buf) {
         uint8_t* base = dense_lds + buf * BUF + wave * 1024;
-        const uint32_t k = stage * ROW_BYTES;
+        const uint32_t k = (st0 + stage) * ROW_BYTES;
 #pragma unroll
         for (uint32_t i = 0; i < BN / LR; i++)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, FH_LDS3(base + i * LR * ROW_BYTES), 16, w_off + i * LR * K * ES, k, 0, 0);
@@ -160,6 +173,69 @@ void dense_gemm_kernel(const T* __restrict__ w, const T* __restrict__ a, uint32_
                     box[(kg * ROWS + r) * PIECES + (at ^ (r & 7))] = (v4f){c[4 * g], c[4 * g + 1], c[4 * g + 2], c[4 * g + 3]};
                 }
         __syncthreads();
+        if constexpr (MODE == DenseEpi::Residual && JP == TM)
+            if (e.parts > 1) {
+                // Stores and loads past the caches of an XCD, 8 bytes a lane in two planes.  A wave's stores have arrived before the barrier that lets the
+                // workgroup count itself in; who counts `parts` sees them all, and leaves the counter at zero for the next launch.
+                constexpr uint32_t PLANE = ROWS * PIECES;
+                uint64_t* mine = e.sums + (size_t)(tile * e.parts + part) * (2 * PLANE);
+#pragma unroll
+                for (uint32_t s = 0; s < STEPS; s++) {
+                    const uint32_t r = s * STEP + tid / PIECES, at = r * PIECES + piece;
+                    if (n >= N || m0 + r >= M) continue;
+                    v4f v = box[r * PIECES + (piece ^ (r & 7))];
+#pragma unroll
+                    for (int k = 1; k < KG; k++) v += box[(k * ROWS + r) * PIECES + (piece ^ (r & 7))];
+                    uint64_t h[2];
+                    __builtin_memcpy(h, &v, 16);
+                    __hip_atomic_store(mine + at, h[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    __hip_atomic_store(mine + PLANE + at, h[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                __shared__ uint32_t arrived;
+                __syncthreads();
+                if (tid == 0) {
+                    arrived = __hip_atomic_fetch_add(e.arrivals + tile, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1;
+                    if (arrived == e.parts) __hip_atomic_store(e.arrivals + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+                __syncthreads();
+                if (arrived != e.parts || n >= N) return;
+                const uint64_t* from = e.sums + (size_t)tile * e.parts * (2 * PLANE);
+#pragma unroll
+                for (uint32_t s0 = 0; s0 < STEPS; s0 += G) {
+                    EpiRow<T, MODE> row[G];
+                    v4f v[G];
+#pragma unroll
+                    for (uint32_t s = 0; s < G; s++) {
+                        const uint32_t m = m0 + (s0 + s) * STEP + tid / PIECES;
+                        v[s] = (v4f){0.f, 0.f, 0.f, 0.f};
+                        if (m < M) row[s] = epilogue_row<T, MODE>(e, m, n);
+                    }
+                    for (uint32_t q = 0; q < e.parts; q++) {
+                        uint64_t h[G][2];
+#pragma unroll
+                        for (uint32_t s = 0; s < G; s++) {
+                            const uint32_t r = min((s0 + s) * STEP + tid / PIECES, M - 1 - m0);      // rows past the end: what another lane adds up
+                            const uint64_t* at = from + (size_t)q * (2 * PLANE) + r * PIECES + piece;
+                            h[s][0] = __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                            h[s][1] = __hip_atomic_load(at + PLANE, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        }
+#pragma unroll
+                        for (uint32_t s = 0; s < G; s++) {
+                            v4f x;
+                            __builtin_memcpy(&x, h[s], 16);
+                            v[s] += x;
+                        }
+                    }
+#pragma unroll
+                    for (uint32_t s = 0; s < G; s++) {
+                        const uint32_t m = m0 + (s0 + s) * STEP + tid / PIECES;
+                        const float f[4] = {v[s][0], v[s][1], v[s][2], v[s][3]};
+                        if (m < M) dense_epilogue<T, MODE>(e, m, n, N, f, cols, row[s]);
+                    }
+                }
+                return;
+            }
         if (n >= N) continue;
 #pragma unroll
         for (uint32_t s0 = 0; s0 < STEPS; s0 += G) {
@@ -375,14 +451,16 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(const T* __restrict__ 
 namespace {
 
 template <typename T, int WN, int WM, int KG, int TN, int TM, int NBUF, DenseEpi MODE>
-void go_gemm(const DenseWeight& w, const void* a, uint32_t lda, uint32_t M, const DenseEpiArgs& e, hipStream_t s) {
+void go_gemm(const DenseWeight& w, const void* a, uint32_t lda, uint32_t M, const DenseEpiArgs& e, hipStream_t s, uint32_t parts = 1) {
     constexpr uint32_t BN = 32 * TN * WN, BM = 32 * TM * WM, stage = (BN + BM) * ROW_BYTES * NBUF, box = dense_box(WN, WM, KG, TN, dense_pass(WN, WM, KG, TN, TM)),
                        lds = stage > box ? stage : box;
     const auto kernel = dense_gemm_kernel<T, WN, WM, KG, TN, TM, NBUF, MODE>;
     static const hipError_t lds_ok = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     (void)lds_ok;
     const uint32_t tn = (w.N + BN - 1) / BN, tm = (M + BM - 1) / BM;
-    fh::launch(kernel, dim3(tn * tm), 64 * WN * WM * KG, lds, s, (const T*)w.p, (const T*)a, lda, M, w.N, w.K, tn, e);
+    DenseEpiArgs args = e;
+    args.parts = parts;
+    fh::launch(kernel, dim3(tn * tm * parts), 64 * WN * WM * KG, lds, s, (const T*)w.p, (const T*)a, lda, M, w.N, w.K, tn, args);
 }
 
 template <typename T, int KS, DenseEpi MODE, DenseIn::Kind IN, int STEPS>
@@ -422,6 +500,28 @@ void go(const DenseWeight& w, const DenseIn& in, uint32_t M, const DenseEpiArgs&
     auto tiles = [&](uint32_t bn, uint32_t bm) { return (uint64_t)((w.N + bn - 1) / bn) * ((M + bm - 1) / bm); };
     constexpr uint64_t CUS = 256;
     if constexpr (sizeof(T) == 2) {
+        // Up to a few tiles of 32 rows a compute unit: the smallest tiles, four waves to the depth of each (us, by the rules below / 32 x 32 / 64 x 32, columns
+        // first; o, down: residual products with two norms): gate 928 x 576 by 65 rows 6.5 / 3.8 / 4.8, by 300 6.5 / 4.2 / 5.0, by 902 (841 and 435 tiles)
+        // 8.3 / 6.1 / 6.2, o 576 x 576 by 300 9.1 / 5.0 / 6.7, by 902 (522) 10.9 / 6.9 / 8.1, down 576 x 1536 by 902 13.3 / 10.9 / 12.7, up 3072 x 576 by 300
+        // (960 and 480) 7.8 / 6.3 / 5.8, gate 6272 x 2048 by 130 (980 and 490) 17.7 / 14.6 / 11.7.  Past that the operands' traffic counts: up 16384 x 2048 by 33
+        // (1024 and 512) 17.9 / 20.2 / 19.4, 2048 x 2048 by 902 rows (1856 and 928) 16.3 / 25.3 / 21.3.  Shallow residual products end in two hyperbolic tangents an
+        // element and gain by more workgroups a little longer (32 columns x 64 rows, 720 tiles: o by 2502 rows 13.0 / 10.5, down 17.8 / 17.1).
+        const uint64_t t64 = tiles(64, 64), t6432 = tiles(64, 32), t128 = tiles(128, 128);
+        if constexpr (MODE == DenseEpi::Residual) {
+            // Deep ones in ranges of the depth, us for 2048 x 8192 before / by 64 x 32 x 8 ranges / 64 x 64 x 4 / 128 x 128 x as many as give every compute unit one:
+            // by 5 rows 35 / 11.7 / 14.6 / 20.8, by 33 35 / 13.5 / 15.9 / 21.4, by 65 35 / 16.4 / 16.2 / 22.2, by 200 36 / - / 22.1 / 24.4, by 300 37 / - / 33.3 / 25.9,
+            // by 500 38 / - / - / 31.5, by 902 59 / - / - / 44.9.
+            if (w.K >= 4096 && e.sums) {
+                const uint32_t large = t128 <= CUS / 2 ? (uint32_t)std::min<uint64_t>(8, CUS / t128) : 1;
+                if (t6432 <= 80) { go_gemm<T, 1, 1, 4, 2, 1, 4, MODE>(w, a, lda, M, e, s, 8); return; }
+                if (t64 <= CUS / 2) { go_gemm<T, 1, 1, 4, 2, 2, 4, MODE>(w, a, lda, M, e, s, 4); return; }
+                if (large > 1) { go_gemm<T, 2, 2, 2, 2, 2, 3, MODE>(w, a, lda, M, e, s, large); return; }
+            }
+        }
+        if (tiles(32, 32) <= 3 * CUS) { go_gemm<T, 1, 1, 4, 1, 1, 4, MODE>(w, a, lda, M, e, s); return; }
+        if (t6432 < 2 * CUS) { go_gemm<T, 1, 1, 4, 2, 1, 4, MODE>(w, a, lda, M, e, s); return; }
+        if constexpr (MODE == DenseEpi::Residual)
+            if (w.K < 2048 && tiles(32, 64) <= 3 * CUS) { go_gemm<T, 1, 2, 2, 1, 1, 4, MODE>(w, a, lda, M, e, s); return; }
         // The largest tile that keeps the chip busy (us, 256 x 256 / 128 x 128 / 128 x 64 / 64 x 64; gate: input products, up: gate and up,
         // res: residual products of a prompt):
         // - 256 x 256, one workgroup a compute unit, if its last round is at least 0.8 full on average: up 16384 x 2048 by 902 rows (256 tiles)
@@ -438,16 +538,22 @@ void go(const DenseWeight& w, const DenseIn& in, uint32_t M, const DenseEpiArgs&
         //   res 2048 x 8192 by 130 rows 35.0 / 59.2, 2048 x 2048 by 520 14.3 / 18.1, but gate 1152 x 576 by 902 8.2 / 7.5.  The shallow form
         //   wins up to four on a compute unit: gate 928 x 576 by 2502 rows (600) 33 / 12.9 / 10.7 / 9.2, up 3072 x 576 by 1344 (1008) - / 12.7 / 11.2 /
         //   11.2, but gate 1728 x 576 by 2502 (1080) 33 / 14.9 / 17.0 / 15.6, up 3072 x 576 by 1500 (1152) 25 / 13.0 / 15.4 / 15.3.
-        const uint64_t t64 = tiles(64, 64), t256 = tiles(256, 256), rounds = (t256 + CUS - 1) / CUS;
+        const uint64_t t256 = tiles(256, 256), rounds = (t256 + CUS - 1) / CUS;
         const bool deep = w.K >= 1024, small = M <= 64 || t64 <= 2 * CUS || (!deep && t64 <= 4 * CUS);
         if (small && deep) go_gemm<T, 1, 1, 4, 2, 2, 4, MODE>(w, a, lda, M, e, s);
         else if (small) go_gemm<T, 2, 2, 1, 1, 1, 2, MODE>(w, a, lda, M, e, s);
         else if (M > 128 && 5 * t256 >= 4 * CUS * rounds) go_gemm<T, 4, 2, 1, 2, 4, 2, MODE>(w, a, lda, M, e, s);
-        else if (tiles(128, 128) > CUS) go_gemm<T, 4, 2, 1, 1, 2, 2, MODE>(w, a, lda, M, e, s);
+        else if (t128 > CUS) go_gemm<T, 4, 2, 1, 1, 2, 2, MODE>(w, a, lda, M, e, s);
         else go_gemm<T, 2, 2, 2, 2, 1, 3, MODE>(w, a, lda, M, e, s);
     } else {
-        // 32-bit: bound by the matrix unit's rate; the large tile when its tiles give most compute units work
-        if (tiles(128, 128) >= 192) go_gemm<T, 2, 2, 1, 2, 2, 2, MODE>(w, a, lda, M, e, s);
+        // 32-bit: bound by the matrix unit's rate; the large tile when its tiles give most compute units work, small ones (as above, two waves to the depth) when
+        // 64 x 64 leave most of them idle: us by 64 x 64 / 32 x 32 / 32 x 64 / 64 x 32, columns first: o 576 x 576 by 300 rows (180 tiles of 32 x 32) 16.8 / 10.3 / 11.0 / 11.7, by 700 (396) 17.5 /
+        // 14.8 / 11.7 / 12.3, up 3072 x 576 by 130 (288 and 240) 15.6 / 12.7 / 13.2 / 10.5, down 576 x 1536 by 20 32.9 / 20.6 / 21.5 / 22.5, up by 700 (1056 and 1056) 31.8 with
+        // 128 x 128 tiles / 34.8 / 28.7 / 29.6.
+        if (tiles(32, 32) <= CUS) go_gemm<T, 1, 1, 2, 1, 1, 4, MODE>(w, a, lda, M, e, s);
+        else if (tiles(64, 32) <= CUS) go_gemm<T, 2, 1, 2, 1, 1, 4, MODE>(w, a, lda, M, e, s);
+        else if (tiles(32, 64) <= 5 * CUS) go_gemm<T, 1, 2, 2, 1, 1, 4, MODE>(w, a, lda, M, e, s);
+        else if (tiles(128, 128) >= 192) go_gemm<T, 2, 2, 1, 2, 2, 2, MODE>(w, a, lda, M, e, s);
         else go_gemm<T, 2, 2, 1, 1, 1, 2, MODE>(w, a, lda, M, e, s);
     }
 }
@@ -468,6 +574,9 @@ void by_mode(const DenseWeight& w, const DenseIn& in, uint32_t M, DenseEpi mode,
 }  // namespace
 
 uint32_t dense_k_max() { return DENSE_K_MAX; }
+// At most 640 tiles and ranges of 64 x 32 results, 512 of 64 x 64 or 256 of 128 x 128; at most 128 tiles.
+size_t dense_sums_bytes() { return (size_t)256 * 128 * 128 * 4; }
+size_t dense_arrivals_bytes() { return 128 * 4; }
 
 void launch_dense(DType t, const DenseWeight& w, const DenseIn& in, uint32_t M, DenseEpi mode, const DenseEpiArgs& e, hipStream_t s) {
     if (M == 0 || w.N == 0) return;
