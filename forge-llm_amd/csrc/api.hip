@@ -231,8 +231,8 @@ int32_t forge_hip_gemm_q(const forge_hip_qweight* w, const float* x_dev, uint32_
             if ((rck = g_twin.reserve(qbytes + (size_t)M * (K / 32) * 4))) return rck;
             int8_t* q2 = reinterpret_cast<int8_t*>(g_twin.ptr());
             uint16_t* sc2 = reinterpret_cast<uint16_t*>(reinterpret_cast<uint8_t*>(g_twin.ptr()) + qbytes);
-            launch_act_twice(q, sc, M, K, q2, sc2, s);
-            launch_gemm(h->twin.w, q2, sc2, M, y_dev, w->w.N, false, false, nullptr, s, split_ws);
+            const ActTwice twice{q2, sc2};
+            launch_gemm(h->twin.w, q, sc, M, y_dev, w->w.N, false, false, nullptr, s, split_ws, nullptr, nullptr, nullptr, nullptr, nullptr, &twice);
         }
         FH_HIP(hipGetLastError());
         return FORGE_HIP_OK;

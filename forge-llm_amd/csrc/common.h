@@ -112,6 +112,8 @@ __device__ __forceinline__ size_t paged_row(const PageTable& pt, uint32_t t) {
 // (the reference's quantiser gives it 1.0), as the fast prefill GEMM takes them.
 void launch_quantize_act(const float* x, uint32_t M, uint32_t K, int8_t* q, uint16_t* sc, hipStream_t s, bool neg_odd = false);
 // rms_norm of M rows; writes f32 `normed` if non-null and the quantised row (q, sc) if q non-null.
+// Prompt rows in fast mode: the norm with its squares added up in any order, codes with odd blocks negated, and, unless null, launch_act_block_sums' output.
+void launch_rmsnorm_rows(const float* x, const float* w, float eps, uint32_t M, uint32_t H, int8_t* q, uint16_t* sc, float* sums, hipStream_t s);
 void launch_rmsnorm(const float* x, const float* w, float eps, uint32_t M, uint32_t H, float* normed, int8_t* q,
                     uint16_t* sc, hipStream_t s, bool neg_odd = false);
 // out = silu(gate)*up over M rows where gate = gu[r][0..I), up = gu[r][I..2I) when fused, else two
@@ -207,9 +209,11 @@ bool gemm_silu_supported(const QWeight& w, uint32_t inter, uint32_t M);
 // fp16 numbers (launch_act_block_sums, kquant_twin_create write them); every element of the result additionally receives
 // sum_b mt_a[m][b] * mt_w[n][b] (before the SiLU epilogue, if any).
 // raw: the activations [M][K] are there and aq, as are not yet.
+// twice (fast mode, Q6_K twins; no isums, SiLU, mt_a or raw): aq, as have depth w.K / 2; room for the copy that launch_act_twice makes, where a kernel needs it.
+struct ActTwice { int8_t* q; uint16_t* sc; };
 void launch_gemm(const QWeight& w, const int8_t* aq, const uint16_t* as, uint32_t M, float* y, uint32_t ldy,
                  bool accumulate, bool exact, int32_t* isums, hipStream_t s, void* split_ws = nullptr, int8_t* silu_q = nullptr,
-                 uint16_t* silu_sc = nullptr, const float* mt_a = nullptr, const float* mt_w = nullptr, const float* raw = nullptr);
+                 uint16_t* silu_sc = nullptr, const float* mt_a = nullptr, const float* mt_w = nullptr, const float* raw = nullptr, const ActTwice* twice = nullptr);
 // gemm_rows.hip -- the fast mode's product for few rows (the arguments of launch_gemm): launch_gemm goes there itself
 bool gemm_rows_supported(const QWeight& w, uint32_t M, bool silu);
 bool gemm_rows_raw(const QWeight& w, uint32_t M, hipStream_t s);

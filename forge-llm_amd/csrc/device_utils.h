@@ -130,4 +130,13 @@ __device__ __forceinline__ uint32_t quantize_block_part(float4 v, uint16_t& scal
     return q0 | (q1 << 8) | (q2 << 16) | (q3 << 24);
 }
 
+// The operands of the minimum term travel as two fp16 numbers in the 4 bytes of an f32 slot: hi = fp16(x), lo = fp16(x - hi)
+// (x to 2^-22 relative).  The GEMM multiplies them on the f16 matrix unit as hi*hi + hi*lo + lo*hi.  Powers of two keep both
+// sides in fp16's range: activation block sums (up to 32 times the largest activation) arrive times 2^-8, coefficients times 2^8.
+__device__ __forceinline__ float hi_lo_f16(float x) {
+    const uint16_t h = f32_to_f16_bits(x);
+    const uint16_t l = f32_to_f16_bits(x - f16_bits_to_f32(h));
+    return __uint_as_float((uint32_t)h | ((uint32_t)l << 16));
+}
+
 }  // namespace fh

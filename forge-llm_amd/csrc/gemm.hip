@@ -101,7 +101,9 @@ struct GemmSplit {
 // MINT: the tile additionally receives sum_b mt_a[m][b] * mt_w[n][b], a matmul of depth K / 32 on the f16 matrix unit (operands
 // as hi | lo pairs of fp16 numbers) in front of the epilogue (the minimum term of a Q4_K matrix: activation block sums times a coefficient per weight block,
 // kquant_prefill.hip) -- so that it costs no pass over the result and may precede the SiLU epilogue.
-template <bool Q4, bool DUMP, bool EXACT, int TM, bool SPLIT = false, bool SILU = false, bool MINT = false>
+// TWICE: K counts every pair of activation blocks twice (a Q6_K twin's hi and lo blocks meet the same activations), which lie there once: a stage's four blocks
+// are read from one pair.  (A copy with the pairs doubled cost 11.1 us by 2502 rows of 8192 columns, and twice the activations' bytes here.)
+template <bool Q4, bool DUMP, bool EXACT, int TM, bool SPLIT = false, bool SILU = false, bool MINT = false, bool TWICE = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 void gemm_q_kernel(const uint8_t* __restrict__ wq, const uint16_t* __restrict__ wsc, const int8_t* __restrict__ aq,
                    const uint16_t* __restrict__ asc, float* __restrict__ y, int32_t* __restrict__ isums, uint32_t M,
@@ -110,6 +112,7 @@ void gemm_q_kernel(const uint8_t* __restrict__ wq, const uint16_t* __restrict__ 
     constexpr bool MAGIC = !EXACT;               // DUMP && !EXACT: the fast arithmetic, with its block sums written out too
     static_assert(!SPLIT || (MAGIC && !DUMP), "K ranges change the order of the block sum: fast mode only");
     static_assert(!SILU || (MAGIC && !DUMP), "the fused SiLU epilogue belongs to the fast mode");
+    static_assert(!TWICE || (MAGIC && !DUMP && !Q4 && !SILU && !MINT), "a Q6_K twin's form");
     static_assert(!MINT || (MAGIC && !DUMP && !Q4), "the extra f32 term belongs to the fast mode on Q8_0-layout matrices (no 1/16 pending)");
 
     const uint32_t tid = threadIdx.x, lane = tid & 63;
@@ -143,7 +146,8 @@ void gemm_q_kernel(const uint8_t* __restrict__ wq, const uint16_t* __restrict__ 
     // ---- loader mapping: load i of wave w fills LDS rows (4i + w) * 8 .. + 8 of a tile, lane -> (row, position)
     const uint32_t ld_row = wave * 8 + (lane >> 3);                        // + 32 i
     const uint32_t ld_chunk = (lane & 7) ^ ((ld_row >> 1) & 7);            // global chunk for LDS position lane & 7
-    const uint32_t a_voff = (m0 + ld_row) * K + ld_chunk * 16;             // + 32 i K + k0
+    const uint32_t Ka = TWICE ? K / 2 : K;                                 // bytes of an activation row
+    const uint32_t a_voff = (m0 + ld_row) * Ka + (TWICE ? ld_chunk & 3 : ld_chunk) * 16;             // + 32 i Ka + k0
     // SILU: tile row j is weight row i0 + (j / 64) * 32 + j % 32 (+ inter for the up half, (j / 32) odd), i0 = 64 tile_x
     const uint32_t s_inter = SILU ? sp.inter : 0u, si0 = tile_x * 64;
     const uint32_t w_voff = (SILU ? si0 + ld_row : n0 + ld_row) * K + ld_chunk * 16;     // Q8_0 only; load i: + w_step[i]
@@ -155,7 +159,7 @@ void gemm_q_kernel(const uint8_t* __restrict__ wq, const uint16_t* __restrict__ 
     const bool sc_is_a = wave < 2;
     const uint32_t sc_row = tid & 127;
     const uint32_t sc_wrow = SILU ? si0 + (sc_row >> 6) * 32 + (sc_row & 31) + ((sc_row >> 5) & 1) * s_inter : n0 + sc_row;
-    const uint32_t sc_voff = (sc_is_a ? m0 + sc_row : sc_wrow) * nblk * 2;
+    const uint32_t sc_voff = sc_is_a ? (m0 + sc_row) * (TWICE ? nblk : nblk * 2) : sc_wrow * nblk * 2;
     // uniform steps from load to load (rows 32 i further on; SILU: 32 (i / 2) further on, odd loads in the up half)
     const uint32_t w_step[4] = {0u, SILU ? s_inter * K : 32 * K, SILU ? 32 * K : 64 * K, SILU ? 32 * K + s_inter * K : 96 * K};
     const uint32_t q4_step = (SILU ? 32u : 64u) * nblk * 16;
@@ -174,15 +178,15 @@ void gemm_q_kernel(const uint8_t* __restrict__ wq, const uint16_t* __restrict__ 
         auto left = [](uint32_t total, uint32_t skip) {
             return (uint32_t)__builtin_amdgcn_readfirstlane((int)(total > skip ? total - skip : 0u));
         };
-        const __amdgpu_buffer_rsrc_t ra_k = __builtin_amdgcn_make_buffer_rsrc((void*)(aq + k0), 0, left(M * K, k0), RSRC_FLAGS);
+        const __amdgpu_buffer_rsrc_t ra_k = __builtin_amdgcn_make_buffer_rsrc((void*)(aq + (TWICE ? k0 / 2 : k0)), 0, left(M * Ka, TWICE ? k0 / 2 : k0), RSRC_FLAGS);
         const __amdgpu_buffer_rsrc_t rw_k = __builtin_amdgcn_make_buffer_rsrc((void*)(wq + kq), 0, left(N * wrow, kq), RSRC_FLAGS);
-        const __amdgpu_buffer_rsrc_t ras_k = __builtin_amdgcn_make_buffer_rsrc((void*)((const uint8_t*)asc + ks), 0, left(M * nblk * 2, ks), RSRC_FLAGS);
+        const __amdgpu_buffer_rsrc_t ras_k = __builtin_amdgcn_make_buffer_rsrc((void*)((const uint8_t*)asc + (TWICE ? ks / 2 : ks)), 0, left(M * (TWICE ? nblk : nblk * 2), TWICE ? ks / 2 : ks), RSRC_FLAGS);
         const __amdgpu_buffer_rsrc_t rws_k = __builtin_amdgcn_make_buffer_rsrc((void*)((const uint8_t*)wsc + ks), 0, left(N * nblk * 2, ks), RSRC_FLAGS);
         if (part & 1) {
 #pragma unroll
             for (int i = 0; i < 2 * TM; i++)
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(ra_k, FH_LDS3(lds + LDS_A + buf * TILE_BYTES + (i * 4 + wave) * 1024), 16,
-                                                         a_voff + i * 32 * K, 0, 0, 0);
+                                                         a_voff + i * 32 * Ka, 0, 0, 0);
         }
         if ((part & 2) && Q4) {
 #pragma unroll
@@ -238,6 +242,7 @@ void gemm_q_kernel(const uint8_t* __restrict__ wq, const uint16_t* __restrict__ 
         uint2 pk;
         pk.x = sc4[0] | (sc4[1] << 16);
         pk.y = sc4[2] | (sc4[3] << 16);
+        if (TWICE && sc_is_a) pk.y = pk.x;         // (taken here: loads of one address twice made the loop spill 3 KB a lane)
         if (MAGIC && !sc_is_a) { pk.x ^= 0x80000000u; pk.y ^= 0x80000000u; }   // odd blocks: minus sign on the weight scale
         *reinterpret_cast<uint2*>(lds + (sc_is_a ? LDS_ASC : LDS_BSC) + slot * SC_SLOT + sc_row * SC_ROW) = pk;
     };
@@ -619,8 +624,14 @@ bool gemm_silu_supported(const QWeight& w, uint32_t inter, uint32_t M) {
 
 void launch_gemm(const QWeight& w, const int8_t* aq, const uint16_t* as, uint32_t M, float* y, uint32_t ldy,
                  bool accumulate, bool exact, int32_t* isums, hipStream_t s, void* split_ws, int8_t* silu_q, uint16_t* silu_sc,
-                 const float* mt_a, const float* mt_w, const float* raw) {
+                 const float* mt_a, const float* mt_w, const float* raw, const ActTwice* twice) {
     if (M == 0 || w.N == 0) return;
+    auto double_pairs = [&]() {               // the activations with every pair of blocks twice
+        launch_act_twice(aq, as, M, w.K / 2, twice->q, twice->sc, s);
+        aq = twice->q;
+        as = twice->sc;
+        twice = nullptr;
+    };
     auto quantise = [&]() {
         if (raw) launch_quantize_act(raw, M, w.K, const_cast<int8_t*>(aq), const_cast<uint16_t*>(as), s, !exact);
         raw = nullptr;
@@ -646,6 +657,7 @@ void launch_gemm(const QWeight& w, const int8_t* aq, const uint16_t* as, uint32_
         if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) n = 256;
         return n > 0 ? n : 256;
     }();
+    if (twice && (m_step != M || n_step != w.N)) double_pairs();
 #define FH_GEMM_LAUNCH_TM(Q4_, DUMP_, EXACT_, TM_)                                                                        \
     do {                                                                                                                \
         static const hipError_t lds_ok = hipFuncSetAttribute((const void*)gemm_q_kernel<Q4_, DUMP_, EXACT_, TM_>,      \
@@ -713,6 +725,7 @@ void launch_gemm(const QWeight& w, const int8_t* aq, const uint16_t* as, uint32_
                 const double tiles_cost = best.cost + (best.items ? 0.0 : 5.0) + (silu ? 4.0 : 0.0);
                 if (!mt_a && gemm_rows_supported(w, M, silu) && gemm_rows_cost(w, M) < tiles_cost) {
                     if (raw && (silu || overlap(raw, (size_t)M * w.K * 4, y, ((size_t)(M - 1) * ldy + w.N) * 4) || !gemm_rows_raw(w, M, s))) quantise();
+                    if (twice) double_pairs();
                     launch_gemm_rows(w, aq, as, M, y, ldy, accumulate, s, silu_q, silu_sc, raw);
                     return;
                 }
@@ -720,19 +733,19 @@ void launch_gemm(const QWeight& w, const int8_t* aq, const uint16_t* as, uint32_
                 if (best.items) { fsp = best.sp; items = best.items; }
             }
             quantise();
-            if (items || silu || mt_a) {
+            if (items || silu || mt_a || twice) {
                 // the fast kernel's variants: tiles cut along K, the SiLU epilogue, the extra f32 term
                 if (silu) { fsp.silu_q = silu_q; fsp.silu_sc = silu_sc; fsp.inter = w.N / 2; }
                 if (mt_a) { fsp.mt_a = mt_a + (size_t)mlo * nblk; fsp.mt_w = mt_w + (size_t)nlo * nblk; }
                 const dim3 grid = items ? dim3(items) : dim3((nc + BN - 1) / BN, (mc + 64 * tm - 1) / (64 * tm));
-                auto go = [&](auto q4_, auto tm_, auto split_, auto silu_, auto mint_) {
+                auto go = [&](auto q4_, auto tm_, auto split_, auto silu_, auto mint_, auto twice_) {
                     constexpr bool Q4_ = decltype(q4_)::value, SPLIT_ = decltype(split_)::value, SILU_ = decltype(silu_)::value,
-                                   MINT_ = decltype(mint_)::value;
+                                   MINT_ = decltype(mint_)::value, TWICE_ = decltype(twice_)::value;
                     constexpr int TM_ = decltype(tm_)::value;
-                    static const hipError_t lds_ok = hipFuncSetAttribute((const void*)gemm_q_kernel<Q4_, false, false, TM_, SPLIT_, SILU_, MINT_>,
+                    static const hipError_t lds_ok = hipFuncSetAttribute((const void*)gemm_q_kernel<Q4_, false, false, TM_, SPLIT_, SILU_, MINT_, TWICE_>,
                                                                          hipFuncAttributeMaxDynamicSharedMemorySize, GEMM_LDS_BYTES);
                     (void)lds_ok;
-                    fh::launch(gemm_q_kernel<Q4_, false, false, TM_, SPLIT_, SILU_, MINT_>, grid, 256, GEMM_LDS_BYTES, s, wq, wsc, aq_c, as_c,
+                    fh::launch(gemm_q_kernel<Q4_, false, false, TM_, SPLIT_, SILU_, MINT_, TWICE_>, grid, 256, GEMM_LDS_BYTES, s, wq, wsc, aq_c, as_c,
                                y_c, is_c, mc, nc, w.K, ldy, accf, fsp);
                 };
                 using T = std::true_type;
@@ -740,8 +753,8 @@ void launch_gemm(const QWeight& w, const int8_t* aq, const uint16_t* as, uint32_
                 using One = std::integral_constant<int, 1>;
                 using Two = std::integral_constant<int, 2>;
                 auto by_tm = [&](auto q4_, auto split_, auto silu_, auto mint_) {
-                    if (tm == 1) go(q4_, One{}, split_, silu_, mint_);
-                    else go(q4_, Two{}, split_, silu_, mint_);
+                    if (tm == 1) go(q4_, One{}, split_, silu_, mint_, F{});
+                    else go(q4_, Two{}, split_, silu_, mint_, F{});
                 };
                 auto by_shape = [&](auto q4_, auto mint_) {
                     if (items && silu) by_tm(q4_, T{}, T{}, mint_);
@@ -749,7 +762,12 @@ void launch_gemm(const QWeight& w, const int8_t* aq, const uint16_t* as, uint32_
                     else if (silu) by_tm(q4_, F{}, T{}, mint_);
                     else by_tm(q4_, F{}, F{}, mint_);
                 };
-                if (mt_a) by_shape(F{}, T{});          // caller: a Q8_0-layout matrix
+                if (twice) {                           // caller: a Q8_0-layout matrix, no extra term, no SiLU
+                    if (items && tm == 1) go(F{}, One{}, T{}, F{}, F{}, T{});
+                    else if (items) go(F{}, Two{}, T{}, F{}, F{}, T{});
+                    else if (tm == 1) go(F{}, One{}, F{}, F{}, F{}, T{});
+                    else go(F{}, Two{}, F{}, F{}, F{}, T{});
+                } else if (mt_a) by_shape(F{}, T{});   // caller: a Q8_0-layout matrix
                 else if (q4) by_shape(T{}, F{});
                 else by_shape(F{}, F{});
                 continue;

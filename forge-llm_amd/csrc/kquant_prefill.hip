@@ -14,8 +14,8 @@
 //         that the GEMM kernel runs on the f16 matrix unit in front of its epilogue (its mt_a / mt_w operands: hi | lo pairs).
 //   Q6_K  w = d * sc_h * q, q = -32..31, sc_h an int8 per 16-element half.  sc_h * q = 64 hi + lo with lo in [-32, 31] and hi
 //         in [-63, 64]: a block becomes two blocks of a matrix of depth 2K, the hi codes under the scale 64 d and the lo codes
-//         under d.  Both scales are exact fp16 numbers (d is one), so nothing is dropped at all; the activations go in twice
-//         (act_twice_kernel).  Blocks 2p, 2p + 1 of a row become hi(2p), hi(2p + 1), lo(2p), lo(2p + 1): neighbours of equal
+//         under d.  Both scales are exact fp16 numbers (d is one), so nothing is dropped at all; the activations count twice
+//         (gemm.hip reads their pairs of blocks twice; for the kernel of few rows act_twice_kernel makes a copy).  Blocks 2p, 2p + 1 of a row become hi(2p), hi(2p + 1), lo(2p), lo(2p + 1): neighbours of equal
 //         scale, which is what the GEMM's alternating bias wants.
 //
 // Integer block sums stay exact; against the order-faithful result the difference is the order of the f32 additions and, for
@@ -26,15 +26,6 @@
 namespace fh {
 
 namespace {
-
-// The operands of the minimum term travel as two fp16 numbers in the 4 bytes of an f32 slot: hi = fp16(x), lo = fp16(x - hi)
-// (x to 2^-22 relative).  The GEMM multiplies them on the f16 matrix unit as hi*hi + hi*lo + lo*hi.  Powers of two keep both
-// sides in fp16's range: activation block sums (up to 32 times the largest activation) arrive times 2^-8, coefficients times 2^8.
-__device__ __forceinline__ float hi_lo_f16(float x) {
-    const uint16_t h = f32_to_f16_bits(x);
-    const uint16_t l = f32_to_f16_bits(x - f16_bits_to_f32(h));
-    return __uint_as_float((uint32_t)h | ((uint32_t)l << 16));
-}
 
 // One thread per (row, 32-element block).  Planes of the source as gemv_kquant.hip lays them out.
 __global__ __launch_bounds__(256) void twin_q4k_kernel(const uint8_t* __restrict__ qs, const uint8_t* __restrict__ meta, uint32_t K, uint64_t total,

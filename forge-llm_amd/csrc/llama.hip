@@ -358,17 +358,19 @@ void enqueue_mixed_prefill_layer(LlamaModel* m, uint32_t l, uint32_t M, uint32_t
 
 // The projections ids[0..n) of a layer multiply the same quantised rows (aq, asc: depth K, odd blocks negated) and write
 // neighbouring columns of y, all on the int8 MFMA GEMM (fast mode): Q8_0 / Q4_0 matrices as they are, K-quant matrices
-// through their twins, which first get what they need of the rows (Q4_K: the scaled block sums; Q6_K: every block twice).
+// through their twins (Q4_K: with the rows' scaled block sums, which are in pbsum if have_sums; Q6_K: as rows whose pairs of blocks count twice).
 // silu_q: the group is gate, up under ONE twin and the launch writes quantize(silu(gate) * up) instead of y.
-static void matmul_group_mfma(LlamaModel* m, Layer& L, const int* ids, int n, const int8_t* aq, const uint16_t* asc, uint32_t M,
-                              uint32_t K, float* y, uint32_t ldy, bool accumulate, int8_t* silu_q = nullptr, uint16_t* silu_sc = nullptr) {
-    hipStream_t s = m->stream;
-    const QWeight* w[7] = {&L.q, &L.k, &L.v, &L.o, &L.gate, &L.up, &L.down};
-    bool sums = false, twice = false;
+static bool wants_sums(const Layer& L, const int* ids, int n) {
     for (int j = 0; j < n; j++)
-        if (L.twin_span[ids[j]]) (L.twin[ids[j]].coef ? sums : twice) = true;
-    if (sums) launch_act_block_sums(aq, asc, M, K, true, m->pbsum.as<float>(), s);
-    if (twice) launch_act_twice(aq, asc, M, K, m->paq3.as<int8_t>(), m->pasc3.as<uint16_t>(), s);
+        if (L.twin_span[ids[j]] && L.twin[ids[j]].coef) return true;
+    return false;
+}
+static void matmul_group_mfma(LlamaModel* m, Layer& L, const int* ids, int n, const int8_t* aq, const uint16_t* asc, uint32_t M,
+                              uint32_t K, float* y, uint32_t ldy, bool accumulate, bool have_sums, int8_t* silu_q = nullptr, uint16_t* silu_sc = nullptr) {
+    hipStream_t s = m->stream;
+    const ActTwice twice{m->paq3.as<int8_t>(), m->pasc3.as<uint16_t>()};
+    const QWeight* w[7] = {&L.q, &L.k, &L.v, &L.o, &L.gate, &L.up, &L.down};
+    if (!have_sums && wants_sums(L, ids, n)) launch_act_block_sums(aq, asc, M, K, true, m->pbsum.as<float>(), s);
     float* col = y;
     for (int j = 0; j < n;) {
         const int id = ids[j];
@@ -380,7 +382,10 @@ static void matmul_group_mfma(LlamaModel* m, Layer& L, const int* ids, int n, co
         }
         const KqTwin& t = L.twin[id];
         if (t.coef) launch_gemm(t.w, aq, asc, M, col, ldy, accumulate, false, nullptr, s, m->gemm_ws.p, silu_q, silu_sc, m->pbsum.as<float>(), t.coef);
-        else launch_gemm(t.w, m->paq3.as<int8_t>(), m->pasc3.as<uint16_t>(), M, col, ldy, accumulate, false, nullptr, s, m->gemm_ws.p, silu_q, silu_sc);
+        else if (silu_q) {                   // the SiLU form has no reader of its own for pairs that count twice
+            launch_act_twice(aq, asc, M, K, twice.q, twice.sc, s);
+            launch_gemm(t.w, twice.q, twice.sc, M, col, ldy, accumulate, false, nullptr, s, m->gemm_ws.p, silu_q, silu_sc);
+        } else launch_gemm(t.w, aq, asc, M, col, ldy, accumulate, false, nullptr, s, m->gemm_ws.p, nullptr, nullptr, nullptr, nullptr, nullptr, &twice);
         col += t.w.N;
         j += L.twin_span[id];
     }
@@ -399,8 +404,8 @@ void enqueue_mixed_prefill_layer_mfma(LlamaModel* m, uint32_t l, uint32_t M, uin
     int8_t* aq = m->paq.as<int8_t>();
     uint16_t* asc = m->pasc.as<uint16_t>();
     static const int qkv_ids[3] = {0, 1, 2}, o_ids[1] = {3}, gu_ids[2] = {4, 5}, down_ids[1] = {6};
-    { StageMark t(m, ST_RMSNORM); launch_rmsnorm(x, L.attn_norm, c.rms_eps, M, H, nullptr, aq, asc, s, true); }
-    { StageMark t(m, ST_QKV); matmul_group_mfma(m, L, qkv_ids, 3, aq, asc, M, H, qkv, QKV, false); }
+    { StageMark t(m, ST_RMSNORM); launch_rmsnorm_rows(x, L.attn_norm, c.rms_eps, M, H, aq, asc, wants_sums(L, qkv_ids, 3) ? m->pbsum.as<float>() : nullptr, s); }
+    { StageMark t(m, ST_QKV); matmul_group_mfma(m, L, qkv_ids, 3, aq, asc, M, H, qkv, QKV, false, true); }
     {
         StageMark t(m, ST_ROPE);
         launch_rope_kv_store(qkv, qkv + QKS, qkv + QKS + KV, QKV, QKV, m->kc(l), m->vc(l), M, base_pos, nullptr, c.heads, c.kv_heads,
@@ -410,18 +415,18 @@ void enqueue_mixed_prefill_layer_mfma(LlamaModel* m, uint32_t l, uint32_t M, uin
         StageMark t(m, ST_ATTN);
         launch_attn_prefill_quant(qkv, QKV, m->kc(l), m->vc(l), aq, asc, M, base_pos, c.heads, c.kv_heads, c.head_dim, 0u, s, true, m->pt);
     }
-    { StageMark t(m, ST_O); matmul_group_mfma(m, L, o_ids, 1, aq, asc, M, QKS, x, H, true); }
-    { StageMark t(m, ST_RMSNORM); launch_rmsnorm(x, L.ffn_norm, c.rms_eps, M, H, nullptr, aq, asc, s, true); }
+    { StageMark t(m, ST_O); matmul_group_mfma(m, L, o_ids, 1, aq, asc, M, QKS, x, H, true, false); }
+    { StageMark t(m, ST_RMSNORM); launch_rmsnorm_rows(x, L.ffn_norm, c.rms_eps, M, H, aq, asc, wants_sums(L, gu_ids, 2) ? m->pbsum.as<float>() : nullptr, s); }
     if (m->prefill_fuse_silu && L.twin_span[4] == 2 && gemm_silu_supported(L.twin[4].w, I, M)) {
         // gate and up under one twin: the GEMM's epilogue writes silu(gate) * up quantised, the [M][2 inter] floats never exist
-        { StageMark t(m, ST_GATE_UP); matmul_group_mfma(m, L, gu_ids, 2, aq, asc, M, H, nullptr, 2 * I, false, m->paq2.as<int8_t>(), m->pasc2.as<uint16_t>()); }
+        { StageMark t(m, ST_GATE_UP); matmul_group_mfma(m, L, gu_ids, 2, aq, asc, M, H, nullptr, 2 * I, false, true, m->paq2.as<int8_t>(), m->pasc2.as<uint16_t>()); }
         aq = m->paq2.as<int8_t>();
         asc = m->pasc2.as<uint16_t>();
     } else {
-        { StageMark t(m, ST_GATE_UP); matmul_group_mfma(m, L, gu_ids, 2, aq, asc, M, H, gu, 2 * I, false); }
+        { StageMark t(m, ST_GATE_UP); matmul_group_mfma(m, L, gu_ids, 2, aq, asc, M, H, gu, 2 * I, false, true); }
         { StageMark t(m, ST_SILU); launch_silu_mul(gu, gu + I, M, I, 2 * I, nullptr, aq, asc, s, true); }
     }
-    { StageMark t(m, ST_DOWN); matmul_group_mfma(m, L, down_ids, 1, aq, asc, M, I, x, H, true); }
+    { StageMark t(m, ST_DOWN); matmul_group_mfma(m, L, down_ids, 1, aq, asc, M, I, x, H, true, false); }
 }
 
 // One decoder layer of a batched prefill: M rows at positions base_pos.. .
@@ -437,7 +442,12 @@ void enqueue_prefill_layer(LlamaModel* m, uint32_t l, uint32_t M, uint32_t base_
     int8_t* aq = m->paq.as<int8_t>();
     uint16_t* asc = m->pasc.as<uint16_t>();
     const bool exact = (c.flags & FORGE_HIP_FLAG_EXACT) != 0;      // the fast GEMM takes the odd blocks of its activations negated
-    { StageMark t(m, ST_RMSNORM); launch_rmsnorm(x, L.attn_norm, c.rms_eps, M, H, nullptr, aq, asc, s, !exact); }
+    auto norm = [&](const float* w) {
+        StageMark t(m, ST_RMSNORM);
+        if (exact) launch_rmsnorm(x, w, c.rms_eps, M, H, nullptr, aq, asc, s);
+        else launch_rmsnorm_rows(x, w, c.rms_eps, M, H, aq, asc, nullptr, s);
+    };
+    norm(L.attn_norm);
     { StageMark t(m, ST_QKV); launch_gemm(L.qkv, aq, asc, M, qkv, QKV, false, exact, nullptr, s, m->gemm_ws.p); }
     {
         StageMark t(m, ST_ROPE);
@@ -456,7 +466,7 @@ void enqueue_prefill_layer(LlamaModel* m, uint32_t l, uint32_t M, uint32_t base_
         { StageMark t(m, ST_QUANT); launch_quantize_act(attn, M, QKS, aq, asc, s, true); }
     }
     { StageMark t(m, ST_O); launch_gemm(L.o, aq, asc, M, x, H, true, exact, nullptr, s, m->gemm_ws.p); }
-    { StageMark t(m, ST_RMSNORM); launch_rmsnorm(x, L.ffn_norm, c.rms_eps, M, H, nullptr, aq, asc, s, !exact); }
+    norm(L.ffn_norm);
     if (m->prefill_fuse_silu && gemm_silu_supported(L.gate_up, I, M)) {
         // the GEMM's epilogue writes silu(gate) * up quantised: the [M][2 I] floats never exist.  The kernel reads `aq` while
         // it runs, so its output goes to the second code buffer and the down projection reads that.
