@@ -82,6 +82,13 @@ bool scratch_at_hand(uint32_t K, hipStream_t s) {
     return hipStreamIsCapturing(s, &st) == hipSuccess && st == hipStreamCaptureStatusNone;
 }
 
+// The same for the GEMM's workspace, of which few rows can do without.
+bool workspace_at_hand(hipStream_t s) {
+    if (g_gemm.capacity() >= gemm_split_workspace_bytes()) return true;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(s, &st) == hipSuccess && st == hipStreamCaptureStatusNone;
+}
+
 // Room for quantised x[M][K] in the shared scratch; returns pointers.
 int32_t act_scratch(uint32_t M, uint32_t K, int8_t** q, uint16_t** sc) {
     const size_t qbytes = align256((size_t)M * K);
@@ -241,7 +248,7 @@ int32_t forge_hip_gemm_q(const forge_hip_qweight* w, const float* x_dev, uint32_
     if (rc) return rc;
     // fast mode may cut tiles along K to fill the CUs: that kernel parks partial tiles in a workspace
     void* split_ws = nullptr;
-    if (!exact && M > 64) {
+    if (!exact && (M > 64 || (w->w.K >= 8192 && workspace_at_hand((hipStream_t)stream)))) {
         const bool fresh = g_gemm.capacity() < gemm_split_workspace_bytes();
         if ((rc = g_gemm.reserve(gemm_split_workspace_bytes()))) return rc;
         // its counters start at zero and are left at zero; cleared on the caller's stream, so that the clear is ordered

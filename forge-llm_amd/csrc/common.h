@@ -216,10 +216,12 @@ void launch_gemm(const QWeight& w, const int8_t* aq, const uint16_t* as, uint32_
                  uint16_t* silu_sc = nullptr, const float* mt_a = nullptr, const float* mt_w = nullptr, const float* raw = nullptr, const ActTwice* twice = nullptr);
 // gemm_rows.hip -- the fast mode's product for few rows (the arguments of launch_gemm): launch_gemm goes there itself
 bool gemm_rows_supported(const QWeight& w, uint32_t M, bool silu);
-bool gemm_rows_raw(const QWeight& w, uint32_t M, hipStream_t s);
-double gemm_rows_cost(const QWeight& w, uint32_t M);
+bool gemm_rows_raw(const QWeight& w, uint32_t M, bool ranged, hipStream_t s);
+// sums (256 partial tiles of 32 x 32 results, 128 counters that are zero between launches): deep products may be cut into ranges of K that meet there.
+struct GemmRowsSums { float* partials; uint32_t* counters; };
+double gemm_rows_cost(const QWeight& w, uint32_t M, bool ranged);
 void launch_gemm_rows(const QWeight& w, const int8_t* aq, const uint16_t* as, uint32_t M, float* y, uint32_t ldy, bool accumulate, hipStream_t s,
-                      int8_t* silu_q, uint16_t* silu_sc, const float* raw = nullptr);
+                      int8_t* silu_q, uint16_t* silu_sc, const float* raw = nullptr, const GemmRowsSums* sums = nullptr);
 // gemm_order.hip -- the same for the order-faithful mode
 bool gemm_order_pays(const QWeight& w, uint32_t M);
 void launch_gemm_order(const QWeight& w, const int8_t* aq, const uint16_t* as, uint32_t M, float* y, uint32_t ldy, bool accumulate, hipStream_t s);

@@ -723,10 +723,13 @@ void launch_gemm(const QWeight& w, const int8_t* aq, const uint16_t* as, uint32_
                 // takes before and after its stages, about 5 us (that of a cut tile is in the cost of meeting), nor the SiLU epilogue, about
                 // 4 us (1024 -> 8192 by 200 rows: 8.8 planned, 15.5 without and 19.0 with it).  The other kernel has no extra f32 term (MINT).
                 const double tiles_cost = best.cost + (best.items ? 0.0 : 5.0) + (silu ? 4.0 : 0.0);
-                if (!mt_a && gemm_rows_supported(w, M, silu) && gemm_rows_cost(w, M) < tiles_cost) {
-                    if (raw && (silu || overlap(raw, (size_t)M * w.K * 4, y, ((size_t)(M - 1) * ldy + w.N) * 4) || !gemm_rows_raw(w, M, s))) quantise();
+                const GemmRowsSums sums{reinterpret_cast<float*>(split_ws),
+                                        reinterpret_cast<uint32_t*>(reinterpret_cast<uint8_t*>(split_ws) + (size_t)GEMM_SPLIT_MAX_ITEMS * BM * BN * sizeof(float))};
+                const bool ranged = split_ws && !silu;
+                if (!mt_a && gemm_rows_supported(w, M, silu) && gemm_rows_cost(w, M, ranged) < tiles_cost) {
+                    if (raw && (silu || overlap(raw, (size_t)M * w.K * 4, y, ((size_t)(M - 1) * ldy + w.N) * 4) || !gemm_rows_raw(w, M, ranged, s))) quantise();
                     if (twice) double_pairs();
-                    launch_gemm_rows(w, aq, as, M, y, ldy, accumulate, s, silu_q, silu_sc, raw);
+                    launch_gemm_rows(w, aq, as, M, y, ldy, accumulate, s, silu_q, silu_sc, raw, ranged ? &sums : nullptr);
                     return;
                 }
                 tm = best.tm;

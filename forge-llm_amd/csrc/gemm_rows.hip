@@ -50,9 +50,13 @@ struct FewArgs {
     uint32_t inter;
     // RAW: the activations as they come; a workgroup's waves quantise pieces of 64 * 4 elements of them into aq and asc, which are the launch's own until it ends
     const float* x;
+    uint32_t parts, range;           // ranges of K (gridDim.z), steps of each (even)
+    float* sums;                     // [workgroup of a range][parts][partial tile]
+    uint32_t* arrivals;              // [workgroup of a range], zero between launches
     unsigned long long *flags, id;   // a piece's flag holds the launch's number when the piece is there
     uint32_t spin_limit;
 };
+constexpr uint32_t FR_PARTS = 4;            // ranges of K at most
 constexpr uint32_t FR_PIECES = 2048;         // flags
 __host__ __device__ inline uint32_t fr_pieces(uint32_t M, uint32_t K) { return (uint32_t)(((uint64_t)M * K / 4 + 63) / 64); }
 __device__ unsigned long long fr_flags[FR_PIECES];
@@ -72,7 +76,8 @@ __device__ __forceinline__ void quantise_piece(const FewArgs& a, uint32_t i, uin
 // One workgroup: 32 MT rows of activations x 32 columns.  SILU: the matrix is [gate; up], a workgroup takes 32 gate columns and the up
 // columns of the same indices and writes quantize(silu(gate) * up) as gemm.hip's epilogue does.
 // G: groups of 8 rows that are worked out of the last tile of 32 (register r of a tile: rows 8 (r / 4) + 4 h + r % 4); the rest is padding.
-template <bool Q4, int WAVES, bool SILU, bool BIASED, int MT, int G, bool RAW>
+// RANGED: a workgroup takes one of a.parts ranges of K.
+template <bool Q4, int WAVES, bool SILU, bool BIASED, int MT, int G, bool RAW, bool RANGED>
 __global__ __launch_bounds__(WAVES * 64) void gemm_rows_kernel(FewArgs a) {
     constexpr int NT = SILU ? 2 : 1, KW = WAVES / NT;         // column tiles; waves that share K of one
     constexpr int THREADS = WAVES * 64, TILE = 1024 * (MT - 1) + 256 * G;
@@ -85,8 +90,9 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_rows_kernel(FewArgs a) {
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
     const uint32_t c = lane & 31, h = lane >> 5;
     const uint32_t nblk = a.K / 32, n0 = blockIdx.x * 32, m0 = blockIdx.y * 32 * MT;
-    const uint32_t steps = (nblk + FR_U - 1) / FR_U, each = (steps + KW - 1) / KW, per = BIASED ? (each + 1) & ~1u : each;
-    const uint32_t s0 = min(steps, wave % KW * per), s1 = min(steps, s0 + per);
+    static_assert(!RANGED || (BIASED && !SILU && !RAW && MT == 1), "deep products");
+    const uint32_t all = (nblk + FR_U - 1) / FR_U, first = RANGED ? min(all, blockIdx.z * a.range) : 0u, steps = RANGED ? min(all, first + a.range) : all, each = (steps - first + KW - 1) / KW, per = BIASED ? (each + 1) & ~1u : each;
+    const uint32_t s0 = min(steps, first + wave % KW * per), s1 = min(steps, s0 + per);
     const uint32_t col0 = n0 + (SILU ? wave / KW * a.inter : 0u);        // this wave's columns: rows col0 .. + 32 of the matrix
     uint8_t* la = lds + wave * WAVE_LDS;                      // this wave's own: no barrier until the partial tiles meet
     uint8_t* lb = la + LA;
@@ -268,8 +274,40 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_rows_kernel(FewArgs a) {
 #pragma unroll
         for (int r = 0; r < regs(t); r++) red[(16 * t + r) * 64 + lane] = acc[t][r];
     __syncthreads();
+    const uint32_t group = RANGED ? blockIdx.y * gridDim.x + blockIdx.x : 0u;
+    float* mine = RANGED ? a.sums + (size_t)group * a.parts * TILE : nullptr;
+    if constexpr (RANGED) {
+        // The ranges' partial tiles meet in memory, past the caches of an XCD.  A wave's stores have arrived before the barrier that lets the workgroup count itself in; who
+        // counts `parts` adds them up in the order of K and leaves the counter at zero.
+        for (uint32_t e = tid; e < TILE; e += THREADS) {
+            float p[KW];
+#pragma unroll
+            for (int w = 0; w < KW; w++) p[w] = reinterpret_cast<const float*>(lds + w * WAVE_LDS)[e];
+#pragma unroll
+            for (int w = 1; w < KW; w++) p[0] = p[0] + p[w];
+            __hip_atomic_store(mine + (size_t)blockIdx.z * TILE + e, p[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __shared__ uint32_t arrived;
+        __syncthreads();
+        if (tid == 0) {
+            arrived = __hip_atomic_fetch_add(a.arrivals + group, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1;
+            if (arrived == a.parts) __hip_atomic_store(a.arrivals + group, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        __syncthreads();
+        if (arrived != a.parts) return;
+    }
     for (uint32_t e = tid; e < TILE; e += THREADS) {
         float v[NT];
+        if constexpr (RANGED) {
+            float p[FR_PARTS];
+#pragma unroll
+            for (uint32_t q = 0; q < FR_PARTS; q++) p[q] = __hip_atomic_load(mine + (size_t)min(q, a.parts - 1) * TILE + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            v[0] = p[0];
+#pragma unroll
+            for (uint32_t q = 1; q < FR_PARTS; q++) v[0] = q < a.parts ? v[0] + p[q] : v[0];
+            if (Q4) v[0] *= 0.0625f;
+        } else
 #pragma unroll
         for (int j = 0; j < NT; j++) {
             float p[KW];
@@ -305,9 +343,11 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_rows_kernel(FewArgs a) {
 template <bool Q4, bool SILU, int MT, int G, bool RAW>
 void launch_groups(const FewArgs& a, hipStream_t s) {
     constexpr int WAVES = 8;       // sixteen leave a wave 128 registers, and two steps in flight do not fit them
-    const dim3 grid(((SILU ? a.inter : a.N) + 31) / 32, (a.M + 32 * MT - 1) / (32 * MT));
-    if (a.K > 4096) fh::launch(gemm_rows_kernel<Q4, WAVES, SILU, true, MT, G, RAW>, grid, WAVES * 64, 0, s, a);
-    else fh::launch(gemm_rows_kernel<Q4, WAVES, SILU, false, MT, G, RAW>, grid, WAVES * 64, 0, s, a);
+    const dim3 grid(((SILU ? a.inter : a.N) + 31) / 32, (a.M + 32 * MT - 1) / (32 * MT), a.parts);
+    if constexpr (!SILU && !RAW && MT == 1)
+        if (a.parts > 1) { fh::launch(gemm_rows_kernel<Q4, WAVES, SILU, true, MT, G, RAW, true>, grid, WAVES * 64, 0, s, a); return; }
+    if (a.K > 4096) fh::launch(gemm_rows_kernel<Q4, WAVES, SILU, true, MT, G, RAW, false>, grid, WAVES * 64, 0, s, a);
+    else fh::launch(gemm_rows_kernel<Q4, WAVES, SILU, false, MT, G, RAW, false>, grid, WAVES * 64, 0, s, a);
 }
 template <bool Q4, bool SILU, int MT, bool RAW>
 void launch_rows(const FewArgs& a, hipStream_t s) {
@@ -339,6 +379,15 @@ bool gemm_rows_supported(const QWeight& w, uint32_t M, bool silu) {
     return (!silu || w.N % 64 == 0) && M <= 65535u * 32u && (uint64_t)M * w.K <= 0x7FFFFFFFull && (uint64_t)w.N * std::max<uint64_t>(w.qs_row_bytes(), w.K / 16) <= 0x7FFFFFFFull;
 }
 
+// Ranges of K, one to a workgroup, for deep products whose tiles leave half the compute units idle: a workgroup takes 20 bytes of weights a nanosecond, and 64 of them 14 us for
+// 8192 -> 2048.  us with the quantiser, whole / in ranges (six operand sets in turn): Q8_0 8192 -> 2048 by 5 rows 15.1 / 11.8, 32 (4 ranges) 16.1 / 11.9, 64 (2) 16.3 / 13.7, 8192 -> 3072
+// by 16 15.3 / 12.2, Q4_0 8192 -> 2048 by 32 14.8 / 12.0.  Not 4096 -> 1024 (by 16 10.8 / 9.5, but by 32 10.9 / 12.0, by 64 10.8 / 11.3), nor two ranges with two rows of tiles
+// to a workgroup (8192 -> 2048 by 100 16.3 / 18.6).
+static uint32_t ranges(const QWeight& w, uint32_t M) {
+    const uint64_t grid = (uint64_t)((w.N + 31) / 32) * ((M + 31) / 32);
+    return w.K >= 8192 && M <= 64 && grid <= 128 ? (uint32_t)std::min<uint64_t>(FR_PARTS, 256 / grid) : 1;
+}
+
 // Rounds of 256 tiles of 32 columns by 32 `mt` rows, one to a compute unit (a SiLU workgroup works two columns of them).
 static uint32_t rounds(const QWeight& w, uint32_t M, uint32_t mt) { return (uint32_t)(((uint64_t)((w.N + 31) / 32) * ((M + 32 * mt - 1) / (32 * mt)) + 255) / 256); }
 
@@ -347,14 +396,17 @@ static uint32_t rounds(const QWeight& w, uint32_t M, uint32_t mt) { return (uint
 // rows 12.4 / 10.6, 64 13.1 / 11.4, 65 (3 rounds against 2) 17.2 / 17.6, 100 21.9 / 18.5; 8192 -> 2048 by 128 17.4 / 22.6, by 256 31.5 / 27.1; 3072 -> 1024
 // by 300 15.5 / 13.9.  The same bits either way.
 static double two_rows_take(const QWeight& w) { return w.K > 4096 ? 1.8 : 1.6; }
-static uint32_t tile_rows(const QWeight& w, uint32_t M) { return two_rows_take(w) * rounds(w, M, 2) < rounds(w, M, 1) ? 2 : 1; }
+static uint32_t tile_rows(const QWeight& w, uint32_t M) {
+    return two_rows_take(w) * rounds(w, M, 2) < rounds(w, M, 1) ? 2 : 1;
+}
 
 // Whether one launch quantises the activations too.  The hand-over of the codes inside it (2 us) hides where a caller's loop waits for the host's launches (9.6 us for two, 6.5 for
 // one), or where they are few.  us, two launches / one, Q4_0: 576 -> 1536 by 2 .. 200 rows 9.7 / 7.4, 2048 -> 2048 by 2 .. 64 9.5 / 7.3, by 128 9.5 / 8.1, 2048 -> 512 by 16 9.6 / 7.4,
 // 128 (two pieces a wave) 9.7 / 9.1, 2048 -> 8192 by 2 9.7 / 7.8, 32 9.6 / 8.7, 64 (two tiles) 11.2 / 11.2, 8192 -> 2048 by 8 13.4 / 12.0, 32 14.4 / 15.3, 3072 -> 8192 by 2 9.6 / 9.2,
 // 16 9.9 / 10.8, 3072 -> 1024 by 16 9.4 / 7.4, 64 9.4 / 9.5; Q8_0 2048 -> 8192 by 16 9.8 / 9.4, 32 9.5 / 9.7.
 // The whole grid has to be at work at a time (512 workgroups: those at work wait until they give up).  Recorded into a graph the launch would find its number from the replay before.
-bool gemm_rows_raw(const QWeight& w, uint32_t M, hipStream_t s) {
+bool gemm_rows_raw(const QWeight& w, uint32_t M, bool ranged, hipStream_t s) {
+    if (ranged && ranges(w, M) > 1) return false;      // 8192 -> 2048 by 2 to 8 rows, one launch / ranges: Q8_0 13.1 / 11.9, Q4_0 12.2 / 11.7
     const uint64_t grid = (w.N + 31) / 32 * (((uint64_t)M + 31) / 32), bytes = (uint64_t)w.N * w.qs_row_bytes();
     const bool pays = M <= 8 ? bytes <= (20u << 20) : M <= 16 ? w.K <= 2048 || bytes <= (4u << 20) : w.K <= 2048 && bytes <= (10u << 20);
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
@@ -366,15 +418,21 @@ bool gemm_rows_raw(const QWeight& w, uint32_t M, hipStream_t s) {
 // 2048 of depth, or what its columns take from memory at 4.8 TB/s (with the quantiser, 1 / 2 / 3 / 4 rounds: K = 2048 9.9 / 14.2 / 18.8 / 23.5,
 // K = 4096 13 / 20 / 27 / 34, K = 8192 17.5 / 29 / 40 / 52).  1422 products of 2 to 1300 rows were timed both ways, with one row of tiles to a
 // workgroup: the kernel that the estimates prefer is within 3 % of the faster one in all but 9, within 8 % in all.
-double gemm_rows_cost(const QWeight& w, uint32_t M) {
-    const uint32_t mt = tile_rows(w, M);
+double gemm_rows_cost(const QWeight& w, uint32_t M, bool ranged) {
+    const uint32_t mt = tile_rows(w, M), parts = ranged && mt == 1 ? ranges(w, M) : 1;
+    if (parts > 1) return 6.0 + 2.7 * w.K / 2048.0 / parts;
     const double columns = std::min<uint32_t>(w.N, 256 * 32), row_bytes = (double)w.qs_row_bytes() + w.K / 16;
     return 2.0 + (double)rounds(w, M, mt) * std::max((mt == 2 ? two_rows_take(w) : 1.0) * (1.8 + 2.7 * w.K / 2048.0), columns * row_bytes / 4.8e6);
 }
 
 void launch_gemm_rows(const QWeight& w, const int8_t* aq, const uint16_t* as, uint32_t M, float* y, uint32_t ldy, bool accumulate, hipStream_t s,
-                      int8_t* silu_q, uint16_t* silu_sc, const float* raw) {
-    FewArgs a{w.qs, w.scales, aq, as, y, M, w.N, w.K, ldy, accumulate ? 1u : 0u, silu_q, silu_sc, w.N / 2, raw, nullptr, 0, 0};
+                      int8_t* silu_q, uint16_t* silu_sc, const float* raw, const GemmRowsSums* sums) {
+    const bool ranged = sums && !silu_q && !raw;
+    const uint32_t mt = raw ? 1 : tile_rows(w, M);
+    FewArgs a{w.qs, w.scales, aq, as, y, M, w.N, w.K, ldy, accumulate ? 1u : 0u, silu_q, silu_sc, w.N / 2, raw, 1, 0, nullptr, nullptr, nullptr, 0, 0};
+    const uint32_t steps = (w.K / 32 + FR_U - 1) / FR_U;
+    if (ranged && mt == 1 && ranges(w, M) > 1) { a.parts = ranges(w, M); a.sums = sums->partials; a.arrivals = sums->counters; }
+    a.range = ((steps + a.parts - 1) / a.parts + 1) & ~1u;
     if (raw) {
         static const uint32_t limit = [] { const char* e = getenv("FORGE_HIP_PD_SPIN_LIMIT"); return e && atoi(e) > 0 ? (uint32_t)atoi(e) : 64u; }();
         a.spin_limit = limit;
@@ -384,7 +442,7 @@ void launch_gemm_rows(const QWeight& w, const int8_t* aq, const uint16_t* as, ui
     }
     const bool q4 = w.wdtype == FORGE_HIP_Q4_0, silu = silu_q != nullptr;
     auto go = [&](auto q4_, auto silu_) {
-        if (tile_rows(w, M) == 2) launch_rows<decltype(q4_)::value, decltype(silu_)::value, 2, false>(a, s);
+        if (mt == 2) launch_rows<decltype(q4_)::value, decltype(silu_)::value, 2, false>(a, s);
         else launch_rows<decltype(q4_)::value, decltype(silu_)::value, 1, false>(a, s);
     };
     if (raw && q4) launch_rows<true, false, 1, true>(a, s);
