@@ -99,7 +99,7 @@ void launch_rmsnorm(const float* x, const float* w, float eps, uint32_t M, uint3
 
 // ---- rmsnorm + quantisation of a prompt's rows (fast mode) ----------------------------------
 // The row stays in registers, and its squares are added up by lanes and waves: the kernel above walks 16 chains of H / 16 additions, in the reference's
-// order, beside which its memory traffic does not count.  us, that kernel / this, 2048 channels: 33 rows 4.8 / 3.4, 2502 rows 10.3 / 8.0.  The block sums that Q4_K prompt
+// order, beside which its memory traffic does not count.  us, that kernel / this, 2048 channels: 33 rows 4.8 / 3.4 to 4.2, 2502 rows 10.3 / 8.0.  The block sums that Q4_K prompt
 // products need come with the codes (a kernel of their own: 4.9 us by 2502 rows).
 template <int NV>
 __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(const float* __restrict__ x, const float* __restrict__ w, float eps, uint32_t H, uint32_t* __restrict__ q,
