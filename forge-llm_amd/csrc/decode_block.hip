@@ -671,6 +671,7 @@ __device__ __forceinline__ bool pb_grouped_layer(const PbArgs& a, const PbLayer&
     const float y = mean * sh->raw[min(gv + tid, ne - 1)], other = lane_xor<1>(y);
     if (tid < group * s.vdim && !(tid & 1u)) stc64(a.tout + (kvh * group * s.vdim + tid) / 2, base + PB_T_OUT, pb_pack(y, other));
     if (a.stamps && role == 0 && tid == 0) a.stamps[5 * l + 2] = wall_clock64();
+    if (a.splits > 1) __syncthreads();       // the other parts lie where a wave that is done lays down the next layer's values
     return true;
 }
 
@@ -1535,7 +1536,7 @@ __global__ __launch_bounds__(PB_THREADS) void decode_block_wide_kernel(PbArgs a)
                 __syncthreads();
             }
             // A head's workgroup: the barriers of what its polling waves do.
-            const uint32_t joins = kind == PB_FIRST ? (cx.wg < a.ns.heads ? 3u : 0u) : cx.wg < grouped_roles ? (a.splits > 1 && cx.wg % a.splits == 0 ? 4u : 3u) : 0u;
+            const uint32_t joins = kind == PB_FIRST ? (cx.wg < a.ns.heads ? 3u : 0u) : cx.wg < grouped_roles ? (a.splits > 1 && cx.wg % a.splits == 0 ? 5u : 3u) : 0u;
             const PbLayer& N = layers[min(l + 1, a.L - 1)];
             PbSet<1, PW_U> wo;
             PbSet<PW_TGA, PW_U> wga;

@@ -25,6 +25,10 @@ def configs(fh):
         "wide_largest": ("kakirax_oracle", kak(2048, 70, [gla(16, 64, 128, 8192), att(32, 8, 64, 64, 8192)], embedding_scale=45.0)),
         "wide_ragged": ("kakirax_oracle", kak(1000, 203, [gla(5, 20, 60, 2077, tau=3.0), att(6, 2, 20, 44, 2077, rot_dims=12), 0, 1], embedding_scale=9.5, eps=3e-3, cap=7.0)),
         "wide_deep": ("kakirax_oracle", kak(90, 80, [att(24, 24, 32, 32, 1601), gla(48, 16, 32, 1601), 0], embedding_scale=8.0)),
+        # records of parts over many waves' strips of LDS; more parts than linear heads
+        "grouped_few_heads": ("kakirax_oracle", kak(64, 80, [att(9, 3, 64, 64, 51)] * 3, embedding_scale=8.0)),
+        "mixed_few_heads": ("kakirax_oracle", kak(64, 80, [att(12, 3, 64, 64, 51), gla(2, 32, 32, 51), 0, 0], embedding_scale=8.0)),
+        "wide_few_heads": ("kakirax_oracle", kak(90, 80, [att(8, 2, 64, 64, 1601), 0, gla(2, 32, 32, 1601), 0], embedding_scale=8.0)),
         "linear_only": ("kakirax_oracle", kak(70, 61, [gla(3, 16, 32, 40), 0], embedding_scale=8.0)),
     }
 
@@ -77,6 +81,27 @@ def test_contexts_of_several_rounds(get, name, monkeypatch):
             x.forward_prefill(ids[:start])
         assert m.decode_launches == 1 and sequence.decode_launches > 1
         for t in ids[start:start + 3]:
+            check(m.forward(int(t)), sequence.forward(int(t)).astype(np.float64), "bfloat16")
+        assert m.decode_launches == 1
+    m.close()
+    sequence.close()
+
+
+@pytest.mark.parametrize("name", ["grouped_few_heads", "mixed_few_heads", "wide_few_heads"])
+def test_parts_over_the_strips_of_all_waves(get, name, monkeypatch):
+    """A key / value head's parts, up to 64 of them, lie where its workgroup's waves keep transposed values: at four, eight and twelve waves that attend (up to 8192 rows of context, up to 16384,
+    beyond) the records reach the strips of waves without a part in adding them up, which are free for the next layer at once."""
+    c = get(name)
+    ids = c.ids(16700, seed=7)
+    m = c.model(max_seq=16700, dtype="bfloat16")
+    monkeypatch.setenv("FORGE_HIP_PERSIST", "0")
+    sequence = c.model(max_seq=16700, dtype="bfloat16")
+    for start in (1300, 2700, 8300, 16500):
+        for x in (m, sequence):
+            x.reset()
+            x.forward_prefill(ids[:start])
+        assert m.decode_launches == 1 and sequence.decode_launches > 1
+        for t in ids[start:start + 12]:
             check(m.forward(int(t)), sequence.forward(int(t)).astype(np.float64), "bfloat16")
         assert m.decode_launches == 1
     m.close()
