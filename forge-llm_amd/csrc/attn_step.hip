@@ -54,7 +54,7 @@ __device__ __forceinline__ void as_one_by_one(const float* q, const uint16_t* kc
                 for (uint32_t c = lane; c < HD; c += 64) d = fmaf(q[(size_t)(h0 + g) * HD + c], f16_bits_to_f32(kc[at + c]), d);
                 d = wave_sum(d) * scale;
                 const float m_new = fmaxf(m, d);
-                if (m_new == -INFINITY) continue;
+                if (m_new == -INFINITY && d == d) continue;      // nothing above -inf yet; fmaxf passes NaN over, which spreads
                 const float alpha = __expf(m - m_new), p = __expf(d - m_new);
                 m = m_new;
                 l = fmaf(l, alpha, p);

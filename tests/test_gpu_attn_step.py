@@ -82,6 +82,23 @@ def test_infinities_and_no_number(fh, torch_gpu, heads, kv_heads, hd, seq):
     assert np.abs(fh.ops.attention_flash(*tail, seq, heads, kv_heads, hd, 0).cpu().numpy() - _want(q, k, v, heads, kv_heads, hd)).max() <= 4e-6
 
 
+@pytest.mark.parametrize("heads,kv_heads,hd,seq", [(32, 8, 64, 40), (32, 8, 64, 700), (32, 32, 96, 200), (12, 2, 128, 100), (3, 3, 128, 1)])
+def test_a_key_without_a_number(fh, torch_gpu, heads, kv_heads, hd, seq):
+    """NaN in a key makes every result of its heads NaN wherever the key stands: the first a wave sees, the last, behind one that scores -inf."""
+    torch = torch_gpu
+    q, k, v = _case(torch, heads, kv_heads, hd, seq, 6)
+    want, rest = _want(q, k, v, heads, kv_heads, hd).reshape(heads, hd), heads // kv_heads
+    for at in sorted({0, min(32, seq - 1), seq // 2, seq - 1}):
+        for behind in (False, True):
+            k2 = k.clone()
+            if behind and at:
+                k2[at // 32 * 32:at, :hd] = -torch.inf * q[:hd].sign()
+            k2[at, 3] = torch.nan
+            got = fh.ops.attention_flash(*_dev(q, k2, v), seq, heads, kv_heads, hd, 0).cpu().numpy().reshape(heads, hd)
+            assert np.isnan(got[:rest]).all(), (at, behind)
+            assert np.abs(got[rest:] - want[rest:]).max(initial=0) <= 4e-6
+
+
 @pytest.mark.parametrize("heads,kv_heads,hd,seq", [(64, 16, 64, 300), (300, 100, 64, 40), (96, 96, 96, 200), (12, 2, 128, 100)])
 def test_result_over_the_inputs(fh, torch_gpu, heads, kv_heads, hd, seq):
     """A result in place of the query, over a part of it or over a part of the cache has the bits of one with a buffer of its own."""
