@@ -53,9 +53,8 @@ __device__ __forceinline__ void as_one_by_one(const float* q, const uint16_t* kc
                 float d = 0.f;
                 for (uint32_t c = lane; c < HD; c += 64) d = fmaf(q[(size_t)(h0 + g) * HD + c], f16_bits_to_f32(kc[at + c]), d);
                 d = wave_sum(d) * scale;
-                const float m_new = fmaxf(m, d);
-                if (m_new == -INFINITY && d == d) continue;      // nothing above -inf yet; fmaxf passes NaN over, which spreads
-                const float alpha = __expf(m - m_new), p = __expf(d - m_new);
+                // a score of -inf has the weight 0, also ahead of all others (0 times an infinite value is no number); fmaxf passes NaN over, the weight does not
+                const float m_new = fmaxf(m, d), alpha = m == -INFINITY ? 0.f : __expf(m - m_new), p = d == -INFINITY ? 0.f : __expf(d - m_new);
                 m = m_new;
                 l = fmaf(l, alpha, p);
                 for (uint32_t c = lane, i = 0; c < HD; c += 64, i++) a[i] = fmaf(p, f16_bits_to_f32(vc[at + c]), a[i] * alpha);

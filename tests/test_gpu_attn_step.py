@@ -71,6 +71,11 @@ def test_infinities_and_no_number(fh, torch_gpu, heads, kv_heads, hd, seq):
     assert np.abs(got[0] - _want(q, k[keep], v[keep], heads, kv_heads, hd).reshape(heads, hd)[0]).max() <= 4e-6
     rest = heads // kv_heads
     assert np.abs(got[rest:] - _want(q, k, v, heads, kv_heads, hd).reshape(heads, hd)[rest:]).max(initial=0) <= 4e-6
+    for first in (0, at):                             # ... but 0 times an infinite value is no number, as in 64 bits
+        k3, v3 = k.clone(), v.clone()
+        k3[first, :hd], v3[first, 7] = -torch.inf * q[:hd].sign(), torch.inf
+        got = fh.ops.attention_flash(*_dev(q, k3, v3), seq, heads, kv_heads, hd, 0).cpu().numpy().reshape(heads, hd)
+        assert np.isnan(got[0, 7]) and np.isfinite(got[0, np.arange(hd) != 7]).all()
     v2 = v.clone()
     v2[at, 3], v2[at, 5] = torch.inf, torch.nan
     got = fh.ops.attention_flash(*_dev(q, k, v2), seq, heads, kv_heads, hd, 0).cpu().numpy().reshape(heads, hd)
