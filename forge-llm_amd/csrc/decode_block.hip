@@ -1647,6 +1647,17 @@ __global__ __launch_bounds__(256) void pb_transpose_kernel(const uint16_t* __res
 
 template <typename S> bool pb_same(const S& a, const S& b) { return memcmp(&a, &b, sizeof(S)) == 0; }
 
+// A mixer's input product as far as its rows are read: the raw part and the heads' gates.  (What pads the matrix behind them would make a workgroup that holds nothing else a reader on which
+// no later phase depends: it might find its input overwritten, and the step would be given up.)
+DenseWeight pb_input(const PbMixer& m) {
+    const uint32_t rows = m.kind == MixerKind::LatentAttention ? m.latent.raw_row() + m.latent.heads * m.latent.vdim
+                        : m.kind == MixerKind::GroupedAttention ? m.grouped.raw_row() + m.grouped.heads * m.grouped.vdim
+                                                                : m.linear.raw_row() + m.linear.heads * m.linear.vdim;
+    DenseWeight w = m.in;
+    w.N = std::min(w.N, rows);
+    return w;
+}
+
 }  // namespace
 
 struct PbState {
@@ -1722,7 +1733,7 @@ int32_t pb_create(const PbModelIn& in, PbState** out) {
     uint32_t g = 1;
     auto need = [&](uint32_t N, uint32_t tiles_each) { g = std::max(g, ((N + 15) / 16 + tiles_each - 1) / tiles_each); };
     for (const PbLayerIn* l : of)
-        if (l) need(l->mixer->in.N, PB_TI);
+        if (l) need(pb_input(*l->mixer).N, PB_TI);
     need(layers[0].gate_up.N, PB_TG);
     need(a.W, 1);
     // ... or, what registers do not hold, all workgroups
@@ -1743,7 +1754,7 @@ int32_t pb_create(const PbModelIn& in, PbState** out) {
         return m;
     };
     for (int k = 0; k < 2; k++)
-        if (of[k]) { a.in[k] = mat(of[k]->mixer->in, wide ? PW_TI : PB_TI, wide ? PW_U : PB_UI); a.o[k] = mat(of[k]->mixer->o, 1, wide ? PW_U : PB_UO); }
+        if (of[k]) { a.in[k] = mat(pb_input(*of[k]->mixer), wide ? PW_TI : PB_TI, wide ? PW_U : PB_UI); a.o[k] = mat(of[k]->mixer->o, 1, wide ? PW_U : PB_UO); }
     a.gate_up = mat(layers[0].gate_up, wide ? PW_TG : PB_TG, wide ? PW_U : PB_UI);
     a.down = mat(layers[0].down, 1, wide ? PW_UD : PB_UD);
     if (in.loop.p) a.loop = mat(in.loop, 1, PB_UL);

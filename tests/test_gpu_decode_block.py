@@ -29,6 +29,10 @@ def configs(fh):
         "grouped_few_heads": ("kakirax_oracle", kak(64, 80, [att(9, 3, 64, 64, 51)] * 3, embedding_scale=8.0)),
         "mixed_few_heads": ("kakirax_oracle", kak(64, 80, [att(12, 3, 64, 64, 51), gla(2, 32, 32, 51), 0, 0], embedding_scale=8.0)),
         "wide_few_heads": ("kakirax_oracle", kak(90, 80, [att(8, 2, 64, 64, 1601), 0, gla(2, 32, 32, 1601), 0], embedding_scale=8.0)),
+        # an odd number of heads of 32 values: rows of the input product that no head reads
+        "latent_odd": ("vabirax_oracle", vab(64, 61, [lay(3, 32, 32, 32, 64, 64, 51, None)] * 2)),
+        "grouped_odd": ("kakirax_oracle", kak(64, 61, [att(3, 1, 32, 32, 51)] * 2, embedding_scale=8.0)),
+        "wide_odd": ("kakirax_oracle", kak(64, 61, [gla(3, 32, 32, 1601), att(3, 1, 32, 32, 1601)], embedding_scale=8.0)),
         "linear_only": ("kakirax_oracle", kak(70, 61, [gla(3, 16, 32, 40), 0], embedding_scale=8.0)),
     }
 
@@ -104,6 +108,24 @@ def test_parts_over_the_strips_of_all_waves(get, name, monkeypatch):
         for t in ids[start:start + 12]:
             check(m.forward(int(t)), sequence.forward(int(t)).astype(np.float64), "bfloat16")
         assert m.decode_launches == 1
+    m.close()
+    sequence.close()
+
+
+@pytest.mark.parametrize("name", ["latent_odd", "grouped_odd", "linear_only", "wide_odd"])
+def test_rows_that_no_head_reads(get, name, monkeypatch):
+    """The last rows of an input product pad it; no workgroup has only those to do (none would wait for it, and it would find its own input overwritten and give up)."""
+    c = get(name)
+    ids = c.ids(500, seed=11)
+    m = c.model(max_seq=500, dtype="bfloat16")
+    monkeypatch.setenv("FORGE_HIP_PERSIST", "0")
+    sequence = c.model(max_seq=500, dtype="bfloat16")
+    for x in (m, sequence):
+        x.forward_prefill(ids[:2])
+    assert m.decode_launches == 1 and sequence.decode_launches > 1
+    for t in ids[2:]:
+        check(m.forward(int(t)), sequence.forward(int(t)).astype(np.float64), "bfloat16")
+    assert m.decode_launches == 1
     m.close()
     sequence.close()
 
