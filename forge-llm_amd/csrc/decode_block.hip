@@ -12,6 +12,8 @@
 //   * All workgroups share the output matrix.
 // A row times a vector is a product of 16 rows on the matrix unit.  Its other 15 columns are free, so a vector that the kernel sequence multiplies in 32-bit goes in as three
 // bfloat16 planes (x = hi + lo + rest, exact) in columns of their own: the same precision, no conversion of weights and no reduction over lanes.
+// What is not finite: an infinite or NaN element of a vector makes a row's product what it is in the sequence's 32-bit sums (infinite, or NaN where it meets a weight of 0). A weight that is
+// infinite makes its row's product NaN, where the sequence could still have an infinity: planes and pieces that pad a product multiply it by 0.
 //
 // Per token in us, kernel sequence / this, by rows of context (sizes of vabirax_135m: 9 heads of 64 + 32, window 1024; kakirax_135m: three layers of linear attention to one of grouped):
 //   latent            20: 882 / 393    200: 890 / 405    900: 905 / 420    2400: 907 / 419
@@ -121,11 +123,12 @@ __device__ __forceinline__ v8bf pb_load8(const __bf16* base, uint32_t off) {
 }
 __device__ __forceinline__ float pb_f32(const float* base, uint32_t i) { return ldg(base + i); }
 
-// Three bfloat16 that add up to x.
+// Three bfloat16 that add up to x: what is past the largest bfloat16 goes on to the next, infinities and NaN to the last.
 __device__ __forceinline__ void pb_split(float x, __bf16& hi, __bf16& lo, __bf16& rest) {
-    hi = (__bf16)x;
+    constexpr float MAX = 0x1.FEp127f;
+    hi = (__bf16)__builtin_amdgcn_fmed3f(x, -MAX, MAX);
     const float r = x - (float)hi;
-    lo = (__bf16)r;
+    lo = (__bf16)__builtin_amdgcn_fmed3f(r, -MAX, MAX);
     rest = (__bf16)(r - (float)lo);
 }
 __device__ __forceinline__ uint32_t pb_pack(float a, float b) {

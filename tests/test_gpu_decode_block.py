@@ -130,6 +130,35 @@ def test_rows_that_no_head_reads(get, name, monkeypatch):
     sequence.close()
 
 
+@pytest.mark.parametrize("ff", [51, 1601])
+def test_a_normed_row_beyond_bfloat16(fh, torch_gpu, tmp_path, ff, monkeypatch):
+    """An element of a normed row between bfloat16's largest number and 32-bit's is finite in its planes, as it is in the kernel sequence's 32-bit row.  Everything but the gates is blind to it,
+    and they close."""
+    from oracle import kakirax_oracle
+    s, c = fh.synth, 3
+    cfg = s.kakirax_config(64, 61, [s.kakirax_gla(2, 32, 32, ff), s.kakirax_attention(2, 1, 32, 32, ff)])
+    t = s.folder_tensors(cfg, 5)
+    t["embed"][:, c] = s.to_bf16([1.0])                                  # the same for all tokens, nearly so when normed
+    for name in ("q", "k", "v", "a1", "g"):
+        t["l0.mix." + name][:, c] = s.to_bf16([-1.0 if name == "g" else 0.0])
+    x = s.from_bf16(t["embed"]).astype(np.float64)
+    z = (x[:, c] - x.mean(1)) / np.sqrt(x.var(1) + 1e-5)
+    t["l0.norm1"][c:c + 1], t["l0.norm1.b"][c] = s.to_bf16([1.0e36 / np.median(z)]), 0x7F7F
+    y = z * s.from_bf16(t["l0.norm1"][c]) + s.from_bf16(t["l0.norm1.b"][c])
+    ids = np.flatnonzero((y > 3.3965e38) & (y < 3.402e38))
+    assert ids.size >= 20
+    case = Case(fh, kakirax_oracle, tmp_path, cfg, t)
+    m = case.model(dtype="bfloat16")
+    monkeypatch.setenv("FORGE_HIP_PERSIST", "0")
+    sequence = case.model(dtype="bfloat16")
+    for i, token in enumerate(ids):
+        got, want = m.forward(int(token)), sequence.forward(int(token))
+        assert (m.decode_launches == 1) and sequence.decode_launches > 1
+        check(got, want.astype(np.float64), "bfloat16")
+    m.close()
+    sequence.close()
+
+
 def bits(x):
     return x.view(np.uint32)
 
