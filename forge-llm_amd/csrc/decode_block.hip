@@ -12,8 +12,9 @@
 //   * All workgroups share the output matrix.
 // A row times a vector is a product of 16 rows on the matrix unit.  Its other 15 columns are free, so a vector that the kernel sequence multiplies in 32-bit goes in as three
 // bfloat16 planes (x = hi + lo + rest, exact) in columns of their own: the same precision, no conversion of weights and no reduction over lanes.
-// What is not finite: an infinite or NaN element of a vector makes a row's product what it is in the sequence's 32-bit sums (infinite, or NaN where it meets a weight of 0). A weight that is
-// infinite makes its row's product NaN, where the sequence could still have an infinity: planes and pieces that pad a product multiply it by 0.
+// What is not finite: an infinite or NaN element of a vector makes a row's product what it is in the sequence's 32-bit sums (infinite, or NaN where it meets a weight of 0).  Weights are finite, since
+// what pads a product multiplies them by 0: a model with others keeps the sequence.  A cached row's elements are taken to be finite as well (an infinite one, a projection past bfloat16's
+// range, may come out as NaN where the sequence has an infinity).
 //
 // Per token in us, kernel sequence / this, by rows of context (sizes of vabirax_135m: 9 heads of 64 + 32, window 1024; kakirax_135m: three layers of linear attention to one of grouped):
 //   latent            20: 882 / 393    200: 890 / 405    900: 905 / 420    2400: 907 / 419
@@ -1648,6 +1649,17 @@ __global__ __launch_bounds__(256) void pb_transpose_kernel(const uint16_t* __res
     out[i] = uk[(size_t)head * dim * rank + j % dim * rank + j / dim];
 }
 
+// flag <- 1 if one of n pieces of eight bfloat16 holds an infinity or NaN
+__global__ __launch_bounds__(256) void pb_not_finite_kernel(const uint4* __restrict__ w, size_t n, uint32_t* flag) {
+    auto odd = [](uint32_t v) { return (v & 0x7F80u) == 0x7F80u || (v & 0x7F800000u) == 0x7F800000u; };
+    bool any = false;
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
+        const uint4 v = w[i];
+        any = any || odd(v.x) || odd(v.y) || odd(v.z) || odd(v.w);
+    }
+    if (any) *flag = 1;
+}
+
 template <typename S> bool pb_same(const S& a, const S& b) { return memcmp(&a, &b, sizeof(S)) == 0; }
 
 // A mixer's input product as far as its rows are read: the raw part and the heads' gates.  (What pads the matrix behind them would make a workgroup that holds nothing else a reader on which
@@ -1786,9 +1798,28 @@ int32_t pb_create(const PbModelIn& in, PbState** out) {
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, st->kernel, PB_THREADS, st->lds) != hipSuccess || per_cu < 1) { (void)hipGetLastError(); return FORGE_HIP_OK; }
     st->grid = (uint32_t)cus;
 
+    uint32_t* flag = st->dev<uint32_t>(4);
+    if (!flag) return FORGE_HIP_OK;
+    FH_HIP(hipMemset(flag, 0, 4));
+    std::vector<const void*> seen;                                   // a layer may run with another one's tensors
+    auto look = [&](const DenseWeight& w) {
+        if (!w.p || std::find(seen.begin(), seen.end(), w.p) != seen.end()) return;
+        seen.push_back(w.p);
+        const size_t n = (size_t)w.N * w.K / 8;
+        fh::launch(pb_not_finite_kernel, dim3((uint32_t)std::min<size_t>((n + 255) / 256, 4096)), 256, 0, nullptr, (const uint4*)w.p, n, flag);
+    };
+    look(in.head);
+    look(in.loop);
+    for (const PbLayerIn& l : layers)
+        for (const DenseWeight* w : {&l.mixer->in, &l.mixer->o, &l.mixer->uq, &l.mixer->ukv, &l.gate_up, &l.down}) look(*w);
+    uint32_t not_finite = 0;
+    FH_HIP(hipGetLastError());
+    FH_HIP(hipMemcpy(&not_finite, flag, 4, hipMemcpyDeviceToHost));
+    if (not_finite) return FORGE_HIP_OK;
+
     std::vector<PbLayer> host(layers.size());
     const uint32_t uk_n = ls.heads * ls.dim * ls.rank;
-    std::vector<std::pair<const void*, const __bf16*>> turned;       // a layer may run with another one's tensors
+    std::vector<std::pair<const void*, const __bf16*>> turned;
     for (size_t l = 0; l < layers.size(); l++) {
         const PbLayerIn& i = layers[l];
         const PbMixer& m = *i.mixer;

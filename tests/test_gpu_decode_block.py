@@ -159,6 +159,22 @@ def test_a_normed_row_beyond_bfloat16(fh, torch_gpu, tmp_path, ff, monkeypatch):
     sequence.close()
 
 
+@pytest.mark.parametrize("name,at", [("latent_ragged", "head"), ("latent_ragged", "l1.mix.uk"), ("latent_ragged", "loop.in"), ("mixed_ragged", "l0.mlp.down"), ("wide_ragged", "l1.mix.o")])
+@pytest.mark.parametrize("bits16", [0x7F80, 0xFF80, 0x7FC0])
+def test_weights_that_are_not_finite(get, name, at, bits16, tmp_path):
+    """A model with such a weight keeps the kernel sequence; one with bfloat16's largest number does not."""
+    c = get(name)
+    for value, one in ((bits16, False), (0x7F7F, True)):
+        t = dict(c.tensors)
+        t[at] = t[at].copy()
+        t[at][-1, -1] = value
+        c.fh.synth.write_model_folder(str(tmp_path), c.cfg, t)
+        m = c.fh.HipModel.from_folder(str(tmp_path), 16, "bfloat16")
+        m.forward(1)
+        assert (m.decode_launches == 1) == one
+        m.close()
+
+
 def bits(x):
     return x.view(np.uint32)
 
