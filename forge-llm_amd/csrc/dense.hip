@@ -450,8 +450,10 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(const T* __restrict__ 
 
 namespace {
 
-template <typename T, int WN, int WM, int KG, int TN, int TM, int NBUF, DenseEpi MODE>
-void go_gemm(const DenseWeight& w, const void* a, uint32_t lda, uint32_t M, const DenseEpiArgs& e, hipStream_t s, uint32_t parts = 1) {
+template <typename T, int WN, int WM, int KG, int TN, int TM, int NBUF, DenseEpi MODE, bool RANGES = false>
+void go_gemm(const DenseWeight& w, const void* a, uint32_t lda, uint32_t M, const DenseEpiArgs& e, hipStream_t s, uint32_t ranges = 1) {
+    static_assert(!RANGES || (MODE == DenseEpi::Residual && dense_pass(WN, WM, KG, TN, TM) == TM), "ranges of the depth meet in an epilogue of one pass");
+    const uint32_t parts = RANGES ? ranges : 1;
     constexpr uint32_t BN = 32 * TN * WN, BM = 32 * TM * WM, stage = (BN + BM) * ROW_BYTES * NBUF, box = dense_box(WN, WM, KG, TN, dense_pass(WN, WM, KG, TN, TM)),
                        lds = stage > box ? stage : box;
     const auto kernel = dense_gemm_kernel<T, WN, WM, KG, TN, TM, NBUF, MODE>;
@@ -513,9 +515,9 @@ void go(const DenseWeight& w, const DenseIn& in, uint32_t M, const DenseEpiArgs&
             // by 500 38 / - / - / 31.5, by 902 59 / - / - / 44.9.
             if (w.K >= 4096 && e.sums) {
                 const uint32_t large = t128 <= CUS / 2 ? (uint32_t)std::min<uint64_t>(8, CUS / t128) : 1;
-                if (t6432 <= 80) { go_gemm<T, 1, 1, 4, 2, 1, 4, MODE>(w, a, lda, M, e, s, 8); return; }
-                if (t64 <= CUS / 2) { go_gemm<T, 1, 1, 4, 2, 2, 4, MODE>(w, a, lda, M, e, s, 4); return; }
-                if (large > 1) { go_gemm<T, 2, 2, 2, 2, 2, 3, MODE>(w, a, lda, M, e, s, large); return; }
+                if (t6432 <= 80) { go_gemm<T, 1, 1, 4, 2, 1, 4, MODE, true>(w, a, lda, M, e, s, 8); return; }
+                if (t64 <= CUS / 2) { go_gemm<T, 1, 1, 4, 2, 2, 4, MODE, true>(w, a, lda, M, e, s, 4); return; }
+                if (large > 1) { go_gemm<T, 2, 2, 2, 2, 2, 3, MODE, true>(w, a, lda, M, e, s, large); return; }
             }
         }
         if (tiles(32, 32) <= 3 * CUS) { go_gemm<T, 1, 1, 4, 1, 1, 4, MODE>(w, a, lda, M, e, s); return; }
