@@ -112,10 +112,10 @@ __device__ __forceinline__ size_t paged_row(const PageTable& pt, uint32_t t) {
 // (the reference's quantiser gives it 1.0), as the fast prefill GEMM takes them.
 void launch_quantize_act(const float* x, uint32_t M, uint32_t K, int8_t* q, uint16_t* sc, hipStream_t s, bool neg_odd = false);
 // rms_norm of M rows; writes f32 `normed` if non-null and the quantised row (q, sc) if q non-null.
-// Prompt rows in fast mode: the norm with its squares added up in any order, codes with odd blocks negated, and, unless null, launch_act_block_sums' output.
-void launch_rmsnorm_rows(const float* x, const float* w, float eps, uint32_t M, uint32_t H, int8_t* q, uint16_t* sc, float* sums, hipStream_t s);
 void launch_rmsnorm(const float* x, const float* w, float eps, uint32_t M, uint32_t H, float* normed, int8_t* q,
                     uint16_t* sc, hipStream_t s, bool neg_odd = false);
+// Prompt rows in fast mode: the norm with its squares added up in any order, codes with odd blocks negated, and, unless null, launch_act_block_sums' output.
+void launch_rmsnorm_rows(const float* x, const float* w, float eps, uint32_t M, uint32_t H, int8_t* q, uint16_t* sc, float* sums, hipStream_t s);
 // out = silu(gate)*up over M rows where gate = gu[r][0..I), up = gu[r][I..2I) when fused, else two
 // pointers; writes f32 out if non-null and quantised (q, sc) if q non-null.
 void launch_silu_mul(const float* gate, const float* up, uint32_t M, uint32_t I, uint32_t row_stride, float* out,
