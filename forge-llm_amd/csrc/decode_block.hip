@@ -81,7 +81,7 @@ struct PbLayer {
 
 struct PbArgs {
     PbMat in[2], o[2], gate_up, down, loop, head;        // in, o: by PbKind
-    uint32_t L, W, Wn, ff, vocab, table_ld, table_n, G, act;
+    uint32_t L, W, Wn, ff, table_ld, table_n, G, act;
     uint32_t splits, splits_max, attend;                 // parts of a context; waves of a workgroup that attend
     LatentShape ls;
     GroupedShape gs;
@@ -1741,7 +1741,7 @@ int32_t pb_create(const PbModelIn& in, PbState** out) {
     st->cooperative = resident_cooperative();
     if (st->cooperative && !coop) return FORGE_HIP_OK;
     PbArgs& a = st->args;
-    a.W = in.width; a.Wn = in.ln_n; a.ff = layers[0].ff; a.vocab = in.head.N; a.L = (uint32_t)layers.size();
+    a.W = in.width; a.Wn = in.ln_n; a.ff = layers[0].ff; a.L = (uint32_t)layers.size();
     a.act = (uint32_t)layers[0].act;
     a.ls = ls; a.gs = gs; a.ns = ns;
     // The fewest workgroups that hold every matrix, then as few tiles each as that many allow.
