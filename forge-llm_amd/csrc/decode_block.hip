@@ -12,9 +12,9 @@
 //   * All workgroups share the output matrix.
 // A row times a vector is a product of 16 rows on the matrix unit.  Its other 15 columns are free, so a vector that the kernel sequence multiplies in 32-bit goes in as three
 // bfloat16 planes (x = hi + lo + rest, exact) in columns of their own: the same precision, no conversion of weights and no reduction over lanes.
-// What is not finite: an infinite or NaN element of a vector makes a row's product what it is in the sequence's 32-bit sums (infinite, or NaN where it meets a weight of 0).  Weights are finite, since
-// what pads a product multiplies them by 0: a model with others keeps the sequence.  A cached row's elements are taken to be finite as well (an infinite one, a projection past bfloat16's
-// range, may come out as NaN where the sequence has an infinity).
+// An element past bfloat16's range would be no number in its planes, and what pads a product multiplies weights and cached rows by 0: both take numbers of ordinary size.  A model has them if
+// no weight is larger than PB_LARGEST (2^32): a normed element is then below 2^40, a projection below 2^87, a gated head's output below 2^126.  A model with a larger weight, an infinity or a NaN
+// keeps the sequence (limits on the elements themselves, two instructions each, cost 4 us of 406 a token).
 //
 // Per token in us, kernel sequence / this, by rows of context (sizes of vabirax_135m: 9 heads of 64 + 32, window 1024; kakirax_135m: three layers of linear attention to one of grouped):
 //   latent            20: 882 / 393    200: 890 / 405    900: 905 / 420    2400: 907 / 419
@@ -126,16 +126,11 @@ __device__ __forceinline__ v8bf pb_load8(const __bf16* base, uint32_t off) {
 }
 __device__ __forceinline__ float pb_f32(const float* base, uint32_t i) { return ldg(base + i); }
 
-// Three bfloat16 that add up to x: what is past the largest bfloat16 goes on to the next, infinities and NaN to the last.
+// Three bfloat16 that add up to x.
 __device__ __forceinline__ void pb_split(float x, __bf16& hi, __bf16& lo, __bf16& rest) {
-    // (the limits as literals: in a register of their own they made the wide form spill, 712 -> 752 us a token)
-    auto in_range = [](float v) {
-        asm("v_min_f32 %0, 0x7f7f0000, %0\n\tv_max_f32 %0, 0xff7f0000, %0" : "+v"(v));
-        return v;
-    };
-    hi = (__bf16)in_range(x);
+    hi = (__bf16)x;
     const float r = x - (float)hi;
-    lo = (__bf16)in_range(r);
+    lo = (__bf16)r;
     rest = (__bf16)(r - (float)lo);
 }
 __device__ __forceinline__ uint32_t pb_pack(float a, float b) {
@@ -1655,13 +1650,15 @@ __global__ __launch_bounds__(256) void pb_transpose_kernel(const uint16_t* __res
     out[i] = uk[(size_t)head * dim * rank + j % dim * rank + j / dim];
 }
 
-// flag <- 1 if one of n pieces of eight bfloat16 holds an infinity or NaN
-__global__ __launch_bounds__(256) void pb_not_finite_kernel(const uint4* __restrict__ w, size_t n, uint32_t* flag) {
-    auto odd = [](uint32_t v) { return (v & 0x7F80u) == 0x7F80u || (v & 0x7F800000u) == 0x7F800000u; };
+// flag <- 1 if one of the weights is larger than PB_LARGEST, infinite or NaN.  Workgroup (.., weights).
+constexpr uint32_t PB_LARGEST = 0x4F800000u;
+struct PbWeights { const uint32_t* w; uint64_t words; uint32_t f32; };      // bfloat16: two to a word
+__global__ __launch_bounds__(256) void pb_large_kernel(const PbWeights* __restrict__ all, uint32_t* flag) {
+    const PbWeights m = all[blockIdx.y];
     bool any = false;
-    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
-        const uint4 v = w[i];
-        any = any || odd(v.x) || odd(v.y) || odd(v.z) || odd(v.w);
+    for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < m.words; i += (uint64_t)gridDim.x * 256) {
+        const uint32_t v = m.w[i];
+        any = any || (m.f32 ? (v & 0x7FFFFFFFu) > PB_LARGEST : (v & 0x7FFF0000u) > PB_LARGEST || (v << 16 & 0x7FFF0000u) > PB_LARGEST);
     }
     if (any) *flag = 1;
 }
@@ -1804,24 +1801,30 @@ int32_t pb_create(const PbModelIn& in, PbState** out) {
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, st->kernel, PB_THREADS, st->lds) != hipSuccess || per_cu < 1) { (void)hipGetLastError(); return FORGE_HIP_OK; }
     st->grid = (uint32_t)cus;
 
-    uint32_t* flag = st->dev<uint32_t>(4);
-    if (!flag) return FORGE_HIP_OK;
-    FH_HIP(hipMemset(flag, 0, 4));
-    std::vector<const void*> seen;                                   // a layer may run with another one's tensors
-    auto look = [&](const DenseWeight& w) {
-        if (!w.p || std::find(seen.begin(), seen.end(), w.p) != seen.end()) return;
-        seen.push_back(w.p);
-        const size_t n = (size_t)w.N * w.K / 8;
-        fh::launch(pb_not_finite_kernel, dim3((uint32_t)std::min<size_t>((n + 255) / 256, 4096)), 256, 0, nullptr, (const uint4*)w.p, n, flag);
+    std::vector<PbWeights> looked;
+    auto look = [&](const void* w, uint64_t n, bool f32) {           // a layer may run with another one's tensors
+        if (w && std::none_of(looked.begin(), looked.end(), [&](const PbWeights& l) { return l.w == w; })) looked.push_back(PbWeights{(const uint32_t*)w, f32 ? n : n / 2, f32 ? 1u : 0u});
     };
-    look(in.head);
-    look(in.loop);
-    for (const PbLayerIn& l : layers)
-        for (const DenseWeight* w : {&l.mixer->in, &l.mixer->o, &l.mixer->uq, &l.mixer->ukv, &l.gate_up, &l.down}) look(*w);
-    uint32_t not_finite = 0;
+    auto look_matrix = [&](const DenseWeight& w) { look(w.p, (uint64_t)w.N * w.K, false); };
+    look_matrix(in.head);
+    look_matrix(in.loop);
+    for (const PbLayerIn& l : layers) {
+        const PbMixer& m = *l.mixer;
+        for (const DenseWeight* w : {&m.in, &m.o, &m.uq, &m.ukv, &l.gate_up, &l.down}) look_matrix(*w);
+        for (const float* w : {latent ? l.norm1.w : l.ln1.w, latent ? l.norm2.w : l.ln2.w}) look(w, 2 * (uint64_t)a.W, true);
+        const bool lat = m.kind == MixerKind::LatentAttention, lin = m.kind == MixerKind::LinearAttention;
+        look(lin ? m.wc : m.wa, lat ? ls.q_rank : lin ? ns.vdim : gs.dim, true);
+        if (!lin) look(m.wb, lat ? ls.rank : gs.dim, true);
+    }
+    PbWeights* looked_dev = st->dev<PbWeights>(looked.size() * sizeof(PbWeights));
+    uint32_t *flag = st->dev<uint32_t>(4), large = 0;
+    if (!looked_dev || !flag) return FORGE_HIP_OK;
+    FH_HIP(hipMemset(flag, 0, 4));
+    FH_HIP(hipMemcpy(looked_dev, looked.data(), looked.size() * sizeof(PbWeights), hipMemcpyHostToDevice));
+    fh::launch(pb_large_kernel, dim3(128, (uint32_t)looked.size()), 256, 0, nullptr, looked_dev, flag);
     FH_HIP(hipGetLastError());
-    FH_HIP(hipMemcpy(&not_finite, flag, 4, hipMemcpyDeviceToHost));
-    if (not_finite) return FORGE_HIP_OK;
+    FH_HIP(hipMemcpy(&large, flag, 4, hipMemcpyDeviceToHost));
+    if (large) return FORGE_HIP_OK;
 
     std::vector<PbLayer> host(layers.size());
     const uint32_t uk_n = ls.heads * ls.dim * ls.rank;
