@@ -47,7 +47,10 @@ namespace {
 constexpr uint32_t PB_POLL = 4, PB_COMP = 8, PB_WAVES = PB_POLL + PB_COMP, PB_THREADS = PB_WAVES * 64, PB_POLL_THREADS = PB_POLL * 64;
 constexpr float PB_LOG2E = 1.4426950408889634f;
 constexpr float PB_NO_KEYS = -3.0e38f;       // maximum of a part without keys: weight 0
-// What registers hold: tiles of 16 rows a workgroup, pieces of 32 columns a wave.
+// Limits of the narrow forms: tiles of 16 rows a workgroup, pieces of 32 columns a wave, and the heads' sizes below.  What they are bound by (one of them raised at a time, compiled, not measured):
+// registers hold no longer cached row (PB_ROW 192 spills 16 bytes a lane) and LDS no longer latent (its transposed values are 120 KB of 159).  The others are the widths of the models at hand: one
+// more tile or piece of a matrix (width 1024, feed-forward 2048) spills nothing in 143 to 161 registers of 168; nor do PB_QR 256 (a polling thread an element), PB_DIM 128 (dim and rot together: 16
+// rows a wave, 192) and PB_VDIM 128.
 constexpr int PB_TI = 2, PB_UI = 3;          // input product
 constexpr int PB_UO = 3;                     // output product
 constexpr int PB_TG = 3;                     // gate;up
@@ -1255,6 +1258,7 @@ __global__ __launch_bounds__(PB_THREADS) void decode_block_kernel(PbArgs a) {
 //   * the next layer's input product goes into LDS while the heads are at work, for which registers have no room: the same time, but no spills with half of gate;up early as well.
 // Without effect: at most 4, 8 or 12 KB of a wave under way, output product and a quarter of gate;up requested a phase earlier (720).  Spilled registers cost more than anything: a spill waits for
 // all loads (28 of them: 758 -> 840).
+// Limits: the width (a fifth piece, 2560, spills 120 bytes a lane more) and gate;up's tiles (ten: 92 more) by registers; the depth of down is what the model at hand has (10240 spills nothing more).
 constexpr uint32_t PW_WIDTH = 2048, PW_FF = 8192;
 constexpr int PW_U = 4, PW_UD = 16;          // pieces of a wave in a half: depth PW_WIDTH, PW_FF
 constexpr int PW_TI = 4, PW_TIL = 3, PW_TG = 8, PW_TGA = 4;      // tiles of a workgroup: input product (the first PW_TIL of them in LDS), gate;up (the first PW_TGA of them requested early)

@@ -381,8 +381,11 @@ bool gemm_rows_supported(const QWeight& w, uint32_t M, bool silu) {
 
 // Ranges of K, one to a workgroup, for deep products whose tiles leave half the compute units idle: a workgroup takes 20 bytes of weights a nanosecond, and 64 of them 14 us for
 // 8192 -> 2048.  us with the quantiser, whole / in ranges (six operand sets in turn): Q8_0 8192 -> 2048 by 5 rows 15.1 / 11.8, 32 (4 ranges) 16.1 / 11.9, 64 (2) 16.3 / 13.7, 8192 -> 3072
-// by 16 15.3 / 12.2, Q4_0 8192 -> 2048 by 32 14.8 / 12.0.  Not 4096 -> 1024 (by 16 10.8 / 9.5, but by 32 10.9 / 12.0, by 64 10.8 / 11.3), nor two ranges with two rows of tiles
-// to a workgroup (8192 -> 2048 by 100 16.3 / 18.6).
+// by 16 15.3 / 12.2, Q4_0 8192 -> 2048 by 32 14.8 / 12.0.  Not two ranges with two rows of tiles to a workgroup (8192 -> 2048 by 100 16.3 / 18.6).
+// Shallower ones, whole (the quantiser in the launch where that pays) / in ranges, by 5, 16, 32 and 64 rows: Q8_0 4096 -> 1024 8.1 / 11.1, 9.1 / 11.1, 10.4 / 11.2, 10.5 / 11.0, 5632 -> 2048 10.2 / 10.9,
+// 11.4 / 10.9, 12.5 / 10.9, 12.7 / 12.0, 7168 -> 2048 12.0 / 10.9, 13.4 / 10.9, 15.0 / 11.5, 15.0 / 13.1; Q4_0 4096 -> 2048 8.4 / 11.2, 8.8 / 11.1, 10.5 / 11.2, 10.7 / 11.0, 5632 -> 2048 10.0 / 11.0,
+// 11.2 / 11.0, 11.8 / 11.0, 12.1 / 12.0, 7168 -> 2048 11.5 / 11.0, 12.6 / 11.0, 13.9 / 11.3, 14.2 / 12.8.  The two meet about 5632; the line is at 8192, the depth of the first measurements, and
+// gives away 1 to 3 us from there on.
 static uint32_t ranges(const QWeight& w, uint32_t M) {
     const uint64_t grid = (uint64_t)((w.N + 31) / 32) * ((M + 31) / 32);
     return w.K >= 8192 && M <= 64 && grid <= 128 ? (uint32_t)std::min<uint64_t>(FR_PARTS, 256 / grid) : 1;
