@@ -17,8 +17,8 @@
 // keeps the sequence (limits on the elements themselves, two instructions each, cost 4 us of 406 a token).
 //
 // Per token in us, kernel sequence / this, by rows of context (sizes of vabirax_135m: 9 heads of 64 + 32, window 1024; kakirax_135m: three layers of linear attention to one of grouped):
-//   latent            20: 882 / 393    200: 890 / 405    900: 905 / 420    2400: 907 / 419
-//   linear, grouped   20: 646 / 414    200: 648 / 420    900: 650 / 424    2400: 654 / 436
+//   latent            20: 886 / 389    200: 895 / 398    900: 900 / 421    2400: 901 / 422
+//   linear, grouped   20: 647 / 402    200: 647 / 408    900: 648 / 412    2400: 648 / 421
 // What bounds it: the chain.  A layer run of the first takes 13 us: input product 1.9, the heads 5.5 (0.6 of them the merge of eight parts), output product 1.5, gate;up 1.8, down 2.0, each
 // of the products 0.4 to 1.2 of waiting for what was handed over, 0.4 on the matrix unit and 0.4 of sums, epilogue and store.  Its weights (7.7 MB) would take 1.6.  What
 // decided the form, measured: branches around the pieces of a product (each read of the vector then waits for the one before) 502 -> 453 at 2400 rows; values transposed ahead of the query, and
@@ -1250,8 +1250,8 @@ __global__ __launch_bounds__(PB_THREADS) void decode_block_kernel(PbArgs a) {
 // 8 rows by two halves of the depth (row r of the product: row r % 8, half r / 8), tile t of a workgroup the grid's tile t G + wg: no row of a 2048-row matrix is left over on 256 workgroups.  A
 // column of the vector is a plane of one half.
 //
-// Per token in us, kernel sequence / this, kakirax_1b (width 2048, feed-forward 8192, three layers of linear attention to one of grouped): 20 rows 849 / 705, 902 855 / 718, 2400 859 / 735,
-// 6000 869 / 748.  What bounds it: the weights (134 MB a layer, 24 us of its 38) and the hand-overs while nothing is on its way (8 us between down's vector and the next input product's, 5 in
+// Per token in us, kernel sequence / this, kakirax_1b (width 2048, feed-forward 8192, three layers of linear attention to one of grouped): 20 rows 837 / 701, 902 838 / 712, 2400 839 / 723,
+// 6000 845 / 738.  What bounds it: the weights (134 MB a layer, 24 us of its 38) and the hand-overs while nothing is on its way (8 us between down's vector and the next input product's, 5 in
 // the others).  A compute unit takes about 64 KB of requests and a wave that has more to ask for stands still, so what decided the form is what stands in front of a barrier (us a token):
 //   * a head's workgroup asks for its next input product only when it has its output product (its polls would wait behind 260 KB): 760 -> 753, and its barriers come first: 753 -> 722;
 //   * down is requested behind the barrier that ends gate;up, not ahead of it: 753 -> 721;
